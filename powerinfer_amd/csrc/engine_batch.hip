@@ -70,6 +70,10 @@ pi_norm mk_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
 int chunk_attention(pi_model * m, BatchState * b, int T, size_t kv_off) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
+    const char * own = getenv("PI_ATTN_CHUNK");
+    if (pi::attn_chunk_rows_fits(hd, T, b->kv_hi, b->att, b->att16, d) && !(own && !strcmp(own, "scalar")))
+        return pi::attn_chunk_rows(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
+                               m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
     if (pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi))
         return pi_k_attn_chunk(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
                                m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);

@@ -746,6 +746,268 @@ __global__ __launch_bounds__(kBlock) void attn_chunk_mfma_kernel(const float * _
 }
 
 // ---------------------------------------------------------------------------------------------------
+// Attention of a prompt chunk, 64 U tokens of one query head per workgroup.  attn_chunk_mfma_kernel reads a head's cells once for 16
+// tokens, holds all their scores in LDS (which ends at about 1850 cells) and is bound by those reads; here a tile of 64 cells is staged
+// once for 64 or 128 tokens and no score leaves the registers, so the cells a chunk may see are not limited.  The soft-max keeps the
+// rounding points of attn_decode_kernel, fp16 in and out of exp relative to the row's maximum over ALL its cells, which is why the
+// keys are gone through twice: first for the maximum (products and comparisons only), then for the weights.  What is left out is the
+// rounding of e / sum to fp16: the weights e are fp16 values as they are, and their sum divides the result.
+// Scores are formed transposed (cells x tokens): a lane's scores belong to one token, and its weights are already the column operand of
+// values^T x weights - which cell a slot of that product's inner dimension stands for is free, so the values are read (transposed,
+// ds_read_tr16) in the order the scores came out.  The sum is one more product, with ones, added up over the tiles in double.
+// Bound by the exponentials (about 40 cycles of VALU per 64 of them) beside 48 of matrix cores.  32 heads of 128, RoPE and store included:
+// 512 tokens behind 0 / 512 / 1024 / 1535: 42 / 59 / 75 / 84 us (attn_chunk_mfma_kernel 61 / 117 / 159, attn_decode_kernel 791 past the
+// cells that one holds); 128 heads of 64 on 8: 43 / 66 / 88 / 109 (94 / 271 / 380 / 493).
+// ---------------------------------------------------------------------------------------------------
+typedef short pi_s4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ pi_u32x2 lds_tr_read(const unsigned char * q) {
+    return __builtin_bit_cast(pi_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pi_s4 *)(__attribute__((address_space(3))) void *)q));
+}
+constexpr int kRowsCells = 64;                 // cells of a tile
+constexpr int kRowsWideGrid = 512;
+template <int HD> constexpr int rows_pitch() { return HD * 2 + 16; }                       // bytes of a staged row: 16 of padding spread the rows over the banks
+template <int HD> constexpr size_t rows_lds() { return (size_t)4 * kRowsCells * rows_pitch<HD>(); }
+
+template <int HD, int U>
+__global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float * __restrict__ q_rot, const __half * __restrict__ k_cache,
+                                                                    const __half * __restrict__ v_cache, int n_head, int n_head_kv, int n_ctx,
+                                                                    const int32_t * __restrict__ pos_p, int T, int n_kv_max, float * __restrict__ out,
+                                                                    int q_stride, int out_stride, __half * __restrict__ out16) {
+    static_assert(HD == 128 || HD == 64, "head size");
+    constexpr int R = 64 * U, NK = kRowsCells, KS = HD / 32, VT = HD / 16, KT = NK / 16, ROW = rows_pitch<HD>(), PPR = HD / 8, NP = NK * PPR / kBlock;
+    extern __shared__ __align__(16) unsigned char smem[];                                  // two tiles of keys, two of values
+    __shared__ int span[2 * kWavesPerBlock], odd[2];
+    const int h = blockIdx.x, kvh = h / (n_head / n_head_kv), t0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * R;      // the tokens that see the most cells first
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    // the most and the fewest cells a token here sees
+    {
+        const int t = t0 + tid % R, nv = t < T ? min(pos_p[t] + 1, n_kv_max) : -1;
+        int hi = nv, lo = nv < 0 ? INT32_MAX : nv;
+        for (int o = 32; o > 0; o >>= 1) { hi = max(hi, __shfl_xor(hi, o, PI_WAVE)); lo = min(lo, __shfl_xor(lo, o, PI_WAVE)); }
+        if (lane == 0) { span[wave] = hi; span[kWavesPerBlock + wave] = lo; }
+        if (tid < 2) odd[tid] = 0;
+    }
+    int nv[U];
+    pi_u32x4 qf[U][KS];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = t0 + wave * 16 * U + u * 16 + i;
+        nv[u] = t < T ? min(pos_p[t] + 1, n_kv_max) : 0;
+        const float * qp = q_rot + (size_t)min(t, T - 1) * q_stride + (size_t)h * HD + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const float4 a = *reinterpret_cast<const float4 *>(qp + s * 32), b = *reinterpret_cast<const float4 *>(qp + s * 32 + 4);
+            qf[u][s] = __builtin_bit_cast(pi_u32x4, pi_h8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w, (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w});
+        }
+    }
+    __syncthreads();
+    int n_keys = span[0], n_all = span[kWavesPerBlock];
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlock; ++w) { n_keys = max(n_keys, span[w]); n_all = min(n_all, span[kWavesPerBlock + w]); }
+    // this thread's pieces of a tile; cells past the last one read the last one again (never a cell that no token here sees)
+    const __half * kb = k_cache + (size_t)kvh * n_ctx * HD + (tid % PPR) * 8;
+    const __half * vb = v_cache + (size_t)kvh * n_ctx * HD + (tid % PPR) * 8;
+    const int row0 = tid / PPR, last = max(n_keys - 1, 0);
+    pi_u32x4 pk[NP], pv[NP];
+    auto fetch = [&](pi_u32x4 * dst, const __half * base, int cb) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) dst[j] = pi_ld16(base + (size_t)min(cb + row0 + j * (kBlock / PPR), last) * HD);
+    };
+    auto place = [&](unsigned char * tile, const pi_u32x4 * src) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) *reinterpret_cast<pi_u32x4 *>(tile + (row0 + j * (kBlock / PPR)) * ROW + (tid % PPR) * 16) = src[j];
+    };
+    auto products = [&](const unsigned char * tile, pi_f4 (*s)[KT]) {
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) s[u][kt] = pi_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < KS; ++c) {
+                const pi_u32x4 a = *reinterpret_cast<const pi_u32x4 *>(tile + (kt * 16 + i) * ROW + c * 64 + g * 16);
+#pragma unroll
+                for (int u = 0; u < U; ++u) s[u][kt] = mma16<__half>(a, qf[u][c], s[u][kt]);
+            }
+        }
+    };
+    constexpr int TILE = NK * ROW;
+    const float scale = pi_inv_sqrt((float)HD);
+
+    // ---- the rows' maxima (two tiles of keys in LDS: one barrier a tile) ----
+    float mx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) mx[u] = -INFINITY;
+    int at = 0;
+    fetch(pk, kb, 0);
+    for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
+        place(smem + at * TILE, pk);
+        __syncthreads();
+        fetch(pk, kb, cb + NK);
+        pi_f4 s[U][KT];
+        products(smem + at * TILE, s);
+        const bool edge = cb + NK > n_all;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx[u] = fmaxf(mx[u], edge && cb + kt * 16 + 4 * g + r >= nv[u] ? -INFINITY : s[u][kt][r]);
+    }
+    float base[U];                                                       // -maximum of the scaled scores
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 16, PI_WAVE));
+        mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 32, PI_WAVE));
+        base[u] = mx[u] == -INFINITY ? 0.0f : -__fmul_rn(mx[u], scale);
+    }
+
+    // ---- weights and values ----
+    double sum[U];
+    pi_f4 o[U][VT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        sum[u] = 0.0;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) o[u][v] = pi_f4{0, 0, 0, 0};
+    }
+    const pi_u32x4 ones{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+    unsigned char * vt = smem + 2 * TILE;
+    fetch(pk, kb, 0);
+    fetch(pv, vb, 0);
+    __syncthreads();                                                     // the last tile of the first pass has been read
+    at = 0;
+    for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
+        const bool edge = cb + NK > n_all;
+        place(smem + at * TILE, pk);
+        place(vt + at * TILE, pv);
+        if (edge) {                                                      // a value that is no number, in a cell that some tokens here do not see
+            unsigned bad = 0;
+#pragma unroll
+            for (int j = 0; j < NP; ++j)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) { const unsigned x = pv[j][w] & 0x7C007C00u; bad |= (x & 0xFFFFu) == 0x7C00u || (x >> 16) == 0x7C00u; }
+            if (bad) odd[at] = 1;
+        }
+        __syncthreads();
+        fetch(pk, kb, cb + NK);
+        fetch(pv, vb, cb + NK);
+        pi_f4 s[U][KT];
+        products(smem + at * TILE, s);
+        pi_u32x4 pb[U][KT / 2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            _Float16 w[4 * KT];
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    // e^x as 2^(x log2 e): fp16 in, fp16 out, the fp32 steps between are good to 1e-6
+                    const float x = (float)(_Float16)fmaf(s[u][kt][r], scale, base[u]);
+                    const float e = __builtin_amdgcn_exp2f(x * 1.4426950408889634f);
+                    w[kt * 4 + r] = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= nv[u] ? 0.0f : e);
+                }
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k) {
+                pb[u][k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
+            }
+            pi_f4 l = pi_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k) l = mma16<__half>(ones, pb[u][k], l);
+            sum[u] += (double)l[0];
+        }
+        const unsigned char * vs = vt + at * TILE;
+        if (edge && odd[at]) {
+            // 0 times such a value is no number either: token by token, the cells it sees only.  The weight of cell (kt, g, r) of token i is
+            // half (kt % 2) * 4 + r of step kt / 2 in lane 16 g + i.
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                for (int c = 0; c < NK; ++c) {
+                    const int kt = c >> 4, from = ((c >> 2) & 3) * 16 + i, half = (kt & 1) * 4 + (c & 3);
+                    unsigned word = 0;
+#pragma unroll
+                    for (int k = 0; k < KT / 2; ++k)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) word = k == (kt >> 1) && q == (half >> 1) ? pb[u][k][q] : word;
+                    const unsigned got = (unsigned)__shfl((int)word, from, PI_WAVE);
+                    const float w = pi_f16_from_bits((uint16_t)(half & 1 ? got >> 16 : got));
+                    if (cb + c >= nv[u]) continue;
+#pragma unroll
+                    for (int v = 0; v < VT; ++v)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) o[u][v][r] = fmaf(w, __half2float(reinterpret_cast<const __half *>(vs + c * ROW)[v * 16 + 4 * g + r]), o[u][v][r]);
+                }
+            continue;
+        }
+        // slot (g, j) of a 32-cell step: cell 4 g + j of its first 16 (j < 4) or of its second 16 - two transposing reads
+#pragma unroll
+        for (int k = 0; k < KT / 2; ++k)
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                const unsigned char * a = vs + (k * 32 + 4 * g + (i >> 2)) * ROW + (v * 16 + (i & 3) * 4) * 2;
+                const pi_u32x2 lo = lds_tr_read(a), hi = lds_tr_read(a + 16 * ROW);
+                const pi_u32x4 fr{lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+                for (int u = 0; u < U; ++u) o[u][v] = mma16<__half>(fr, pb[u][k], o[u][v]);
+            }
+    }
+    // o[u][v][r] = out[token i][v * 16 + 4 g + r]
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = t0 + wave * 16 * U + u * 16 + i;
+        if (t >= T) continue;
+        const float inv = (float)(1.0 / sum[u]);
+        float * po = out + (size_t)t * out_stride + (size_t)h * HD + 4 * g;
+        __half * ph = out16 ? out16 + (size_t)t * out_stride + (size_t)h * HD + 4 * g : nullptr;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const float4 y{__fmul_rn(o[u][v][0], inv), __fmul_rn(o[u][v][1], inv), __fmul_rn(o[u][v][2], inv), __fmul_rn(o[u][v][3], inv)};
+            *reinterpret_cast<float4 *>(po + v * 16) = y;
+            if (ph) {
+                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                *reinterpret_cast<h4 *>(ph + v * 16) = h4{(_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w};
+            }
+        }
+    }
+}
+
+// RoPE + KV store of a chunk's tokens, all heads of a token by one workgroup (or by gridDim.y of them, heads in turn): the angles are
+// formed once a token instead of once a head, bit for bit those of rope_kv_store_kernel, and the rest is a copy at the rate of memory.
+__global__ __launch_bounds__(kBlock) void rope_kv_chunk_kernel(const float * __restrict__ qkv, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                                                               const int32_t * __restrict__ pos_p, int n_ctx, float * __restrict__ q_rot,
+                                                               __half * __restrict__ k_cache, __half * __restrict__ v_cache, int qkv_stride, int q_stride) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    float2 * cs = reinterpret_cast<float2 *>(smem);                      // [hd / 2]
+    const int t = blockIdx.x, tid = threadIdx.x, half = hd / 2, pos = pos_p[t];
+    for (int j = tid; j < half; j += kBlock) {
+        const float theta = rope_angle((float)pos, j, mode, theta_scale, freq_scale);
+        cs[j] = make_float2(cosf(theta), sinf(theta));
+    }
+    __syncthreads();
+    const float * src = qkv + (size_t)t * qkv_stride;
+    float * qd = q_rot + (size_t)t * q_stride;
+    const int pairs = (n_head + 2 * n_head_kv) * half;
+    for (int e = blockIdx.y * kBlock + tid; e < pairs; e += gridDim.y * kBlock) {
+        const int h = e / half, j = e % half;
+        const bool value = h >= n_head + n_head_kv;
+        const int i0 = (mode & 2) && !value ? j : 2 * j, i1 = (mode & 2) && !value ? j + half : 2 * j + 1;
+        const float x0 = src[(size_t)h * hd + i0], x1 = src[(size_t)h * hd + i1];
+        if (value) {
+            __half * dst = v_cache + ((size_t)(h - n_head - n_head_kv) * n_ctx + pos) * hd;
+            dst[i0] = __float2half_rn(x0); dst[i1] = __float2half_rn(x1);
+            continue;
+        }
+        const float c = cs[j].x, s = cs[j].y;
+        const float y0 = __fsub_rn(__fmul_rn(x0, c), __fmul_rn(x1, s)), y1 = __fadd_rn(__fmul_rn(x0, s), __fmul_rn(x1, c));
+        if (h < n_head) {
+            qd[(size_t)h * hd + i0] = y0; qd[(size_t)h * hd + i1] = y1;
+        } else {
+            __half * dst = k_cache + ((size_t)(h - n_head) * n_ctx + pos) * hd;
+            dst[i0] = __float2half_rn(y0); dst[i1] = __float2half_rn(y1);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------
 // One token's attention on the layouts of the reference's own KV cache (llm_build_kv_store / llm_build_kqv, llama.cpp:4383-4418,
 // 4764-4850): K cells [cell][n_head_kv * hd] fp16, V transposed [n_head_kv * hd][n_ctx] fp16.  What its graph spreads over eleven nodes
 // - RoPE of q and k, the two copies into the cache, K.q, scale, + mask, soft-max, V.p and the gather of the heads - is one launch, one
@@ -903,6 +1165,55 @@ __global__ __launch_bounds__(kBlock) void attn_ggml_kernel(const float * __restr
 }
 
 }  // namespace
+
+namespace {
+constexpr size_t kChunkMfmaLds = 156 * 1024;
+size_t chunk_mfma_lds(int hd, int n_kv_max) { return sizeof(float) * 16 * (size_t)(((n_kv_max + 31) & ~31) + 4) + (size_t)kWavesPerBlock * hd * kAcVtStride * 2; }
+
+int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
+                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st) {
+    // 16 tokens and fewer: a workgroup per head and token (16 tokens, 32 heads of 128, attention included: 11.8 against 12.3 us); a chunk's angles
+    // are worth forming once a token from there on.  A workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
+    if (T <= kBtMaxT) {
+        hipLaunchKernelGGL(rope_kv_store_kernel, dim3(n_head + 2 * n_head_kv, T), dim3(hd / 2), 0, st,
+                           qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
+        return pi::check_launch("rope_kv_store");
+    }
+    const int split = T >= 512 ? 1 : T >= 128 ? 4 : 16;
+    hipLaunchKernelGGL(rope_kv_chunk_kernel, dim3(T, split), dim3(kBlock), sizeof(float2) * (hd / 2), st, qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot,
+                       (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
+    return pi::check_launch("rope_kv_chunk");
+}
+
+template <int HD, int U>
+int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_cache, int n_head, int n_head_kv, int n_ctx, const int32_t * pos, int T, int n_kv_max, float * out,
+                      int out_stride, void * out_f16, hipStream_t st) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_kernel<HD, U>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
+    if (raised != hipSuccess) return pi::hip_fail(raised, "attn_chunk_rows: LDS size");
+    hipLaunchKernelGGL((attn_chunk_rows_kernel<HD, U>), dim3(n_head, (T + 64 * U - 1) / (64 * U)), dim3(kBlock), rows_lds<HD>(), st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
+                       n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, n_head * HD, out_stride, (__half *)out_f16);
+    return pi::check_launch("attn_chunk_rows");
+}
+}  // namespace
+
+namespace pi {
+// head sizes and alignments of attn_chunk_rows_kernel (outputs are stored four columns at a time), and where it is the faster one: fewer than
+// 32 tokens against many cells are better off with attn_chunk_mfma_kernel, whose waves split the cells (17 tokens, 1817 cells, 32 heads of
+// 128: 59 us here, 49 there; 317 cells: 17.5 and 17.7; 48 tokens, 1848 cells: 62 and 102)
+bool attn_chunk_rows_fits(int hd, int T, int n_kv_max, const void * out, const void * out_f16, int out_stride) {
+    return (hd == 64 || hd == 128) && T > kBtMaxT && (T >= 32 || n_kv_max <= 512 || chunk_mfma_lds(hd, n_kv_max) > kChunkMfmaLds) && out_stride % 4 == 0 &&
+           ((uintptr_t)out & 15) == 0 && ((uintptr_t)out_f16 & 7) == 0;
+}
+int attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
+                    int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16, hipStream_t st) {
+    int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    if (rc != PI_OK) return rc;
+    const bool two = (long long)n_head * ((T + 127) / 128) >= kRowsWideGrid;
+#define PI_ROWS(HD, U) launch_chunk_rows<HD, U>(q_rot, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
+    return hd == 128 ? (two ? PI_ROWS(128, 2) : PI_ROWS(128, 1)) : (two ? PI_ROWS(64, 2) : PI_ROWS(64, 1));
+#undef PI_ROWS
+}
+}  // namespace pi
 
 extern "C" {
 
@@ -1068,18 +1379,20 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || hd <= 0 || hd % 8 || hd / 2 > 1024 || kBlock % (hd / 8) || PI_WAVE % (hd / 8) || (mode != 0 && mode != 2))
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad head geometry or mode");
     hipStream_t st = (hipStream_t)stream;
+    const char * own = getenv("PI_ATTN_CHUNK");
+    const bool scalar = own && !strcmp(own, "scalar");
+    if (!scalar && pi_k_attn_chunk_supported(hd, n_ctx, n_kv_max) && pi::attn_chunk_rows_fits(hd, T, n_kv_max, out, out_f16, out_stride))
+        return pi::attn_chunk_rows(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, n_kv_max, q_rot, k_cache, v_cache, out, out_stride, out_f16, st);
     // all K/V rows of the chunk are in the cache before any token of the chunk attends
-    hipLaunchKernelGGL(rope_kv_store_kernel, dim3(n_head + 2 * n_head_kv, T), dim3(hd / 2), 0, st,
-                       qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
+    rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     // 16 tokens per workgroup on the matrix cores where the head size and the context fit (scores of 16 tokens in LDS)
     const int s_stride = ((n_kv_max + 31) & ~31) + 4;
-    const size_t sh_mfma = sizeof(float) * 16 * (size_t)s_stride + (size_t)kWavesPerBlock * hd * kAcVtStride * 2;
-    const char * own = getenv("PI_ATTN_CHUNK");
-    if ((hd == 128 || hd == 64) && T > 1 && sh_mfma <= 156 * 1024 && !(own && !strcmp(own, "scalar"))) {
+    const size_t sh_mfma = chunk_mfma_lds(hd, n_kv_max);
+    if ((hd == 128 || hd == 64) && T > 1 && sh_mfma <= kChunkMfmaLds && !scalar) {
         static bool raised[2] = {false, false};
         if (!raised[hd == 64]) {
-            if (hd == 128) PI_HIP_TRY(hipFuncSetAttribute((const void *)attn_chunk_mfma_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024));
-            else           PI_HIP_TRY(hipFuncSetAttribute((const void *)attn_chunk_mfma_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024));
+            if (hd == 128) PI_HIP_TRY(hipFuncSetAttribute((const void *)attn_chunk_mfma_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kChunkMfmaLds));
+            else           PI_HIP_TRY(hipFuncSetAttribute((const void *)attn_chunk_mfma_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kChunkMfmaLds));
             raised[hd == 64] = true;
         }
         const dim3 grid(n_head, (T + 15) / 16);
@@ -1099,9 +1412,7 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
 int pi_k_attn_chunk_supported(int hd, int n_ctx, int n_kv_max) {
     if (hd <= 0 || hd % 8 || kBlock % (hd / 8) || PI_WAVE % (hd / 8) || n_ctx <= 0) return 0;
     if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;
-    const int s_stride = ((n_kv_max + 31) & ~31) + 4;
-    const size_t sh_mfma = sizeof(float) * 16 * (size_t)s_stride + (size_t)kWavesPerBlock * hd * kAcVtStride * 2;
-    if ((hd == 128 || hd == 64) && sh_mfma <= 156 * 1024) return 1;
+    if ((hd == 128 || hd == 64) && chunk_mfma_lds(hd, n_kv_max) <= kChunkMfmaLds) return 1;
     return sizeof(float) * ((size_t)n_ctx + (size_t)(kBlock / (hd / 8)) * hd) <= 60 * 1024;
 }
 
@@ -1113,8 +1424,7 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (mode != 0 && mode != 2) || hd % 2 || hd / 2 > 1024 || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_chunk_long: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(rope_kv_store_kernel, dim3(n_head + 2 * n_head_kv, T), dim3(hd / 2), 0, st,
-                       qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
+    rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)T * n_head * n_parts * hd;

@@ -1,0 +1,79 @@
+"""Attention of long prompt chunks, 64 or 128 tokens of a head per workgroup (attn_chunk_rows_kernel): against float64 on the rounded
+operands, at the edges of its row and cell tiles, and with values that are no numbers in cells that a token does not see."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def rotated(x, pos, mode, hd):
+    """x [T, heads, hd]; the angles in float32, advanced by repeated products as the kernels form them."""
+    scale = np.float32(np.float32(10000.0) ** np.float32(-2.0 / hd))
+    th = np.empty((len(pos), hd // 2), np.float32)
+    th[:, 0] = pos
+    for i in range(1, hd // 2):
+        th[:, i] = th[:, i - 1] * scale
+    c, s = np.cos(th)[:, None].astype(np.float64), np.sin(th)[:, None].astype(np.float64)
+    a, b = (slice(0, hd // 2), slice(hd // 2, hd)) if mode == 2 else (slice(0, hd, 2), slice(1, hd, 2))
+    y = np.empty(x.shape)
+    y[..., a], y[..., b] = x[..., a] * c - x[..., b] * s, x[..., a] * s + x[..., b] * c
+    return y
+
+
+def run(hd, nh, nkv, mode, past, T, n_ctx, spoil=None):
+    from powerinfer_amd import lib as pl
+    L = pl.init()
+    rng = np.random.default_rng(hd + nh + past + T)
+    gqa, d = nkv * hd, nh * hd
+    kc = rng.standard_normal((nkv, n_ctx, hd)).astype(np.float16)
+    vc = rng.standard_normal((nkv, n_ctx, hd)).astype(np.float16)
+    kc[:, past + T:], vc[:, past + T:] = np.nan, np.nan                     # cells never written
+    qkv = rng.standard_normal((T, d + 2 * gqa)).astype(np.float32)
+    if spoil is not None:
+        qkv[spoil, d + gqa:] = np.inf
+    pos = np.arange(past, past + T, dtype=np.int32)
+    dq, dpos, dk, dv = pl.DevBuf(host=qkv), pl.DevBuf(host=pos), pl.DevBuf(host=kc), pl.DevBuf(host=vc)
+    rot, out, out16 = pl.DevBuf(T * d * 4), pl.DevBuf(T * d * 4), pl.DevBuf(T * d * 2)
+    pl.check(L.pi_memset(out.ptr, 0xFF, out.nbytes), "memset")
+    theta = float(np.float32(10000.0) ** np.float32(-2.0 / hd))
+    print("rows", hd, nh, nkv, mode, past, T, flush=True)
+    pl.check(L.pi_k_attn_chunk(dq.ptr, d + 2 * gqa, T, nh, nkv, hd, mode, theta, 1.0, dpos.ptr, n_ctx, past + T, rot.ptr, dk.ptr, dv.ptr, out.ptr, d, out16.ptr, None), "attn_chunk")
+    pl.sync()
+    got = out.download(np.float32).reshape(T, nh, hd)
+    with np.errstate(invalid="ignore", over="ignore"):
+        assert np.array_equal(out16.download(np.float16).reshape(T, nh, hd), got.astype(np.float16), equal_nan=True)
+    k, v = dk.download(np.float16).reshape(nkv, n_ctx, hd).astype(np.float64), dv.download(np.float16).reshape(nkv, n_ctx, hd).astype(np.float64)
+    want_k = rotated(qkv[:, d:d + gqa].reshape(T, nkv, hd), pos, mode, hd).transpose(1, 0, 2)
+    assert np.abs(k[:, past:past + T] - want_k).max() < 4e-3 * np.abs(want_k).max()               # rounded to fp16
+    assert np.array_equal(v[:, past:past + T], qkv[:, d + gqa:].reshape(T, nkv, hd).transpose(1, 0, 2).astype(np.float16).astype(np.float64), equal_nan=True)
+    q = rotated(qkv[:, :d].reshape(T, nh, hd), pos, mode, hd).astype(np.float16).astype(np.float64)
+    heads = range(nh) if nh <= 8 else sorted(set(rng.integers(0, nh, 6)) | {0, nh - 1})
+    seen = np.arange(past + T)[None] <= pos[:, None]
+    want = {}
+    for a in heads:
+        g = a * nkv // nh
+        s = np.where(seen, q[:, a] @ k[g, :past + T].T / np.sqrt(hd), -np.inf)
+        e = np.exp(s - s.max(1, keepdims=True))
+        e /= e.sum(1, keepdims=True)
+        want[a] = e @ (v[g, :past + T] if spoil is None else np.where(np.isfinite(v[g, :past + T]), v[g, :past + T], 0))
+    return got, want
+
+
+# fp16(s - max) is off by up to 2^-10 for |s - max| in [2, 4) and the weight by as much of itself, 6e-4 in the root mean square of a row
+@pytest.mark.parametrize("hd,nh,nkv,mode,past,T,n_ctx", [
+    (128, 4, 4, 0, 0, 32, 64), (128, 4, 4, 0, 0, 63, 64), (128, 4, 4, 0, 1, 64, 96), (128, 4, 2, 0, 63, 65, 160), (64, 8, 2, 2, 0, 127, 160), (64, 4, 4, 0, 64, 128, 192),
+    (64, 8, 1, 2, 5, 129, 160), (128, 2, 2, 2, 1900, 90, 2400), (128, 2, 1, 0, 0, 512, 512), (64, 256, 8, 2, 30, 129, 160), (128, 256, 8, 0, 3, 190, 224)])
+def test_rows_match_float64(hd, nh, nkv, mode, past, T, n_ctx):
+    got, want = run(hd, nh, nkv, mode, past, T, n_ctx)
+    for a, w in want.items():
+        err = np.linalg.norm(got[:, a] - w) / np.linalg.norm(w)
+        assert err < 2e-3, (a, err)
+
+
+@pytest.mark.parametrize("hd,T,spoil", [(128, 70, 40), (64, 150, 149), (128, 40, 0)])
+def test_a_value_that_is_no_number_reaches_the_tokens_that_see_it_only(hd, T, spoil):
+    got, want = run(hd, 2, 2, 0, 10, T, 192, spoil=spoil)
+    for a, w in want.items():
+        assert np.isfinite(got[:spoil, a]).all() and not np.isfinite(got[spoil:, a]).any()
+        if spoil:
+            assert np.linalg.norm(got[:spoil, a] - w[:spoil]) / np.linalg.norm(w[:spoil]) < 2e-3
