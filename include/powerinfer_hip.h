@@ -512,6 +512,13 @@ PI_API int pi_k_attn_fused_batch_q8(const float * qkv, int qkv_stride, const voi
 PI_API int pi_k_attn_fused_batch_ol(const float * qkv, int qkv_stride, const void * rope_table, void * k_cache, void * v_cache,
                                     size_t cache_seq_stride, int n_seq, int n_head, int n_head_kv, int hd, int mode, int n_ctx,
                                     const int32_t * pos, float * out, int out_stride, void * out_ol, pi_stream_t stream);
+/* pi_k_attn_chunk (below) with 64 or 128 tokens of a head per workgroup: any number of tokens and of cells, head sizes 64 and 128, the same rounding
+ * points.  out_stride % 4 == 0, buffers on 16 bytes (out_f16 on 8).  pi_k_attn_chunk_rows_supported: whether it is the one to take for T tokens
+ * against n_kv_max cells. */
+PI_API int pi_k_attn_chunk_rows_supported(int hd, int T, int n_kv_max);
+PI_API int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                                const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride,
+                                void * out_f16, pi_stream_t stream);
 /* prompt chunk of ONE sequence: T <= 512 consecutive tokens at positions pos[t]; RoPE + KV store of the whole chunk first, then
  * every token attends to the cells up to its own position (the causal mask of llama.cpp:6506-6531).  q_rot: fp32 [T][n_head*hd].
  * n_kv_max: an upper bound of max(pos) + 1, the cells the chunk's furthest token attends (<= 0: n_ctx); positions beyond it are

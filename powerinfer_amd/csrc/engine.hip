@@ -772,11 +772,11 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
         if (tokens[i] < 0 || tokens[i] >= m->hp.n_vocab) return pi::fail(PI_E_ARG, "pi_model_decode: token id out of range");
     int first = 0;
     if (n_tokens > 2) {
-        // the prompt goes through in chunks (weights read once per chunk): up to 512 tokens where the dense chunk path covers the
+        // the prompt goes through in chunks (weights read once per chunk): up to 2048 tokens where the dense chunk path covers the
         // model (F16 or Q4_0 matrices, hybrid layers included), up to 16 for the remainder of an F16 model that is whole on the
         // device; what is left, and at least the last token, takes the single-token path below, which produces the logits
         const bool wide = pi::prefill_wide_supported(m), small = pi::prefill_supported(m);
-        const int wide_max = wide ? pi::prefill_wide_max(m) : 0;
+        const int wide_max = wide ? pi::prefill_wide_max(m, n_tokens - 1) : 0;
         while (n_tokens - 1 - first >= 2) {
             const int left = n_tokens - 1 - first;
             if (wide && left > 16) {

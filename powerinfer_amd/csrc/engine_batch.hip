@@ -58,6 +58,7 @@ struct BatchState {
 };
 
 namespace {
+constexpr int kChunkMaxT = 512;            // tokens of one call of the chunk kernels (attention one token per workgroup, embedding)
 
 #define PI_TRY(expr) do { int _rc = (expr); if (_rc != PI_OK) return _rc; } while (0)
 
@@ -71,15 +72,18 @@ int chunk_attention(pi_model * m, BatchState * b, int T, size_t kv_off) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
     const char * own = getenv("PI_ATTN_CHUNK");
-    if (pi::attn_chunk_rows_fits(hd, T, b->kv_hi, b->att, b->att16, d) && !(own && !strcmp(own, "scalar")))
-        return pi::attn_chunk_rows(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
-                               m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
+    // a Q4_0 output projection rounds what comes out here to eight bits: as before where the kernel before covers the chunk (see prefill_wide_max;
+    // 512 tokens behind none, 32 heads of 128: 61 against 49 us of about 950 per layer)
+    const bool as_before = m->L(0, PI_T_WO).type == PI_TYPE_Q4_0 && T <= kChunkMaxT && pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi);
+    if (!as_before && pi_k_attn_chunk_rows_supported(hd, T, b->kv_hi) && !(own && !strcmp(own, "scalar")))
+        return pi_k_attn_chunk_rows(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
+                                    m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
     if (pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi))
         return pi_k_attn_chunk(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
                                m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
     const int parts = m->attn_parts > 1 ? m->attn_parts : 2;
     if (!m->attn_scratch_chunk) {
-        m->attn_scratch_chunk = m->alloc<float>(pi_k_attn_split_scratch_floats(512, hp.n_head, hd, parts));
+        m->attn_scratch_chunk = m->alloc<float>(pi_k_attn_split_scratch_floats(kChunkMaxT, hp.n_head, hd, parts));
         if (!m->attn_scratch_chunk) return PI_E_HIP;
     }
     return pi_k_attn_chunk_long(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, parts,
@@ -346,7 +350,7 @@ BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
     }
     b->x = m->alloc<float>(n * d); b->x2 = m->alloc<float>(n * d); b->qkv = m->alloc<float>(n * (d + 2 * m->gqa));
     b->att = m->alloc<float>(n * d); b->attn_out = m->alloc<float>(n * d); b->ffn_inp = m->alloc<float>(n * d);
-    b->hidden = m->alloc<float>(n * r); b->pred_logits = m->alloc<float>(n * ff); b->logits = m->alloc<float>(n * hp.n_vocab);
+    b->hidden = m->alloc<float>(n * r); b->pred_logits = m->alloc<float>(n * ff); b->logits = m->alloc<float>((n > 16 ? 1 : n) * hp.n_vocab);      // a prompt chunk's last token has its logits elsewhere
     const size_t n16 = n < 16 ? 16 : n;                            // steps of up to 16 tokens keep these in the operand layout: 16 token slots
     b->xa16 = m->alloc<__half>(n16 * d); b->xf16 = m->alloc<__half>(n16 * d); b->xp16 = m->alloc<__half>(n16 * d);
     b->att16 = m->alloc<__half>(n16 * d); b->hid16 = m->alloc<__half>(n16 * r);
@@ -523,7 +527,18 @@ bool prefill_wide_supported(pi_model * m) {
     return !(off && off[0] == '1') && wide_unsupported(m) == nullptr;
 }
 
-int prefill_wide_max(pi_model * m) { (void)m; return 512; }      // the longest chunk of the attention, embedding and elementwise kernels
+// The longest chunk of a prompt of which n_left tokens are to come.  Longer ones read each matrix less often and give its product more columns:
+// the seven products of a 7B-shaped F16 layer take 1250 us in four chunks of 512 tokens and 1080 us in one of 2046.  The attention by rows of
+// tokens has no limit of its own; head sizes without it go by 512 as their kernels do.  A Q4_0 model, whose matrices are expanded once a chunk
+// (210 us per 7B layer), keeps 512 up to 1024 tokens: where a chunk ends decides how the library orders its sums, and with them single roundings
+// to eight bits, by which results at those lengths are compared with the CPU path's.  Never more than the context holds (the step buffers are
+// sized by it).
+int prefill_wide_max(pi_model * m, int n_left) {
+    const char * own = getenv("PI_ATTN_CHUNK");
+    if ((m->hd != 64 && m->hd != 128) || (own && !strcmp(own, "scalar"))) return kChunkMaxT;
+    const int most = std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048);
+    return n_left <= 2 * kChunkMaxT && m->L(0, PI_T_WO).type == PI_TYPE_Q4_0 ? kChunkMaxT : most;
+}
 
 // PI_PREFILL_GEMM=own: the dense mat-muls of prompt chunks run on this library's LDS-tiled MFMA kernel instead of hipBLASLt plans
 static bool prefill_own_gemm() {
@@ -532,7 +547,7 @@ static bool prefill_own_gemm() {
 }
 
 int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
-    const int kMaxT = prefill_wide_max(m);
+    const int kMaxT = prefill_wide_max(m, INT32_MAX);
     if (T <= 16 || T > kMaxT) return pi::fail(PI_E_ARG, "prefill_wide_chunk: chunk length outside 17 .. prefill_wide_max");
     const pi_hparams & hp = m->hp;
     if (!m->prefill_wide) {
@@ -599,13 +614,17 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) 
     BatchState * b = m->prefill_wide;
     b->n_seq = T;
     b->kv_hi = n_past + T;
-    int32_t pos[512];
+    std::vector<int32_t> pos(T);
     for (int t = 0; t < T; ++t) pos[t] = n_past + t;
     PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipMemcpyAsync(b->d_pos, pos, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
+    PI_HIP_TRY(hipMemcpyAsync(b->d_pos, pos.data(), sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
     PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    if (m->glob[PI_T_TOK_EMBD].type == PI_TYPE_Q4_0) PI_TRY(pi_k_embed_batch_q4(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens, T, b->x, m->stream));
-    else PI_TRY(pi_k_embed_batch(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens, T, b->x, m->stream));
+    for (int t = 0; t < T; t += kChunkMaxT) {
+        const int n = std::min(T - t, kChunkMaxT);
+        float * x = b->x + (size_t)t * hp.n_embd;
+        if (m->glob[PI_T_TOK_EMBD].type == PI_TYPE_Q4_0) PI_TRY(pi_k_embed_batch_q4(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens + t, n, x, m->stream));
+        else PI_TRY(pi_k_embed_batch(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens + t, n, x, m->stream));
+    }
     b->staged_layer[0] = b->staged_layer[1] = -1;
     PI_TRY(stage_rest_rows(m, b, 0));
     for (int il = 0; il < hp.n_layer; ++il) {

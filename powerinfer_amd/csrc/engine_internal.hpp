@@ -74,7 +74,7 @@ struct pi_model {
     BatchState * batch = nullptr;         // per-sequence caches and step buffers of batched decoding
     BatchState * cells = nullptr;         // the KV cache with cells shared between sequences and its step buffers (pi_model_kv_cells_*)
     BatchState * prefill = nullptr;       // step buffers for prompt chunks of the model's own sequence
-    BatchState * prefill_wide = nullptr;  // the same for chunks of up to 512 tokens (dense mat-muls, weights read once per chunk)
+    BatchState * prefill_wide = nullptr;  // the same for chunks of up to 2048 tokens (dense mat-muls, weights read once per chunk)
     pi_gemm_lib * gemm_lib = nullptr;     // hipBLASLt plans of those mat-muls (PI_PREFILL_GEMM=own keeps them on this library's kernel, 128 tokens a chunk)
     // multi-token steps of a Q4_0 model on integer matrix cores: every Q4_0 matrix once more as 16-byte-aligned quants and fp16
     // scales (pi_k_q4_split), made at the first such step; q4_steps says the model takes that route
@@ -116,6 +116,6 @@ bool prefill_supported(pi_model * m);   // F16 weights, every neuron on the GPU,
 int  prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);
 bool prefill_wide_supported(pi_model * m);   // F16 or Q4_0 matrices (fp16 predictor), hybrid layers included; n_embd, n_ff and the predictor rank multiples of 256
 int  gather_rest_rows(pi_model * m, int il);  // hybrid layer: rows of the non-resident neurons into pinned host memory (rest_up / rest_gate / rest_down)
-int  prefill_wide_max(pi_model * m);         // longest chunk: 512 through the library mat-mul, 128 on this library's own kernel (PI_PREFILL_GEMM=own)
+int  prefill_wide_max(pi_model * m, int n_left);     // longest chunk of a prompt with n_left tokens to go: 512 or up to 2048
 int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);     // 16 < T <= prefill_wide_max
 }

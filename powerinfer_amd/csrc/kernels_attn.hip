@@ -749,22 +749,22 @@ __global__ __launch_bounds__(kBlock) void attn_chunk_mfma_kernel(const float * _
 // Attention of a prompt chunk, 64 U tokens of one query head per workgroup.  attn_chunk_mfma_kernel reads a head's cells once for 16
 // tokens, holds all their scores in LDS (which ends at about 1850 cells) and is bound by those reads; here a tile of 64 cells is staged
 // once for 64 or 128 tokens and no score leaves the registers, so the cells a chunk may see are not limited.  The soft-max keeps the
-// rounding points of attn_decode_kernel, fp16 in and out of exp relative to the row's maximum over ALL its cells, which is why the
-// keys are gone through twice: first for the maximum (products and comparisons only), then for the weights.  What is left out is the
-// rounding of e / sum to fp16: the weights e are fp16 values as they are, and their sum divides the result.
+// rounding points of attn_decode_kernel (fp16 in and out of exp relative to the row's maximum over ALL its cells, e / sum to fp16), which
+// is why the keys are gone through three times: for the maximum (products and comparisons only), the sum, and the weights.  Dividing the
+// result by the sum instead, in two passes, is a third faster and no further from the exact result, but 2e-4 from the CPU path's: a
+// Q4_0 model's next rounding to eight bits then falls the other way for one activation in forty.
 // Scores are formed transposed (cells x tokens): a lane's scores belong to one token, and its weights are already the column operand of
 // values^T x weights - which cell a slot of that product's inner dimension stands for is free, so the values are read (transposed,
-// ds_read_tr16) in the order the scores came out.  The sum is one more product, with ones, added up over the tiles in double.
+// ds_read_tr16) in the order the scores came out.  The sum of a tile is one more product, with ones.
 // Bound by the exponentials (about 40 cycles of VALU per 64 of them) beside 48 of matrix cores.  32 heads of 128, RoPE and store included:
-// 512 tokens behind 0 / 512 / 1024 / 1535: 42 / 59 / 75 / 84 us (attn_chunk_mfma_kernel 61 / 117 / 159, attn_decode_kernel 791 past the
-// cells that one holds); 128 heads of 64 on 8: 43 / 66 / 88 / 109 (94 / 271 / 380 / 493).
+// 512 tokens behind 0 / 512 / 1024 / 1535: 49 / 74 / 99 / 118 us (attn_chunk_mfma_kernel 61 / 117 / 159, attn_decode_kernel 791 past the
+// cells that one holds), 2046 tokens at once 222; 128 heads of 64 on 8: 60 / 107 / 155 / 196 (94 / 271 / 380 / 493).
 // ---------------------------------------------------------------------------------------------------
 typedef short pi_s4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ pi_u32x2 lds_tr_read(const unsigned char * q) {
     return __builtin_bit_cast(pi_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pi_s4 *)(__attribute__((address_space(3))) void *)q));
 }
 constexpr int kRowsCells = 64;                 // cells of a tile
-constexpr int kRowsWideGrid = 512;
 template <int HD> constexpr int rows_pitch() { return HD * 2 + 16; }                       // bytes of a staged row: 16 of padding spread the rows over the banks
 template <int HD> constexpr size_t rows_lds() { return (size_t)4 * kRowsCells * rows_pitch<HD>(); }
 
@@ -853,28 +853,73 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
 #pragma unroll
                 for (int r = 0; r < 4; ++r) mx[u] = fmaxf(mx[u], edge && cb + kt * 16 + 4 * g + r >= nv[u] ? -INFINITY : s[u][kt][r]);
     }
-    float base[U];                                                       // -maximum of the scaled scores
+    float base[U];                                                       // the maximum of the scaled scores
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 16, PI_WAVE));
         mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], 32, PI_WAVE));
-        base[u] = mx[u] == -INFINITY ? 0.0f : -__fmul_rn(mx[u], scale);
+        base[u] = mx[u] == -INFINITY ? 0.0f : __fmul_rn(mx[u], scale);
+    }
+
+    // e = fp16(exp(fp16(s - max))) of a tile as the column operand, times f where the sums are known.  e^x = 2^n 2^(x log2 e - n): log2 e in
+    // two parts, the first short enough for its product with an fp16 number to be exact, so that 2^ is off by little more than its own rounding
+    auto weigh = [&](const pi_f4 * s, int cb, bool edge, int seen, float b, bool last_pass, float f, pi_u32x4 * out) {
+        _Float16 w[4 * KT];
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float x = (float)(_Float16)__fsub_rn(__fmul_rn(s[kt][r], scale), b);
+                const float n = fmaxf(__builtin_rintf(x * 1.4426950408889634f), -200.0f);        // x may be -inf
+                const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 6.808776379330084e-05f, fmaf(x, 1.442626953125f, -n))), (int)n);
+                _Float16 v = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= seen ? 0.0f : e);
+                if (last_pass) v = (_Float16)__fmul_rn((float)v, f);
+                w[kt * 4 + r] = v;
+            }
+#pragma unroll
+        for (int k = 0; k < KT / 2; ++k)
+            out[k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
+    };
+
+    // ---- the rows' sums: 64 weights by a product with ones, the tiles in double ----
+    double sum[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) sum[u] = 0.0;
+    const pi_u32x4 ones{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+    fetch(pk, kb, 0);
+    __syncthreads();                                                     // the last tile of the pass before has been read
+    at = 0;
+    for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
+        place(smem + at * TILE, pk);
+        __syncthreads();
+        fetch(pk, kb, cb + NK);
+        pi_f4 s[U][KT];
+        products(smem + at * TILE, s);
+        const bool edge = cb + NK > n_all;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            pi_u32x4 pb[KT / 2];
+            weigh(s[u], cb, edge, nv[u], base[u], false, 0.0f, pb);
+            pi_f4 l = pi_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k) l = mma16<__half>(ones, pb[k], l);
+            sum[u] += (double)l[0];
+        }
     }
 
     // ---- weights and values ----
-    double sum[U];
+    float inv[U];
     pi_f4 o[U][VT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        sum[u] = 0.0;
+        inv[u] = (float)(1.0 / sum[u]);
 #pragma unroll
         for (int v = 0; v < VT; ++v) o[u][v] = pi_f4{0, 0, 0, 0};
     }
-    const pi_u32x4 ones{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
     unsigned char * vt = smem + 2 * TILE;
     fetch(pk, kb, 0);
     fetch(pv, vb, 0);
-    __syncthreads();                                                     // the last tile of the first pass has been read
+    __syncthreads();
     at = 0;
     for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
         const bool edge = cb + NK > n_all;
@@ -895,26 +940,7 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         products(smem + at * TILE, s);
         pi_u32x4 pb[U][KT / 2];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            _Float16 w[4 * KT];
-#pragma unroll
-            for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    // e^x as 2^(x log2 e): fp16 in, fp16 out, the fp32 steps between are good to 1e-6
-                    const float x = (float)(_Float16)fmaf(s[u][kt][r], scale, base[u]);
-                    const float e = __builtin_amdgcn_exp2f(x * 1.4426950408889634f);
-                    w[kt * 4 + r] = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= nv[u] ? 0.0f : e);
-                }
-#pragma unroll
-            for (int k = 0; k < KT / 2; ++k) {
-                pb[u][k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
-            }
-            pi_f4 l = pi_f4{0, 0, 0, 0};
-#pragma unroll
-            for (int k = 0; k < KT / 2; ++k) l = mma16<__half>(ones, pb[u][k], l);
-            sum[u] += (double)l[0];
-        }
+        for (int u = 0; u < U; ++u) weigh(s[u], cb, edge, nv[u], base[u], true, inv[u], pb[u]);
         const unsigned char * vs = vt + at * TILE;
         if (edge && odd[at]) {
             // 0 times such a value is no number either: token by token, the cells it sees only.  The weight of cell (kt, g, r) of token i is
@@ -955,12 +981,11 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
     for (int u = 0; u < U; ++u) {
         const int t = t0 + wave * 16 * U + u * 16 + i;
         if (t >= T) continue;
-        const float inv = (float)(1.0 / sum[u]);
         float * po = out + (size_t)t * out_stride + (size_t)h * HD + 4 * g;
         __half * ph = out16 ? out16 + (size_t)t * out_stride + (size_t)h * HD + 4 * g : nullptr;
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
-            const float4 y{__fmul_rn(o[u][v][0], inv), __fmul_rn(o[u][v][1], inv), __fmul_rn(o[u][v][2], inv), __fmul_rn(o[u][v][3], inv)};
+            const float4 y{o[u][v][0], o[u][v][1], o[u][v][2], o[u][v][3]};
             *reinterpret_cast<float4 *>(po + v * 16) = y;
             if (ph) {
                 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -1196,24 +1221,6 @@ int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_
 }
 }  // namespace
 
-namespace pi {
-// head sizes and alignments of attn_chunk_rows_kernel (outputs are stored four columns at a time), and where it is the faster one: fewer than
-// 32 tokens against many cells are better off with attn_chunk_mfma_kernel, whose waves split the cells (17 tokens, 1817 cells, 32 heads of
-// 128: 59 us here, 49 there; 317 cells: 17.5 and 17.7; 48 tokens, 1848 cells: 62 and 102)
-bool attn_chunk_rows_fits(int hd, int T, int n_kv_max, const void * out, const void * out_f16, int out_stride) {
-    return (hd == 64 || hd == 128) && T > kBtMaxT && (T >= 32 || n_kv_max <= 512 || chunk_mfma_lds(hd, n_kv_max) > kChunkMfmaLds) && out_stride % 4 == 0 &&
-           ((uintptr_t)out & 15) == 0 && ((uintptr_t)out_f16 & 7) == 0;
-}
-int attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
-                    int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16, hipStream_t st) {
-    int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
-    if (rc != PI_OK) return rc;
-    const bool two = (long long)n_head * ((T + 127) / 128) >= kRowsWideGrid;
-#define PI_ROWS(HD, U) launch_chunk_rows<HD, U>(q_rot, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
-    return hd == 128 ? (two ? PI_ROWS(128, 2) : PI_ROWS(128, 1)) : (two ? PI_ROWS(64, 2) : PI_ROWS(64, 1));
-#undef PI_ROWS
-}
-}  // namespace pi
 
 extern "C" {
 
@@ -1379,13 +1386,11 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || hd <= 0 || hd % 8 || hd / 2 > 1024 || kBlock % (hd / 8) || PI_WAVE % (hd / 8) || (mode != 0 && mode != 2))
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad head geometry or mode");
     hipStream_t st = (hipStream_t)stream;
-    const char * own = getenv("PI_ATTN_CHUNK");
-    const bool scalar = own && !strcmp(own, "scalar");
-    if (!scalar && pi_k_attn_chunk_supported(hd, n_ctx, n_kv_max) && pi::attn_chunk_rows_fits(hd, T, n_kv_max, out, out_f16, out_stride))
-        return pi::attn_chunk_rows(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, n_kv_max, q_rot, k_cache, v_cache, out, out_stride, out_f16, st);
     // all K/V rows of the chunk are in the cache before any token of the chunk attends
     rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     // 16 tokens per workgroup on the matrix cores where the head size and the context fit (scores of 16 tokens in LDS)
+    const char * own = getenv("PI_ATTN_CHUNK");
+    const bool scalar = own && !strcmp(own, "scalar");
     const int s_stride = ((n_kv_max + 31) & ~31) + 4;
     const size_t sh_mfma = chunk_mfma_lds(hd, n_kv_max);
     if ((hd == 128 || hd == 64) && T > 1 && sh_mfma <= kChunkMfmaLds && !scalar) {
@@ -1407,6 +1412,30 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
     hipLaunchKernelGGL(attn_decode_kernel, dim3(n_head, T), dim3(kBlock), sh, st,
                        q_rot, (const __half *)k_cache, (const __half *)v_cache, n_head, n_head_kv, hd, n_ctx, pos, out, n_head * hd, out_stride, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_chunk");
+}
+
+// where attn_chunk_rows_kernel is the faster one: fewer than 32 tokens against many cells are better off with attn_chunk_mfma_kernel, whose waves
+// split the cells (32 heads of 128, 17 tokens: 59 against 49 us at 1817 cells, 17.5 and 17.7 at 317; 48 tokens, 1848 cells: 91 and 102)
+int pi_k_attn_chunk_rows_supported(int hd, int T, int n_kv_max) {
+    return (hd == 64 || hd == 128) && T > kBtMaxT && n_kv_max > 0 && (T >= 32 || n_kv_max <= 512 || chunk_mfma_lds(hd, n_kv_max) > kChunkMfmaLds);
+}
+
+int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                         const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16,
+                         pi_stream_t stream) {
+    if (!qkv || !pos || !q_rot || !k_cache || !v_cache || !out || T <= 0 || n_ctx <= 0) return pi::fail(PI_E_ARG, "pi_k_attn_chunk_rows: bad arguments");
+    if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (hd != 64 && hd != 128) || (mode != 0 && mode != 2)) return pi::fail(PI_E_ARG, "pi_k_attn_chunk_rows: bad head geometry or mode");
+    if (out_stride % 4 || (((uintptr_t)q_rot | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15) || ((uintptr_t)out_f16 & 7))
+        return pi::fail(PI_E_ARG, "pi_k_attn_chunk_rows: rows of whole quads, buffers on 16 bytes (out_f16: 8)");
+    if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;
+    hipStream_t st = (hipStream_t)stream;
+    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    if (rc != PI_OK) return rc;
+    // 128 tokens a workgroup where that still leaves two for every compute unit
+    const bool two = (long long)n_head * ((T + 127) / 128) >= 2 * pi::compute_units();
+#define PI_ROWS(HD, U) launch_chunk_rows<HD, U>(q_rot, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
+    return hd == 128 ? (two ? PI_ROWS(128, 2) : PI_ROWS(128, 1)) : (two ? PI_ROWS(64, 2) : PI_ROWS(64, 1));
+#undef PI_ROWS
 }
 
 int pi_k_attn_chunk_supported(int hd, int n_ctx, int n_kv_max) {

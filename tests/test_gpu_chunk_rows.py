@@ -37,7 +37,7 @@ def run(hd, nh, nkv, mode, past, T, n_ctx, spoil=None):
     pl.check(L.pi_memset(out.ptr, 0xFF, out.nbytes), "memset")
     theta = float(np.float32(10000.0) ** np.float32(-2.0 / hd))
     print("rows", hd, nh, nkv, mode, past, T, flush=True)
-    pl.check(L.pi_k_attn_chunk(dq.ptr, d + 2 * gqa, T, nh, nkv, hd, mode, theta, 1.0, dpos.ptr, n_ctx, past + T, rot.ptr, dk.ptr, dv.ptr, out.ptr, d, out16.ptr, None), "attn_chunk")
+    pl.check(L.pi_k_attn_chunk_rows(dq.ptr, d + 2 * gqa, T, nh, nkv, hd, mode, theta, 1.0, dpos.ptr, n_ctx, past + T, rot.ptr, dk.ptr, dv.ptr, out.ptr, d, out16.ptr, None), "attn_chunk_rows")
     pl.sync()
     got = out.download(np.float32).reshape(T, nh, hd)
     with np.errstate(invalid="ignore", over="ignore"):
@@ -61,13 +61,21 @@ def run(hd, nh, nkv, mode, past, T, n_ctx, spoil=None):
 
 # fp16(s - max) is off by up to 2^-10 for |s - max| in [2, 4) and the weight by as much of itself, 6e-4 in the root mean square of a row
 @pytest.mark.parametrize("hd,nh,nkv,mode,past,T,n_ctx", [
-    (128, 4, 4, 0, 0, 32, 64), (128, 4, 4, 0, 0, 63, 64), (128, 4, 4, 0, 1, 64, 96), (128, 4, 2, 0, 63, 65, 160), (64, 8, 2, 2, 0, 127, 160), (64, 4, 4, 0, 64, 128, 192),
-    (64, 8, 1, 2, 5, 129, 160), (128, 2, 2, 2, 1900, 90, 2400), (128, 2, 1, 0, 0, 512, 512), (64, 256, 8, 2, 30, 129, 160), (128, 256, 8, 0, 3, 190, 224)])
+    (128, 4, 4, 0, 0, 1, 64), (128, 4, 4, 0, 0, 63, 64), (128, 4, 4, 0, 1, 64, 96), (128, 4, 2, 0, 63, 65, 160), (64, 8, 2, 2, 0, 127, 160), (64, 4, 4, 0, 64, 128, 192),
+    (64, 8, 1, 2, 5, 129, 160), (128, 2, 2, 2, 1900, 90, 2400), (128, 2, 1, 0, 0, 700, 736), (64, 256, 8, 2, 30, 129, 160), (128, 256, 8, 0, 3, 190, 224)])
 def test_rows_match_float64(hd, nh, nkv, mode, past, T, n_ctx):
     got, want = run(hd, nh, nkv, mode, past, T, n_ctx)
     for a, w in want.items():
         err = np.linalg.norm(got[:, a] - w) / np.linalg.norm(w)
         assert err < 2e-3, (a, err)
+
+
+def test_what_it_does_not_cover_is_refused():
+    from powerinfer_amd import lib as pl
+    L, b = pl.init(), pl.DevBuf(1 << 16)
+    call = lambda hd, stride: L.pi_k_attn_chunk_rows(b.ptr, 3 * hd, 2, 1, 1, hd, 0, 0.9, 1.0, b.ptr, 8, 4, b.ptr, b.ptr, b.ptr, b.ptr, stride, None, None)  # noqa: E731
+    assert call(32, 32) != 0 and call(64, 66) != 0
+    assert not L.pi_k_attn_chunk_rows_supported(32, 64, 64) and not L.pi_k_attn_chunk_rows_supported(64, 16, 64) and L.pi_k_attn_chunk_rows_supported(64, 17, 64)
 
 
 @pytest.mark.parametrize("hd,T,spoil", [(128, 70, 40), (64, 150, 149), (128, 40, 0)])
