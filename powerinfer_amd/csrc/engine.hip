@@ -131,6 +131,18 @@ pi_norm make_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
 #define PI_TRY(expr) do { int _rc = (expr); if (_rc != PI_OK) return _rc; } while (0)
 
 // ---- one layer, everything on the GPU --------------------------------------------------------------
+// Adds a matrix's leading rows, at most `bytes` of them and in units of rows_per_unit, to what a launch requests ahead; returns the bytes left.
+// Units of a size or an address that 16-byte loads cannot take whole are left to the launch that needs them.
+size_t ahead_rows(pi::Ahead & a, const Tensor & t, int rows_per_unit, int slot, size_t bytes) {
+    if (!t.dev || (t.type != PI_TYPE_F16 && t.type != PI_TYPE_Q4_0)) return bytes;
+    const size_t row = t.type == PI_TYPE_F16 ? (size_t)t.ne0 * 2 : (size_t)t.ne0 / 32 * 18, unit = row * rows_per_unit;
+    if (!unit || unit % 16 || unit > bytes || ((uintptr_t)t.dev & 15)) return bytes;
+    size_t n = (size_t)t.ne1 / rows_per_unit;
+    if (n > bytes / unit) n = bytes / unit;
+    a.p[slot] = t.dev; a.units[slot] = (int)n; a.unit_bytes[slot] = (int)unit;
+    return bytes - n * unit;
+}
+
 int layer_forward(pi_model * m, int il, bool last_token) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, ff = hp.n_ff, hd = m->hd, gqa = m->gqa;
@@ -163,6 +175,17 @@ int layer_forward(pi_model * m, int il, bool last_token) {
                                                nullptr, nullptr, m->ws, m->stream2));
     }
 
+    // Attention of one token leaves HBM idle for the 8 us it takes at a few hundred cells, so its launch asks for the matrices behind it, wo and fc1,
+    // up to the 32 MB that HBM gives in that time (more makes the launch longer: 40 MB with 96 workgroups 490 us a token, 32 MB 479).  128
+    // workgroups: 8 layers of 32 F16 heads take 474 us a token, 64 take 500, 96 479, 192 477, none 509; Q4_0 split 289 -> 277 us.
+    // Not where Falcon's FFN runs beside the attention: HBM is not idle there (40B widths: 601 us with and without).
+    pi::Ahead ahead;
+    if (!branch) {
+        const size_t left = ahead_rows(ahead, wo, 4, 0, (size_t)32 << 20);
+        ahead_rows(ahead, fc1, 4, 1, left);
+        ahead.blocks = 128;
+    }
+
     // attention
     pi_norm an;
     if (!falcon) an = make_norm(1, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), nullptr);
@@ -173,8 +196,8 @@ int layer_forward(pi_model * m, int il, bool last_token) {
         PI_TRY(pi_k_attn_split(m->qkv, 0, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, 0, 1, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0,
                                hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, 0, nullptr, st));
     } else if (m->rope_table) {
-        PI_TRY(pi_k_attn_fused(m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0,
-                               hp.n_ctx, m->d_pos, m->att, st));
+        PI_TRY(pi::attn_fused(m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0,
+                              hp.n_ctx, m->d_pos, m->att, ahead, st));
     } else {
         PI_TRY(pi_k_rope_kv_store(m->qkv, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0, m->theta_scale, m->freq_scale, m->d_pos, hp.n_ctx,
                                   m->q_rot, m->k_cache + kv_off, m->v_cache + kv_off, st));

@@ -179,6 +179,7 @@ __global__ __launch_bounds__(kBlock) void attn_decode_kernel(const float * __res
 // own q head and the k head of its group (cos/sin from the table), rounds k and v to fp16 as the cache does,
 // and attends over cells [0, pos) from the cache plus the new cell from LDS, so it never reads what this
 // launch writes; the first query head of each group stores k and v.
+// Workgroups from n_head on (a single sequence only) request weights of later launches and take no part (load_ahead).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kAttnBlock = 1024;        // 16 waves per head: 64 (hd 128) or 128 (hd 64) cache cells per pass
 constexpr int kAttnPre = 4;             // passes whose K and V rows are requested before the prologue
@@ -192,7 +193,8 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
                                                             int n_head, int n_head_kv, int hd, int mode, int n_ctx,
                                                             const int32_t * __restrict__ pos_p, float * __restrict__ out,
                                                             int qkv_stride, size_t cache_seq_stride, int out_stride, __half * __restrict__ out16, int out16_ol,
-                                                            int8_t * __restrict__ q8_q, float * __restrict__ q8_d, int * __restrict__ q8_s) {
+                                                            int8_t * __restrict__ q8_q, float * __restrict__ q8_d, int * __restrict__ q8_s, Ahead ahead) {
+    if ((int)blockIdx.x >= n_head) { load_ahead(ahead, (int)blockIdx.x - n_head); return; }
     // q8_q != nullptr: the output also as the Q8_0 blocks an integer mat-mul of a Q4_0 matrix multiplies with (the blocks, scales and
     // -8 * sums pi_k_norm_q8_blocks makes of the same values: a head's hd outputs are whole blocks of 32, one per half-wave)
     // blockIdx.y = sequence of a batched step (its own token, position and cache); 0 for single-sequence decoding
@@ -1284,16 +1286,24 @@ int pi_k_attn_decode_supported(int hd, int n_ctx) {
            sizeof(float) * ((size_t)n_ctx + (size_t)(kBlock / (hd / 8)) * hd) <= kAttnLdsLimit;
 }
 
-int pi_k_attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
-                    int n_ctx, const int32_t * pos, float * out, pi_stream_t stream) {
+}  // extern "C"
+namespace pi {
+int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
+               int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream) {
     if (!qkv || !rope_table || !k_cache || !v_cache || !pos || !out) return pi::fail(PI_E_ARG, "pi_k_attn_fused: null pointer");
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || !attn_fused_geometry_ok(hd) || (mode != 0 && mode != 2))
         return pi::fail(PI_E_ARG, "pi_k_attn_fused: head size must be 8 * (a divisor of 64), at most 128; mode 0 or 2");
     const size_t sh = attn_fused_lds_bytes(hd, n_ctx);
     if (sh > kAttnLdsLimit) return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_fused: context too long for the single-pass kernel");
-    hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock>, dim3(n_head), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, 0, (size_t)0, 0, nullptr, 0, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock>, dim3(n_head + ahead.blocks), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
+                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, 0, (size_t)0, 0, nullptr, 0, nullptr, nullptr, nullptr, ahead);
     return pi::check_launch("pi_k_attn_fused");
+}
+}  // namespace pi
+extern "C" {
+int pi_k_attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
+                    int n_ctx, const int32_t * pos, float * out, pi_stream_t stream) {
+    return pi::attn_fused(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, pi::Ahead{}, stream);
 }
 
 // ---- attention with the cells of a head split over n_parts workgroups --------------------------------------------
@@ -1351,10 +1361,10 @@ static int attn_fused_batch(const float * qkv, int qkv_stride, const void * rope
     const int n_cu = pi::compute_units();
     if (n_cu > 0 && n_seq * n_head > 2 * n_cu)
         hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock / 2>, dim3(n_head, n_seq), dim3(kAttnBlock / 2), attn_fused_lds_bytes(hd, n_ctx, kAttnBlock / 2), (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s);
+                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{});
     else
         hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock>, dim3(n_head, n_seq), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s);
+                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{});
     return pi::check_launch("pi_k_attn_fused_batch");
 }
 

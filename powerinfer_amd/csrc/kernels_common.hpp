@@ -183,6 +183,26 @@ __device__ __forceinline__ float apply_epilogue(float v, int epi, const float * 
     return v;
 }
 
+// Decoding one token alternates between mat-vecs, which take what HBM gives, and launches that are a chain of latencies on a few compute units
+// (attention of one token) during which HBM idles.  Such a launch carries extra workgroups that request the weights of the mat-vecs behind
+// it, which then find them in the last-level cache or in the L2 of their XCD: workgroups go to the eight XCDs in turn and a mat-vec's
+// workgroup b starts with rows 4 b .. 4 b + 3, so unit u (four rows) is requested by a workgroup of XCD u % 8.  Two loads of 16 bytes in
+// flight a thread; four measured the same.  k: this workgroup's number among the extra ones.  Nothing is kept of what is read.
+// The same in the launches that add partial vectors (4.5 us, too short: 510 -> 535 us a token) and in fc1's mat-vec (586) lost time.
+using pi::Ahead;
+__device__ __forceinline__ void load_ahead(const Ahead & a, int k) {
+    const int x = blockIdx.x & 7, step = (int)blockDim.x * 16;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+        for (int u = x + 8 * (k >> 3); u < a.units[r]; u += a.blocks) {
+            const unsigned char * p = (const unsigned char *)a.p[r] + (size_t)u * a.unit_bytes[r];
+            for (int o = (int)threadIdx.x * 16; o < a.unit_bytes[r]; o += 2 * step) {
+                const pi_u32x4 v = pi_ld16(p + o), w = pi_ld16(p + min(o + step, a.unit_bytes[r] - 16));
+                asm volatile("" :: "v"(v), "v"(w));
+            }
+        }
+}
+
 // shapes and operand types the step kernels and their callers agree on
 typedef _Float16 pi_h8 __attribute__((ext_vector_type(8)));
 typedef __bf16   pi_b8 __attribute__((ext_vector_type(8)));
