@@ -991,16 +991,18 @@ int cold_post_token(ColdPath * c) {
     return PI_OK;
 }
 
+const uint32_t * cold_status(ColdPath * c) { return c->async ? c->d_status : nullptr; }
+
 // the stream has been synchronised: every posted layer has been answered, or something gave up
-int cold_drain(ColdPath * c) {
+int cold_drain(ColdPath * c, const uint32_t * fetched) {
     if (!c->async) return PI_OK;
     const auto t0 = std::chrono::steady_clock::now();
     while (c->served.load(std::memory_order_acquire) != c->posted.load() && !c->failed.load()) {
         relax();
         if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(30)) { c->failed.store(true); break; }
     }
-    uint32_t status = 0;
-    if (pi_memcpy_d2h(&status, c->d_status, 4) != PI_OK) return PI_E_HIP;
+    uint32_t status = fetched ? *fetched : 0;
+    if (!fetched && pi_memcpy_d2h(&status, c->d_status, 4) != PI_OK) return PI_E_HIP;
     if (status != 0 || c->failed.load()) return fail(PI_E_STATE, "cold path: a hand-over between the stream and the host threads timed out");
     return PI_OK;
 }

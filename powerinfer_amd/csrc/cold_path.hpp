@@ -33,7 +33,8 @@ int        cold_layer_f16(ColdPath * c, int il, pi_model * m, hipStream_t st, bo
 bool       cold_async(const ColdPath * c);
 bool       cold_every_layer_async(const ColdPath * c);   // no hybrid layer needs the launching thread: the token loop can be one graph
 int        cold_post_token(ColdPath * c);
-int        cold_drain(ColdPath * c);
+int        cold_drain(ColdPath * c, const uint32_t * status);          // status: the word behind cold_status, where the caller has fetched it already; null: read here
+const uint32_t * cold_status(ColdPath * c);                           // the hand-overs' status word on the device; null: none
 int        cold_layer_q4_queue(ColdPath * c, int il, pi_model * m, hipStream_t st);
 int        cold_layer_f16_queue(ColdPath * c, int il, pi_model * m, hipStream_t st);     // F16 layers at 4096 columns: one hand-over each way
 bool       cold_layer_async(const ColdPath * c, int il);

@@ -29,10 +29,6 @@ size_t row_bytes(int type, int64_t ne0) {
     }
 }
 
-__global__ void set_state_kernel(int32_t * token, int32_t * pos, int32_t t, int32_t p) {
-    if (threadIdx.x == 0) { *token = t; *pos = p; }
-}
-
 // greedy choice of the finished step + bookkeeping for the next one: the chosen token becomes the next
 // input, the position advances, the token and the step's total active-row count are logged
 __global__ __launch_bounds__(1024) void argmax_advance_kernel(const float * __restrict__ logits, int n, int32_t * token, int32_t * pos,
@@ -332,12 +328,15 @@ int layer_forward(pi_model * m, int il, bool last_token) {
 }
 
 // one token: embedding -> layers -> (final norm + lm-head + greedy)
-int token_forward(pi_model * m, bool want_logits, bool last_token) {
+// (token < 0: the one the device's state names; otherwise this one, at position pos)
+int token_forward(pi_model * m, bool want_logits, bool last_token, int32_t token = -1, int32_t pos = 0) {
     const pi_hparams & hp = m->hp;
     hipStream_t st = m->stream;
     // the host threads expect this token's hybrid layers (a graph under construction runs nothing: its replays are announced one by one)
     if (pi::cold_async(m->cold) && !m->capture && !m->building_graph) PI_TRY(pi::cold_post_token(m->cold));
-    PI_TRY(pi_k_embed(m->glob[PI_T_TOK_EMBD].type, m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, m->d_token, m->x, st));
+    const Tensor & table = m->glob[PI_T_TOK_EMBD];
+    if (token < 0) PI_TRY(pi_k_embed(table.type, table.dev, hp.n_embd, m->d_token, m->x, st));
+    else PI_TRY(pi::embed_start(table.type, table.dev, hp.n_embd, token, pos, m->d_token, m->d_pos, m->d_step, m->x, st));
     for (int il = 0; il < hp.n_layer; ++il) PI_TRY(layer_forward(m, il, last_token));
     if (want_logits) {
         const bool falcon = hp.arch == PI_ARCH_FALCON;
@@ -474,6 +473,7 @@ void pi_model_free(pi_model * m) {
     if (m->ws) pi_workspace_destroy(m->ws);
     for (void * p : m->owned) pi_free(p);
     for (void * p : m->pinned) (void)hipHostFree(p);
+    m->stage.release();
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -757,6 +757,7 @@ int pi_model_finalize(pi_model * m) {
         m->cold = pi::cold_create(m);
         if (!m->cold) return PI_E_STATE;
     }
+    m->stage.init(sizeof(float) * 16 * (size_t)hp.n_vocab);
     PI_HIP_TRY(hipDeviceSynchronize());
     m->finalized = true;
     return PI_OK;
@@ -817,18 +818,16 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
     }
     for (int i = first; i < n_tokens; ++i) {
         const bool last = i == n_tokens - 1;
-        hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, m->stream, m->d_token, m->d_pos, tokens[i], n_past + i);
-        PI_TRY(pi::check_launch("set_state"));
-        PI_TRY(token_forward(m, last, last));
+        PI_TRY(token_forward(m, last, last, tokens[i], n_past + i));
     }
     // greedy choice on the device; the state then points at the next position
-    PI_HIP_TRY(hipMemsetAsync(m->d_step, 0, 4, m->stream));
     PI_TRY(launch_advance(m));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    if (m->cold) PI_TRY(pi::cold_drain(m->cold));
     int32_t tok = -1;
-    PI_TRY(pi_memcpy_d2h(&tok, m->d_token, 4));
-    if (logits_out) PI_TRY(pi_memcpy_d2h(logits_out, m->logits, sizeof(float) * m->hp.n_vocab));
+    uint32_t status = 0;
+    const uint32_t * d_status = m->cold ? pi::cold_status(m->cold) : nullptr;
+    const pi::HostCopy results[] = {{m->d_token, &tok, 4}, {d_status, d_status ? &status : nullptr, 4}, {m->logits, logits_out, sizeof(float) * m->hp.n_vocab}};
+    PI_TRY(m->stage.fetch(results, 3, m->stream));
+    if (m->cold) PI_TRY(pi::cold_drain(m->cold, &status));
     return tok;
 }
 
@@ -876,7 +875,7 @@ int pi_model_generate(pi_model * m, int n_steps, int32_t * out_tokens, float * m
     }
     PI_HIP_TRY(hipEventRecord(m->ev1, m->stream));
     PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    if (m->cold) PI_TRY(pi::cold_drain(m->cold));
+    if (m->cold) PI_TRY(pi::cold_drain(m->cold, nullptr));
     if (ms_out) PI_HIP_TRY(hipEventElapsedTime(ms_out, m->ev0, m->ev1));
     PI_TRY(pi_memcpy_d2h(out_tokens, m->d_out_tokens, sizeof(int32_t) * n_steps));
     return PI_OK;

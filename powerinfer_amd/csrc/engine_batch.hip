@@ -685,18 +685,30 @@ void batch_destroy(pi_model * m) {
 }  // namespace pi
 
 namespace {
+// a step's tokens and positions as the kernel's arguments: no copy out of the caller's memory and no wait for one
+struct StepStart { int32_t token[16], pos[16]; };
+__global__ void step_start_kernel(StepStart in, int n, int32_t * __restrict__ tokens, int32_t * __restrict__ pos, int32_t * __restrict__ step) {
+    const int t = threadIdx.x;
+    if (t < n) { tokens[t] = in.token[t]; pos[t] = in.pos[t]; }
+    if (t == 0) *step = 0;
+}
+
 // after a step has completed: which layers run their FFN dense in the next one
-int choose_dense_layers(pi_model * m, BatchState * b) {
+bool dense_layers_possible(pi_model * m) { return m->hp.n_ff % 128 == 0 && m->hp.n_embd % 128 == 0 && !m->q4_steps; }   // the dense mat-muls' shapes; the integer route has no dense form
+int choose_dense_layers(pi_model * m, BatchState * b, const std::vector<int32_t> & u) {
     const pi_hparams & hp = m->hp;
-    if (hp.n_ff % 128 || hp.n_embd % 128 || m->q4_steps) return PI_OK;            // the dense mat-muls' shapes; the integer route has no dense form
-    std::vector<int32_t> u(hp.n_layer);
-    PI_TRY(pi_memcpy_d2h(u.data(), b->n_union, sizeof(int32_t) * hp.n_layer));
+    if (!dense_layers_possible(m)) return PI_OK;
     for (int il = 0; il < hp.n_layer; ++il) {
         const bool dense = b->dense_above <= 0.0f || (b->dense_above < 1.0f && (float)u[il] > b->dense_above * (float)hp.n_ff);
         if (dense) PI_TRY(ensure_down_rows(m, il));
         b->dense_ffn[il] = dense ? 1 : 0;
     }
     return PI_OK;
+}
+int choose_dense_layers(pi_model * m, BatchState * b) {
+    std::vector<int32_t> u(m->hp.n_layer);
+    if (dense_layers_possible(m)) PI_TRY(pi_memcpy_d2h(u.data(), b->n_union, sizeof(int32_t) * u.size()));
+    return choose_dense_layers(m, b, u);
 }
 }  // namespace
 
@@ -746,16 +758,17 @@ int pi_model_batch_decode(pi_model * m, const int32_t * tokens, const int32_t * 
         if (tokens[t] < 0 || tokens[t] >= m->hp.n_vocab) return pi::fail(PI_E_ARG, "pi_model_batch_decode: token id out of range");
         if (positions[t] < 0 || positions[t] >= m->hp.n_ctx) return pi::fail(PI_E_ARG, "pi_model_batch_decode: position outside the context");
     }
-    PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * b->n_seq, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipMemcpyAsync(b->d_pos, positions, sizeof(int32_t) * b->n_seq, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipMemsetAsync(b->d_step, 0, 4, m->stream));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));          // the host arrays may be pageable: finish the copies before returning control
+    StepStart in;
+    for (int t = 0; t < b->n_seq; ++t) { in.token[t] = tokens[t]; in.pos[t] = positions[t]; }
+    hipLaunchKernelGGL(step_start_kernel, dim3(1), dim3(64), 0, m->stream, in, b->n_seq, b->d_tokens, b->d_pos, b->d_step);
+    PI_TRY(pi::check_launch("step_start"));
     PI_TRY(batch_step(m, m->batch));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    PI_TRY(choose_dense_layers(m, b));
-    if (next_tokens) PI_TRY(pi_memcpy_d2h(next_tokens, b->d_tokens, sizeof(int32_t) * b->n_seq));
-    if (logits_out) PI_TRY(pi_memcpy_d2h(logits_out, b->logits, sizeof(float) * (size_t)b->n_seq * m->hp.n_vocab));
-    return PI_OK;
+    std::vector<int32_t> u(m->hp.n_layer);
+    const pi::HostCopy results[] = {{b->n_union, dense_layers_possible(m) ? u.data() : nullptr, sizeof(int32_t) * u.size()},
+                                    {b->d_tokens, next_tokens, sizeof(int32_t) * b->n_seq},
+                                    {b->logits, logits_out, sizeof(float) * (size_t)b->n_seq * m->hp.n_vocab}};
+    PI_TRY(m->stage.fetch(results, 3, m->stream));
+    return choose_dense_layers(m, b, u);
 }
 
 int pi_model_batch_generate(pi_model * m, int n_steps, int32_t * out_tokens, float * ms_out) {
@@ -915,10 +928,9 @@ int pi_model_kv_cells_decode(pi_model * m, const int32_t * tokens, const int32_t
     PI_HIP_TRY(hipMemsetAsync(b->d_step, 0, 4, m->stream));
     PI_HIP_TRY(hipStreamSynchronize(m->stream));
     PI_TRY(batch_step(m, b));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
+    const pi::HostCopy results[] = {{b->d_tokens, next_tokens, sizeof(int32_t) * n_tokens}, {b->logits, logits_out, sizeof(float) * (size_t)n_tokens * m->hp.n_vocab}};
+    PI_TRY(m->stage.fetch(results, 2, m->stream));
     kv.move_head(kv.head + n_tokens);
-    if (next_tokens) PI_TRY(pi_memcpy_d2h(next_tokens, b->d_tokens, sizeof(int32_t) * n_tokens));
-    if (logits_out) PI_TRY(pi_memcpy_d2h(logits_out, b->logits, sizeof(float) * (size_t)n_tokens * m->hp.n_vocab));
     return PI_OK;
 }
 

@@ -4,6 +4,7 @@
 #include "../../include/powerinfer_hip.h"
 #include "cold_path.hpp"
 #include "kv_cells.hpp"
+#include "runtime.hpp"
 
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
@@ -50,6 +51,7 @@ struct pi_model {
     float *attn_scratch = nullptr;        // partial results of those workgroups for one token
     float *attn_scratch_chunk = nullptr;  // and for a prompt chunk (allocated at the first chunk that needs it)
 
+    pi::HostStage stage;                  // results on their way to the caller
     hipGraphExec_t graph_exec = nullptr;
     hipGraph_t graph = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -1476,6 +1476,7 @@ int layers_finalize(pi_model * m) {
     s->g_work = m->alloc<int32_t>(4 * items);
     s->g_out = m->alloc<int32_t>((size_t)s->max_steps * kMaxLockstep);
     if (!s->g_work || !s->g_out) return PI_E_HIP;
+    m->stage.init(sizeof(float) * 16 * (size_t)m->hp.n_vocab);
     PI_HIP_TRY(hipDeviceSynchronize());
     m->finalized = true;
     return PI_OK;
@@ -1673,13 +1674,13 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             const size_t V = m->hp.n_vocab;
             PI_TRY(pass_head(m, d_rows + r0, n));
             if (next_tokens) for (int k = 0; k < n; k += 16) PI_TRY(pi_k_argmax_batch(s->logits + k * V, (int)V, std::min(16, n - k), s->d_next + k, nullptr, nullptr, nullptr, 0, m->stream));
-            PI_HIP_TRY(hipStreamSynchronize(m->stream));
             std::vector<int32_t> nx(next_tokens ? n : 0);
-            if (next_tokens) PI_TRY(pi_memcpy_d2h(nx.data(), s->d_next, 4 * (size_t)n));
             for (int k = 0; k < n; ) {                              // runs of places that follow one another leave in one copy
                 int e = k + 1;
                 while (e < n && place[r0 + e] == place[r0 + k] + (e - k)) ++e;
-                if (logits_out) PI_TRY(pi_memcpy_d2h(logits_out + (size_t)place[r0 + k] * V, s->logits + (size_t)k * V, sizeof(float) * V * (e - k)));
+                const pi::HostCopy results[] = {{s->d_next, next_tokens && k == 0 ? nx.data() : nullptr, 4 * (size_t)n},
+                                                {s->logits + (size_t)k * V, logits_out ? logits_out + (size_t)place[r0 + k] * V : nullptr, sizeof(float) * V * (e - k)}};
+                PI_TRY(m->stage.fetch(results, 2, m->stream));
                 if (next_tokens) for (int j = k; j < e; ++j) next_tokens[place[r0 + j]] = nx[j];
                 k = e;
             }

@@ -495,13 +495,20 @@ __global__ __launch_bounds__(kBlock) void gemv_q4_kernel(const pi_block_q4_0 * _
     }
 }
 
-__global__ void embed_f16_kernel(const __half * __restrict__ table, int cols, const int32_t * __restrict__ token, float * __restrict__ x) {
-    const __half * row = table + (size_t)(*token) * cols;
+// state: the token loop's state, written where the host names the token (embed_start); token is then null
+struct TokenStart { int32_t token, pos; int32_t * d_token, * d_pos, * d_step; };
+__device__ __forceinline__ int32_t start_token(const int32_t * token, const TokenStart & s) {
+    if (token) return *token;
+    if (blockIdx.x == 0 && threadIdx.x == 0) { *s.d_token = s.token; *s.d_pos = s.pos; *s.d_step = 0; }
+    return s.token;
+}
+__global__ void embed_f16_kernel(const __half * __restrict__ table, int cols, const int32_t * __restrict__ token, float * __restrict__ x, TokenStart start) {
+    const __half * row = table + (size_t)start_token(token, start) * cols;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cols; i += gridDim.x * blockDim.x) x[i] = __half2float(row[i]);
 }
 // blockIdx.y = token of a chunk (0 for a single token)
-__global__ void embed_q4_kernel(const pi_block_q4_0 * __restrict__ table, int cols, const int32_t * __restrict__ token, float * __restrict__ x) {
-    const pi_block_q4_0 * row = table + (size_t)token[blockIdx.y] * (cols / 32);
+__global__ void embed_q4_kernel(const pi_block_q4_0 * __restrict__ table, int cols, const int32_t * __restrict__ token, float * __restrict__ x, TokenStart start) {
+    const pi_block_q4_0 * row = table + (size_t)start_token(token ? token + blockIdx.y : nullptr, start) * (cols / 32);
     x += (size_t)blockIdx.y * cols;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cols; i += gridDim.x * blockDim.x) {
         const pi_block_q4_0 * b = row + (i >> 5);
@@ -728,18 +735,31 @@ int pi_k_gemv_multi_f16(const void * const * W, const int * rows, int n_mat, int
 
 int pi_k_embed_batch_q4(const void * table_q4, int cols, const int32_t * tokens, int T, float * x, pi_stream_t stream) {
     if (!table_q4 || !tokens || !x || cols <= 0 || cols % 32 || T <= 0 || T > kChunkMaxT) return pi::fail(PI_E_ARG, "pi_k_embed_batch_q4: bad arguments");
-    hipLaunchKernelGGL(embed_q4_kernel, dim3((cols + 255) / 256, T), dim3(256), 0, (hipStream_t)stream, (const pi_block_q4_0 *)table_q4, cols, tokens, x);
+    hipLaunchKernelGGL(embed_q4_kernel, dim3((cols + 255) / 256, T), dim3(256), 0, (hipStream_t)stream, (const pi_block_q4_0 *)table_q4, cols, tokens, x, TokenStart{});
     return pi::check_launch("pi_k_embed_batch_q4");
+}
+
+static int embed_one(int wtype, const void * table, int cols, const int32_t * token, const TokenStart & start, float * x, hipStream_t st) {
+    const int blocks = (cols + 255) / 256;
+    if (wtype == PI_TYPE_F16)       hipLaunchKernelGGL(embed_f16_kernel, dim3(blocks), dim3(256), 0, st, (const __half *)table, cols, token, x, start);
+    else if (wtype == PI_TYPE_Q4_0) hipLaunchKernelGGL(embed_q4_kernel, dim3(blocks), dim3(256), 0, st, (const pi_block_q4_0 *)table, cols, token, x, start);
+    else return pi::fail(PI_E_UNSUPPORTED, "pi_k_embed: table type must be F16 or Q4_0");
+    return pi::check_launch("pi_k_embed");
 }
 
 int pi_k_embed(int wtype, const void * table, int cols, const int32_t * token, float * x, pi_stream_t stream) {
     if (!table || !token || !x || cols <= 0) return pi::fail(PI_E_ARG, "pi_k_embed: bad arguments");
-    const int blocks = (cols + 255) / 256;
-    if (wtype == PI_TYPE_F16)       hipLaunchKernelGGL(embed_f16_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (const __half *)table, cols, token, x);
-    else if (wtype == PI_TYPE_Q4_0) hipLaunchKernelGGL(embed_q4_kernel, dim3(blocks), dim3(256), 0, (hipStream_t)stream, (const pi_block_q4_0 *)table, cols, token, x);
-    else return pi::fail(PI_E_UNSUPPORTED, "pi_k_embed: table type must be F16 or Q4_0");
-    return pi::check_launch("pi_k_embed");
+    return embed_one(wtype, table, cols, token, TokenStart{}, x, (hipStream_t)stream);
 }
+
+}  // extern "C"
+namespace pi {
+int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream) {
+    if (!table || !d_token || !d_pos || !d_step || !x || cols <= 0) return fail(PI_E_ARG, "embed_start: bad arguments");
+    return embed_one(wtype, table, cols, nullptr, TokenStart{token, pos, d_token, d_pos, d_step}, x, (hipStream_t)stream);
+}
+}  // namespace pi
+extern "C" {
 
 int pi_k_argmax(const float * logits, int n, int32_t * token_out, pi_stream_t stream) {
     if (!logits || !token_out || n <= 0) return pi::fail(PI_E_ARG, "pi_k_argmax: bad arguments");

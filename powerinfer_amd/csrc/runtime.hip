@@ -36,6 +36,86 @@ int compute_units() {
 }
 }  // namespace pi
 
+namespace {
+struct CopyOut { const uint32_t * src[pi::HostStage::kMaxCopies]; uint32_t words[pi::HostStage::kMaxCopies], at[pi::HostStage::kMaxCopies]; };
+__global__ __launch_bounds__(256) void copy_out_kernel(CopyOut c, uint32_t * __restrict__ dst) {
+    const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+#pragma unroll
+    for (int r = 0; r < pi::HostStage::kMaxCopies; ++r) {
+        const uint32_t * s = c.src[r];
+        uint32_t * d = dst + c.at[r];
+        uint32_t done = 0;
+        if (((uintptr_t)s & 15) == 0) {                             // (places in the buffer are multiples of 64 bytes)
+            const uint32_t n4 = c.words[r] / 4;
+            for (uint32_t i = i0; i < n4; i += step) reinterpret_cast<uint4 *>(d)[i] = reinterpret_cast<const uint4 *>(s)[i];
+            done = n4 * 4;
+        }
+        for (uint32_t i = done + i0; i < c.words[r]; i += step) d[i] = s[i];
+    }
+}
+}  // namespace
+
+namespace pi {
+void HostStage::init(size_t usual_bytes) {
+    if (pin) return;
+    const size_t want = usual_bytes + 4096;
+    n_pieces = want > kPiece ? kPieces : 1;
+    piece = n_pieces > 1 ? kPiece : (want + 4095) / 4096 * 4096;
+    if (hipHostMalloc((void **)&pin, piece * n_pieces, hipHostMallocDefault) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
+    for (int i = 0; i < n_pieces && pin; ++i)
+        if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) { ev[i] = nullptr; (void)hipGetLastError(); release(); }
+}
+
+void HostStage::release() {
+    for (hipEvent_t & e : ev) if (e) { (void)hipEventDestroy(e); e = nullptr; }
+    if (pin) { (void)hipHostFree(pin); pin = nullptr; }
+}
+
+int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
+    HostCopy c[kMaxCopies];
+    int m = 0;
+    size_t small = 0, at[kMaxCopies] = {};
+    for (int i = 0; i < n; ++i)
+        if (copies[i].host && copies[i].bytes) { if (m == kMaxCopies) return fail(PI_E_ARG, "fetch: too many results"); c[m++] = copies[i]; }
+    for (int i = 0; i + 1 < m; ++i) { at[i] = small; small += (c[i].bytes + 63) / 64 * 64; }
+    if (!pin || small > 4096) {
+        PI_HIP_TRY(hipStreamSynchronize(st));
+        for (int i = 0; i < m; ++i) PI_HIP_TRY(hipMemcpy(c[i].host, c[i].dev, c[i].bytes, hipMemcpyDeviceToHost));
+        return PI_OK;
+    }
+    if (m == 0) { PI_HIP_TRY(hipStreamSynchronize(st)); return PI_OK; }
+    // the last result in pieces; the first one leaves room for the others
+    const HostCopy & big = c[m - 1];
+    size_t sent = 0, taken = 0;                                     // bytes of it
+    size_t from[kPieces] = {}, len[kPieces] = {};
+    int queued = 0, fetched = 0;
+    while (taken < big.bytes) {
+        while (sent < big.bytes && queued - fetched < n_pieces) {
+            const int slot = queued % n_pieces;
+            const size_t head = queued ? 0 : small;
+            const size_t b = big.bytes - sent < piece - head ? big.bytes - sent : piece - head;
+            CopyOut o{};
+            for (int i = 0; i + 1 < m && !queued; ++i) { o.src[i] = (const uint32_t *)c[i].dev; o.words[i] = (uint32_t)(c[i].bytes / 4); o.at[i] = (uint32_t)(at[i] / 4); }
+            o.src[kMaxCopies - 1] = (const uint32_t *)((const unsigned char *)big.dev + sent); o.words[kMaxCopies - 1] = (uint32_t)(b / 4); o.at[kMaxCopies - 1] = (uint32_t)(head / 4);
+            const unsigned blocks = (unsigned)((b / 16 + 255) / 256);
+            hipLaunchKernelGGL(copy_out_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, st, o, reinterpret_cast<uint32_t *>(pin + (size_t)slot * piece));
+            if (const int rc = check_launch("copy_out")) return rc;
+            from[slot] = sent; len[slot] = b; sent += b; ++queued;
+            if (sent < big.bytes) PI_HIP_TRY(hipEventRecord(ev[slot], st));
+        }
+        const int slot = fetched % n_pieces;
+        const bool last = sent == big.bytes && fetched + 1 == queued;
+        if (last) PI_HIP_TRY(hipStreamSynchronize(st));
+        else PI_HIP_TRY(hipEventSynchronize(ev[slot]));
+        const unsigned char * s = pin + (size_t)slot * piece;
+        if (!fetched) for (int i = 0; i + 1 < m; ++i) memcpy(c[i].host, s + at[i], c[i].bytes);
+        memcpy((unsigned char *)big.host + from[slot], s + (fetched ? 0 : small), len[slot]);
+        taken += len[slot]; ++fetched;
+    }
+    return PI_OK;
+}
+}  // namespace pi
+
 extern "C" {
 
 const char * pi_last_error(void) { return pi::g_err; }

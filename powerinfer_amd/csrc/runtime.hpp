@@ -5,6 +5,8 @@
 
 #include "../../include/powerinfer_hip.h"
 
+#include <stddef.h>
+
 namespace pi {
 
 // Weights that a launch requests ahead of the one that reads them (load_ahead in kernels_common.hpp): up to two matrices in units of unit_bytes (a
@@ -18,9 +20,29 @@ int  check_launch(const char * what);                  // hipGetLastError() afte
 int  compute_units();                                  // compute units of the current device (0 on error); cached per device, allocates nothing
 int  noalloc_setup();                                  // resolves the static scratch array of pi_k_sparse_ffn_noalloc on the current device
 
+// A call's results on their way from the device to the caller's memory.  A copy to pageable memory costs 13 us for 4 bytes and 62 us for the
+// 128 KB of 32000 logits, each with a wait of its own; here one small kernel behind the call's last one stores all of them in pinned
+// memory, one wait covers both, and a memcpy (3 us for 128 KB, still in the host's cache) brings them home.  Larger results (2 MB: 16
+// rows of logits) travel in pieces of 512 KB, each copied while the next ones cross the link.  Part of one model, used by one call at a time.
+struct HostCopy { const void * dev; void * host; size_t bytes; };        // multiples of 4 bytes, dev 4-byte aligned; host null: not wanted
+struct HostStage {
+    static constexpr int kPieces = 4, kMaxCopies = 4;
+    static constexpr size_t kPiece = (size_t)512 << 10;
+    unsigned char * pin = nullptr;         // null (no pinned memory to be had): ordinary copies
+    size_t piece = 0; int n_pieces = 0;
+    hipEvent_t ev[kPieces] = {};
+    void init(size_t usual_bytes);
+    void release();
+    // queues the copies behind what the stream holds and returns when the stream is done and the results are in place; all but the
+    // last copy together fit in 4 KB of the first piece (else ordinary copies)
+    int fetch(const HostCopy * copies, int n, hipStream_t st);
+};
+
 // pi_k_attn_fused with such extra workgroups
 int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream);
+// the embedding row of a token that the host names; also writes the token loop's state (token, position, step counter 0)
+int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
 
 }  // namespace pi
 

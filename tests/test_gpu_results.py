@@ -1,0 +1,29 @@
+"""Results leave the device through pinned pieces of 512 KB (HostStage): logits whose size lies at the edges of a piece and of the ring of four."""
+import numpy as np
+import pytest
+
+from powerinfer_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_vocab", [33, 8128, 8192, 9001, 32768, 40003])
+def test_logits_arrive_whole(n_vocab):
+    """16 equal sequences: equal rows, each the single sequence's logits to within the two kernels' orders of summation (products of 512
+    fp16-rounded values: 1e-2 of the largest, the bound the batch tests use), and next tokens that are the rows' maxima."""
+    from powerinfer_amd.model import Model
+    hp = synth.hparams("llama-tiny", n_vocab=n_vocab, n_ctx=64, seed=11, sparse_threshold=-1e30)        # every neuron active: no mask to flip on a last place
+    gm = Model(hp).load(synth.make_model(hp))
+    gm.batch_init(16)
+    for pos, tok in enumerate([3, n_vocab - 1, 7]):
+        print(n_vocab, pos, flush=True)
+        one, lg1 = gm.decode([tok], pos)
+        nxt, lg = gm.batch_decode([tok] * 16, [pos] * 16)
+        assert one == int(lg1.argmax()) and lg.shape == (16, n_vocab)
+        assert np.isfinite(lg).all() and (lg == lg[0]).all() and (nxt == lg.argmax(1)).all()
+        assert np.abs(lg[0] - lg1).max() <= 1e-2 * np.abs(lg1).max()
+        none, nothing = gm.batch_decode([tok] * 16, [pos] * 16, want_logits=False)
+        assert nothing is None and (none == nxt).all()
+        again, lg2 = gm.decode([tok], pos, want_logits=False)
+        assert again == one and lg2 is None
+    gm.close()
