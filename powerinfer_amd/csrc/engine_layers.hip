@@ -783,7 +783,9 @@ int experts(pi_model * m, Layer & L, const void * h, const Step & in) {
     const pi_layer_desc & d = L.d;
     const int T = in.T, D = m->hp.n_embd, per = d.ffn == PI_FFN_GLU_MOE ? 2 : 1;
     hipStream_t st = m->stream;
-    const int tile_n = (long long)T * d.n_top > 96LL * d.n_expert ? 128 : 64;       // tokens per tile, by the tokens an expert has on average
+    // tokens per tile, by the tokens an expert has on average: the large tiles read the weights once where most experts have more than 64
+    // tokens (64 experts 1408 x 2048, us with 64 and 128: 47 tokens 145 + 84 and 154 + 73; 72 tokens 197 + 101 and 161 + 81; 94 tokens 204 + 102 and 163 + 85)
+    const int tile_n = (long long)T * d.n_top > 52LL * d.n_expert ? 128 : 64;
     PI_TRY(pi_k_moe_sort(s->ids, T * d.n_top, d.n_expert, s->off, s->perm, s->inv, tile_n, s->tiles, s->n_tiles, st));
     pi_group_gemm g{};
     g.W = L.up; g.w_gs = (size_t)per * d.expert_ff * s->d_ld; g.rows = per * d.expert_ff; g.cols = s->d_ld; g.ldw = s->d_ld; g.n_group = d.n_expert; g.alpha = 1.0f;

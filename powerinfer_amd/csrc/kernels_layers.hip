@@ -368,44 +368,14 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int32_t * __restri
 // (g.tiles) or, without a list, every group has ceil(T / BN) of them.  The units are dealt out so that an XCD works through a
 // contiguous range of them: the row tiles of a token tile, and the token tiles of a group, share that XCD's L2.
 // ---------------------------------------------------------------------------------------------------------------------------------
-template <int BM, int BN, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192 ? 3 : 2)) void group_tile_kernel(pi_group_gemm g, int nx, int max_units) {
-    using Tile = GemmTile<bf16, BM, BN, WGM, WGN>;
-    constexpr int WM = Tile::WM, WN = Tile::WN, MT = Tile::MT, NT = Tile::NT;
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int tt = (g.T + BN - 1) / BN;                       // token tiles of a group without a list
-    const int units = g.off ? *g.n_tiles * nx : max_units;
-    const int per = (units + 7) / 8, unit = (int)(blockIdx.x % 8) * per + (int)blockIdx.x / 8;
-    if ((int)blockIdx.x / 8 >= per || unit >= units) return;
-    const int tx = unit % nx, ty = unit / nx;
-    int grp, lo, n;                                           // group, first token (place), tokens from there on
-    if (g.off) {
-        const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
-        grp = t.x; lo = t.y; n = g.off[grp + 1] - lo;
-    } else {
-        grp = ty / tt; lo = (ty % tt) * BN; n = g.T - lo;
-    }
-    n = min(n, BN);
-    const int row0 = tx * BM;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
-    const int wm = wave % WGM, wn = wave / WGM;
-    const bf16 * W = (const bf16 *)g.W + (size_t)grp * g.w_gs;
-    const bf16 * x = (const bf16 *)g.x + (g.off ? 0 : (size_t)grp * g.x_gs);
-    const bf16 * ga[Tile::ACH]; const bf16 * gb[Tile::BCH];
-#pragma unroll
-    for (int j = 0; j < Tile::ACH; ++j) ga[j] = W + (size_t)min(row0 + Tile::chunk_row(j), g.rows - 1) * g.ldw + Tile::chunk_col();
-#pragma unroll
-    for (int j = 0; j < Tile::BCH; ++j) {
-        const int s = lo + min(Tile::chunk_row(j), n - 1);
-        gb[j] = x + (size_t)(g.gather ? g.gather[s] / g.gather_div : s) * g.ldx + Tile::chunk_col();
-    }
-    pi_f4 acc[MT][NT];
-    Tile::run(smem, ga, gb, g.cols / kGtBK, acc);
+// a wave's 16 x 16 tiles of outputs, rows from row0 and tokens from tok0 of the token tile (group grp, places lo .. lo + n - 1); lane = 16 q + i
+template <int MT, int NT>
+__device__ __forceinline__ void group_store(const pi_group_gemm & g, int grp, int lo, int n, int row0, int tok0, int q, int i, const pi_f4 (&acc)[MT][NT]) {
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int nn = 0; nn < NT; ++nn) {
-            const int row = row0 + wm * WM + m * 16 + 4 * q, tok = wn * WN + nn * 16 + i;
+            const int row = row0 + m * 16 + 4 * q, tok = tok0 + nn * 16 + i;
             if (tok >= n || row >= g.rows) continue;
             const float alpha = g.pair_w ? g.alpha * g.pair_w[g.gather[lo + tok]] : g.alpha;
             if (g.glu) {                               // rows in (gate, up) pairs: a lane holds two of them
@@ -444,6 +414,274 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192
                 else for (int r = 0; r < 4 && row + r < g.rows; ++r) y[r] = b[r];
             }
         }
+}
+
+template <int BM, int BN, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192 ? 3 : 2)) void group_tile_kernel(pi_group_gemm g, int nx, int max_units) {
+    using Tile = GemmTile<bf16, BM, BN, WGM, WGN>;
+    constexpr int WM = Tile::WM, WN = Tile::WN, MT = Tile::MT, NT = Tile::NT;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tt = (g.T + BN - 1) / BN;                       // token tiles of a group without a list
+    const int units = g.off ? *g.n_tiles * nx : max_units;
+    const int per = (units + 7) / 8, unit = (int)(blockIdx.x % 8) * per + (int)blockIdx.x / 8;
+    if ((int)blockIdx.x / 8 >= per || unit >= units) return;
+    const int tx = unit % nx, ty = unit / nx;
+    int grp, lo, n;                                           // group, first token (place), tokens from there on
+    if (g.off) {
+        const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
+        grp = t.x; lo = t.y; n = g.off[grp + 1] - lo;
+    } else {
+        grp = ty / tt; lo = (ty % tt) * BN; n = g.T - lo;
+    }
+    n = min(n, BN);
+    const int row0 = tx * BM;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    const int wm = wave % WGM, wn = wave / WGM;
+    const bf16 * W = (const bf16 *)g.W + (size_t)grp * g.w_gs;
+    const bf16 * x = (const bf16 *)g.x + (g.off ? 0 : (size_t)grp * g.x_gs);
+    const bf16 * ga[Tile::ACH]; const bf16 * gb[Tile::BCH];
+#pragma unroll
+    for (int j = 0; j < Tile::ACH; ++j) ga[j] = W + (size_t)min(row0 + Tile::chunk_row(j), g.rows - 1) * g.ldw + Tile::chunk_col();
+#pragma unroll
+    for (int j = 0; j < Tile::BCH; ++j) {
+        const int s = lo + min(Tile::chunk_row(j), n - 1);
+        gb[j] = x + (size_t)(g.gather ? g.gather[s] / g.gather_div : s) * g.ldx + Tile::chunk_col();
+    }
+    pi_f4 acc[MT][NT];
+    Tile::run(smem, ga, gb, g.cols / kGtBK, acc);
+    group_store(g, grp, lo, n, row0 + wm * WM, wn * WN, q, i, acc);
+}
+
+// The same through LDS, where outputs come in whole pieces of 16 bytes: the lanes' quads of rows, written as they are, are runs of 32 bytes a
+// token (8 us for 256 x 128 outputs of a workgroup); eight tokens at a time, turned in 2 KB of the wave's own, leave in runs of up to 256
+// bytes.  One kind of epilogue at a time, as the code runs once a unit and its instructions come from L2 each time.
+enum { kStorePlain, kStoreRelu2, kStoreGlu };
+template <int KIND, int MT, int NT>
+__device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int grp, int lo, int n, int row0, int tok0, int lane, const pi_f4 (&acc)[MT][NT], unsigned char * turn) {
+    constexpr int kRow = KIND == kStoreGlu ? MT * 16 : MT * 32, kPieces = kRow / 16, kToks = 64 / kPieces;      // bytes and pieces of a token, tokens a store instruction takes
+    asm volatile("" : "+v"(lane));                     // what follows is computed here, not kept in registers across the products
+    const int i = lane & 15, q = lane >> 4;
+    const float one = g.glu_plain_up ? 0.0f : 1.0f;
+    const int out0 = KIND == kStoreGlu ? row0 / 2 : row0, outs = KIND == kStoreGlu ? g.rows / 2 : g.rows;
+    const int piece = lane % kPieces, first = lane / kPieces;
+#pragma unroll
+    for (int nn = 0; nn < NT; ++nn) {
+        const int tok = tok0 + nn * 16 + i;
+        const float alpha = g.pair_w ? g.alpha * g.pair_w[g.gather[lo + min(tok, n - 1)]] : g.alpha;
+        __builtin_amdgcn_sched_barrier(0);
+        uint2 out[MT];                                              // this lane's four rows (Glu: two outputs) of every 16
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if constexpr (KIND == kStoreGlu) {
+                const bf16 v[2] = {(bf16)clamped_glu(acc[m][nn][0] * alpha, acc[m][nn][1] * alpha, g.glu_limit, g.glu_gain, one),
+                                   (bf16)clamped_glu(acc[m][nn][2] * alpha, acc[m][nn][3] * alpha, g.glu_limit, g.glu_gain, one)};
+                out[m].x = __builtin_bit_cast(uint32_t, v);
+            } else {
+                bf16 b[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = acc[m][nn][r] * alpha;
+                    if (KIND == kStoreRelu2) { v = fmaxf(v, 0.0f); v *= v; }
+                    b[r] = (bf16)v;
+                }
+                out[m] = __builtin_bit_cast(uint2, b);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {                               // tokens 0 .. 7 of the sixteen, then 8 .. 15
+            unsigned char * mine = turn + (i & 7) * kRow;
+            if ((i >> 3) == h) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    if constexpr (KIND == kStoreGlu) *reinterpret_cast<uint32_t *>(mine + (m ^ (i & 7) % kPieces) * 16 + q * 4) = out[m].x;
+                    else *reinterpret_cast<uint2 *>(mine + ((2 * m + (q >> 1)) ^ ((i & 7) % kPieces)) * 16 + (q & 1) * 8) = out[m];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int kTurnWaves = (8 * kPieces + 63) / 64;
+#pragma unroll
+            for (int t0 = 0; t0 < kTurnWaves; ++t0) {
+                const int t = t0 * kToks + first, to = tok0 + nn * 16 + 8 * h + t;
+                const pi_u32x4 v = *reinterpret_cast<const pi_u32x4 *>(turn + (t & 7) * kRow + (piece ^ ((t & 7) % kPieces)) * 16);
+                if (t < 8 && to < n && out0 + piece * 8 < outs)
+                    *reinterpret_cast<pi_u32x4 *>((bf16 *)g.y + (g.off ? 0 : (size_t)grp * g.y_gs) + (size_t)(lo + to) * g.ldy + out0 + piece * 8) = v;
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------------------------
+// The same product in large tiles: 256 rows x 128 tokens, one workgroup per compute unit that stays for all of its units.  Four waves
+// multiply (128 x 64 outputs each), four copy: a stage of 64 columns goes from memory straight to LDS, three stages deep and on
+// into the next unit, and a copy that has to wait for the memory's queues holds up no matrix instruction (copying from the
+// multiplying waves themselves: 238 us for the first product below).  A multiplying wave reads the fragments of a stage's second 32 columns
+// under the products of the first and those of the next stage's first 32 under the products of the second, with the one barrier
+// of a stage in between: behind it the next stage is whole and the present one is free to be copied over.  LDS rows and swizzle are GemmTile's; a
+// copy's 64 lanes bring eight rows of 128 bytes and take the swizzle on the side they read from.  Where half a tile or less is
+// wanted (128 rows, 64 tokens) the four waves share that half, 64 x 64 outputs each.  The sums are formed in GemmTile's order.
+// Measured (us; 128 x 128 tiles of GemmTile before): 64 experts of 192 tokens on average, 1408 x 4096: 301 -> 218, 4096 x 1408:
+// 307 -> 227 (weights alone: 123 at 6 TB/s); one group of 12288: 199 -> 144, 1 PFLOP/s; 16 experts of 128: 51 -> 45 and 38 -> 34.
+// ---------------------------------------------------------------------------------------------------------------------------------
+constexpr int kGwM = 256, kGwN = 128, kGwStages = 3, kGwStage = (kGwM + kGwN) * kGtRow, kGwTurn = 2048, kGwLds = kGwStages * kGwStage + 64 + 4 * kGwTurn;
+__global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int nx, int max_units) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tt = (g.T + kGwN - 1) / kGwN;
+    const int units = g.off ? *g.n_tiles * nx : max_units;
+    const int per = (units + 7) / 8, step = (int)gridDim.x / 8, end = min(((int)blockIdx.x % 8 + 1) * per, units);
+    int unit = (int)(blockIdx.x % 8) * per + (int)blockIdx.x / 8;
+    if (unit >= end) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    const int nk = g.cols / kGtBK;
+    const bool whole = !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0;
+    struct Place { int grp, lo, n, row0; };
+    Place * places = reinterpret_cast<Place *>(smem + kGwStages * kGwStage);      // of this unit and the three behind it, written by the first copying wave
+    auto place = [&](int u) {
+        Place p;
+        const int tx = u % nx, ty = u / nx;
+        if (g.off) {
+            const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
+            p.grp = t.x; p.lo = t.y; p.n = g.off[p.grp + 1] - p.lo;
+        } else {
+            p.grp = ty / tt; p.lo = (ty % tt) * kGwN; p.n = g.T - p.lo;
+        }
+        p.n = min(p.n, kGwN);
+        p.row0 = tx * kGwM;
+        return p;
+    };
+    if (wave >= 4) {
+        // A wave that copies.  Of each stage eight times eight rows of W and four times eight of x are its own, each 128 bytes; lane l brings
+        // the piece that belongs at place l % 8 of row l / 8
+        const int w = wave - 4, piece = ((lane & 7) ^ (lane >> 3)) * 16;
+        uint32_t va[8];
+        size_t vb[4];
+        const unsigned char * fa, * fb;
+        int k = 0, c = 0;
+        auto aim = [&](int u) {
+            const Place p = place(u);
+            if (w == 0 && lane == 0) places[c & 3] = p;
+            ++c;
+            fa = (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs);
+            fb = (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs));
+#pragma unroll
+            for (int j = 0; j < 8; ++j) va[j] = (uint32_t)min(p.row0 + 64 * w + 8 * j + (lane >> 3), g.rows - 1) * (uint32_t)(g.ldw * 2) + piece;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int at = p.lo + min(32 * w + 8 * j + (lane >> 3), p.n - 1);
+                vb[j] = (size_t)(g.gather ? g.gather[at] / g.gather_div : at) * (size_t)g.ldx * 2 + piece;
+            }
+        };
+        typedef const __attribute__((address_space(1))) void * gptr;
+        typedef __attribute__((address_space(3))) void * lptr;
+        auto copy_stage = [&](unsigned char * stage) {             // past the last unit the last stage is copied again, and not used
+#pragma unroll
+            for (int j = 0; j < 8; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + (size_t)k * kGtRow + va[j]), (lptr)(stage + (64 * w + 8 * j) * kGtRow), 16, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) __builtin_amdgcn_global_load_lds((gptr)(fb + (size_t)k * kGtRow + vb[j]), (lptr)(stage + (kGwM + 32 * w + 8 * j) * kGtRow), 16, 0, 0);
+            if (++k < nk) return;
+            if (unit + step < end) { unit += step; k = 0; aim(unit); } else k = nk - 1;
+        };
+        int total = 0;
+        for (int u = unit; u < end; u += step) total += nk;
+        aim(unit);
+        for (int st = 0; st < kGwStages; ++st) copy_stage(smem + st * kGwStage);
+        __builtin_amdgcn_s_waitcnt(0x4078);                         // vmcnt(24): the first stage; lgkmcnt(0): its place
+        __builtin_amdgcn_s_barrier();
+        for (int t = 0, cb = 0; t < total; ++t) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0x007C);                     // vmcnt(12): the stage after t; lgkmcnt(0): a place
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            copy_stage(smem + cb * kGwStage);
+            cb = cb == kGwStages - 1 ? 0 : cb + 1;
+        }
+        __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0): no copy may arrive in LDS that is no longer this workgroup's
+        return;
+    }
+    unsigned char * turn = smem + kGwStages * kGwStage + 64 + wave * kGwTurn;
+    int cb = 0;                                                    // the stage that is being multiplied
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int koff[2] = {(q ^ (i & 7)) * 16, ((4 + q) ^ (i & 7)) * 16};
+    auto run = [&](auto mt, const Place & p, int rb, int tb) {      // rows rb .. and tokens tb .. of the tile are this wave's
+        constexpr int MT = decltype(mt)::value;
+        pi_f4 acc[MT][4];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[m][n] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        pi_u32x4 f0a[MT], f0b[4], f1a[MT], f1b[4];
+        const int oa = (rb + i) * kGtRow, ob = (kGwM + tb + i) * kGtRow;
+        auto ld = [&](int stage, int off) { return *reinterpret_cast<const pi_u32x4 *>(smem + stage * kGwStage + off); };
+#pragma unroll
+        for (int m = 0; m < MT; ++m) f0a[m] = ld(cb, oa + koff[0] + m * 16 * kGtRow);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) f0b[n] = ld(cb, ob + koff[0] + n * 16 * kGtRow);
+        // a group: the four MFMAs of one fragment of W.  A phase's reads follow its first RD groups' MFMAs: they never stand before an MFMA
+        // that waits for older ones, and the last groups cover their latency
+        constexpr int RD = MT / 2, RA = MT / RD, RB = 4 / RD;
+        for (int kt = 0; kt < nk; ++kt) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) acc[m][n] = mma16<bf16>(f0a[m], f0b[n], acc[m][n]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (m < RD) {
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) f1b[RB * m + r] = ld(cb, ob + koff[1] + (RB * m + r) * 16 * kGtRow);
+#pragma unroll
+                    for (int r = 0; r < RA; ++r) f1a[RA * m + r] = ld(cb, oa + koff[1] + (RA * m + r) * 16 * kGtRow);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the next stage has arrived (two more are on their way), and nobody reads this one any more
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);                     // lgkmcnt(0)
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            cb = cb == kGwStages - 1 ? 0 : cb + 1;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) acc[m][n] = mma16<bf16>(f1a[m], f1b[n], acc[m][n]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (m < RD) {
+#pragma unroll
+                    for (int r = 0; r < RB; ++r) f0b[RB * m + r] = ld(cb, ob + koff[0] + (RB * m + r) * 16 * kGtRow);
+#pragma unroll
+                    for (int r = 0; r < RA; ++r) f0a[RA * m + r] = ld(cb, oa + koff[0] + (RA * m + r) * 16 * kGtRow);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (whole && g.glu) group_store_turned<kStoreGlu>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
+        else if (whole && g.relu2) group_store_turned<kStoreRelu2>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
+        else if (whole) group_store_turned<kStorePlain>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
+        else group_store(g, p.grp, p.lo, p.n, p.row0 + rb, tb, q, i, acc);
+    };
+    for (int c = 0; unit < end; unit += step, ++c) {
+        const int * pl = reinterpret_cast<const int *>(places + (c & 3));
+        Place p;
+        p.grp = __builtin_amdgcn_readfirstlane(pl[0]); p.lo = __builtin_amdgcn_readfirstlane(pl[1]); p.n = __builtin_amdgcn_readfirstlane(pl[2]); p.row0 = __builtin_amdgcn_readfirstlane(pl[3]);
+        if (g.rows - p.row0 <= 128) run(std::integral_constant<int, 4>{}, p, 64 * (wave & 1), 64 * (wave >> 1));
+        else if (p.n <= 64) run(std::integral_constant<int, 4>{}, p, 64 * wave, 0);
+        else run(std::integral_constant<int, 8>{}, p, 128 * (wave & 1), 64 * (wave >> 1));
+    }
+}
+
+int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
+    static bool raised = false;
+    if (!raised) {
+        PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&group_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
+        raised = true;
+    }
+    const int nx = (g.rows + kGwM - 1) / kGwM;
+    const long long units = (long long)nx * (g.off ? g.max_tiles : (long long)g.n_group * ((g.T + kGwN - 1) / kGwN));
+    if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: too many tiles");
+    const long long blocks = std::min((units + 7) / 8 * 8, (long long)256);
+    hipLaunchKernelGGL(group_wide_kernel, dim3((unsigned)blocks), dim3(512), kGwLds, st, g, nx, (int)units);
+    return pi::check_launch("pi_k_group_gemm_tile");
 }
 
 template <int BM, int BN, int WGM, int WGN> int launch_group_tile(const pi_group_gemm & g, hipStream_t st) {
@@ -639,6 +877,9 @@ int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream
         return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: bad arguments");
     if ((((uintptr_t)g->W | (uintptr_t)g->x | (uintptr_t)g->y) & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: operands must be 16-byte aligned");
     hipStream_t st = (hipStream_t)stream;
+    // 256-row tiles from the second half on, and at least four stages for a unit's ends to hide behind: measured as fast or faster at every number of
+    // tokens and groups from there on (32 heads' 256 x 512 products of 128 tokens: 11.4 us both; 4096 x 512 by 2048 tokens 20.6 -> 16.1)
+    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31)) return launch_group_wide(*g, st);
     if (tile_n == 128) return launch_group_tile<128, 128, 2, 2>(*g, st);
     if (tile_n == 64) return g->rows <= 64 ? launch_group_tile<64, 64, 2, 2>(*g, st) : launch_group_tile<128, 64, 2, 2>(*g, st);
     return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: tile_n must be 64 or 128");

@@ -1,0 +1,80 @@
+"""The grouped product's large tiles (256 rows x 128 tokens, group_wide_kernel): bit for bit the small tiles' results, whose order of sums
+it keeps, and within bf16's rounding of float64, at the edges of tiles, halves of tiles, stages and units."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from powerinfer_amd import lib as pl
+from test_gpu_latent_ops import dev, fetch, group_args, i32, rounded, store
+
+pytestmark = pytest.mark.gpu
+
+
+def run(g, tile, n, ldy, y_f32):
+    y = pl.DevBuf.zeros(4 * n * ldy + 64)
+    g.y = y.ptr
+    pl.check(pl.init().pi_k_group_gemm_tile(C.byref(g), tile, None))
+    pl.sync()
+    got = y.download(np.uint32 if y_f32 else np.uint16)
+    assert not got[n * ldy:].any()                                            # nothing behind the last row
+    return got[:n * ldy].reshape(n, ldy), fetch(y, pl.F32 if y_f32 else pl.BF16, (n, ldy))
+
+
+def same(a, b, y_f32):
+    """Equal, and where the order of a float's operations is the compiler's (the GLU's), within one unit of the last place."""
+    assert np.abs(a.astype(np.int64) - b.astype(np.int64)).max() <= 1
+
+
+@pytest.mark.parametrize("rows,cols,kind,y_f32", [(129 + 7, 256, "plain", 0), (256, 320, "relu2", 0), (264, 256, "plain", 1), (384, 512, "glu", 0), (392, 256, "relu2", 0),
+                                                  (270, 256, "plain", 0), (528, 384, "glu", 0), (400, 256, "pair", 0), (300, 256, "glu", 0)])
+def test_experts_of_uneven_size(rows, cols, kind, y_f32):
+    rng = np.random.default_rng(rows + cols)
+    counts = [0, 1, 16, 63, 64, 65, 127, 128, 129, 300, 0, 193]
+    E, n, div = len(counts), sum(counts), 3
+    T = (n + div - 1) // div
+    W = rounded(rng.standard_normal((E, rows, cols)) / np.sqrt(cols))
+    x = rounded(rng.standard_normal((T, cols)))
+    perm = rng.permutation(T * div)[:n].astype(np.int32)
+    pw = rng.random(T * div).astype(np.float32)
+    off = np.concatenate([[0], np.cumsum(counts)])
+    glu = kind in ("glu", "pair")
+    ldy = ((rows // 2 if glu else rows) + 7) // 8 * 8
+    bufs = [store(W.reshape(-1, cols), pl.BF16), store(x, pl.BF16), i32(off), i32(perm), dev(pw)]
+    res = {}
+    for tile in (64, 128):
+        tl = np.array([(e, p) for e in range(E) for p in range(off[e], off[e + 1], tile)], np.int32)
+        tb, nb = i32(tl), i32([len(tl)])
+        g = group_args(W=bufs[0].ptr, w_gs=rows * cols, rows=rows, cols=cols, ldw=cols, n_group=E, x=bufs[1].ptr, ldx=cols, T=T, ldy=ldy, y_f32=y_f32, relu2=int(kind == "relu2"),
+                       alpha=1.25, off=bufs[2].ptr, gather=bufs[3].ptr, gather_div=div, tiles=tb.ptr, n_tiles=nb.ptr, max_tiles=len(tl) + 3, glu=int(glu), glu_limit=5.0, glu_gain=1.5,
+                       pair_w=bufs[4].ptr if kind == "pair" else None)
+        print(rows, cols, kind, tile, flush=True)
+        res[tile] = run(g, tile, n, ldy, y_f32)
+    same(res[64][0], res[128][0], y_f32)
+    if glu:
+        return                                                                # (the small tiles' own tests hold them against float64)
+    got = res[128][1]
+    for e in range(E):
+        s = slice(off[e], off[e + 1])
+        want = 1.25 * (x[perm[s] // div].astype(np.float64) @ W[e].T.astype(np.float64))
+        want = np.maximum(want, 0) ** 2 if kind == "relu2" else want
+        if want.size:
+            assert np.abs(got[s, :rows] - want).max() <= (1e-5 if y_f32 else 2.0 ** -7) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("groups,rows,cols,T", [(1, 512, 512, 2048), (3, 192, 256, 129), (2, 1024, 320, 40)])
+def test_groups_without_a_list(groups, rows, cols, T):
+    """Every group's own inputs, and more units than compute units."""
+    rng = np.random.default_rng(T)
+    W = rounded(rng.standard_normal((groups, rows, cols)) / np.sqrt(cols))
+    x = rounded(rng.standard_normal((T, groups, cols)))
+    wb, xb = store(W.reshape(-1, cols), pl.BF16), store(x.reshape(-1, cols), pl.BF16)
+    ldy = groups * rows
+    res = {}
+    for tile in (64, 128):
+        g = group_args(W=wb.ptr, w_gs=rows * cols, rows=rows, cols=cols, ldw=cols, n_group=groups, x=xb.ptr, x_gs=cols, ldx=groups * cols, T=T, y_gs=rows, ldy=ldy, alpha=1.0)
+        print(groups, rows, cols, T, tile, flush=True)
+        res[tile] = run(g, tile, T, ldy, 0)
+    same(res[64][0], res[128][0], 0)
+    want = np.einsum("tgc,grc->tgr", x.astype(np.float64), W.astype(np.float64)).reshape(T, ldy)
+    assert np.abs(res[128][1] - want).max() <= 2.0 ** -7 * np.abs(want).max()
