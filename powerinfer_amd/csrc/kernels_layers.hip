@@ -522,22 +522,34 @@ __device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int 
 // Measured (us; 128 x 128 tiles of GemmTile before): 64 experts of 192 tokens on average, 1408 x 4096: 301 -> 218, 4096 x 1408:
 // 307 -> 227 (weights alone: 123 at 6 TB/s); one group of 12288: 199 -> 144, 1 PFLOP/s; 16 experts of 128: 51 -> 45 and 38 -> 34.
 // ---------------------------------------------------------------------------------------------------------------------------------
-constexpr int kGwM = 256, kGwN = 128, kGwStages = 3, kGwStage = (kGwM + kGwN) * kGtRow, kGwTurn = 2048, kGwLds = kGwStages * kGwStage + 64 + 4 * kGwTurn;
-__global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int nx, int max_units) {
+constexpr int kGwM = 256, kGwN = 128, kGwStages = 3, kGwStage = (kGwM + kGwN) * kGtRow, kGwTurn = 2048, kGwLds = kGwStages * kGwStage + 128 + 4 * kGwTurn;
+// n_tiles: token tiles of a product without a list.  The units (token tile, 256 rows) are dealt out so that an XCD works through a contiguous
+// range of them: first the row tiles of more than 128 rows, then the shorter ones, which take half the time.  What does not fill the
+// XCD's workgroups once more at the end is cut into halves of 128 rows if that gives no workgroup two of them.
+__global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int n_tiles) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int tt = (g.T + kGwN - 1) / kGwN;
-    const int units = g.off ? *g.n_tiles * nx : max_units;
-    const int per = (units + 7) / 8, step = (int)gridDim.x / 8, end = min(((int)blockIdx.x % 8 + 1) * per, units);
-    int unit = (int)(blockIdx.x % 8) * per + (int)blockIdx.x / 8;
-    if (unit >= end) return;
+    if (g.off) n_tiles = *g.n_tiles;
+    const int nx = (g.rows + kGwM - 1) / kGwM, last = g.rows - (nx - 1) * kGwM, nl = last > kGwM / 2 ? nx : nx - 1;     // row tiles; those of more than half
+    const int xcd = (int)blockIdx.x % 8, slot = (int)blockIdx.x / 8, slots = (int)gridDim.x / 8;
+    const int per_long = (n_tiles * nl + 7) / 8, per_short = nl < nx ? (n_tiles + 7) / 8 : 0;
+    const int n_long = max(min(n_tiles * nl - xcd * per_long, per_long), 0), n_short = max(min(nl < nx ? n_tiles - xcd * per_short : 0, per_short), 0);
+    const int rounds = (n_long + n_short) / slots, rest = (n_long + n_short) % slots;
+    const bool halves = rest > 0 && 2 * rest <= slots;
+    // the c-th unit of this workgroup: its number among the XCD's, and for a half of one its first row
+    const int rest_unit = rounds * slots + (halves ? slot / 2 : slot), rest_row = halves ? slot % 2 * (kGwM / 2) : 0;
+    const int count = rounds + (slot < (halves ? 2 * rest : rest) && !(rest_row && rest_unit >= n_long) ? 1 : 0);
+    if (count == 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
     const int nk = g.cols / kGtBK;
     const bool whole = !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0;
-    struct Place { int grp, lo, n, row0; };
+    struct Place { int grp, lo, n, row0, rows; };
     Place * places = reinterpret_cast<Place *>(smem + kGwStages * kGwStage);      // of this unit and the three behind it, written by the first copying wave
-    auto place = [&](int u) {
+    auto place = [&](int c) {
         Place p;
-        const int tx = u % nx, ty = u / nx;
+        const int u = c < rounds ? c * slots + slot : rest_unit;
+        const int at = u < n_long ? xcd * per_long + u : xcd * per_short + u - n_long;
+        const int tx = u < n_long ? at % nl : nx - 1, ty = u < n_long ? at / nl : at;
         if (g.off) {
             const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
             p.grp = t.x; p.lo = t.y; p.n = g.off[p.grp + 1] - p.lo;
@@ -545,7 +557,8 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
             p.grp = ty / tt; p.lo = (ty % tt) * kGwN; p.n = g.T - p.lo;
         }
         p.n = min(p.n, kGwN);
-        p.row0 = tx * kGwM;
+        p.row0 = tx * kGwM + (c < rounds ? 0 : rest_row);
+        p.rows = min(g.rows - p.row0, c < rounds || !halves ? kGwM : kGwM / 2);
         return p;
     };
     if (wave >= 4) {
@@ -556,14 +569,14 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
         size_t vb[4];
         const unsigned char * fa, * fb;
         int k = 0, c = 0;
-        auto aim = [&](int u) {
-            const Place p = place(u);
+        auto aim = [&]() {
+            const Place p = place(c);
             if (w == 0 && lane == 0) places[c & 3] = p;
             ++c;
             fa = (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs);
             fb = (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs));
 #pragma unroll
-            for (int j = 0; j < 8; ++j) va[j] = (uint32_t)min(p.row0 + 64 * w + 8 * j + (lane >> 3), g.rows - 1) * (uint32_t)(g.ldw * 2) + piece;
+            for (int j = 0; j < 8; ++j) va[j] = (uint32_t)(p.row0 + min(64 * w + 8 * j + (lane >> 3), p.rows - 1)) * (uint32_t)(g.ldw * 2) + piece;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int at = p.lo + min(32 * w + 8 * j + (lane >> 3), p.n - 1);
@@ -578,11 +591,10 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
 #pragma unroll
             for (int j = 0; j < 4; ++j) __builtin_amdgcn_global_load_lds((gptr)(fb + (size_t)k * kGtRow + vb[j]), (lptr)(stage + (kGwM + 32 * w + 8 * j) * kGtRow), 16, 0, 0);
             if (++k < nk) return;
-            if (unit + step < end) { unit += step; k = 0; aim(unit); } else k = nk - 1;
+            if (c < count) { k = 0; aim(); } else k = nk - 1;
         };
-        int total = 0;
-        for (int u = unit; u < end; u += step) total += nk;
-        aim(unit);
+        const int total = count * nk;
+        aim();
         for (int st = 0; st < kGwStages; ++st) copy_stage(smem + st * kGwStage);
         __builtin_amdgcn_s_waitcnt(0x4078);                         // vmcnt(24): the first stage; lgkmcnt(0): its place
         __builtin_amdgcn_s_barrier();
@@ -597,7 +609,7 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
         __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0): no copy may arrive in LDS that is no longer this workgroup's
         return;
     }
-    unsigned char * turn = smem + kGwStages * kGwStage + 64 + wave * kGwTurn;
+    unsigned char * turn = smem + kGwStages * kGwStage + 128 + wave * kGwTurn;
     int cb = 0;                                                    // the stage that is being multiplied
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -660,11 +672,12 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
         else if (whole) group_store_turned<kStorePlain>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
         else group_store(g, p.grp, p.lo, p.n, p.row0 + rb, tb, q, i, acc);
     };
-    for (int c = 0; unit < end; unit += step, ++c) {
+    for (int c = 0; c < count; ++c) {
         const int * pl = reinterpret_cast<const int *>(places + (c & 3));
         Place p;
         p.grp = __builtin_amdgcn_readfirstlane(pl[0]); p.lo = __builtin_amdgcn_readfirstlane(pl[1]); p.n = __builtin_amdgcn_readfirstlane(pl[2]); p.row0 = __builtin_amdgcn_readfirstlane(pl[3]);
-        if (g.rows - p.row0 <= 128) run(std::integral_constant<int, 4>{}, p, 64 * (wave & 1), 64 * (wave >> 1));
+        p.rows = __builtin_amdgcn_readfirstlane(pl[4]);
+        if (p.rows <= 128) run(std::integral_constant<int, 4>{}, p, 64 * (wave & 1), 64 * (wave >> 1));
         else if (p.n <= 64) run(std::integral_constant<int, 4>{}, p, 64 * wave, 0);
         else run(std::integral_constant<int, 8>{}, p, 128 * (wave & 1), 64 * (wave >> 1));
     }
@@ -676,11 +689,10 @@ int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
         PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&group_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
         raised = true;
     }
-    const int nx = (g.rows + kGwM - 1) / kGwM;
-    const long long units = (long long)nx * (g.off ? g.max_tiles : (long long)g.n_group * ((g.T + kGwN - 1) / kGwN));
+    const long long tiles = g.off ? g.max_tiles : (long long)g.n_group * ((g.T + kGwN - 1) / kGwN), units = tiles * ((g.rows + kGwM - 1) / kGwM);
     if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: too many tiles");
-    const long long blocks = std::min((units + 7) / 8 * 8, (long long)256);
-    hipLaunchKernelGGL(group_wide_kernel, dim3((unsigned)blocks), dim3(512), kGwLds, st, g, nx, (int)units);
+    const long long blocks = std::min((2 * units + 7) / 8 * 8, (long long)256);
+    hipLaunchKernelGGL(group_wide_kernel, dim3((unsigned)blocks), dim3(512), kGwLds, st, g, (int)tiles);
     return pi::check_launch("pi_k_group_gemm_tile");
 }
 
