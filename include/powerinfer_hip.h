@@ -365,6 +365,11 @@ PI_API int pi_k_batch_sparse_ffn_q4(const float * logits, int T, int ff, float t
                                     const void * gate_quants, const void * gate_scales, const void * down_quants, const void * down_scales, int cols,
                                     const void * xq, const float * xd, const int32_t * xs8, int epilogue, const float * add1, const float * add2, float * out,
                                     float * h, float * hq, int32_t * union_rows, int32_t * n_union, pi_workspace * ws, pi_stream_t stream);
+/* The same from the matrices themselves (gate_f16 null: relu(up)): both products of a chunk's normalised fp16 input xn_f16[T][cols] and h in one
+ * kernel.  Rows of up and gate [ff][cols]; logits [T][ff]; all operands 16-byte aligned. */
+PI_API int pi_k_ffn_wide_supported(int ff, int cols);
+PI_API int pi_k_ffn_wide_f16(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, float threshold,
+                             void * h_f16, pi_stream_t stream);
 PI_API int pi_k_ffn_h_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream);
 PI_API int pi_k_transpose_f16(const void * in_f16, int rows, int cols, void * out_f16, pi_stream_t stream);
 

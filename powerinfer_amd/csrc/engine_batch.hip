@@ -456,14 +456,21 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     }
     PI_TRY(chunk_gemm(m, fc1.dev, r, d, b->xp16, T, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
     PI_TRY(chunk_gemm(m, fc2.dev, ff, r, b->hid16, T, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
-    PI_TRY(chunk_weight(m, b, il, PI_T_FFN_UP, ff, d, &W));
-    PI_TRY(chunk_gemm(m, W, ff, d, ffn_x, T, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
-    if (!falcon) {
+    // F16 layers whole on the device: up, gate and h in one kernel.  Not for few tokens of large matrices, which the library's plans stream faster
+    // (17 / 64 / 128 tokens, us, library and one kernel: 11008 x 4096 45 / 60 / 70 and 45 / 46 / 49; 13824 x 5120 58 / 74 / 95 and 79 / 86 / 95)
+    const bool one_kernel = m->gemm_lib && up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(ff, d) &&
+                            (T > 96 || (long long)ff * d <= 48LL << 20);
+    if (!one_kernel) {
+        PI_TRY(chunk_weight(m, b, il, PI_T_FFN_UP, ff, d, &W));
+        PI_TRY(chunk_gemm(m, W, ff, d, ffn_x, T, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
+    }
+    if (!falcon && !one_kernel) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_GATE, ff, d, &W));
         PI_TRY(chunk_gemm(m, W, ff, d, ffn_x, T, PI_EPI_NONE, nullptr, nullptr, b->gate_out, nullptr));
     }
-    if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
-    else                           PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
+    if (one_kernel) PI_TRY(pi_k_ffn_wide_f16(up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, b->pred_logits, hp.sparse_threshold, b->h16, st));
+    else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
+    else PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     const void * Wd = m->down_rows[il];
     if (!Wd) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_DOWN_T, ff, d, &W));

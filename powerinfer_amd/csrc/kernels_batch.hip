@@ -1,6 +1,6 @@
 // Steps of several tokens: 2..16 sequences in lockstep or a prompt chunk of one sequence.  Dense and sparse mat-muls on the matrix
 // cores, the union of the tokens' active rows, norm + rounding passes, Q4_0 expansion and row assembly for prompt chunks.
-#include "gemm_tile.hpp"
+#include "gemm_wide.hpp"
 #include "mixers.hpp"
 
 namespace {
@@ -362,6 +362,67 @@ __global__ void ffn_h_f16_kernel(const float * __restrict__ up, const float * __
         h16[i] = __float2half_rn(h);
     }
 }
+// The same straight from the matrices, in the large tiles of gemm_wide: a tile holds 64 rows of up, the 64 rows of gate of the same neurons and
+// twice that again (PAIRS), or 256 rows of up alone; a lane then holds both factors of its neurons, and neither of them (90 MB each
+// for 2048 tokens of 11008 neurons) goes to memory.  The products' sums are formed in 32-column steps in fp32, as in the tiles of
+// the dense mat-mul.  11008 x 4096 twice, us (two library products and ffn_h_f16_kernel before): 2047 tokens 675 -> 327 (1.13
+// PFLOP/s), 1024 tokens 222 -> 174, 256 tokens 109 -> 61, 64 tokens 60 -> 46; 32768 x 8192 alone, 2047 tokens: 1100 -> 941.
+template <bool PAIRS> struct FfnProduct {
+    static constexpr bool kPairs = PAIRS;
+    const __half * up, * gate, * x; const float * logits; float thr; __half * h16;
+    int ff, cols, T, nk;
+    __device__ __forceinline__ WidePlace place(const WideDeal & deal, int c) const {
+        WidePlace p;
+        int ty;
+        deal.unit(c, ty, p.row0, p.rows);
+        p.grp = 0; p.lo = ty * kGwN; p.n = min(T - p.lo, kGwN);
+        return p;
+    }
+    __device__ __forceinline__ const unsigned char * base_a(const WidePlace &, int w) const { return (const unsigned char *)(PAIRS && (w & 1) ? gate : up); }
+    __device__ __forceinline__ const unsigned char * base_b(const WidePlace & p) const { return (const unsigned char *)(x + (size_t)p.lo * cols); }
+    __device__ __forceinline__ uint32_t off_a(const WidePlace & p, int r) const { return (uint32_t)(PAIRS ? p.row0 / 2 + r / 128 * 64 + r % 64 : p.row0 + r) * (uint32_t)(cols * 2); }
+    __device__ __forceinline__ size_t off_b(const WidePlace &, int r) const { return (size_t)r * cols * 2; }
+    template <int MT> __device__ __forceinline__ void store(const WidePlace & p, int rb, int tb, const pi_f4 (&acc)[MT][4], unsigned char * turn, int lane) const {
+        constexpr int MO = PAIRS ? MT / 2 : MT;
+        asm volatile("" : "+v"(lane));                 // what follows is computed here, not kept in registers across the products
+        const int i = lane & 15, q = lane >> 4, n0 = PAIRS ? p.row0 / 2 + rb / 128 * 64 + rb % 128 : p.row0 + rb;          // this wave's first neuron
+        const int left = ff - n0;                      // (a multiple of 64: whole tiles of 16 neurons or none)
+        float4 lg[2][MO];
+        auto fetch = [&](int nn) {
+            const float * l = logits + (size_t)(p.lo + min(tb + nn * 16 + i, p.n - 1)) * ff + n0 + 4 * q;
+#pragma unroll
+            for (int m = 0; m < MO; ++m) lg[nn & 1][m] = *reinterpret_cast<const float4 *>(l + (m * 16 < left ? m * 16 : 0));
+        };
+        if (left <= 0) return;
+        fetch(0);
+#pragma unroll
+        for (int nn = 0; nn < 4; ++nn) {
+            if (nn < 3) fetch(nn + 1);
+            uint2 out[MO];
+#pragma unroll
+            for (int m = 0; m < MO; ++m) {
+                const float l[4] = {lg[nn & 1][m].x, lg[nn & 1][m].y, lg[nn & 1][m].z, lg[nn & 1][m].w};
+                __half h[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float u = acc[m][nn][r], v = PAIRS ? __fmul_rn(fmaxf(acc[(m + MO) % MT][nn][r], 0.0f), u) : fmaxf(u, 0.0f);
+                    h[r] = __float2half_rn(!(l[r] < thr) ? v : 0.0f);
+                }
+                out[m] = __builtin_bit_cast(uint2, h);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            store_turned<8>(out, turn, lane, [&](int t, int piece) -> void * {
+                const int to = tb + nn * 16 + t;
+                return to < p.n && piece * 8 < left ? h16 + (size_t)(p.lo + to) * ff + n0 + piece * 8 : nullptr;
+            });
+        }
+    }
+};
+template <bool PAIRS> __global__ __launch_bounds__(512, 1) void ffn_wide_kernel(FfnProduct<PAIRS> prod) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    gemm_wide<__half>(prod, WideDeal(PAIRS ? 2 * prod.ff : prod.ff, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
+}
+
 // out[c][r] = in[r][c] for an fp16 matrix [rows][cols] (32 x 32 tiles through LDS)
 __global__ void transpose_f16_kernel(const __half * __restrict__ in, int rows, int cols, __half * __restrict__ out) {
     __shared__ __half t[32][33];
@@ -1179,6 +1240,28 @@ int pi_k_ffn_h_f16(const float * up, const float * gate, const float * logits, f
     hipLaunchKernelGGL(ffn_h_f16_kernel, dim3(1024), dim3(256), 0, (hipStream_t)stream, up, gate, logits, threshold, (size_t)T * ff, (__half *)h_f16, 0);
     return pi::check_launch("pi_k_ffn_h_f16");
 }
+int pi_k_ffn_wide_supported(int ff, int cols) { return ff > 0 && ff % 128 == 0 && cols >= 4 * kGtBK && cols % kGtBK == 0 && (long long)ff * cols < (1LL << 31); }
+
+int pi_k_ffn_wide_f16(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, float threshold, void * h_f16, pi_stream_t stream) {
+    if (!up_f16 || !xn_f16 || !logits || !h_f16 || T <= 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: bad arguments");
+    if (!pi_k_ffn_wide_supported(ff, cols)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_ffn_wide_f16: ff must be a multiple of 128, cols a multiple of 64 and at least 256");
+    if ((((uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)xn_f16 | (uintptr_t)logits | (uintptr_t)h_f16) & 15) != 0)
+        return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: operands must be 16-byte aligned");
+    const long long units = (long long)(((gate_f16 ? 2 * ff : ff) + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
+    if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: too many tiles");
+    static bool raised = false;
+    if (!raised) {
+        PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ffn_wide_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
+        PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ffn_wide_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
+        raised = true;
+    }
+#define PI_FFN_WIDE(P) hipLaunchKernelGGL(ffn_wide_kernel<P>, dim3(wide_blocks(units)), dim3(512), kGwLds, (hipStream_t)stream, \
+    FfnProduct<P>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, logits, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK})
+    if (gate_f16) PI_FFN_WIDE(true); else PI_FFN_WIDE(false);
+#undef PI_FFN_WIDE
+    return pi::check_launch("pi_k_ffn_wide_f16");
+}
+
 int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream) {
     if (!up || !logits || !h_f16 || T <= 0 || ff <= 0 || ff % 64) return pi::fail(PI_E_ARG, "pi_k_ffn_h_q8_f16: n_ff must be a multiple of 64");
     hipLaunchKernelGGL(ffn_h_f16_kernel, dim3(1024), dim3(256), 0, (hipStream_t)stream, up, gate, logits, threshold, (size_t)T * ff, (__half *)h_f16, 1);

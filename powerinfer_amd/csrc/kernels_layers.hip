@@ -1,7 +1,7 @@
 // Operators of the models that are described layer by layer, apart from attention: embedding + norm, the pair of norms of a parallel
 // layer, grouped mat-muls (heads of a latent attention, experts), rotation angles, expert choice, and the sum that closes a layer.
 // Templated on the storage of activations: bf16 (matrix cores on bf16 operands, fp32 accumulation) or fp32.
-#include "gemm_tile.hpp"
+#include "gemm_wide.hpp"
 #include "layer_types.hpp"
 #include "mixers.hpp"
 #include "route.hpp"
@@ -452,24 +452,18 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192
     group_store(g, grp, lo, n, row0 + wm * WM, wn * WN, q, i, acc);
 }
 
-// The same through LDS, where outputs come in whole pieces of 16 bytes: the lanes' quads of rows, written as they are, are runs of 32 bytes a
-// token (8 us for 256 x 128 outputs of a workgroup); eight tokens at a time, turned in 2 KB of the wave's own, leave in runs of up to 256
-// bytes.  One kind of epilogue at a time, as the code runs once a unit and its instructions come from L2 each time.
+// The same through LDS (store_turned), one kind of epilogue at a time: the code runs once a unit and its instructions come from L2 each time.
 enum { kStorePlain, kStoreRelu2, kStoreGlu };
 template <int KIND, int MT, int NT>
 __device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int grp, int lo, int n, int row0, int tok0, int lane, const pi_f4 (&acc)[MT][NT], unsigned char * turn) {
-    constexpr int kRow = KIND == kStoreGlu ? MT * 16 : MT * 32, kPieces = kRow / 16, kToks = 64 / kPieces;      // bytes and pieces of a token, tokens a store instruction takes
     asm volatile("" : "+v"(lane));                     // what follows is computed here, not kept in registers across the products
-    const int i = lane & 15, q = lane >> 4;
     const float one = g.glu_plain_up ? 0.0f : 1.0f;
     const int out0 = KIND == kStoreGlu ? row0 / 2 : row0, outs = KIND == kStoreGlu ? g.rows / 2 : g.rows;
-    const int piece = lane % kPieces, first = lane / kPieces;
 #pragma unroll
     for (int nn = 0; nn < NT; ++nn) {
-        const int tok = tok0 + nn * 16 + i;
-        const float alpha = g.pair_w ? g.alpha * g.pair_w[g.gather[lo + min(tok, n - 1)]] : g.alpha;
+        const float alpha = g.pair_w ? g.alpha * g.pair_w[g.gather[lo + min(tok0 + nn * 16 + (lane & 15), n - 1)]] : g.alpha;
         __builtin_amdgcn_sched_barrier(0);
-        uint2 out[MT];                                              // this lane's four rows (Glu: two outputs) of every 16
+        uint2 out[MT];
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             if constexpr (KIND == kStoreGlu) {
@@ -487,69 +481,23 @@ __device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int 
                 out[m] = __builtin_bit_cast(uint2, b);
             }
         }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {                               // tokens 0 .. 7 of the sixteen, then 8 .. 15
-            unsigned char * mine = turn + (i & 7) * kRow;
-            if ((i >> 3) == h) {
-#pragma unroll
-                for (int m = 0; m < MT; ++m) {
-                    if constexpr (KIND == kStoreGlu) *reinterpret_cast<uint32_t *>(mine + (m ^ (i & 7) % kPieces) * 16 + q * 4) = out[m].x;
-                    else *reinterpret_cast<uint2 *>(mine + ((2 * m + (q >> 1)) ^ ((i & 7) % kPieces)) * 16 + (q & 1) * 8) = out[m];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            constexpr int kTurnWaves = (8 * kPieces + 63) / 64;
-#pragma unroll
-            for (int t0 = 0; t0 < kTurnWaves; ++t0) {
-                const int t = t0 * kToks + first, to = tok0 + nn * 16 + 8 * h + t;
-                const pi_u32x4 v = *reinterpret_cast<const pi_u32x4 *>(turn + (t & 7) * kRow + (piece ^ ((t & 7) % kPieces)) * 16);
-                if (t < 8 && to < n && out0 + piece * 8 < outs)
-                    *reinterpret_cast<pi_u32x4 *>((bf16 *)g.y + (g.off ? 0 : (size_t)grp * g.y_gs) + (size_t)(lo + to) * g.ldy + out0 + piece * 8) = v;
-            }
-        }
+        store_turned<KIND == kStoreGlu ? 4 : 8>(out, turn, lane, [&](int t, int piece) -> void * {
+            const int to = tok0 + nn * 16 + t;
+            return to < n && out0 + piece * 8 < outs ? (bf16 *)g.y + (g.off ? 0 : (size_t)grp * g.y_gs) + (size_t)(lo + to) * g.ldy + out0 + piece * 8 : nullptr;
+        });
     }
 }
 
-// ---------------------------------------------------------------------------------------------------------------------------------
-// The same product in large tiles: 256 rows x 128 tokens, one workgroup per compute unit that stays for all of its units.  Four waves
-// multiply (128 x 64 outputs each), four copy: a stage of 64 columns goes from memory straight to LDS, three stages deep and on
-// into the next unit, and a copy that has to wait for the memory's queues holds up no matrix instruction (copying from the
-// multiplying waves themselves: 238 us for the first product below).  A multiplying wave reads the fragments of a stage's second 32 columns
-// under the products of the first and those of the next stage's first 32 under the products of the second, with the one barrier
-// of a stage in between: behind it the next stage is whole and the present one is free to be copied over.  LDS rows and swizzle are GemmTile's; a
-// copy's 64 lanes bring eight rows of 128 bytes and take the swizzle on the side they read from.  Where half a tile or less is
-// wanted (128 rows, 64 tokens) the four waves share that half, 64 x 64 outputs each.  The sums are formed in GemmTile's order.
-// Measured (us; 128 x 128 tiles of GemmTile before): 64 experts of 192 tokens on average, 1408 x 4096: 301 -> 218, 4096 x 1408:
-// 307 -> 227 (weights alone: 123 at 6 TB/s); one group of 12288: 199 -> 144, 1 PFLOP/s; 16 experts of 128: 51 -> 45 and 38 -> 34.
-// ---------------------------------------------------------------------------------------------------------------------------------
-constexpr int kGwM = 256, kGwN = 128, kGwStages = 3, kGwStage = (kGwM + kGwN) * kGtRow, kGwTurn = 2048, kGwLds = kGwStages * kGwStage + 128 + 4 * kGwTurn;
-// n_tiles: token tiles of a product without a list.  The units (token tile, 256 rows) are dealt out so that an XCD works through a contiguous
-// range of them: first the row tiles of more than 128 rows, then the shorter ones, which take half the time.  What does not fill the
-// XCD's workgroups once more at the end is cut into halves of 128 rows if that gives no workgroup two of them.
-__global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int n_tiles) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int tt = (g.T + kGwN - 1) / kGwN;
-    if (g.off) n_tiles = *g.n_tiles;
-    const int nx = (g.rows + kGwM - 1) / kGwM, last = g.rows - (nx - 1) * kGwM, nl = last > kGwM / 2 ? nx : nx - 1;     // row tiles; those of more than half
-    const int xcd = (int)blockIdx.x % 8, slot = (int)blockIdx.x / 8, slots = (int)gridDim.x / 8;
-    const int per_long = (n_tiles * nl + 7) / 8, per_short = nl < nx ? (n_tiles + 7) / 8 : 0;
-    const int n_long = max(min(n_tiles * nl - xcd * per_long, per_long), 0), n_short = max(min(nl < nx ? n_tiles - xcd * per_short : 0, per_short), 0);
-    const int rounds = (n_long + n_short) / slots, rest = (n_long + n_short) % slots;
-    const bool halves = rest > 0 && 2 * rest <= slots;
-    // the c-th unit of this workgroup: its number among the XCD's, and for a half of one its first row
-    const int rest_unit = rounds * slots + (halves ? slot / 2 : slot), rest_row = halves ? slot % 2 * (kGwM / 2) : 0;
-    const int count = rounds + (slot < (halves ? 2 * rest : rest) && !(rest_row && rest_unit >= n_long) ? 1 : 0);
-    if (count == 0) return;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
-    const int nk = g.cols / kGtBK;
-    const bool whole = !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0;
-    struct Place { int grp, lo, n, row0, rows; };
-    Place * places = reinterpret_cast<Place *>(smem + kGwStages * kGwStage);      // of this unit and the three behind it, written by the first copying wave
-    auto place = [&](int c) {
-        Place p;
-        const int u = c < rounds ? c * slots + slot : rest_unit;
-        const int at = u < n_long ? xcd * per_long + u : xcd * per_short + u - n_long;
-        const int tx = u < n_long ? at % nl : nx - 1, ty = u < n_long ? at / nl : at;
+// the same product in the large tiles of gemm_wide
+struct GroupProduct {
+    static constexpr bool kPairs = false;
+    const pi_group_gemm & g;
+    int nk, tt;                                                     // tt: token tiles of a group without a list
+    bool whole;
+    __device__ __forceinline__ WidePlace place(const WideDeal & deal, int c) const {
+        WidePlace p;
+        int ty;
+        deal.unit(c, ty, p.row0, p.rows);
         if (g.off) {
             const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
             p.grp = t.x; p.lo = t.y; p.n = g.off[p.grp + 1] - p.lo;
@@ -557,130 +505,24 @@ __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int
             p.grp = ty / tt; p.lo = (ty % tt) * kGwN; p.n = g.T - p.lo;
         }
         p.n = min(p.n, kGwN);
-        p.row0 = tx * kGwM + (c < rounds ? 0 : rest_row);
-        p.rows = min(g.rows - p.row0, c < rounds || !halves ? kGwM : kGwM / 2);
         return p;
-    };
-    if (wave >= 4) {
-        // A wave that copies.  Of each stage eight times eight rows of W and four times eight of x are its own, each 128 bytes; lane l brings
-        // the piece that belongs at place l % 8 of row l / 8
-        const int w = wave - 4, piece = ((lane & 7) ^ (lane >> 3)) * 16;
-        uint32_t va[8];
-        size_t vb[4];
-        const unsigned char * fa, * fb;
-        int k = 0, c = 0;
-        auto aim = [&]() {
-            const Place p = place(c);
-            if (w == 0 && lane == 0) places[c & 3] = p;
-            ++c;
-            fa = (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs);
-            fb = (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs));
-#pragma unroll
-            for (int j = 0; j < 8; ++j) va[j] = (uint32_t)(p.row0 + min(64 * w + 8 * j + (lane >> 3), p.rows - 1)) * (uint32_t)(g.ldw * 2) + piece;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int at = p.lo + min(32 * w + 8 * j + (lane >> 3), p.n - 1);
-                vb[j] = (size_t)(g.gather ? g.gather[at] / g.gather_div : at) * (size_t)g.ldx * 2 + piece;
-            }
-        };
-        typedef const __attribute__((address_space(1))) void * gptr;
-        typedef __attribute__((address_space(3))) void * lptr;
-        auto copy_stage = [&](unsigned char * stage) {             // past the last unit the last stage is copied again, and not used
-#pragma unroll
-            for (int j = 0; j < 8; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + (size_t)k * kGtRow + va[j]), (lptr)(stage + (64 * w + 8 * j) * kGtRow), 16, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) __builtin_amdgcn_global_load_lds((gptr)(fb + (size_t)k * kGtRow + vb[j]), (lptr)(stage + (kGwM + 32 * w + 8 * j) * kGtRow), 16, 0, 0);
-            if (++k < nk) return;
-            if (c < count) { k = 0; aim(); } else k = nk - 1;
-        };
-        const int total = count * nk;
-        aim();
-        for (int st = 0; st < kGwStages; ++st) copy_stage(smem + st * kGwStage);
-        __builtin_amdgcn_s_waitcnt(0x4078);                         // vmcnt(24): the first stage; lgkmcnt(0): its place
-        __builtin_amdgcn_s_barrier();
-        for (int t = 0, cb = 0; t < total; ++t) {
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(0x007C);                     // vmcnt(12): the stage after t; lgkmcnt(0): a place
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            copy_stage(smem + cb * kGwStage);
-            cb = cb == kGwStages - 1 ? 0 : cb + 1;
-        }
-        __builtin_amdgcn_s_waitcnt(0x0F70);                         // vmcnt(0): no copy may arrive in LDS that is no longer this workgroup's
-        return;
     }
-    unsigned char * turn = smem + kGwStages * kGwStage + 128 + wave * kGwTurn;
-    int cb = 0;                                                    // the stage that is being multiplied
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const int koff[2] = {(q ^ (i & 7)) * 16, ((4 + q) ^ (i & 7)) * 16};
-    auto run = [&](auto mt, const Place & p, int rb, int tb) {      // rows rb .. and tokens tb .. of the tile are this wave's
-        constexpr int MT = decltype(mt)::value;
-        pi_f4 acc[MT][4];
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int n = 0; n < 4; ++n) acc[m][n] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
-        pi_u32x4 f0a[MT], f0b[4], f1a[MT], f1b[4];
-        const int oa = (rb + i) * kGtRow, ob = (kGwM + tb + i) * kGtRow;
-        auto ld = [&](int stage, int off) { return *reinterpret_cast<const pi_u32x4 *>(smem + stage * kGwStage + off); };
-#pragma unroll
-        for (int m = 0; m < MT; ++m) f0a[m] = ld(cb, oa + koff[0] + m * 16 * kGtRow);
-#pragma unroll
-        for (int n = 0; n < 4; ++n) f0b[n] = ld(cb, ob + koff[0] + n * 16 * kGtRow);
-        // a group: the four MFMAs of one fragment of W.  A phase's reads follow its first RD groups' MFMAs: they never stand before an MFMA
-        // that waits for older ones, and the last groups cover their latency
-        constexpr int RD = MT / 2, RA = MT / RD, RB = 4 / RD;
-        for (int kt = 0; kt < nk; ++kt) {
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-#pragma unroll
-                for (int n = 0; n < 4; ++n) acc[m][n] = mma16<bf16>(f0a[m], f0b[n], acc[m][n]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (m < RD) {
-#pragma unroll
-                    for (int r = 0; r < RB; ++r) f1b[RB * m + r] = ld(cb, ob + koff[1] + (RB * m + r) * 16 * kGtRow);
-#pragma unroll
-                    for (int r = 0; r < RA; ++r) f1a[RA * m + r] = ld(cb, oa + koff[1] + (RA * m + r) * 16 * kGtRow);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // the next stage has arrived (two more are on their way), and nobody reads this one any more
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(0xC07F);                     // lgkmcnt(0)
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            cb = cb == kGwStages - 1 ? 0 : cb + 1;
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-#pragma unroll
-                for (int n = 0; n < 4; ++n) acc[m][n] = mma16<bf16>(f1a[m], f1b[n], acc[m][n]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (m < RD) {
-#pragma unroll
-                    for (int r = 0; r < RB; ++r) f0b[RB * m + r] = ld(cb, ob + koff[0] + (RB * m + r) * 16 * kGtRow);
-#pragma unroll
-                    for (int r = 0; r < RA; ++r) f0a[RA * m + r] = ld(cb, oa + koff[0] + (RA * m + r) * 16 * kGtRow);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        }
+    __device__ __forceinline__ const unsigned char * base_a(const WidePlace & p, int) const { return (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs); }
+    __device__ __forceinline__ const unsigned char * base_b(const WidePlace & p) const { return (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs)); }
+    __device__ __forceinline__ uint32_t off_a(const WidePlace & p, int r) const { return (uint32_t)(p.row0 + r) * (uint32_t)(g.ldw * 2); }
+    __device__ __forceinline__ size_t off_b(const WidePlace & p, int r) const { return (size_t)(g.gather ? g.gather[p.lo + r] / g.gather_div : p.lo + r) * (size_t)g.ldx * 2; }
+    template <int MT> __device__ __forceinline__ void store(const WidePlace & p, int rb, int tb, const pi_f4 (&acc)[MT][4], unsigned char * turn, int lane) const {
         if (whole && g.glu) group_store_turned<kStoreGlu>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
         else if (whole && g.relu2) group_store_turned<kStoreRelu2>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
         else if (whole) group_store_turned<kStorePlain>(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane, acc, turn);
-        else group_store(g, p.grp, p.lo, p.n, p.row0 + rb, tb, q, i, acc);
-    };
-    for (int c = 0; c < count; ++c) {
-        const int * pl = reinterpret_cast<const int *>(places + (c & 3));
-        Place p;
-        p.grp = __builtin_amdgcn_readfirstlane(pl[0]); p.lo = __builtin_amdgcn_readfirstlane(pl[1]); p.n = __builtin_amdgcn_readfirstlane(pl[2]); p.row0 = __builtin_amdgcn_readfirstlane(pl[3]);
-        p.rows = __builtin_amdgcn_readfirstlane(pl[4]);
-        if (p.rows <= 128) run(std::integral_constant<int, 4>{}, p, 64 * (wave & 1), 64 * (wave >> 1));
-        else if (p.n <= 64) run(std::integral_constant<int, 4>{}, p, 64 * wave, 0);
-        else run(std::integral_constant<int, 8>{}, p, 128 * (wave & 1), 64 * (wave >> 1));
+        else group_store(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane >> 4, lane & 15, acc);
     }
+};
+// n_tiles: token tiles of a product without a list
+__global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int n_tiles) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const GroupProduct prod{g, g.cols / kGtBK, (g.T + kGwN - 1) / kGwN, !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0};
+    gemm_wide<bf16>(prod, WideDeal(g.rows, g.off ? *g.n_tiles : n_tiles, g.n_group > 1 ? 1 : kGwBand), smem);       // (bands of experts' tiles measured no better)
 }
 
 int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
@@ -691,8 +533,7 @@ int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
     }
     const long long tiles = g.off ? g.max_tiles : (long long)g.n_group * ((g.T + kGwN - 1) / kGwN), units = tiles * ((g.rows + kGwM - 1) / kGwM);
     if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: too many tiles");
-    const long long blocks = std::min((2 * units + 7) / 8 * 8, (long long)256);
-    hipLaunchKernelGGL(group_wide_kernel, dim3((unsigned)blocks), dim3(512), kGwLds, st, g, (int)tiles);
+    hipLaunchKernelGGL(group_wide_kernel, dim3(wide_blocks(units)), dim3(512), kGwLds, st, g, (int)tiles);
     return pi::check_launch("pi_k_group_gemm_tile");
 }
 

@@ -78,3 +78,27 @@ def test_groups_without_a_list(groups, rows, cols, T):
     same(res[64][0], res[128][0], 0)
     want = np.einsum("tgc,grc->tgr", x.astype(np.float64), W.astype(np.float64)).reshape(T, ldy)
     assert np.abs(res[128][1] - want).max() <= 2.0 ** -7 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("ff,cols,T", [(128, 256, 1), (384, 320, 64), (256, 512, 65), (640, 256, 129), (2176, 256, 300)])
+def test_sparse_ffn_of_a_chunk(ff, cols, T, gated):
+    """Up, gate, mask and product in one kernel: h within fp16's rounding of float64 where the fp32 sums' own error leaves it (products of
+    `cols` terms of fp16 values: 2^-11 of h and 1e-5 of the largest), exact zeros where the predictor says so, threshold and NaN included."""
+    L, rng = pl.init(), np.random.default_rng(ff + T)
+    up, gate, x = ((rng.standard_normal(s) / np.sqrt(s[1]) ** (s[0] != T)).astype(np.float16) for s in ((ff, cols), (ff, cols), (T, cols)))
+    lg = rng.standard_normal((T, ff)).astype(np.float32)
+    lg[0, :3] = [0.25, np.nan, -np.inf]
+    b = [dev(a) for a in (up, gate, x, lg)]
+    h = pl.DevBuf(2 * T * ff + 64)
+    pl.check(L.pi_memset(h.ptr, 0xAB, h.nbytes))
+    print(ff, cols, T, gated, flush=True)
+    pl.check(L.pi_k_ffn_wide_f16(b[0].ptr, b[1].ptr if gated else None, ff, cols, b[2].ptr, T, b[3].ptr, 0.25, h.ptr, None))
+    pl.sync()
+    raw = h.download(np.float16)
+    assert (raw[T * ff:].view(np.uint16) == 0xABAB).all()
+    got = raw[:T * ff].reshape(T, ff).astype(np.float64)
+    u, g = (x.astype(np.float64) @ w.T.astype(np.float64) for w in (up, gate))
+    want = np.where(~(lg < 0.25), np.maximum(g, 0) * u if gated else np.maximum(u, 0), 0)
+    assert (got[lg < 0.25] == 0).all()
+    assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 1e-5 * np.abs(want).max() + 2.0 ** -25).all()
