@@ -66,9 +66,36 @@ __device__ __forceinline__ double pi_wave_sum_f64(double v) {
     const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
+// (a lane outside a step's rows keeps its own value)
+template <int CTRL, int ROW_MASK> __device__ __forceinline__ float pi_dpp_max(float v) {
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROW_MASK, 0xF, false)));
+}
 __device__ __forceinline__ float pi_wave_max(float v) {
-#pragma unroll
-    for (int o = PI_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, PI_WAVE));
+    v = pi_dpp_max<PI_DPP_XOR1, 0xF>(v);
+    v = pi_dpp_max<PI_DPP_XOR2, 0xF>(v);
+    v = pi_dpp_max<PI_DPP_HALF_MIRROR, 0xF>(v);
+    v = pi_dpp_max<PI_DPP_MIRROR, 0xF>(v);
+    v = pi_dpp_max<PI_DPP_BCAST15, 0xA>(v);
+    v = pi_dpp_max<PI_DPP_BCAST31, 0xC>(v);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+// The sum over the n lanes (n = 2^k) of an aligned group, in every one of them, with the pairs of the butterfly v += v[lane ^ n / 2], ..,
+// v[lane ^ 1]: 16 and 8 lanes by lane permutations of the VALU (a rotation by n / 4 inside a group of equal halves is the butterfly's
+// partner), other sizes (N = 0) through the LDS crossbar.
+template <int N> __device__ __forceinline__ float pi_group_sum(float v, int n) {
+    if constexpr (N == 16) {
+        v += pi_dpp_f32<0x128, 0xF>(v);                             // row_ror:8
+        v += pi_dpp_f32<0x124, 0xF>(v);                             // row_ror:4
+    } else if constexpr (N == 8) {
+        const int up = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xF, 0x5, false);        // row_shl:4, lanes 0..3 and 8..11 take lane + 4
+        v += __int_as_float(__builtin_amdgcn_update_dpp(up, __float_as_int(v), 0x114, 0xF, 0xA, false)); // row_shr:4, the others lane - 4
+    }
+    if constexpr (N == 16 || N == 8) {
+        v += pi_dpp_f32<PI_DPP_XOR2, 0xF>(v);
+        v += pi_dpp_f32<PI_DPP_XOR1, 0xF>(v);
+    } else {
+        for (int o = n / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, PI_WAVE);
+    }
     return v;
 }
 __device__ __forceinline__ int pi_wave_sum_i32(int v) {

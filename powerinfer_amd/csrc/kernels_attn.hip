@@ -187,7 +187,8 @@ constexpr int kAttnBatch = 4;           // passes behind those whose rows are re
 // BLOCK threads per head: kAttnBlock for a single sequence and for steps whose workgroups all fit on the chip at once (two of 1024
 // threads per compute unit); half of that where they do not (16 sequences x 40 heads are 640 workgroups against 512 places: a
 // quarter of the units ran a second round, 48 us at 530 cells; with 512 threads four fit a unit and all 640 run together).
-template <int BLOCK>
+// LPP: hd / 8, the lanes of a cell, where it is 16 or 8 (0: any)
+template <int BLOCK, int LPP>
 __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
                                                             __half * __restrict__ k_cache, __half * __restrict__ v_cache,
                                                             int n_head, int n_head_kv, int hd, int mode, int n_ctx,
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
     const bool leader = (h % grp_sz) == 0;
     // the cache cells of the first kAttnPre passes do not depend on anything computed here: their K and V rows are requested
     // now and travel during the rotation, the scores and the softmax (one memory round trip instead of three in a row)
-    const int lpp = hd / 8;
+    const int lpp = LPP ? LPP : hd / 8;
     const int sub = tid % lpp, grp = tid / lpp, ngrp = BLOCK / lpp;
     const __half * kb = k_cache + (size_t)kvh * n_ctx * hd;
     const __half * vb = v_cache + (size_t)kvh * n_ctx * hd;
@@ -258,22 +259,23 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
 #pragma unroll
     for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
 #pragma unroll
-    for (int i = 0; i < kAttnPre; ++i) {
-        if (i * ngrp < n_kv) {
+    for (int i = 0; i < kAttnPre; ++i) {                            // (a row past the last is whatever the registers hold, and not used)
+        if (i * ngrp < pos) {
             const int c = i * ngrp + grp;
-            float d = 0.0f;
-            if (c < pos) d = pi_dot8(kpre[i], qf, 0.0f);
-            else if (c == pos) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
-            }
-            for (int o = lpp / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, PI_WAVE);
-            if (c < n_kv && sub == 0) s[c] = __fmul_rn(d, scale);
+            const float d = pi_group_sum<LPP>(pi_dot8(kpre[i], qf, 0.0f), lpp);
+            if (c < pos && sub == 0) s[c] = __fmul_rn(d, scale);
         }
+    }
+    if (grp == pos % ngrp) {                                        // the new cell
+        float d = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
+        d = pi_group_sum<LPP>(d, lpp);
+        if (sub == 0) s[pos] = __fmul_rn(d, scale);
     }
     // the passes behind the prefetched ones, kAttnBatch at a time: their rows are requested together and cost one trip to memory
     // instead of one each (the same dots in the same order)
-    for (int c0 = kAttnPre * ngrp; c0 < n_kv; c0 += kAttnBatch * ngrp) {
+    for (int c0 = kAttnPre * ngrp; c0 < pos; c0 += kAttnBatch * ngrp) {
         pi_u32x4 kk[kAttnBatch];
 #pragma unroll
         for (int u = 0; u < kAttnBatch; ++u) {
@@ -282,16 +284,10 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
         }
 #pragma unroll
         for (int u = 0; u < kAttnBatch; ++u) {
-            if (c0 + u * ngrp < n_kv) {
+            if (c0 + u * ngrp < pos) {
                 const int c = c0 + u * ngrp + grp;
-                float d = 0.0f;
-                if (c < pos) d = pi_dot8(kk[u], qf, 0.0f);
-                else if (c == pos) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) d = fmaf(kcur[sub * 8 + i], qf[i], d);
-                }
-                for (int o = lpp / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, PI_WAVE);
-                if (c < n_kv && sub == 0) s[c] = __fmul_rn(d, scale);
+                const float d = pi_group_sum<LPP>(pi_dot8(kk[u], qf, 0.0f), lpp);
+                if (c < pos && sub == 0) s[c] = __fmul_rn(d, scale);
             }
         }
     }
@@ -355,7 +351,13 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
     __syncthreads();
     for (int e = tid; e < hd; e += BLOCK) {
         float v = part[e];
-        for (int g = 1; g < ngrp; ++g) v += part[g * hd + e];
+        for (int g0 = 0; g0 < ngrp; g0 += 8) {                     // (ngrp: a multiple of 8; eight reads in flight, added in order)
+            float t[8];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) t[g] = part[(g0 + g) * hd + e];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
+        }
         out[(size_t)h * hd + e] = v;
         if (out16) out16[out16_ol ? pi_ol_index(blockIdx.y, h * hd + e) : (size_t)h * hd + e] = __float2half_rn(v);
         if (q8_q) {                                               // (hd % 32 == 0: the lanes of a block run this together)
@@ -384,13 +386,16 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
 // points of the CPU path's table, ggml.c:10747-10759), l = sum e_i in double and acc = sum v_i * e_i, and hands (m, l, acc) to
 // attn_merge_kernel, which rescales by exp(m - M), adds the parts in order and divides by the total.  Against one workgroup per head,
 // which knows the global maximum before it rounds, results differ in the last places of the fp16 roundings (1e-4 of the output).
+// Bound by the trips to memory of a part's rows: eight passes of K and V are in flight at any time (four at the start and then one by one: 21.9 us
+// for 32 heads of 128 at 3000 cells in 8 parts, 49 MB; now 15.4; 128 heads of 64 at 1024 cells in 2 parts 20.6 -> 12.0), the
+// sums over a cell's lanes are VALU permutations, and the sum over the groups reads LDS eight at a time.
 // ---------------------------------------------------------------------------------------------------
 // FROM_CACHE: the token's own K / V row is in the cache already and qkv holds its rotated q only ([n_head * hd] per token; a prompt chunk
 // behind rope_kv_store_kernel): nothing is rotated or stored, every cell is read from the cache.
 constexpr int kAttnPartBlock = 512;
-constexpr int kAttnPartPre = 4;
-template <bool FROM_CACHE>
-__global__ __launch_bounds__(kAttnPartBlock) void attn_part_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
+constexpr int kAttnPartPre = 8;          // passes whose K and V rows are in flight: one use of a row requests the row eight passes on
+template <bool FROM_CACHE, int LPP>
+__global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
                                                                    __half * __restrict__ k_cache, __half * __restrict__ v_cache,
                                                                    int n_head, int n_head_kv, int hd, int mode, int n_ctx, int s_cap,
                                                                    const int32_t * __restrict__ pos_p, float * __restrict__ part_acc, float * __restrict__ part_ml,
@@ -417,17 +422,17 @@ __global__ __launch_bounds__(kAttnPartBlock) void attn_part_kernel(const float *
     const float * qsrc = qkv + (size_t)h * hd;
     const float * ksrc = qkv + (size_t)(n_head + kvh) * hd;
     const float * vsrc = qkv + (size_t)(n_head + n_head_kv + kvh) * hd;
-    const int lpp = hd / 8;
+    const int lpp = LPP ? LPP : hd / 8;
     const int sub = tid % lpp, grp = tid / lpp, ngrp = kAttnPartBlock / lpp;
     const __half * kb = k_cache + (size_t)kvh * n_ctx * hd;
     const __half * vb = v_cache + (size_t)kvh * n_ctx * hd;
     const int n_old = (owns_new ? hi - 1 : hi) - lo;              // cells of this part that live in the cache
     pi_u32x4 kpre[kAttnPartPre], vpre[kAttnPartPre];
+    const __half * kr = kb + (size_t)lo * hd + sub * 8, * vr = vb + (size_t)lo * hd + sub * 8;
 #pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) {
-        const int c = i * ngrp + grp;
-        if (c < n_old) { kpre[i] = pi_ld16(kb + (size_t)(lo + c) * hd + sub * 8); vpre[i] = pi_ld16(vb + (size_t)(lo + c) * hd + sub * 8); }
-    }
+    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_old) kpre[i] = pi_ld16(kr + (size_t)c * hd); }
+#pragma unroll
+    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_old) vpre[i] = pi_ld16(vr + (size_t)c * hd); }
     if (FROM_CACHE) {
         if (tid < hd) qs[tid] = pi_round_f16(qsrc[tid]);
     } else if (tid < hd / 2) {
@@ -457,30 +462,20 @@ __global__ __launch_bounds__(kAttnPartBlock) void attn_part_kernel(const float *
     float qf[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
+    for (int c0 = 0; c0 < n_old; c0 += kAttnPartPre * ngrp)
 #pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) {
-        if (i * ngrp < n_mine) {
-            const int c = i * ngrp + grp;
-            float d = 0.0f;
-            if (c < n_old) d = pi_dot8(kpre[i], qf, 0.0f);
-            else if (c < n_mine) {
-#pragma unroll
-                for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
-            }
-            for (int o = lpp / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, PI_WAVE);
-            if (c < n_mine && sub == 0) s[c] = __fmul_rn(d, scale);
+        for (int i = 0; i < kAttnPartPre; ++i) {                    // (a row past the last is whatever the registers hold, and not used)
+            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
+            const float d = pi_group_sum<LPP>(pi_dot8(kpre[i], qf, 0.0f), lpp);
+            if (next < n_old) kpre[i] = pi_ld16(kr + (size_t)next * hd);
+            if (c < n_old && sub == 0) s[c] = __fmul_rn(d, scale);
         }
-    }
-    for (int c0 = kAttnPartPre * ngrp; c0 < n_mine; c0 += ngrp) {
-        const int c = c0 + grp;
+    if (owns_new && grp == n_old % ngrp) {
         float d = 0.0f;
-        if (c < n_old) d = pi_dot8(pi_ld16(kb + (size_t)(lo + c) * hd + sub * 8), qf, 0.0f);
-        else if (c < n_mine) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) d = fmaf(kcur[sub * 8 + i], qf[i], d);
-        }
-        for (int o = lpp / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, PI_WAVE);
-        if (c < n_mine && sub == 0) s[c] = __fmul_rn(d, scale);
+        for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
+        d = pi_group_sum<LPP>(d, lpp);
+        if (sub == 0) s[n_old] = __fmul_rn(d, scale);
     }
     __syncthreads();
 
@@ -498,38 +493,36 @@ __global__ __launch_bounds__(kAttnPartBlock) void attn_part_kernel(const float *
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
+    for (int c0 = 0; c0 < n_old; c0 += kAttnPartPre * ngrp)
 #pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) {
-        const int c = i * ngrp + grp;
-        if (c < n_mine) {
-            const float p = s[c];
-            float vf[8];
-            if (c < n_old) pi_unpack8(vpre[i], vf);
-            else {
+        for (int i = 0; i < kAttnPartPre; ++i) {
+            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
+            if (c < n_old) {
+                const float p = s[c];
+                float vf[8];
+                pi_unpack8(vpre[i], vf);
+                if (next < n_old) vpre[i] = pi_ld16(vr + (size_t)next * hd);
 #pragma unroll
-                for (int k = 0; k < 8; ++k) vf[k] = vcur[sub * 8 + k];
+                for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], p, acc[k]);
             }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], p, acc[k]);
         }
-    }
-    for (int c = kAttnPartPre * ngrp + grp; c < n_mine; c += ngrp) {
-        const float p = s[c];
-        float vf[8];
-        if (c < n_old) pi_unpack8(pi_ld16(vb + (size_t)(lo + c) * hd + sub * 8), vf);
-        else {
+    if (owns_new && grp == n_old % ngrp) {                          // (the new cell is its group's last)
+        const float p = s[n_old];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) vf[i] = vcur[sub * 8 + i];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = fmaf(vf[i], p, acc[i]);
+        for (int k = 0; k < 8; ++k) acc[k] = fmaf(vcur[sub * 8 + k], p, acc[k]);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
     __syncthreads();
     for (int e = tid; e < hd; e += kAttnPartBlock) {
         float v = part[e];
-        for (int g = 1; g < ngrp; ++g) v += part[g * hd + e];
+        for (int g0 = 0; g0 < ngrp; g0 += 8) {                     // (ngrp: a multiple of 8; eight reads in flight, added in order)
+            float t[8];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) t[g] = part[(g0 + g) * hd + e];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
+        }
         part_acc[slot * hd + e] = v;
     }
     if (tid == 0) { part_ml[slot * 2] = n_mine > 0 ? mx : -INFINITY; part_ml[slot * 2 + 1] = (float)sum; }
@@ -538,18 +531,37 @@ __global__ __launch_bounds__(kAttnPartBlock) void attn_part_kernel(const float *
 // out[h][e] = sum_s acc_s[e] * exp(m_s - M) / sum_s l_s * exp(m_s - M), parts in ascending order; one workgroup of hd threads per head
 __global__ void attn_merge_kernel(const float * __restrict__ part_acc, const float * __restrict__ part_ml, int n_parts, int hd,
                                   float * __restrict__ out, int out_stride, __half * __restrict__ out16) {
+    constexpr int kAtOnce = 16;                                    // parts whose values are requested together
     const int h = blockIdx.x, n_head = gridDim.x, e = threadIdx.x;
     const size_t slot0 = ((size_t)blockIdx.y * n_head + h) * n_parts;
-    float M = -INFINITY;
-    for (int sp = 0; sp < n_parts; ++sp) M = fmaxf(M, part_ml[(slot0 + sp) * 2]);
-    float L = 0.0f, v = 0.0f;
-    for (int sp = 0; sp < n_parts; ++sp) {
-        const float m = part_ml[(slot0 + sp) * 2], l = part_ml[(slot0 + sp) * 2 + 1];
-        if (l > 0.0f) {
-            const float w = expf(__fsub_rn(m, M));
-            L = fmaf(l, w, L);
-            v = fmaf(part_acc[(slot0 + sp) * hd + e], w, v);
+    float m[kAtOnce], l[kAtOnce], a[kAtOnce], M = -INFINITY;
+    auto fetch = [&](int s0, bool values) {
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int sp = min(s0 + j, n_parts - 1);
+            m[j] = part_ml[(slot0 + sp) * 2]; l[j] = part_ml[(slot0 + sp) * 2 + 1];
+            if (values) a[j] = part_acc[(slot0 + sp) * hd + e];
         }
+    };
+    fetch(0, true);
+    for (int s0 = 0;;) {
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) M = fmaxf(M, m[j]);        // (the last part more than once)
+        if ((s0 += kAtOnce) >= n_parts) break;
+        fetch(s0, false);
+    }
+    if (n_parts > kAtOnce) fetch(0, true);
+    float L = 0.0f, v = 0.0f;
+    for (int s0 = 0;;) {
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j)
+            if (s0 + j < n_parts && l[j] > 0.0f) {
+                const float w = expf(__fsub_rn(m[j], M));
+                L = fmaf(l[j], w, L);
+                v = fmaf(a[j], w, v);
+            }
+        if ((s0 += kAtOnce) >= n_parts) break;
+        fetch(s0, true);
     }
     v = pi_div(v, L);
     out[(size_t)blockIdx.y * out_stride + (size_t)h * hd + e] = v;
@@ -1287,6 +1299,10 @@ int pi_k_attn_decode_supported(int hd, int n_ctx) {
 }
 
 }  // extern "C"
+
+// the lanes of a cell are a constant for the two usual head sizes (their sums are then lane permutations)
+#define PI_ATTN_LPP(...) do { if (hd == 128) { constexpr int LPP = 16; __VA_ARGS__; } else if (hd == 64) { constexpr int LPP = 8; __VA_ARGS__; } \
+                              else { constexpr int LPP = 0; __VA_ARGS__; } } while (0)
 namespace pi {
 int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream) {
@@ -1295,8 +1311,8 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
         return pi::fail(PI_E_ARG, "pi_k_attn_fused: head size must be 8 * (a divisor of 64), at most 128; mode 0 or 2");
     const size_t sh = attn_fused_lds_bytes(hd, n_ctx);
     if (sh > kAttnLdsLimit) return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_fused: context too long for the single-pass kernel");
-    hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock>, dim3(n_head + ahead.blocks), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, 0, (size_t)0, 0, nullptr, 0, nullptr, nullptr, nullptr, ahead);
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_fused_kernel<kAttnBlock, LPP>), dim3(n_head + ahead.blocks), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
+                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, 0, (size_t)0, 0, nullptr, 0, nullptr, nullptr, nullptr, ahead));
     return pi::check_launch("pi_k_attn_fused");
 }
 }  // namespace pi
@@ -1328,8 +1344,8 @@ int pi_k_attn_split(const float * qkv, int qkv_stride, const void * rope_table, 
     float * acc = scratch;
     float * ml = scratch + (size_t)n_seq * n_head * n_parts * hd;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(attn_part_kernel<false>, dim3(n_head, n_parts, n_seq), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, qkv, (const float2 *)rope_table,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml, qkv_stride, cache_seq_stride);
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<false, LPP>), dim3(n_head, n_parts, n_seq), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, qkv, (const float2 *)rope_table,
+                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml, qkv_stride, cache_seq_stride));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_seq), dim3(hd), 0, st, acc, ml, n_parts, hd, out, out_stride, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_split");
 }
@@ -1343,8 +1359,8 @@ int pi_k_attn_split_cached(const float * q_rot, const void * k_cache, const void
     float * acc = scratch;
     float * ml = scratch + (size_t)n_tok * n_head * n_parts * hd;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(attn_part_kernel<true>, dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
-                       (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0);
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
+                       (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_tok), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)nullptr);
     return pi::check_launch("pi_k_attn_split_cached");
 }
@@ -1360,11 +1376,11 @@ static int attn_fused_batch(const float * qkv, int qkv_stride, const void * rope
     if (sh > kAttnLdsLimit) return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_fused_batch: context too long for the single-pass kernel");
     const int n_cu = pi::compute_units();
     if (n_cu > 0 && n_seq * n_head > 2 * n_cu)
-        hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock / 2>, dim3(n_head, n_seq), dim3(kAttnBlock / 2), attn_fused_lds_bytes(hd, n_ctx, kAttnBlock / 2), (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{});
+        PI_ATTN_LPP(hipLaunchKernelGGL((attn_fused_kernel<kAttnBlock / 2, LPP>), dim3(n_head, n_seq), dim3(kAttnBlock / 2), attn_fused_lds_bytes(hd, n_ctx, kAttnBlock / 2), (hipStream_t)stream, qkv, (const float2 *)rope_table,
+                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{}));
     else
-        hipLaunchKernelGGL(attn_fused_kernel<kAttnBlock>, dim3(n_head, n_seq), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
-                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{});
+        PI_ATTN_LPP(hipLaunchKernelGGL((attn_fused_kernel<kAttnBlock, LPP>), dim3(n_head, n_seq), dim3(kAttnBlock), sh, (hipStream_t)stream, qkv, (const float2 *)rope_table,
+                           (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, out, qkv_stride, cache_seq_stride, out_stride, (__half *)out_f16, out16_ol, (int8_t *)q8_q, q8_d, q8_s, Ahead{}));
     return pi::check_launch("pi_k_attn_fused_batch");
 }
 
@@ -1467,8 +1483,8 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)T * n_head * n_parts * hd;
-    hipLaunchKernelGGL(attn_part_kernel<true>, dim3(n_head, n_parts, T), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0);
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, T), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
+                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, T), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_chunk_long");
 }

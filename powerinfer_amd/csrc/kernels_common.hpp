@@ -29,7 +29,13 @@ __device__ double block_sum_f64(double v, double * red) {
     if (lane == 0) red[wave] = v;
     __syncthreads();
     double s = 0.0;
-    for (int i = 0; i < nw; ++i) s += red[i];
+    for (int i = 0; i < nw; i += 4) {                              // four reads in flight, added in order
+        double t[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[j] = red[min(i + j, nw - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) if (i + j < nw) s += t[j];
+    }
     return s;
 }
 __device__ float block_max_f32(float v, float * red) {
@@ -39,7 +45,9 @@ __device__ float block_max_f32(float v, float * red) {
     if (lane == 0) red[wave] = v;
     __syncthreads();
     float s = red[0];
-    for (int i = 1; i < nw; ++i) s = fmaxf(s, red[i]);
+    for (int i = 0; i < nw; i += 4)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s = fmaxf(s, red[min(i + j, nw - 1)]);
     return s;
 }
 
