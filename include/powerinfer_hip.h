@@ -384,6 +384,9 @@ PI_API int pi_k_norm_q8_round_f16(const float * x, int T, int cols, const pi_nor
 PI_API int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream);
 PI_API int pi_k_dequant_q4_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                                void * out_f16, pi_stream_t stream);
+/* the same transposed, out_f16[cols][rows]: rows % 8 == 0, cols % 256 == 0, operands 16-byte aligned (else PI_E_UNSUPPORTED) */
+PI_API int pi_k_dequant_q4_t_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
+                               void * out_f16, pi_stream_t stream);
 /* the same assembly for an fp16 matrix of a hybrid layer (rows % 32 == 0, cols % 8 == 0), and the embedding rows of a chunk from a Q4_0 table */
 PI_API int pi_k_assemble_rows_f16(const void * W_f16, const void * W_rest_f16, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                                   void * out_f16, pi_stream_t stream);

@@ -391,11 +391,9 @@ int chunk_gemm(pi_model * m, const void * W, int rows, int cols, const void * xn
     return pi_k_gemm_tile_f16(W, rows, cols, xn, T, epi, add1, add2, y, y16, 0, m->stream);
 }
 
-// a matrix of layer il as fp16 rows for a chunk's mat-mul: an F16 matrix that is whole on the device as stored; a Q4_0 one expanded into
-// the chunk's scratch (values (q - 8) * d rounded to fp16); an FFN matrix of a hybrid layer assembled there from the compact matrix of the
-// resident neurons and the non-resident rows in pinned host memory, which the kernel reads over the host link once per chunk
-int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int cols, const void ** out) {
-    Tensor & t = m->L(il, kind);
+// where a hybrid layer's FFN matrix has the rows of its other neurons, and which are whose (nulls: the matrix is whole)
+struct ChunkSource { const void * rest; const uint32_t * hot_words; const int32_t * hot_prefix; };
+ChunkSource chunk_source(pi_model * m, BatchState * b, int il, int kind) {
     const bool ffn = kind == PI_T_FFN_UP || kind == PI_T_FFN_GATE || kind == PI_T_FFN_DOWN_T;
     const bool split = ffn && m->L(il, PI_T_GPU_BUCKET).dev != nullptr;
     const void * rest = !split ? nullptr : kind == PI_T_FFN_UP ? m->rest_up[il] : kind == PI_T_FFN_GATE ? m->rest_gate[il] : m->rest_down[il];
@@ -403,18 +401,31 @@ int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int c
         const int which = kind == PI_T_FFN_UP ? 0 : kind == PI_T_FFN_GATE ? 1 : 2;
         rest = b->stage[il & 1] + (size_t)which * b->stage_rows * b->stage_row_bytes;
     }
-    const uint32_t * hw = split ? m->hot_words[il] : nullptr;
-    const int32_t * hpx = split ? m->hot_prefix[il] : nullptr;
+    return {rest, split ? m->hot_words[il] : nullptr, split ? m->hot_prefix[il] : nullptr};
+}
+
+// a matrix of layer il as fp16 rows for a chunk's mat-mul: an F16 matrix that is whole on the device as stored; a Q4_0 one expanded into
+// the chunk's scratch (values (q - 8) * d rounded to fp16); an FFN matrix of a hybrid layer assembled there from the compact matrix of the
+// resident neurons and the non-resident rows in pinned host memory, which the kernel reads over the host link once per chunk
+int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int cols, const void ** out) {
+    Tensor & t = m->L(il, kind);
+    const ChunkSource c = chunk_source(m, b, il, kind);
     if (t.type == PI_TYPE_Q4_0) {
-        PI_TRY(pi_k_dequant_q4_f16(t.dev, rest, hw, hpx, rows, cols, b->w16, m->stream));
+        PI_TRY(pi_k_dequant_q4_f16(t.dev, c.rest, c.hot_words, c.hot_prefix, rows, cols, b->w16, m->stream));
         *out = b->w16;
-    } else if (split) {
-        PI_TRY(pi_k_assemble_rows_f16(t.dev, rest, hw, hpx, rows, cols, b->w16, m->stream));
+    } else if (c.hot_words) {
+        PI_TRY(pi_k_assemble_rows_f16(t.dev, c.rest, c.hot_words, c.hot_prefix, rows, cols, b->w16, m->stream));
         *out = b->w16;
     } else {
         *out = t.dev;
     }
     return PI_OK;
+}
+
+// the down projection of a Q4_0 layer with its neurons contiguous, in w16t
+int chunk_down_q4(pi_model * m, BatchState * b, int il, int ff, int d) {
+    const ChunkSource c = chunk_source(m, b, il, PI_T_FFN_DOWN_T);
+    return pi_k_dequant_q4_t_f16(m->L(il, PI_T_FFN_DOWN_T).dev, c.rest, c.hot_words, c.hot_prefix, ff, d, b->w16t, m->stream);
 }
 
 int wide_layer(pi_model * m, BatchState * b, int il) {
@@ -472,6 +483,10 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     const void * Wd = m->down_rows[il];
+    if (!Wd && down.type == PI_TYPE_Q4_0) {
+        const int rc = chunk_down_q4(m, b, il, ff, d);
+        if (rc != PI_E_UNSUPPORTED) { PI_TRY(rc); Wd = b->w16t; }
+    }
     if (!Wd) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_DOWN_T, ff, d, &W));
         PI_TRY(pi_k_transpose_f16(W, ff, d, b->w16t, st));

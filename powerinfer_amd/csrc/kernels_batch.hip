@@ -1300,17 +1300,107 @@ __global__ void dequant_q4_f16_kernel(const pi_block_q4_0 * __restrict__ W, cons
         for (int k = 0; k < 4; ++k) dst[k] = reinterpret_cast<const pi_u32x4 *>(o)[k];
     }
 }
+// The same 128 blocks at a time (2304 bytes in a row: one row of 4096 columns): a workgroup brings them to LDS in pieces of 16 bytes and writes
+// 16 bytes a thread, neighbours side by side.  A thread a block reads two odd pieces of 18 bytes and leaves four pieces 64 bytes
+// apart; 11008 x 4096 took 38 us that way.
+constexpr int kDqBlocks = 128, kDqBytes = kDqBlocks * 18;
+__device__ __forceinline__ const unsigned char * q4_row(const pi_block_q4_0 * W, const pi_block_q4_0 * W_rest, const uint32_t * hot_words, const int32_t * hot_prefix, int row, int nb) {
+    if (!hot_words) return reinterpret_cast<const unsigned char *>(W + (size_t)row * nb);
+    const uint32_t hot = hot_words[row >> 5];
+    const int bit = row & 31, base = hot_prefix[row >> 5], below = __popc(hot & ((1u << bit) - 1u));
+    return reinterpret_cast<const unsigned char *>((hot >> bit) & 1u ? W + (size_t)(base + below) * nb : W_rest + (size_t)((row & ~31) - base + bit - below) * nb);
+}
+__global__ __launch_bounds__(kBlock) void dequant_q4_f16_units_kernel(const pi_block_q4_0 * __restrict__ W, const pi_block_q4_0 * __restrict__ W_rest,
+                                                                      const uint32_t * __restrict__ hot_words, const int32_t * __restrict__ hot_prefix,
+                                                                      int nb, int n_units, __half * __restrict__ out) {
+    __shared__ __align__(16) unsigned char raw[2][kDqBytes];
+    const int per_row = nb / kDqBlocks, tid = threadIdx.x;
+    auto source = [&](int u) { return q4_row(W, W_rest, hot_words, hot_prefix, u / per_row, nb) + (size_t)(u % per_row) * kDqBytes; };
+    pi_u32x4 v{};
+    int u = blockIdx.x;
+    if (u < n_units && tid < kDqBytes / 16) v = pi_ld_stream(source(u) + tid * 16);
+    for (int b = 0; u < n_units; u += gridDim.x, b ^= 1) {
+        if (tid < kDqBytes / 16) *reinterpret_cast<pi_u32x4 *>(raw[b] + tid * 16) = v;
+        const int next = u + gridDim.x;
+        if (next < n_units && tid < kDqBytes / 16) v = pi_ld_stream(source(next) + tid * 16);
+        __syncthreads();                                            // (one barrier: the other half is written next, behind the next barrier's reads)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int piece = tid + k * kBlock, blk = piece >> 2, sub = piece & 3;      // eight values: low or high nibbles of eight bytes
+            const unsigned char * p = raw[b] + blk * 18;
+            const float d = pi_f16_from_bits(*reinterpret_cast<const uint16_t *>(p));
+            const uint16_t * q = reinterpret_cast<const uint16_t *>(p + 2 + (sub & 1) * 8);
+            __align__(16) __half o[8];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int w = (q[j] >> ((sub >> 1) * 4)) & 0x0F0F;
+                o[2 * j] = __float2half_rn(__fmul_rn((float)((w & 0xFF) - 8), d));
+                o[2 * j + 1] = __float2half_rn(__fmul_rn((float)((w >> 8) - 8), d));
+            }
+            *reinterpret_cast<pi_u32x4 *>(out + (size_t)u * kDqBlocks * 32 + piece * 8) = *reinterpret_cast<const pi_u32x4 *>(o);
+        }
+    }
+}
+// out[c][r] of the same: 64 rows x 256 columns a workgroup, nine pieces of 16 bytes a row to LDS; eight rows of a column leave as 16 bytes, the
+// 64 rows of a column as 128 in a row.  Against expanding and transposing (38 + 53 us at 11008 x 4096) the fp16 matrix goes to memory once.
+constexpr int kDtRows = 64, kDtCols = 256, kDtBytes = kDtCols / 32 * 18, kDtStride = kDtBytes + 4;      // (37 words a row: rows fall on different banks)
+__global__ __launch_bounds__(kBlock) void dequant_q4_t_f16_kernel(const pi_block_q4_0 * __restrict__ W, const pi_block_q4_0 * __restrict__ W_rest,
+                                                                  const uint32_t * __restrict__ hot_words, const int32_t * __restrict__ hot_prefix,
+                                                                  int rows, int nb, __half * __restrict__ out) {
+    __shared__ __align__(16) unsigned char raw[kDtRows * kDtStride];
+    const int r0 = blockIdx.y * kDtRows, c0 = blockIdx.x * kDtCols, tid = threadIdx.x;
+    constexpr int kPieces = kDtBytes / 16;
+    for (int k = tid; k < kDtRows * kPieces; k += kBlock) {
+        const int r = k / kPieces, p = k % kPieces;
+        const pi_u32x4 v = pi_ld_stream(q4_row(W, W_rest, hot_words, hot_prefix, min(r0 + r, rows - 1), nb) + (size_t)blockIdx.x * kDtBytes + p * 16);
+        uint32_t * d = reinterpret_cast<uint32_t *>(raw + r * kDtStride + p * 16);
+        d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+    }
+    __syncthreads();
+    const int rg = tid & 7;
+    if (r0 + rg * 8 >= rows) return;                                // (rows % 8 == 0)
+    for (int c = tid >> 3; c < kDtCols; c += kBlock / 8) {
+        const int blk = c >> 5, j = c & 31;
+        __align__(16) __half o[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const unsigned char * p = raw + (rg * 8 + r) * kDtStride + blk * 18;
+            const int q = (p[2 + (j & 15)] >> (j >> 4 << 2)) & 0x0F;
+            o[r] = __float2half_rn(__fmul_rn((float)(q - 8), pi_f16_from_bits(*reinterpret_cast<const uint16_t *>(p))));
+        }
+        *reinterpret_cast<pi_u32x4 *>(out + (size_t)(c0 + c) * rows + r0 + rg * 8) = *reinterpret_cast<const pi_u32x4 *>(o);
+    }
+}
 int pi_k_dequant_q4_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                         void * out_f16, pi_stream_t stream) {
     if (!W_q4 || !out_f16 || rows <= 0 || cols <= 0 || cols % 32) return pi::fail(PI_E_ARG, "pi_k_dequant_q4_f16: bad arguments");
     if ((hot_words == nullptr) != (hot_prefix == nullptr) || (hot_words && !W_rest_q4) || (hot_words && rows % 32))
         return pi::fail(PI_E_ARG, "pi_k_dequant_q4_f16: hot_words, hot_prefix and the second matrix go together (rows % 32 == 0)");
     const size_t n = (size_t)rows * (cols / 32);
+    if (n % kDqBlocks == 0 && (!hot_words || cols / 32 % kDqBlocks == 0) && (((uintptr_t)W_q4 | (uintptr_t)W_rest_q4 | (uintptr_t)out_f16) & 15) == 0 && n / kDqBlocks < (1u << 30)) {
+        // whole units: of the rows, or without hot words of the matrix as one row
+        const int units = (int)(n / kDqBlocks), nb = hot_words ? cols / 32 : kDqBlocks;
+        hipLaunchKernelGGL(dequant_q4_f16_units_kernel, dim3((unsigned)std::min(units, 4096)), dim3(kBlock), 0, (hipStream_t)stream, (const pi_block_q4_0 *)W_q4, (const pi_block_q4_0 *)W_rest_q4,
+                           hot_words, hot_prefix, nb, units, (__half *)out_f16);
+        return pi::check_launch("pi_k_dequant_q4_f16");
+    }
     size_t blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     hipLaunchKernelGGL(dequant_q4_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const pi_block_q4_0 *)W_q4, (const pi_block_q4_0 *)W_rest_q4,
                        hot_words, hot_prefix, rows, cols / 32, (__half *)out_f16);
     return pi::check_launch("pi_k_dequant_q4_f16");
+}
+
+int pi_k_dequant_q4_t_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
+                          void * out_f16, pi_stream_t stream) {
+    if (!W_q4 || !out_f16 || rows <= 0 || cols <= 0) return pi::fail(PI_E_ARG, "pi_k_dequant_q4_t_f16: bad arguments");
+    if ((hot_words == nullptr) != (hot_prefix == nullptr) || (hot_words && (!W_rest_q4 || rows % 32)))
+        return pi::fail(PI_E_ARG, "pi_k_dequant_q4_t_f16: hot_words, hot_prefix and the second matrix go together (rows % 32 == 0)");
+    if (rows % 8 || cols % kDtCols || rows > 65535 * kDtRows || (((uintptr_t)W_q4 | (uintptr_t)W_rest_q4 | (uintptr_t)out_f16) & 15) != 0)
+        return pi::fail(PI_E_UNSUPPORTED, "pi_k_dequant_q4_t_f16: rows % 8 == 0, cols % 256 == 0, operands 16-byte aligned");
+    hipLaunchKernelGGL(dequant_q4_t_f16_kernel, dim3(cols / kDtCols, (rows + kDtRows - 1) / kDtRows), dim3(kBlock), 0, (hipStream_t)stream, (const pi_block_q4_0 *)W_q4,
+                       (const pi_block_q4_0 *)W_rest_q4, hot_words, hot_prefix, rows, cols / 32, (__half *)out_f16);
+    return pi::check_launch("pi_k_dequant_q4_t_f16");
 }
 // the full fp16 matrix of a hybrid layer from the compact matrix of the resident neurons and the matrix of the others (both in
 // ascending neuron order); one workgroup per row, 16 bytes per lane and pass

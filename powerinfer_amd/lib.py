@@ -190,6 +190,7 @@ _SIGS = {
     "pi_k_norm_q8_round_f16": (_i, [_vp, _i, _i, C.POINTER(Norm), _vp, _vp, _vp]),
     "pi_k_ffn_h_q8_f16": (_i, [_vp, _vp, _vp, _f, _i, _i, _vp, _vp]),
     "pi_k_dequant_q4_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
+    "pi_k_dequant_q4_t_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "pi_k_assemble_rows_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "pi_k_embed_batch_q4": (_i, [_vp, _i, _vp, _i, _vp, _vp]),
     "pi_k_host_signal": (_i, [_vp, _vp, _i, _i, _vp]),

@@ -44,3 +44,34 @@ def test_busy_groups_and_odd_addresses(has_gate, r, threshold):
     if threshold == 0.0:
         ou = under(L, d, ff, ol.Q4_0, has_gate, x, one["logits"])
         assert rel_err(out[0][0], ou["h"]) < 1e-4 and rel_err(out[0][1], ou["out"]) < FFN_REL_TOL
+
+
+@pytest.mark.parametrize("rows,cols,hot_frac", [(32, 4096, 1.0), (200, 256, 1.0), (72, 512, 1.0), (96, 4096, 0.6), (64, 8192, 0.0), (32, 96, 1.0), (160, 768, 0.3)])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_expanded_matrices(rows, cols, hot_frac, shift):
+    """A Q4_0 matrix as fp16, rows or columns contiguous, by units of 128 blocks and without them: exactly (q - 8) * d rounded to fp16."""
+    L, rng = pl.init(), np.random.default_rng(rows + cols)
+    wq = synth.quantize_q4_0((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    want = np.zeros((rows, cols), np.float32)
+    ol.oracle().pio_dequantize_row_q4_0(ol._ptr(wq), ol._ptr(want), rows * cols)
+    gid = rng.random(rows) < hot_frac
+    words, prefix = None, None
+    if hot_frac < 1.0:
+        bits = np.packbits(gid.reshape(-1, 32), axis=1, bitorder="little").view(np.uint32).ravel()
+        words, prefix = pl.DevBuf(host=bits), pl.DevBuf(host=np.concatenate([[0], np.cumsum(gid.reshape(-1, 32).sum(1))[:-1]]).astype(np.int32))
+    place = lambda a: Shifted(pl.DevBuf(host=np.concatenate([a.reshape(-1).view(np.uint8), np.zeros(16, np.uint8)]))) if shift else pl.DevBuf(host=np.concatenate([a.reshape(-1).view(np.uint8), np.zeros(16, np.uint8)]))  # noqa: E731
+    hot, rest = place(wq[gid] if words else wq), place(wq[~gid]) if words else None
+    p = lambda b: b.ptr if b is not None else None  # noqa: E731
+    for name, t in (("pi_k_dequant_q4_f16", False), ("pi_k_dequant_q4_t_f16", True)):
+        out = pl.DevBuf(2 * rows * cols + 64)
+        pl.check(L.pi_memset(out.ptr, 0xAB, out.nbytes))
+        print(name, rows, cols, hot_frac, shift, flush=True)
+        rc = getattr(L, name)(hot.ptr, p(rest), p(words), p(prefix), rows, cols, out.ptr, None)
+        if t and (shift or cols % 256):
+            assert rc != 0
+            continue
+        pl.check(rc, name)
+        pl.sync()
+        got = out.download(np.float16)
+        assert (got[rows * cols:].view(np.uint16) == 0xABAB).all()
+        assert np.array_equal(got[:rows * cols].reshape((cols, rows) if t else (rows, cols)), (want.T if t else want).astype(np.float16))
