@@ -265,52 +265,73 @@ __global__ __launch_bounds__(kBlock, 2) void gemv_multi_f16_reg_kernel(GemvMulti
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Register-resident Q4_0 mat-vec for cols == 4096 * CB.  A Q4_0 row of 4096 weights is 128 blocks of 18 bytes =
-// 2304 bytes = 64 lanes x 36 bytes: lane l reads the block pair (2l, 2l+1) of each 4096-column group with two
-// 16-byte loads and one 4-byte load (4-byte aligned) and meets it with the matching 64 int8 activations, their two
-// Q8_0 scales and block sums, all held in registers.  The nibbles are used unsigned through v_dot4_i32_i8 and
-// 8 * sum(x) is subtracted per block, which is exact in int32; the result is scaled by d_w * d_x in fp32 as
-// vec_dot_q4_0_q8_0 does (ggml-quants.c:2512-2650).  The prologue (norm, then Q8_0 quantisation as the x86
-// quantize_row_q8_0 does: d = amax / 127 kept as fp16, q = rint(x * 127 / amax), ggml-quants.c:702-760) is shared by
-// the four waves through LDS.  Four rows (two for CB = 2) of loads are in flight per lane.
+// Q4_0 mat-vec for cols == 4096 * CB.  A Q4_0 row of 4096 weights is 128 blocks of 18 bytes = 2304 bytes = 64 lanes x 36 bytes: lane l
+// meets the block pair (2l, 2l+1) of each 4096-column group with the matching 64 int8 activations, their two Q8_0 scales and block sums,
+// all held in registers.  The nibbles are used unsigned through v_dot4_i32_i8 and 8 * sum(x) is subtracted per block, which is exact in
+// int32; the result is scaled by d_w * d_x in fp32 as vec_dot_q4_0_q8_0 does (ggml-quants.c:2512-2650).  The prologue (norm, then Q8_0
+// quantisation as the x86 quantize_row_q8_0 does: d = amax / 127 kept as fp16, q = rint(x * 127 / amax), ggml-quants.c:702-760) is
+// shared by the four waves through LDS.
+// A fifth wave copies rows straight to LDS, a row for each of the other four a step and NBUF steps ahead, from the first moment on: the matrix
+// is on its way under the prologue, which is half of the launch, and a lane takes its 36 bytes from LDS, where 36 bytes a lane fall on
+// different banks (from memory they were three loads at odd places each).  One barrier a step: behind it the step's rows are there and
+// the previous step's slots are free.  12288 x 4096 behind an RMSNorm 10.8 -> 9.7 us, 32000 x 4096 20.2 -> 16.1,
+// 8192 x 8192 12.6 -> 9.1, 65024 x 8192 69 -> 54 (5.5 TB/s); matrices on a multiple of 4 bytes only, copied by single words, 10.9 -> 10.0 and 20.2 -> 22.3.
 // ---------------------------------------------------------------------------------------------------
-typedef uint32_t pi_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-
+constexpr int kQ4Threads = kBlock + PI_WAVE;
 template <int CB, int KIND, int TAG>
-__global__ __launch_bounds__(kBlock, 2) void gemv_q4_reg_kernel(const unsigned char * __restrict__ W, const float * __restrict__ x,
+__global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsigned char * __restrict__ W, const float * __restrict__ x,
                                                              const float * __restrict__ nw, const float * __restrict__ nb, float eps,
                                                              int epi, const float * __restrict__ add1, const float * __restrict__ add2,
-                                                             float * __restrict__ y, int rows) {
+                                                             float * __restrict__ y, int rows, int a16) {
     constexpr int cols = CB * 4096, NCH = cols / 512, nblk = cols / 32;
-    constexpr int NBUF = 4 / CB;
+    constexpr int NBUF = CB == 1 ? 5 : 2;                          // steps in LDS
     constexpr int MYCH = NCH / kWavesPerBlock;
     constexpr size_t row_bytes = (size_t)nblk * 18;
     __shared__ __align__(16) int8_t xq[cols];
     __shared__ float xd[nblk];
     __shared__ int   xsum[nblk];
     __shared__ double red[2][kWavesPerBlock];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    __shared__ __align__(16) unsigned char ring[NBUF][kWavesPerBlock][row_bytes];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n_waves = gridDim.x * kWavesPerBlock, wid = blockIdx.x * kWavesPerBlock + wave;
 
-    uint32_t D[NBUF][CB][9];
-    float r1[NBUF], r2[NBUF];
-    auto issue = [&](int b, int r) {
-        if (r < rows) {
+    const int steps = (rows - 1 - (int)blockIdx.x * kWavesPerBlock) / n_waves + 1;         // (of the first wave: the others' may be one fewer)
+    if (wave == kWavesPerBlock) {
+        constexpr int kCopies = kWavesPerBlock * (int)((row_bytes + 1023) / 1024);         // of a step
+        static_assert((NBUF - 1) * kCopies <= 63, "the counter of loads in flight");
+        typedef const __attribute__((address_space(1))) void * gptr;
+        typedef __attribute__((address_space(3))) void * lptr;
+        auto copy_step = [&](int s) {
 #pragma unroll
-            for (int g = 0; g < CB; ++g) {
-                const unsigned char * p = W + (size_t)r * row_bytes + g * 2304 + lane * 36;
-                const pi_u32x4_a4 v0 = __builtin_nontemporal_load(reinterpret_cast<const pi_u32x4_a4 *>(p));
-                const pi_u32x4_a4 v1 = __builtin_nontemporal_load(reinterpret_cast<const pi_u32x4_a4 *>(p + 16));
-                D[b][g][0] = v0.x; D[b][g][1] = v0.y; D[b][g][2] = v0.z; D[b][g][3] = v0.w;
-                D[b][g][4] = v1.x; D[b][g][5] = v1.y; D[b][g][6] = v1.z; D[b][g][7] = v1.w;
-                D[b][g][8] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t *>(p + 32));
+            for (int w = 0; w < kWavesPerBlock; ++w) {
+                const unsigned char * p = W + (size_t)min((int)blockIdx.x * kWavesPerBlock + w + s * n_waves, rows - 1) * row_bytes;
+                unsigned char * to = ring[s % NBUF][w];
+                if (a16) {
+#pragma unroll
+                    for (int o = 0; o < (int)row_bytes; o += 1024)
+                        if (o + lane * 16 < (int)row_bytes) __builtin_amdgcn_global_load_lds((gptr)(p + o + lane * 16), (lptr)(to + o), 16, 0, 0);
+                } else {
+#pragma unroll
+                    for (int o = 0; o < (int)row_bytes; o += 256) __builtin_amdgcn_global_load_lds((gptr)(p + o + lane * 4), (lptr)(to + o), 4, 0, 0);
+                }
             }
-            if (epi >= PI_EPI_ADD) r1[b] = add1[r];
-            if (epi == PI_EPI_ADD2) r2[b] = add2[r];
+        };
+        for (int s = 0; s < min(steps, NBUF); ++s) copy_step(s);
+        for (int k = 0; k <= KIND; ++k) __builtin_amdgcn_s_barrier();                      // the prologue's
+        for (int s = 0; s < steps; ++s) {
+            const int behind = min(steps - 1 - s, s ? NBUF - 2 : NBUF - 1);               // steps on their way behind this one (step s - 1's slot is filled below)
+            if (!a16 || behind == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCopies) : "memory");
+            else if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NBUF > 2 ? 2 * kCopies : 0) : "memory");
+            else if (behind == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NBUF > 3 ? 3 * kCopies : 0) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NBUF > 4 ? 4 * kCopies : 0) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (s > 0 && s - 1 + NBUF < steps) copy_step(s - 1 + NBUF);
         }
-    };
-#pragma unroll
-    for (int b = 0; b < NBUF; ++b) { r1[b] = 0.0f; r2[b] = 0.0f; issue(b, wid + b * n_waves); }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // no copy may arrive in LDS that is no longer this workgroup's
+        return;
+    }
 
     // ---- shared prologue: norm, Q8_0 quantisation -------------------------------------------------------------
     {
@@ -403,38 +424,43 @@ __global__ __launch_bounds__(kBlock, 2) void gemv_q4_reg_kernel(const unsigned c
         sx[g][0] = xsum[b0]; sx[g][1] = xsum[b0 + 1];
     }
 
-    for (int r = wid; r < rows; r += NBUF * n_waves) {
-#pragma unroll
-        for (int b = 0; b < NBUF; ++b) {
-            const int rr = r + b * n_waves;
-            if (rr < rows) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int g = 0; g < CB; ++g) {
-                    const uint32_t * d9 = D[b][g];
-                    int s0 = 0, s1 = 0;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const uint32_t q0 = __builtin_amdgcn_alignbit(d9[k + 1], d9[k], 16);       // bytes 2 + 4k .. 5 + 4k of the pair
-                        s0 = __builtin_amdgcn_sdot4((int)(q0 & 0x0F0F0F0Fu), X[g][k], s0, false);
-                        s0 = __builtin_amdgcn_sdot4((int)((q0 >> 4) & 0x0F0F0F0Fu), X[g][4 + k], s0, false);
-                        const uint32_t q1 = d9[5 + k];
-                        s1 = __builtin_amdgcn_sdot4((int)(q1 & 0x0F0F0F0Fu), X[g][8 + k], s1, false);
-                        s1 = __builtin_amdgcn_sdot4((int)((q1 >> 4) & 0x0F0F0F0Fu), X[g][12 + k], s1, false);
-                    }
-                    s0 -= 8 * sx[g][0];
-                    s1 -= 8 * sx[g][1];
-                    acc = fmaf(__fmul_rn(pi_f16_from_bits((uint16_t)(d9[0] & 0xffffu)), dx[g][0]), (float)s0, acc);
-                    acc = fmaf(__fmul_rn(pi_f16_from_bits((uint16_t)(d9[4] >> 16)), dx[g][1]), (float)s1, acc);
-                }
-                acc = pi_wave_sum(acc);
-                if (epi == PI_EPI_RELU) acc = fmaxf(acc, 0.0f);
-                else if (epi == PI_EPI_ADD) acc = __fadd_rn(acc, r1[b]);
-                else if (epi == PI_EPI_ADD2) acc = __fadd_rn(__fadd_rn(acc, r1[b]), r2[b]);
-                if (lane == 0) y[rr] = acc;
-            }
-            issue(b, rr + NBUF * n_waves);
+    for (int s = 0; s < steps; ++s) {
+        const int rr = wid + s * n_waves;
+        float r1 = 0.0f, r2 = 0.0f;
+        if (rr < rows) {
+            if (epi >= PI_EPI_ADD) r1 = add1[rr];
+            if (epi == PI_EPI_ADD2) r2 = add2[rr];
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // the last step's row has been read
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (rr >= rows) continue;
+        float acc = 0.0f;
+#pragma unroll
+        for (int g = 0; g < CB; ++g) {
+            uint32_t d9[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) d9[k] = *reinterpret_cast<const uint32_t *>(ring[s % NBUF][wave] + g * 2304 + lane * 36 + k * 4);
+            int s0 = 0, s1 = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t q0 = __builtin_amdgcn_alignbit(d9[k + 1], d9[k], 16);       // bytes 2 + 4k .. 5 + 4k of the pair
+                s0 = __builtin_amdgcn_sdot4((int)(q0 & 0x0F0F0F0Fu), X[g][k], s0, false);
+                s0 = __builtin_amdgcn_sdot4((int)((q0 >> 4) & 0x0F0F0F0Fu), X[g][4 + k], s0, false);
+                const uint32_t q1 = d9[5 + k];
+                s1 = __builtin_amdgcn_sdot4((int)(q1 & 0x0F0F0F0Fu), X[g][8 + k], s1, false);
+                s1 = __builtin_amdgcn_sdot4((int)((q1 >> 4) & 0x0F0F0F0Fu), X[g][12 + k], s1, false);
+            }
+            s0 -= 8 * sx[g][0];
+            s1 -= 8 * sx[g][1];
+            acc = fmaf(__fmul_rn(pi_f16_from_bits((uint16_t)(d9[0] & 0xffffu)), dx[g][0]), (float)s0, acc);
+            acc = fmaf(__fmul_rn(pi_f16_from_bits((uint16_t)(d9[4] >> 16)), dx[g][1]), (float)s1, acc);
+        }
+        acc = pi_wave_sum(acc);
+        if (epi == PI_EPI_RELU) acc = fmaxf(acc, 0.0f);
+        else if (epi == PI_EPI_ADD) acc = __fadd_rn(acc, r1);
+        else if (epi == PI_EPI_ADD2) acc = __fadd_rn(__fadd_rn(acc, r1), r2);
+        if (lane == 0) y[rr] = acc;
     }
 }
 
@@ -688,7 +714,7 @@ int pi_k_gemv(int wtype, const void * W, int rows, int cols, const float * x, co
             const int rblocks = rows >= n_waves ? kGemvBlocks : (rows + kWavesPerBlock - 1) / kWavesPerBlock;
             const int tag = rows >= 16384 ? 1 : 0;
             const unsigned char * wb = (const unsigned char *)W;
-#define PI_GEMV_Q4(CB, KIND, TAG) hipLaunchKernelGGL((gemv_q4_reg_kernel<CB, KIND, TAG>), dim3(rblocks), dim3(kBlock), 0, st, wb, x, na.w, na.b, na.eps, epilogue, add1, add2, y, rows)
+#define PI_GEMV_Q4(CB, KIND, TAG) hipLaunchKernelGGL((gemv_q4_reg_kernel<CB, KIND, TAG>), dim3(rblocks), dim3(kQ4Threads), 0, st, wb, x, na.w, na.b, na.eps, epilogue, add1, add2, y, rows, ((uintptr_t)W & 15) == 0)
 #define PI_GEMV_Q4_K(CB, KIND) do { if (tag == 1) PI_GEMV_Q4(CB, KIND, 1); else PI_GEMV_Q4(CB, KIND, 0); } while (0)
 #define PI_GEMV_Q4_N(CB) do { if (na.kind == 0) PI_GEMV_Q4_K(CB, 0); else if (na.kind == 1) PI_GEMV_Q4_K(CB, 1); else PI_GEMV_Q4_K(CB, 2); } while (0)
             if (cols == 4096) PI_GEMV_Q4_N(1); else PI_GEMV_Q4_N(2);
