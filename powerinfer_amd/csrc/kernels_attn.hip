@@ -346,18 +346,23 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
             }
         }
     }
+    // (fewer cells than groups: the groups behind hold zeros, of which one is added for all)
+    const int n_grp = min(ngrp, (n_kv + 7) & ~7);
+    if (grp < n_grp) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
+        for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
+    }
     __syncthreads();
     for (int e = tid; e < hd; e += BLOCK) {
         float v = part[e];
-        for (int g0 = 0; g0 < ngrp; g0 += 8) {                     // (ngrp: a multiple of 8; eight reads in flight, added in order)
+        for (int g0 = 0; g0 < n_grp; g0 += 8) {                    // (ngrp: a multiple of 8; eight reads in flight, added in order)
             float t[8];
 #pragma unroll
             for (int g = 0; g < 8; ++g) t[g] = part[(g0 + g) * hd + e];
 #pragma unroll
             for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
         }
+        if (n_grp < ngrp) v += 0.0f;
         out[(size_t)h * hd + e] = v;
         if (out16) out16[out16_ol ? pi_ol_index(blockIdx.y, h * hd + e) : (size_t)h * hd + e] = __float2half_rn(v);
         if (q8_q) {                                               // (hd % 32 == 0: the lanes of a block run this together)

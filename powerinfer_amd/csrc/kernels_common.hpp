@@ -58,6 +58,46 @@ __device__ float block_max_f32(float v, float * red) {
 // ---------------------------------------------------------------------------------------------------
 __device__ void stage_x_f16(__half * xs, const float * __restrict__ x, int cols, NormArgs na, double * red) {
     float mean = 0.0f, scale = 1.0f;
+    constexpr int kHeld = 4;
+    if (cols <= kHeld * (int)blockDim.x) {
+        // short vectors: the values and the norm's weights are requested together and stay in registers (the same operations in the same order)
+        float xv[kHeld], wv[kHeld], bv[kHeld];
+        const bool has_w = na.kind != 0 && na.w, has_b = na.kind != 0 && na.b;
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * blockDim.x;
+            xv[k] = i < cols ? x[i] : 0.0f;
+            wv[k] = has_w && i < cols ? na.w[i] : 1.0f;
+            bv[k] = has_b && i < cols ? na.b[i] : 0.0f;
+        }
+        if (na.kind == 1) {
+            double s = 0.0;
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) s += (double)__fmul_rn(xv[k], xv[k]);
+            scale = pi_inv_sqrt((float)(block_sum_f64(s, red) / cols) + na.eps);
+        } else if (na.kind == 2) {
+            double s = 0.0, s2 = 0.0;
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) s += (double)xv[k];
+            mean = (float)(block_sum_f64(s, red) / cols);
+#pragma unroll
+            for (int k = 0; k < kHeld; ++k) { const float v = __fsub_rn(xv[k], mean); if (threadIdx.x + k * blockDim.x < (unsigned)cols) s2 += (double)__fmul_rn(v, v); }
+            scale = pi_inv_sqrt((float)(block_sum_f64(s2, red) / cols) + na.eps);
+        }
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int i = threadIdx.x + k * blockDim.x;
+            float v = xv[k];
+            if (na.kind != 0) {
+                v = __fmul_rn(na.kind == 2 ? __fsub_rn(v, mean) : v, scale);
+                if (has_w) v = __fmul_rn(v, wv[k]);
+                if (has_b) v = __fadd_rn(v, bv[k]);
+            }
+            if (i < cols) xs[i] = __float2half_rn(v);
+        }
+        __syncthreads();
+        return;
+    }
     if (na.kind == 1) {
         double s = 0.0;
         for (int i = threadIdx.x; i < cols; i += blockDim.x) { const float v = x[i]; s += (double)__fmul_rn(v, v); }
