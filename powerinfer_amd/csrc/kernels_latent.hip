@@ -330,8 +330,13 @@ __global__ __launch_bounds__(256) void latent_attn_f32_kernel(pi_latent_attn p) 
 // transposed (keys x tokens), so that a lane's scores belong to one token, its soft-max needs two shuffles, and its weights are already
 // the column operand of the second product (values^T x weights) - which key a slot of that product's inner dimension stands for is free,
 // so the value operand is read in the order the scores came out.  64 keys at a time through LDS, the next 64 in registers.
+// Bound by the matrix and vector units (32 heads of 128 + 64 columns, 2048 tokens: 215 TFLOP/s at first): the soft-max runs in base 2, so that
+// a weight costs a subtraction and one v_exp_f32 instead of expf's dozen, and the rotated columns' cells are known a step ahead, where the
+// look-up under the fetch let every piece wait for memory: 200 -> 117 us.  (Pairing long with short tiles on a CU: 124 us.)
 // ---------------------------------------------------------------------------------------------------------------------------------
 constexpr int kXKeys = 64, kXTok = 128;
+constexpr float kLog2e = 1.4426950408889634f;
+__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 template <int KS, int VT>              // 32-column steps of a key row (unrotated | rotated, zero padded); 16-column tiles of a value row
 __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_expanded p, int n_qt, int hp) {
     constexpr int KROW = KS * 64 + 16, VROW = VT * 32 + 16, KP = KS * 4 * kXKeys / 256, VP = VT * 2 * kXKeys / 256;      // bytes per LDS row; pieces per thread
@@ -361,13 +366,18 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             qf[u][s] = c < dk ? pi_ld16(src) : pi_u32x4{0, 0, 0, 0};
         }
     pi_u32x4 kr[KP], vr[VP];
+    int cell[KP];                                      // the cache cells of the next fetch, requested a step before it: looked up inside it, each would be waited for
+    auto cells = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < KP; ++j) cell[j] = p.list[min(k0 + (tid + 256 * j) / (KS * 4), n_keys - 1)];
+    };
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < KP; ++j) {
             const int e = tid + 256 * j, key = min(k0 + e / (KS * 4), n_keys - 1), c = (e % (KS * 4)) * 8;
-            const bf16 * src = c < p.dim ? (const bf16 *)p.keys + ((size_t)key * p.n_head + h) * p.dim + c
-                                         : (const bf16 *)p.cache + (size_t)p.list[key] * p.kd + p.rank_ld + (min(c, dk - 8) - p.dim);
-            kr[j] = pi_ld16(src);                      // (unconditional loads: past the end of a row its last piece, zeroed on the way to LDS)
+            const bf16 * un = (const bf16 *)p.keys + ((size_t)key * p.n_head + h) * p.dim + c;
+            const bf16 * rot = (const bf16 *)p.cache + (size_t)cell[j] * p.kd + p.rank_ld + (min(c, dk - 8) - p.dim);
+            kr[j] = pi_ld16(c < p.dim ? un : rot);     // (unconditional loads: past the end of a row its last piece, zeroed on the way to LDS)
         }
 #pragma unroll
         for (int j = 0; j < VP; ++j) {
@@ -375,7 +385,10 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             vr[j] = pi_ld16((const bf16 *)p.values + ((size_t)key * p.n_head + h) * p.vdim + c);
         }
     };
+    cells(0);
     fetch(0);
+    cells(kXKeys);
+    const float c2 = p.scale * kLog2e;                 // scores and maxima in base 2: a weight is one subtraction and one v_exp_f32
     float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
     pi_f4 o[2][VT];
 #pragma unroll
@@ -390,6 +403,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
         for (int j = 0; j < VP; ++j) { const int e = tid + 256 * j; *reinterpret_cast<pi_u32x4 *>(vs + (e / (VT * 2)) * VROW + (e % (VT * 2)) * 16) = vr[j]; }
         __syncthreads();
         fetch(k0 + kXKeys);
+        cells(k0 + 2 * kXKeys);
         pi_f4 s[2][4];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -410,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = s[u][kt][r] * p.scale;
+                    float v = s[u][kt][r] * c2;
                     if (edge && k0 + kt * 16 + 4 * g + r >= nv[u]) v = -INFINITY;
                     s[u][kt][r] = v;
                     mx = fmaxf(mx, v);
@@ -418,14 +432,14 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             mx = fmaxf(mx, __shfl_xor(mx, 16, PI_WAVE));
             mx = fmaxf(mx, __shfl_xor(mx, 32, PI_WAVE));
             const float mn = fmaxf(m[u], mx), base = mn == -INFINITY ? 0.0f : mn;
-            const float a = expf(m[u] - base);         // 0 while nothing has been seen
+            const float a = exp2_hw(m[u] - base);       // 0 while nothing has been seen
             m[u] = mn;
             float sum = 0.0f;
             bf16 w[16];
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) { const float e = expf(s[u][kt][r] - base); sum += e; w[kt * 4 + r] = (bf16)e; }
+                for (int r = 0; r < 4; ++r) { const float e = exp2_hw(s[u][kt][r] - base); sum += e; w[kt * 4 + r] = (bf16)e; }
             l[u] = l[u] * a + sum;
 #pragma unroll
             for (int v = 0; v < VT; ++v) { o[u][v][0] *= a; o[u][v][1] *= a; o[u][v][2] *= a; o[u][v][3] *= a; }
@@ -449,13 +463,13 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
                 o[1][v] = mfma_bf16(f, pb[1][k], o[1][v]);
             }
     }
-    const float sink = p.sink[h];
+    const float sink = p.sink[h] * kLog2e;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         float sum = l[u];
         sum += __shfl_xor(sum, 16, PI_WAVE);
         sum += __shfl_xor(sum, 32, PI_WAVE);
-        const float mf = fmaxf(m[u], sink), a = m[u] == -INFINITY ? 0.0f : expf(m[u] - mf), f = a / (sum * a + expf(sink - mf));
+        const float mf = fmaxf(m[u], sink), a = m[u] == -INFINITY ? 0.0f : exp2_hw(m[u] - mf), f = a / (sum * a + exp2_hw(sink - mf));
         if (q0 + wave * 32 + u * 16 + i >= p.T) continue;
         bf16 * out = (bf16 *)p.att + (size_t)tok[u] * p.ld_att + h * p.vdim;
 #pragma unroll
