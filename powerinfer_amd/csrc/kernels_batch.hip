@@ -105,6 +105,73 @@ __global__ __launch_bounds__(1024) void norm_round_f16_kernel(const float * __re
     }
 }
 
+// The same with 256 threads a row and 16-byte accesses (cols % 4 == 0, cols <= 8192, 16-byte rows, no Q8_0 blocks): 16 waves a row leave two rows
+// on a CU, each with its own memory trip and barriers.  It is the faster one everywhere, by the most where rows are many: 2046 tokens of
+// 512 / 4096 / 8192 columns 17.9 / 20.0 / 26.6 -> 5.1 / 10.6 / 19.2 us (4096: 50 MB), 16 tokens of 4096 4.7 -> 4.2 us.
+__global__ __launch_bounds__(256) void norm_round_rows_kernel(const float * __restrict__ x, int cols, NormArgs na, __half * __restrict__ out, __half * __restrict__ out_plain, int ol) {
+    __shared__ double red[4];
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    constexpr int N = 8;
+    const int tid = threadIdx.x, last = cols - 4;
+    const float * xt = x + (size_t)blockIdx.x * cols;
+    const bool has_w = na.kind != 0 && na.w, has_b = na.kind != 0 && na.b;
+    float4 xv[N], wv[N], bv[N];                        // requested together: one memory trip
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        if (k * 1024 < cols) {
+            const int i = min(4 * tid + k * 1024, last);
+            xv[k] = *reinterpret_cast<const float4 *>(xt + i);
+            if (has_w) wv[k] = *reinterpret_cast<const float4 *>(na.w + i);
+            if (has_b) bv[k] = *reinterpret_cast<const float4 *>(na.b + i);
+        }
+    float mean = 0.0f, scale = 1.0f;
+    if (na.kind == 1) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (4 * tid + k * 1024 < cols) s += ((double)__fmul_rn(xv[k].x, xv[k].x) + (double)__fmul_rn(xv[k].y, xv[k].y)) + ((double)__fmul_rn(xv[k].z, xv[k].z) + (double)__fmul_rn(xv[k].w, xv[k].w));
+        scale = pi_inv_sqrt((float)(block_sum_f64(s, red) / cols) + na.eps);
+    } else if (na.kind == 2) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (4 * tid + k * 1024 < cols) s += ((double)xv[k].x + (double)xv[k].y) + ((double)xv[k].z + (double)xv[k].w);
+        mean = (float)(block_sum_f64(s, red) / cols);
+        s = 0.0;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (4 * tid + k * 1024 < cols) {
+                const float v[4] = {__fsub_rn(xv[k].x, mean), __fsub_rn(xv[k].y, mean), __fsub_rn(xv[k].z, mean), __fsub_rn(xv[k].w, mean)};
+                s += ((double)__fmul_rn(v[0], v[0]) + (double)__fmul_rn(v[1], v[1])) + ((double)__fmul_rn(v[2], v[2]) + (double)__fmul_rn(v[3], v[3]));
+            }
+        scale = pi_inv_sqrt((float)(block_sum_f64(s, red) / cols) + na.eps);
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int i = 4 * tid + k * 1024;
+        if (i >= cols) break;
+        float v[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
+        const size_t at = ol ? pi_ol_index(blockIdx.x, i) : (size_t)blockIdx.x * cols + i;           // (a piece of eight columns is contiguous in both)
+        if (out_plain) *reinterpret_cast<h4 *>(out_plain + at) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        if (na.kind != 0) {
+            const float w[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w}, b[4] = {bv[k].x, bv[k].y, bv[k].z, bv[k].w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                v[q] = __fmul_rn(na.kind == 2 ? __fsub_rn(v[q], mean) : v[q], scale);
+                if (has_w) v[q] = __fmul_rn(v[q], w[q]);
+                if (has_b) v[q] = __fadd_rn(v[q], b[q]);
+            }
+        }
+        *reinterpret_cast<h4 *>(out + at) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+    }
+}
+
+void launch_norm_round(const float * x, int T, int cols, NormArgs na, void * out, void * out_plain, int ol, hipStream_t st) {
+    if (cols % 4 == 0 && cols <= 8192 && (((uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b | (uintptr_t)out | (uintptr_t)out_plain) & 15) == 0)
+        hipLaunchKernelGGL(norm_round_rows_kernel, dim3(T), dim3(256), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, ol);
+    else hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, 0, ol);
+}
+
 // y[t][row] = epi( W[row] . xn[t] ), t < T <= 16.  A workgroup owns 16*RT rows; its four waves split the columns in
 // quarters (cols % 128 == 0) and merge their 16 x 16 accumulator tiles through LDS in wave order.  A wave loads each
 // activation fragment once per 32-column step and uses it for its RT row tiles (the activations of a step are 16 x cols
@@ -1081,13 +1148,13 @@ extern "C" {
 
 int pi_k_norm_round_f16(const float * x, int T, int cols, const pi_norm * norm, void * out_f16, void * out_plain_f16, pi_stream_t stream) {
     if (!x || !out_f16 || T <= 0 || cols <= 0) return pi::fail(PI_E_ARG, "pi_k_norm_round_f16: bad arguments");
-    hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, (hipStream_t)stream, x, cols, to_norm(norm), (__half *)out_f16, (__half *)out_plain_f16, 0, 0);
+    launch_norm_round(x, T, cols, to_norm(norm), out_f16, out_plain_f16, 0, (hipStream_t)stream);
     return pi::check_launch("pi_k_norm_round_f16");
 }
 
 int pi_k_norm_round_f16_ol(const float * x, int T, int cols, const pi_norm * norm, void * out_ol, void * out_plain_ol, pi_stream_t stream) {
     if (!x || !out_ol || T <= 0 || T > kBtMaxT || cols <= 0 || cols % 8) return pi::fail(PI_E_ARG, "pi_k_norm_round_f16_ol: 1 <= T <= 16 and cols % 8 == 0 required");
-    hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, (hipStream_t)stream, x, cols, to_norm(norm), (__half *)out_ol, (__half *)out_plain_ol, 0, 1);
+    launch_norm_round(x, T, cols, to_norm(norm), out_ol, out_plain_ol, 1, (hipStream_t)stream);
     return pi::check_launch("pi_k_norm_round_f16_ol");
 }
 
