@@ -305,65 +305,82 @@ __global__ __launch_bounds__(256) void mix_and_up_kernel(pi_gqa_attn p, pi_gate_
 }
 
 // ---------------------------------------------------------------------------------------------------------------------------------
-// what closes a layer: out[t] = x[t] + (W_o att[t] + sum over the token's experts of W_down[e] act[pair]), 16 rows a workgroup (or, what closes a
-// sublayer in front of its norm: out[t] = alpha x[t] + gate * W att[t]).  The
-// pieces of 256 columns of W_o and of every expert of the step form one list that the waves take in turn.
+// what closes a layer: out[t] = x[t] + (W_o att[t] + sum over the token's experts of W_down[e] act[pair]), 16 or 8 rows a workgroup (or, what
+// closes a sublayer in front of its norm: out[t] = alpha x[t] + gate * W att[t]).  The pieces of 256 (8 rows: 512) columns of W_o and of every
+// expert of the step form one list that the waves take in turn.
+// Bound by the weights.  A piece's tokens were once read when its turn came: loads return in order, so each piece also waited for the weights
+// requested after it and a wave had one piece in flight instead of two; and 16 rows a workgroup leave half the compute units idle at 2048 rows.
+// 16 tokens, 2048 rows, 51 of 64 experts of 1408 (306 MB) and dense layers in turn: 65.7 us a layer, 56 with 8 rows and both requested
+// together, 52.6 with the requests free of branches.
 // ---------------------------------------------------------------------------------------------------------------------------------
-template <int NW>
+template <int NW, int RT>      // waves, rows a workgroup
 __global__ __launch_bounds__(64 * NW) void layer_out_step_kernel(pi_layer_out a) {
-    __shared__ __align__(16) unsigned char tiles[NW][16 * kWsStride];
+    constexpr int COLS = 4096 / RT, NX = COLS / 32, LR = COLS / 8, PITCH = COLS * 2 + 16;      // columns of a piece (eight loads of a wave), its steps of 32, lanes of a row, bytes of a staged row
+    __shared__ __align__(16) unsigned char tiles[NW][RT * PITCH];
     __shared__ StepExperts se;
     __shared__ int first[kStepExperts];
     // (eight waves: the workgroup's LDS exceeds half a compute unit's, so that no two share one while others idle)
     static_assert(NW < 8 || sizeof(tiles) + sizeof(se) + sizeof(first) > 80 * 1024, "one workgroup per compute unit");
-    const int tid = threadIdx.x, wave = tid >> 6;
-    const WaveStream ws(tiles[wave]);
-    const int row0 = blockIdx.x * 16, n_o = a.wo ? (a.ld_att + 255) / 256 : 0, n_e = a.ids ? (a.ld_act + 255) / 256 : 1;
-    const int tok = min(ws.i, a.T - 1);
-    const bf16 * wo = (const bf16 *)a.wo, * down = (const bf16 *)a.down;
-    pi_u32x4 ld[2][8];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * RT, n_o = a.wo ? (a.ld_att + COLS - 1) / COLS : 0, n_e = a.ids ? (a.ld_act + COLS - 1) / COLS : 1;
+    const int tok = min(i, a.T - 1);
+    pi_u32x4 ld[2][8], x[2][NX];
+    int left[2];                                       // columns of the piece and behind it; 0: the token has no part in it
     pi_f4 acc = pi_f4{0, 0, 0, 0};
-    auto load = [&](pi_u32x4 (&l)[8], int ss) {
-        if (ss < n_o) { ws.load(l, wo, a.ld_att, row0, a.rows, ss * 256, a.ld_att); return; }
-        const int k = (ss - n_o) / n_e, c = (ss - n_o) % n_e;
-        ws.load(l, down + (size_t)se.expert[k] * a.rows * a.ld_act, a.ld_act, row0, a.rows, c * 256, a.ld_act);
+    // a piece's weights and its tokens' values are requested together, two pieces ahead and without branches (past the end: the last columns again)
+    auto request = [&](pi_u32x4 (&l)[8], pi_u32x4 (&v)[NX], int & rest, int ss) {
+        const bool att = ss < n_o;
+        const int k = att ? 0 : (ss - n_o) / n_e, c = (att ? ss : (ss - n_o) % n_e) * COLS, cols = att ? a.ld_att : a.ld_act;
+        const bf16 * w = att ? (const bf16 *)a.wo : (const bf16 *)a.down + (size_t)se.expert[k] * a.rows * a.ld_act;
+        const int at = min(c + (lane % LR) * 8, cols - 8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) l[j] = pi_ld_stream(w + (size_t)min(row0 + j * (RT / 8) + lane / LR, a.rows - 1) * cols + at);
+        const int pair = att ? tok : se.slot[k][i];
+        const bf16 * xp = (att ? (const bf16 *)a.att : (const bf16 *)a.act) + (size_t)max(pair, 0) * cols;
+#pragma unroll
+        for (int st = 0; st < NX; ++st) v[st] = pi_ld16(xp + min(c + st * 32, cols - 32) + g * 8);
+        rest = pair >= 0 ? cols - c : 0;
     };
     // the attention's pieces are requested before the experts are known
-    if (wave < n_o) load(ld[0], wave);
-    if (wave + NW < n_o) load(ld[1], wave + NW);
+    if (wave < n_o) request(ld[0], x[0], left[0], wave);
+    if (wave + NW < n_o) request(ld[1], x[1], left[1], wave + NW);
     const int n_exp = a.ids ? step_experts(se, first, a.ids, a.T * a.top, a.top, a.n_expert) : 0, n_ss = n_o + n_exp * n_e;
-    if (wave >= n_o && wave < n_ss) load(ld[0], wave);
-    if (wave + NW >= n_o && wave + NW < n_ss) load(ld[1], wave + NW);
-    for (int s0 = wave; s0 < n_ss; s0 += 2 * NW) {
+    const int m = wave < n_ss ? (n_ss - wave + NW - 1) / NW : 0;                 // this wave's pieces: wave, wave + NW, ...
+    if (wave >= n_o && m > 0) request(ld[0], x[0], left[0], wave);
+    if (wave + NW >= n_o && m > 1) request(ld[1], x[1], left[1], wave + NW);
+    auto multiply = [&](const pi_u32x4 (&l)[8], const pi_u32x4 (&v)[NX], int rest) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<pi_u32x4 *>(tiles[wave] + (j * (RT / 8) + lane / LR) * PITCH + (lane % LR) * 16) = l[j];
+#pragma unroll
+        for (int st = 0; st < NX; ++st)
+            acc = mma16<bf16>(*reinterpret_cast<const pi_u32x4 *>(tiles[wave] + (i % RT) * PITCH + (4 * st + g) * 16), st * 32 < rest ? v[st] : pi_u32x4{0, 0, 0, 0}, acc);
+    };
+    // (no branch around a request while pieces are left for both buffers: what a wait leaves in flight is then known when it is compiled)
+    int it = 0;
+    for (; it + 4 <= m; it += 2)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            const int ss = s0 + b * NW;
-            if (ss < n_ss) {
-                const bool att = ss < n_o;
-                const int k = att ? 0 : (ss - n_o) / n_e, c = (att ? ss : (ss - n_o) % n_e) * 256, cols = att ? a.ld_att : a.ld_act;
-                const int pair = att ? 0 : se.slot[k][ws.i];
-                const bf16 * xp = att ? (const bf16 *)a.att + (size_t)tok * a.ld_att : (const bf16 *)a.act + (size_t)max(pair, 0) * a.ld_act;
-                pi_u32x4 x[8];
-#pragma unroll
-                for (int st = 0; st < 8; ++st) x[st] = c + st * 32 < cols && pair >= 0 ? pi_ld16(xp + c + st * 32 + ws.g * 8) : pi_u32x4{0, 0, 0, 0};
-                ws.multiply(ld[b], x, acc);
-                if (ss + 2 * NW < n_ss) load(ld[b], ss + 2 * NW);
-            }
+            multiply(ld[b], x[b], left[b]);
+            request(ld[b], x[b], left[b], wave + (it + 2 + b) * NW);
         }
-    }
+    const int rem = m - it;
+    if (rem >= 1) multiply(ld[0], x[0], left[0]);
+    if (rem == 3) request(ld[0], x[0], left[0], wave + (it + 2) * NW);
+    if (rem >= 2) multiply(ld[1], x[1], left[1]);
+    if (rem == 3) multiply(ld[0], x[0], left[0]);
     float (*cs)[17] = reinterpret_cast<float (*)[17]>(tiles[wave]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) cs[4 * ws.g + r][ws.i] = acc[r];
+    for (int r = 0; r < 4; ++r) if (4 * g + r < RT) cs[4 * g + r][i] = acc[r];
     __syncthreads();
-    if (tid >= 256) return;
-    const int t = tid >> 4, row = row0 + (tid & 15);
+    if (tid >= 16 * RT) return;
+    const int t = tid / RT, row = row0 + tid % RT;
     if (row >= a.rows || t >= a.T) return;
     float v = 0.0f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) v += reinterpret_cast<float (*)[17]>(tiles[w])[tid & 15][t];
+    for (int w = 0; w < NW; ++w) v += reinterpret_cast<float (*)[17]>(tiles[w])[tid % RT][t];
     if (a.gate_z) v *= sigmoid_f32(a.gate_z[(size_t)t * a.ld_gate + a.off_gate + row] + a.gate_b[row]);
-    const float x = a.x ? a.x[(size_t)t * a.rows + row] : 0.0f;
-    v += a.scaled ? a.alpha * x : x;
+    const float x0 = a.x ? a.x[(size_t)t * a.rows + row] : 0.0f;
+    v += a.scaled ? a.alpha * x0 : x0;
     a.out[(size_t)t * a.rows + row] = v;
     if (a.keep) a.keep[(size_t)t * a.rows + row] = v;
 }
@@ -439,9 +456,11 @@ int pi_k_layer_out_step(const pi_layer_out * a, pi_stream_t stream) {
         (a->ids && (!a->down || !a->act || a->ld_act <= 0 || a->ld_act % 32 || a->top <= 0 || a->T * a->top > kStepPairs || a->n_expert <= 0 || a->n_expert > kStepExperts)))
         return pi::fail(PI_E_ARG, "pi_k_layer_out_step: bad arguments");
     // eight waves a workgroup when every workgroup has a compute unit to itself, four (and several workgroups a unit) beyond
-    const int n = (a->rows + 15) / 16;
-    if (n <= pi::compute_units() ) hipLaunchKernelGGL(layer_out_step_kernel<8>, dim3(n), dim3(512), 0, (hipStream_t)stream, *a);
-    else hipLaunchKernelGGL(layer_out_step_kernel<4>, dim3(n), dim3(256), 0, (hipStream_t)stream, *a);
+    // Eight rows a workgroup (half of each matrix tile repeats them) while 16 would leave half the units without one.
+    const int n = (a->rows + 15) / 16, cus = pi::compute_units();
+    if (2 * n <= cus) hipLaunchKernelGGL((layer_out_step_kernel<8, 8>), dim3((a->rows + 7) / 8), dim3(512), 0, (hipStream_t)stream, *a);
+    else if (n <= cus) hipLaunchKernelGGL((layer_out_step_kernel<8, 16>), dim3(n), dim3(512), 0, (hipStream_t)stream, *a);
+    else hipLaunchKernelGGL((layer_out_step_kernel<4, 16>), dim3(n), dim3(256), 0, (hipStream_t)stream, *a);
     return pi::check_launch("pi_k_layer_out_step");
 }
 
