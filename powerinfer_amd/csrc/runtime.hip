@@ -1,4 +1,5 @@
 // Device/runtime plumbing of the C ABI: init, memory, copies, events, error string.
+#include <mutex>
 #include "runtime.hpp"
 #include "../../include/powerinfer_hip.h"
 
@@ -56,19 +57,43 @@ __global__ __launch_bounds__(256) void copy_out_kernel(CopyOut c, uint32_t * __r
 }  // namespace
 
 namespace pi {
+namespace {
+std::mutex pinned_lock;
+struct { unsigned char * p; size_t bytes; } pinned_kept[HostStage::kKept];
+int pinned_n = 0, pinned_users = 0;
+}  // namespace
+
 void HostStage::init(size_t usual_bytes) {
-    if (pin) return;
+    if (counted) return;
     const size_t want = usual_bytes + 4096;
     n_pieces = want > kPiece ? kPieces : 1;
     piece = n_pieces > 1 ? kPiece : (want + 4095) / 4096 * 4096;
-    if (hipHostMalloc((void **)&pin, piece * n_pieces, hipHostMallocDefault) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
+    counted = true;
+    {
+        std::lock_guard<std::mutex> held(pinned_lock);
+        ++pinned_users;
+        for (int i = 0; i < pinned_n && !pin; ++i)
+            if (pinned_kept[i].bytes == piece * n_pieces) { pin = pinned_kept[i].p; pinned_kept[i] = pinned_kept[--pinned_n]; }
+    }
+    if (!pin && hipHostMalloc((void **)&pin, piece * n_pieces, hipHostMallocPortable) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
     for (int i = 0; i < n_pieces && pin; ++i)
         if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) { ev[i] = nullptr; (void)hipGetLastError(); release(); }
 }
 
 void HostStage::release() {
     for (hipEvent_t & e : ev) if (e) { (void)hipEventDestroy(e); e = nullptr; }
-    if (pin) { (void)hipHostFree(pin); pin = nullptr; }
+    if (!counted) return;
+    counted = false;
+    unsigned char * out[kKept + 1];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> held(pinned_lock);
+        if (pin && !busy && pinned_n < kKept) { pinned_kept[pinned_n].p = pin; pinned_kept[pinned_n++].bytes = piece * n_pieces; }
+        else if (pin) out[n++] = pin;
+        if (--pinned_users == 0) while (pinned_n) out[n++] = pinned_kept[--pinned_n].p;
+    }
+    pin = nullptr;
+    while (n) (void)hipHostFree(out[--n]);
 }
 
 int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
@@ -84,6 +109,7 @@ int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
         return PI_OK;
     }
     if (m == 0) { PI_HIP_TRY(hipStreamSynchronize(st)); return PI_OK; }
+    busy = true;                                                    // until the stream has been waited for
     // the last result in pieces; the first one leaves room for the others
     const HostCopy & big = c[m - 1];
     size_t sent = 0, taken = 0;                                     // bytes of it
@@ -112,6 +138,7 @@ int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
         memcpy((unsigned char *)big.host + from[slot], s + (fetched ? 0 : small), len[slot]);
         taken += len[slot]; ++fetched;
     }
+    busy = false;
     return PI_OK;
 }
 }  // namespace pi

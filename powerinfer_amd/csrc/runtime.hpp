@@ -23,16 +23,17 @@ int  noalloc_setup();                                  // resolves the static sc
 // A call's results on their way from the device to the caller's memory.  A copy to pageable memory costs 13 us for 4 bytes and 62 us for the
 // 128 KB of 32000 logits, each with a wait of its own; here one small kernel behind the call's last one stores all of them in pinned
 // memory, one wait covers both, and a memcpy (3 us for 128 KB, still in the host's cache) brings them home.  Larger results (2 MB: 16
-// rows of logits) travel in pieces of 512 KB through two places, each copied while the next one crosses the link.  Four places are 80 us of a
-// 13B step of 16 tokens faster, but pinning 2 MB costs a new model 0.7 ms and its first call 0.2 ms; 128 KB pieces lose 200 us of that step.
-// Part of one model, used by one call at a time.
+// rows of logits) travel in pieces of 512 KB, each copied while the next ones cross the link.  Part of one model, used by one call at a time.
+// Pinning 2 MB takes 0.7 ms and the first call on them 0.2 to 0.3 ms more: a model that goes leaves its memory to the next ones (at most kKept
+// such buffers; the last model of the process gives all of them back).
 struct HostCopy { const void * dev; void * host; size_t bytes; };        // multiples of 4 bytes, dev 4-byte aligned; host null: not wanted
 struct HostStage {
-    static constexpr int kPieces = 2, kMaxCopies = 4;
+    static constexpr int kPieces = 4, kMaxCopies = 4, kKept = 4;
     static constexpr size_t kPiece = (size_t)512 << 10;
     unsigned char * pin = nullptr;         // null (no pinned memory to be had): ordinary copies
     size_t piece = 0; int n_pieces = 0;
     hipEvent_t ev[kPieces] = {};
+    bool counted = false, busy = false;    // one of the pool's users; a call ended early, work on the memory may be left
     void init(size_t usual_bytes);
     void release();
     // queues the copies behind what the stream holds and returns when the stream is done and the results are in place; all but the

@@ -27,3 +27,32 @@ def test_logits_arrive_whole(n_vocab):
         again, lg2 = gm.decode([tok], pos, want_logits=False)
         assert again == one and lg2 is None
     gm.close()
+
+
+def test_models_that_come_and_go():
+    """A model's pinned memory passes to the next one: models made and closed in turn on four threads, every result as the first model's."""
+    import threading
+
+    from powerinfer_amd.model import Model
+    hp = synth.hparams("llama-tiny", n_vocab=9001, n_ctx=64, seed=11, sparse_threshold=-1e30)
+    weights, toks = synth.make_model(hp), [5, 8999, 17]
+
+    def rows():
+        gm = Model(hp).load(weights)
+        out = [gm.decode([t], k)[1].copy() for k, t in enumerate(toks)]
+        gm.close()
+        return np.stack(out)
+
+    want, got = rows(), []
+
+    def work():
+        for _ in range(3):
+            got.append(rows())
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    print(len(got), flush=True)
+    assert len(got) == 12 and all(np.array_equal(g, want) for g in got)
