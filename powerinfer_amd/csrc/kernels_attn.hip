@@ -774,16 +774,24 @@ __global__ __launch_bounds__(kBlock) void attn_chunk_mfma_kernel(const float * _
 // Q4_0 model's next rounding to eight bits then falls the other way for one activation in forty.
 // Scores are formed transposed (cells x tokens): a lane's scores belong to one token, and its weights are already the column operand of
 // values^T x weights - which cell a slot of that product's inner dimension stands for is free, so the values are read (transposed,
-// ds_read_tr16) in the order the scores came out.  The sum of a tile is one more product, with ones.
+// ds_read_tr16) in the order the scores came out.  A row's sum is exact, whatever the order.
 // Bound by the exponentials (about 40 cycles of VALU per 64 of them) beside 48 of matrix cores.  32 heads of 128, RoPE and store included:
-// 512 tokens behind 0 / 512 / 1024 / 1535: 49 / 74 / 99 / 118 us (attn_chunk_mfma_kernel 61 / 117 / 159, attn_decode_kernel 791 past the
-// cells that one holds), 2046 tokens at once 222; 128 heads of 64 on 8: 60 / 107 / 155 / 196 (94 / 271 / 380 / 493).
+// 512 tokens behind 0 / 512 / 1024 / 1535: 43 / 65 / 87 / 110 us (attn_chunk_mfma_kernel 51 / 104 / 145, attn_decode_kernel 700 past the
+// cells that one holds), 2046 tokens at once 196 (190 with the sums of 64 weights in float32); 128 heads of 64 on 8: 52 / 98 / 143 / 186
+// (75 / 255 / 364 / 479).
 // ---------------------------------------------------------------------------------------------------
 typedef short pi_s4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ pi_u32x2 lds_tr_read(const unsigned char * q) {
     return __builtin_bit_cast(pi_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) pi_s4 *)(__attribute__((address_space(3))) void *)q));
 }
 constexpr int kRowsCells = 64;                 // cells of a tile
+// a soft-max weight (fp16, 0 .. 1) in units of 2^-24; no number counts 0 (the instruction's result, where a C++ conversion has none): its weight
+// itself takes it to the output
+__device__ __forceinline__ uint32_t weight_units(_Float16 w) {
+    uint32_t n;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(n) : "v"((float)w * 16777216.0f));
+    return n;
+}
 template <int HD> constexpr int rows_pitch() { return HD * 2 + 16; }                       // bytes of a staged row: 16 of padding spread the rows over the banks
 template <int HD> constexpr size_t rows_lds() { return (size_t)4 * kRowsCells * rows_pitch<HD>(); }
 
@@ -880,10 +888,8 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         base[u] = mx[u] == -INFINITY ? 0.0f : __fmul_rn(mx[u], scale);
     }
 
-    // e = fp16(exp(fp16(s - max))) of a tile as the column operand, times f where the sums are known.  e^x = 2^n 2^(x log2 e - n): log2 e in
-    // two parts, the first short enough for its product with an fp16 number to be exact, so that 2^ is off by little more than its own rounding
-    auto weigh = [&](const pi_f4 * s, int cb, bool edge, int seen, float b, bool last_pass, float f, pi_u32x4 * out) {
-        _Float16 w[4 * KT];
+    // e = fp16(exp(fp16(s - max))) of a lane's cells of a tile.  e^x = 2^n 2^(x log2 e - n): log2 e in two parts, the first short enough for its product with an fp16 number to be exact, so that 2^ is off by little more than its own rounding
+    auto weigh = [&](const pi_f4 * s, int cb, bool edge, int seen, float b, _Float16 * w) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
@@ -891,22 +897,30 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
                 const float x = (float)(_Float16)__fsub_rn(__fmul_rn(s[kt][r], scale), b);
                 const float n = fmaxf(__builtin_rintf(x * 1.4426950408889634f), -200.0f);        // x may be -inf
                 const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 6.808776379330084e-05f, fmaf(x, 1.442626953125f, -n))), (int)n);
-                _Float16 v = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= seen ? 0.0f : e);
-                if (last_pass) v = (_Float16)__fmul_rn((float)v, f);
-                w[kt * 4 + r] = v;
+                w[kt * 4 + r] = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= seen ? 0.0f : e);
             }
-#pragma unroll
-        for (int k = 0; k < KT / 2; ++k)
-            out[k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
     };
 
-    // ---- the rows' sums: 64 weights by a product with ones, the tiles in double ----
+    // ---- the rows' sums, exact as the CPU path's sums in double are: a weight is a whole number of 2^-24, of which a lane adds 16 a tile ----
     double sum[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) sum[u] = 0.0;
-    const pi_u32x4 ones{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+    auto add_weights = [&](const _Float16 * w, double & to) {
+        uint32_t part = 0;                                               // at most 2^28
+#pragma unroll
+        for (int k = 0; k < 4 * KT; ++k) part += weight_units(w[k]);
+        to += (double)part;
+    };
+    auto total = [&]() {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            sum[u] += __shfl_xor(sum[u], 16, PI_WAVE);
+            sum[u] += __shfl_xor(sum[u], 32, PI_WAVE);
+            sum[u] *= 5.9604644775390625e-08;                            // 2^-24
+        }
+    };
     fetch(pk, kb, 0);
-    __syncthreads();                                                     // the last tile of the pass before has been read
+    __syncthreads();                                                 // the last tile of the pass before has been read
     at = 0;
     for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
         place(smem + at * TILE, pk);
@@ -917,14 +931,12 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         const bool edge = cb + NK > n_all;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            pi_u32x4 pb[KT / 2];
-            weigh(s[u], cb, edge, nv[u], base[u], false, 0.0f, pb);
-            pi_f4 l = pi_f4{0, 0, 0, 0};
-#pragma unroll
-            for (int k = 0; k < KT / 2; ++k) l = mma16<__half>(ones, pb[k], l);
-            sum[u] += (double)l[0];
+            _Float16 w[4 * KT];
+            weigh(s[u], cb, edge, nv[u], base[u], w);
+            add_weights(w, sum[u]);
         }
     }
+    total();
 
     // ---- weights and values ----
     float inv[U];
@@ -959,7 +971,15 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         products(smem + at * TILE, s);
         pi_u32x4 pb[U][KT / 2];
 #pragma unroll
-        for (int u = 0; u < U; ++u) weigh(s[u], cb, edge, nv[u], base[u], true, inv[u], pb[u]);
+        for (int u = 0; u < U; ++u) {
+            _Float16 w[4 * KT];
+            weigh(s[u], cb, edge, nv[u], base[u], w);
+#pragma unroll
+            for (int k = 0; k < 4 * KT; ++k) w[k] = (_Float16)__fmul_rn((float)w[k], inv[u]);
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k)
+                pb[u][k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
+        }
         const unsigned char * vs = vt + at * TILE;
         if (edge && odd[at]) {
             // 0 times such a value is no number either: token by token, the cells it sees only.  The weight of cell (kt, g, r) of token i is

@@ -70,6 +70,59 @@ def test_rows_match_float64(hd, nh, nkv, mode, past, T, n_ctx):
         assert err < 2e-3, (a, err)
 
 
+def exact_weights(T, past, seed, whole, n_ctx):
+    """Scores, cells and queries that every step up to the weights forms without rounding but the CPU path's own: (qkv, K, V, what comes out bit
+    for bit).  Scores are multiples of 1/128, the values of cell c a one in column c % 64, so that a column is the exact sum of its
+    cells' weights.  whole: the weights are not divided by their sum before they meet the values."""
+    hd = 64
+    rng = np.random.default_rng(seed)
+    q, k = np.zeros((T, hd), np.float32), np.zeros((past + T, hd), np.float32)
+    q[:, 0], q[:, 1] = rng.integers(1, 4, T) / 4, 1
+    k[:, 0], k[:, 1] = rng.integers(-60, 1, past + T), rng.integers(-8, 9, past + T) * 0.25          # s / 8: -5.6 q .. 0.3
+    k[rng.integers(0, past + T, 3 + (past + T) // 40), 0] = rng.integers(20, 90)
+    v = np.zeros((past + T, hd), np.float16)
+    v[np.arange(past + T), np.arange(past + T) % hd] = 1
+    s = (q.astype(np.float64) @ k.T.astype(np.float64)).astype(np.float32) * np.float32(0.125)
+    seen = np.arange(past + T)[None] <= (past + np.arange(T))[:, None]
+    x = np.where(seen, s - np.where(seen, s, -np.inf).max(1, keepdims=True), -np.inf)
+    x = x if whole else x.astype(np.float16)
+    ex = np.exp(x.astype(np.float64))
+    e = ex.astype(np.float16)
+    vals = np.unique(ex[seen])                                            # no exponential lies within two units of float32 of where fp16 rounds the other way
+    for d in (-2, 2):
+        assert np.array_equal((vals * (1 + d * 2.0 ** -23)).astype(np.float16), vals.astype(np.float16))
+    total = e.astype(np.float64).sum(1, keepdims=True)
+    w = e.astype(np.float64) if whole else (e.astype(np.float32) * (1.0 / total).astype(np.float32)).astype(np.float16).astype(np.float64)
+    out = w @ v.astype(np.float64)
+    if whole:
+        out = (out.astype(np.float32) / total.astype(np.float32)).astype(np.float64)
+    qkv = np.concatenate([q, k[past:], v[past:].astype(np.float32)], 1)
+    kc, vc = np.full((n_ctx, hd), np.nan, np.float16), np.full((n_ctx, hd), np.nan, np.float16)
+    kc[:past], vc[:past] = k[:past], v[:past]
+    return qkv, kc, vc, out
+
+
+def rows_of(qkv, kc, vc, T, past, n_ctx):
+    from powerinfer_amd import lib as pl
+    L = pl.init()
+    dq, dk, dv, dpos = pl.DevBuf(host=qkv), pl.DevBuf(host=kc), pl.DevBuf(host=vc), pl.DevBuf(host=np.arange(past, past + T, dtype=np.int32))
+    rot, out = pl.DevBuf(T * 64 * 4), pl.DevBuf(T * 64 * 4)
+    pl.check(L.pi_k_attn_chunk_rows(dq.ptr, 192, T, 1, 1, 64, 0, 1.0, 0.0, dpos.ptr, n_ctx, past + T, rot.ptr, dk.ptr, dv.ptr, out.ptr, 64, None, None), "attn_chunk_rows")
+    pl.sync()
+    return out.download(np.float32).reshape(T, 64)
+
+
+@pytest.mark.parametrize("T,past", [(700, 0), (130, 1500), (40, 300), (1900, 148)])
+def test_weights_are_those_of_a_sum_in_double_bit_for_bit(T, past):
+    """The soft-max's sum holds every bit of its weights, large and subnormal ones in one tile: 1 / sum, and with it the rounding of each
+    weight to fp16, are the CPU path's."""
+    wrong, n_ctx = 0, past + T + 8
+    for seed in range(4):
+        qkv, kc, vc, want = exact_weights(T, past, 100 * seed + T, False, n_ctx)
+        wrong += int((rows_of(qkv, kc, vc, T, past, n_ctx) != want).any(1).sum())
+    assert wrong == 0, f"{wrong} of {4 * T} rows"
+
+
 def test_what_it_does_not_cover_is_refused():
     from powerinfer_amd import lib as pl
     L, b = pl.init(), pl.DevBuf(1 << 16)
