@@ -521,8 +521,9 @@ PI_API int pi_k_attn_fused_batch_ol(const float * qkv, int qkv_stride, const voi
                                     size_t cache_seq_stride, int n_seq, int n_head, int n_head_kv, int hd, int mode, int n_ctx,
                                     const int32_t * pos, float * out, int out_stride, void * out_ol, pi_stream_t stream);
 /* pi_k_attn_chunk (below) with 64 or 128 tokens of a head per workgroup: any number of tokens and of cells, head sizes 64 and 128, the same rounding
- * points.  out_stride % 4 == 0, buffers on 16 bytes (out_f16 on 8).  pi_k_attn_chunk_rows_supported: whether it is the one to take for T tokens
- * against n_kv_max cells. */
+ * points; where pi_k_attn_chunk_supported says no the scores' differences are not rounded and the weights divided behind the values (one rounding
+ * fewer than pi_k_attn_chunk_long).  out_stride % 4 == 0, buffers on 16 bytes (out_f16 on 8).  pi_k_attn_chunk_rows_supported: whether it
+ * is the one to take for T tokens against n_kv_max cells. */
 PI_API int pi_k_attn_chunk_rows_supported(int hd, int T, int n_kv_max);
 PI_API int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                                 const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride,

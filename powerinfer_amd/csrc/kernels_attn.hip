@@ -795,7 +795,11 @@ __device__ __forceinline__ uint32_t weight_units(_Float16 w) {
 template <int HD> constexpr int rows_pitch() { return HD * 2 + 16; }                       // bytes of a staged row: 16 of padding spread the rows over the banks
 template <int HD> constexpr size_t rows_lds() { return (size_t)4 * kRowsCells * rows_pitch<HD>(); }
 
-template <int HD, int U>
+// WHOLE: the weights meet the values before they are divided (e in fp16, the fp32 result divided once), as the parts of attn_part_kernel do, which
+// is where decoding goes in caches beyond what attn_decode_kernel holds.  Those round fp16(s - max) by their part's maximum, closer to a
+// score than the row's: here s - max stays as it is (40 tokens, 4 heads of 128, 2540 cells, error of the output: four parts 3.6e-4,
+// rounded by the row's maximum 4.3e-4).  The keys are then gone through twice: 512 tokens behind 3000, 32 heads of 128: 177 -> 138 us.
+template <int HD, int U, bool WHOLE>
 __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float * __restrict__ q_rot, const __half * __restrict__ k_cache,
                                                                     const __half * __restrict__ v_cache, int n_head, int n_head_kv, int n_ctx,
                                                                     const int32_t * __restrict__ pos_p, int T, int n_kv_max, float * __restrict__ out,
@@ -888,15 +892,16 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         base[u] = mx[u] == -INFINITY ? 0.0f : __fmul_rn(mx[u], scale);
     }
 
-    // e = fp16(exp(fp16(s - max))) of a lane's cells of a tile.  e^x = 2^n 2^(x log2 e - n): log2 e in two parts, the first short enough for its product with an fp16 number to be exact, so that 2^ is off by little more than its own rounding
+    // e = fp16(exp(fp16(s - max))) of a lane's cells of a tile.  e^x = 2^n 2^(x log2 e - n): log2 e in
+    // two parts, so that 2^ is off by little more than its own rounding
     auto weigh = [&](const pi_f4 * s, int cb, bool edge, int seen, float b, _Float16 * w) {
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = (float)(_Float16)__fsub_rn(__fmul_rn(s[kt][r], scale), b);
-                const float n = fmaxf(__builtin_rintf(x * 1.4426950408889634f), -200.0f);        // x may be -inf
-                const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 6.808776379330084e-05f, fmaf(x, 1.442626953125f, -n))), (int)n);
+                const float d = __fsub_rn(__fmul_rn(s[kt][r], scale), b), x = WHOLE ? d : (float)(_Float16)d;
+                const float n = fmaxf(__builtin_rintf(x * 1.44269504f), -200.0f);                // x may be -inf
+                const float e = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, 1.92596303e-08f, fmaf(x, 1.44269502f, -n))), (int)n);
                 w[kt * 4 + r] = (_Float16)(edge && cb + kt * 16 + 4 * g + r >= seen ? 0.0f : e);
             }
     };
@@ -919,31 +924,33 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
             sum[u] *= 5.9604644775390625e-08;                            // 2^-24
         }
     };
-    fetch(pk, kb, 0);
-    __syncthreads();                                                 // the last tile of the pass before has been read
-    at = 0;
-    for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
-        place(smem + at * TILE, pk);
-        __syncthreads();
-        fetch(pk, kb, cb + NK);
-        pi_f4 s[U][KT];
-        products(smem + at * TILE, s);
-        const bool edge = cb + NK > n_all;
+    if constexpr (!WHOLE) {
+        fetch(pk, kb, 0);
+        __syncthreads();                                                 // the last tile of the pass before has been read
+        at = 0;
+        for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
+            place(smem + at * TILE, pk);
+            __syncthreads();
+            fetch(pk, kb, cb + NK);
+            pi_f4 s[U][KT];
+            products(smem + at * TILE, s);
+            const bool edge = cb + NK > n_all;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            _Float16 w[4 * KT];
-            weigh(s[u], cb, edge, nv[u], base[u], w);
-            add_weights(w, sum[u]);
+            for (int u = 0; u < U; ++u) {
+                _Float16 w[4 * KT];
+                weigh(s[u], cb, edge, nv[u], base[u], w);
+                add_weights(w, sum[u]);
+            }
         }
+        total();
     }
-    total();
 
     // ---- weights and values ----
     float inv[U];
     pi_f4 o[U][VT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        inv[u] = (float)(1.0 / sum[u]);
+        inv[u] = WHOLE ? 1.0f : (float)(1.0 / sum[u]);
 #pragma unroll
         for (int v = 0; v < VT; ++v) o[u][v] = pi_f4{0, 0, 0, 0};
     }
@@ -974,8 +981,11 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         for (int u = 0; u < U; ++u) {
             _Float16 w[4 * KT];
             weigh(s[u], cb, edge, nv[u], base[u], w);
+            if constexpr (WHOLE) add_weights(w, sum[u]);
+            else {
 #pragma unroll
-            for (int k = 0; k < 4 * KT; ++k) w[k] = (_Float16)__fmul_rn((float)w[k], inv[u]);
+                for (int k = 0; k < 4 * KT; ++k) w[k] = (_Float16)__fmul_rn((float)w[k], inv[u]);
+            }
 #pragma unroll
             for (int k = 0; k < KT / 2; ++k)
                 pb[u][k] = __builtin_bit_cast(pi_u32x4, pi_h8{w[k * 8], w[k * 8 + 1], w[k * 8 + 2], w[k * 8 + 3], w[k * 8 + 4], w[k * 8 + 5], w[k * 8 + 6], w[k * 8 + 7]});
@@ -1015,6 +1025,7 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
                 for (int u = 0; u < U; ++u) o[u][v] = mma16<__half>(fr, pb[u][k], o[u][v]);
             }
     }
+    if constexpr (WHOLE) total();
     // o[u][v][r] = out[token i][v * 16 + 4 g + r]
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -1024,7 +1035,8 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
         __half * ph = out16 ? out16 + (size_t)t * out_stride + (size_t)h * HD + 4 * g : nullptr;
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
-            const float4 y{o[u][v][0], o[u][v][1], o[u][v][2], o[u][v][3]};
+            float4 y{o[u][v][0], o[u][v][1], o[u][v][2], o[u][v][3]};
+            if constexpr (WHOLE) { const float d = (float)sum[u]; y = float4{pi_div(y.x, d), pi_div(y.y, d), pi_div(y.z, d), pi_div(y.w, d)}; }
             *reinterpret_cast<float4 *>(po + v * 16) = y;
             if (ph) {
                 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
@@ -1314,12 +1326,12 @@ int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_he
     return pi::check_launch("rope_kv_chunk");
 }
 
-template <int HD, int U>
+template <int HD, int U, bool WHOLE>
 int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_cache, int n_head, int n_head_kv, int n_ctx, const int32_t * pos, int T, int n_kv_max, float * out,
                       int out_stride, void * out_f16, hipStream_t st) {
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_kernel<HD, U>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_kernel<HD, U, WHOLE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
     if (raised != hipSuccess) return pi::hip_fail(raised, "attn_chunk_rows: LDS size");
-    hipLaunchKernelGGL((attn_chunk_rows_kernel<HD, U>), dim3(n_head, (T + 64 * U - 1) / (64 * U)), dim3(kBlock), rows_lds<HD>(), st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
+    hipLaunchKernelGGL((attn_chunk_rows_kernel<HD, U, WHOLE>), dim3(n_head, (T + 64 * U - 1) / (64 * U)), dim3(kBlock), rows_lds<HD>(), st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
                        n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, n_head * HD, out_stride, (__half *)out_f16);
     return pi::check_launch("attn_chunk_rows");
 }
@@ -1549,8 +1561,12 @@ int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, i
     if (rc != PI_OK) return rc;
     // 128 tokens a workgroup where that still leaves two for every compute unit
     const bool two = (long long)n_head * ((T + 127) / 128) >= 2 * pi::compute_units();
-#define PI_ROWS(HD, U) launch_chunk_rows<HD, U>(q_rot, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
-    return hd == 128 ? (two ? PI_ROWS(128, 2) : PI_ROWS(128, 1)) : (two ? PI_ROWS(64, 2) : PI_ROWS(64, 1));
+    // pi_k_attn_chunk's rounding points where it covers the cache; no more than pi_k_attn_chunk_long's beyond
+    const bool whole = !pi_k_attn_chunk_supported(hd, n_ctx, n_kv_max);
+#define PI_ROWS(HD, U, W) launch_chunk_rows<HD, U, W>(q_rot, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
+#define PI_ROWS_U(HD, U) (whole ? PI_ROWS(HD, U, true) : PI_ROWS(HD, U, false))
+    return hd == 128 ? (two ? PI_ROWS_U(128, 2) : PI_ROWS_U(128, 1)) : (two ? PI_ROWS_U(64, 2) : PI_ROWS_U(64, 1));
+#undef PI_ROWS_U
 #undef PI_ROWS
 }
 

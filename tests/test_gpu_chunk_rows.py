@@ -123,6 +123,52 @@ def test_weights_are_those_of_a_sum_in_double_bit_for_bit(T, past):
     assert wrong == 0, f"{wrong} of {4 * T} rows"
 
 
+@pytest.mark.parametrize("T,past", [(70, 2600), (700, 2400), (2048, 500)])
+def test_weights_of_a_large_cache_are_divided_once_in_float32(T, past):
+    """Caches beyond what decoding holds in one workgroup: as in pi_k_attn_chunk_long, which took these chunks, a weight meets its value as fp16(exp)
+    and the fp32 result is divided.  Sums of 40 such products are within 40 units of 2^-24 of the whole, the division within two."""
+    from powerinfer_amd import lib as pl
+    n_ctx = 14000
+    assert not pl.init().pi_k_attn_chunk_supported(64, n_ctx, past + T)
+    qkv, kc, vc, want = exact_weights(T, past, T, True, n_ctx)
+    got = rows_of(qkv, kc, vc, T, past, n_ctx)
+    err = np.abs(got - want).max(1) / np.abs(want).max(1)
+    assert err.max() < 42 * 2.0 ** -24, err.max()
+
+
+@pytest.mark.parametrize("hd,T,past", [(128, 40, 2500), (64, 130, 2600)])
+def test_no_further_from_float64_than_the_kernel_that_splits_cells(hd, T, past):
+    """Against pi_k_attn_chunk_long on one cache, which rounds fp16(s - max of the part) and fp16(exp); here only the latter."""
+    from powerinfer_amd import lib as pl
+    L = pl.init()
+    n_ctx, nh, parts = 14000, 4, 4
+    rng = np.random.default_rng(T)
+    d = nh * hd
+    kc, vc = rng.standard_normal((nh, n_ctx, hd)).astype(np.float16), rng.standard_normal((nh, n_ctx, hd)).astype(np.float16)
+    qkv = rng.standard_normal((T, 3 * d)).astype(np.float32)
+    pos = np.arange(past, past + T, dtype=np.int32)
+    dq, dpos, dk, dv = pl.DevBuf(host=qkv), pl.DevBuf(host=pos), pl.DevBuf(host=kc), pl.DevBuf(host=vc)
+    rot, out, scr = pl.DevBuf(T * d * 4), pl.DevBuf(T * d * 4), pl.DevBuf(int(L.pi_k_attn_split_scratch_floats(T, nh, hd, parts)) * 4)
+    theta, got = float(np.float32(10000.0) ** np.float32(-2.0 / hd)), []
+    for rows in (True, False):
+        if rows:
+            rc = L.pi_k_attn_chunk_rows(dq.ptr, 3 * d, T, nh, nh, hd, 0, theta, 1.0, dpos.ptr, n_ctx, past + T, rot.ptr, dk.ptr, dv.ptr, out.ptr, d, None, None)
+        else:
+            rc = L.pi_k_attn_chunk_long(dq.ptr, 3 * d, T, nh, nh, hd, 0, theta, 1.0, dpos.ptr, n_ctx, parts, scr.ptr, rot.ptr, dk.ptr, dv.ptr, out.ptr, None, None)
+        pl.check(rc, "attention")
+        pl.sync()
+        got.append(out.download(np.float32).reshape(T, nh, hd).astype(np.float64))
+    k, v = dk.download(np.float16).reshape(nh, n_ctx, hd).astype(np.float64), dv.download(np.float16).reshape(nh, n_ctx, hd).astype(np.float64)
+    q = rot.download(np.float32).reshape(T, nh, hd).astype(np.float16).astype(np.float64)
+    want = np.empty((T, nh, hd))
+    for a in range(nh):
+        s = np.where(np.arange(past + T)[None] <= pos[:, None], q[:, a] @ k[a, :past + T].T / np.sqrt(hd), -np.inf)
+        e = np.exp(s - s.max(1, keepdims=True))
+        want[:, a] = e / e.sum(1, keepdims=True) @ v[a, :past + T]
+    errs = [np.linalg.norm(g - want) / np.linalg.norm(want) for g in got]
+    assert errs[0] <= errs[1], errs
+
+
 def test_what_it_does_not_cover_is_refused():
     from powerinfer_amd import lib as pl
     L, b = pl.init(), pl.DevBuf(1 << 16)
