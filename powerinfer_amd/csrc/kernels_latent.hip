@@ -330,13 +330,15 @@ __global__ __launch_bounds__(256) void latent_attn_f32_kernel(pi_latent_attn p) 
 // transposed (keys x tokens), so that a lane's scores belong to one token, its soft-max needs two shuffles, and its weights are already
 // the column operand of the second product (values^T x weights) - which key a slot of that product's inner dimension stands for is free,
 // so the value operand is read in the order the scores came out.  64 keys at a time through LDS, the next 64 in registers.
-// Bound by the matrix and vector units (32 heads of 128 + 64 columns, 2048 tokens: 215 TFLOP/s at first): the soft-max runs in base 2, so that
-// a weight costs a subtraction and one v_exp_f32 instead of expf's dozen, and the rotated columns' cells are known a step ahead, where the
-// look-up under the fetch let every piece wait for memory: 200 -> 117 us.  (Pairing long with short tiles on a CU: 124 us.)
+// Bound by the matrix and vector units (32 heads of 128 + 64 columns, 2048 tokens: 215 TFLOP/s at first): a weight costs a subtraction, a product
+// and one v_exp_f32 instead of expf's dozen, and the rotated columns' cells are known a step ahead, where the look-up under the fetch
+// let every piece wait for memory: 185 -> 111 us.  (Pairing long with short tiles on a CU: 7 us more; log2 e in two parts: 135 us.)
+// Scores, maxima and sinks stay in the natural base: scaled by log2 e one beyond 2.3e38 overflows.  Weights are rounded to bf16, which is what
+// the output's error comes from: against float64, 84 heads of 256 tokens, 1.98e-3, with expf the same within 1 part in 1e5.
 // ---------------------------------------------------------------------------------------------------------------------------------
 constexpr int kXKeys = 64, kXTok = 128;
-constexpr float kLog2e = 1.4426950408889634f;
-__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+// e^x of a weight, x <= 0: off by |x| 2^-24 beside the 2^-9 of its rounding to bf16
+__device__ __forceinline__ float exp_weight(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
 template <int KS, int VT>              // 32-column steps of a key row (unrotated | rotated, zero padded); 16-column tiles of a value row
 __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_expanded p, int n_qt, int hp) {
     constexpr int KROW = KS * 64 + 16, VROW = VT * 32 + 16, KP = KS * 4 * kXKeys / 256, VP = VT * 2 * kXKeys / 256;      // bytes per LDS row; pieces per thread
@@ -388,7 +390,6 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
     cells(0);
     fetch(0);
     cells(kXKeys);
-    const float c2 = p.scale * kLog2e;                 // scores and maxima in base 2: a weight is one subtraction and one v_exp_f32
     float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.0f, 0.0f};
     pi_f4 o[2][VT];
 #pragma unroll
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = s[u][kt][r] * c2;
+                    float v = s[u][kt][r] * p.scale;
                     if (edge && k0 + kt * 16 + 4 * g + r >= nv[u]) v = -INFINITY;
                     s[u][kt][r] = v;
                     mx = fmaxf(mx, v);
@@ -432,14 +433,14 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
             mx = fmaxf(mx, __shfl_xor(mx, 16, PI_WAVE));
             mx = fmaxf(mx, __shfl_xor(mx, 32, PI_WAVE));
             const float mn = fmaxf(m[u], mx), base = mn == -INFINITY ? 0.0f : mn;
-            const float a = exp2_hw(m[u] - base);       // 0 while nothing has been seen
+            const float a = exp_weight(m[u] - base);    // 0 while nothing has been seen
             m[u] = mn;
             float sum = 0.0f;
             bf16 w[16];
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) { const float e = exp2_hw(s[u][kt][r] - base); sum += e; w[kt * 4 + r] = (bf16)e; }
+                for (int r = 0; r < 4; ++r) { const float e = exp_weight(s[u][kt][r] - base); sum += e; w[kt * 4 + r] = (bf16)e; }
             l[u] = l[u] * a + sum;
 #pragma unroll
             for (int v = 0; v < VT; ++v) { o[u][v][0] *= a; o[u][v][1] *= a; o[u][v][2] *= a; o[u][v][3] *= a; }
@@ -463,13 +464,13 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_attn_kernel(pi_latent_
                 o[1][v] = mfma_bf16(f, pb[1][k], o[1][v]);
             }
     }
-    const float sink = p.sink[h] * kLog2e;
+    const float sink = p.sink[h];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         float sum = l[u];
         sum += __shfl_xor(sum, 16, PI_WAVE);
         sum += __shfl_xor(sum, 32, PI_WAVE);
-        const float mf = fmaxf(m[u], sink), a = m[u] == -INFINITY ? 0.0f : exp2_hw(m[u] - mf), f = a / (sum * a + exp2_hw(sink - mf));
+        const float mf = fmaxf(m[u], sink), a = m[u] == -INFINITY ? 0.0f : expf(m[u] - mf), f = a / (sum * a + expf(sink - mf));
         if (q0 + wave * 32 + u * 16 + i >= p.T) continue;
         bf16 * out = (bf16 *)p.att + (size_t)tok[u] * p.ld_att + h * p.vdim;
 #pragma unroll

@@ -334,6 +334,35 @@ def test_expanded_attention(H, dim, rot, vdim, rank, T, start):
     close(c.run(1), want, t)
 
 
+def expanded(c, T):
+    """pi_k_latent_attn_expanded of a case of one sequence whose last T positions query."""
+    L, t = pl.init(), pl.BF16
+    n, H, dim, rot, vdim, rank = int(c.pos[-1]) + 1, c.H, c.dim, c.rot, c.vdim, c.rank
+    lat = c.cells[c.lists[0, :n], :rank]
+    keys = store(np.einsum("nr,hdr->nhd", lat, c.uk), t)
+    vals = store(np.einsum("nr,hvr->nhv", lat, c.uv), t)
+    q_un = np.zeros((T, H, c.dim_ld), np.float32)
+    q_un[..., :dim] = c.q[..., :dim]
+    ql, qu, cache, lst, nv, sk = store(c.latent_queries(), t), store(q_un, t), store(c.cells, t), i32(c.lists[0]), i32(c.pos + 1), dev(c.sink)
+    ld = (H * vdim + 127) // 128 * 128
+    att = pl.DevBuf.zeros(2 * T * ld)
+    a = pl.LatentExpanded()
+    a.q_un, a.q_lat, a.keys, a.values, a.cache, a.list, a.n_vis, a.sink, a.att = (b.ptr for b in (qu, ql, keys, vals, cache, lst, nv, sk, att))
+    a.tok0, a.T, a.n_head, a.dim, a.dim_ld, a.rot_dim, a.vdim, a.rank_ld, a.kd, a.ld_att, a.scale = 0, T, H, dim, c.dim_ld, rot, vdim, c.rank_ld, c.kd, ld, c.scale
+    pl.check(L.pi_k_latent_attn_expanded(C.byref(a), None))
+    pl.sync()
+    return fetch(att, t, (T, ld))[:, :H * vdim].reshape(T, H, vdim)
+
+
+@pytest.mark.parametrize("sink", [-3.4e38, -60.0, 60.0, 2.5e38])
+def test_expanded_attention_with_sinks_of_any_size(sink):
+    """Also near the largest and the lowest number of float32: the whole weight is the sink's, or none of it."""
+    c = Case(pl.BF16, 3, 32, 16, 32, 64, [70], [list(range(70))], 3)
+    c.sink = np.full(3, sink, np.float32)
+    got, want = expanded(c, 70), c.want()
+    assert np.abs(got - want).max() < 2e-2 * max(np.abs(want).max(), 1e-3)
+
+
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("own", [True, False])
 def test_latent_prep(t, own):
