@@ -15,6 +15,8 @@
 struct BatchState {
     int n_seq = 0, max_steps = 4096;
     int kv_hi = 0;                        // prompt chunks: cells the chunk's last token attends (its position + 1)
+    int rows = 0;                         // tokens the step buffers hold
+    bool scalar_attention = false;        // this chunk's attention: one token per workgroup (pi::WideRoute)
     // lockstep decoding: layers whose union of active rows was above dense_above * n_ff in the last step run their FFN dense
     // (>= 1: never, the default: the union kernels are the faster ones at every union fraction measured, see batch_layer)
     std::vector<char> dense_ffn, graph_dense;
@@ -71,11 +73,10 @@ pi_norm mk_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
 int chunk_attention(pi_model * m, BatchState * b, int T, size_t kv_off) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
-    const char * own = getenv("PI_ATTN_CHUNK");
-    // a Q4_0 output projection rounds what comes out here to eight bits: as before where the kernel before covers the chunk (see prefill_wide_max;
+    // a Q4_0 output projection rounds what comes out here to eight bits: as before where the kernel before covers the chunk (see prefill_wide_route;
     // 512 tokens behind none, 32 heads of 128: 61 against 49 us of about 950 per layer)
     const bool as_before = m->L(0, PI_T_WO).type == PI_TYPE_Q4_0 && T <= kChunkMaxT && pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi);
-    if (!as_before && pi_k_attn_chunk_rows_supported(hd, T, b->kv_hi) && !(own && !strcmp(own, "scalar")))
+    if (!as_before && pi_k_attn_chunk_rows_supported(hd, T, b->kv_hi) && !b->scalar_attention)
         return pi_k_attn_chunk_rows(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
                                     m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
     if (pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi))
@@ -337,7 +338,7 @@ BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, ff = hp.n_ff, r = (int)m->L(0, PI_T_FC1).ne1;
     BatchState * b = new BatchState();
-    b->n_seq = T;
+    b->n_seq = b->rows = T;
     b->cache_seq_stride = (size_t)hp.n_layer * hp.n_head_kv * hp.n_ctx * m->hd;
     const size_t n = T;
     bool ok = true;
@@ -555,11 +556,11 @@ bool prefill_wide_supported(pi_model * m) {
 // (210 us per 7B layer), keeps 512 up to 1024 tokens: where a chunk ends decides how the library orders its sums, and with them single roundings
 // to eight bits, by which results at those lengths are compared with the CPU path's.  Never more than the context holds (the step buffers are
 // sized by it).
-int prefill_wide_max(pi_model * m, int n_left) {
+static int wide_rows_max(pi_model * m) { return m->hd == 64 || m->hd == 128 ? std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048) : kChunkMaxT; }
+WideRoute prefill_wide_route(pi_model * m, int n_left) {
     const char * own = getenv("PI_ATTN_CHUNK");
-    if ((m->hd != 64 && m->hd != 128) || (own && !strcmp(own, "scalar"))) return kChunkMaxT;
-    const int most = std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048);
-    return n_left <= 2 * kChunkMaxT && m->L(0, PI_T_WO).type == PI_TYPE_Q4_0 ? kChunkMaxT : most;
+    const bool scalar = own && !strcmp(own, "scalar"), q4 = n_left <= 2 * kChunkMaxT && m->L(0, PI_T_WO).type == PI_TYPE_Q4_0;
+    return {scalar, scalar || q4 ? kChunkMaxT : wide_rows_max(m)};
 }
 
 // PI_PREFILL_GEMM=own: the dense mat-muls of prompt chunks run on this library's LDS-tiled MFMA kernel instead of hipBLASLt plans
@@ -568,9 +569,9 @@ static bool prefill_own_gemm() {
     return own && !strcmp(own, "own");
 }
 
-int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
-    const int kMaxT = prefill_wide_max(m, INT32_MAX);
-    if (T <= 16 || T > kMaxT) return pi::fail(PI_E_ARG, "prefill_wide_chunk: chunk length outside 17 .. prefill_wide_max");
+int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const WideRoute & route) {
+    const int kMaxT = wide_rows_max(m);                // what the model allows, not what this call asks for: the buffers serve later calls too
+    if (T <= 16 || T > route.most) return pi::fail(PI_E_ARG, "prefill_wide_chunk: chunk length outside the route's");
     const pi_hparams & hp = m->hp;
     if (!m->prefill_wide) {
         if (!prefill_own_gemm() && !m->gemm_lib) {
@@ -634,8 +635,10 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) 
         m->prefill_wide = b;
     }
     BatchState * b = m->prefill_wide;
+    if (T > b->rows) return pi::fail(PI_E_STATE, "prefill_wide_chunk: step buffers too small");
     b->n_seq = T;
     b->kv_hi = n_past + T;
+    b->scalar_attention = route.scalar;
     std::vector<int32_t> pos(T);
     for (int t = 0; t < T; ++t) pos[t] = n_past + t;
     PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));

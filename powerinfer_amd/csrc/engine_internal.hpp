@@ -118,6 +118,8 @@ bool prefill_supported(pi_model * m);   // F16 weights, every neuron on the GPU,
 int  prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);
 bool prefill_wide_supported(pi_model * m);   // F16 or Q4_0 matrices (fp16 predictor), hybrid layers included; n_embd, n_ff and the predictor rank multiples of 256
 int  gather_rest_rows(pi_model * m, int il);  // hybrid layer: rows of the non-resident neurons into pinned host memory (rest_up / rest_gate / rest_down)
-int  prefill_wide_max(pi_model * m, int n_left);     // longest chunk of a prompt with n_left tokens to go: 512 or up to 2048
-int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);     // 16 < T <= prefill_wide_max
+// how one call's prompt goes through wide chunks, decided once for the call (PI_ATTN_CHUNK may change between calls)
+struct WideRoute { bool scalar; int most; };  // attention one token per workgroup; longest chunk: 512 or up to 2048
+WideRoute prefill_wide_route(pi_model * m, int n_left);     // a prompt with n_left tokens to go
+int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const WideRoute & route);     // 16 < T <= route.most
 }
