@@ -1308,7 +1308,7 @@ namespace {
 constexpr size_t kChunkMfmaLds = 156 * 1024;
 size_t chunk_mfma_lds(int hd, int n_kv_max) { return sizeof(float) * 16 * (size_t)(((n_kv_max + 31) & ~31) + 4) + (size_t)kWavesPerBlock * hd * kAcVtStride * 2; }
 
-int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
+[[nodiscard]] int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
                   float * q_rot, void * k_cache, void * v_cache, hipStream_t st) {
     // 16 tokens and fewer: a workgroup per head and token (16 tokens, 32 heads of 128, attention included: 11.8 against 12.3 us); a chunk's angles
     // are worth forming once a token from there on.  A workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
@@ -1515,7 +1515,8 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad head geometry or mode");
     hipStream_t st = (hipStream_t)stream;
     // all K/V rows of the chunk are in the cache before any token of the chunk attends
-    rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    if (rc != PI_OK) return rc;
     // 16 tokens per workgroup on the matrix cores where the head size and the context fit (scores of 16 tokens in LDS)
     const char * own = getenv("PI_ATTN_CHUNK");
     const bool scalar = own && !strcmp(own, "scalar");
@@ -1585,7 +1586,8 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (mode != 0 && mode != 2) || hd % 2 || hd / 2 > 1024 || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_chunk_long: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
     hipStream_t st = (hipStream_t)stream;
-    rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    if (rc != PI_OK) return rc;
     const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)T * n_head * n_parts * hd;
