@@ -44,10 +44,13 @@ struct WideDeal {
     // the c-th of them: its token tile, its first row and how many there are
     __device__ __forceinline__ void unit(int c, int & ty, int & row0, int & n_rows) const {
         const int u = c < rounds ? c * slots + slot : rest_unit;
-        const int at = u < n_long ? xcd * per_long + u : xcd * per_short + u - n_long;
-        const int b0 = at / (band * nl) * band, high = min(band, n_tiles - b0), in = at - b0 * nl;
-        ty = u < n_long ? b0 + in % high : at;
-        row0 = (u < n_long ? in / high : (rows - 1) / kGwM) * kGwM + (c < rounds ? 0 : rest_row);
+        if (u < n_long) {
+            const int at = xcd * per_long + u, b0 = at / (band * nl) * band, high = min(band, n_tiles - b0), in = at - b0 * nl;
+            ty = b0 + in % high; row0 = in / high * kGwM;
+        } else {
+            ty = xcd * per_short + u - n_long; row0 = (rows - 1) / kGwM * kGwM;
+        }
+        if (c >= rounds) row0 += rest_row;
         n_rows = min(rows - row0, c < rounds || !halves ? kGwM : kGwM / 2);
     }
 };
