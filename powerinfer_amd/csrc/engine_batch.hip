@@ -16,7 +16,7 @@ struct BatchState {
     int n_seq = 0, max_steps = 4096;
     int kv_hi = 0;                        // prompt chunks: cells the chunk's last token attends (its position + 1)
     int rows = 0;                         // tokens the step buffers hold
-    bool scalar_attention = false;        // this chunk's attention: one token per workgroup (pi::WideRoute)
+    pi::WideRoute route{};                // how this chunk goes
     // lockstep decoding: layers whose union of active rows was above dense_above * n_ff in the last step run their FFN dense
     // (>= 1: never, the default: the union kernels are the faster ones at every union fraction measured, see batch_layer)
     std::vector<char> dense_ffn, graph_dense;
@@ -69,26 +69,26 @@ pi_norm mk_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
     return n;
 }
 
-// attention of a prompt chunk of the model's own sequence: the chunk kernels where the context fits them, the split-over-cells path beyond
-int chunk_attention(pi_model * m, BatchState * b, int T, size_t kv_off) {
+// attention of tokens t0 .. t0 + n - 1 of a prompt chunk of the model's own sequence, which see cells up to kv_hi: the chunk kernels where the
+// context fits them, the split-over-cells path beyond
+int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size_t kv_off) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
-    // a Q4_0 output projection rounds what comes out here to eight bits: as before where the kernel before covers the chunk (see prefill_wide_route;
-    // 512 tokens behind none, 32 heads of 128: 61 against 49 us of about 950 per layer)
-    const bool as_before = m->L(0, PI_T_WO).type == PI_TYPE_Q4_0 && T <= kChunkMaxT && pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi);
-    if (!as_before && pi_k_attn_chunk_rows_supported(hd, T, b->kv_hi) && !b->scalar_attention)
-        return pi_k_attn_chunk_rows(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
-                                    m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
-    if (pi_k_attn_chunk_supported(hd, hp.n_ctx, b->kv_hi))
-        return pi_k_attn_chunk(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, b->kv_hi, b->q_rot,
-                               m->k_cache + kv_off, m->v_cache + kv_off, b->att, d, b->att16, m->stream);
+    const float * qkv = b->qkv + (size_t)t0 * (d + 2 * gqa);
+    const int32_t * pos = b->d_pos + t0;
+    float * q_rot = b->q_rot + (size_t)t0 * d, * att = b->att + (size_t)t0 * d;
+    __half * att16 = b->att16 + (size_t)t0 * d, * k = m->k_cache + kv_off, * v = m->v_cache + kv_off;
+    if (!b->route.scalar && pi_k_attn_chunk_rows_supported(hd, n, kv_hi) && !(b->route.pieces && pi::attn_chunk_by_16(hd, kv_hi)))
+        return pi_k_attn_chunk_rows(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, att, d, att16, m->stream);
+    if (pi_k_attn_chunk_supported(hd, hp.n_ctx, kv_hi))
+        return pi_k_attn_chunk(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, att, d, att16, m->stream);
     const int parts = m->attn_parts > 1 ? m->attn_parts : 2;
     if (!m->attn_scratch_chunk) {
         m->attn_scratch_chunk = m->alloc<float>(pi_k_attn_split_scratch_floats(kChunkMaxT, hp.n_head, hd, parts));
         if (!m->attn_scratch_chunk) return PI_E_HIP;
     }
-    return pi_k_attn_chunk_long(b->qkv, d + 2 * gqa, T, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, b->d_pos, hp.n_ctx, parts,
-                                m->attn_scratch_chunk, b->q_rot, m->k_cache + kv_off, m->v_cache + kv_off, b->att, b->att16, m->stream);
+    return pi_k_attn_chunk_long(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, parts, m->attn_scratch_chunk, q_rot, k, v, att, att16,
+                                m->stream);
 }
 
 // fp16 mat-mul input for a matrix of the given type: rounded to fp16, for a Q4_0 matrix through Q8_0 blocks first (the CPU path
@@ -149,7 +149,6 @@ int ensure_q4_split(pi_model * m) {
     return PI_OK;
 }
 
-int chunk_attention(pi_model * m, BatchState * b, int T, size_t kv_off);
 
 // One layer of a step of up to 16 tokens of a Q4_0 model: the mat-muls of the Q4_0 matrices on integer matrix cores against the
 // Q8_0 blocks of their inputs (the CPU path's arithmetic), the F16 predictor as in an F16 model.
@@ -180,7 +179,7 @@ int batch_layer_q4(pi_model * m, BatchState * b, int il) {
     if (b->unified)
         PI_TRY(cells_attention(m, b, il, T));
     else if (b->prefill)
-        PI_TRY(chunk_attention(m, b, T, kv_off));
+        PI_TRY(chunk_attention(m, b, 0, T, b->kv_hi, kv_off));
     else if (hd % 32 == 0)                                         // lockstep: the attention writes the Q8_0 blocks of its output itself
         PI_TRY(pi_k_attn_fused_batch_q8(b->qkv, d + 2 * gqa, m->rope_table, b->k_cache + kv_off, b->v_cache + kv_off, b->cache_seq_stride, T,
                                         hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0, hp.n_ctx, b->d_pos, b->att, d, b->qa, b->da, b->sa, st));
@@ -246,7 +245,7 @@ int batch_layer(pi_model * m, BatchState * b, int il) {
     if (b->unified)
         PI_TRY(cells_attention(m, b, il, T));
     else if (b->prefill)
-        PI_TRY(chunk_attention(m, b, T, kv_off));
+        PI_TRY(chunk_attention(m, b, 0, T, b->kv_hi, kv_off));
     else
         PI_TRY(pi_k_attn_fused_batch_ol(b->qkv, d + 2 * gqa, m->rope_table, b->k_cache + kv_off, b->v_cache + kv_off, b->cache_seq_stride, T,
                                         hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0, hp.n_ctx, b->d_pos, b->att, d, b->att16, st));
@@ -385,11 +384,21 @@ namespace {
 // one layer of a wide prompt chunk (16 < T <= 128): every mat-mul reads its matrix once for the chunk; with that many tokens the union
 // of the active sets is nearly every neuron, so gate/up run dense and the predictor's mask turns into exact zeros of h (what the
 // sparse operators compute, term by term: an inactive neuron contributes nothing to the down projection)
+// f(t0, n) for the pieces of the chunk's tokens that products and attention take at a time (pi::WideRoute)
+template <typename F> int in_pieces(BatchState * b, F && f) {
+    const int T = b->n_seq, step = b->route.pieces ? kChunkMaxT : T;
+    for (int t0 = 0; t0 < T; t0 += step) PI_TRY(f(t0, std::min(step, T - t0)));
+    return PI_OK;
+}
 // one dense mat-mul of a chunk: the library's plan for long chunks, this library's own kernel otherwise
-int chunk_gemm(pi_model * m, const void * W, int rows, int cols, const void * xn, int T, int epi, const float * add1, const float * add2,
-               float * y, void * y16) {
-    if (m->gemm_lib) return pi_gemm_lib_f16(m->gemm_lib, W, rows, cols, xn, T, epi, add1, add2, y, y16, m->stream);
-    return pi_k_gemm_tile_f16(W, rows, cols, xn, T, epi, add1, add2, y, y16, 0, m->stream);
+int chunk_gemm(pi_model * m, BatchState * b, const void * W, int rows, int cols, const __half * xn, int epi, const float * add1, const float * add2, float * y, __half * y16) {
+    return in_pieces(b, [&](int t0, int n) {
+        const size_t o = (size_t)t0 * rows;
+        const float * a1 = add1 ? add1 + o : nullptr, * a2 = add2 ? add2 + o : nullptr;
+        __half * h = y16 ? y16 + o : nullptr;
+        if (m->gemm_lib) return pi_gemm_lib_f16(m->gemm_lib, W, rows, cols, xn + (size_t)t0 * cols, n, epi, a1, a2, y + o, h, m->stream);
+        return pi_k_gemm_tile_f16(W, rows, cols, xn + (size_t)t0 * cols, n, epi, a1, a2, y + o, h, 0, m->stream);
+    });
 }
 
 // where a hybrid layer's FFN matrix has the rows of its other neurons, and which are whose (nulls: the matrix is whole)
@@ -448,37 +457,37 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
     PI_TRY(batch_input(wqkv.type, x, T, d, &an, b->xa16, falcon ? b->xp16 : nullptr, st));
     PI_TRY(chunk_weight(m, b, il, PI_T_WQKV, d + 2 * gqa, d, &W));
-    PI_TRY(chunk_gemm(m, W, d + 2 * gqa, d, b->xa16, T, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr));
-    PI_TRY(chunk_attention(m, b, T, kv_off));
+    PI_TRY(chunk_gemm(m, b, W, d + 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr));
+    PI_TRY(in_pieces(b, [&](int t0, int n) { return chunk_attention(m, b, t0, n, b->kv_hi - (T - t0 - n), kv_off); }));
     if (wo.type == PI_TYPE_Q4_0) PI_TRY(pi_k_norm_q8_round_f16(b->att, T, d, &plain, b->att16, nullptr, st));
     PI_TRY(chunk_weight(m, b, il, PI_T_WO, d, d, &W));
     pi_norm fn;
     const __half * ffn_x = b->xf16;
     if (!falcon) {
-        PI_TRY(chunk_gemm(m, W, d, d, b->att16, T, PI_EPI_ADD, x, nullptr, b->ffn_inp, nullptr));
+        PI_TRY(chunk_gemm(m, b, W, d, d, b->att16, PI_EPI_ADD, x, nullptr, b->ffn_inp, nullptr));
         fn = mk_norm(1, hp.norm_eps, m->L(il, PI_T_FFN_NORM), nullptr);
         PI_TRY(batch_input(up.type, b->ffn_inp, T, d, &fn, b->xf16, b->xp16, st));
     } else {
-        PI_TRY(chunk_gemm(m, W, d, d, b->att16, T, PI_EPI_NONE, nullptr, nullptr, b->attn_out, nullptr));
+        PI_TRY(chunk_gemm(m, b, W, d, d, b->att16, PI_EPI_NONE, nullptr, nullptr, b->attn_out, nullptr));
         fn = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         // the FFN branch reads the layer input under its own norm; with a single norm it shares the attention branch's rows unless
         // the two matrices want different containers (fp16 against Q8_0 blocks)
         if (m->L(il, PI_T_ATTN_NORM_2).dev || up.type != wqkv.type) PI_TRY(batch_input(up.type, x, T, d, &fn, b->xf16, nullptr, st));
         else ffn_x = b->xa16;
     }
-    PI_TRY(chunk_gemm(m, fc1.dev, r, d, b->xp16, T, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
-    PI_TRY(chunk_gemm(m, fc2.dev, ff, r, b->hid16, T, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
+    PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
+    PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
     // F16 layers whole on the device: up, gate and h in one kernel.  Not for few tokens of large matrices, which the library's plans stream faster
     // (17 / 64 / 128 tokens, us, library and one kernel: 11008 x 4096 45 / 60 / 70 and 45 / 46 / 49; 13824 x 5120 58 / 74 / 95 and 79 / 86 / 95)
     const bool one_kernel = m->gemm_lib && up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(ff, d) &&
                             (T > 96 || (long long)ff * d <= 48LL << 20);
     if (!one_kernel) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_UP, ff, d, &W));
-        PI_TRY(chunk_gemm(m, W, ff, d, ffn_x, T, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
+        PI_TRY(chunk_gemm(m, b, W, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
     }
     if (!falcon && !one_kernel) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_GATE, ff, d, &W));
-        PI_TRY(chunk_gemm(m, W, ff, d, ffn_x, T, PI_EPI_NONE, nullptr, nullptr, b->gate_out, nullptr));
+        PI_TRY(chunk_gemm(m, b, W, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out, nullptr));
     }
     if (one_kernel) PI_TRY(pi_k_ffn_wide_f16(up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, b->pred_logits, hp.sparse_threshold, b->h16, st));
     else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
@@ -493,8 +502,8 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
         PI_TRY(pi_k_transpose_f16(W, ff, d, b->w16t, st));
         Wd = b->w16t;
     }
-    if (!falcon) PI_TRY(chunk_gemm(m, Wd, d, ff, b->h16, T, PI_EPI_ADD, b->ffn_inp, nullptr, b->x2, nullptr));
-    else         PI_TRY(chunk_gemm(m, Wd, d, ff, b->h16, T, PI_EPI_ADD2, b->attn_out, x, b->x2, nullptr));
+    if (!falcon) PI_TRY(chunk_gemm(m, b, Wd, d, ff, b->h16, PI_EPI_ADD, b->ffn_inp, nullptr, b->x2, nullptr));
+    else         PI_TRY(chunk_gemm(m, b, Wd, d, ff, b->h16, PI_EPI_ADD2, b->attn_out, x, b->x2, nullptr));
     std::swap(b->x, b->x2);
     return PI_OK;
 }
@@ -550,17 +559,22 @@ bool prefill_wide_supported(pi_model * m) {
     return !(off && off[0] == '1') && wide_unsupported(m) == nullptr;
 }
 
-// The longest chunk of a prompt of which n_left tokens are to come.  Longer ones read each matrix less often and give its product more columns:
-// the seven products of a 7B-shaped F16 layer take 1250 us in four chunks of 512 tokens and 1080 us in one of 2046.  The attention by rows of
-// tokens has no limit of its own; head sizes without it go by 512 as their kernels do.  A Q4_0 model, whose matrices are expanded once a chunk
-// (210 us per 7B layer), keeps 512 up to 1024 tokens: where a chunk ends decides how the library orders its sums, and with them single roundings
-// to eight bits, by which results at those lengths are compared with the CPU path's.  Never more than the context holds (the step buffers are
-// sized by it).
+// Long chunks read each matrix less often and give its product more columns: the seven products of a 7B-shaped F16 layer take 1250 us in four
+// chunks of 512 tokens and 1080 us in one of 2046.  The attention by rows of tokens has no limit of its own; head sizes without it go by 512 as
+// their kernels do.  Never more than the context holds.
 static int wide_rows_max(pi_model * m) { return m->hd == 64 || m->hd == 128 ? std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048) : kChunkMaxT; }
-WideRoute prefill_wide_route(pi_model * m, int n_left) {
+WideRoute prefill_wide_route(pi_model * m) {
     const char * own = getenv("PI_ATTN_CHUNK");
-    const bool scalar = own && !strcmp(own, "scalar"), q4 = n_left <= 2 * kChunkMaxT && m->L(0, PI_T_WO).type == PI_TYPE_Q4_0;
-    return {scalar, scalar || q4 ? kChunkMaxT : wide_rows_max(m)};
+    WideRoute r{own && !strcmp(own, "scalar"), false, 0};
+    for (int il = 0; il < m->hp.n_layer && !r.pieces; ++il)
+        for (int k : {PI_T_WQKV, PI_T_WO, PI_T_FFN_UP, PI_T_FFN_GATE, PI_T_FFN_DOWN_T}) r.pieces = r.pieces || m->L(il, k).type == PI_TYPE_Q4_0;
+    r.most = r.scalar ? kChunkMaxT : wide_rows_max(m);
+    return r;
+}
+// (with pieces a chunk ends where chunks of 512 would: what is left behind a whole one and too short for the next goes its own way)
+int WideRoute::chunk(int left) const {
+    const int T = std::min(left, most), over = T % kChunkMaxT;
+    return pieces && T > kChunkMaxT && over <= 16 ? T - over : T;
 }
 
 // PI_PREFILL_GEMM=own: the dense mat-muls of prompt chunks run on this library's LDS-tiled MFMA kernel instead of hipBLASLt plans
@@ -638,7 +652,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, 
     if (T > b->rows) return pi::fail(PI_E_STATE, "prefill_wide_chunk: step buffers too small");
     b->n_seq = T;
     b->kv_hi = n_past + T;
-    b->scalar_attention = route.scalar;
+    b->route = route;
     std::vector<int32_t> pos(T);
     for (int t = 0; t < T; ++t) pos[t] = n_past + t;
     PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));

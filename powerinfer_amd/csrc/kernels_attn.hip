@@ -1337,6 +1337,9 @@ int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_
 }
 }  // namespace
 
+namespace pi {
+bool attn_chunk_by_16(int hd, int n_kv_max) { return (hd == 64 || hd == 128) && chunk_mfma_lds(hd, n_kv_max) <= kChunkMfmaLds; }
+}  // namespace pi
 
 extern "C" {
 
@@ -1574,7 +1577,7 @@ int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, i
 int pi_k_attn_chunk_supported(int hd, int n_ctx, int n_kv_max) {
     if (hd <= 0 || hd % 8 || kBlock % (hd / 8) || PI_WAVE % (hd / 8) || n_ctx <= 0) return 0;
     if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;
-    if ((hd == 128 || hd == 64) && chunk_mfma_lds(hd, n_kv_max) <= kChunkMfmaLds) return 1;
+    if (pi::attn_chunk_by_16(hd, n_kv_max)) return 1;
     return sizeof(float) * ((size_t)n_ctx + (size_t)(kBlock / (hd / 8)) * hd) <= 60 * 1024;
 }
 

@@ -30,3 +30,19 @@ def test_a_prompt_behind_one_with_another_attention(first, then, monkeypatch):
     _, want = f.decode(b, 0)
     f.close()
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("name,hot", [("llama-tiny", 1.0), ("falcon-tiny", 1.0), ("llama-tiny", 0.6)])
+def test_cells_of_a_q4_prompt_do_not_depend_on_what_follows(name, hot):
+    """Q4_0: the first 512 tokens leave the same cells behind, bit for bit, whether 90 or 1500 tokens come after them: products and attention
+    keep one order of sums, so that no activation is rounded to eight bits the other way because the prompt is longer."""
+    hp = synth.hparams(name, n_rank=256, n_ctx=2100, seed=9, wtype=synth.Q4_0, hot_frac=hot)
+    model = synth.make_model(hp)
+    rng = np.random.default_rng(4)
+    prompt = rng.integers(0, hp.n_vocab, 2048).astype(np.int32)
+    m, after = fresh(hp, model), {}
+    for n in (602, 1001, 1030, 1100, 1541, 2048):
+        m.decode(prompt[:n], 0)
+        after[n] = m.decode([5], 512)[1]
+    m.close()
+    assert all(np.array_equal(a, after[602]) for a in after.values()), {n: float(np.abs(a - after[602]).max()) for n, a in after.items()}
