@@ -800,12 +800,12 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
         // model (F16 or Q4_0 matrices, hybrid layers included), up to 16 for the remainder of an F16 model that is whole on the
         // device; what is left, and at least the last token, takes the single-token path below, which produces the logits
         const bool wide = pi::prefill_wide_supported(m), small = pi::prefill_supported(m);
-        const pi::WideRoute route = wide ? pi::prefill_wide_route(m) : pi::WideRoute{};
+        pi::WideRoute route = wide ? pi::prefill_wide_route(m) : pi::WideRoute{};
         while (n_tokens - 1 - first >= 2) {
             const int left = n_tokens - 1 - first;
             if (wide && left > 16) {
-                const int T = route.chunk(left);
-                PI_TRY(pi::prefill_wide_chunk(m, tokens + first, T, n_past + first, route));
+                const int T = pi::prefill_wide_chunk(m, tokens + first, left, n_past + first, route);
+                if (T < 0) return T;
                 first += T;
             } else if (small) {
                 const int T = left < 16 ? left : 16;

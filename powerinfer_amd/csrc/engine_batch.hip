@@ -16,6 +16,7 @@ struct BatchState {
     int n_seq = 0, max_steps = 4096;
     int kv_hi = 0;                        // prompt chunks: cells the chunk's last token attends (its position + 1)
     int rows = 0;                         // tokens the step buffers hold
+    std::vector<void *> sized;            // wide prompt chunks: the buffers of that size (the model's, given back when longer prompts come)
     pi::WideRoute route{};                // how this chunk goes
     // lockstep decoding: layers whose union of active rows was above dense_above * n_ff in the last step run their FFN dense
     // (>= 1: never, the default: the union kernels are the faster ones at every union fraction measured, see batch_layer)
@@ -333,10 +334,9 @@ const char * batch_unsupported(pi_model * m) {
 }
 
 // step buffers for up to T tokens; caches only for independent sequences
-BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
+bool step_buffers(pi_model * m, BatchState * b, int T, bool with_caches) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, ff = hp.n_ff, r = (int)m->L(0, PI_T_FC1).ne1;
-    BatchState * b = new BatchState();
     b->n_seq = b->rows = T;
     b->cache_seq_stride = (size_t)hp.n_layer * hp.n_head_kv * hp.n_ctx * m->hd;
     const size_t n = T;
@@ -350,12 +350,12 @@ BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
     }
     b->x = m->alloc<float>(n * d); b->x2 = m->alloc<float>(n * d); b->qkv = m->alloc<float>(n * (d + 2 * m->gqa));
     b->att = m->alloc<float>(n * d); b->attn_out = m->alloc<float>(n * d); b->ffn_inp = m->alloc<float>(n * d);
-    b->hidden = m->alloc<float>(n * r); b->pred_logits = m->alloc<float>(n * ff); b->logits = m->alloc<float>((n > 16 ? 1 : n) * hp.n_vocab);      // a prompt chunk's last token has its logits elsewhere
+    b->hidden = m->alloc<float>(n * r); b->pred_logits = m->alloc<float>(n * ff); b->logits = m->alloc<float>((n > 16 ? 1 : n) * hp.n_vocab);      // a prompt chunk's last token has its logits and its choice elsewhere
     const size_t n16 = n < 16 ? 16 : n;                            // steps of up to 16 tokens keep these in the operand layout: 16 token slots
     b->xa16 = m->alloc<__half>(n16 * d); b->xf16 = m->alloc<__half>(n16 * d); b->xp16 = m->alloc<__half>(n16 * d);
     b->att16 = m->alloc<__half>(n16 * d); b->hid16 = m->alloc<__half>(n16 * r);
     b->d_tokens = m->alloc<int32_t>(n); b->d_pos = m->alloc<int32_t>(n); b->d_step = m->alloc<int32_t>(1);
-    b->d_out_tokens = m->alloc<int32_t>((size_t)b->max_steps * n); b->union_rows = m->alloc<int32_t>(ff); b->n_union = m->alloc<int32_t>(hp.n_layer);
+    b->d_out_tokens = m->alloc<int32_t>((size_t)b->max_steps * (n > 16 ? 1 : n)); b->union_rows = m->alloc<int32_t>(ff); b->n_union = m->alloc<int32_t>(hp.n_layer);
     if (m->L(0, PI_T_WQKV).type == PI_TYPE_Q4_0 && d % 32 == 0) {          // steps of a Q4_0 model on integer matrix cores
         b->qa = m->alloc<unsigned char>((size_t)16 * d); b->qf = m->alloc<unsigned char>((size_t)16 * d);
         b->da = m->alloc<float>((size_t)d / 32 * 16); b->df = m->alloc<float>((size_t)d / 32 * 16);
@@ -370,12 +370,14 @@ BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
         ok = ok && b->up_out && b->gate_out && b->h16;
         b->dense_ffn.assign(hp.n_layer, 0);
     }
-    if (!ok || !b->x || !b->x2 || !b->qkv || !b->att || !b->attn_out || !b->ffn_inp || !b->hidden || !b->pred_logits || !b->logits ||
-        !b->xa16 || !b->xf16 || !b->xp16 || !b->att16 || !b->hid16 || !b->d_tokens || !b->d_pos || !b->d_step || !b->d_out_tokens || !b->union_rows || !b->n_union) {
-        delete b;
-        return nullptr;
-    }
-    return b;
+    return ok && b->x && b->x2 && b->qkv && b->att && b->attn_out && b->ffn_inp && b->hidden && b->pred_logits && b->logits && b->xa16 && b->xf16 && b->xp16 && b->att16 && b->hid16 &&
+           b->d_tokens && b->d_pos && b->d_step && b->d_out_tokens && b->union_rows && b->n_union;
+}
+BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
+    BatchState * b = new BatchState();
+    if (step_buffers(m, b, T, with_caches)) return b;
+    delete b;
+    return nullptr;
 }
 
 }  // namespace
@@ -438,6 +440,15 @@ int chunk_down_q4(pi_model * m, BatchState * b, int il, int ff, int d) {
     return pi_k_dequant_q4_t_f16(m->L(il, PI_T_FFN_DOWN_T).dev, c.rest, c.hot_words, c.hot_prefix, ff, d, b->w16t, m->stream);
 }
 
+// F16 layers whole on the device: up, gate and h in one kernel.  Not for few tokens of large matrices, which the
+// library's plans stream faster (17 / 64 / 128 tokens, us, library and one kernel: 11008 x 4096 45 / 60 / 70 and 45 / 46 / 49; 13824 x 5120
+// 58 / 74 / 95 and 79 / 86 / 95)
+constexpr int kFfnOneRows = 96;
+bool ffn_in_one(pi_model * m, int il) {
+    return m->gemm_lib && m->L(il, PI_T_FFN_UP).type == PI_TYPE_F16 && m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(m->hp.n_ff, m->hp.n_embd);
+}
+bool ffn_large(pi_model * m) { return (long long)m->hp.n_ff * m->hp.n_embd > 48LL << 20; }
+
 int wide_layer(pi_model * m, BatchState * b, int il) {
     const pi_hparams & hp = m->hp;
     const int T = b->n_seq, d = hp.n_embd, ff = hp.n_ff, hd = m->hd, gqa = m->gqa;
@@ -477,10 +488,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
     PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
-    // F16 layers whole on the device: up, gate and h in one kernel.  Not for few tokens of large matrices, which the library's plans stream faster
-    // (17 / 64 / 128 tokens, us, library and one kernel: 11008 x 4096 45 / 60 / 70 and 45 / 46 / 49; 13824 x 5120 58 / 74 / 95 and 79 / 86 / 95)
-    const bool one_kernel = m->gemm_lib && up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(ff, d) &&
-                            (T > 96 || (long long)ff * d <= 48LL << 20);
+    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m));
     if (!one_kernel) {
         PI_TRY(chunk_weight(m, b, il, PI_T_FFN_UP, ff, d, &W));
         PI_TRY(chunk_gemm(m, b, W, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
@@ -562,7 +570,7 @@ bool prefill_wide_supported(pi_model * m) {
 // Long chunks read each matrix less often and give its product more columns: the seven products of a 7B-shaped F16 layer take 1250 us in four
 // chunks of 512 tokens and 1080 us in one of 2046.  The attention by rows of tokens has no limit of its own; head sizes without it go by 512 as
 // their kernels do.  Never more than the context holds.
-static int wide_rows_max(pi_model * m) { return m->hd == 64 || m->hd == 128 ? std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048) : kChunkMaxT; }
+static int wide_rows_max(const pi_model * m) { return m->hd == 64 || m->hd == 128 ? std::min(std::max(m->hp.n_ctx, kChunkMaxT), 2048) : kChunkMaxT; }
 WideRoute prefill_wide_route(pi_model * m) {
     const char * own = getenv("PI_ATTN_CHUNK");
     WideRoute r{own && !strcmp(own, "scalar"), false, 0};
@@ -583,17 +591,40 @@ static bool prefill_own_gemm() {
     return own && !strcmp(own, "own");
 }
 
-int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const WideRoute & route) {
-    const int kMaxT = wide_rows_max(m);                // what the model allows, not what this call asks for: the buffers serve later calls too
-    if (T <= 16 || T > route.most) return pi::fail(PI_E_ARG, "prefill_wide_chunk: chunk length outside the route's");
+// Step buffers for `rows` tokens in the place of those a state has.  Up and gate products of their own get the rows that some layer takes there
+// (a 7B-shaped F16 model: 0.52 GB for 2048 tokens instead of 0.70).
+static int wide_buffers(pi_model * m, BatchState * b, int rows) {
+    PI_HIP_TRY(hipStreamSynchronize(m->stream));
+    m->give_back(b->sized);
+    b->rows = 0;
+    int apart = 0;
+    for (int il = 0; il < m->hp.n_layer; ++il) apart = std::max(apart, !ffn_in_one(m, il) ? rows : ffn_large(m) ? kFfnOneRows : 0);
+    const bool falcon = m->hp.arch == PI_ARCH_FALCON;
+    const size_t mark = m->owned.size(), ff = m->hp.n_ff;
+    bool ok = step_buffers(m, b, rows, false);
+    b->up_out = b->gate_out = nullptr;
+    if (apart) {
+        b->up_out = m->alloc<float>(apart * ff);
+        if (!falcon) b->gate_out = m->alloc<float>(apart * ff);
+        ok = ok && b->up_out && (falcon || b->gate_out);
+    }
+    b->h16 = m->alloc<__half>(rows * ff);
+    b->sized.assign(m->owned.begin() + mark, m->owned.end());
+    if (ok && b->h16) return PI_OK;
+    m->give_back(b->sized);
+    b->rows = 0;
+    (void)hipGetLastError();                           // the next launch's check is not to find this
+    return PI_E_HIP;
+}
+
+int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route) {
     const pi_hparams & hp = m->hp;
     if (!m->prefill_wide) {
         if (!prefill_own_gemm() && !m->gemm_lib) {
             m->gemm_lib = pi_gemm_lib_create((size_t)64 << 20);
             if (!m->gemm_lib) return PI_E_HIP;
         }
-        BatchState * b = batch_alloc(m, kMaxT, false);
-        if (!b) return PI_E_HIP;
+        BatchState * b = new BatchState();
         // until the state is complete every early return undoes what was created here (the device buffers stay with the model's
         // allocation list; the mat-mul library is kept for the next attempt)
         struct SetupGuard {
@@ -607,10 +638,6 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, 
             }
         } guard{m, b};
         b->prefill = true;
-        b->up_out = m->alloc<float>((size_t)kMaxT * hp.n_ff);
-        b->gate_out = hp.arch == PI_ARCH_FALCON ? nullptr : m->alloc<float>((size_t)kMaxT * hp.n_ff);
-        b->h16 = m->alloc<__half>((size_t)kMaxT * hp.n_ff);
-        if (!b->up_out || (hp.arch != PI_ARCH_FALCON && !b->gate_out) || !b->h16) return PI_E_HIP;
         // the down projection of a chunk is a mat-mul whose reduction runs over the neurons.  An F16 layer that is whole on the device
         // gets one more copy of it with the neurons contiguous (n_embd x n_ff fp16; the decode loop keeps the row-per-neuron layout);
         // Q4_0 and hybrid layers expand one matrix at a time into scratch instead, so that prompts leave the model's footprint as
@@ -649,7 +676,17 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, 
         m->prefill_wide = b;
     }
     BatchState * b = m->prefill_wide;
-    if (T > b->rows) return pi::fail(PI_E_STATE, "prefill_wide_chunk: step buffers too small");
+    // The buffers follow the prompts: 512 tokens, doubled when a longer chunk comes.  Where that much memory is not to be had, this call goes by 512.
+    int T = route.chunk(left);
+    if (T > b->rows) {
+        int rows = kChunkMaxT;
+        while (rows < T) rows *= 2;
+        if (wide_buffers(m, b, std::min(rows, std::max(wide_rows_max(m), T))) != PI_OK) {
+            route.most = kChunkMaxT;
+            T = route.chunk(left);
+            PI_TRY(wide_buffers(m, b, kChunkMaxT));
+        }
+    }
     b->n_seq = T;
     b->kv_hi = n_past + T;
     b->route = route;
@@ -673,7 +710,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, 
         PI_TRY(wide_layer(m, b, il));
         if (staged) { PI_HIP_TRY(hipEventRecord(b->ev_free[il & 1], m->stream)); b->free_recorded[il & 1] = true; }
     }
-    return PI_OK;
+    return T;
 }
 
 bool prefill_supported(pi_model * m) {

@@ -106,6 +106,10 @@ struct pi_model {
         if (p) owned.push_back(p);
         return (T *)p;
     }
+    void give_back(std::vector<void *> & ps) {
+        for (void * p : ps) { owned.erase(std::find(owned.begin(), owned.end(), p)); (void)pi_free(p); }
+        ps.clear();
+    }
 };
 
 namespace pi {
@@ -132,5 +136,5 @@ int  prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);
 bool prefill_wide_supported(pi_model * m);   // F16 or Q4_0 matrices (fp16 predictor), hybrid layers included; n_embd, n_ff and the predictor rank multiples of 256
 int  gather_rest_rows(pi_model * m, int il);  // hybrid layer: rows of the non-resident neurons into pinned host memory (rest_up / rest_gate / rest_down)
 WideRoute prefill_wide_route(pi_model * m);
-int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const WideRoute & route);     // 16 < T <= route.most
+int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route);     // left > 16; the tokens taken, or an error (< 0)
 }

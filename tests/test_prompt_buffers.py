@@ -1,0 +1,54 @@
+"""Step buffers of long prompts, on the CPU (fake_hip): how much memory a model takes for the prompts it has seen, what it does where that much is
+not to be had, and which kernels its layers go through."""
+import fake_hip
+
+MODEL = """
+import numpy as np
+from powerinfer_amd import lib as pl, synth
+from powerinfer_amd.model import KIND, Model
+
+def made(**kw):
+    hp = synth.hparams("llama-tiny", n_rank=256, n_ctx=2100, seed=9, use_rates=False, **kw)
+    return Model(hp).load(synth.make_model(hp)), hp
+
+def prompt(m, n):
+    F.fake_clear_counts()
+    m.decode(np.zeros(n, np.int32), 0)
+    return F.fake_live()
+"""
+
+
+def test_buffers_follow_the_prompts():
+    """512 tokens first, twice and four times that when longer prompts come, nothing back and forth.  A resident F16 model has no up and gate products."""
+    fake_hip.run(MODEL + """
+m, hp = made()
+a, b, c, d, e = (prompt(m, n) for n in (20, 500, 700, 1500, 2040))
+assert a == b < c < d == e == prompt(m, 30), (a, b, c, d, e)
+token = (c - b) / 512
+assert abs((d - c) / 1024 - token) < 0.05 * token, (d - c, c - b)
+need = 4 * (6 * hp.n_embd + 3 * hp.n_embd + hp.n_rank + hp.n_ff) + 2 * (4 * hp.n_embd + hp.n_rank + hp.n_ff)
+assert need <= token < need + 1024, (token, need)
+q, _ = made(wtype=synth.Q4_0)
+a, b = prompt(q, 700), prompt(q, 1500)
+assert (b - a) / 1024 >= need + 8 * hp.n_ff
+m.close(); q.close()
+""")
+
+
+def test_without_memory_for_long_chunks_a_prompt_goes_by_512():
+    fake_hip.run(MODEL + """
+m, hp = made()
+prompt(m, 20)
+at_512 = F.fake_live()
+prompt(m, 2040)
+assert count("attn_chunk_rows") == hp.n_layer
+at_2048 = F.fake_live()
+n, hp = made()
+prompt(n, 20)
+F.fake_limit((at_2048 - at_512) // 2)
+prompt(n, 2040)
+assert count("attn_chunk_rows") == 4 * hp.n_layer, count("attn_chunk_rows")
+F.fake_limit(C.c_size_t(-1).value)
+prompt(n, 2040)                          # memory is there again
+assert count("attn_chunk_rows") == hp.n_layer
+""")
