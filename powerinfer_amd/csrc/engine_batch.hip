@@ -440,12 +440,14 @@ int chunk_down_q4(pi_model * m, BatchState * b, int il, int ff, int d) {
     return pi_k_dequant_q4_t_f16(m->L(il, PI_T_FFN_DOWN_T).dev, c.rest, c.hot_words, c.hot_prefix, ff, d, b->w16t, m->stream);
 }
 
-// F16 layers whole on the device: up, gate and h in one kernel.  Not for few tokens of large matrices, which the
+// F16 layers whole on the device: up, gate and h in one kernel (its matrices on 16 bytes).  Not for few tokens of large matrices, which the
 // library's plans stream faster (17 / 64 / 128 tokens, us, library and one kernel: 11008 x 4096 45 / 60 / 70 and 45 / 46 / 49; 13824 x 5120
 // 58 / 74 / 95 and 79 / 86 / 95)
 constexpr int kFfnOneRows = 96;
 bool ffn_in_one(pi_model * m, int il) {
-    return m->gemm_lib && m->L(il, PI_T_FFN_UP).type == PI_TYPE_F16 && m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(m->hp.n_ff, m->hp.n_embd);
+    const Tensor & up = m->L(il, PI_T_FFN_UP), & gate = m->L(il, PI_T_FFN_GATE);
+    return m->gemm_lib && up.type == PI_TYPE_F16 && m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_F16 && !m->L(il, PI_T_GPU_BUCKET).dev && pi_k_ffn_wide_supported(m->hp.n_ff, m->hp.n_embd) &&
+           (((uintptr_t)up.dev | (m->hp.arch == PI_ARCH_FALCON ? 0 : (uintptr_t)gate.dev)) & 15) == 0;
 }
 bool ffn_large(pi_model * m) { return (long long)m->hp.n_ff * m->hp.n_embd > 48LL << 20; }
 
