@@ -275,14 +275,17 @@ __global__ __launch_bounds__(kBlock, 2) void gemv_multi_f16_reg_kernel(GemvMulti
 // is on its way under the prologue, which is half of the launch, and a lane takes its 36 bytes from LDS, where 36 bytes a lane fall on
 // different banks (from memory they were three loads at odd places each).  One barrier a step: behind it the step's rows are there and
 // the previous step's slots are free.  12288 x 4096 behind an RMSNorm 10.8 -> 9.7 us, 32000 x 4096 20.2 -> 16.1,
-// 8192 x 8192 12.6 -> 9.1, 65024 x 8192 69 -> 54 (5.5 TB/s); matrices on a multiple of 4 bytes only, copied by single words, 10.9 -> 10.0 and 20.2 -> 22.3.
+// 8192 x 8192 12.6 -> 9.1, 65024 x 8192 69 -> 54 (5.5 TB/s).
+// OFF: a matrix on a multiple of 4 bytes only.  Its rows are copied from the multiple of 16 before them, one piece more, and the lanes read that
+// much further on (the 16 bytes around its first and last byte lie on their page): 10.8 -> 9.9, 20.1 -> 16.1, 12.7 -> 9.4, 70 -> 57 us
+// (copied by single words: 32000 x 4096 21.6).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kQ4Threads = kBlock + PI_WAVE;
-template <int CB, int KIND, int TAG>
+template <int CB, int KIND, int TAG, bool OFF>
 __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsigned char * __restrict__ W, const float * __restrict__ x,
                                                              const float * __restrict__ nw, const float * __restrict__ nb, float eps,
                                                              int epi, const float * __restrict__ add1, const float * __restrict__ add2,
-                                                             float * __restrict__ y, int rows, int a16) {
+                                                             float * __restrict__ y, int rows) {
     constexpr int cols = CB * 4096, NCH = cols / 512, nblk = cols / 32;
     constexpr int NBUF = CB == 1 ? 5 : 2;                          // steps in LDS
     constexpr int MYCH = NCH / kWavesPerBlock;
@@ -291,7 +294,8 @@ __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsign
     __shared__ float xd[nblk];
     __shared__ int   xsum[nblk];
     __shared__ double red[2][kWavesPerBlock];
-    __shared__ __align__(16) unsigned char ring[NBUF][kWavesPerBlock][row_bytes];
+    __shared__ __align__(16) unsigned char ring[NBUF][kWavesPerBlock][row_bytes + (OFF ? 16 : 0)];
+    const int mis = OFF ? (int)((uintptr_t)W & 15) : 0;            // a multiple of 4; rows are multiples of 16
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n_waves = gridDim.x * kWavesPerBlock, wid = blockIdx.x * kWavesPerBlock + wave;
 
@@ -306,21 +310,16 @@ __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsign
             for (int w = 0; w < kWavesPerBlock; ++w) {
                 const unsigned char * p = W + (size_t)min((int)blockIdx.x * kWavesPerBlock + w + s * n_waves, rows - 1) * row_bytes;
                 unsigned char * to = ring[s % NBUF][w];
-                if (a16) {
 #pragma unroll
-                    for (int o = 0; o < (int)row_bytes; o += 1024)
-                        if (o + lane * 16 < (int)row_bytes) __builtin_amdgcn_global_load_lds((gptr)(p + o + lane * 16), (lptr)(to + o), 16, 0, 0);
-                } else {
-#pragma unroll
-                    for (int o = 0; o < (int)row_bytes; o += 256) __builtin_amdgcn_global_load_lds((gptr)(p + o + lane * 4), (lptr)(to + o), 4, 0, 0);
-                }
+                for (int o = 0; o < (int)row_bytes; o += 1024)
+                    if (o + 1024 <= (int)row_bytes || o + lane * 16 < (int)row_bytes + mis) __builtin_amdgcn_global_load_lds((gptr)(p - mis + o + lane * 16), (lptr)(to + o), 16, 0, 0);
             }
         };
         for (int s = 0; s < min(steps, NBUF); ++s) copy_step(s);
         for (int k = 0; k <= KIND; ++k) __builtin_amdgcn_s_barrier();                      // the prologue's
         for (int s = 0; s < steps; ++s) {
             const int behind = min(steps - 1 - s, s ? NBUF - 2 : NBUF - 1);               // steps on their way behind this one (step s - 1's slot is filled below)
-            if (!a16 || behind == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (behind == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             else if (behind == 1) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kCopies) : "memory");
             else if (behind == 2) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NBUF > 2 ? 2 * kCopies : 0) : "memory");
             else if (behind == 3) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(NBUF > 3 ? 3 * kCopies : 0) : "memory");
@@ -440,7 +439,7 @@ __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsign
         for (int g = 0; g < CB; ++g) {
             uint32_t d9[9];
 #pragma unroll
-            for (int k = 0; k < 9; ++k) d9[k] = *reinterpret_cast<const uint32_t *>(ring[s % NBUF][wave] + g * 2304 + lane * 36 + k * 4);
+            for (int k = 0; k < 9; ++k) d9[k] = *reinterpret_cast<const uint32_t *>(ring[s % NBUF][wave] + mis + g * 2304 + lane * 36 + k * 4);
             int s0 = 0, s1 = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -734,13 +733,15 @@ int pi_k_gemv(int wtype, const void * W, int rows, int cols, const float * x, co
             const int rblocks = rows >= n_waves ? kGemvBlocks : (rows + kWavesPerBlock - 1) / kWavesPerBlock;
             const int tag = rows >= 16384 ? 1 : 0;
             const unsigned char * wb = (const unsigned char *)W;
-#define PI_GEMV_Q4(CB, KIND, TAG) hipLaunchKernelGGL((gemv_q4_reg_kernel<CB, KIND, TAG>), dim3(rblocks), dim3(kQ4Threads), 0, st, wb, x, na.w, na.b, na.eps, epilogue, add1, add2, y, rows, ((uintptr_t)W & 15) == 0)
+#define PI_GEMV_Q4_O(CB, KIND, TAG, OFF) hipLaunchKernelGGL((gemv_q4_reg_kernel<CB, KIND, TAG, OFF>), dim3(rblocks), dim3(kQ4Threads), 0, st, wb, x, na.w, na.b, na.eps, epilogue, add1, add2, y, rows)
+#define PI_GEMV_Q4(CB, KIND, TAG) do { if ((uintptr_t)W & 15) PI_GEMV_Q4_O(CB, KIND, TAG, true); else PI_GEMV_Q4_O(CB, KIND, TAG, false); } while (0)
 #define PI_GEMV_Q4_K(CB, KIND) do { if (tag == 1) PI_GEMV_Q4(CB, KIND, 1); else PI_GEMV_Q4(CB, KIND, 0); } while (0)
 #define PI_GEMV_Q4_N(CB) do { if (na.kind == 0) PI_GEMV_Q4_K(CB, 0); else if (na.kind == 1) PI_GEMV_Q4_K(CB, 1); else PI_GEMV_Q4_K(CB, 2); } while (0)
             if (cols == 4096) PI_GEMV_Q4_N(1); else PI_GEMV_Q4_N(2);
 #undef PI_GEMV_Q4_N
 #undef PI_GEMV_Q4_K
 #undef PI_GEMV_Q4
+#undef PI_GEMV_Q4_O
             return pi::check_launch("pi_k_gemv");
         }
         if (rpw == 8)      hipLaunchKernelGGL(gemv_q4_kernel<8>, dim3(blocks), dim3(kBlock), sh, st, w, x, na, epilogue, add1, add2, y, rows, cols);

@@ -46,6 +46,22 @@ def test_busy_groups_and_odd_addresses(has_gate, r, threshold):
         assert rel_err(out[0][0], ou["h"]) < 1e-4 and rel_err(out[0][1], ou["out"]) < FFN_REL_TOL
 
 
+@pytest.mark.parametrize("rows,cols", [(5, 4096), (12290, 4096), (6145, 8192)])
+def test_mat_vec_of_a_matrix_on_4_bytes(rows, cols):
+    """Every multiple of 4 behind a multiple of 16: the bits of the aligned matrix."""
+    L, rng, want = pl.init(), np.random.default_rng(rows), None
+    raw = synth.quantize_q4_0((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)).reshape(-1).view(np.uint8)
+    dx, y = pl.DevBuf(host=rng.standard_normal(cols).astype(np.float32)), pl.DevBuf(4 * rows)
+    for off in (0, 4, 8, 12):
+        dw = pl.DevBuf(host=np.concatenate([np.zeros(off, np.uint8), raw, np.zeros(16, np.uint8)]))
+        print(rows, cols, off, flush=True)
+        pl.check(L.pi_k_gemv(pl.Q4_0, dw.ptr + off, rows, cols, dx.ptr, None, pl.EPI_NONE, None, None, y.ptr, None))
+        pl.sync()
+        got = y.download(np.float32)
+        want = got if want is None else want
+        assert np.array_equal(got, want) and got.any(), off
+
+
 @pytest.mark.parametrize("rows,cols,hot_frac", [(32, 4096, 1.0), (200, 256, 1.0), (72, 512, 1.0), (96, 4096, 0.6), (64, 8192, 0.0), (32, 96, 1.0), (160, 768, 0.3)])
 @pytest.mark.parametrize("shift", [0, 2])
 def test_expanded_matrices(rows, cols, hot_frac, shift):
