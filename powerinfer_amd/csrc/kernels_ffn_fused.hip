@@ -548,31 +548,30 @@ __global__ __launch_bounds__(kPfBlock) void ffn_reduce_kernel(const float * __re
 // bytes of nibbles.  Read lane by lane that is two loads at odd places that the address unit takes apart (0.7 us a neuron of up and
 // gate with eight waves on a unit); here 18 lanes bring the 288 bytes to LDS in one copy, and the lane picks four aligned words there.
 // LLaMA-7B layer, all neurons here: 19.3 -> 17.1 us, and 0.3 -> 0.1 us a neuron of the down rows, which now travel with the others.
-// (q4_slice_fetch_any: a row that does not start on a multiple of 16 bytes, by single shorts.)
+// A matrix that does not start on a multiple of 16 bytes is copied from the multiple before: one piece more, and the lanes pick that much
+// further on (the 16 bytes around its first and last byte lie on their page): 11008 neurons, a tenth / two fifths active, 16 / 29 us where rows
+// copied by single shorts took 31 / 61.  q4_slice_fetch_odd: at an odd address, byte by byte.
 // ---------------------------------------------------------------------------------------------------
-constexpr int kQ4Slice = 288;
-__device__ __forceinline__ void q4_slice_fetch(const unsigned char * src, unsigned char * slot, int lane) {
-    if (lane < kQ4Slice / 16)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + lane * 16), (__attribute__((address_space(3))) void *)slot, 16, 0, 0);
+constexpr int kQ4Slice = 288, kQ4Slot = kQ4Slice + 16;
+template <bool ANY> __device__ __forceinline__ void q4_slice_fetch(const unsigned char * src, unsigned char * slot, int lane) {
+    const int mis = ANY ? (int)((uintptr_t)src & 15) : 0;
+    if (lane * 16 < kQ4Slice + mis)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src - mis + lane * 16), (__attribute__((address_space(3))) void *)slot, 16, 0, 0);
 }
-__device__ __forceinline__ void q4_slice_fetch_any(const unsigned char * src, unsigned char * slot, int lane) {
+__device__ __forceinline__ void q4_slice_fetch_odd(const unsigned char * src, unsigned char * slot, int lane) {
 #pragma unroll 1
-    for (int k = lane; k < kQ4Slice / 2; k += PI_WAVE) {
-        uint16_t v;
-        __builtin_memcpy(&v, src + 2 * k, 2);
-        reinterpret_cast<uint16_t *>(slot)[k] = v;
-    }
+    for (int k = lane; k < kQ4Slice; k += PI_WAVE) slot[k] = src[k];
 }
-// block lane / 4 of a slice: its scale and the bytes 8 * (lane & 1) .. + 7 of its nibbles.  Block b starts at byte 18 b: in the middle of a word
-// where b is odd
-__device__ __forceinline__ void q4_slice_pick(const unsigned char * slot, int lane, uint32_t (&q)[2], uint16_t & d) {
+// block lane / 4 of a slice that starts `mis` (even) bytes into its slot: its scale and the bytes 8 * (lane & 1) .. + 7 of its nibbles.  The block
+// starts at a whole word or in the middle of one
+__device__ __forceinline__ void q4_slice_pick(const unsigned char * slot, int mis, int lane, uint32_t (&q)[2], uint16_t & d) {
     const uint32_t * w = reinterpret_cast<const uint32_t *>(slot);
-    const int b = lane >> 2, k = 18 * b >> 2, m = k + 2 * (lane & 1);
+    const int a = mis + 18 * (lane >> 2), k = a >> 2, m = k + 2 * (lane & 1);
     const uint32_t t0 = w[m], t1 = w[m + 1], t2 = w[m + 2], s = w[k];
-    const bool odd = b & 1;
-    d = (uint16_t)(odd ? s >> 16 : s);
-    q[0] = odd ? t1 : (t0 >> 16 | t1 << 16);
-    q[1] = odd ? t2 : (t1 >> 16 | t2 << 16);
+    const bool half = a & 2;
+    d = (uint16_t)(half ? s >> 16 : s);
+    q[0] = half ? t1 : (t0 >> 16 | t1 << 16);
+    q[1] = half ? t2 : (t1 >> 16 | t2 << 16);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -593,6 +592,7 @@ __device__ __forceinline__ void q4_slice_pick(const unsigned char * slot, int la
 struct __attribute__((packed)) pi_q8_host_block { uint16_t d; int8_t qs[32]; };
 constexpr int kSide = 2;                   // neurons whose wave sums are formed side by side (4: 17.4 us and, for the resident share of a split layer, 10.9 against 9.9)
 
+// ANY: matrices that do not all start on multiples of 16 (odd_address: one at an odd address).
 // SPLIT: the neurons outside the hot words are computed here too, from a second pair of matrices that holds exactly those
 // neurons' rows in ascending order (rows in pinned host memory, fetched over the host link by the loads below).
 // PHASE 1 / 2 cut the launch in two for a hybrid layer whose host share should start as early as possible: 1 stops behind the
@@ -603,7 +603,7 @@ constexpr int kSide = 2;                   // neurons whose wave sums are formed
 // or SPLIT) the launch goes on with the down projection: h of the group is quantised as the CPU path quantises the dense vector
 // (ggml.c:14465-14618), and each wave adds its 512-column slice of the down rows of the neurons with a non-zero quant, in ascending
 // order and with axpy_q4_groups_kernel's arithmetic; the workgroup's partial output vector goes to `partial` for ffn_reduce_kernel.
-template <int RCH, bool GATE, bool SPLIT, int PHASE = 0, bool FUSE = false>
+template <int RCH, bool GATE, bool SPLIT, int PHASE = 0, bool FUSE = false, bool ANY = false>
 __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __half * __restrict__ W2, const float * __restrict__ hidden,
                                                                      const pi_block_q4_0 * __restrict__ Wup, const pi_block_q4_0 * __restrict__ Wgate,
                                                                      const pi_block_q4_0 * __restrict__ Wup_rest, const pi_block_q4_0 * __restrict__ Wgate_rest,
@@ -613,7 +613,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
                                                                      float * __restrict__ h_dense, pi_q8_host_block * __restrict__ xq_out,
                                                                      float * __restrict__ logits2,
                                                                      const pi_block_q4_0 * __restrict__ Wd, const pi_block_q4_0 * __restrict__ Wd_rest,
-                                                                     float * __restrict__ partial, HostAnnounce ann, int aligned) {
+                                                                     float * __restrict__ partial, HostAnnounce ann, int odd_address) {
     static_assert(!FUSE || PHASE == 0, "the two-phase form of a hybrid layer leaves the down projection to its own launch");
     if (PHASE == 2 && ann.flags && blockIdx.x == 0 && threadIdx.x == 0) {
         // what was queued before this launch is complete and visible to the host (the kernel boundary released at system scope):
@@ -622,12 +622,12 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
         *ann.seq = sq;
         __hip_atomic_store(ann.flags, sq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
-    constexpr int cols = 4096, r = RCH * 512, nb = cols / 32, CH = kPfChunk;
+    constexpr int cols = 4096, r = RCH * 512, nb = cols / 32, CH = kPfChunk, kSlot = ANY ? kQ4Slot : kQ4Slice;
     __shared__ float  hs[32];
     __shared__ float  lg[32];
     __shared__ double red[2][kPfWaves];
     __shared__ float  part[kPfWaves][CH][2];
-    __shared__ __align__(16) unsigned char slices[PHASE == 1 ? 16 : kPfWaves * (FUSE ? 3 : 2) * CH * kQ4Slice];       // of the chunk's up, gate and, first chunk, down rows
+    __shared__ __align__(16) unsigned char slices[PHASE == 1 ? 16 : kPfWaves * (FUSE ? 3 : 2) * CH * kSlot];       // of the chunk's up, gate and, first chunk, down rows
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int n0 = blockIdx.x * 32;
     const int cbase = wave * 512 + lane * 8;
@@ -769,13 +769,17 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
     // ---- B -------------------------------------------------------------------------------------------------
     const int n = __popc(sel);
     const int shift = (sub >> 1) * 4;
-    unsigned char * const mine = slices + wave * (FUSE ? 3 : 2) * CH * kQ4Slice;
-    auto slot = [&](int kind, int j) { return mine + (kind * CH + j) * kQ4Slice; };
+    unsigned char * const mine = slices + wave * (FUSE ? 3 : 2) * CH * kSlot;
+    auto slot = [&](int kind, int j) { return mine + (kind * CH + j) * kSlot; };
     auto row_of = [&](const pi_block_q4_0 * W, const pi_block_q4_0 * W_rest, int bit) {
         const int below = __popc(hot & ((1u << bit) - 1u));
         const bool rest = SPLIT && !((hot >> bit) & 1u);               // n0 - base_row neurons outside the hot set lie before this group
         const size_t row = rest ? (size_t)(n0 - base_row + bit - below) : (size_t)(base_row + below);
         return reinterpret_cast<const unsigned char *>(rest ? W_rest : W) + row * (nb * 18) + wave * kQ4Slice;
+    };
+    const bool odd = ANY && odd_address;
+    auto mis_of = [&](const pi_block_q4_0 * W, const pi_block_q4_0 * W_rest, int bit) {        // rows and slices are multiples of 16 bytes
+        return !ANY || odd ? 0 : (int)((uintptr_t)(SPLIT && !((hot >> bit) & 1u) ? W_rest : W) & 15);
     };
     int first[CH];                                                     // FUSE: the first chunk's neurons
     uint32_t todo = sel;
@@ -787,17 +791,17 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
             if (j < nn) { nrn[j] = n0 + __ffs(todo) - 1; todo &= todo - 1; } else nrn[j] = nrn[j ? j - 1 : 0];
             if (c0 == 0) first[j] = nrn[j] - n0;
         }
-        if (aligned) {
+        if (!odd) {
 #pragma unroll
             for (int j = 0; j < CH; ++j)
                 if (j < nn) {
-                    q4_slice_fetch(row_of(Wup, Wup_rest, nrn[j] - n0), slot(0, j), lane);
-                    if (GATE) q4_slice_fetch(row_of(Wgate, Wgate_rest, nrn[j] - n0), slot(1, j), lane);
+                    q4_slice_fetch<ANY>(row_of(Wup, Wup_rest, nrn[j] - n0), slot(0, j), lane);
+                    if (GATE) q4_slice_fetch<ANY>(row_of(Wgate, Wgate_rest, nrn[j] - n0), slot(1, j), lane);
                 }
             if (FUSE && c0 == 0) {
                 // the down rows travel behind them; CH of them whatever n is, so that the wait is for the others alone
 #pragma unroll
-                for (int j = 0; j < CH; ++j) q4_slice_fetch(row_of(Wd, Wd_rest, first[j]), slot(2, j), lane);
+                for (int j = 0; j < CH; ++j) q4_slice_fetch<ANY>(row_of(Wd, Wd_rest, first[j]), slot(2, j), lane);
                 asm volatile("s_waitcnt vmcnt(%0)" :: "n"(CH) : "memory");
             } else {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -809,9 +813,9 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
             for (int j = 0; j < nn; ++j) {
                 const int bit = __ffs(left) - 1;
                 left &= left - 1;
-                q4_slice_fetch_any(row_of(Wup, Wup_rest, bit), slot(0, j), lane);
-                if (GATE) q4_slice_fetch_any(row_of(Wgate, Wgate_rest, bit), slot(1, j), lane);
-                if (FUSE && c0 == 0) q4_slice_fetch_any(row_of(Wd, Wd_rest, bit), slot(2, j), lane);
+                q4_slice_fetch_odd(row_of(Wup, Wup_rest, bit), slot(0, j), lane);
+                if (GATE) q4_slice_fetch_odd(row_of(Wgate, Wgate_rest, bit), slot(1, j), lane);
+                if (FUSE && c0 == 0) q4_slice_fetch_odd(row_of(Wd, Wd_rest, bit), slot(2, j), lane);
             }
             asm volatile("" ::: "memory");
         }
@@ -823,7 +827,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
 #pragma unroll
             for (int jj = 0; jj < kSide; ++jj) {
                 uint32_t q[2]; uint16_t d;
-                q4_slice_pick(slot(0, j0 + jj), lane, q, d);
+                q4_slice_pick(slot(0, j0 + jj), mis_of(Wup, Wup_rest, nrn[j0 + jj] - n0), lane, q, d);
                 int su = __builtin_amdgcn_sdot4((int)((q[0] >> shift) & 0x0F0F0F0Fu), xq0, 0, false);
                 su = __builtin_amdgcn_sdot4((int)((q[1] >> shift) & 0x0F0F0F0Fu), xq1, su, false) - 8 * sx;
                 su += pi_dpp_i32<PI_DPP_XOR1, 0xF>(su);
@@ -831,7 +835,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
                 pu[jj] = sub == 0 ? __fmul_rn(__fmul_rn(pi_f16_from_bits(d), dx), (float)su) : 0.0f;
                 pg[jj] = 0.0f;
                 if (GATE) {
-                    q4_slice_pick(slot(1, j0 + jj), lane, q, d);
+                    q4_slice_pick(slot(1, j0 + jj), mis_of(Wgate, Wgate_rest, nrn[j0 + jj] - n0), lane, q, d);
                     int sg = __builtin_amdgcn_sdot4((int)((q[0] >> shift) & 0x0F0F0F0Fu), xq0, 0, false);
                     sg = __builtin_amdgcn_sdot4((int)((q[1] >> shift) & 0x0F0F0F0Fu), xq1, sg, false) - 8 * sx;
                     sg += pi_dpp_i32<PI_DPP_XOR1, 0xF>(sg);
@@ -874,9 +878,9 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
         // neurons that add something, ascending
-        auto add_row = [&](const unsigned char * row, int alpha) {
+        auto add_row = [&](const unsigned char * row, int bit, int alpha) {
             uint32_t q[2]; uint16_t dw;
-            q4_slice_pick(row, lane, q, dw);
+            q4_slice_pick(row, mis_of(Wd, Wd_rest, bit), lane, q, dw);
             const float d = __fmul_rn(pi_f16_from_bits(dw), dh);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -891,7 +895,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
             if (j < n) {
                 later &= later - 1;
                 const int alpha = __builtin_amdgcn_readlane(qh, first[j]);
-                if (alpha != 0) add_row(slot(2, j), alpha);
+                if (alpha != 0) add_row(slot(2, j), first[j], alpha);
             }
         later &= (uint32_t)__ballot(qh != 0);
         while (later) {
@@ -899,11 +903,11 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_upgate_q4_kernel(const __hal
             uint32_t next = later;
             for (int j = 0; j < nrows; ++j) {
                 const unsigned char * src = row_of(Wd, Wd_rest, __ffs(next) - 1);
-                if (aligned) q4_slice_fetch(src, slot(0, j), lane); else q4_slice_fetch_any(src, slot(0, j), lane);
+                if (!odd) q4_slice_fetch<ANY>(src, slot(0, j), lane); else q4_slice_fetch_odd(src, slot(0, j), lane);
                 next &= next - 1;
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            for (int j = 0; j < nrows; ++j) { add_row(slot(0, j), __builtin_amdgcn_readlane(qh, __ffs(later) - 1)); later &= later - 1; }
+            for (int j = 0; j < nrows; ++j) { const int bit = __ffs(later) - 1; add_row(slot(0, j), bit, __builtin_amdgcn_readlane(qh, bit)); later &= later - 1; }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // the slots are free again
         }
         float4 * po = reinterpret_cast<float4 *>(partial + (size_t)blockIdx.x * cols + cbase);
@@ -1038,11 +1042,11 @@ __global__ void host_wait_kernel(const uint32_t * __restrict__ seq, uint32_t * _
 
 }  // namespace
 
-// rows of 2304 bytes of matrices that start on multiples of 16 (null: not there)
-static int q4_rows_aligned(std::initializer_list<const void *> m) {
+// where these matrices start (null: not there): 0 where all of them are on multiples of 16, else whether one is at an odd address, + 2
+static int q4_starts(std::initializer_list<const void *> m) {
     uintptr_t all = 0;
     for (const void * p : m) all |= (uintptr_t)p;
-    return (all & 15) == 0;
+    return all & 15 ? 2 + (int)(all & 1) : 0;
 }
 
 extern "C" {
@@ -1077,11 +1081,14 @@ int pi_k_pred_upgate_q4_split(const void * fc2_f16, int ff, int r, const float *
     const pi_block_q4_0 * u = (const pi_block_q4_0 *)up_q4; const pi_block_q4_0 * g = (const pi_block_q4_0 *)gate_q4;
     const dim3 grid(ff / 32), block(kPfBlock);
     const pi_block_q4_0 * ur = (const pi_block_q4_0 *)up_rest_q4; const pi_block_q4_0 * gr = (const pi_block_q4_0 *)gate_rest_q4;
-#define PI_PQ_LAUNCH(RCH, GATE, SPLIT) hipLaunchKernelGGL((pred_upgate_q4_kernel<RCH, GATE, SPLIT>), grid, block, 0, st, w2, hidden, u, g, ur, gr, x, na, threshold, hot_words, hot_prefix, logits, ws->words, ws->words_hot, h_dense, (pi_q8_host_block *)xq8_out, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, q4_rows_aligned({u, g, ur, gr}))
-#define PI_PQ_LAUNCH_S(RCH, GATE) do { if (ur) PI_PQ_LAUNCH(RCH, GATE, true); else PI_PQ_LAUNCH(RCH, GATE, false); } while (0)
+#define PI_PQ_LAUNCH(RCH, GATE, SPLIT, ANY) hipLaunchKernelGGL((pred_upgate_q4_kernel<RCH, GATE, SPLIT, 0, false, ANY>), grid, block, 0, st, w2, hidden, u, g, ur, gr, x, na, threshold, hot_words, hot_prefix, logits, ws->words, ws->words_hot, h_dense, (pi_q8_host_block *)xq8_out, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, starts & 1)
+    const int starts = q4_starts({u, g, ur, gr});
+#define PI_PQ_LAUNCH_A(RCH, GATE, SPLIT) do { if (starts) PI_PQ_LAUNCH(RCH, GATE, SPLIT, true); else PI_PQ_LAUNCH(RCH, GATE, SPLIT, false); } while (0)
+#define PI_PQ_LAUNCH_S(RCH, GATE) do { if (ur) PI_PQ_LAUNCH_A(RCH, GATE, true); else PI_PQ_LAUNCH_A(RCH, GATE, false); } while (0)
     if (r == 1024) { if (g) PI_PQ_LAUNCH_S(2, true); else PI_PQ_LAUNCH_S(2, false); }
     else           { if (g) PI_PQ_LAUNCH_S(1, true); else PI_PQ_LAUNCH_S(1, false); }
 #undef PI_PQ_LAUNCH_S
+#undef PI_PQ_LAUNCH_A
 #undef PI_PQ_LAUNCH
     return pi::check_launch("pi_k_pred_upgate_q4");
 }
@@ -1103,11 +1110,14 @@ int pi_k_sparse_ffn_q4_partials(const void * fc2_f16, int ff, int r, const float
     const pi_block_q4_0 * u = (const pi_block_q4_0 *)up_q4; const pi_block_q4_0 * g = (const pi_block_q4_0 *)gate_q4; const pi_block_q4_0 * dn = (const pi_block_q4_0 *)down_t_q4;
     const pi_block_q4_0 * ur = (const pi_block_q4_0 *)up_rest_q4; const pi_block_q4_0 * gr = (const pi_block_q4_0 *)gate_rest_q4; const pi_block_q4_0 * dr = (const pi_block_q4_0 *)down_t_rest_q4;
     const dim3 grid(ff / 32), block(kPfBlock);
-#define PI_PQF(RCH, GATE, SPLIT) hipLaunchKernelGGL((pred_upgate_q4_kernel<RCH, GATE, SPLIT, 0, true>), grid, block, 0, st, w2, hidden, u, g, ur, gr, x, na, threshold, hot_words, hot_prefix, logits, ws->words, (uint32_t *)nullptr, h_dense, (pi_q8_host_block *)nullptr, (float *)nullptr, dn, dr, ws->ffn_partial, HostAnnounce{nullptr, nullptr}, q4_rows_aligned({u, g, dn, ur, gr, dr}))
-#define PI_PQF_S(RCH, GATE) do { if (split) PI_PQF(RCH, GATE, true); else PI_PQF(RCH, GATE, false); } while (0)
+#define PI_PQF(RCH, GATE, SPLIT, ANY) hipLaunchKernelGGL((pred_upgate_q4_kernel<RCH, GATE, SPLIT, 0, true, ANY>), grid, block, 0, st, w2, hidden, u, g, ur, gr, x, na, threshold, hot_words, hot_prefix, logits, ws->words, (uint32_t *)nullptr, h_dense, (pi_q8_host_block *)nullptr, (float *)nullptr, dn, dr, ws->ffn_partial, HostAnnounce{nullptr, nullptr}, starts & 1)
+    const int starts = q4_starts({u, g, dn, ur, gr, dr});
+#define PI_PQF_A(RCH, GATE, SPLIT) do { if (starts) PI_PQF(RCH, GATE, SPLIT, true); else PI_PQF(RCH, GATE, SPLIT, false); } while (0)
+#define PI_PQF_S(RCH, GATE) do { if (split) PI_PQF_A(RCH, GATE, true); else PI_PQF_A(RCH, GATE, false); } while (0)
     if (r == 1024) { if (g) PI_PQF_S(2, true); else PI_PQF_S(2, false); }
     else           { if (g) PI_PQF_S(1, true); else PI_PQF_S(1, false); }
 #undef PI_PQF_S
+#undef PI_PQF_A
 #undef PI_PQF
     return pi::check_launch("pi_k_sparse_ffn_q4_partials");
 }
@@ -1147,8 +1157,10 @@ int pi_k_upgate_q4_hot_rows(int ff, float threshold, const void * up_q4, const v
     const dim3 grid(ff / 32), block(kPfBlock);
     const pi_block_q4_0 * none = nullptr;
     const pi_block_q4_0 * u = (const pi_block_q4_0 *)up_q4; const pi_block_q4_0 * g = (const pi_block_q4_0 *)gate_q4;
-#define PI_PQ2(GATE) hipLaunchKernelGGL((pred_upgate_q4_kernel<1, GATE, false, 2>), grid, block, 0, (hipStream_t)stream, (const __half *)nullptr, (const float *)nullptr, u, g, none, none, x, na, threshold, hot_words, hot_prefix, (float *)nullptr, ws->words, ws->words_hot, h_dense, (pi_q8_host_block *)nullptr, const_cast<float *>(logits_dev), none, none, (float *)nullptr, HostAnnounce{announce_seq, announce_flags}, q4_rows_aligned({u, g}))
-    if (g) PI_PQ2(true); else PI_PQ2(false);
+    const int starts = q4_starts({u, g});
+#define PI_PQ2(GATE, ANY) hipLaunchKernelGGL((pred_upgate_q4_kernel<1, GATE, false, 2, false, ANY>), grid, block, 0, (hipStream_t)stream, (const __half *)nullptr, (const float *)nullptr, u, g, none, none, x, na, threshold, hot_words, hot_prefix, (float *)nullptr, ws->words, ws->words_hot, h_dense, (pi_q8_host_block *)nullptr, const_cast<float *>(logits_dev), none, none, (float *)nullptr, HostAnnounce{announce_seq, announce_flags}, starts & 1)
+    if (starts) { if (g) PI_PQ2(true, true); else PI_PQ2(false, true); }
+    else        { if (g) PI_PQ2(true, false); else PI_PQ2(false, false); }
 #undef PI_PQ2
     return pi::check_launch("pi_k_upgate_q4_hot_rows");
 }

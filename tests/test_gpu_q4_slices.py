@@ -46,6 +46,30 @@ def test_busy_groups_and_odd_addresses(has_gate, r, threshold):
         assert rel_err(out[0][0], ou["h"]) < 1e-4 and rel_err(out[0][1], ou["out"]) < FFN_REL_TOL
 
 
+@pytest.mark.parametrize("has_gate,r,threshold", [(True, 1024, 0.0), (False, 512, -3e38)])
+def test_rows_at_any_address(has_gate, r, threshold):
+    """Up, gate and down matrices that start 4, 8, 12, 14 bytes behind a multiple of 16, at odd addresses, and each at another: the bits of aligned ones."""
+    from powerinfer_amd.ops import SparseFFN
+
+    class At:
+        def __init__(self, buf, by):
+            self.buf = pl.DevBuf(host=np.concatenate([np.zeros(by, np.uint8), buf.download(np.uint8), np.zeros(31 - by, np.uint8)]))
+            self.ptr = self.buf.ptr + by
+
+    d, ff = 4096, 512
+    L = synth.make_ffn_layer(seed=r, d=d, ff=ff, r=r, wtype=ol.Q4_0, has_gate=has_gate, mean_rate=0.4, T=1)
+    x, want = np.ascontiguousarray(L["x"][:1], np.float32)[0], None
+    for at in ((0, 0, 0), (4, 4, 4), (8, 12, 14), (2, 0, 12), (14, 14, 0), (1, 1, 1), (15, 2, 0), (0, 4, 7)):
+        ffn = SparseFFN(d, ff, r, ol.Q4_0, L["up"], L["gate"], L["down_t"], L["fc1"], L["fc2"], threshold=threshold)
+        for name, by in zip(("up", "gate", "down"), at):
+            if getattr(ffn, name) is not None:
+                setattr(ffn, name, At(getattr(ffn, name), by))
+        print(has_gate, r, at, flush=True)
+        got = ffn.forward_q4_one_launch(x, x)
+        want = want or got
+        assert np.array_equal(got["h"], want["h"]) and np.array_equal(got["out"], want["out"]) and want["out"].any(), at
+
+
 @pytest.mark.parametrize("rows,cols", [(5, 4096), (12290, 4096), (6145, 8192)])
 def test_mat_vec_of_a_matrix_on_4_bytes(rows, cols):
     """Every multiple of 4 behind a multiple of 16: the bits of the aligned matrix."""
