@@ -306,17 +306,19 @@ __global__ __launch_bounds__(256) void mix_and_up_kernel(pi_gqa_attn p, pi_gate_
 
 // ---------------------------------------------------------------------------------------------------------------------------------
 // what closes a layer: out[t] = x[t] + (W_o att[t] + sum over the token's experts of W_down[e] act[pair]), 16 or 8 rows a workgroup (or, what
-// closes a sublayer in front of its norm: out[t] = alpha x[t] + gate * W att[t]).  The pieces of 256 (8 rows: 512) columns of W_o and of every
-// expert of the step form one list that the waves take in turn.
+// closes a sublayer in front of its norm: out[t] = alpha x[t] + gate * W att[t]).  The pieces of 256 columns of W_o and of every
+// expert of the step form one list that the waves take in turn; with 8 rows a wave takes two of its pieces at a time, one behind the
+// other in the tile, so that sums are formed in one order whatever the rows.
 // Bound by the weights.  A piece's tokens were once read when its turn came: loads return in order, so each piece also waited for the weights
 // requested after it and a wave had one piece in flight instead of two; and 16 rows a workgroup leave half the compute units idle at 2048 rows.
 // 16 tokens, 2048 rows, 51 of 64 experts of 1408 (306 MB) and dense layers in turn: 65.7 us a layer, 56 with 8 rows and both requested
-// together, 52.6 with the requests free of branches.
+// together, 53 with the requests free of branches.
 // ---------------------------------------------------------------------------------------------------------------------------------
 template <int NW, int RT>      // waves, rows a workgroup
 __global__ __launch_bounds__(64 * NW) void layer_out_step_kernel(pi_layer_out a) {
-    constexpr int COLS = 4096 / RT, NX = COLS / 32, LR = COLS / 8, PITCH = COLS * 2 + 16;      // columns of a piece (eight loads of a wave), its steps of 32, lanes of a row, bytes of a staged row
-    __shared__ __align__(16) unsigned char tiles[NW][RT * PITCH];
+    constexpr int COLS = 256, NX = COLS / 32, LR = COLS / 8, PITCH = COLS * 2 + 16;      // columns of a piece, its steps of 32, lanes of a row, bytes of a staged row
+    constexpr int NP = 16 / RT, NL = 8 / NP;           // pieces a turn (their rows together fill the tile of 16), loads of a piece
+    __shared__ __align__(16) unsigned char tiles[NW][16 * PITCH];
     __shared__ StepExperts se;
     __shared__ int first[kStepExperts];
     // (eight waves: the workgroup's LDS exceeds half a compute unit's, so that no two share one while others idle)
@@ -324,65 +326,84 @@ __global__ __launch_bounds__(64 * NW) void layer_out_step_kernel(pi_layer_out a)
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
     const int row0 = blockIdx.x * RT, n_o = a.wo ? (a.ld_att + COLS - 1) / COLS : 0, n_e = a.ids ? (a.ld_act + COLS - 1) / COLS : 1;
     const int tok = min(i, a.T - 1);
-    pi_u32x4 ld[2][8], x[2][NX];
-    int left[2];                                       // columns of the piece and behind it; 0: the token has no part in it
+    pi_u32x4 ld[2][8], x[2][NP * NX];
+    int left[2][NP];                                   // columns of a piece and behind it; 0: the token has no part in it
     pi_f4 acc = pi_f4{0, 0, 0, 0};
-    // a piece's weights and its tokens' values are requested together, two pieces ahead and without branches (past the end: the last columns again)
-    auto request = [&](pi_u32x4 (&l)[8], pi_u32x4 (&v)[NX], int & rest, int ss) {
+    // a piece's weights and its tokens' values are requested together, two turns ahead and without branches (past the end: the last columns again)
+    auto request_piece = [&](pi_u32x4 * l, pi_u32x4 * v, int & rest, int ss) {
         const bool att = ss < n_o;
         const int k = att ? 0 : (ss - n_o) / n_e, c = (att ? ss : (ss - n_o) % n_e) * COLS, cols = att ? a.ld_att : a.ld_act;
         const bf16 * w = att ? (const bf16 *)a.wo : (const bf16 *)a.down + (size_t)se.expert[k] * a.rows * a.ld_act;
         const int at = min(c + (lane % LR) * 8, cols - 8);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) l[j] = pi_ld_stream(w + (size_t)min(row0 + j * (RT / 8) + lane / LR, a.rows - 1) * cols + at);
+        for (int j = 0; j < NL; ++j) l[j] = pi_ld_stream(w + (size_t)min(row0 + 2 * j + lane / LR, a.rows - 1) * cols + at);
         const int pair = att ? tok : se.slot[k][i];
         const bf16 * xp = (att ? (const bf16 *)a.att : (const bf16 *)a.act) + (size_t)max(pair, 0) * cols;
 #pragma unroll
         for (int st = 0; st < NX; ++st) v[st] = pi_ld16(xp + min(c + st * 32, cols - 32) + g * 8);
         rest = pair >= 0 ? cols - c : 0;
     };
-    // the attention's pieces are requested before the experts are known
-    if (wave < n_o) request(ld[0], x[0], left[0], wave);
-    if (wave + NW < n_o) request(ld[1], x[1], left[1], wave + NW);
-    const int n_exp = a.ids ? step_experts(se, first, a.ids, a.T * a.top, a.top, a.n_expert) : 0, n_ss = n_o + n_exp * n_e;
-    const int m = wave < n_ss ? (n_ss - wave + NW - 1) / NW : 0;                 // this wave's pieces: wave, wave + NW, ...
-    if (wave >= n_o && m > 0) request(ld[0], x[0], left[0], wave);
-    if (wave + NW >= n_o && m > 1) request(ld[1], x[1], left[1], wave + NW);
-    auto multiply = [&](const pi_u32x4 (&l)[8], const pi_u32x4 (&v)[NX], int rest) {
+    // turn t of this wave's pieces wave, wave + NW, ..: pieces t NP .. of them, in this order, as far as `upto` goes
+    auto piece_of = [&](int t, int p) { return wave + (t * NP + p) * NW; };
+    auto request = [&](int b, int t, int from, int upto) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) *reinterpret_cast<pi_u32x4 *>(tiles[wave] + (j * (RT / 8) + lane / LR) * PITCH + (lane % LR) * 16) = l[j];
-#pragma unroll
-        for (int st = 0; st < NX; ++st)
-            acc = mma16<bf16>(*reinterpret_cast<const pi_u32x4 *>(tiles[wave] + (i % RT) * PITCH + (4 * st + g) * 16), st * 32 < rest ? v[st] : pi_u32x4{0, 0, 0, 0}, acc);
+        for (int p = 0; p < NP; ++p)
+            if (piece_of(t, p) >= from && piece_of(t, p) < upto) request_piece(&ld[b][p * NL], &x[b][p * NX], left[b][p], piece_of(t, p));
     };
-    // (no branch around a request while pieces are left for both buffers: what a wait leaves in flight is then known when it is compiled)
-    int it = 0;
-    for (; it + 4 <= m; it += 2)
+    // the attention's pieces are requested before the experts are known
+    request(0, 0, 0, n_o);
+    request(1, 1, 0, n_o);
+    const int n_exp = a.ids ? step_experts(se, first, a.ids, a.T * a.top, a.top, a.n_expert) : 0, n_ss = n_o + n_exp * n_e;
+    const int m = wave < n_ss ? (n_ss - wave + NW - 1) / NW : 0, whole = m / NP;           // this wave's pieces; whole turns of them
+    request(0, 0, n_o, n_ss);
+    request(1, 1, n_o, n_ss);
+    auto multiply = [&](int b, int n) {                // n: pieces of the turn
+#pragma unroll
+        for (int j = 0; j < 8; ++j) *reinterpret_cast<pi_u32x4 *>(tiles[wave] + (2 * j + lane / LR) * PITCH + (lane % LR) * 16) = ld[b][j];
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            if (p < n) {
+#pragma unroll
+                for (int st = 0; st < NX; ++st)
+                    acc = mma16<bf16>(*reinterpret_cast<const pi_u32x4 *>(tiles[wave] + (p * RT + i % RT) * PITCH + (4 * st + g) * 16),
+                                      st * 32 < left[b][p] ? x[b][p * NX + st] : pi_u32x4{0, 0, 0, 0}, acc);
+            }
+    };
+    // (no branch around a request while whole turns are left for both buffers: what a wait leaves in flight is then known when it is compiled)
+    int t = 0;
+    for (; t + 4 <= whole; t += 2)
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
-            multiply(ld[b], x[b], left[b]);
-            request(ld[b], x[b], left[b], wave + (it + 2 + b) * NW);
+            multiply(b, NP);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) request_piece(&ld[b][p * NL], &x[b][p * NX], left[b][p], piece_of(t + 2 + b, p));
         }
-    const int rem = m - it;
-    if (rem >= 1) multiply(ld[0], x[0], left[0]);
-    if (rem == 3) request(ld[0], x[0], left[0], wave + (it + 2) * NW);
-    if (rem >= 2) multiply(ld[1], x[1], left[1]);
-    if (rem == 3) multiply(ld[0], x[0], left[0]);
+    // up to four turns, the last of which may be short of a piece
+    const int turns = (m + NP - 1) / NP - t;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        if (b < turns) {
+            multiply(b, m - (t + b) * NP);
+            if (b + 2 < turns) request(b, t + b + 2, 0, n_ss);
+        }
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        if (b + 2 < turns) multiply(b, m - (t + b + 2) * NP);
     float (*cs)[17] = reinterpret_cast<float (*)[17]>(tiles[wave]);
 #pragma unroll
     for (int r = 0; r < 4; ++r) if (4 * g + r < RT) cs[4 * g + r][i] = acc[r];
     __syncthreads();
     if (tid >= 16 * RT) return;
-    const int t = tid / RT, row = row0 + tid % RT;
-    if (row >= a.rows || t >= a.T) return;
+    const int tk = tid / RT, row = row0 + tid % RT;
+    if (row >= a.rows || tk >= a.T) return;
     float v = 0.0f;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) v += reinterpret_cast<float (*)[17]>(tiles[w])[tid % RT][t];
-    if (a.gate_z) v *= sigmoid_f32(a.gate_z[(size_t)t * a.ld_gate + a.off_gate + row] + a.gate_b[row]);
-    const float x0 = a.x ? a.x[(size_t)t * a.rows + row] : 0.0f;
+    for (int w = 0; w < NW; ++w) v += reinterpret_cast<float (*)[17]>(tiles[w])[tid % RT][tk];
+    if (a.gate_z) v *= sigmoid_f32(a.gate_z[(size_t)tk * a.ld_gate + a.off_gate + row] + a.gate_b[row]);
+    const float x0 = a.x ? a.x[(size_t)tk * a.rows + row] : 0.0f;
     v += a.scaled ? a.alpha * x0 : x0;
-    a.out[(size_t)t * a.rows + row] = v;
-    if (a.keep) a.keep[(size_t)t * a.rows + row] = v;
+    a.out[(size_t)tk * a.rows + row] = v;
+    if (a.keep) a.keep[(size_t)tk * a.rows + row] = v;
 }
 
 }  // namespace

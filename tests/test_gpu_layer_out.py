@@ -51,3 +51,26 @@ def test_closing_a_layer(rows, ld_att, E, top, ld_act, T):
     n = ld_att + top * ld_act                                         # products of bf16 are exact in fp32: only their sum rounds
     assert (np.abs(got - want) <= (n / 8 + 32) * 2.0 ** -24 * mag).all()
     assert np.array_equal(keep.download(np.float32).reshape(T, rows), got)
+
+
+@pytest.mark.parametrize("ld_att,E,top,ld_act,T", [(2048, 9, 3, 1408, 16), (32, 0, 0, 0, 1), (4096, 0, 0, 0, 5), (0, 5, 2, 288, 3), (544, 40, 6, 544, 16), (0, 2, 2, 4096, 7), (6144, 3, 1, 96, 2)])
+def test_rows_a_workgroup_do_not_change_the_sums(ld_att, E, top, ld_act, T):
+    """A matrix's first rows by themselves (8 rows a workgroup) and inside one of twice as many (16): the same bits."""
+    L, rng = pl.init(), np.random.default_rng(ld_att + E + T)
+    many, few = 4096, 1000                                            # 256 and 63 workgroups of 16 rows for 256 compute units
+    wo, att = bf16(rng.standard_normal((many, max(ld_att, 32)))), bf16(rng.standard_normal((T, max(ld_att, 32))))
+    down, act = bf16(rng.standard_normal((max(E, 1), many, max(ld_act, 32)))), bf16(rng.standard_normal((T, max(top, 1), max(ld_act, 32))))
+    ids = np.stack([rng.permutation(max(E, 1))[:max(top, 1)] for _ in range(T)]).astype(np.int32)
+    got = []
+    for rows in (few, many):
+        out, s = pl.DevBuf.zeros(4 * T * rows), pl.LayerOut()
+        hold = [pl.DevBuf(host=np.ascontiguousarray(a)) for a in (wo[:rows], att, down[:, :rows], act, ids)]
+        s.rows, s.T, s.out = rows, T, out.ptr
+        if ld_att:
+            s.wo, s.att, s.ld_att = hold[0].ptr, hold[1].ptr, ld_att
+        if E:
+            s.down, s.act, s.ids, s.ld_act, s.top, s.n_expert = hold[2].ptr, hold[3].ptr, hold[4].ptr, ld_act, top, E
+        print(rows, ld_att, E, top, ld_act, T, flush=True)
+        pl.check(L.pi_k_layer_out_step(C.byref(s), None))
+        got.append(out.download(np.float32).reshape(T, rows)[:, :few])
+    assert np.array_equal(*got) and got[0].any()
