@@ -960,7 +960,7 @@ def test_prompt_chunks_match_token_by_token(arch, wtype):
                                                    ("llama-tiny", dict(n_rank=256, n_ctx=192), 40, "lib"),
                                                    ("llama-7b", dict(n_layer=2, n_ctx=640), 600, "lib")])
 def test_wide_prompt_chunks_match_the_oracle(name, kw, n_prompt, gemm, monkeypatch):
-    """Prompts longer than 16 tokens go through chunks of up to 512 (dense mat-muls through the library, or on this library's own
+    """Prompts longer than 16 tokens go through chunks of up to 2048, here of up to 599 (dense mat-muls through the library, or on this library's own
     LDS-tiled mat-mul kernel with PI_PREFILL_GEMM=own; every weight row read once per chunk, the predictor's mask applied as zeros
     of h), then chunks of 16, then the last token alone.  On a margin-protected model (no neuron can flip, greedy
     decisions keep their distance) the logits after the prompt and of the steps behind it agree with the CPU oracle within the
@@ -1007,7 +1007,7 @@ def test_wide_prompt_chunks_match_the_oracle(name, kw, n_prompt, gemm, monkeypat
                                                              ("falcon-tiny", synth.F16, 0.5, dict(n_rank=256, n_ctx=192), 60),
                                                              ("llama-7b", synth.Q4_0, 0.6, dict(n_layer=2, n_ctx=640), 600)])
 def test_wide_prompt_chunks_of_q4_and_hybrid_models(name, wtype, hot_frac, kw, n_prompt):
-    """Prompts of Q4_0 models and of models with a VRAM split also go through chunks of up to 512 tokens: a Q4_0 matrix is expanded
+    """Prompts of Q4_0 models and of models with a VRAM split also go through such chunks, products of Q4_0 models 512 tokens at a time: a Q4_0 matrix is expanded
     to fp16 for the chunk ((q - 8) * d) and multiplied with the values the CPU path's Q8_0 blocks keep of the activations, a
     hybrid layer's FFN matrices are assembled from the resident rows and the others' rows in pinned host memory.  On a
     margin-protected model the logits after the prompt and of the steps behind it agree with the CPU oracle within the stated

@@ -81,7 +81,7 @@ def test_groups_without_a_list(groups, rows, cols, T):
 
 
 @pytest.mark.parametrize("gated", [True, False])
-@pytest.mark.parametrize("ff,cols,T", [(128, 256, 1), (384, 320, 64), (256, 512, 65), (640, 256, 129), (2176, 256, 300)])
+@pytest.mark.parametrize("ff,cols,T", [(128, 256, 1), (384, 320, 64), (256, 512, 65), (640, 256, 129), (2176, 256, 300), (4352, 256, 3000)])
 def test_sparse_ffn_of_a_chunk(ff, cols, T, gated):
     """Up, gate, mask and product in one kernel: h within fp16's rounding of float64 where the fp32 sums' own error leaves it (products of
     `cols` terms of fp16 values: 2^-11 of h and 1e-5 of the largest), exact zeros where the predictor says so, threshold and NaN included."""

@@ -337,10 +337,10 @@ def test_north_star_long_context_allocation(arch, seed):
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("n_prompt", [300, 2200])
 def test_prompt_and_decode_at_a_context_beyond_the_chunk_kernels(n_prompt):
-    """n_ctx 16384, far more cells than the chunk kernels' LDS holds.  What a chunk needs is sized by the cells it attends, not by the
-    cache: a 300-token prompt still runs 16 tokens per workgroup on the matrix cores; a 2200-token prompt starts there and, from about
-    1850 cells on, goes through pi_k_attn_chunk_long (every token's cells split over several workgroups).  The token loop takes
-    pi_k_attn_split.  Prompt and 12 decoded tokens against the oracle, token by token."""
+    """n_ctx 16384, far more cells than the chunk kernels' LDS holds.  What a chunk needs is sized by the cells it attends, not by the cache.  The model's
+    predictor rank of 128 keeps it from the wide chunks (multiples of 256; test_gpu_prompt_chunks.py has those): its prompts go by 16
+    tokens, on the matrix cores as far as 1850 cells, then through pi_k_attn_chunk_long (every token's cells split over several
+    workgroups).  The token loop takes pi_k_attn_split.  Prompt and 12 decoded tokens against the oracle, token by token."""
     from powerinfer_amd.model import Model
     hp = synth.hparams("llama-tiny", n_ctx=16384, seed=23, **NS)
     model = synth.make_model(hp)

@@ -46,3 +46,56 @@ def test_cells_of_a_q4_prompt_do_not_depend_on_what_follows(name, hot):
         after[n] = m.decode([5], 512)[1]
     m.close()
     assert all(np.array_equal(a, after[602]) for a in after.values()), {n: float(np.abs(a - after[602]).max()) for n, a in after.items()}
+
+
+LONG = [("llama-tiny", synth.F16, 1.0, 1600, [1500]), ("falcon-tiny", synth.F16, 1.0, 2400, [2300]), ("llama-tiny", synth.F16, 1.0, 16384, [2300]),
+        ("llama-tiny", synth.F16, 1.0, 2400, [1100, 1200]), ("llama-tiny", synth.F16, 0.6, 1300, [1200]),
+        ("llama-tiny", synth.Q4_0, 1.0, 1300, [1200]), ("falcon-tiny", synth.Q4_0, 1.0, 2100, [600, 1400]), ("llama-tiny", synth.Q4_0, 0.6, 1300, [1200])]
+
+
+def eval_behind(om, prompt, steps, cur=None):
+    """Logits behind the prompt and of the steps on; the tokens of the steps: given, or greedy.  (logits, tokens)"""
+    tok, lg = om.eval(prompt, 0)
+    out, toks = [lg], [tok]
+    for i in range(steps):
+        tok, lg = om.eval([cur[i] if cur else toks[-1]], len(prompt) + i)
+        out.append(lg)
+        toks.append(tok)
+    return out, toks
+
+
+@pytest.mark.timeout(600)
+@pytest.mark.parametrize("name,wtype,hot,n_ctx,parts", LONG)
+def test_long_prompts_match_the_oracle(name, wtype, hot, n_ctx, parts):
+    """Chunks of more than 600 tokens, a remainder behind 2048 of them, a second chunk behind cells of the first, a cache beyond what the chunk kernels
+    hold, Q4_0 and split models: the logits behind the prompt and six steps on against the CPU path, every greedy token, on margin-protected
+    models.  F16: within 1e-2.  Q4_0: within that or twice what the CPU path departs from itself when its norm weights move by one unit in
+    the last place, either way (an activation rounded to eight bits the other way is a visible share of a dot product)."""
+    import oracle_lib as ol
+    hp = synth.hparams(name, n_rank=256, n_ctx=n_ctx, seed=5, pred_margin=True, head_pair=2048, wtype=wtype, hot_frac=hot)
+    model = synth.make_model(hp)
+    prompt = np.random.default_rng(8).integers(0, hp.n_vocab, sum(parts)).astype(np.int32)
+    rel = lambda a, b: float(np.abs(a - b).max() / np.abs(b).max())  # noqa: E731
+    om = ol.OracleModel(model)
+    want, toks = eval_behind(om, [int(t) for t in prompt], 6)
+    om.close()
+    median = most = 1e-2
+    for to in (0.0, 2.0) if wtype == synth.Q4_0 else ():
+        moved = dict(model, layers=[dict(L, attn_norm=np.nextafter(L["attn_norm"], np.float32(to))) for L in model["layers"]])
+        om = ol.OracleModel(moved)
+        own = [rel(a, b) for a, b in zip(eval_behind(om, [int(t) for t in prompt], 6, toks)[0], want)]
+        om.close()
+        median, most = max(median, 2 * float(np.median(own))), max(most, 2 * max(own))
+    m, at = fresh(hp, model), 0
+    for n in parts:
+        tok, lg = m.decode(prompt[at:at + n], at)
+        at += n
+    errs, got = [rel(lg, want[0])], [tok]
+    for i in range(6):
+        tok, lg = m.decode([toks[i]], at + i)
+        errs.append(rel(lg, want[i + 1]))
+        got.append(tok)
+    m.close()
+    print(name, wtype, hot, parts, f"median {np.median(errs):.4f} of {median:.4f}, most {max(errs):.4f} of {most:.4f}", flush=True)
+    assert got == toks
+    assert np.median(errs) <= median and max(errs) <= most, errs
