@@ -17,7 +17,7 @@ LIB = os.path.join(HERE, "libpowerinfer_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-pthread",
-    # packed-FP32 instructions are not to be generated on this hardware pool
+    # no packed-FP32 instructions: some of their forms have given wrong results now and then
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # a product and a sum fuse into one FMA only where the source writes them as one expression: hipcc's default ("fast") also
     # fuses across statements and through __fmul_rn / __fadd_rn (plain * and + in the HIP headers), which moves results by one

@@ -383,7 +383,7 @@ BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
 }  // namespace
 
 namespace {
-// one layer of a wide prompt chunk (16 < T <= 128): every mat-mul reads its matrix once for the chunk; with that many tokens the union
+// one layer of a wide prompt chunk (16 < T <= 2048): every mat-mul reads its matrix once for the chunk; with that many tokens the union
 // of the active sets is nearly every neuron, so gate/up run dense and the predictor's mask turns into exact zeros of h (what the
 // sparse operators compute, term by term: an inactive neuron contributes nothing to the down projection)
 // f(t0, n) for the pieces of the chunk's tokens that products and attention take at a time (pi::WideRoute)

@@ -90,7 +90,7 @@ struct pi_model {
     BatchState * cells = nullptr;         // the KV cache with cells shared between sequences and its step buffers (pi_model_kv_cells_*)
     BatchState * prefill = nullptr;       // step buffers for prompt chunks of the model's own sequence
     BatchState * prefill_wide = nullptr;  // the same for chunks of up to 2048 tokens (dense mat-muls, weights read once per chunk)
-    pi_gemm_lib * gemm_lib = nullptr;     // hipBLASLt plans of those mat-muls (PI_PREFILL_GEMM=own keeps them on this library's kernel, 128 tokens a chunk)
+    pi_gemm_lib * gemm_lib = nullptr;     // hipBLASLt plans of those mat-muls (PI_PREFILL_GEMM=own keeps them on this library's kernel)
     // multi-token steps of a Q4_0 model on integer matrix cores: every Q4_0 matrix once more as 16-byte-aligned quants and fp16
     // scales (pi_k_q4_split), made at the first such step; q4_steps says the model takes that route
     struct Q4Split { const void * quants; const void * scales; };

@@ -783,8 +783,10 @@ int experts(pi_model * m, Layer & L, const void * h, const Step & in) {
     const pi_layer_desc & d = L.d;
     const int T = in.T, D = m->hp.n_embd, per = d.ffn == PI_FFN_GLU_MOE ? 2 : 1;
     hipStream_t st = m->stream;
-    // tokens per tile, by the tokens an expert has on average: the large tiles read the weights once where most experts have more than 64
-    // tokens (64 experts 1408 x 2048, us with 64 and 128: 47 tokens 145 + 84 and 154 + 73; 72 tokens 197 + 101 and 161 + 81; 94 tokens 204 + 102 and 163 + 85)
+    // tokens per tile, by the tokens an expert has on average (multinomial counts): tiles of 128 read the weights once where tiles of 64 start to
+    // need two.  Both products of seven shapes (experts x ff x width; us with tiles of 64 and 128 at 48 / 56 / 72 tokens): 64 x 1408 x 2048
+    // 222, 228 / 245, 232 / 291, 243; 64 x 1408 x 4096 429, 435 / 469, 438 / 591, 452; 8 x 4096 x 4096 153, 173 / 178, 174 / 255, 177;
+    // 32 x 512 x 1024 25, 28 / 33, 28 / 33, 29; 16 x 1408, 128 x 768 and 256 x 512 x 2048 alike up to 48 and 7 to 13 % apart at 56
     const int tile_n = (long long)T * d.n_top > 52LL * d.n_expert ? 128 : 64;
     PI_TRY(pi_k_moe_sort(s->ids, T * d.n_top, d.n_expert, s->off, s->perm, s->inv, tile_n, s->tiles, s->n_tiles, st));
     pi_group_gemm g{};
