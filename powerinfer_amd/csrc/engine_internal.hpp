@@ -29,8 +29,9 @@ namespace pi {
 // How one call's prompt goes through wide chunks, decided once for the call (PI_ATTN_CHUNK may change between calls).  pieces: the model has Q4_0
 // matrices.  Their inputs are rounded to eight bits, where another order of sums moves single roundings and with them the logits by 1 to
 // 3 %: such prompts keep one order whatever their length, products of 512 tokens at a time and the attention by 16 tokens as far as it
-// holds the cells, and a chunk of up to 2048 tokens shares only the expansion of its matrices (210 us per 7B layer).  Four 7B layers, 1000 /
-// 1537 / 1900 tokens, ms: chunks of 512 expanded one by one 4.8 / - / -, so 4.3 / 6.3 / 8.0, products and attention of whole chunks - / 4.8 / 5.6.
+// holds the cells, and a chunk of up to 2048 tokens shares only the expansion of its matrices (210 us per 7B layer).  Four 7B layers, ms: 1000
+// tokens 4.3 (4.8 in chunks of 512, each with its own expansion), 1537 and 1900 tokens 6.3 and 8.0 (4.8 and 5.6 with products and attention of
+// whole chunks).
 struct WideRoute {
     bool scalar, pieces;      // attention one token per workgroup
     int most;                 // longest chunk: 512 or up to 2048
