@@ -381,9 +381,19 @@ PI_API int pi_k_transpose_f16(const void * in_f16, int rows, int cols, void * ou
  * matrix of the resident neurons and the matrix of the others (hot_words / hot_prefix as for pi_k_pred_upgate_q4_split).  The
  * products then differ from the CPU path's only by the fp16 rounding of the two factors. */
 PI_API int pi_k_norm_q8_round_f16(const float * x, int T, int cols, const pi_norm * norm, void * out_f16, void * out_plain_f16, pi_stream_t stream);
+/* the same with out / h in the operand layout, 16 tokens by 16 (buffers of ceil(T / 16) * 16 rows; operands on 16 bytes) */
+PI_API int pi_k_norm_q8_round_f16_ol(const float * x, int T, int cols, const pi_norm * norm, void * out_ol, void * out_plain_f16, pi_stream_t stream);
+PI_API int pi_k_ffn_h_q8_f16_ol(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_ol, pi_stream_t stream);
 PI_API int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream);
 PI_API int pi_k_dequant_q4_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                                void * out_f16, pi_stream_t stream);
+/* y = epi(W . x) straight from the blocks (transposed != 0: W stored as [cols][rows], the down projection): the values of expanding W with
+ * pi_k_dequant_q4_f16, with sums in one order at every T.  x in the operand layout, 16 tokens by 16 (ceil(T / 16) * 16 * cols
+ * values; those of tokens past T are read and not used).  cols % 256 == 0, rows % 64 == 0, rows * cols < 2^31 (what _supported says), W on 4
+ * bytes, the other operands on 16 (else PI_E_UNSUPPORTED).  tile = 0 lets the library choose; 100 * (rows / 16) + 10 * (token tiles a wave) + waves forces one. */
+PI_API int pi_k_gemm_q4_chunk_supported(int rows, int cols);
+PI_API int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, const void * x_ol, int T, int epilogue, const float * add1, const float * add2,
+                              float * y, int tile, pi_stream_t stream);
 /* the same transposed, out_f16[cols][rows]: rows % 8 == 0, cols % 256 == 0, operands 16-byte aligned (else PI_E_UNSUPPORTED) */
 PI_API int pi_k_dequant_q4_t_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                                void * out_f16, pi_stream_t stream);

@@ -434,6 +434,30 @@ int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int c
     return PI_OK;
 }
 
+// Q4_0 matrices that are whole on the device are multiplied straight from their blocks in chunks of up to 512 tokens; what they read is then in
+// the operand layout (out_ol).  Expanding first writes and reads the matrix in fp16 once more than that: us, expanded and multiplied by
+// the library / straight, 17, 130 and 512 tokens: 12288 x 4096 42 / 15, 51 / 21, 74 / 63; 4096 x 11008 transposed 46 / 25, 66 / 39,
+// 89 / 67; 13824 x 5120 54 / 19, 66 / 30, 99 / 86.  Longer chunks share one expansion among their pieces: four of 512 of 13824 x 5120
+// take 300 us so, and would take 344.
+bool direct_q4(pi_model * m, BatchState * b, int il, int kind) {
+    const Tensor & t = m->L(il, kind);
+    const bool ffn = kind == PI_T_FFN_UP || kind == PI_T_FFN_GATE || kind == PI_T_FFN_DOWN_T;
+    const int d = m->hp.n_embd, ff = m->hp.n_ff;
+    const int rows = kind == PI_T_WQKV ? d + 2 * m->gqa : kind == PI_T_FFN_UP || kind == PI_T_FFN_GATE ? ff : d, cols = kind == PI_T_FFN_DOWN_T ? ff : d;
+    return m->gemm_lib && b->n_seq <= kChunkMaxT && t.type == PI_TYPE_Q4_0 && !(ffn && m->L(il, PI_T_GPU_BUCKET).dev) && pi_k_gemm_q4_chunk_supported(rows, cols) && ((uintptr_t)t.dev & 3) == 0;
+}
+// the product with matrix `kind`, straight or the other way
+int chunk_product(pi_model * m, BatchState * b, int il, int kind, bool direct, int rows, int cols, const __half * xn, int epi, const float * add1, const float * add2, float * y) {
+    if (direct) return pi_k_gemm_q4_chunk(m->L(il, kind).dev, rows, cols, 0, xn, b->n_seq, epi, add1, add2, y, 0, m->stream);
+    const void * W = nullptr;
+    PI_TRY(chunk_weight(m, b, il, kind, rows, cols, &W));
+    return chunk_gemm(m, b, W, rows, cols, xn, epi, add1, add2, y, nullptr);
+}
+// what a matrix reads: x under its norm in the container of its type, and plain in fp16
+int chunk_input(int wtype, bool ol, const float * x, int T, int cols, const pi_norm * norm, void * out16, void * plain16, hipStream_t st) {
+    return ol ? pi_k_norm_q8_round_f16_ol(x, T, cols, norm, out16, plain16, st) : batch_input(wtype, x, T, cols, norm, out16, plain16, st);
+}
+
 // the down projection of a Q4_0 layer with its neurons contiguous, in w16t
 int chunk_down_q4(pi_model * m, BatchState * b, int il, int ff, int d) {
     const ChunkSource c = chunk_source(m, b, il, PI_T_FFN_DOWN_T);
@@ -463,45 +487,46 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     const size_t kv_off = (size_t)il * hp.n_head_kv * hp.n_ctx * hd;
     float * x = b->x;
     const void * W = nullptr;
+    const bool qkv_ol = direct_q4(m, b, il, PI_T_WQKV), wo_ol = direct_q4(m, b, il, PI_T_WO), down_ol = direct_q4(m, b, il, PI_T_FFN_DOWN_T);
+    const bool up_ol = direct_q4(m, b, il, PI_T_FFN_UP) && (falcon || direct_q4(m, b, il, PI_T_FFN_GATE));
     const pi_norm plain{0, 0.0f, nullptr, nullptr};
     pi_norm an;
     if (!falcon) an = mk_norm(1, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), nullptr);
     else if (m->L(il, PI_T_ATTN_NORM_2).dev) an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
-    PI_TRY(batch_input(wqkv.type, x, T, d, &an, b->xa16, falcon ? b->xp16 : nullptr, st));
-    PI_TRY(chunk_weight(m, b, il, PI_T_WQKV, d + 2 * gqa, d, &W));
-    PI_TRY(chunk_gemm(m, b, W, d + 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr));
+    PI_TRY(chunk_input(wqkv.type, qkv_ol, x, T, d, &an, b->xa16, falcon ? b->xp16 : nullptr, st));
+    PI_TRY(chunk_product(m, b, il, PI_T_WQKV, qkv_ol, d + 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv));
     PI_TRY(in_pieces(b, [&](int t0, int n) { return chunk_attention(m, b, t0, n, b->kv_hi - (T - t0 - n), kv_off); }));
-    if (wo.type == PI_TYPE_Q4_0) PI_TRY(pi_k_norm_q8_round_f16(b->att, T, d, &plain, b->att16, nullptr, st));
-    PI_TRY(chunk_weight(m, b, il, PI_T_WO, d, d, &W));
+    if (wo.type == PI_TYPE_Q4_0) PI_TRY(chunk_input(wo.type, wo_ol, b->att, T, d, &plain, b->att16, nullptr, st));
     pi_norm fn;
     const __half * ffn_x = b->xf16;
     if (!falcon) {
-        PI_TRY(chunk_gemm(m, b, W, d, d, b->att16, PI_EPI_ADD, x, nullptr, b->ffn_inp, nullptr));
+        PI_TRY(chunk_product(m, b, il, PI_T_WO, wo_ol, d, d, b->att16, PI_EPI_ADD, x, nullptr, b->ffn_inp));
         fn = mk_norm(1, hp.norm_eps, m->L(il, PI_T_FFN_NORM), nullptr);
-        PI_TRY(batch_input(up.type, b->ffn_inp, T, d, &fn, b->xf16, b->xp16, st));
+        PI_TRY(chunk_input(up.type, up_ol, b->ffn_inp, T, d, &fn, b->xf16, b->xp16, st));
     } else {
-        PI_TRY(chunk_gemm(m, b, W, d, d, b->att16, PI_EPI_NONE, nullptr, nullptr, b->attn_out, nullptr));
+        PI_TRY(chunk_product(m, b, il, PI_T_WO, wo_ol, d, d, b->att16, PI_EPI_NONE, nullptr, nullptr, b->attn_out));
         fn = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         // the FFN branch reads the layer input under its own norm; with a single norm it shares the attention branch's rows unless
-        // the two matrices want different containers (fp16 against Q8_0 blocks)
-        if (m->L(il, PI_T_ATTN_NORM_2).dev || up.type != wqkv.type) PI_TRY(batch_input(up.type, x, T, d, &fn, b->xf16, nullptr, st));
+        // the two matrices want different containers (fp16 against Q8_0 blocks) or layouts
+        if (m->L(il, PI_T_ATTN_NORM_2).dev || up.type != wqkv.type || up_ol != qkv_ol) PI_TRY(chunk_input(up.type, up_ol, x, T, d, &fn, b->xf16, nullptr, st));
         else ffn_x = b->xa16;
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
     PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
     const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m));
-    if (!one_kernel) {
-        PI_TRY(chunk_weight(m, b, il, PI_T_FFN_UP, ff, d, &W));
-        PI_TRY(chunk_gemm(m, b, W, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out, nullptr));
-    }
-    if (!falcon && !one_kernel) {
-        PI_TRY(chunk_weight(m, b, il, PI_T_FFN_GATE, ff, d, &W));
-        PI_TRY(chunk_gemm(m, b, W, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out, nullptr));
-    }
+    if (!one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_UP, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out));
+    if (!falcon && !one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_GATE, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out));
     if (one_kernel) PI_TRY(pi_k_ffn_wide_f16(up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, b->pred_logits, hp.sparse_threshold, b->h16, st));
+    else if (down_ol) PI_TRY(pi_k_ffn_h_q8_f16_ol(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
+    if (down_ol) {
+        const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
+        PI_TRY(pi_k_gemm_q4_chunk(down.dev, d, ff, 1, b->h16, T, falcon ? PI_EPI_ADD2 : PI_EPI_ADD, a1, a2, b->x2, 0, st));
+        std::swap(b->x, b->x2);
+        return PI_OK;
+    }
     const void * Wd = m->down_rows[il];
     if (!Wd && down.type == PI_TYPE_Q4_0) {
         const int rc = chunk_down_q4(m, b, il, ff, d);

@@ -18,22 +18,31 @@ namespace {
 
 // the value a Q8_0 block keeps of v: q * fp16(amax / 127) with q = rint(v * 127 / amax) and amax over the 32 consecutive elements
 // the 32 lanes of a half-wave hold (quantize_row_q8_0, x86 path, ggml-quants.c:702-760), rounded to fp16 for a mat-mul input
+template <int N> __device__ __forceinline__ void q8_block_values(float (&v)[N], float amax) {       // values of a block whose largest magnitude is amax
+    const float d = pi_round_f16(pi_div(amax, 127.0f)), id = (amax != 0.0f) ? pi_div(127.0f, amax) : 0.0f;
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = __fmul_rn((float)(int)rintf(__fmul_rn(v[q], id)), d);
+}
 __device__ __forceinline__ float q8_block_value(float v) {
     float amax = fabsf(v);
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, PI_WAVE));
-    const float d = pi_round_f16(pi_div(amax, 127.0f)), id = (amax != 0.0f) ? pi_div(127.0f, amax) : 0.0f;
-    return __fmul_rn((float)(int)rintf(__fmul_rn(v, id)), d);
+    float one[1] = {v};
+    q8_block_values(one, amax);
+    return one[0];
 }
+
+// Token t, column i of tokens in the operand layout, 16 by 16
+__device__ __forceinline__ size_t ol_index_of(int t, int i, int cols) { return (size_t)(t >> 4) * 16 * cols + pi_ol_index(t & 15, i); }
 
 // q8 != 0 (cols % 32 == 0, cols <= 8192): the normalised row goes through Q8_0 blocks of 32 before the fp16 rounding, which is what
 // a Q4_0 mat-mul of the CPU path multiplies with (ggml_vec_dot_q4_0_q8_0, ggml-quants.c:2512-2650)
-// ol != 0: both outputs in the operand layout of the 16-token mat-muls (pi_ol_index) instead of [token][cols].
+// ol bit 0: out in the operand layout of the 16-token mat-muls, 16 tokens by 16 (pi_ol_index), instead of [token][cols]; bit 1: out_plain
 __global__ __launch_bounds__(1024) void norm_round_f16_kernel(const float * __restrict__ x, int cols, NormArgs na, __half * __restrict__ out,
                                                               __half * __restrict__ out_plain, int q8, int ol) {
     __shared__ double red[16];
     const float * xt = x + (size_t)blockIdx.x * cols;
-    auto at = [&](int i) -> size_t { return ol ? pi_ol_index(blockIdx.x, i) : (size_t)blockIdx.x * cols + i; };
+    auto at = [&](int i, int bit) -> size_t { return ol & bit ? ol_index_of(blockIdx.x, i, cols) : (size_t)blockIdx.x * cols + i; };
     float mean = 0.0f, scale = 1.0f;
     if (cols <= 8 * 1024) {
         // one memory round trip: the row, the norm weights and the bias are requested together and stay in registers
@@ -67,14 +76,14 @@ __global__ __launch_bounds__(1024) void norm_round_f16_kernel(const float * __re
         for (int k = 0; k < 8; ++k) {
             const int i = threadIdx.x + k * 1024;
             float v = xv[k];
-            if (i < cols && out_plain) out_plain[at(i)] = __float2half_rn(v);
+            if (i < cols && out_plain) out_plain[at(i, 2)] = __float2half_rn(v);
             if (na.kind != 0) {
                 v = __fmul_rn(na.kind == 2 ? __fsub_rn(v, mean) : v, scale);
                 if (na.w) v = __fmul_rn(v, wv[k]);
                 if (na.b) v = __fadd_rn(v, bv[k]);
             }
             if (q8) v = q8_block_value(i < cols ? v : 0.0f);          // every lane takes part in the block's maximum
-            if (i < cols) out[at(i)] = __float2half_rn(v);
+            if (i < cols) out[at(i, 1)] = __float2half_rn(v);
         }
         return;
     }
@@ -95,20 +104,23 @@ __global__ __launch_bounds__(1024) void norm_round_f16_kernel(const float * __re
     }
     for (int i = threadIdx.x; i < cols; i += blockDim.x) {
         float v = xt[i];
-        if (out_plain) out_plain[at(i)] = __float2half_rn(v);
+        if (out_plain) out_plain[at(i, 2)] = __float2half_rn(v);
         if (na.kind != 0) {
             v = __fmul_rn(na.kind == 2 ? __fsub_rn(v, mean) : v, scale);
             if (na.w) v = __fmul_rn(v, na.w[i]);
             if (na.b) v = __fadd_rn(v, na.b[i]);
         }
-        out[at(i)] = __float2half_rn(v);
+        out[at(i, 1)] = __float2half_rn(v);
     }
 }
 
-// The same with 256 threads a row and 16-byte accesses (cols % 4 == 0, cols <= 8192, 16-byte rows, no Q8_0 blocks): 16 waves a row leave two rows
+// The same with 256 threads a row and 16-byte accesses (cols % 4 == 0, cols <= 8192, 16-byte rows): 16 waves a row leave two rows
 // on a CU, each with its own memory trip and barriers.  It is the faster one everywhere, by the most where rows are many: 2046 tokens of
-// 512 / 4096 / 8192 columns 17.9 / 20.0 / 26.6 -> 5.1 / 10.6 / 19.2 us (4096: 50 MB), 16 tokens of 4096 4.7 -> 4.2 us.
-__global__ __launch_bounds__(256) void norm_round_rows_kernel(const float * __restrict__ x, int cols, NormArgs na, __half * __restrict__ out, __half * __restrict__ out_plain, int ol) {
+// 512 / 4096 / 8192 columns 17.9 / 20.0 / 26.6 -> 5.1 / 10.6 / 19.2 us (4096: 50 MB), 16 tokens of 4096 4.7 -> 4.2 us.  Q8: blocks of 32
+// are eight lanes, and the two divisions of a block are taken once for four values (130 tokens of 4096: 8.1 -> 5.3 us).
+// ol, plain_ol: which of the outputs are in the operand layout.
+template <bool Q8>
+__global__ __launch_bounds__(256) void norm_round_rows_kernel(const float * __restrict__ x, int cols, NormArgs na, __half * __restrict__ out, __half * __restrict__ out_plain, int ol, int plain_ol) {
     __shared__ double red[4];
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     constexpr int N = 8;
@@ -151,8 +163,8 @@ __global__ __launch_bounds__(256) void norm_round_rows_kernel(const float * __re
         const int i = 4 * tid + k * 1024;
         if (i >= cols) break;
         float v[4] = {xv[k].x, xv[k].y, xv[k].z, xv[k].w};
-        const size_t at = ol ? pi_ol_index(blockIdx.x, i) : (size_t)blockIdx.x * cols + i;           // (a piece of eight columns is contiguous in both)
-        if (out_plain) *reinterpret_cast<h4 *>(out_plain + at) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        const size_t at_row = (size_t)blockIdx.x * cols + i, at_ol = ol_index_of(blockIdx.x, i, cols);        // (a piece of eight columns is contiguous in both)
+        if (out_plain) *reinterpret_cast<h4 *>(out_plain + (plain_ol ? at_ol : at_row)) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
         if (na.kind != 0) {
             const float w[4] = {wv[k].x, wv[k].y, wv[k].z, wv[k].w}, b[4] = {bv[k].x, bv[k].y, bv[k].z, bv[k].w};
 #pragma unroll
@@ -162,14 +174,27 @@ __global__ __launch_bounds__(256) void norm_round_rows_kernel(const float * __re
                 if (has_b) v[q] = __fadd_rn(v[q], b[q]);
             }
         }
-        *reinterpret_cast<h4 *>(out + at) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
+        if constexpr (Q8) {                            // (cols % 32 == 0: the eight lanes of a block go on together)
+            float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+            amax = pi_dpp_max<PI_DPP_HALF_MIRROR, 0xF>(pi_dpp_max<PI_DPP_XOR2, 0xF>(pi_dpp_max<PI_DPP_XOR1, 0xF>(amax)));
+            q8_block_values(v, amax);
+        }
+        *reinterpret_cast<h4 *>(out + (ol ? at_ol : at_row)) = h4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
     }
 }
 
+bool norm_rows_wide(const float * x, int cols, const NormArgs & na, const void * out, const void * out_plain) {
+    return cols % 4 == 0 && cols <= 8192 && (((uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b | (uintptr_t)out | (uintptr_t)out_plain) & 15) == 0;
+}
+void launch_norm_q8(const float * x, int T, int cols, NormArgs na, void * out, void * out_plain, int ol, hipStream_t st) {
+    if (norm_rows_wide(x, cols, na, out, out_plain))
+        hipLaunchKernelGGL(norm_round_rows_kernel<true>, dim3(T), dim3(256), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, ol, 0);
+    else hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, 1, ol);
+}
 void launch_norm_round(const float * x, int T, int cols, NormArgs na, void * out, void * out_plain, int ol, hipStream_t st) {
-    if (cols % 4 == 0 && cols <= 8192 && (((uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b | (uintptr_t)out | (uintptr_t)out_plain) & 15) == 0)
-        hipLaunchKernelGGL(norm_round_rows_kernel, dim3(T), dim3(256), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, ol);
-    else hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, 0, ol);
+    if (norm_rows_wide(x, cols, na, out, out_plain))
+        hipLaunchKernelGGL(norm_round_rows_kernel<false>, dim3(T), dim3(256), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, ol, ol);
+    else hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, st, x, cols, na, (__half *)out, (__half *)out_plain, 0, ol ? 3 : 0);
 }
 
 // y[t][row] = epi( W[row] . xn[t] ), t < T <= 16.  A workgroup owns 16*RT rows; its four waves split the columns in
@@ -427,6 +452,33 @@ __global__ void ffn_h_f16_kernel(const float * __restrict__ up, const float * __
         if (!(logits[i] < thr)) h = gate ? __fmul_rn(fmaxf(gate[i], 0.0f), up[i]) : fmaxf(up[i], 0.0f);
         if (q8) h = q8_block_value(h);
         h16[i] = __float2half_rn(h);
+    }
+}
+// The Q8_0 form into the operand layout, eight neurons a thread: pieces of 16 bytes (130 tokens of 11008: 8.3 us, as by rows)
+__global__ __launch_bounds__(256) void ffn_h_q8_ol_kernel(const float * __restrict__ up, const float * __restrict__ gate, const float * __restrict__ logits, float thr,
+                                                       int T, int ff, __half * __restrict__ h16) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    const size_t n = (size_t)T * (ff / 8);
+    // (n % 4 == 0, and a block's four threads go on together)
+    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (size_t)gridDim.x * blockDim.x) {
+        float4 u[2], g[2], l[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            u[k] = reinterpret_cast<const float4 *>(up)[2 * j + k]; l[k] = reinterpret_cast<const float4 *>(logits)[2 * j + k];
+            g[k] = gate ? reinterpret_cast<const float4 *>(gate)[2 * j + k] : u[k];
+        }
+        float v[8], amax = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float uu = (&u[e >> 2].x)[e & 3], gg = (&g[e >> 2].x)[e & 3], ll = (&l[e >> 2].x)[e & 3];
+            v[e] = ll < thr ? 0.0f : gate ? __fmul_rn(fmaxf(gg, 0.0f), uu) : fmaxf(uu, 0.0f);
+            amax = fmaxf(amax, fabsf(v[e]));
+        }
+        amax = pi_dpp_max<PI_DPP_XOR2, 0xF>(pi_dpp_max<PI_DPP_XOR1, 0xF>(amax));
+        q8_block_values(v, amax);
+        const int t = (int)(j / (ff / 8)), c = (int)(j % (ff / 8)) * 8;
+        *reinterpret_cast<h8 *>(h16 + ol_index_of(t, c, ff)) =
+            h8{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3], (_Float16)v[4], (_Float16)v[5], (_Float16)v[6], (_Float16)v[7]};
     }
 }
 // The same straight from the matrices, in the large tiles of gemm_wide: a tile holds 64 rows of up, the 64 rows of gate of the same neurons and
@@ -1160,8 +1212,14 @@ int pi_k_norm_round_f16_ol(const float * x, int T, int cols, const pi_norm * nor
 
 int pi_k_norm_q8_round_f16(const float * x, int T, int cols, const pi_norm * norm, void * out_f16, void * out_plain_f16, pi_stream_t stream) {
     if (!x || !out_f16 || T <= 0 || cols <= 0 || cols % 32 || cols > 8 * 1024) return pi::fail(PI_E_ARG, "pi_k_norm_q8_round_f16: cols must be a multiple of 32, at most 8192");
-    hipLaunchKernelGGL(norm_round_f16_kernel, dim3(T), dim3(1024), 0, (hipStream_t)stream, x, cols, to_norm(norm), (__half *)out_f16, (__half *)out_plain_f16, 1, 0);
+    launch_norm_q8(x, T, cols, to_norm(norm), out_f16, out_plain_f16, 0, (hipStream_t)stream);
     return pi::check_launch("pi_k_norm_q8_round_f16");
+}
+
+int pi_k_norm_q8_round_f16_ol(const float * x, int T, int cols, const pi_norm * norm, void * out_ol, void * out_plain_f16, pi_stream_t stream) {
+    if (!x || !out_ol || T <= 0 || cols <= 0 || cols % 32 || cols > 8 * 1024) return pi::fail(PI_E_ARG, "pi_k_norm_q8_round_f16_ol: cols must be a multiple of 32, at most 8192");
+    launch_norm_q8(x, T, cols, to_norm(norm), out_ol, out_plain_f16, 1, (hipStream_t)stream);
+    return pi::check_launch("pi_k_norm_q8_round_f16_ol");
 }
 
 }  // extern "C"
@@ -1333,6 +1391,14 @@ int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits
     if (!up || !logits || !h_f16 || T <= 0 || ff <= 0 || ff % 64) return pi::fail(PI_E_ARG, "pi_k_ffn_h_q8_f16: n_ff must be a multiple of 64");
     hipLaunchKernelGGL(ffn_h_f16_kernel, dim3(1024), dim3(256), 0, (hipStream_t)stream, up, gate, logits, threshold, (size_t)T * ff, (__half *)h_f16, 1);
     return pi::check_launch("pi_k_ffn_h_q8_f16");
+}
+
+int pi_k_ffn_h_q8_f16_ol(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_ol, pi_stream_t stream) {
+    if (!up || !logits || !h_ol || T <= 0 || ff <= 0 || ff % 64) return pi::fail(PI_E_ARG, "pi_k_ffn_h_q8_f16_ol: n_ff must be a multiple of 64");
+    if ((((uintptr_t)up | (uintptr_t)gate | (uintptr_t)logits | (uintptr_t)h_ol) & 15) != 0) return pi::fail(PI_E_UNSUPPORTED, "pi_k_ffn_h_q8_f16_ol: operands must be 16-byte aligned");
+    const size_t pieces = (size_t)T * (ff / 8);
+    hipLaunchKernelGGL(ffn_h_q8_ol_kernel, dim3((unsigned)std::min<size_t>((pieces + 255) / 256, 8192)), dim3(256), 0, (hipStream_t)stream, up, gate, logits, threshold, T, ff, (__half *)h_ol);
+    return pi::check_launch("pi_k_ffn_h_q8_f16_ol");
 }
 
 // W[rows][cols] in Q4_0 blocks -> fp16 (value (q - 8) * d, dequantize_row_q4_0, ggml-quants.c:1074-1092), one thread per block.  With hot
