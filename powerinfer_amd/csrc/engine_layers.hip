@@ -162,6 +162,7 @@ struct LayerState {
     float * scratch = nullptr;                         // partial sums of a split attention
     float * logits = nullptr; void * h_head = nullptr; int32_t * d_next = nullptr;
     int32_t * h_in = nullptr, * d_in = nullptr; size_t in_cap = 0;       // a pass's integers: pinned host side and device side
+    bool in_flight = false;                                              // a copy from the host side may still run
     float * streams = nullptr; size_t streams_cap = 0; int streams_T = 0;
     // lockstep decoding and the greedy loop
     int n_seq = 0;
@@ -177,6 +178,13 @@ namespace {
 __global__ void cells_append_kernel(const int32_t * __restrict__ app, int n, int32_t * __restrict__ lists, size_t ld) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) lists[(size_t)app[3 * i] * ld + app[3 * i + 1]] = app[3 * i + 2];
+}
+
+// the same for the few cells of a step, which then need no copy
+struct AppendArgs { static constexpr size_t kMost = 3 * 64; int32_t v[kMost]; };
+__global__ void cells_append_args_kernel(AppendArgs app, int n, int32_t * __restrict__ lists, size_t ld) {
+    const int i = threadIdx.x;
+    if (i < n) lists[(size_t)app.v[3 * i] * ld + app.v[3 * i + 1]] = app.v[3 * i + 2];
 }
 
 bool bf16_mode(const LayerState * s) { return s->opts.compute == PI_TYPE_BF16; }
@@ -1324,13 +1332,31 @@ template <typename F> bool keeps_whole(LayerState * s, F && edit) {
     return (lost & left) == 0;
 }
 
+// the pinned side of a pass's integers may be written
+int inputs_free(pi_model * m) {
+    if (m->lay->in_flight) PI_HIP_TRY(hipStreamSynchronize(m->stream));
+    m->lay->in_flight = false;
+    return PI_OK;
+}
+int copy_inputs(pi_model * m, size_t n) {
+    m->lay->in_flight = true;
+    PI_HIP_TRY(hipMemcpyAsync(m->lay->d_in, m->lay->h_in, 4 * n, hipMemcpyHostToDevice, m->stream));
+    return PI_OK;
+}
+
 int upload_appends(pi_model * m, const std::vector<int32_t> & app) {
     if (app.empty()) return PI_OK;
     LayerState * s = m->lay;
+    if (app.size() <= AppendArgs::kMost) {                         // a step's cells travel as arguments: no copy, and nothing to wait for
+        AppendArgs args;
+        memcpy(args.v, app.data(), app.size() * 4);
+        hipLaunchKernelGGL(cells_append_args_kernel, dim3(1), dim3(64), 0, m->stream, args, (int)(app.size() / 3), s->lists, (size_t)s->kv.n);
+        return pi::check_launch("cells_append");
+    }
     PI_TRY(ensure_inputs(m, app.size()));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));                   // the staging buffer's last copy is done
+    PI_TRY(inputs_free(m));
     memcpy(s->h_in, app.data(), app.size() * 4);
-    PI_HIP_TRY(hipMemcpyAsync(s->d_in, s->h_in, app.size() * 4, hipMemcpyHostToDevice, m->stream));
+    PI_TRY(copy_inputs(m, app.size()));
     const int n = (int)(app.size() / 3);
     hipLaunchKernelGGL(cells_append_kernel, dim3((n + 255) / 256), dim3(256), 0, m->stream, s->d_in, n, s->lists, (size_t)s->kv.n);
     return pi::check_launch("cells_append");
@@ -1629,14 +1655,14 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         items.insert(items.end(), others.begin(), others.end());
         const size_t n_in = (size_t)8 * T + items.size() + rows.size();
         PI_TRY(ensure_inputs(m, n_in));
-        PI_HIP_TRY(hipStreamSynchronize(m->stream));
+        PI_TRY(inputs_free(m));
         int32_t * h = s->h_in;
         memcpy(h, tokens + t0, 4 * (size_t)T); memcpy(h + T, positions + t0, 4 * (size_t)T); memcpy(h + 2 * T, cells.data() + t0, 4 * (size_t)T);
         memcpy(h + 3 * T, vis.data() + t0, 4 * (size_t)T); memcpy(h + 4 * T, seq.data() + t0, 4 * (size_t)T);
         memcpy(h + 5 * T, prev.data() + t0, 4 * (size_t)T);      // (the items behind start on a multiple of 16 bytes)
         if (!items.empty()) memcpy(h + 8 * T, items.data(), 4 * items.size());
         if (!rows.empty()) memcpy(h + 8 * T + items.size(), rows.data(), 4 * rows.size());
-        PI_HIP_TRY(hipMemcpyAsync(s->d_in, h, 4 * n_in, hipMemcpyHostToDevice, m->stream));
+        PI_TRY(copy_inputs(m, n_in));
         in.tokens = s->d_in; in.pos = s->d_in + T; in.cell = s->d_in + 2 * T; in.n_vis = s->d_in + 3 * T; in.seq = s->d_in + 4 * T; in.prev = s->d_in + 5 * T;
         in.conv = s->d_in + 8 * T + at_conv;
         in.lin = s->d_in + 8 * T + at_lin; in.lin_long = in.lin + 4 * in.n_lin; in.lin_first = in.lin_long + 4 * in.n_lin_long; in.lin_chunks = in.lin_first + in.n_lin_long;
@@ -1691,6 +1717,7 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         }
     }
     PI_HIP_TRY(hipStreamSynchronize(m->stream));
+    s->in_flight = false;
     return PI_OK;
 }
 
