@@ -1308,7 +1308,20 @@ namespace {
 constexpr size_t kChunkMfmaLds = 156 * 1024;
 size_t chunk_mfma_lds(int hd, int n_kv_max) { return sizeof(float) * 16 * (size_t)(((n_kv_max + 31) & ~31) + 4) + (size_t)kWavesPerBlock * hd * kAcVtStride * 2; }
 
-[[nodiscard]] int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
+template <int HD, int U, bool WHOLE>
+int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_cache, int n_head, int n_head_kv, int n_ctx, const int32_t * pos, int T, int n_kv_max, float * out,
+                      int out_stride, void * out_f16, hipStream_t st) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_kernel<HD, U, WHOLE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
+    if (raised != hipSuccess) return pi::hip_fail(raised, "attn_chunk_rows: LDS size");
+    hipLaunchKernelGGL((attn_chunk_rows_kernel<HD, U, WHOLE>), dim3(n_head, (T + 64 * U - 1) / (64 * U)), dim3(kBlock), rows_lds<HD>(), st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
+                       n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, n_head * HD, out_stride, (__half *)out_f16);
+    return pi::check_launch("attn_chunk_rows");
+}
+}  // namespace
+
+namespace pi {
+// keys and values of T tokens to their cells, rotated queries to q_rot; n_head 0: rows of k and v alone (no q_rot)
+int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
                   float * q_rot, void * k_cache, void * v_cache, hipStream_t st) {
     // 16 tokens and fewer: a workgroup per head and token (16 tokens, 32 heads of 128, attention included: 11.8 against 12.3 us); a chunk's angles
     // are worth forming once a token from there on.  A workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
@@ -1325,19 +1338,6 @@ size_t chunk_mfma_lds(int hd, int n_kv_max) { return sizeof(float) * 16 * (size_
                        (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
     return pi::check_launch("rope_kv_chunk");
 }
-
-template <int HD, int U, bool WHOLE>
-int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_cache, int n_head, int n_head_kv, int n_ctx, const int32_t * pos, int T, int n_kv_max, float * out,
-                      int out_stride, void * out_f16, hipStream_t st) {
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_kernel<HD, U, WHOLE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
-    if (raised != hipSuccess) return pi::hip_fail(raised, "attn_chunk_rows: LDS size");
-    hipLaunchKernelGGL((attn_chunk_rows_kernel<HD, U, WHOLE>), dim3(n_head, (T + 64 * U - 1) / (64 * U)), dim3(kBlock), rows_lds<HD>(), st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
-                       n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, n_head * HD, out_stride, (__half *)out_f16);
-    return pi::check_launch("attn_chunk_rows");
-}
-}  // namespace
-
-namespace pi {
 bool attn_chunk_by_16(int hd, int n_kv_max) { return (hd == 64 || hd == 128) && chunk_mfma_lds(hd, n_kv_max) <= kChunkMfmaLds; }
 }  // namespace pi
 
@@ -1518,7 +1518,7 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad head geometry or mode");
     hipStream_t st = (hipStream_t)stream;
     // all K/V rows of the chunk are in the cache before any token of the chunk attends
-    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     if (rc != PI_OK) return rc;
     // 16 tokens per workgroup on the matrix cores where the head size and the context fit (scores of 16 tokens in LDS)
     const char * own = getenv("PI_ATTN_CHUNK");
@@ -1561,7 +1561,7 @@ int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, i
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk_rows: rows of whole quads, buffers on 16 bytes (out_f16: 8)");
     if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;
     hipStream_t st = (hipStream_t)stream;
-    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     if (rc != PI_OK) return rc;
     // 128 tokens a workgroup where that still leaves two for every compute unit
     const bool two = (long long)n_head * ((T + 127) / 128) >= 2 * pi::compute_units();
@@ -1589,7 +1589,7 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (mode != 0 && mode != 2) || hd % 2 || hd / 2 > 1024 || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_chunk_long: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
     hipStream_t st = (hipStream_t)stream;
-    const int rc = rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
+    const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     if (rc != PI_OK) return rc;
     const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;

@@ -46,6 +46,8 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream);
 // whether pi_k_attn_chunk takes the tokens of a chunk against n_kv_max cells 16 at a time on the matrix cores
 bool attn_chunk_by_16(int hd, int n_kv_max);
+int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
+                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st);
 // the embedding row of a token that the host names; also writes the token loop's state (token, position, step counter 0)
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
 
