@@ -124,7 +124,10 @@ struct Step {
     const int32_t *lin = nullptr, *lin_long = nullptr, *lin_first = nullptr, *lin_chunks = nullptr;
     int n_lin = 0, n_lin_long = 0, n_lin_chunks = 0;
     const int32_t * conv = nullptr; int n_conv = 0;    // items of the convolutions
+    // the tokens whose logits are wanted, in this order (-1: not said, every token's stream is)
+    const int32_t * rows = nullptr; int n_rows = -1;
 };
+constexpr int kTailRows = 16;            // rows the last layer goes on with: what the kernels of a step hold
 
 }  // namespace
 
@@ -156,6 +159,9 @@ struct LayerState {
     void *lin_q = nullptr, *lin_k = nullptr, *lin_v = nullptr, *lin_states = nullptr;
     void *h_a = nullptr, *h_b = nullptr, *q_un = nullptr, *q_lat = nullptr, *o_lat = nullptr, *att = nullptr, *act = nullptr, *y_exp = nullptr;
     int32_t *ids = nullptr, *perm = nullptr, *inv = nullptr, *off = nullptr, *tiles = nullptr, *n_tiles = nullptr;
+    // rows of x, x2, att, ids, wts that the last layer goes on with, and of a gate; in their places (tail) behind that layer's attention
+    float *x_tail = nullptr, *x2_tail = nullptr, *wts_tail = nullptr, *gate_tail = nullptr; void * att_tail = nullptr; int32_t * ids_tail = nullptr;
+    bool tail = false;
     float *heads = nullptr, *v_first = nullptr, *stats = nullptr;        // the heads' results ahead of their mixture, the first values of the step's tokens
     std::vector<float *> cs;                           // per rotation [cap][dims / 2] (cos, sin)
     bf16_t * expanded = nullptr; size_t expanded_cap = 0;      // keys and values of a long run's cells
@@ -185,6 +191,19 @@ struct AppendArgs { static constexpr size_t kMost = 3 * 64; int32_t v[kMost]; };
 __global__ void cells_append_args_kernel(AppendArgs app, int n, int32_t * __restrict__ lists, size_t ld) {
     const int i = threadIdx.x;
     if (i < n) lists[(size_t)app.v[3 * i] * ld + app.v[3 * i + 1]] = app.v[3 * i + 2];
+}
+
+// rows[r] of up to five arrays, in whole 4-byte words: 16 bytes a thread where rows allow it
+struct TailCopies { int n = 0; const unsigned char * src[5]; size_t ld[5]; int bytes[5]; unsigned char * dst[5]; };
+__global__ __launch_bounds__(256) void tail_rows_kernel(const int32_t * __restrict__ rows, TailCopies c) {
+    const int r = blockIdx.x, k = blockIdx.y, n = c.bytes[k];
+    const unsigned char * src = c.src[k] + (size_t)rows[r] * c.ld[k];
+    unsigned char * dst = c.dst[k] + (size_t)r * n;
+    if (((uintptr_t)src | (uintptr_t)dst | (uintptr_t)n) % 16 == 0) {
+        for (int i = threadIdx.x * 16; i < n; i += 256 * 16) *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+    } else {
+        for (int i = threadIdx.x * 4; i < n; i += 256 * 4) *reinterpret_cast<uint32_t *>(dst + i) = *reinterpret_cast<const uint32_t *>(src + i);
+    }
 }
 
 bool bf16_mode(const LayerState * s) { return s->opts.compute == PI_TYPE_BF16; }
@@ -636,6 +655,8 @@ int ensure_capacity(pi_model * m, int T) {
         carve(s->q_un, n * qu * es); carve(s->q_lat, n * ql * es); carve(s->o_lat, n * ol * es); carve(s->att, n * at * es);
         carve(s->rl, n * E * 4); carve(s->wts, n * top * 4); carve(s->ids, n * top * 4); carve(s->perm, n * top * 4); carve(s->inv, n * top * 4);
         carve(s->off, (E + 1) * 4); carve(s->act, n * ff * es); carve(s->y_exp, n * top * D * es);
+        carve(s->x_tail, kTailRows * D * 4); carve(s->x2_tail, kTailRows * D * 4); carve(s->gate_tail, kTailRows * D * 4); carve(s->att_tail, kTailRows * at * es);
+        carve(s->ids_tail, kTailRows * top * 4); carve(s->wts_tail, kTailRows * top * 4);
         carve(s->tiles, (n * top / 64 + E + 1) * 8); carve(s->n_tiles, 4);
         carve(s->x0, s->opts.loop_times > 0 ? n * D * 4 : 0);
         carve(s->lin_o, n * lo * 4); carve(s->lin_q, n * lq * 2); carve(s->lin_k, n * lq * 2); carve(s->lin_v, n * lv * 2); carve(s->lin_states, ls);
@@ -771,6 +792,38 @@ int attend_expanded(pi_model * m, const Layer & L, const Layer & src, const Step
     return pi_k_latent_attn_expanded(&a, st);
 }
 
+// The last layer of a pass: nobody reads more of it than its cells and states and the wanted tokens' stream.  Behind its attention a long pass goes on with
+// those tokens alone, as a step of so few does (four layers, 4096 wide, one token wanted: 2048 tokens with 64 experts of 1408 3.75 -> 3.22 ms, 2460 tokens of
+// gated recurrences 5.69 -> 5.01).
+bool tail_of(pi_model * m, const Layer & L, const LayerRun & r, const Step & in, const float * keep) {
+    LayerState * s = m->lay;
+    return bf16_mode(s) && &r == &s->order.back() && !keep && in.T > kTailRows && in.n_rows >= 0 && in.n_rows <= kTailRows &&
+           pi_k_layer_step_supported(std::max(in.n_rows, 1), L.moe() ? L.d.n_expert : 0, L.moe() ? L.d.n_top : 0);
+}
+// the tail's rows and the whole pass's change places
+void swap_tail(LayerState * s) {
+    std::swap(s->x, s->x_tail); std::swap(s->x2, s->x2_tail); std::swap(s->att, s->att_tail); std::swap(s->ids, s->ids_tail); std::swap(s->wts, s->wts_tail);
+    s->tail = !s->tail;
+}
+// ld: columns of a row of att; routed: the experts are chosen already; gate (optional): n_embd values of the rows of s->z from there on
+int take_tail(pi_model * m, const Layer & L, const Step & in, int ld, bool routed, const float * gate) {
+    LayerState * s = m->lay;
+    const int D = m->hp.n_embd;
+    TailCopies c;
+    const auto add = [&](const void * src, size_t ld_bytes, int bytes, void * dst) {
+        c.src[c.n] = (const unsigned char *)src; c.ld[c.n] = ld_bytes; c.bytes[c.n] = bytes; c.dst[c.n] = (unsigned char *)dst;
+        ++c.n;
+    };
+    add(s->x, 4 * (size_t)D, 4 * D, s->x_tail);
+    add(s->att, 2 * (size_t)ld, 2 * ld, s->att_tail);
+    if (routed) { add(s->ids, 4 * (size_t)L.d.n_top, 4 * L.d.n_top, s->ids_tail); add(s->wts, 4 * (size_t)L.d.n_top, 4 * L.d.n_top, s->wts_tail); }
+    if (gate) add(gate, 4 * (size_t)L.z_rows, 4 * D, s->gate_tail);
+    hipLaunchKernelGGL(tail_rows_kernel, dim3(in.n_rows, c.n), dim3(256), 0, m->stream, in.rows, c);
+    PI_TRY(pi::check_launch("tail_rows"));
+    swap_tail(s);
+    return PI_OK;
+}
+
 int mix_latent(pi_model * m, Layer & L, const Step & in) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
@@ -782,7 +835,7 @@ int mix_latent(pi_model * m, Layer & L, const Step & in) {
     PI_TRY(pi_k_latent_prep(type, &p, st));
     if (in.work[L.hc].n > 0) PI_TRY(attend_latent(m, L, src, in));
     if (bf16_mode(s)) for (const Step::Run & r : in.runs[L.hc]) PI_TRY(attend_expanded(m, L, src, in, r));
-    return dense(m, L.wo, m->hp.n_embd, L.hv_ld, s->att, T, s->mix);
+    return PI_OK;
 }
 
 // the experts of the chosen pairs (s->ids): relu^2 or, with a gate, clamped GLU in between; s->y_exp holds a row per pair, in expert order
@@ -817,6 +870,28 @@ int ffn_moe(pi_model * m, Layer & L, const Step & in) {
     PI_TRY(dense(m, L.router, d.n_expert, s->d_ld, s->h_b, in.T, s->rl));
     PI_TRY(pi_k_route(s->rl, in.T, d.n_expert, d.n_top, d.n_group, d.n_group_keep, L.bias, s->ids, s->wts, m->stream));
     return experts(m, L, s->h_b, in);
+}
+
+// the last layer behind its attention, for the wanted tokens
+int latent_tail(pi_model * m, Layer & L, const Step & in) {
+    LayerState * s = m->lay;
+    const pi_layer_desc & d = L.d;
+    const int D = m->hp.n_embd, R = in.n_rows;
+    hipStream_t st = m->stream;
+    if (R == 0) return PI_OK;
+    PI_TRY(take_tail(m, L, in, L.hv_ld, false, nullptr));
+    pi_layer_out o{};
+    o.x = s->x; o.wo = L.wo; o.att = s->att; o.rows = D; o.ld_att = L.hv_ld; o.T = R; o.out = s->x2;
+    if (L.moe()) {
+        PI_TRY(pi_k_norm_pair(PI_TYPE_BF16, s->x, nullptr, R, D, m->hp.norm_eps, L.norm_b, s->h_b, nullptr, nullptr, s->d_ld, 1, st));
+        PI_TRY(pi_k_gemm_bf16_ol(L.router, d.n_expert, s->d_ld, s->h_b, R, PI_EPI_NONE, nullptr, nullptr, s->rl, nullptr, st));
+        PI_TRY(pi_k_route(s->rl, R, d.n_expert, d.n_top, d.n_group, d.n_group_keep, L.bias, s->ids, s->wts, st));
+        PI_TRY(pi::expert_relu2_step(L.up, d.n_expert, d.expert_ff, s->d_ld, s->h_b, R, s->ids, s->wts, d.n_top, s->act, L.ff_ld, st));
+        o.down = L.down; o.act = s->act; o.ids = s->ids; o.ld_act = L.ff_ld; o.top = d.n_top; o.n_expert = d.n_expert;
+    }
+    PI_TRY(pi_k_layer_out_step(&o, st));
+    std::swap(s->x, s->x2);
+    return PI_OK;
 }
 
 // grouped-query attention over one list of work items
@@ -923,14 +998,27 @@ int one_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in,
         PI_TRY(pi_k_gqa_prep(type, &p, &f, st));
         PI_TRY(attend_grouped(m, L, r.pass, in, step, parts));
     }
+    const auto close = [&](int n) -> int {
+        pi_layer_out o{};
+        o.x = s->x; o.wo = L.wo; o.att = s->att; o.rows = D; o.ld_att = L.close_ld; o.T = n; o.out = s->x2; o.keep = keep;
+        if (moe) { o.down = L.down; o.act = s->act; o.ids = s->ids; o.ld_act = L.ff_ld; o.top = d.n_top; o.n_expert = d.n_expert; }
+        return pi_k_layer_out_step(&o, st);
+    };
     if (step) {
         if (moe || linear || parts.n_parts > 1)
             PI_TRY(pi_k_mix_up_step(parts.n_parts > 1 ? &parts : nullptr, linear ? &gate : nullptr, L.up, d.n_expert, d.expert_ff, s->d_ld, d.expert_limit, d.glu_gain, s->h_a, T,
                                     moe ? s->ids : nullptr, s->wts, d.n_top, s->act, L.ff_ld, st));
-        pi_layer_out o{};
-        o.x = s->x; o.wo = L.wo; o.att = s->att; o.rows = D; o.ld_att = L.close_ld; o.T = T; o.out = s->x2; o.keep = keep;
-        if (moe) { o.down = L.down; o.act = s->act; o.ids = s->ids; o.ld_act = L.ff_ld; o.top = d.n_top; o.n_expert = d.n_expert; }
-        return pi_k_layer_out_step(&o, st);
+        return close(T);
+    }
+    if (tail_of(m, L, r, in, keep)) {
+        const int R = in.n_rows;
+        if (R == 0) return PI_OK;
+        PI_TRY(take_tail(m, L, in, L.close_ld, moe, nullptr));
+        if (moe) {
+            PI_TRY(pi_k_layer_norm(type, s->x, nullptr, R, D, m->hp.norm_eps, L.norm_a, nullptr, nullptr, s->h_a, s->d_ld, 1, st));
+            PI_TRY(pi_k_mix_up_step(nullptr, nullptr, L.up, d.n_expert, d.expert_ff, s->d_ld, d.expert_limit, d.glu_gain, s->h_a, R, s->ids, s->wts, d.n_top, s->act, L.ff_ld, st));
+        }
+        return close(R);
     }
     PI_TRY(dense(m, L.wo, D, L.close_ld, s->att, T, s->mix));
     if (moe) PI_TRY(experts(m, L, s->h_a, in));
@@ -943,8 +1031,10 @@ int one_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in,
 int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in, float * keep) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
-    const int T = in.T, D = m->hp.n_embd, type = s->opts.compute;
-    const bool step = bf16_mode(s) && pi_k_layer_step_supported(T, 0, 0), grouped = d.mixer == PI_MIXER_GROUPED;
+    int T = in.T;
+    const int D = m->hp.n_embd, type = s->opts.compute;
+    bool step = bf16_mode(s) && pi_k_layer_step_supported(T, 0, 0);
+    const bool grouped = d.mixer == PI_MIXER_GROUPED;
     hipStream_t st = m->stream;
     if (step) PI_TRY(pi_k_gemm_bf16_ol(L.w_z, L.z_rows, s->d_ld, s->h_a, T, PI_EPI_NONE, nullptr, nullptr, s->z, nullptr, st));
     else PI_TRY(dense(m, L.w_z, L.z_rows, s->d_ld, s->h_a, T, s->z));
@@ -960,6 +1050,12 @@ int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in
         if (L.rec.on() || parts.n_parts > 1)
             PI_TRY(pi_k_mix_up_step(parts.n_parts > 1 ? &parts : nullptr, L.rec.on() ? &gate : nullptr, nullptr, 0, 0, 0, 0.0f, 0.0f, nullptr, T, nullptr, nullptr, 0, nullptr, 0, st));
     } else if (L.rec.on()) PI_TRY(pi_k_gate_norm(type, &gate, st));
+    const bool gated = d.gated_residual != 0, ffn = d.ffn == PI_FFN_GLU, tail = tail_of(m, L, r, in, keep);
+    if (tail) {
+        if (in.n_rows == 0) return PI_OK;
+        PI_TRY(take_tail(m, L, in, L.close_ld, false, gated ? s->z + L.off_gate : nullptr));
+        T = in.n_rows; step = true;
+    }
     // x = norm(alpha x + gate * W att), with the next product's operand
     const auto close = [&](const void * W, int ld, const float * gz, int ld_gate, int off_gate, const float * gb, const float * w, float * kept) -> int {
         pi_res_norm n{};
@@ -976,8 +1072,7 @@ int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in
         }
         return pi_k_res_norm(type, &n, st);
     };
-    const bool gated = d.gated_residual != 0, ffn = d.ffn == PI_FFN_GLU;
-    PI_TRY(close(L.wo, L.close_ld, gated ? s->z : nullptr, L.z_rows, L.off_gate, L.gate_b, L.norm_a, ffn ? nullptr : keep));
+    PI_TRY(close(L.wo, L.close_ld, !gated ? nullptr : tail ? s->gate_tail : s->z, tail ? D : L.z_rows, tail ? 0 : L.off_gate, L.gate_b, L.norm_a, ffn ? nullptr : keep));
     if (!ffn) return PI_OK;
     if (step) {
         const uint16_t * W = (const uint16_t *)L.w_ffn;
@@ -997,8 +1092,10 @@ int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in
 int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in, float * keep) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
-    const int T = in.T, D = m->hp.n_embd, type = s->opts.compute;
-    const bool moe = L.moe(), step = bf16_mode(s) && pi_k_layer_step_supported(T, moe ? d.n_expert : 0, moe ? d.n_top : 0);
+    int T = in.T;
+    const int D = m->hp.n_embd, type = s->opts.compute;
+    const bool moe = L.moe();
+    bool step = bf16_mode(s) && pi_k_layer_step_supported(T, moe ? d.n_expert : 0, moe ? d.n_top : 0);
     hipStream_t st = m->stream;
     if (L.conv) {
         pi_conv_norm c{};
@@ -1033,6 +1130,11 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
             PI_TRY(pi_k_gqa_stats(&a, s->stats, st));
             PI_TRY(pi_k_gqa_talk(&a, &x, s->stats, talk.items, talk.n, st));
         }
+    }
+    if (tail_of(m, L, r, in, keep)) {
+        if (in.n_rows == 0) return PI_OK;
+        PI_TRY(take_tail(m, L, in, L.close_ld, false, nullptr));
+        T = in.n_rows; step = true;
     }
     pi_layer_out o{};
     o.rows = D; o.T = T; o.out = s->mix;
@@ -1118,8 +1220,14 @@ int pass_layers(pi_model * m, const Step & in) {
             std::swap(s->x, s->x2);
             continue;
         }
-        PI_TRY(pi_k_norm_pair(type, s->x, nullptr, T, D, m->hp.norm_eps, L.norm_a, s->h_a, moe ? L.norm_b : nullptr, moe ? s->h_b : nullptr, s->d_ld, 0, st));
+        const bool tail = tail_of(m, L, s->order[k], in, keep), both = moe && !tail;
+        PI_TRY(pi_k_norm_pair(type, s->x, nullptr, T, D, m->hp.norm_eps, L.norm_a, s->h_a, both ? L.norm_b : nullptr, both ? s->h_b : nullptr, s->d_ld, 0, st));
         PI_TRY(mix_latent(m, L, in));
+        if (tail) {
+            PI_TRY(latent_tail(m, L, in));
+            continue;
+        }
+        PI_TRY(dense(m, L.wo, D, L.hv_ld, s->att, T, s->mix));
         if (moe) PI_TRY(ffn_moe(m, L, in));
         PI_TRY(pi_k_moe_combine(type, s->x, s->mix, s->y_exp, s->inv, moe ? s->wts : nullptr, moe ? L.d.n_top : 0, T, D, s->x2, keep, st));
         std::swap(s->x, s->x2);
@@ -1697,12 +1805,14 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             s->streams_T = T;
         }
         PI_TRY(ensure_expanded(m, in));
-        PI_TRY(pass_layers(m, in));
         const int32_t * d_rows = s->d_in + 8 * T + items.size();
+        in.rows = d_rows; in.n_rows = (int)rows.size();
+        struct Whole { LayerState * s; ~Whole() { if (s->tail) swap_tail(s); } } whole{s};      // however the pass ends, the buffers are in their own places behind it
+        PI_TRY(pass_layers(m, in));
         for (int r0 = 0; r0 < (int)rows.size(); r0 += kHeadRows) {
             const int n = std::min(kHeadRows, (int)rows.size() - r0);
             const size_t V = m->hp.n_vocab;
-            PI_TRY(pass_head(m, d_rows + r0, n));
+            PI_TRY(pass_head(m, s->tail ? nullptr : d_rows + r0, n));
             if (next_tokens) for (int k = 0; k < n; k += 16) PI_TRY(pi_k_argmax_batch(s->logits + k * V, (int)V, std::min(16, n - k), s->d_next + k, nullptr, nullptr, nullptr, 0, m->stream));
             std::vector<int32_t> nx(next_tokens ? n : 0);
             for (int k = 0; k < n; ) {                              // runs of places that follow one another leave in one copy

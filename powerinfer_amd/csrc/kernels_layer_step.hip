@@ -472,6 +472,22 @@ int pi_k_expert_up_step(const void * up, int n_expert, int ff, int cols, float l
     return pi::check_launch("pi_k_expert_up_step");
 }
 
+}  // extern "C"
+
+namespace pi {
+int expert_relu2_step(const void * up, int n_expert, int ff, int cols, const void * x_ol, int T, const int32_t * ids, const float * weights, int top, void * act, int ld_act,
+                      pi_stream_t stream) {
+    if (!up || !x_ol || !ids || !weights || !act || T <= 0 || T > kBtMaxT || n_expert <= 0 || ff <= 0 || cols <= 0 || cols % 32 || top <= 0 || T * top > kStepPairs || ld_act < ff)
+        return fail(PI_E_ARG, "expert_relu2_step: bad arguments");
+    const int tiles = (ff + 15) / 16;
+    hipLaunchKernelGGL(mix_and_up_kernel, dim3(tiles * T * top), dim3(256), kUpLds, (hipStream_t)stream, pi_gqa_attn{}, pi_gate_norm{}, 0, 0,
+                       ExpertUp{(const bf16 *)up, ff, cols, (const bf16 *)x_ol, ids, weights, T, top, (bf16 *)act, ld_act}, tiles);
+    return check_launch("expert_relu2_step");
+}
+}  // namespace pi
+
+extern "C" {
+
 int pi_k_layer_out_step(const pi_layer_out * a, pi_stream_t stream) {
     if (!a || (a->wo ? !a->att || a->ld_att <= 0 || a->ld_att % 32 : !a->ids) || !a->out || (a->gate_z && (!a->gate_b || a->off_gate < 0 || a->off_gate + a->rows > a->ld_gate)) || a->rows <= 0 || a->T <= 0 || a->T > kBtMaxT ||
         (a->ids && (!a->down || !a->act || a->ld_act <= 0 || a->ld_act % 32 || a->top <= 0 || a->T * a->top > kStepPairs || a->n_expert <= 0 || a->n_expert > kStepExperts)))

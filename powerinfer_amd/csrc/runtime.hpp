@@ -48,6 +48,9 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
 bool attn_chunk_by_16(int hd, int n_kv_max);
 int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
                   float * q_rot, void * k_cache, void * v_cache, hipStream_t st);
+// pi_k_expert_up_step with act = weight * relu(up[e] x)^2 (up [n_expert][ff][cols])
+int expert_relu2_step(const void * up, int n_expert, int ff, int cols, const void * x_ol, int T, const int32_t * ids, const float * weights, int top, void * act, int ld_act,
+                      pi_stream_t stream);
 // the embedding row of a token that the host names; also writes the token loop's state (token, position, step counter 0)
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
 

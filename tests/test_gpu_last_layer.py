@@ -1,10 +1,17 @@
-"""The last layer of prompts: sparse models keep only its keys and values for the tokens of a chunk."""
+"""The last layer of prompts: sparse models keep only its keys and values for the tokens of a chunk, models described layer by layer go on behind its
+attention with the tokens whose logits are wanted."""
 import numpy as np
 import pytest
 
-from powerinfer_amd import synth
+import fikevik_models
+import lerasun_models
+import pibalorn_models
+import pufivik_models
+from lerasun_models import row_errors, tokens
+from powerinfer_amd import fikevik, lerasun, pibalorn, pufivik, synth
 
 pytestmark = pytest.mark.gpu
+FAMILIES = {"lerasun": (lerasun, lerasun_models), "pibalorn": (pibalorn, pibalorn_models), "fikevik": (fikevik, fikevik_models), "pufivik": (pufivik, pufivik_models)}
 
 
 @pytest.mark.parametrize("name,layers,hot", [("llama-tiny", 1, 1.0), ("llama-tiny", 3, 1.0), ("falcon-tiny", 1, 1.0), ("falcon-tiny", 2, 1.0), ("llama-tiny", 2, 0.6)])
@@ -24,3 +31,27 @@ def test_a_step_behind_a_prompt(name, layers, hot, n):
     a.close()
     b.close()
     assert np.abs(got - want).max() < 1e-2 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("family", FAMILIES)
+@pytest.mark.parametrize("make", ["even_config", "odd_config"])
+@pytest.mark.parametrize("n,want", [(17, [16]), (17, []), (40, [39, 3, 3]), (150, list(range(134, 150))), (150, list(range(133, 150))), (150, [])])
+def test_wanted_rows(family, make, n, want):
+    """One, none, some (out of order, twice), as many as a step holds and one more: logits against a pass that keeps every token's stream (the rows of
+    the last layer are then products of the same bf16 values in another order, with the experts' sum rounded to bf16 on the way: 2^-8 of
+    a row, times four), and the step behind, whose cells and states are the same, bit for bit."""
+    lib, mod = FAMILIES[family]
+    cfg = getattr(mod, make)()
+    toks, out = tokens(cfg, n + 1, n), []
+    w = mod.weights(cfg, 17)
+    for keep in (True, False):
+        m = lib.build(cfg, w, n_ctx=512)
+        m.kv_cells_init(512)
+        m.set_capture(keep)
+        lg = m.kv_cells_step(toks[:n], range(n), [1] * n, want)[1]
+        m.set_capture(False)
+        out.append((lg, m.kv_cells_step(toks[n:], [n], [1], [0])[1]))
+        m.close()
+    (full, after), (got, then) = out
+    assert np.array_equal(after, then)
+    assert len(want) == 0 or (full.shape == got.shape == (len(want), full.shape[1]) and row_errors(got, full).max() < 2 ** -6)
