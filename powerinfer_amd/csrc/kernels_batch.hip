@@ -276,6 +276,7 @@ __global__ __launch_bounds__(kBlock) void gemm_t16_kernel(const EL * __restrict_
 // instruction (8 instructions = its 16 rows x 256 columns), drops the tile into a wave-private LDS buffer with a padded
 // row stride (conflict-free both ways) and reads it back in operand layout.  No workgroup barrier is involved: the
 // buffer belongs to one wave and LDS operations of a wave complete in order.  Two 256-column tiles of loads are in flight.
+// Bound by the weights: 32000 x 5120 at 6.2 TB/s, 32000 x 4096 at 6.2, 4096 x 4096 at 3.5 (launch, first loads and the closing sums).
 constexpr int kGlStride = 512 + 16;               // bytes per LDS row: 256 fp16 + one 16-byte pad
 // a second matrix of the same width with its own input and output (no epilogue) in the same launch; rows 0: none
 struct SecondGemm { const void * W; const void * x; int rows; float * y; };
@@ -299,50 +300,76 @@ __global__ __launch_bounds__(64 * NW) void gemm_t16_lds_kernel(const EL * __rest
     const int row0 = bx * 16 * RT;
     const int tok = i < T ? i : T - 1;
     // the 256-column super-steps of a row are dealt round-robin to the NW waves: wave w takes steps w, w + NW, ...
-    const EL * bp = (lay & 1) ? xn + (g * 16 + i) * 8 : xn + (size_t)tok * cols + g * 8;
+    const EL * bp = (lay & 1) ? xn + (g * 16 + tok) * 8 : xn + (size_t)tok * cols + g * 8;
     const int bstep = (lay & 1) ? 512 : 32;        // halves from one 32-column step's fragment to the next
     unsigned char * mytile = tile[wave];
     pi_f4 acc[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) acc[rt] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
     const int n_ss = (cols / 256 - wave + NW - 1) / NW;      // super-steps of this wave
-    pi_u32x4 ld[2][RT][8];
-    auto issue = [&](int buf, int ss) {
-        if (ss < n_ss) {
+    // Workgroups run side by side, at the same columns of rows a power of two apart as a rule: where a workgroup's rows span a multiple of 256 KB those
+    // fall on few of the memory's channels, and each workgroup then starts a super-step further on.  (2048 columns of 16 rows gain as well; at
+    // 128 KB the memory spreads them by itself, and a shift undoes that.)  us, without and with: 32000 x 4096 55.7 / 42.1, 12288 x 4096
+    // 27.4 / 21.3, 8192 x 8192 30.6 / 24.3, 65024 x 8192 201 / 165 (32 rows a workgroup); 32000 x 2048 29.1 / 27.0, 4096 x 4096 9.5 / 12.8
+    // (16 rows); 5120 columns alike.
+    constexpr int kSpan = 32 * RT;                       // bytes a column of the workgroup's rows takes
+    const int n_all = cols / 256, first = kSpan * cols % (256 << 10) == 0 || kSpan * cols == 64 << 10 ? bx % n_all : 0;
+    auto place = [&](int k) { k = wave + k * NW + first; return k >= n_all ? k - n_all : k; };
+    pi_u32x4 ld[2][RT][8], xb[8];
+    // Loads return in the order they are requested: a super-step's tokens are requested behind its own weights and in front of the next ones', so
+    // that waiting for them leaves a whole super-step of weights on its way
+    auto weights = [&](int buf, int ss) {
 #pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    int r = row0 + rt * 16 + 2 * j + lr;
-                    r = r < rows ? r : rows - 1;
-                    ld[buf][rt][j] = pi_ld_stream(W + (size_t)r * cols + (wave + ss * NW) * 256 + lc * 8);
-                }
-        }
+            for (int j = 0; j < 8; ++j) ld[buf][rt][j] = pi_ld_stream(W + (size_t)min(row0 + rt * 16 + 2 * j + lr, rows - 1) * cols + place(ss) * 256 + lc * 8);
     };
-    issue(0, 0);
-    issue(1, 1);
-    for (int ss = 0; ss < n_ss; ss += 2) {
+    auto tokens = [&](int ss) {
+#pragma unroll
+        for (int st = 0; st < 8; ++st) xb[st] = pi_ld16(bp + (place(ss) * 8 + st) * bstep);
+    };
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) *reinterpret_cast<pi_u32x4 *>(mytile + (2 * j + lr) * kGlStride + lc * 16) = ld[buf][rt][j];
+#pragma unroll
+            for (int st = 0; st < 8; ++st) {
+                const pi_u32x4 a = *reinterpret_cast<const pi_u32x4 *>(mytile + i * kGlStride + (4 * st + g) * 16);
+                acc[rt] = mma16<EL>(a, xb[st], acc[rt]);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (n_ss > 0) { weights(0, 0); tokens(0); }
+    __builtin_amdgcn_sched_barrier(0);
+    if (n_ss > 1) weights(1, 1);
+    // (no branch around a request while both buffers have one to come: what a wait leaves in flight is then known when it is compiled)
+    int ss = 0;
+    for (; ss + 4 <= n_ss; ss += 2)
 #pragma unroll
         for (int buf = 0; buf < 2; ++buf) {
-            const int cur = ss + buf;
-            if (cur < n_ss) {
-                pi_u32x4 b[8];
-#pragma unroll
-                for (int st = 0; st < 8; ++st) b[st] = pi_ld16(bp + ((wave + cur * NW) * 8 + st) * bstep);
-#pragma unroll
-                for (int rt = 0; rt < RT; ++rt) {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) *reinterpret_cast<pi_u32x4 *>(mytile + (2 * j + lr) * kGlStride + lc * 16) = ld[buf][rt][j];
-#pragma unroll
-                    for (int st = 0; st < 8; ++st) {
-                        const pi_u32x4 a = *reinterpret_cast<const pi_u32x4 *>(mytile + i * kGlStride + (4 * st + g) * 16);
-                        acc[rt] = mma16<EL>(a, b[st], acc[rt]);
-                    }
-                }
-            }
-            issue(buf, cur + 2);
+            multiply(buf);
+            tokens(ss + buf + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            weights(buf, ss + buf + 2);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    }
+    const int left = n_ss - ss;                         // up to three
+    if (left > 2) {
+        multiply(0);
+        tokens(ss + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        weights(0, ss + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+        tokens(ss + 2);
+        multiply(0);
+    } else if (left > 1) {
+        multiply(0);
+        tokens(ss + 1);
+        multiply(1);
+    } else if (left > 0) multiply(0);
     // the waves' accumulator tiles meet in LDS, each in the front of its wave's own (now idle) staging buffer
     auto cs = [&](int w, int r, int c) -> float & { return reinterpret_cast<float *>(tile[w])[r * 17 + c]; };
     const int rr = threadIdx.x >> 4, t = threadIdx.x & 15;
@@ -1242,7 +1269,11 @@ static int gemm_launch(const char * who, const void * W, int rows, int cols, con
     if (cols % 256 == 0) {
         // waves per workgroup: when every workgroup has a compute unit to itself (at most one per unit), eight waves keep twice
         // the loads in flight per unit; with more workgroups than units the chip is full with four
-        const int rtl = rt >= 2 ? 2 : 1;
+        // 16 rows a workgroup also where 32 would give some units a second one and others none (10240 x 4096, us: 17.9 against 19.0; 9216 x 8192
+        // 31.9 / 34.6; 12288 x 4096 21.6 / 21.3) and, beyond one for every unit, for short rows (2048 columns: 9216 rows 11.2 / 12.6, 32000 27.0 / 28.2;
+        // 11008 x 1024 6.9 / 7.6)
+        const int n32 = (rows + 31) / 32, cus = pi::compute_units();
+        const int rtl = rt >= 2 && (n32 <= cus || (2 * n32 >= 3 * cus && cols > 2048)) ? 2 : 1;
         const bool wide = (rows + 16 * rtl - 1) / (16 * rtl) <= pi::compute_units();
         if (rtl == 2) { if (wide) PI_GEMM_LDS(2, 8); else PI_GEMM_LDS(2, 4); }
         else { if (wide) PI_GEMM_LDS(1, 8); else PI_GEMM_LDS(1, 4); }
