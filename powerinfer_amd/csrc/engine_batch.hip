@@ -738,17 +738,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_pas
     b->n_seq = T;
     b->kv_hi = n_past + T;
     b->route = route;
-    std::vector<int32_t> pos(T);
-    for (int t = 0; t < T; ++t) pos[t] = n_past + t;
-    PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipMemcpyAsync(b->d_pos, pos.data(), sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    for (int t = 0; t < T; t += kChunkMaxT) {
-        const int n = std::min(T - t, kChunkMaxT);
-        float * x = b->x + (size_t)t * hp.n_embd;
-        if (m->glob[PI_T_TOK_EMBD].type == PI_TYPE_Q4_0) PI_TRY(pi_k_embed_batch_q4(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens + t, n, x, m->stream));
-        else PI_TRY(pi_k_embed_batch(m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, b->d_tokens + t, n, x, m->stream));
-    }
+    PI_TRY(pi::embed_chunk(m->glob[PI_T_TOK_EMBD].type, m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, tokens, T, n_past, b->x, b->d_pos, m->stream));
     b->staged_layer[0] = b->staged_layer[1] = -1;
     PI_TRY(stage_rest_rows(m, b, 0));
     for (int il = 0; il < hp.n_layer; ++il) {
@@ -778,13 +768,7 @@ int prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
     BatchState * b = m->prefill;
     b->n_seq = T;
     b->kv_hi = n_past + T;
-    int32_t pos[16];
-    for (int t = 0; t < T; ++t) pos[t] = n_past + t;
-    PI_HIP_TRY(hipMemcpyAsync(b->d_tokens, tokens, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipMemcpyAsync(b->d_pos, pos, sizeof(int32_t) * T, hipMemcpyHostToDevice, m->stream));
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
-    if (m->glob[PI_T_TOK_EMBD].type == PI_TYPE_Q4_0) PI_TRY(pi_k_embed_batch_q4(m->glob[PI_T_TOK_EMBD].dev, m->hp.n_embd, b->d_tokens, T, b->x, m->stream));
-    else PI_TRY(pi_k_embed_batch(m->glob[PI_T_TOK_EMBD].dev, m->hp.n_embd, b->d_tokens, T, b->x, m->stream));
+    PI_TRY(pi::embed_chunk(m->glob[PI_T_TOK_EMBD].type, m->glob[PI_T_TOK_EMBD].dev, m->hp.n_embd, tokens, T, n_past, b->x, b->d_pos, m->stream));
     for (int il = 0; il < m->hp.n_layer; ++il) PI_TRY(batch_layer(m, b, il));
     return PI_OK;
 }

@@ -563,6 +563,43 @@ __global__ void embed_q4_kernel(const pi_block_q4_0 * __restrict__ table, int co
         x[i] = __fmul_rn((float)(q - 8), pi_f16_from_bits(dbits));
     }
 }
+// Rows of a chunk's tokens, which travel as the kernel's arguments: copying 130 of them and their positions to the device and waiting for the copies took
+// 31 us ahead of a prompt's first product (a prompt of 131: 1913 -> 1882 us).  Eight values a thread; wide: rows and x on 16 bytes.
+struct ChunkTokens { static constexpr int kMost = 512; int32_t id[kMost]; };
+template <bool Q4>
+__global__ __launch_bounds__(256) void embed_chunk_kernel(const void * __restrict__ table, int cols, ChunkTokens tokens, int pos0, float * __restrict__ x, int32_t * __restrict__ pos, int wide) {
+    const int t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (blockIdx.x == 0 && threadIdx.x == 0) pos[t] = pos0 + t;
+    if (c >= cols) return;
+    float v[8];
+    if (Q4) {
+        const pi_block_q4_0 * b = (const pi_block_q4_0 *)table + (size_t)tokens.id[t] * (cols / 32) + c / 32;
+        uint16_t dbits; __builtin_memcpy(&dbits, &b->d, 2);
+        const float d = pi_f16_from_bits(dbits);
+        const int j = c & 15, high = c & 16 ? 4 : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = __fmul_rn((float)(((b->qs[j + k] >> high) & 0x0F) - 8), d);
+    } else {
+        const __half * row = (const __half *)table + (size_t)tokens.id[t] * cols + c;
+        if (wide) {
+            const pi_u32x4 raw = *reinterpret_cast<const pi_u32x4 *>(row);
+            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = pi_f16_from_bits((uint16_t)(w[k / 2] >> (16 * (k & 1))));
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = c + k < cols ? __half2float(row[k]) : 0.0f;
+        }
+    }
+    float * o = x + (size_t)t * cols + c;
+    if (wide) {
+        *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4 *>(o + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) if (c + k < cols) o[k] = v[k];
+    }
+}
 
 // first maximum wins (std::max_element, llama.cpp:8617-8631)
 __global__ __launch_bounds__(1024) void argmax_kernel(const float * __restrict__ logits, int n, int32_t * __restrict__ token_out) {
@@ -804,6 +841,20 @@ namespace pi {
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream) {
     if (!table || !d_token || !d_pos || !d_step || !x || cols <= 0) return fail(PI_E_ARG, "embed_start: bad arguments");
     return embed_one(wtype, table, cols, nullptr, TokenStart{token, pos, d_token, d_pos, d_step}, x, (hipStream_t)stream);
+}
+int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream) {
+    const bool q4 = wtype == PI_TYPE_Q4_0;
+    if (!table || !tokens || !x || !d_pos || cols <= 0 || T <= 0 || (q4 && cols % 32)) return fail(PI_E_ARG, "embed_chunk: bad arguments");
+    if (!q4 && wtype != PI_TYPE_F16) return fail(PI_E_UNSUPPORTED, "embed_chunk: table type must be F16 or Q4_0");
+    const int wide = cols % 8 == 0 && (((uintptr_t)x | (q4 ? 0 : (uintptr_t)table)) & 15) == 0;
+    for (int t0 = 0; t0 < T; t0 += ChunkTokens::kMost) {
+        const int n = T - t0 < ChunkTokens::kMost ? T - t0 : ChunkTokens::kMost;
+        ChunkTokens ids{};
+        for (int t = 0; t < n; ++t) ids.id[t] = tokens[t0 + t];
+        hipLaunchKernelGGL(q4 ? embed_chunk_kernel<true> : embed_chunk_kernel<false>, dim3((cols + 2047) / 2048, n), dim3(256), 0, (hipStream_t)stream, table, cols, ids, pos + t0,
+                           x + (size_t)t0 * cols, d_pos + t0, wide);
+    }
+    return check_launch("embed_chunk");
 }
 }  // namespace pi
 extern "C" {
