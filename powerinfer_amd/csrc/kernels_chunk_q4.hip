@@ -294,12 +294,14 @@ template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hip
 }
 
 // Tiles as 100 * (16-row tiles) + 10 * (16-token tiles a wave) + waves
-constexpr int kCqTiles[] = {112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624, 634};
+// (634 is there for a caller that asks for it: one round of it takes as long as two of 333 or 334, two workgroups of which share a unit.  17 to 24
+// token tiles of 7B shapes went there: 11008 x 4096, us, 280 tokens 53.3 -> 36.7, 360 tokens 55.0 -> 42.2; 12288 x 4096 54.3 -> 39.9)
+constexpr int kCqTiles[] = {112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624};
 constexpr int kCqTilesT[] = {212, 213, 215, 223, 422, 423, 424, 434};
 // What a launch takes goes with the rounds of workgroups over the compute units times what 32 columns of a tile take of a unit, in clocks: the
 // tokens' fragments at 64 bytes a clock, the matrix instructions of a SIMD, or the latency of a step where both are little; transposed, the
-// lines of 128 bytes that 18 or 36 are taken of, and the tokens.  Of 130 measured launches (17 .. 512 tokens, the matrices of 7B, 13B and
-// 40B shapes) the choice is the fastest in 112 and within 10 % of it in all.
+// lines of 128 bytes that 18 or 36 are taken of, and the tokens.  Of 152 measured launches (19 lengths of 17 .. 512 tokens, the matrices of 7B
+// and 13B shapes) the choice is within 10 % of the fastest in 150 and 12 % slower in the worst, 0.4 % on average.
 int cq_choose(int rows, int T, bool trans, int units) {
     const int * tiles = trans ? kCqTilesT : kCqTiles, n = trans ? (int)(sizeof kCqTilesT / sizeof(int)) : (int)(sizeof kCqTiles / sizeof(int));
     int best = tiles[0];
