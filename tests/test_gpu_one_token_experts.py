@@ -4,6 +4,7 @@ import pytest
 
 import test_gpu_gqa_ops
 import test_gpu_latent_ops
+import test_gpu_layer_out
 import test_gpu_pufivik_ops
 
 pytestmark = pytest.mark.gpu
@@ -22,3 +23,10 @@ def test_weighted_at_their_input(E, top, ff, cols):
 @pytest.mark.parametrize("E,top,ff,D", [(5, 3, 403, 2048), (4, 4, 129, 4096)])
 def test_squared_beside_values(E, top, ff, D):
     test_gpu_latent_ops.test_step_kernels(1, 4, 16, 8, 24, 40, E, top, ff, D, 4)
+
+
+@pytest.mark.parametrize("rows,ld_att,E,top,ld_act", [(4096, 0, 8, 6, 1408), (2048, 4864, 7, 6, 1408), (5120, 4096, 3, 2, 32), (1, 4096, 0, 0, 0), (257, 4128, 0, 0, 0), (4099, 8192, 9, 8, 2048), (100, 0, 1, 1, 32),
+                                                        (16000, 512, 2, 2, 96), (17000, 512, 2, 2, 96), (300, 20480, 0, 0, 0), (300, 20512, 2, 2, 4096)])
+def test_closing_a_layer(rows, ld_att, E, top, ld_act):
+    """One to six pieces a thread and more than that, up to as many rows as a workgroup takes and more, parts of a last piece."""
+    test_gpu_layer_out.test_closing_a_layer(rows, ld_att, E, top, ld_act, 1)
