@@ -126,6 +126,8 @@ struct Step {
     const int32_t * conv = nullptr; int n_conv = 0;    // items of the convolutions
     // the tokens whose logits are wanted, in this order (-1: not said, every token's stream is)
     const int32_t * rows = nullptr; int n_rows = -1;
+    // (latent attention) the last layer has no cells of its own: these tokens as a step, which is then all that is run of it
+    const Step * last = nullptr;
 };
 constexpr int kTailRows = 16;            // rows the last layer goes on with: what the kernels of a step hold
 
@@ -805,7 +807,7 @@ void swap_tail(LayerState * s) {
     std::swap(s->x, s->x_tail); std::swap(s->x2, s->x2_tail); std::swap(s->att, s->att_tail); std::swap(s->ids, s->ids_tail); std::swap(s->wts, s->wts_tail);
     s->tail = !s->tail;
 }
-// ld: columns of a row of att; routed: the experts are chosen already; gate (optional): n_embd values of the rows of s->z from there on
+// ld: columns of a row of att (0: not wanted); routed: the experts are chosen already; gate (optional): n_embd values of the rows of s->z from there on
 int take_tail(pi_model * m, const Layer & L, const Step & in, int ld, bool routed, const float * gate) {
     LayerState * s = m->lay;
     const int D = m->hp.n_embd;
@@ -815,7 +817,7 @@ int take_tail(pi_model * m, const Layer & L, const Step & in, int ld, bool route
         ++c.n;
     };
     add(s->x, 4 * (size_t)D, 4 * D, s->x_tail);
-    add(s->att, 2 * (size_t)ld, 2 * ld, s->att_tail);
+    if (ld > 0) add(s->att, 2 * (size_t)ld, 2 * ld, s->att_tail);
     if (routed) { add(s->ids, 4 * (size_t)L.d.n_top, 4 * L.d.n_top, s->ids_tail); add(s->wts, 4 * (size_t)L.d.n_top, 4 * L.d.n_top, s->wts_tail); }
     if (gate) add(gate, 4 * (size_t)L.z_rows, 4 * D, s->gate_tail);
     hipLaunchKernelGGL(tail_rows_kernel, dim3(in.n_rows, c.n), dim3(256), 0, m->stream, in.rows, c);
@@ -1182,6 +1184,12 @@ int step_layer(pi_model * m, Layer & L, const Step & in, float * keep) {
     return pi_k_layer_out_step(&o, st);
 }
 
+int rope_angles(pi_model * m, int rot, const int32_t * pos, int T) {
+    LayerState * s = m->lay;
+    const Rotation & r = s->rots[rot];
+    return r.scaling ? pi_k_rope_angles_table(pos, T, r.dims, r.freq, r.length(), s->cs[rot], m->stream) : pi_k_rope_angles(pos, T, r.dims, r.base, s->cs[rot], m->stream);
+}
+
 int pass_layers(pi_model * m, const Step & in) {
     LayerState * s = m->lay;
     const int type = s->opts.compute, T = in.T, D = m->hp.n_embd;
@@ -1194,10 +1202,7 @@ int pass_layers(pi_model * m, const Step & in) {
         n.x = n.out = s->x; n.T = T; n.cols = D; n.h = s->h_a; n.ld = s->d_ld; n.ol = bf16_mode(s) && pi_k_layer_step_supported(T, 0, 0);
         PI_TRY(pi_k_res_norm(type, &n, st));
     }
-    for (size_t k = 0; k < s->rots.size(); ++k) {
-        const Rotation & r = s->rots[k];
-        PI_TRY(r.scaling ? pi_k_rope_angles_table(in.pos, T, r.dims, r.freq, r.length(), s->cs[k], st) : pi_k_rope_angles(in.pos, T, r.dims, r.base, s->cs[k], st));
-    }
+    for (size_t k = 0; k < s->rots.size(); ++k) PI_TRY(rope_angles(m, (int)k, in.pos, T));
     for (size_t k = 0; k < s->order.size(); ++k) {
         Layer & L = s->layers[s->order[k].layer];
         const bool moe = L.moe();
@@ -1221,6 +1226,14 @@ int pass_layers(pi_model * m, const Step & in) {
             continue;
         }
         const bool tail = tail_of(m, L, s->order[k], in, keep), both = moe && !tail;
+        if (tail && in.last) {
+            if (in.n_rows == 0) return PI_OK;
+            PI_TRY(take_tail(m, L, in, 0, false, nullptr));
+            PI_TRY(rope_angles(m, L.rot, in.last->pos, in.n_rows));
+            PI_TRY(step_layer(m, L, *in.last, nullptr));
+            std::swap(s->x, s->x2);
+            continue;
+        }
         PI_TRY(pi_k_norm_pair(type, s->x, nullptr, T, D, m->hp.norm_eps, L.norm_a, s->h_a, both ? L.norm_b : nullptr, both ? s->h_b : nullptr, s->d_ld, 0, st));
         PI_TRY(mix_latent(m, L, in));
         if (tail) {
@@ -1761,6 +1774,25 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         }
         const size_t at_others = items.size();
         items.insert(items.end(), others.begin(), others.end());
+        // a last layer without cells of its own: its work items for the wanted tokens, their positions, cells in sight and sequences
+        const Layer & end = s->layers[s->order.back().layer];
+        const int R = (int)rows.size();
+        Step one;
+        size_t at_one = 0;
+        const bool alone = s->family == kTwoNorms && bf16_mode(s) && !m->capture && !end.own_kv && T > kTailRows && R <= kTailRows;
+        int one_items = 0, one_vis = 0;
+        if (alone) {
+            std::vector<int32_t> seq_r, vis_r, work;
+            for (int r : rows) { seq_r.push_back(seq[t0 + r]); vis_r.push_back(vis[t0 + r]); one_vis = std::max(one_vis, vis[t0 + r]); }
+            work_items(seq_r.data(), vis_r.data(), R, s->kinds[end.hc], work, nullptr);
+            one_items = (int)work.size() / 4;
+            items.resize((items.size() + 3) / 4 * 4);
+            at_one = items.size();
+            items.insert(items.end(), work.begin(), work.end());
+            for (int r : rows) items.push_back(positions[t0 + r]);
+            items.insert(items.end(), vis_r.begin(), vis_r.end());
+            items.insert(items.end(), seq_r.begin(), seq_r.end());
+        }
         const size_t n_in = (size_t)8 * T + items.size() + rows.size();
         PI_TRY(ensure_inputs(m, n_in));
         PI_TRY(inputs_free(m));
@@ -1806,7 +1838,14 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         }
         PI_TRY(ensure_expanded(m, in));
         const int32_t * d_rows = s->d_in + 8 * T + items.size();
-        in.rows = d_rows; in.n_rows = (int)rows.size();
+        in.rows = d_rows; in.n_rows = R;
+        if (alone) {
+            const int32_t * at = s->d_in + 8 * T + at_one;
+            one.T = R; one.pos = at + 4 * one_items; one.n_vis = one.pos + R; one.seq = one.n_vis + R;
+            one.work.resize(s->kinds.size());
+            one.work[end.hc] = Step::Work{at, one_items, choose_parts(s, one_items, one_vis)};
+            in.last = &one;
+        }
         struct Whole { LayerState * s; ~Whole() { if (s->tail) swap_tail(s); } } whole{s};      // however the pass ends, the buffers are in their own places behind it
         PI_TRY(pass_layers(m, in));
         for (int r0 = 0; r0 < (int)rows.size(); r0 += kHeadRows) {

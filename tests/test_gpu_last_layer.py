@@ -55,3 +55,29 @@ def test_wanted_rows(family, make, n, want):
     (full, after), (got, then) = out
     assert np.array_equal(after, then)
     assert len(want) == 0 or (full.shape == got.shape == (len(want), full.shape[1]) and row_errors(got, full).max() < 2 ** -6)
+
+
+@pytest.mark.parametrize("want", [[29], [69, 29, 0], list(range(54, 70)), []])
+def test_wanted_rows_of_a_layer_without_cells(want):
+    """Latent attention whose last layer reads the cells of the one before: two sequences' tokens in one pass, wanted rows of one and both (out of order),
+    as many as a step holds, none.  The attention of these is the latent form instead of the expanded one, so against the CPU path, as
+    test_gpu_lerasun.py has it."""
+    import plain_latent
+    import test_gpu_lerasun as lt
+    cfg = lerasun_models.config(96, 101, [lerasun_models.layer(4, 16, 8, 24, 40), lerasun_models.layer(4, 16, 8, 24, 40, kv_from=0, moe=(6, 2, 3, 2, 24))])
+    w = lerasun_models.weights(cfg, 17)
+    a, b = tokens(cfg, 30, 1), tokens(cfg, 40, 2)
+    m = lerasun.build(cfg, w, n_ctx=512)
+    m.kv_cells_init(512)
+    got = m.kv_cells_step(a + b, list(range(30)) + list(range(40)), [1] * 30 + [2] * 40, want)[1]
+    after = m.kv_cells_step([5, 6], [30, 40], [1, 2], [0, 1])[1]
+    m.close()
+    runs = []
+    for toks in (a + [5], b + [6]):
+        p = plain_latent.PlainModel(cfg, w)
+        lg = p.feed(toks)
+        runs.append(lt.Logits(lg, np.asarray(p.margins)))
+    full = lt.Logits(np.concatenate([np.asarray(runs[0])[:30], np.asarray(runs[1])[:40]]), np.concatenate([runs[0].margins[:30], runs[1].margins[:40]]))
+    if want:
+        lt.check(got, full[want], lt.pl.BF16)
+    lt.check(after, lt.Logits(np.stack([np.asarray(r)[-1] for r in runs]), np.array([r.margins[-1] for r in runs])), lt.pl.BF16)
