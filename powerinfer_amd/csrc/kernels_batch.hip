@@ -513,10 +513,13 @@ __global__ __launch_bounds__(256) void ffn_h_q8_ol_kernel(const float * __restri
 // for 2048 tokens of 11008 neurons) goes to memory.  The products' sums are formed in 32-column steps in fp32, as in the tiles of
 // the dense mat-mul.  11008 x 4096 twice, us (two library products and ffn_h_f16_kernel before): 2047 tokens 675 -> 327 (1.13
 // PFLOP/s), 1024 tokens 222 -> 174, 256 tokens 109 -> 61, 64 tokens 60 -> 46; 32768 x 8192 alone, 2047 tokens: 1100 -> 941.
-template <bool PAIRS> struct FfnProduct {
+// MASK: which neurons are active comes as bits (MaskProduct) instead of logits: a 16 x 16 tile's bit l of word r is its lane l's r-th neuron, as the
+// accumulators lie.
+template <bool PAIRS, bool MASK> struct FfnProduct {
     static constexpr bool kPairs = PAIRS;
     const __half * up, * gate, * x; const float * logits; float thr; __half * h16;
     int ff, cols, T, nk;
+    const unsigned long long * mask;
     __device__ __forceinline__ WidePlace place(const WideDeal & deal, int c) const {
         WidePlace p;
         int ty;
@@ -533,8 +536,9 @@ template <bool PAIRS> struct FfnProduct {
         asm volatile("" : "+v"(lane));                 // what follows is computed here, not kept in registers across the products
         const int i = lane & 15, q = lane >> 4, n0 = PAIRS ? p.row0 / 2 + rb / 128 * 64 + rb % 128 : p.row0 + rb;          // this wave's first neuron
         const int left = ff - n0;                      // (a multiple of 64: whole tiles of 16 neurons or none)
-        float4 lg[2][MO];
+        float4 lg[MASK ? 1 : 2][MO];
         auto fetch = [&](int nn) {
+            if constexpr (MASK) return;
             const float * l = logits + (size_t)(p.lo + min(tb + nn * 16 + i, p.n - 1)) * ff + n0 + 4 * q;
 #pragma unroll
             for (int m = 0; m < MO; ++m) lg[nn & 1][m] = *reinterpret_cast<const float4 *>(l + (m * 16 < left ? m * 16 : 0));
@@ -545,14 +549,17 @@ template <bool PAIRS> struct FfnProduct {
         for (int nn = 0; nn < 4; ++nn) {
             if (nn < 3) fetch(nn + 1);
             uint2 out[MO];
+            const unsigned long long * bits = MASK ? mask + ((size_t)min((p.lo + tb) / 16 + nn, (T - 1) / 16) * (ff / 16) + n0 / 16) * 4 : nullptr;
 #pragma unroll
             for (int m = 0; m < MO; ++m) {
-                const float l[4] = {lg[nn & 1][m].x, lg[nn & 1][m].y, lg[nn & 1][m].z, lg[nn & 1][m].w};
+                const float4 lm = MASK ? float4{} : lg[MASK ? 0 : nn & 1][m];
+                const float l[4] = {lm.x, lm.y, lm.z, lm.w};
                 __half h[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float u = acc[m][nn][r], v = PAIRS ? __fmul_rn(fmaxf(acc[(m + MO) % MT][nn][r], 0.0f), u) : fmaxf(u, 0.0f);
-                    h[r] = __float2half_rn(!(l[r] < thr) ? v : 0.0f);
+                    const bool on = MASK ? (bits[(m * 16 < left ? m : 0) * 4 + r] >> lane & 1) != 0 : !(l[r] < thr);
+                    h[r] = __float2half_rn(on ? v : 0.0f);
                 }
                 out[m] = __builtin_bit_cast(uint2, h);
             }
@@ -564,7 +571,46 @@ template <bool PAIRS> struct FfnProduct {
         }
     }
 };
-template <bool PAIRS> __global__ __launch_bounds__(512, 1) void ffn_wide_kernel(FfnProduct<PAIRS> prod) {
+// The predictor's second product, of which that is all anybody reads: 2047 tokens of 11008 neurons are 2.8 MB of bits instead of 90 of logits, written here
+// and read by the FFN's first half.  Four 7B-shaped layers, us, library product with logits and this: 2047 tokens 3829 -> 3696, 600 1692 -> 1665, 300 1318 ->
+// 1285, 131 1055 -> 1031, 100 957 -> 949; 13B 400 tokens 1408 -> 1378, 40B 700 tokens 1550 -> 1531.
+struct MaskProduct {
+    static constexpr bool kPairs = false;
+    const __half * W, * x; float thr; unsigned long long * mask;
+    int rows, cols, T, nk;
+    __device__ __forceinline__ WidePlace place(const WideDeal & deal, int c) const {
+        WidePlace p;
+        int ty;
+        deal.unit(c, ty, p.row0, p.rows);
+        p.grp = 0; p.lo = ty * kGwN; p.n = min(T - p.lo, kGwN);
+        return p;
+    }
+    __device__ __forceinline__ const unsigned char * base_a(const WidePlace &, int) const { return (const unsigned char *)W; }
+    __device__ __forceinline__ const unsigned char * base_b(const WidePlace & p) const { return (const unsigned char *)(x + (size_t)p.lo * cols); }
+    __device__ __forceinline__ uint32_t off_a(const WidePlace & p, int r) const { return (uint32_t)(p.row0 + r) * (uint32_t)(cols * 2); }
+    __device__ __forceinline__ size_t off_b(const WidePlace &, int r) const { return (size_t)r * cols * 2; }
+    template <int MT> __device__ __forceinline__ void store(const WidePlace & p, int rb, int tb, const pi_f4 (&acc)[MT][4], unsigned char *, int lane) const {
+        const int left = min(p.rows - rb, 16 * MT) / 16;             // (rows % 128 == 0: whole tiles)
+#pragma unroll
+        for (int nn = 0; nn < 4; ++nn) {
+            const int tile = (p.lo + tb) / 16 + nn;
+            if (tile > (T - 1) / 16) break;
+            unsigned long long mine = 0;                             // lane 4 m + r: word r of tile m
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const unsigned long long w0 = __ballot(!(acc[m][nn][0] < thr)), w1 = __ballot(!(acc[m][nn][1] < thr)), w2 = __ballot(!(acc[m][nn][2] < thr)), w3 = __ballot(!(acc[m][nn][3] < thr));
+                const unsigned long long w = lane & 2 ? (lane & 1 ? w3 : w2) : lane & 1 ? w1 : w0;
+                if (lane >> 2 == m) mine = w;
+            }
+            if (lane < 4 * left) mask[((size_t)tile * (rows / 16) + (p.row0 + rb) / 16) * 4 + lane] = mine;
+        }
+    }
+};
+__global__ __launch_bounds__(512, 1) void mask_wide_kernel(MaskProduct prod) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    gemm_wide<__half>(prod, WideDeal(prod.rows, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
+}
+template <bool PAIRS, bool MASK> __global__ __launch_bounds__(512, 1) void ffn_wide_kernel(FfnProduct<PAIRS, MASK> prod) {
     extern __shared__ __align__(16) unsigned char smem[];
     gemm_wide<__half>(prod, WideDeal(PAIRS ? 2 * prod.ff : prod.ff, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
 }
@@ -1379,6 +1425,45 @@ static int gemm_tile_launch(const void * W, int rows, int cols, const void * xn_
     return pi::check_launch("pi_k_gemm_tile");
 }
 
+// logits or mask, not both
+static int ffn_wide(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, const unsigned long long * mask, float threshold, void * h_f16,
+                    pi_stream_t stream) {
+    if (!up_f16 || !xn_f16 || !h_f16 || T <= 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: bad arguments");
+    if (!pi_k_ffn_wide_supported(ff, cols)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_ffn_wide_f16: ff must be a multiple of 128, cols a multiple of 64 and at least 256");
+    if ((((uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)xn_f16 | (uintptr_t)logits | (uintptr_t)h_f16) & 15) != 0)
+        return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: operands must be 16-byte aligned");
+    const long long units = (long long)(((gate_f16 ? 2 * ff : ff) + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
+    if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: too many tiles");
+    const auto launch = [&](auto pairs, auto masked) -> int {
+        constexpr bool P = decltype(pairs)::value, M = decltype(masked)::value;
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&ffn_wide_kernel<P, M>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
+        if (raised != hipSuccess) return pi::hip_fail(raised, "ffn_wide: LDS size");
+        hipLaunchKernelGGL((ffn_wide_kernel<P, M>), dim3(wide_blocks(units)), dim3(512), kGwLds, (hipStream_t)stream,
+                           FfnProduct<P, M>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, logits, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK, mask});
+        return pi::check_launch("pi_k_ffn_wide_f16");
+    };
+    const std::true_type yes{}; const std::false_type no{};
+    if (mask) return gate_f16 ? launch(yes, yes) : launch(no, yes);
+    return gate_f16 ? launch(yes, no) : launch(no, no);
+}
+
+namespace pi {
+// the predictor's second product [ff][rank] by hid [T][rank] and, under its bits, the FFN's first half as pi_k_ffn_wide_f16; mask: (T + 15) / 16 * ff / 16 * 4 words
+int ffn_wide_predicted(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold,
+                       void * mask, void * h_f16, hipStream_t st) {
+    if (!fc2_f16 || !hid_f16 || !mask || T <= 0 || !pi_k_ffn_wide_supported(ff, rank) || (((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)mask) & 15) != 0)
+        return fail(PI_E_ARG, "ffn_wide_predicted: bad arguments");
+    const long long units = (long long)((ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
+    if (units > (1 << 30)) return fail(PI_E_ARG, "ffn_wide_predicted: too many tiles");
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&mask_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
+    if (raised != hipSuccess) return hip_fail(raised, "mask_wide: LDS size");
+    hipLaunchKernelGGL(mask_wide_kernel, dim3(wide_blocks(units)), dim3(512), kGwLds, st, MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, (unsigned long long *)mask, ff, rank,
+                       T, rank / kGtBK});
+    if (const int rc = check_launch("mask_wide")) return rc;
+    return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, nullptr, (const unsigned long long *)mask, threshold, h_f16, st);
+}
+}  // namespace pi
+
 extern "C" {
 
 int pi_k_gemm_tile_f16(const void * W, int rows, int cols, const void * xn_f16, int T, int epilogue, const float * add1, const float * add2,
@@ -1399,23 +1484,8 @@ int pi_k_ffn_h_f16(const float * up, const float * gate, const float * logits, f
 int pi_k_ffn_wide_supported(int ff, int cols) { return ff > 0 && ff % 128 == 0 && cols >= 4 * kGtBK && cols % kGtBK == 0 && (long long)ff * cols < (1LL << 31); }
 
 int pi_k_ffn_wide_f16(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, float threshold, void * h_f16, pi_stream_t stream) {
-    if (!up_f16 || !xn_f16 || !logits || !h_f16 || T <= 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: bad arguments");
-    if (!pi_k_ffn_wide_supported(ff, cols)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_ffn_wide_f16: ff must be a multiple of 128, cols a multiple of 64 and at least 256");
-    if ((((uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)xn_f16 | (uintptr_t)logits | (uintptr_t)h_f16) & 15) != 0)
-        return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: operands must be 16-byte aligned");
-    const long long units = (long long)(((gate_f16 ? 2 * ff : ff) + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
-    if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: too many tiles");
-    static bool raised = false;
-    if (!raised) {
-        PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ffn_wide_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
-        PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&ffn_wide_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds));
-        raised = true;
-    }
-#define PI_FFN_WIDE(P) hipLaunchKernelGGL(ffn_wide_kernel<P>, dim3(wide_blocks(units)), dim3(512), kGwLds, (hipStream_t)stream, \
-    FfnProduct<P>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, logits, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK})
-    if (gate_f16) PI_FFN_WIDE(true); else PI_FFN_WIDE(false);
-#undef PI_FFN_WIDE
-    return pi::check_launch("pi_k_ffn_wide_f16");
+    if (!logits) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: bad arguments");
+    return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, logits, nullptr, threshold, h_f16, stream);
 }
 
 int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream) {

@@ -15,7 +15,7 @@ FAMILIES = {"lerasun": (lerasun, lerasun_models), "pibalorn": (pibalorn, pibalor
 
 
 @pytest.mark.parametrize("name,layers,hot,ff", [("llama-tiny", 1, 1.0, 8192), ("llama-tiny", 3, 1.0, 8192), ("falcon-tiny", 1, 1.0, 8192), ("falcon-tiny", 2, 1.0, 8192), ("llama-tiny", 2, 0.6, 8192),
-                                                ("llama-tiny", 2, 1.0, 4096)])
+                                                ("llama-tiny", 2, 1.0, 4096), ("llama-tiny", 3, 1.0, 8448), ("falcon-tiny", 2, 1.0, 8448)])
 @pytest.mark.parametrize("n", [3, 17, 18, 34, 131, 530])
 def test_a_step_behind_a_prompt(name, layers, hot, ff, n):
     """Logits of the step behind a prompt, whose cells a chunk wrote, against those behind the same tokens one by one: both are sums of the same fp16
