@@ -285,9 +285,8 @@ template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hip
     constexpr size_t lds = (size_t)2 * kCqSteps * MT * 1024;
     a.nx = (a.rows + 16 * MT - 1) / (16 * MT); a.ny = ((a.T + 15) / 16 + NT * WN - 1) / (NT * WN);
     if constexpr (lds > 64 * 1024) {
-        static bool raised = false;
-        if (!raised) PI_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        raised = true;
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (raised != hipSuccess) return pi::hip_fail(raised, "pi_k_gemm_q4_chunk: LDS size");
     }
     hipLaunchKernelGGL((gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), dim3((unsigned)(8 * ((a.nx + 7) / 8) * a.ny)), dim3(cq_threads(MT, WN, TRANS)), lds, st, a);
     return pi::check_launch("pi_k_gemm_q4_chunk");
