@@ -455,17 +455,18 @@ int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int c
     return PI_OK;
 }
 
-// Q4_0 matrices that are whole on the device are multiplied straight from their blocks in chunks of up to 512 tokens; what they read is then in
+// Q4_0 matrices that are whole on the device are multiplied straight from their blocks in chunks of fewer than 512 tokens; what they read is then in
 // the operand layout (out_ol).  Expanding first writes and reads the matrix in fp16 once more than that: us, expanded and multiplied by
-// the library / straight, 17, 130 and 512 tokens: 12288 x 4096 42 / 15, 51 / 21, 74 / 63; 4096 x 11008 transposed 46 / 25, 66 / 39,
-// 89 / 67; 13824 x 5120 54 / 19, 66 / 30, 99 / 86.  Longer chunks share one expansion among their pieces: four of 512 of 13824 x 5120
-// take 300 us so, and would take 344.
+// the library / straight, 17 and 130 tokens: 12288 x 4096 42 / 15, 51 / 21; 4096 x 11008 transposed 46 / 25, 66 / 39; 13824 x 5120 54 / 19,
+// 66 / 30.  Longer chunks share one expansion among their pieces: four of 512 of 13824 x 5120 take 300 us so, and would take 344.  512
+// tokens by themselves would gain too (74 / 63, 89 / 67, 99 / 86), but they are a piece of a longer chunk when 17 tokens more follow, and
+// their cells are to be the same either way.
 bool direct_q4(pi_model * m, BatchState * b, int il, int kind) {
     const Tensor & t = m->L(il, kind);
     const bool ffn = kind == PI_T_FFN_UP || kind == PI_T_FFN_GATE || kind == PI_T_FFN_DOWN_T;
     const int d = m->hp.n_embd, ff = m->hp.n_ff;
     const int rows = kind == PI_T_WQKV ? d + 2 * m->gqa : kind == PI_T_FFN_UP || kind == PI_T_FFN_GATE ? ff : d, cols = kind == PI_T_FFN_DOWN_T ? ff : d;
-    return m->gemm_lib && b->n_seq <= kChunkMaxT && t.type == PI_TYPE_Q4_0 && !(ffn && m->L(il, PI_T_GPU_BUCKET).dev) && pi_k_gemm_q4_chunk_supported(rows, cols) && ((uintptr_t)t.dev & 3) == 0;
+    return m->gemm_lib && b->n_seq < kChunkMaxT && t.type == PI_TYPE_Q4_0 && !(ffn && m->L(il, PI_T_GPU_BUCKET).dev) && pi_k_gemm_q4_chunk_supported(rows, cols) && ((uintptr_t)t.dev & 3) == 0;
 }
 // the product with matrix `kind`, straight or the other way
 int chunk_product(pi_model * m, BatchState * b, int il, int kind, bool direct, int rows, int cols, const __half * xn, int epi, const float * add1, const float * add2, float * y) {

@@ -48,6 +48,20 @@ def test_cells_of_a_q4_prompt_do_not_depend_on_what_follows(name, hot):
     assert all(np.array_equal(a, after[602]) for a in after.values()), {n: float(np.abs(a - after[602]).max()) for n, a in after.items()}
 
 
+@pytest.mark.parametrize("name,hot", [("llama-tiny", 1.0), ("falcon-tiny", 1.0), ("llama-tiny", 0.6)])
+def test_a_whole_piece_of_a_q4_prompt_goes_one_way(name, hot):
+    """Q4_0: up to 16 tokens behind the first 512 leave these a chunk of their own, 17 make them a piece of a longer one: the same cells, bit for bit."""
+    hp = synth.hparams(name, n_rank=256, n_ctx=700, seed=9, wtype=synth.Q4_0, hot_frac=hot)
+    model = synth.make_model(hp)
+    prompt = np.random.default_rng(4).integers(0, hp.n_vocab, 602).astype(np.int32)
+    m, after = fresh(hp, model), {}
+    for n in (513, 520, 529, 530, 602):                 # (the token that ends a prompt goes by itself)
+        m.decode(prompt[:n], 0)
+        after[n] = m.decode([5], 512)[1]
+    m.close()
+    assert all(np.array_equal(a, after[602]) for a in after.values()), {n: float(np.abs(a - after[602]).max()) for n, a in after.items()}
+
+
 LONG = [("llama-tiny", synth.F16, 1.0, 1600, [1500]), ("falcon-tiny", synth.F16, 1.0, 2400, [2300]), ("llama-tiny", synth.F16, 1.0, 16384, [2300]),
         ("llama-tiny", synth.F16, 1.0, 2400, [1100, 1200]), ("llama-tiny", synth.F16, 0.6, 1300, [1200]),
         ("llama-tiny", synth.Q4_0, 1.0, 1300, [1200]), ("falcon-tiny", synth.Q4_0, 1.0, 2100, [600, 1400]), ("llama-tiny", synth.Q4_0, 0.6, 1300, [1200])]
