@@ -508,18 +508,16 @@ __global__ __launch_bounds__(512) void layer_out_one_kernel(pi_layer_out a, int 
     float x[J][8];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-        const int q = min(tid + 512 * j, total - 1);    // (past the end the last piece again, times zero)
+        const int q = min(tid + 512 * j, total - 1);    // (past the end the last piece again, not used)
         const bool att = q < n_att;
         const int k = att ? 0 : (q - n_att) / n_act, c = (att ? q : (q - n_att) % n_act) * 8;
         ldw[j] = att ? a.ld_att : a.ld_act;
         w[j] = (att ? (const bf16 *)a.wo : (const bf16 *)a.down + (size_t)a.ids[k] * a.rows * a.ld_act) + (size_t)row0 * ldw[j] + c;
         const pi_u32x4 v = pi_ld16((att ? (const bf16 *)a.att : (const bf16 *)a.act + (size_t)k * a.ld_act) + c);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x[j][2 * e] = tid + 512 * j < total ? __uint_as_float(v[e] << 16) : 0.0f;
-            x[j][2 * e + 1] = tid + 512 * j < total ? __uint_as_float(v[e] & 0xFFFF0000u) : 0.0f;
-        }
+        for (int e = 0; e < 4; ++e) { x[j][2 * e] = __uint_as_float(v[e] << 16); x[j][2 * e + 1] = __uint_as_float(v[e] & 0xFFFF0000u); }
     }
+    const bool last = tid + 512 * (J - 1) < total;      // the others hold a piece less (not one times zero: a weight may be infinite)
     pi_u32x4 ld[2][D][J];
     auto request = [&](int b, int g) {                  // past the end the last row again, not used
 #pragma unroll
@@ -530,15 +528,17 @@ __global__ __launch_bounds__(512) void layer_out_one_kernel(pi_layer_out a, int 
     auto multiply = [&](int b, int g) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            float s[2] = {0.0f, 0.0f};
+            float s[2] = {0.0f, 0.0f}, less = 0.0f;
 #pragma unroll
-            for (int j = 0; j < J; ++j)
+            for (int j = 0; j < J; ++j) {
+                if (j == J - 1) less = s[0] + s[1];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     s[0] = fmaf(__uint_as_float(ld[b][d][j][e] << 16), x[j][2 * e], s[0]);
                     s[1] = fmaf(__uint_as_float(ld[b][d][j][e] & 0xFFFF0000u), x[j][2 * e + 1], s[1]);
                 }
-            const float t = pi_wave_sum(s[0] + s[1]);
+            }
+            const float t = pi_wave_sum(last ? s[0] + s[1] : less);
             if (lane == 0 && g * D + d < n) part[wave][g * D + d] = t;
         }
     };

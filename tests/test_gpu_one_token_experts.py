@@ -1,11 +1,15 @@
 """One token's experts by streams of rows: first matrices of 2048, 4096 and 8192 columns, with fewer rows than workgroups, experts that end within a
 workgroup's rows, and beside the launch's other parts - the operators' own comparisons at these sizes."""
+import ctypes as C
+
+import numpy as np
 import pytest
 
 import test_gpu_gqa_ops
 import test_gpu_latent_ops
 import test_gpu_layer_out
 import test_gpu_pufivik_ops
+from powerinfer_amd import lib as pl
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +34,16 @@ def test_squared_beside_values(E, top, ff, D):
 def test_closing_a_layer(rows, ld_att, E, top, ld_act):
     """One to six pieces a thread and more than that, up to as many rows as a workgroup takes and more, parts of a last piece."""
     test_gpu_layer_out.test_closing_a_layer(rows, ld_att, E, top, ld_act, 1)
+
+
+@pytest.mark.parametrize("ld_att", [32, 4128, 8192, 12320])
+def test_infinite_weights_close_a_layer(ld_att):
+    """Threads without a last piece of their own hold it again: an infinite weight there is one term of its row's sum and no zero times infinity."""
+    L, rng, rows = pl.init(), np.random.default_rng(ld_att), 4100
+    wo, att = test_gpu_layer_out.bf16(rng.standard_normal((rows, ld_att))), test_gpu_layer_out.bf16(0.5 + rng.random((1, ld_att)))
+    wo[7, ld_att - 1], wo[rows - 1, ld_att - 8] = test_gpu_layer_out.bf16([np.inf, -np.inf])
+    w, a, out, s = pl.DevBuf(host=wo), pl.DevBuf(host=att), pl.DevBuf.zeros(4 * rows), pl.LayerOut()
+    s.wo, s.att, s.ld_att, s.rows, s.T, s.out = w.ptr, a.ptr, ld_att, rows, 1, out.ptr
+    pl.check(L.pi_k_layer_out_step(C.byref(s), None))
+    got = out.download(np.float32)
+    assert got[7] == np.inf and got[-1] == -np.inf and np.isfinite(np.delete(got, [7, rows - 1])).all()
