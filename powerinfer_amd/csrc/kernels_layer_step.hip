@@ -356,10 +356,15 @@ __device__ __forceinline__ void expert_up_any(const ExpertUp & a, int b, int n_t
     else if (a.cols == 4096) expert_up_one<2>(a, b, smem);
     else expert_up_one<4>(a, b, smem);
 }
-// workgroups of the experts' first matrices; one token of 2048, 4096 or 8192 columns goes by streams
+// Workgroups of the experts' first matrices.  One token of 2048, 4096 or 8192 columns goes by streams.  Of 2048 columns eight rows are one group of requests, and
+// streams pay with 32 rows or more each or where two groups are full or nearly so: below and between, a tile of 16 rows is done in one trip and
+// most tiles side by side, while a stream asks for a group more than it has.  us, tiles / streams, experts x rows: 2048 columns 1 x 32 4.8 / 5.8,
+// 4 x 512 6.3 / 8.5, 2 x 2816 9.3 / 9.5, 4 x 2048 11.1 / 10.1, 6 x 1536 13.1 / 14.2, 6 x 2816 19.5 / 19.5, 8 x 2048 19.9 / 16.2; 4096 columns 1 x 32
+// 7.2 / 5.0, 4 x 512 9.0 / 8.5, 6 x 2816 30.8 / 25.5; 8192 columns 1 x 32 11.6 / 5.4, 4 x 512 15.2 / 10.7.
 inline int up_blocks(ExpertUp & u, int n_tiles) {
-    const int units = u.top * u.ff / (u.glu ? 2 : 1), most = 2 * pi::compute_units();
-    if (u.T == 1 && most > 0 && (u.cols == 2048 || u.cols == 4096 || u.cols == 8192) && (units + most - 1) / most * (u.glu ? 2 : 1) * 16 <= kUpLds) {
+    const int per_unit = u.glu ? 2 : 1, units = u.top * u.ff / per_unit, most = 2 * pi::compute_units(), rows = most > 0 ? (units + most - 1) / most * per_unit : 0;
+    const bool pays = u.cols == 4096 || u.cols == 8192 || (u.cols == 2048 && (rows >= 32 || (rows >= 14 && rows <= 16)));
+    if (u.T == 1 && most > 0 && pays && rows * 16 <= kUpLds) {
         u.streams = units < most ? units : most;
         return u.streams;
     }

@@ -15,7 +15,7 @@ std::map<const void *, std::string> & names() { static std::map<const void *, st
 std::map<std::string, int> counts;
 std::map<void *, size_t> live;
 size_t live_bytes = 0, peak_bytes = 0, limit_bytes = ~(size_t)0;
-int n_launch = 0, fail_at = -1;
+int n_launch = 0, fail_at = -1, grid_x = 0;
 hipError_t last = hipSuccess;
 char some[64];
 template <typename T> hipError_t give(T * p) { *p = (T)some; return hipSuccess; }
@@ -24,6 +24,7 @@ template <typename T> hipError_t give(T * p) { *p = (T)some; return hipSuccess; 
 extern "C" {
 void fake_fail_launch(int k) { n_launch = 0; fail_at = k; last = hipSuccess; }
 int fake_launches() { return n_launch; }
+int fake_grid() { return grid_x; }                     // workgroups of the last launch
 void fake_limit(size_t free_bytes) { limit_bytes = free_bytes == ~(size_t)0 ? free_bytes : live_bytes + free_bytes; }
 size_t fake_live() { return live_bytes; }
 size_t fake_peak() { size_t p = peak_bytes; peak_bytes = live_bytes; return p; }
@@ -38,7 +39,7 @@ void ** __hipRegisterFatBinary(const void *) { return (void **)some; }
 void __hipUnregisterFatBinary(void **) {}
 void __hipRegisterFunction(void **, const void * f, char *, const char * name, unsigned, void *, void *, void *, void *, int *) { names()[f] = name; }
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 g, dim3, size_t, hipStream_t) { grid_x = g.x; return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 * g, dim3 * b, size_t * sh, hipStream_t * st) { *g = dim3(1); *b = dim3(1); *sh = 0; *st = nullptr; return hipSuccess; }
 hipError_t hipLaunchKernel(const void * f, dim3, dim3, void **, size_t, hipStream_t) {
     ++counts[names()[f]];

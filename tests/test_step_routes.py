@@ -1,0 +1,31 @@
+"""How one token's step goes through its matrices, on the CPU (fake_hip): by streams of rows where these are the faster way, in tiles where those are."""
+import fake_hip
+
+CALLS = """
+from powerinfer_amd import lib as pl
+L, P = pl.load(), 1 << 20
+def closing(rows, ld_att, top=0, ld_act=0, T=1):
+    s = pl.LayerOut()
+    s.rows, s.T, s.out = rows, T, P
+    if ld_att:
+        s.wo, s.att, s.ld_att = P, P, ld_att
+    if top:
+        s.down, s.act, s.ids, s.ld_act, s.top, s.n_expert = P, P, P, ld_act, top, 8
+    F.fake_clear_counts()
+    assert L.pi_k_layer_out_step(C.byref(s), None) == 0
+    return count("layer_out_one"), count("layer_out_step")
+def first(top, ff, cols, T=1):              # workgroups; ff gate rows and as many up rows
+    assert L.pi_k_mix_up_step(None, None, P, 8, ff, cols, 0.9, 1.7, P, T, P, P, top, P, (ff + 31) // 32 * 32, None) == 0
+    return F.fake_grid()
+"""
+
+
+def test_first_matrices_of_experts():
+    fake_hip.run(CALLS + """
+tiles = lambda top, ff: (2 * ff + 15) // 16 * top
+for top, ff, cols in ((1, 16, 2048), (6, 704, 2048), (8, 959, 2048), (1, 3072, 2048), (1, 4097, 2048), (1, 7680, 2048), (6, 1408, 1024), (6, 1408, 5120)):
+    assert first(top, ff, cols) == tiles(top, ff), (top, ff, cols)
+for top, ff, cols, want in ((8, 1024, 2048, 512), (6, 1408, 2048, 512), (1, 7681, 2048, 512), (1, 3073, 2048, 512), (4, 1024, 2048, 512), (1, 1, 4096, 1), (6, 1408, 4096, 512), (2, 64, 8192, 128)):
+    assert first(top, ff, cols) == want, (top, ff, cols)
+assert first(6, 1408, 4096, T=2) == 2 * tiles(6, 1408)
+""")
