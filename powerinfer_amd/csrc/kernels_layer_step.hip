@@ -663,8 +663,16 @@ int pi_k_layer_out_step(const pi_layer_out * a, pi_stream_t stream) {
     // eight waves a workgroup when every workgroup has a compute unit to itself, four (and several workgroups a unit) beyond
     // Eight rows a workgroup (half of each matrix tile repeats them) while 16 would leave half the units without one.
     const int n = (a->rows + 15) / 16, cus = pi::compute_units();
-    const int pieces = ((a->wo ? a->ld_att / 8 : 0) + (a->ids ? a->top * (a->ld_act / 8) : 0) + 511) / 512, per = cus > 0 ? (a->rows + cus - 1) / cus : kOneRows + 1;
-    if (a->T == 1 && pieces <= kOnePieces && per <= kOneRows) {
+    // One token goes by streams of rows from a second piece for some threads on: up to 4096 columns (W_o's and the experts' together) part of a workgroup has
+    // none, and the tiles are the faster ones where the matrix is small.  With experts, which the tiles look up first, streams pay from there down
+    // to 3072 columns; with 4096 for more than 2048 rows, except where the tiles are two for every unit; and with more rows than that from 2048 columns on.
+    // us, tiles / streams: 2048 x 2048 4.8 / 5.9, 2048 x 4096 7.0 / 7.4, 4096 x 1024 4.4 / 5.7, 4096 x 3072 7.2 / 7.5, 8192 x 4096 15.7 / 16.4; 2048 x (2048 + 2 x
+    // 256) 6.2 / 6.3; 2048 x (2048 + 2 x 704) 6.9 / 6.7, 4096 x 4096 9.8 / 8.5, 12288 x 2048 15.0 / 12.8, 1024 x 6144 7.2 / 6.3, 2048 x 6144 8.3 / 7.2, 5120 x
+    // 12288 29.2 / 21.9.
+    const int columns = (a->wo ? a->ld_att : 0) + (a->ids ? a->top * a->ld_act : 0);
+    const int pieces = (columns / 8 + 511) / 512, per = cus > 0 ? (a->rows + cus - 1) / cus : kOneRows + 1;
+    const bool streams = columns > (a->ids ? 3072 : 4096) || (columns == 4096 && a->rows > 2048 && n != 2 * cus) || (columns >= 2048 && n > 2 * cus);
+    if (a->T == 1 && streams && pieces <= kOnePieces && per <= kOneRows) {
         const dim3 grid((a->rows + per - 1) / per);
         switch (pieces) {
             case 1: hipLaunchKernelGGL(layer_out_one_kernel<1>, grid, dim3(512), 0, (hipStream_t)stream, *a, per); break;

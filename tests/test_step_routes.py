@@ -20,6 +20,16 @@ def first(top, ff, cols, T=1):              # workgroups; ff gate rows and as ma
 """
 
 
+def test_closing_a_layer():
+    fake_hip.run(CALLS + """
+for a in ((2049, 4096), (4096, 4096), (12288, 4096), (1, 4128), (256, 6144), (8192, 4128), (4096, 11008), (2048, 2048, 6, 1408), (4096, 2048, 2, 1024), (4096, 4096, 8, 2048),
+          (2048, 2048, 2, 704), (1024, 1056, 2, 1024), (12288, 2048)):
+    assert closing(*a) == (1, 0), a
+for a in ((4096, 4064), (2048, 4096), (8192, 4096), (2048, 2048), (64, 64), (256, 256, 8, 128), (1024, 1024, 4, 512), (1024, 1024, 2, 1024), (8192, 3072), (12288, 2016), (16385, 6144), (4096, 32768), (4096, 4096, 6, 1408, 2)):
+    assert closing(*a) == (0, 1), a
+""")
+
+
 def test_first_matrices_of_experts():
     fake_hip.run(CALLS + """
 tiles = lambda top, ff: (2 * ff + 15) // 16 * top
