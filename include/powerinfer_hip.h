@@ -370,6 +370,10 @@ PI_API int pi_k_batch_sparse_ffn_q4(const float * logits, int T, int ff, float t
 PI_API int pi_k_ffn_wide_supported(int ff, int cols);
 PI_API int pi_k_ffn_wide_f16(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, float threshold,
                              void * h_f16, pi_stream_t stream);
+/* The same under a predictor whose second product fc2[ff][rank] by hid_f16[T][rank] is formed here and leaves bits instead of logits: rank as cols there (what
+ * _supported(ff, rank) says).  mask: ceil(T / 16) * ff / 16 * 32 bytes on 16; bit l of word r of a tile of 16 tokens and 16 neurons is token l % 16, neuron 4 * (l / 16) + r. */
+PI_API int pi_k_ffn_wide_predicted_f16(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols,
+                                       const void * xn_f16, int T, float threshold, void * mask, void * h_f16, pi_stream_t stream);
 PI_API int pi_k_ffn_h_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream);
 PI_API int pi_k_transpose_f16(const void * in_f16, int rows, int cols, void * out_f16, pi_stream_t stream);
 

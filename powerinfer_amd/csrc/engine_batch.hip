@@ -544,7 +544,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     if (!bits) PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
     if (!one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_UP, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out));
     if (!falcon && !one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_GATE, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out));
-    if (bits) PI_TRY(pi::ffn_wide_predicted(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, st));
+    if (bits) PI_TRY(pi_k_ffn_wide_predicted_f16(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, st));
     else if (one_kernel) PI_TRY(pi_k_ffn_wide_f16(up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, b->pred_logits, hp.sparse_threshold, b->h16, st));
     else if (down_ol) PI_TRY(pi_k_ffn_h_q8_f16_ol(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));

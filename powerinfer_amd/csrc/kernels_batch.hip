@@ -1451,23 +1451,6 @@ static int ffn_wide(const void * up_f16, const void * gate_f16, int ff, int cols
     return gate_f16 ? launch(yes, no) : launch(no, no);
 }
 
-namespace pi {
-// the predictor's second product [ff][rank] by hid [T][rank] and, under its bits, the FFN's first half as pi_k_ffn_wide_f16; mask: (T + 15) / 16 * ff / 16 * 4 words
-int ffn_wide_predicted(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold,
-                       void * mask, void * h_f16, hipStream_t st) {
-    if (!fc2_f16 || !hid_f16 || !mask || T <= 0 || !pi_k_ffn_wide_supported(ff, rank) || (((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)mask) & 15) != 0)
-        return fail(PI_E_ARG, "ffn_wide_predicted: bad arguments");
-    const long long units = (long long)((ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
-    if (units > (1 << 30)) return fail(PI_E_ARG, "ffn_wide_predicted: too many tiles");
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&mask_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
-    if (raised != hipSuccess) return hip_fail(raised, "mask_wide: LDS size");
-    hipLaunchKernelGGL(mask_wide_kernel, dim3(wide_blocks(units)), dim3(512), kGwLds, st, MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, (unsigned long long *)mask, ff, rank,
-                       T, rank / kGtBK});
-    if (const int rc = check_launch("mask_wide")) return rc;
-    return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, nullptr, (const unsigned long long *)mask, threshold, h_f16, st);
-}
-}  // namespace pi
-
 extern "C" {
 
 int pi_k_gemm_tile_f16(const void * W, int rows, int cols, const void * xn_f16, int T, int epilogue, const float * add1, const float * add2,
@@ -1490,6 +1473,21 @@ int pi_k_ffn_wide_supported(int ff, int cols) { return ff > 0 && ff % 128 == 0 &
 int pi_k_ffn_wide_f16(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, float threshold, void * h_f16, pi_stream_t stream) {
     if (!logits) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_f16: bad arguments");
     return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, logits, nullptr, threshold, h_f16, stream);
+}
+
+int pi_k_ffn_wide_predicted_f16(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T,
+                                float threshold, void * mask, void * h_f16, pi_stream_t stream) {
+    if (!fc2_f16 || !hid_f16 || !mask || T <= 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_predicted_f16: bad arguments");
+    if (!pi_k_ffn_wide_supported(ff, rank)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_ffn_wide_predicted_f16: ff must be a multiple of 128, the rank a multiple of 64 and at least 256");
+    if ((((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)mask) & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_predicted_f16: operands must be 16-byte aligned");
+    const long long units = (long long)((ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
+    if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_predicted_f16: too many tiles");
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&mask_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
+    if (raised != hipSuccess) return pi::hip_fail(raised, "mask_wide: LDS size");
+    hipLaunchKernelGGL(mask_wide_kernel, dim3(wide_blocks(units)), dim3(512), kGwLds, (hipStream_t)stream,
+                       MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, (unsigned long long *)mask, ff, rank, T, rank / kGtBK});
+    if (const int rc = pi::check_launch("mask_wide")) return rc;
+    return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, nullptr, (const unsigned long long *)mask, threshold, h_f16, stream);
 }
 
 int pi_k_ffn_h_q8_f16(const float * up, const float * gate, const float * logits, float threshold, int T, int ff, void * h_f16, pi_stream_t stream) {

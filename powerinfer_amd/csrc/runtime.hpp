@@ -53,9 +53,6 @@ int expert_relu2_step(const void * up, int n_expert, int ff, int cols, const voi
                       pi_stream_t stream);
 // the embedding row of a token that the host names; also writes the token loop's state (token, position, step counter 0)
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
-// pi_k_ffn_wide_f16 under a predictor whose second product [ff][rank] by hid_f16 [T][rank] leaves bits instead of logits (rank as cols there)
-int ffn_wide_predicted(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold,
-                       void * mask, void * h_f16, hipStream_t st);
 // the embedding rows of tokens that the host names, at positions from `pos` on, and these positions
 int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream);
 

@@ -185,6 +185,7 @@ _SIGS = {
     "pi_k_gemm_tile_bf16": (_i, [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
     "pi_k_ffn_wide_supported": (_i, [_i, _i]),
     "pi_k_ffn_wide_f16": (_i, [_vp, _vp, _i, _i, _vp, _i, _vp, _f, _vp, _vp]),
+    "pi_k_ffn_wide_predicted_f16": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _vp, _i, _f, _vp, _vp, _vp]),
     "pi_k_ffn_h_f16": (_i, [_vp, _vp, _vp, _f, _i, _i, _vp, _vp]),
     "pi_k_transpose_f16": (_i, [_vp, _i, _i, _vp, _vp]),
     "pi_k_norm_q8_round_f16": (_i, [_vp, _i, _i, C.POINTER(Norm), _vp, _vp, _vp]),

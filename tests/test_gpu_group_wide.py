@@ -102,3 +102,45 @@ def test_sparse_ffn_of_a_chunk(ff, cols, T, gated):
     want = np.where(~(lg < 0.25), np.maximum(g, 0) * u if gated else np.maximum(u, 0), 0)
     assert (got[lg < 0.25] == 0).all()
     assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 1e-5 * np.abs(want).max() + 2.0 ** -25).all()
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("ff,rank,cols,T", [(128, 256, 256, 1), (384, 320, 256, 15), (128, 256, 320, 16), (256, 1024, 256, 17), (640, 256, 256, 64), (384, 256, 512, 65), (2176, 320, 256, 128),
+                                            (640, 512, 256, 129), (1152, 256, 256, 301), (4352, 256, 256, 3000)])
+def test_sparse_ffn_under_bits(ff, rank, cols, T, gated):
+    """The predictor's second product leaves bits: factors are small whole numbers, whose sums fp32 holds exactly in any order, so that thresholds are met exactly
+    (active) and missed by one; a token whose hidden vector has a NaN is active everywhere, infinite ones as their sums say.  The bits are
+    float64's; h is bounded as above."""
+    L, rng = pl.init(), np.random.default_rng(ff + T + rank)
+    up, gate, x = ((rng.standard_normal(s) / np.sqrt(s[1]) ** (s[0] != T)).astype(np.float16) for s in ((ff, cols), (ff, cols), (T, cols)))
+    fc2, hid = rng.integers(-3, 4, (ff, rank)).astype(np.float16), rng.integers(0, 3, (T, rank)).astype(np.float16)
+    fc2[:, 5] = np.where(fc2[:, 5] == 0, 1, fc2[:, 5])
+    if T > 2:
+        hid[1, 7], hid[T - 1, 5] = np.nan, np.inf
+    lg = (hid.astype(np.float64) @ fc2.astype(np.float64).T).astype(np.float32)
+    thr = float(np.sort(lg[0])[ff // 2])
+    active = ~(lg < thr)
+    assert (lg[0] == thr).any() and active.any() and not active.all()
+    b = [dev(a) for a in (fc2, hid, up, gate, x)]
+    h, mask = pl.DevBuf(2 * T * ff + 64), pl.DevBuf((T + 15) // 16 * ff * 2 + 64)
+    for d in (h, mask):
+        pl.check(L.pi_memset(d.ptr, 0xAB, d.nbytes))
+    print(ff, rank, cols, T, gated, flush=True)
+    pl.check(L.pi_k_ffn_wide_predicted_f16(b[0].ptr, rank, b[1].ptr, b[2].ptr, b[3].ptr if gated else None, ff, cols, b[4].ptr, T, thr, mask.ptr, h.ptr, None))
+    pl.sync()
+    words, raw = mask.download(np.uint64), h.download(np.float16)
+    assert (words[-8:] == 0xABABABABABABABAB).all() and (raw[T * ff:].view(np.uint16) == 0xABAB).all()
+    bits = (words[:-8].reshape(-1, ff // 16, 4, 1) >> np.arange(64, dtype=np.uint64) & np.uint64(1)).reshape(-1, ff // 16, 4, 4, 16)      # [tile][neurons][r][l / 16][token]
+    assert np.array_equal(bits.transpose(0, 4, 1, 3, 2).reshape(-1, ff)[:T] != 0, active)
+    got = raw[:T * ff].reshape(T, ff).astype(np.float64)
+    u, g = (x.astype(np.float64) @ w.T.astype(np.float64) for w in (up, gate))
+    want = np.where(active, np.maximum(g, 0) * u if gated else np.maximum(u, 0), 0)
+    assert (got[~active] == 0).all()
+    assert (np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 1e-5 * np.abs(want).max() + 2.0 ** -25).all()
+
+
+def test_what_products_under_bits_refuse():
+    L = pl.init()
+    d = pl.DevBuf.zeros(1 << 20)
+    call = lambda rank=256, ff=128, cols=256, fc2=d.ptr, mask=d.ptr, T=3: L.pi_k_ffn_wide_predicted_f16(fc2, rank, d.ptr, d.ptr, None, ff, cols, d.ptr, T, 0.0, mask, d.ptr, None)  # noqa: E731
+    assert call(rank=128) != 0 and call(ff=64) != 0 and call(rank=300) != 0 and call(T=0) != 0 and call(fc2=d.ptr + 8) != 0 and call(mask=None) != 0 and call(mask=d.ptr + 8) != 0
