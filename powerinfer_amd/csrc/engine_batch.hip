@@ -496,6 +496,15 @@ bool ffn_in_one(pi_model * m, int il) {
            (((uintptr_t)up.dev | (m->hp.arch == PI_ARCH_FALCON ? 0 : (uintptr_t)gate.dev)) & 15) == 0;
 }
 bool ffn_large(pi_model * m) { return (long long)m->hp.n_ff * m->hp.n_embd > 48LL << 20; }
+// Bits instead of logits between the predictor and such a kernel (pi_k_ffn_wide_predicted_f16).  The product that leaves them has tiles of 256 x 128 alone, which are
+// few for a short chunk: a token tile or less of smaller matrices takes the library's plan and logits.  Both products and the FFN, us, logits / bits: 11008
+// x 4096 of rank 1024, 17 tokens 60 / 62, 64 62 / 65, 128 65 / 69, 129 71 / 68, 400 116 / 111; 4096 x 1024 of rank 256, 64 tokens 16.2 / 17.1, 400 22.0 / 18.7;
+// 13824 x 5120, 128 tokens 105 / 104; 32768 x 8192, 128 tokens 167 / 152.
+constexpr int kBitsRows = 128;
+bool ffn_bits(pi_model * m, int il, int T) {
+    const Tensor & fc2 = m->L(il, PI_T_FC2);
+    return (T > kBitsRows || ffn_large(m)) && pi_k_ffn_wide_supported(m->hp.n_ff, (int)m->L(il, PI_T_FC1).ne1) && ((uintptr_t)fc2.dev & 15) == 0;
+}
 
 int wide_layer(pi_model * m, BatchState * b, int il) {
     const pi_hparams & hp = m->hp;
@@ -540,7 +549,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
         else ffn_x = b->xa16;
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
-    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && pi_k_ffn_wide_supported(ff, r) && ((uintptr_t)fc2.dev & 15) == 0;
+    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, T);
     if (!bits) PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
     if (!one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_UP, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out));
     if (!falcon && !one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_GATE, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out));

@@ -577,7 +577,7 @@ template <bool PAIRS, bool MASK> struct FfnProduct {
 };
 // The predictor's second product, of which that is all anybody reads: 2047 tokens of 11008 neurons are 2.8 MB of bits instead of 90 of logits, written here
 // and read by the FFN's first half.  Four 7B-shaped layers, us, library product with logits and this: 2047 tokens 3829 -> 3696, 600 1692 -> 1665, 300 1318 ->
-// 1285, 131 1055 -> 1031, 100 957 -> 949; 13B 400 tokens 1408 -> 1378, 40B 700 tokens 1550 -> 1531.
+// 1285; 13B 400 tokens 1408 -> 1378, 40B 700 tokens 1550 -> 1531.
 struct MaskProduct {
     static constexpr bool kPairs = false;
     const __half * W, * x; float thr; unsigned long long * mask;

@@ -75,3 +75,14 @@ for off in (0, 8):
     assert (count("ffn_wide"), count("ffn_h_f16")) == ((hp.n_layer, 0) if off == 0 else (0, hp.n_layer)), off
     m.close()
 """)
+
+
+def test_chunks_whose_predictors_leave_bits():
+    """Longer than one token tile; shorter ones, for which its tiles are too few, take the library's product and logits."""
+    fake_hip.run(MODEL + """
+m, hp = made()
+for n, bits in ((30, 0), (129, 0), (130, 1), (600, 1)):
+    prompt(m, n)
+    assert (count("mask_wide") > 0) == bits and count("ffn_wide") > 0, n
+m.close()
+""")
