@@ -185,15 +185,16 @@ int batch_layer_q4(pi_model * m, BatchState * b, int il) {
     else if (m->L(il, PI_T_ATTN_NORM_2).dev) an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
     // (the predictor's fp16 inputs, xp16 and hid16, are kept in the operand layout of the 16-token fp16 mat-muls)
-    PI_TRY(pi_k_norm_q8_blocks_ol(x, T, d, &an, b->qa, b->da, b->sa, falcon ? b->xp16 : nullptr, st));   // Falcon: the predictor reads the layer input as plain fp16
+    const bool cells = b->prefill && cells_only(m, il);
+    PI_TRY(pi_k_norm_q8_blocks_ol(x, T, d, &an, b->qa, b->da, b->sa, falcon && !cells ? b->xp16 : nullptr, st));   // Falcon: the predictor reads the layer input as plain fp16
+    const auto wqkv = W(PI_T_WQKV), wo = W(PI_T_WO);
+    PI_TRY(pi_k_gemm_q4_t16(wqkv.quants, wqkv.scales, d + 2 * gqa, d, b->qa, b->da, b->sa, T, PI_EPI_NONE, nullptr, nullptr, b->qkv, st));
+    if (cells) return chunk_store(m, b, b->qkv + d, d + 2 * gqa, kv_off);
     if (falcon) {
         // the FFN branch reads the layer input too, under its own norm (with a single norm: the attention's)
         pi_norm fn = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         PI_TRY(pi_k_norm_q8_blocks(x, T, d, m->L(il, PI_T_ATTN_NORM_2).dev ? &fn : &an, b->qf, b->df, b->sf, nullptr, st));
     }
-    const auto wqkv = W(PI_T_WQKV), wo = W(PI_T_WO);
-    PI_TRY(pi_k_gemm_q4_t16(wqkv.quants, wqkv.scales, d + 2 * gqa, d, b->qa, b->da, b->sa, T, PI_EPI_NONE, nullptr, nullptr, b->qkv, st));
-    if (b->prefill && cells_only(m, il)) return chunk_store(m, b, b->qkv + d, d + 2 * gqa, kv_off);
     if (b->unified)
         PI_TRY(cells_attention(m, b, il, T));
     else if (b->prefill)
@@ -258,8 +259,9 @@ int batch_layer(pi_model * m, BatchState * b, int il) {
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
     // the fp16 inputs of the step's mat-muls (xa16, xf16, xp16, hid16, and att16 of a lockstep step) are kept in the matrix cores'
     // operand layout; the attention of a prompt chunk and of the shared-cell cache write att16 token-major
-    PI_TRY(pi_k_norm_round_f16_ol(x, T, d, &an, b->xa16, falcon ? b->xp16 : nullptr, st));    // Falcon: the predictor reads the raw layer input
-    if (b->prefill && cells_only(m, il)) {                            // (the rows of k and v)
+    const bool cells = b->prefill && cells_only(m, il);
+    PI_TRY(pi_k_norm_round_f16_ol(x, T, d, &an, b->xa16, falcon && !cells ? b->xp16 : nullptr, st));    // Falcon: the predictor reads the raw layer input
+    if (cells) {                                                      // (the rows of k and v)
         PI_TRY(pi_k_gemm_f16_ol((const __half *)wqkv.dev + (size_t)d * d, 2 * gqa, d, b->xa16, T, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr, st));
         return chunk_store(m, b, b->qkv, 2 * gqa, kv_off);
     }
@@ -375,7 +377,8 @@ bool step_buffers(pi_model * m, BatchState * b, int T, bool with_caches) {
     const size_t n16 = n < 16 ? 16 : n;                            // steps of up to 16 tokens keep these in the operand layout: 16 token slots
     b->xa16 = m->alloc<__half>(n16 * d); b->xf16 = m->alloc<__half>(n16 * d); b->xp16 = m->alloc<__half>(n16 * d);
     b->att16 = m->alloc<__half>(n16 * d); b->hid16 = m->alloc<__half>(n16 * r);
-    b->d_tokens = m->alloc<int32_t>(n); b->d_pos = m->alloc<int32_t>(n); b->d_step = m->alloc<int32_t>(1);
+    b->d_tokens = b->prefill ? nullptr : m->alloc<int32_t>(n);       // (a prompt chunk's travel as kernel arguments)
+    b->d_pos = m->alloc<int32_t>(n); b->d_step = m->alloc<int32_t>(1);
     b->d_out_tokens = m->alloc<int32_t>((size_t)b->max_steps * (n > 16 ? 1 : n)); b->union_rows = m->alloc<int32_t>(ff); b->n_union = m->alloc<int32_t>(hp.n_layer);
     if (m->L(0, PI_T_WQKV).type == PI_TYPE_Q4_0 && d % 32 == 0) {          // steps of a Q4_0 model on integer matrix cores
         b->qa = m->alloc<unsigned char>((size_t)16 * d); b->qf = m->alloc<unsigned char>((size_t)16 * d);
@@ -392,10 +395,11 @@ bool step_buffers(pi_model * m, BatchState * b, int T, bool with_caches) {
         b->dense_ffn.assign(hp.n_layer, 0);
     }
     return ok && b->x && b->x2 && b->qkv && b->att && b->attn_out && b->ffn_inp && b->hidden && b->pred_logits && b->logits && b->xa16 && b->xf16 && b->xp16 && b->att16 && b->hid16 &&
-           b->d_tokens && b->d_pos && b->d_step && b->d_out_tokens && b->union_rows && b->n_union;
+           (b->prefill || b->d_tokens) && b->d_pos && b->d_step && b->d_out_tokens && b->union_rows && b->n_union;
 }
-BatchState * batch_alloc(pi_model * m, int T, bool with_caches) {
+BatchState * batch_alloc(pi_model * m, int T, bool with_caches, bool prefill = false) {
     BatchState * b = new BatchState();
+    b->prefill = prefill;
     if (step_buffers(m, b, T, with_caches)) return b;
     delete b;
     return nullptr;
@@ -525,7 +529,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     if (!falcon) an = mk_norm(1, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), nullptr);
     else if (m->L(il, PI_T_ATTN_NORM_2).dev) an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
-    PI_TRY(chunk_input(wqkv.type, qkv_ol, x, T, d, &an, b->xa16, falcon ? b->xp16 : nullptr, st));
+    PI_TRY(chunk_input(wqkv.type, qkv_ol, x, T, d, &an, b->xa16, falcon && !wide_cells_only(m, il) ? b->xp16 : nullptr, st));
     if (wide_cells_only(m, il) && wqkv.type == PI_TYPE_F16) {              // the rows of k and v (a Q4_0 matrix: all of them, in the order of sums of every other layer)
         PI_TRY(chunk_gemm(m, b, (const __half *)wqkv.dev + (size_t)d * d, 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr));
         return chunk_store(m, b, b->qkv, 2 * gqa, kv_off);
@@ -777,9 +781,8 @@ int prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
     if (T < 1 || T > 16) return pi::fail(PI_E_ARG, "prefill_chunk: 1 <= T <= 16");
     if (batch_unsupported(m) != nullptr) PI_TRY(ensure_q4_split(m));          // a Q4_0 model: the integer matrix-core route
     if (!m->prefill) {
-        m->prefill = batch_alloc(m, 16, false);
+        m->prefill = batch_alloc(m, 16, false, true);
         if (!m->prefill) return PI_E_HIP;
-        m->prefill->prefill = true;
     }
     BatchState * b = m->prefill;
     b->n_seq = T;

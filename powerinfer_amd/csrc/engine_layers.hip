@@ -1032,7 +1032,7 @@ int one_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in,
 // The residual gate's rows are a product of their own then.  A whole pass of four layers of 11008 neurons, us, apart and in one: 300 tokens 1422 / 1517, 1024
 // 2689 / 2717, 1280 3195 / 3248, 1400 3519 / 3441, 2043 4918 / 4665; of 5632 neurons, 1200 1526 / 1522, 1400 1612 / 1593.
 bool glu_in_one(pi_model * m, const Layer & L, int T) {
-    return bf16_mode(m->lay) && T >= kGluInOne && L.glu_ld == L.d.glu_ff && L.off_gate_ffn >= 2 * L.d.glu_ff;
+    return bf16_mode(m->lay) && T >= kGluInOne && L.glu_ld == L.d.glu_ff;
 }
 
 // A layer whose norms come after the sums.  Steps of up to 16 tokens (bf16): joint projection, what lies behind it (queries and cells beside the

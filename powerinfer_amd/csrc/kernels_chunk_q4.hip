@@ -293,8 +293,8 @@ template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hip
 }
 
 // Tiles as 100 * (16-row tiles) + 10 * (16-token tiles a wave) + waves
-// (634 is there for a caller that asks for it: one round of it takes as long as two of 333 or 334, two workgroups of which share a unit.  17 to 24
-// token tiles of 7B shapes went there: 11008 x 4096, us, 280 tokens 53.3 -> 36.7, 360 tokens 55.0 -> 42.2; 12288 x 4096 54.3 -> 39.9)
+// (no 96 rows with three token tiles for each of four waves: one round of that takes as long as two of 333 or 334, two workgroups of which share a
+// unit.  17 to 24 token tiles of 7B shapes: 11008 x 4096, us, 280 tokens 53.3 / 36.7, 360 tokens 55.0 / 42.2; 12288 x 4096 54.3 / 39.9)
 constexpr int kCqTiles[] = {112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624};
 constexpr int kCqTilesT[] = {212, 213, 215, 223, 422, 423, 424, 434};
 // What a launch takes goes with the rounds of workgroups over the compute units times what 32 columns of a tile take of a unit, in clocks: the
@@ -338,7 +338,7 @@ int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, co
     if (!transposed) {
         switch (tile) {
             PI_CQ1(1, 1, 2); PI_CQ1(1, 2, 2); PI_CQ1(1, 2, 3); PI_CQ1(2, 1, 5); PI_CQ1(2, 3, 2); PI_CQ1(3, 1, 4); PI_CQ1(3, 2, 3); PI_CQ1(3, 3, 3);
-            PI_CQ1(3, 3, 4); PI_CQ1(4, 1, 4); PI_CQ1(4, 2, 3); PI_CQ1(4, 2, 4); PI_CQ1(6, 2, 4); PI_CQ1(6, 3, 4); PI_CQ1(4, 3, 4); PI_CQ1(4, 4, 4);
+            PI_CQ1(3, 3, 4); PI_CQ1(4, 1, 4); PI_CQ1(4, 2, 3); PI_CQ1(4, 2, 4); PI_CQ1(6, 2, 4); PI_CQ1(4, 3, 4); PI_CQ1(4, 4, 4);
         }
     } else {
         switch (tile) {

@@ -9,7 +9,7 @@ from powerinfer_amd import lib as pl
 from powerinfer_amd import synth
 
 pytestmark = pytest.mark.gpu
-TILES = {0: [112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624, 634], 1: [212, 213, 215, 223, 422, 423, 424, 434]}
+TILES = {0: [112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624], 1: [212, 213, 215, 223, 422, 423, 424, 434]}
 
 
 def operand_layout(x):
