@@ -1,5 +1,5 @@
 """One token's experts by streams of rows: first matrices of 2048, 4096 and 8192 columns, with fewer rows than workgroups, experts that end within a
-workgroup's rows, and beside the launch's other parts - the operators' own comparisons at these sizes."""
+workgroup's rows, sizes of 2048 columns that go in tiles, and beside the launch's other parts - the operators' own comparisons at these sizes."""
 import ctypes as C
 
 import numpy as np
@@ -19,12 +19,12 @@ def test_beside_merges_and_gates(E, top, ff, cols, what):
     test_gpu_gqa_ops.test_step_launch_beside_the_experts(1, E, top, ff, cols, what)
 
 
-@pytest.mark.parametrize("E,top,ff,cols", [(7, 6, 171, 4096), (4, 3, 700, 2048), (3, 2, 65, 8192)])
+@pytest.mark.parametrize("E,top,ff,cols", [(7, 6, 171, 4096), (4, 3, 700, 2048), (4, 3, 1101, 2048), (3, 2, 65, 8192)])
 def test_weighted_at_their_input(E, top, ff, cols):
     test_gpu_pufivik_ops.test_experts_of_a_step(1, E, top, ff, cols)
 
 
-@pytest.mark.parametrize("E,top,ff,D", [(5, 3, 403, 2048), (4, 4, 129, 4096)])
+@pytest.mark.parametrize("E,top,ff,D", [(5, 3, 403, 2048), (5, 3, 2403, 2048), (4, 4, 129, 4096)])
 def test_squared_beside_values(E, top, ff, D):
     test_gpu_latent_ops.test_step_kernels(1, 4, 16, 8, 24, 40, E, top, ff, D, 4)
 

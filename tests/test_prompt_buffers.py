@@ -86,3 +86,23 @@ for n, bits in ((30, 0), (129, 0), (130, 1), (600, 1)):
     assert (count("mask_wide") > 0) == bits and count("ffn_wide") > 0, n
 m.close()
 """)
+
+
+def test_dense_feed_forwards_in_one_product():
+    """From 1400 tokens on, where the rows of gate and up come in tiles of 128: gate, up and GLU are one product a layer (test_gpu_glu_in_one.py has
+    these passes on the GPU).  Padded ones and shorter passes go apart."""
+    fake_hip.run("""
+import fikevik_models as fm
+from lerasun_models import tokens
+from powerinfer_amd import fikevik
+for ff, whole in ((128, 1), (192, 0), (256, 1), (320, 0), (384, 1)):
+    cfg = fm.config(256, 200, [fm.gla(2, 64, 64, mlp=fm.dense(ff)), fm.gla(4, 32, 64, mlp=fm.dense(ff))])
+    m = fikevik.build(cfg, fm.weights(cfg, 5), n_ctx=2048, max_batch=2048)
+    m.kv_cells_init(2048)
+    for n in (1399, 1400, 1537):
+        F.fake_clear_counts()
+        m.kv_cells_step(tokens(cfg, n, 3), range(n), [1] * n, list(range(17)))
+        assert count("group_wide") == (2 if whole and n >= 1400 else 0), (ff, n)
+        m.kv_cells_clear()
+    m.close()
+""")
