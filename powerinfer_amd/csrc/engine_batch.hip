@@ -93,14 +93,10 @@ int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size
 }
 
 // A prompt chunk leaves nothing of the last layer but its keys and values: its tokens' logits are nobody's, and the token that ends the prompt goes
-// through the layer by itself.  What lies behind the store is not formed (eight 7B-shaped layers: 2046 F16 tokens 9.19 -> 8.29 ms, 130 Q4_0 tokens
-// 2.09 -> 1.91).
+// through the layer by itself.  What lies behind the store is not formed, which is one layer's share of a prompt and the less the deeper the model: eight
+// 7B-shaped layers, 2046 F16 tokens 9.19 -> 8.29 ms, 130 Q4_0 tokens 2.09 -> 1.91; 32 of them, 1024 F16 tokens 20.89 -> 20.49; three of
+// 512 x 4096, 200 tokens 391 -> 335 us.
 bool cells_only(const pi_model * m, int il) { return il == m->hp.n_layer - 1; }
-// The same for wide chunks, of layers whose FFN matrices have 4 M weights or more.  Smaller ones, test models among them, go through whole as the others do:
-// the tests of the routes count a chunk's launches layer by layer (512 x 4096, three layers: 200 tokens 391 us, and 335 without the
-// last; the step kernels' chunks of 16 tokens have no such line).
-constexpr long long kWideCells = 4 << 20;
-bool wide_cells_only(const pi_model * m, int il) { return cells_only(m, il) && (long long)m->hp.n_embd * m->hp.n_ff >= kWideCells; }
 // kv: the chunk's rows of k | v, `stride` floats apart
 int chunk_store(pi_model * m, BatchState * b, const float * kv, int stride, size_t kv_off) {
     const pi_hparams & hp = m->hp;
@@ -529,13 +525,13 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     if (!falcon) an = mk_norm(1, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), nullptr);
     else if (m->L(il, PI_T_ATTN_NORM_2).dev) an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
     else an = mk_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
-    PI_TRY(chunk_input(wqkv.type, qkv_ol, x, T, d, &an, b->xa16, falcon && !wide_cells_only(m, il) ? b->xp16 : nullptr, st));
-    if (wide_cells_only(m, il) && wqkv.type == PI_TYPE_F16) {              // the rows of k and v (a Q4_0 matrix: all of them, in the order of sums of every other layer)
+    PI_TRY(chunk_input(wqkv.type, qkv_ol, x, T, d, &an, b->xa16, falcon && !cells_only(m, il) ? b->xp16 : nullptr, st));
+    if (cells_only(m, il) && wqkv.type == PI_TYPE_F16) {              // the rows of k and v (a Q4_0 matrix: all of them, in the order of sums of every other layer)
         PI_TRY(chunk_gemm(m, b, (const __half *)wqkv.dev + (size_t)d * d, 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv, nullptr));
         return chunk_store(m, b, b->qkv, 2 * gqa, kv_off);
     }
     PI_TRY(chunk_product(m, b, il, PI_T_WQKV, qkv_ol, d + 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv));
-    if (wide_cells_only(m, il)) return chunk_store(m, b, b->qkv + d, d + 2 * gqa, kv_off);
+    if (cells_only(m, il)) return chunk_store(m, b, b->qkv + d, d + 2 * gqa, kv_off);
     PI_TRY(in_pieces(b, [&](int t0, int n) { return chunk_attention(m, b, t0, n, b->kv_hi - (T - t0 - n), kv_off); }));
     if (wo.type == PI_TYPE_Q4_0) PI_TRY(chunk_input(wo.type, wo_ol, b->att, T, d, &plain, b->att16, nullptr, st));
     pi_norm fn;
@@ -614,7 +610,7 @@ namespace {
 // queues the copies of layer il's non-resident rows into its staging buffer on the copy stream (after the layer that used the
 // buffer last has finished with it) and marks the buffer; layers that are whole on the device need nothing
 int stage_rest_rows(pi_model * m, BatchState * b, int il) {
-    if (il >= m->hp.n_layer || wide_cells_only(m, il) || !b->copy_stream || !m->L(il, PI_T_GPU_BUCKET).dev) return PI_OK;
+    if (il >= m->hp.n_layer || cells_only(m, il) || !b->copy_stream || !m->L(il, PI_T_GPU_BUCKET).dev) return PI_OK;
     const int s = il & 1;
     const size_t n_rest = (size_t)m->hp.n_ff - (size_t)m->L(il, PI_T_GPU_BUCKET).ne0;
     const size_t rb = m->L(il, PI_T_FFN_UP).type == PI_TYPE_Q4_0 ? (size_t)(m->hp.n_embd / 32) * 18 : (size_t)m->hp.n_embd * 2;
@@ -720,7 +716,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_pas
             if (m->L(il, PI_T_WO).type == PI_TYPE_Q4_0) w16 = std::max(w16, (size_t)hp.n_embd * hp.n_embd);
             if (split || m->L(il, PI_T_FFN_UP).type == PI_TYPE_Q4_0 || m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_Q4_0) w16 = std::max(w16, (size_t)hp.n_ff * hp.n_embd);
             if (split || m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_Q4_0) { scratch = true; continue; }
-            if (!wide_cells_only(m, il)) PI_TRY(ensure_down_rows(m, il));
+            if (!cells_only(m, il)) PI_TRY(ensure_down_rows(m, il));
         }
         if (w16) b->w16 = m->alloc<__half>(w16);
         if (scratch) b->w16t = m->alloc<__half>((size_t)hp.n_embd * hp.n_ff);

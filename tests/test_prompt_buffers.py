@@ -41,16 +41,16 @@ m, hp = made()
 prompt(m, 20)
 at_512 = F.fake_live()
 prompt(m, 2040)
-assert count("attn_chunk_rows") == hp.n_layer
+assert count("attn_chunk_rows") == hp.n_layer - 1               # (of the last layer a chunk leaves its keys and values)
 at_2048 = F.fake_live()
 n, hp = made()
 prompt(n, 20)
 F.fake_limit((at_2048 - at_512) // 2)
 prompt(n, 2040)
-assert count("attn_chunk_rows") == 4 * hp.n_layer, count("attn_chunk_rows")
+assert count("attn_chunk_rows") == 4 * (hp.n_layer - 1), count("attn_chunk_rows")
 F.fake_limit(C.c_size_t(-1).value)
 prompt(n, 2040)                          # memory is there again
-assert count("attn_chunk_rows") == hp.n_layer
+assert count("attn_chunk_rows") == hp.n_layer - 1
 """)
 
 
@@ -72,7 +72,7 @@ for off in (0, 8):
         m.set_tensor_device(il, "ffn_up", p + off, pl.F16, up.shape[1], up.shape[0])
     m.finalize()
     prompt(m, 200)
-    assert (count("ffn_wide"), count("ffn_h_f16")) == ((hp.n_layer, 0) if off == 0 else (0, hp.n_layer)), off
+    assert (count("ffn_wide"), count("ffn_h_f16")) == ((hp.n_layer - 1, 0) if off == 0 else (0, hp.n_layer - 1)), off
     m.close()
 """)
 
