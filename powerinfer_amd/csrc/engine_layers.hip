@@ -796,8 +796,8 @@ int attend_expanded(pi_model * m, const Layer & L, const Layer & src, const Step
 }
 
 // The last layer of a pass: nobody reads more of it than its cells and states and the wanted tokens' stream.  Behind its attention a long pass goes on with
-// those tokens alone, as a step of so few does (four layers, 4096 wide, one token wanted: 2048 tokens with 64 experts of 1408 3.75 -> 3.22 ms, 2460 tokens of
-// gated recurrences 5.69 -> 5.01).
+// those tokens alone, as a step of so few does.  That is a part of one layer, and of a pass the less the deeper the model (one token wanted, 4096 wide, four
+// layers, where it is most: 2048 tokens with 64 experts of 1408 3.75 -> 3.22 ms, 2460 tokens of gated recurrences 5.69 -> 5.01).
 bool tail_of(pi_model * m, const Layer & L, const LayerRun & r, const Step & in, const float * keep) {
     LayerState * s = m->lay;
     return bf16_mode(s) && &r == &s->order.back() && !keep && in.T > kTailRows && in.n_rows >= 0 && in.n_rows <= kTailRows &&

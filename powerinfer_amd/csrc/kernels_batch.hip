@@ -283,8 +283,10 @@ struct SecondGemm { const void * W; const void * x; int rows; float * y; };
 // rows of the first matrix are gate and up rows in turn: out [T][ld] = clamped GLU (instead of y)
 constexpr int kEpiGlu = PI_EPI_ADD2 + 1;
 struct GluOut { void * out; int ld; float limit, gain, one; };
+// (two waves a SIMD: 32 rows and four waves came to 263 registers without that bound, and a unit then holds one workgroup instead of two: 32000 x 4096
+// 46.2 / 42.0 us, 22016 x 4096 34.0 / 31.4)
 template <typename EL, int RT, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_t16_lds_kernel(const EL * __restrict__ W, const EL * __restrict__ xn, int T, int rows, int cols,
+__global__ __launch_bounds__(64 * NW, 2) void gemm_t16_lds_kernel(const EL * __restrict__ W, const EL * __restrict__ xn, int T, int rows, int cols,
                                                                   int epi, const float * __restrict__ add1, const float * __restrict__ add2, float * __restrict__ y,
                                                                   EL * __restrict__ y16, float thr, unsigned char * __restrict__ row_any, int lay, SecondGemm two, GluOut glu) {
     const int n_first = (rows + 16 * RT - 1) / (16 * RT);

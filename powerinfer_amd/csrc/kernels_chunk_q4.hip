@@ -17,12 +17,13 @@ namespace {
 // the weights do (with both operands copied to LDS and every wave expanding its own rows, 130 tokens of 12288 x 4096 took 33 us).
 // A byte under 0x64 is 1024 + it in fp16, so q - 8 takes a permutation, a mask and one FMA for two (exact), and the product with d rounds
 // once, as the float product of the expanding kernels does.
-// The sums go over 32 columns a step in fp32, ascending, in parts that are added at the end: eight of a transposed matrix, two of one with
-// more than twice as many rows as columns, each of whole 128-column slabs, the longer ones first.  They are the parts in which the library's
-// plans add up such matrices of a 7B-shaped model behind 129 .. 139 tokens, so that results stay bit for bit what they were there (an
-// activation that is rounded to eight bits the other way moves logits by 1e-2, and the tests against the CPU path stand that close), and
-// here they are the same at every length.  Error against 64 bits, one sum / parts: 12288 x 4096 4.1e-7 / 2.9e-7, 4096 x 11008
-// transposed 6.7e-7 / 2.4e-7.
+// The sums go over 32 columns a step in fp32, ascending, in parts of whole 128-column slabs, the longer ones first, that are added at the end: eight of a
+// transposed matrix, two of one with more than twice as many rows as columns, at every length and in every tile.  More parts round less:
+// relative error against 64 bits in one / two / four / eight parts, 130 tokens: 4096 x 4096 and 12288 x 4096 4.1e-7 / 2.9e-7 / 2.1e-7 / 1.6e-7,
+// 32768 x 8192 5.7e-7 / 4.1e-7 / 2.9e-7 / 2.1e-7, 4096 x 11008 transposed 5.9e-7 / 4.1e-7 / 3.0e-7 / 2.2e-7, 8192 x 32768 1.02e-6 / 7.2e-7 /
+// 5.1e-7 / 3.6e-7; expanded and multiplied by the library 4.1e-7, 5.7e-7, 5.9e-7 and 6.2e-7.  The longest sums, of the transposed
+// matrices, have the most; one part would be enough elsewhere, and two are kept where results have them: another order of sums rounds
+// activations to eight bits the other way here and there, which moves a model's logits by 1e-2.
 // What bounds it at 130 tokens of 12288 x 4096 (21 us; the blocks alone 5, the matrix instructions 6): about 12 us are launch, first
 // trip and last stores, which one workgroup a unit does not overlap with its products; the rest is shared about evenly between the
 // tokens' way from the L2 (270 MB), expanding and multiplying.
