@@ -356,14 +356,16 @@ __device__ __forceinline__ void expert_up_any(const ExpertUp & a, int b, int n_t
     else if (a.cols == 4096) expert_up_one<2>(a, b, smem);
     else expert_up_one<4>(a, b, smem);
 }
-// Workgroups of the experts' first matrices.  One token of 2048, 4096 or 8192 columns goes by streams.  Of 2048 columns eight rows are one group of requests, and
-// streams pay with 32 rows or more each or where two groups are full or nearly so: below and between, a tile of 16 rows is done in one trip and
-// most tiles side by side, while a stream asks for a group more than it has.  us, tiles / streams, experts x rows: 2048 columns 1 x 32 4.8 / 5.8,
-// 4 x 512 6.3 / 8.5, 2 x 2816 9.3 / 9.5, 4 x 2048 11.1 / 10.1, 6 x 1536 13.1 / 14.2, 6 x 2816 19.5 / 19.5, 8 x 2048 19.9 / 16.2; 4096 columns 1 x 32
+// Workgroups of the experts' first matrices.  One token of 2048, 4096 or 8192 columns goes by streams.  Of 2048 columns a group of requests is eight rows and
+// a stream asks for them two groups at a time, so its time goes with its rows in sixteens, while a tile of 16 rows is done in one trip and most
+// tiles side by side: streams pay from 15 rows each on, where few of the rows asked for are missing.  us, tiles / streams, six experts, by
+// rows a stream: 8 8.8 / 9.6, 14 10.1 / 10.3, 16 11.9 / 10.6, 18 12.7 / 14.5, 24 13.6 / 15.3, 28 17.1 / 16.0, 32 18.7 / 16.6, 34 19.4 / 20.2, 38 20.8 /
+// 20.6, 48 25.0 / 21.6, 50 25.0 / 25.2, 56 27.7 / 25.8, 66 32.0 / 30.3 (6 x 2816 rows are 34 each).  Experts x rows of 4096 columns: 1 x 32
 // 7.2 / 5.0, 4 x 512 9.0 / 8.5, 6 x 2816 30.8 / 25.5; 8192 columns 1 x 32 11.6 / 5.4, 4 x 512 15.2 / 10.7.
 inline int up_blocks(ExpertUp & u, int n_tiles) {
     const int per_unit = u.glu ? 2 : 1, units = u.top * u.ff / per_unit, most = 2 * pi::compute_units(), rows = most > 0 ? (units + most - 1) / most * per_unit : 0;
-    const bool pays = u.cols == 4096 || u.cols == 8192 || (u.cols == 2048 && (rows >= 32 || (rows >= 14 && rows <= 16)));
+    const int missing = (rows + 15) / 16 * 16 - rows;
+    const bool pays = u.cols == 4096 || u.cols == 8192 || (u.cols == 2048 && rows >= 15 && 4 * missing <= rows + 2);
     if (u.T == 1 && most > 0 && pays && rows * 16 <= kUpLds) {
         u.streams = units < most ? units : most;
         return u.streams;

@@ -14,12 +14,12 @@ from powerinfer_amd import lib as pl
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("E,top,ff,cols,what", [(3, 2, 5, 2048, "gate"), (9, 6, 333, 4096, "both"), (2, 1, 514, 8192, "none"), (8, 8, 1027, 2048, "merge"), (1, 1, 1, 4096, "none")])
+@pytest.mark.parametrize("E,top,ff,cols,what", [(3, 2, 5, 2048, "gate"), (9, 6, 333, 4096, "both"), (2, 1, 514, 8192, "none"), (8, 8, 1027, 2048, "merge"), (8, 8, 1501, 2048, "merge"), (1, 1, 1, 4096, "none")])
 def test_beside_merges_and_gates(E, top, ff, cols, what):
     test_gpu_gqa_ops.test_step_launch_beside_the_experts(1, E, top, ff, cols, what)
 
 
-@pytest.mark.parametrize("E,top,ff,cols", [(7, 6, 171, 4096), (4, 3, 700, 2048), (4, 3, 1101, 2048), (3, 2, 65, 8192)])
+@pytest.mark.parametrize("E,top,ff,cols", [(7, 6, 171, 4096), (4, 3, 700, 2048), (4, 3, 1361, 2048), (3, 2, 65, 8192)])
 def test_weighted_at_their_input(E, top, ff, cols):
     test_gpu_pufivik_ops.test_experts_of_a_step(1, E, top, ff, cols)
 

@@ -33,9 +33,10 @@ for a in ((4096, 4064), (2048, 4096), (8192, 4096), (2048, 2048), (64, 64), (256
 def test_first_matrices_of_experts():
     fake_hip.run(CALLS + """
 tiles = lambda top, ff: (2 * ff + 15) // 16 * top
-for top, ff, cols in ((1, 16, 2048), (6, 704, 2048), (8, 959, 2048), (1, 3072, 2048), (1, 4097, 2048), (1, 7680, 2048), (6, 1408, 1024), (6, 1408, 5120)):
+for top, ff, cols in ((1, 16, 2048), (6, 704, 2048), (4, 896, 2048), (6, 1408, 2048), (1, 4097, 2048), (1, 6144, 2048), (1, 12800, 2048), (6, 1408, 1024), (6, 1408, 5120)):
     assert first(top, ff, cols) == tiles(top, ff), (top, ff, cols)
-for top, ff, cols, want in ((8, 1024, 2048, 512), (6, 1408, 2048, 512), (1, 7681, 2048, 512), (1, 3073, 2048, 512), (4, 1024, 2048, 512), (1, 1, 4096, 1), (6, 1408, 4096, 512), (2, 64, 8192, 128)):
+for top, ff, cols, want in ((8, 1024, 2048, 512), (8, 959, 2048, 512), (4, 1024, 2048, 512), (1, 6145, 2048, 512), (1, 9217, 2048, 512), (1, 12801, 2048, 512), (6, 2816, 2048, 512),
+                            (1, 1, 4096, 1), (6, 1408, 4096, 512), (2, 64, 8192, 128)):
     assert first(top, ff, cols) == want, (top, ff, cols)
 assert first(6, 1408, 4096, T=2) == 2 * tiles(6, 1408)
 """)
