@@ -458,7 +458,8 @@ int chunk_weight(pi_model * m, BatchState * b, int il, int kind, int rows, int c
 // Q4_0 matrices that are whole on the device are multiplied straight from their blocks in chunks of fewer than 512 tokens; what they read is then in
 // the operand layout (out_ol).  Expanding first writes and reads the matrix in fp16 once more than that: us, expanded and multiplied by
 // the library / straight, 17 and 130 tokens: 12288 x 4096 42 / 15, 51 / 21; 4096 x 11008 transposed 46 / 25, 66 / 39; 13824 x 5120 54 / 19,
-// 66 / 30.  Longer chunks share one expansion among their pieces: four of 512 of 13824 x 5120 take 300 us so, and would take 344.  512
+// 66 / 30; of 17 shapes from 1024 x 512 to 32768 x 8192 at nine lengths only 2048 x 5632 transposed at 17 tokens is slower, 17.1 / 19.6 (in a layer whose other
+// products save 10 to 20 each).  Longer chunks share one expansion among their pieces: four of 512 of 13824 x 5120 take 300 us so, and would take 344.  512
 // tokens by themselves would gain too (74 / 63, 89 / 67, 99 / 86), but they are a piece of a longer chunk when 17 tokens more follow, and
 // their cells are to be the same either way.
 bool direct_q4(pi_model * m, BatchState * b, int il, int kind) {
