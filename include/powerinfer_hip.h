@@ -542,6 +542,12 @@ PI_API int pi_k_attn_chunk_rows_supported(int hd, int T, int n_kv_max);
 PI_API int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                                 const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride,
                                 void * out_f16, pi_stream_t stream);
+/* pi_k_attn_chunk_rows in one pass over the keys: no rounding of s - max, weights of fp16 divided behind the values, their sum in double.  More than 16
+ * tokens, head sizes 64 and 128; qkv_stride and out_stride whole quads, buffers on 16 bytes (out_f16 on 8).  q_f16: the rotated queries rounded to
+ * fp16, [T][n_head*hd]; out or out_f16 may be NULL. */
+PI_API int pi_k_attn_chunk_once(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                                const int32_t * pos, int n_ctx, int n_kv_max, void * q_f16, void * k_cache, void * v_cache, float * out, int out_stride,
+                                void * out_f16, pi_stream_t stream);
 /* prompt chunk of ONE sequence: T <= 512 consecutive tokens at positions pos[t]; RoPE + KV store of the whole chunk first, then
  * every token attends to the cells up to its own position (the causal mask of llama.cpp:6506-6531).  q_rot: fp32 [T][n_head*hd].
  * n_kv_max: an upper bound of max(pos) + 1, the cells the chunk's furthest token attends (<= 0: n_ctx); positions beyond it are

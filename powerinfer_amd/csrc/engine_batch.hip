@@ -70,8 +70,10 @@ pi_norm mk_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
     return n;
 }
 
-// attention of tokens t0 .. t0 + n - 1 of a prompt chunk of the model's own sequence, which see cells up to kv_hi: the chunk kernels where the
-// context fits them, the split-over-cells path beyond
+// attention of tokens t0 .. t0 + n - 1 of a prompt chunk of the model's own sequence, which see cells up to kv_hi: one pass over the keys where nothing of
+// the model is rounded to eight bits behind it and there are more than 16 tokens (against 16 tokens a workgroup, attn_chunk_mfma_kernel: 17
+// tokens 13.2 / 10.2 us, behind 1700 cells 48 / 37; 100 tokens 17.7 / 13.0), else the chunk kernels where the context fits them, the
+// split-over-cells path beyond
 int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size_t kv_off) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
@@ -79,6 +81,8 @@ int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size
     const int32_t * pos = b->d_pos + t0;
     float * q_rot = b->q_rot + (size_t)t0 * d, * att = b->att + (size_t)t0 * d;
     __half * att16 = b->att16 + (size_t)t0 * d, * k = m->k_cache + kv_off, * v = m->v_cache + kv_off;
+    if (!b->route.scalar && !b->route.pieces && (hd == 64 || hd == 128) && n > 16)
+        return pi_k_attn_chunk_once(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, nullptr, d, att16, m->stream);
     if (!b->route.scalar && pi_k_attn_chunk_rows_supported(hd, n, kv_hi) && !(b->route.pieces && pi::attn_chunk_by_16(hd, kv_hi)))
         return pi_k_attn_chunk_rows(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, att, d, att16, m->stream);
     if (pi_k_attn_chunk_supported(hd, hp.n_ctx, kv_hi))

@@ -1046,6 +1046,199 @@ __global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_kernel(const float 
     }
 }
 
+// The same 64 U tokens of a head against their cells in ONE pass over the keys: weights relative to a maximum that grows as the cells come, values
+// under the undivided weights (fp16), one division at the end.  For models of F16 matrices, whose next rounding is to fp16: against the three passes
+// above the result has two roundings fewer a weight (of s - max and of e / sum), and no eight-bit step behind it that a last place could turn.
+// A row's base is raised only where a score exceeds it by more than 2^8 (weights up to 256 in fp16, the sums in their wider types): then what
+// has been added so far is scaled down, which is rare, and no lane needs its neighbours' maxima to know that it is not needed.
+// The weights' sum is a product too (with ones, exact products of the same fp16 weights), a tile of 64 cells at a time, added up in double.
+// Bound by LDS (a tile's keys and values pass to each of four waves: about as many cycles as its products) and the exponentials between the two products.
+// RoPE and store included, three passes / one: 32 heads of 128, 2046 tokens 200 / 80 us, 512 42 / 25, 512 behind 1024 87 / 42, 64 15.0 / 11.7; 128
+// heads of 64 on 8, 1900 tokens 323 / 105; error against float64 (2046 tokens) 3.9e-4 / 2.6e-4.
+template <int HD, int U>
+__global__ __launch_bounds__(kBlock, 2) void attn_chunk_rows_once_kernel(const __half * __restrict__ q16, const __half * __restrict__ k_cache, const __half * __restrict__ v_cache,
+                                                                         int n_head, int n_head_kv, int n_ctx, const int32_t * __restrict__ pos_p, int T, int n_kv_max, int fold,
+                                                                         float * __restrict__ out, int out_stride, __half * __restrict__ out16) {
+    static_assert(HD == 128 || HD == 64, "head size");
+    constexpr int R = 64 * U, NK = kRowsCells, KS = HD / 32, VT = HD / 16, KT = NK / 16, ROW = rows_pitch<HD>(), PPR = HD / 8, NP = NK * PPR / kBlock;
+    extern __shared__ __align__(16) unsigned char smem[];                                  // two tiles of keys, two of values
+    __shared__ int span[2 * kWavesPerBlock], odd[2];
+    // the tokens that see the most cells first; where all workgroups run at once (fold) the second half of them the other way round, so that a
+    // unit's two have the same number of cells together
+    const int nb = (int)gridDim.y, y = (int)blockIdx.y, half = (nb + 1) / 2, tb = fold && y >= half ? y - half : nb - 1 - y;
+    const int h = blockIdx.x, kvh = h / (n_head / n_head_kv), t0 = tb * R;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+    // the most and the fewest cells a token here sees
+    {
+        const int t = t0 + tid % R, nv = t < T ? min(pos_p[t] + 1, n_kv_max) : -1;
+        int hi = nv, lo = nv < 0 ? INT32_MAX : nv;
+        for (int o = 32; o > 0; o >>= 1) { hi = max(hi, __shfl_xor(hi, o, PI_WAVE)); lo = min(lo, __shfl_xor(lo, o, PI_WAVE)); }
+        if (lane == 0) { span[wave] = hi; span[kWavesPerBlock + wave] = lo; }
+        if (tid < 2) odd[tid] = 0;
+    }
+    int nv[U];
+    pi_u32x4 qf[U][KS];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = t0 + wave * 16 * U + u * 16 + i;
+        nv[u] = t < T ? min(pos_p[t] + 1, n_kv_max) : 0;
+        const __half * qp = q16 + ((size_t)min(t, T - 1) * n_head + h) * HD + 8 * g;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) qf[u][s] = pi_ld16(qp + s * 32);
+    }
+    __syncthreads();
+    int n_keys = span[0], n_all = span[kWavesPerBlock];
+#pragma unroll
+    for (int w = 1; w < kWavesPerBlock; ++w) { n_keys = max(n_keys, span[w]); n_all = min(n_all, span[kWavesPerBlock + w]); }
+    // this thread's pieces of a tile; cells past the last one read the last one again (never a cell that no token here sees)
+    const __half * kb = k_cache + (size_t)kvh * n_ctx * HD + (tid % PPR) * 8;
+    const __half * vb = v_cache + (size_t)kvh * n_ctx * HD + (tid % PPR) * 8;
+    const int row0 = tid / PPR, last = max(n_keys - 1, 0);
+    pi_u32x4 pk[NP], pv[NP];
+    auto fetch = [&](pi_u32x4 * dst, const __half * base, int cb) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) dst[j] = pi_ld16(base + (size_t)min(cb + row0 + j * (kBlock / PPR), last) * HD);
+    };
+    auto place = [&](unsigned char * tile, const pi_u32x4 * src) {
+#pragma unroll
+        for (int j = 0; j < NP; ++j) *reinterpret_cast<pi_u32x4 *>(tile + (row0 + j * (kBlock / PPR)) * ROW + (tid % PPR) * 16) = src[j];
+    };
+    constexpr int TILE = NK * ROW;
+    const float to2 = pi_inv_sqrt((float)HD) * 1.44269504f, room = 8.0f / to2;             // e^(s / sqrt(HD)) = 2^(s to2)
+    const pi_u32x4 ones{0x3C003C00u, 0x3C003C00u, 0x3C003C00u, 0x3C003C00u};
+
+    float limit[U], base2[U];                                            // a score beyond it raises the base; the base as a power of two (0 while there is none)
+    double sum[U];
+    pi_f4 o[U][VT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        limit[u] = -INFINITY; base2[u] = 0.0f; sum[u] = 0.0;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) o[u][v] = pi_f4{0, 0, 0, 0};
+    }
+    unsigned char * vt = smem + 2 * TILE;
+    fetch(pk, kb, 0);
+    fetch(pv, vb, 0);
+    int at = 0;
+    for (int cb = 0; cb < n_keys; cb += NK, at ^= 1) {
+        const bool edge = cb + NK > n_all;
+        place(smem + at * TILE, pk);
+        place(vt + at * TILE, pv);
+        if (edge) {                                                      // a value that is no number, in a cell that some tokens here do not see
+            unsigned bad = 0;
+#pragma unroll
+            for (int j = 0; j < NP; ++j)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) { const unsigned x = pv[j][w] & 0x7C007C00u; bad |= (x & 0xFFFFu) == 0x7C00u || (x >> 16) == 0x7C00u; }
+            if (bad) odd[at] = 1;
+        }
+        __syncthreads();
+        fetch(pk, kb, cb + NK);
+        fetch(pv, vb, cb + NK);
+        pi_f4 s[U][KT];
+        const unsigned char * tile = smem + at * TILE;
+#pragma unroll
+        for (int kt = 0; kt < KT; ++kt) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) s[u][kt] = pi_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int c = 0; c < KS; ++c) {
+                const pi_u32x4 a = *reinterpret_cast<const pi_u32x4 *>(tile + (kt * 16 + i) * ROW + c * 64 + g * 16);
+#pragma unroll
+                for (int u = 0; u < U; ++u) s[u][kt] = mma16<__half>(a, qf[u][c], s[u][kt]);
+            }
+        }
+        if (edge) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[u][kt][r] = cb + kt * 16 + 4 * g + r >= nv[u] ? -INFINITY : s[u][kt][r];
+        }
+        pi_u32x4 pb[U][KT / 2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float top = s[u][0][0];
+#pragma unroll
+            for (int k = 1; k < 4 * KT; ++k) top = fmaxf(top, s[u][k >> 2][k & 3]);
+            if (__any(top > limit[u])) {
+                top = fmaxf(top, __shfl_xor(top, 16, PI_WAVE));
+                top = fmaxf(top, __shfl_xor(top, 32, PI_WAVE));
+                if (top > limit[u] - room) {                             // (limit -inf: -inf)
+                    const float b = top * to2, down = limit[u] == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(base2[u] - b);
+                    limit[u] = top + room; base2[u] = b;
+                    sum[u] *= (double)down;
+#pragma unroll
+                    for (int v = 0; v < VT; ++v) o[u][v] *= down;
+                }
+            }
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            typedef float f2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+            for (int k = 0; k < 2 * KT; ++k) {
+                const f2 e{__builtin_amdgcn_exp2f(fmaf(s[u][k >> 1][2 * (k & 1)], to2, -base2[u])), __builtin_amdgcn_exp2f(fmaf(s[u][k >> 1][2 * (k & 1) + 1], to2, -base2[u]))};
+                pb[u][k >> 2][k & 3] = __builtin_bit_cast(unsigned, __builtin_convertvector(e, h2));
+            }
+            pi_f4 n{0, 0, 0, 0};
+#pragma unroll
+            for (int k = 0; k < KT / 2; ++k) n = mma16<__half>(ones, pb[u][k], n);
+            sum[u] += (double)n[0];
+        }
+        const unsigned char * vs = vt + at * TILE;
+        if (edge && odd[at]) {
+            // 0 times such a value is no number either: token by token, the cells it sees only.  The weight of cell (kt, g, r) of token i is
+            // half (kt % 2) * 4 + r of step kt / 2 in lane 16 g + i.
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                for (int c = 0; c < NK; ++c) {
+                    const int kt = c >> 4, from = ((c >> 2) & 3) * 16 + i, hw = (kt & 1) * 4 + (c & 3);
+                    unsigned word = 0;
+#pragma unroll
+                    for (int k = 0; k < KT / 2; ++k)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) word = k == (kt >> 1) && q == (hw >> 1) ? pb[u][k][q] : word;
+                    const unsigned got = (unsigned)__shfl((int)word, from, PI_WAVE);
+                    const float w = pi_f16_from_bits((uint16_t)(hw & 1 ? got >> 16 : got));
+                    if (cb + c >= nv[u]) continue;
+#pragma unroll
+                    for (int v = 0; v < VT; ++v)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) o[u][v][r] = fmaf(w, __half2float(reinterpret_cast<const __half *>(vs + c * ROW)[v * 16 + 4 * g + r]), o[u][v][r]);
+                }
+            continue;
+        }
+        // slot (g, j) of a 32-cell step: cell 4 g + j of its first 16 (j < 4) or of its second 16 - two transposing reads
+#pragma unroll
+        for (int k = 0; k < KT / 2; ++k)
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                const unsigned char * a = vs + (k * 32 + 4 * g + (i >> 2)) * ROW + (v * 16 + (i & 3) * 4) * 2;
+                const pi_u32x2 lo = lds_tr_read(a), hi = lds_tr_read(a + 16 * ROW);
+                const pi_u32x4 fr{lo.x, lo.y, hi.x, hi.y};
+#pragma unroll
+                for (int u = 0; u < U; ++u) o[u][v] = mma16<__half>(fr, pb[u][k], o[u][v]);
+            }
+    }
+    // o[u][v][r] = out[token i][v * 16 + 4 g + r]
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = t0 + wave * 16 * U + u * 16 + i;
+        if (t >= T) continue;
+        const float inv = (float)(1.0 / sum[u]);
+        const size_t to = (size_t)t * out_stride + (size_t)h * HD + 4 * g;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const float4 y{o[u][v][0] * inv, o[u][v][1] * inv, o[u][v][2] * inv, o[u][v][3] * inv};
+            if (out) *reinterpret_cast<float4 *>(out + to + v * 16) = y;
+            if (out16) {
+                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+                *reinterpret_cast<h4 *>(out16 + to + v * 16) = h4{(_Float16)y.x, (_Float16)y.y, (_Float16)y.z, (_Float16)y.w};
+            }
+        }
+    }
+}
+
 // RoPE + KV store of a chunk's tokens, all heads of a token by one workgroup (or by gridDim.y of them, heads in turn): the angles are
 // formed once a token instead of once a head, bit for bit those of rope_kv_store_kernel, and the rest is a copy at the rate of memory.
 __global__ __launch_bounds__(kBlock) void rope_kv_chunk_kernel(const float * __restrict__ qkv, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
@@ -1087,7 +1280,9 @@ __global__ __launch_bounds__(kBlock) void rope_kv_chunk_kernel(const float * __r
 // such pieces of a thread requested before the angles are formed.  The loop above made a memory trip an iteration, two values in it: 2046 tokens,
 // 32 heads of 128 (167 MB in and out): 48 us, here 33 (what
 // a copy of as much takes).
+// Q16: the rotated queries leave rounded to fp16, rows of n_head * hd of them (what attn_chunk_rows_once_kernel reads: half the bytes of both launches).
 constexpr int kRopeUn = 6;
+template <bool Q16>
 __global__ __launch_bounds__(kBlock) void rope_kv_chunk_wide_kernel(const float * __restrict__ qkv, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                                                                      const int32_t * __restrict__ pos_p, int n_ctx, float * __restrict__ q_rot,
                                                                      __half * __restrict__ k_cache, __half * __restrict__ v_cache, int qkv_stride, int q_stride) {
@@ -1130,13 +1325,14 @@ __global__ __launch_bounds__(kBlock) void rope_kv_chunk_wide_kernel(const float 
                     x0 = y0; x1 = y1;
                 }
             }
-            if (h < n_head) {
+            if (!Q16 && h < n_head) {
                 float * dst = qd + (size_t)h * hd + j * step;
                 *reinterpret_cast<float4 *>(dst) = make_float4(x[0], x[1], x[2], x[3]);
                 *reinterpret_cast<float4 *>(dst + second) = make_float4(x[4], x[5], x[6], x[7]);
             } else {
                 const int hk = h - n_head;
-                __half * dst = (hk < n_head_kv ? k_cache + ((size_t)hk * n_ctx + pos) * hd : v_cache + ((size_t)(hk - n_head_kv) * n_ctx + pos) * hd) + j * step;
+                __half * dst = (h < n_head ? reinterpret_cast<__half *>(q_rot) + (size_t)t * q_stride + (size_t)h * hd
+                                : hk < n_head_kv ? k_cache + ((size_t)hk * n_ctx + pos) * hd : v_cache + ((size_t)(hk - n_head_kv) * n_ctx + pos) * hd) + j * step;
                 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
                 *reinterpret_cast<h4 *>(dst) = h4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
                 *reinterpret_cast<h4 *>(dst + second) = h4{(_Float16)x[4], (_Float16)x[5], (_Float16)x[6], (_Float16)x[7]};
@@ -1317,12 +1513,22 @@ int launch_chunk_rows(const float * q_rot, const void * k_cache, const void * v_
                        n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, n_head * HD, out_stride, (__half *)out_f16);
     return pi::check_launch("attn_chunk_rows");
 }
+template <int HD, int U>
+int launch_chunk_once(const void * q16, const void * k_cache, const void * v_cache, int n_head, int n_head_kv, int n_ctx, const int32_t * pos, int T, int n_kv_max, float * out, int out_stride,
+                      void * out_f16, hipStream_t st) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_chunk_rows_once_kernel<HD, U>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds<HD>());
+    if (raised != hipSuccess) return pi::hip_fail(raised, "attn_chunk_once: LDS size");
+    const int blocks = (T + 64 * U - 1) / (64 * U);
+    hipLaunchKernelGGL((attn_chunk_rows_once_kernel<HD, U>), dim3(n_head, blocks), dim3(kBlock), rows_lds<HD>(), st, (const __half *)q16, (const __half *)k_cache, (const __half *)v_cache,
+                       n_head, n_head_kv, n_ctx, pos, T, n_kv_max, (long long)n_head * blocks <= 2 * pi::compute_units() ? 1 : 0, out, out_stride, (__half *)out_f16);
+    return pi::check_launch("attn_chunk_once");
+}
 }  // namespace
 
 namespace pi {
 // keys and values of T tokens to their cells, rotated queries to q_rot; n_head 0: rows of k and v alone (no q_rot)
 int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
-                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st) {
+                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st, bool q16) {
     // 16 tokens and fewer: a workgroup per head and token (16 tokens, 32 heads of 128, attention included: 11.8 against 12.3 us); a chunk's angles
     // are worth forming once a token from there on.  A workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
     if (T <= kBtMaxT) {
@@ -1333,7 +1539,8 @@ int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_he
     const int split = T >= 512 ? 1 : T >= 128 ? 4 : 16;
     // 16-byte rows: heads of a multiple of eight values, and everything that starts on one
     const bool wide = hd % 8 == 0 && qkv_stride % 4 == 0 && (((uintptr_t)qkv | (uintptr_t)q_rot | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
-    const auto kernel = wide ? rope_kv_chunk_wide_kernel : rope_kv_chunk_kernel;
+    if (q16 && (!wide || T <= kBtMaxT)) return pi::fail(PI_E_ARG, "rope_kv_chunk: fp16 queries need rows of 16 bytes and more than 16 tokens");
+    const auto kernel = q16 ? rope_kv_chunk_wide_kernel<true> : wide ? rope_kv_chunk_wide_kernel<false> : rope_kv_chunk_kernel;
     hipLaunchKernelGGL(kernel, dim3(T, split), dim3(kBlock), sizeof(float2) * (hd / 2), st, qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot,
                        (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
     return pi::check_launch("rope_kv_chunk");
@@ -1572,6 +1779,23 @@ int pi_k_attn_chunk_rows(const float * qkv, int qkv_stride, int T, int n_head, i
     return hd == 128 ? (two ? PI_ROWS_U(128, 2) : PI_ROWS_U(128, 1)) : (two ? PI_ROWS_U(64, 2) : PI_ROWS_U(64, 1));
 #undef PI_ROWS_U
 #undef PI_ROWS
+}
+
+int pi_k_attn_chunk_once(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                         const int32_t * pos, int n_ctx, int n_kv_max, void * q_f16, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16,
+                         pi_stream_t stream) {
+    if (!qkv || !pos || !q_f16 || !k_cache || !v_cache || (!out && !out_f16) || T <= kBtMaxT || n_ctx <= 0) return pi::fail(PI_E_ARG, "pi_k_attn_chunk_once: bad arguments");
+    if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (hd != 64 && hd != 128) || (mode != 0 && mode != 2)) return pi::fail(PI_E_ARG, "pi_k_attn_chunk_once: bad head geometry or mode");
+    if (qkv_stride % 4 || out_stride % 4 || (((uintptr_t)qkv | (uintptr_t)q_f16 | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)out) & 15) || ((uintptr_t)out_f16 & 7))
+        return pi::fail(PI_E_ARG, "pi_k_attn_chunk_once: rows of whole quads, buffers on 16 bytes (out_f16: 8)");
+    if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;
+    hipStream_t st = (hipStream_t)stream;
+    const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, (float *)q_f16, k_cache, v_cache, st, true);
+    if (rc != PI_OK) return rc;
+    const bool two = (long long)n_head * ((T + 127) / 128) >= 2 * pi::compute_units();
+#define PI_ONCE(HD, U) launch_chunk_once<HD, U>(q_f16, k_cache, v_cache, n_head, n_head_kv, n_ctx, pos, T, n_kv_max, out, out_stride, out_f16, st)
+    return hd == 128 ? (two ? PI_ONCE(128, 2) : PI_ONCE(128, 1)) : (two ? PI_ONCE(64, 2) : PI_ONCE(64, 1));
+#undef PI_ONCE
 }
 
 int pi_k_attn_chunk_supported(int hd, int n_ctx, int n_kv_max) {

@@ -47,7 +47,7 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
 // whether pi_k_attn_chunk takes the tokens of a chunk against n_kv_max cells 16 at a time on the matrix cores
 bool attn_chunk_by_16(int hd, int n_kv_max);
 int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
-                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st);
+                  float * q_rot, void * k_cache, void * v_cache, hipStream_t st, bool q16 = false);
 // pi_k_expert_up_step with act = weight * relu(up[e] x)^2 (up [n_expert][ff][cols])
 int expert_relu2_step(const void * up, int n_expert, int ff, int cols, const void * x_ol, int T, const int32_t * ids, const float * weights, int top, void * act, int ld_act,
                       pi_stream_t stream);
