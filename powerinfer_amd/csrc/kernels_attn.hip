@@ -387,22 +387,29 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
 // (18 us per 7B layer at 600 cells, growing by 2.4 us per 100 cells); with n_parts workgroups per head every unit takes a share and
 // the score buffer in LDS holds n_ctx / n_parts cells instead of all of them.
 // Part s owns cells [n_kv * s / n, n_kv * (s + 1) / n); the last part holds the new cell: it rotates and stores k, stores v, and
-// uses them from LDS.  Every part rotates q, computes its scores, e_i = fp16(exp(fp16(s_i - m))) with ITS maximum m (the rounding
-// points of the CPU path's table, ggml.c:10747-10759), l = sum e_i in double and acc = sum v_i * e_i, and hands (m, l, acc) to
-// attn_merge_kernel, which rescales by exp(m - M), adds the parts in order and divides by the total.  Against one workgroup per head,
-// which knows the global maximum before it rounds, results differ in the last places of the fp16 roundings (1e-4 of the output).
-// Bound by the trips to memory of a part's rows: eight passes of K and V are in flight at any time (four at the start and then one by one: 21.9 us
-// for 32 heads of 128 at 3000 cells in 8 parts, 49 MB; now 15.4; 128 heads of 64 at 1024 cells in 2 parts 20.6 -> 12.0), the
-// sums over a cell's lanes are VALU permutations, and the sum over the groups reads LDS eight at a time.
+// uses them from LDS.  Every part rotates q and goes through its cells once: a group of lanes holds a cell's K and V row, and keeps a maximum
+// m, l = sum of e^(s - m) and acc = sum of v e^(s - m) of the cells it has seen, so that nothing waits for another group before the
+// rows have been read; at the end the groups' three meet in LDS.  The part hands (m, l, acc) to attn_merge_kernel, which rescales by exp(m - M), adds
+// the parts in order and divides by the total.  Weights stay in fp32 (the single workgroup's are rounded to fp16: the two differ by
+// those roundings, 1e-4 of the output).
+// Bound by the trips to memory of a part's rows.  Eight cells of a group, K and V, are on their way at any time, requested without a guard (a guarded
+// load makes the compiler wait for all the others; rows past the last cell are the last one again), and what the rotation needs ahead of
+// them, because loads return in order.  Merge included, against scores, soft-max and values one after the other with guarded loads: 32 heads of 128 in
+// 8 parts, 1030 cells 12.4 -> 11.0 us, 3001 19.4 -> 16.1 (49 MB), 32000 in 16 parts 97 -> 93; 128 heads of 64 in 2 parts, 1030 cells 14.2 -> 11.7.
 // ---------------------------------------------------------------------------------------------------
 // FROM_CACHE: the token's own K / V row is in the cache already and qkv holds its rotated q only ([n_head * hd] per token; a prompt chunk
 // behind rope_kv_store_kernel): nothing is rotated or stored, every cell is read from the cache.
 constexpr int kAttnPartBlock = 512;
-constexpr int kAttnPartPre = 8;          // passes whose K and V rows are in flight: one use of a row requests the row eight passes on
+constexpr int kAttnPartCells = 4;        // cells of a group that are requested, scored and weighed together; two such batches are in flight
+constexpr int kAttnPartFloats = kAttnPartBlock * 8;      // [groups][hd]
+static size_t attn_part_lds(int hd) {    // the groups' sums, two words of each, what the parts of a head's values add up to, and q, k, v
+    return sizeof(float) * (kAttnPartFloats + 2 * (size_t)(kAttnPartFloats / hd) + kAttnPartBlock + 2 * (size_t)(kAttnPartBlock / hd) + 3 * (size_t)hd);
+}
+static size_t attn_rounded_lds(int hd, int s_cap) { return sizeof(float) * ((size_t)s_cap + kAttnPartFloats + 3 * (size_t)hd); }
 template <bool FROM_CACHE, int LPP>
 __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
                                                                    __half * __restrict__ k_cache, __half * __restrict__ v_cache,
-                                                                   int n_head, int n_head_kv, int hd, int mode, int n_ctx, int s_cap,
+                                                                   int n_head, int n_head_kv, int hd, int mode, int n_ctx,
                                                                    const int32_t * __restrict__ pos_p, float * __restrict__ part_acc, float * __restrict__ part_ml,
                                                                    int qkv_stride, size_t cache_seq_stride) {
     qkv += (size_t)blockIdx.z * qkv_stride;
@@ -410,78 +417,207 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     v_cache += (size_t)blockIdx.z * cache_seq_stride;
     pos_p += blockIdx.z;
     extern __shared__ __align__(16) unsigned char smem[];
-    float * s    = reinterpret_cast<float *>(smem);               // [s_cap] scores of this part, then e_i
-    float * part = s + s_cap;                                     // [groups][hd]
-    float * qs   = part + (kAttnPartBlock / (hd / 8)) * hd;       // [hd] rotated q, rounded to fp16
+    const int lpp = LPP ? LPP : hd / 8, ngrp = kAttnPartBlock / lpp, n_sum = kAttnPartBlock / hd;      // (hd divides 512; eight groups to each of the n_sum sums)
+    float * part = reinterpret_cast<float *>(smem);               // [ngrp][hd]
+    float * gm = part + kAttnPartFloats, * gl = gm + ngrp;        // [ngrp] the groups' maxima and sums
+    float * half = gl + ngrp;                                     // [n_sum][hd]
+    float * hm = half + kAttnPartBlock, * hl = hm + n_sum;        // [n_sum]
+    float * qs = hl + n_sum;                                      // [hd] rotated q, rounded to fp16
     float * kcur = qs + hd;                                       // [hd] rotated k of this position, rounded to fp16
     float * vcur = kcur + hd;                                     // [hd]
-    __shared__ double red[16];
-    __shared__ float redf[16];
     const int h = blockIdx.x, n_parts = gridDim.y, sp = blockIdx.y, grp_sz = n_head / n_head_kv, kvh = h / grp_sz;
     const int tid = threadIdx.x;
     const int pos = *pos_p, n_kv = pos + 1;
     const int lo = (int)((long long)n_kv * sp / n_parts), hi = (int)((long long)n_kv * (sp + 1) / n_parts);
     const bool owns_new = !FROM_CACHE && sp == n_parts - 1;        // hi == n_kv: the new cell is this part's last
     const size_t slot = ((size_t)blockIdx.z * n_head + h) * n_parts + sp;
-    if (hi - lo > s_cap) return;                                  // cannot happen for pos < n_ctx (the launcher sizes s_cap); never write past LDS
     const float * qsrc = qkv + (size_t)h * hd;
-    const float * ksrc = qkv + (size_t)(n_head + kvh) * hd;
-    const float * vsrc = qkv + (size_t)(n_head + n_head_kv + kvh) * hd;
-    const int lpp = LPP ? LPP : hd / 8;
-    const int sub = tid % lpp, grp = tid / lpp, ngrp = kAttnPartBlock / lpp;
-    const __half * kb = k_cache + (size_t)kvh * n_ctx * hd;
-    const __half * vb = v_cache + (size_t)kvh * n_ctx * hd;
+    const int sub = tid % lpp, grp = tid / lpp;
     const int n_old = (owns_new ? hi - 1 : hi) - lo;              // cells of this part that live in the cache
-    pi_u32x4 kpre[kAttnPartPre], vpre[kAttnPartPre];
-    const __half * kr = kb + (size_t)lo * hd + sub * 8, * vr = vb + (size_t)lo * hd + sub * 8;
+    // what is rotated: pair (or value) tid of the head, every thread one
+    float q0 = 0, q1 = 0, k0 = 0, k1 = 0, v0 = 0;
+    float2 cs{1, 0};
+    const int pair = tid % (hd / 2), i0 = (mode & 2) ? pair : 2 * pair, i1 = (mode & 2) ? pair + hd / 2 : 2 * pair + 1;
+    if constexpr (FROM_CACHE) q0 = qsrc[tid % hd];
+    else {
+        const float * ksrc = qkv + (size_t)(n_head + kvh) * hd, * vsrc = ksrc + (size_t)n_head_kv * hd;
+        cs = rope_table[(size_t)pos * (hd / 2) + pair];
+        q0 = qsrc[i0]; q1 = qsrc[i1]; k0 = ksrc[i0]; k1 = ksrc[i1]; v0 = vsrc[tid % hd];
+    }
+    const __half * kr = k_cache + ((size_t)kvh * n_ctx + lo) * hd + sub * 8, * vr = v_cache + ((size_t)kvh * n_ctx + lo) * hd + sub * 8;
+    pi_u32x4 kk[2][kAttnPartCells], vv[2][kAttnPartCells];
+    auto fetch = [&](auto slot, int c0) {
+        constexpr int S = decltype(slot)::value;
 #pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_old) kpre[i] = pi_ld16(kr + (size_t)c * hd); }
-#pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_old) vpre[i] = pi_ld16(vr + (size_t)c * hd); }
-    if (FROM_CACHE) {
-        if (tid < hd) qs[tid] = pi_round_f16(qsrc[tid]);
-    } else if (tid < hd / 2) {
-        const float2 cs = rope_table[(size_t)pos * (hd / 2) + tid];
-        const int i0 = (mode & 2) ? tid : 2 * tid;
-        const int i1 = (mode & 2) ? tid + hd / 2 : 2 * tid + 1;
-        const float q0 = qsrc[i0], q1 = qsrc[i1];
-        qs[i0] = pi_round_f16(__fsub_rn(__fmul_rn(q0, cs.x), __fmul_rn(q1, cs.y)));
-        qs[i1] = pi_round_f16(__fadd_rn(__fmul_rn(q0, cs.y), __fmul_rn(q1, cs.x)));
-        if (owns_new) {
-            const float k0 = ksrc[i0], k1 = ksrc[i1];
-            const __half ka = __float2half_rn(__fsub_rn(__fmul_rn(k0, cs.x), __fmul_rn(k1, cs.y)));
-            const __half kc = __float2half_rn(__fadd_rn(__fmul_rn(k0, cs.y), __fmul_rn(k1, cs.x)));
-            kcur[i0] = __half2float(ka); kcur[i1] = __half2float(kc);
-            if ((h % grp_sz) == 0) { __half * kdst = k_cache + ((size_t)kvh * n_ctx + pos) * hd; kdst[i0] = ka; kdst[i1] = kc; }
+        for (int u = 0; u < kAttnPartCells; ++u) {
+            const size_t c = (size_t)max(min(c0 + u * ngrp + grp, n_old - 1), 0) * hd;
+            kk[S][u] = pi_ld16(kr + c); vv[S][u] = pi_ld16(vr + c);
         }
-    } else if (owns_new && tid < hd / 2 + hd) {
-        const int e = tid - hd / 2;
-        const __half v = __float2half_rn(vsrc[e]);
-        vcur[e] = __half2float(v);
-        if ((h % grp_sz) == 0) v_cache[((size_t)kvh * n_ctx + pos) * hd + e] = v;
+    };
+    using First = std::integral_constant<int, 0>;
+    using Second = std::integral_constant<int, 1>;
+    const int step = kAttnPartCells * ngrp;
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(First{}, 0);
+    fetch(Second{}, step);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FROM_CACHE) {
+        if (tid < hd) qs[tid] = pi_round_f16(q0);
+    } else {
+        if (tid < hd / 2) {
+            qs[i0] = pi_round_f16(__fsub_rn(__fmul_rn(q0, cs.x), __fmul_rn(q1, cs.y)));
+            qs[i1] = pi_round_f16(__fadd_rn(__fmul_rn(q0, cs.y), __fmul_rn(q1, cs.x)));
+        }
+        if (owns_new && tid < hd) {
+            const bool store = (h % grp_sz) == 0;
+            const size_t cell = ((size_t)kvh * n_ctx + pos) * hd;
+            if (tid < hd / 2) {
+                const __half ka = __float2half_rn(__fsub_rn(__fmul_rn(k0, cs.x), __fmul_rn(k1, cs.y)));
+                const __half kc = __float2half_rn(__fadd_rn(__fmul_rn(k0, cs.y), __fmul_rn(k1, cs.x)));
+                kcur[i0] = __half2float(ka); kcur[i1] = __half2float(kc);
+                if (store) { k_cache[cell + i0] = ka; k_cache[cell + i1] = kc; }
+            }
+            const __half v = __float2half_rn(v0);
+            vcur[tid] = __half2float(v);
+            if (store) v_cache[cell + tid] = v;
+        }
     }
     __syncthreads();
 
     const float scale = pi_inv_sqrt((float)hd);
-    const int n_mine = hi - lo;
-    float qf[8];
+    float qf[8], acc[8], m = -INFINITY, l = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
-    for (int c0 = 0; c0 < n_old; c0 += kAttnPartPre * ngrp)
+    for (int i = 0; i < 8; ++i) { qf[i] = qs[sub * 8 + i]; acc[i] = 0.0f; }
+    // N cells' scores and values into m, l and acc; f(u, e, acc): the values of cell u under the weight e
+    auto add = [&](auto n, const float * s, auto && f) {
+        constexpr int N = decltype(n)::value;
+        float top = m;
 #pragma unroll
-        for (int i = 0; i < kAttnPartPre; ++i) {                    // (a row past the last is whatever the registers hold, and not used)
-            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
-            const float d = pi_group_sum<LPP>(pi_dot8(kpre[i], qf, 0.0f), lpp);
-            if (next < n_old) kpre[i] = pi_ld16(kr + (size_t)next * hd);
-            if (c < n_old && sub == 0) s[c] = __fmul_rn(d, scale);
+        for (int u = 0; u < N; ++u) top = fmaxf(top, s[u]);
+        const float base = top == -INFINITY ? 0.0f : top, down = __expf(__fsub_rn(m, base));
+        m = top; l *= down;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] *= down;
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const float e = __expf(__fsub_rn(s[u], base));
+            l += e;
+            f(u, e);
         }
+    };
+    auto batch = [&](auto slot, int c0) {
+        constexpr int S = decltype(slot)::value;
+        float s[kAttnPartCells];
+#pragma unroll
+        for (int u = 0; u < kAttnPartCells; ++u) s[u] = pi_group_sum<LPP>(pi_dot8(kk[S][u], qf, 0.0f), lpp);
+#pragma unroll
+        for (int u = 0; u < kAttnPartCells; ++u) s[u] = c0 + u * ngrp + grp < n_old ? __fmul_rn(s[u], scale) : -INFINITY;
+        add(std::integral_constant<int, kAttnPartCells>{}, s, [&](int u, float e) {
+            float vf[8];
+            pi_unpack8(vv[S][u], vf);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], e, acc[k]);
+        });
+    };
+    for (int c0 = 0; c0 < n_old; c0 += 2 * step) {
+        batch(First{}, c0);
+        if (c0 + step >= n_old) break;
+        fetch(First{}, c0 + 2 * step);
+        batch(Second{}, c0 + step);
+        fetch(Second{}, c0 + 3 * step);
+    }
     if (owns_new && grp == n_old % ngrp) {
         float d = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
-        d = pi_group_sum<LPP>(d, lpp);
-        if (sub == 0) s[n_old] = __fmul_rn(d, scale);
+        d = __fmul_rn(pi_group_sum<LPP>(d, lpp), scale);
+        add(std::integral_constant<int, 1>{}, &d, [&](int, float e) {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc[k] = fmaf(vcur[sub * 8 + k], e, acc[k]);
+        });
     }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
+    if (sub == 0) { gm[grp] = m; gl[grp] = l; }
+    __syncthreads();
+    // value e of eight groups by every thread, then of the n_sum sums of eight by one
+    {
+        const int e = tid % hd, j = tid / hd;
+        float M = -INFINITY, L = 0.0f, v = 0.0f;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) M = fmaxf(M, gm[j * 8 + g]);
+        const float base = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+            const float w = __expf(__fsub_rn(gm[j * 8 + g], base));
+            L = fmaf(gl[j * 8 + g], w, L);
+            v = fmaf(part[(j * 8 + g) * hd + e], w, v);
+        }
+        half[j * hd + e] = v;
+        if (e == 0) { hm[j] = M; hl[j] = L; }
+    }
+    __syncthreads();
+    if (tid < hd) {
+        float M = -INFINITY, L = 0.0f, v = 0.0f;
+        for (int j = 0; j < n_sum; ++j) M = fmaxf(M, hm[j]);
+        const float base = M == -INFINITY ? 0.0f : M;
+        for (int j = 0; j < n_sum; ++j) {
+            const float w = __expf(__fsub_rn(hm[j], base));
+            L = fmaf(hl[j], w, L);
+            v = fmaf(half[j * hd + tid], w, v);
+        }
+        part_acc[slot * hd + tid] = v;
+        if (tid == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = L; }
+    }
+}
+
+// The same for the tokens of a prompt chunk (pi_k_attn_chunk_long; K / V rows and rotated queries are stored): scores first, then e_i = fp16(exp(fp16(s_i - m))) with the part's
+// maximum m, the rounding points of the CPU path's table (ggml.c:10747-10759), then the values.
+constexpr int kAttnPartPre = 8;          // passes whose K and V rows are in flight: one use of a row requests the row eight passes on
+template <int LPP>
+__global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_rounded_kernel(const float * __restrict__ q_rot, const __half * __restrict__ k_cache, const __half * __restrict__ v_cache, int n_head, int n_head_kv,
+                                                                             int hd, int n_ctx, int s_cap, const int32_t * __restrict__ pos_p, float * __restrict__ part_acc,
+                                                                             float * __restrict__ part_ml, int q_stride) {
+    q_rot += (size_t)blockIdx.z * q_stride;
+    pos_p += blockIdx.z;
+    extern __shared__ __align__(16) unsigned char smem[];
+    float * s    = reinterpret_cast<float *>(smem);               // [s_cap] scores of this part, then e_i
+    float * part = s + s_cap;                                     // [groups][hd]
+    float * qs   = part + kAttnPartFloats;                        // [hd] rotated q, rounded to fp16
+    __shared__ double red[16];
+    __shared__ float redf[16];
+    const int h = blockIdx.x, n_parts = gridDim.y, sp = blockIdx.y, grp_sz = n_head / n_head_kv, kvh = h / grp_sz;
+    const int tid = threadIdx.x;
+    const int n_kv = *pos_p + 1;
+    const int lo = (int)((long long)n_kv * sp / n_parts), hi = (int)((long long)n_kv * (sp + 1) / n_parts);
+    const size_t slot = ((size_t)blockIdx.z * n_head + h) * n_parts + sp;
+    if (hi - lo > s_cap) return;                                  // cannot happen for pos < n_ctx (the launcher sizes s_cap); never write past LDS
+    const int lpp = LPP ? LPP : hd / 8;
+    const int sub = tid % lpp, grp = tid / lpp, ngrp = kAttnPartBlock / lpp;
+    const __half * kb = k_cache + (size_t)kvh * n_ctx * hd;
+    const __half * vb = v_cache + (size_t)kvh * n_ctx * hd;
+    const int n_mine = hi - lo;
+    pi_u32x4 kpre[kAttnPartPre], vpre[kAttnPartPre];
+    const __half * kr = kb + (size_t)lo * hd + sub * 8, * vr = vb + (size_t)lo * hd + sub * 8;
+#pragma unroll
+    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_mine) kpre[i] = pi_ld16(kr + (size_t)c * hd); }
+#pragma unroll
+    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_mine) vpre[i] = pi_ld16(vr + (size_t)c * hd); }
+    if (tid < hd) qs[tid] = pi_round_f16(q_rot[(size_t)h * hd + tid]);
+    __syncthreads();
+
+    const float scale = pi_inv_sqrt((float)hd);
+    float qf[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
+    for (int c0 = 0; c0 < n_mine; c0 += kAttnPartPre * ngrp)
+#pragma unroll
+        for (int i = 0; i < kAttnPartPre; ++i) {                    // (a row past the last is whatever the registers hold, and not used)
+            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
+            const float d = pi_group_sum<LPP>(pi_dot8(kpre[i], qf, 0.0f), lpp);
+            if (next < n_mine) kpre[i] = pi_ld16(kr + (size_t)next * hd);
+            if (c < n_mine && sub == 0) s[c] = __fmul_rn(d, scale);
+        }
     __syncthreads();
 
     float mx = -INFINITY;
@@ -498,24 +634,19 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    for (int c0 = 0; c0 < n_old; c0 += kAttnPartPre * ngrp)
+    for (int c0 = 0; c0 < n_mine; c0 += kAttnPartPre * ngrp)
 #pragma unroll
         for (int i = 0; i < kAttnPartPre; ++i) {
             const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
-            if (c < n_old) {
+            if (c < n_mine) {
                 const float p = s[c];
                 float vf[8];
                 pi_unpack8(vpre[i], vf);
-                if (next < n_old) vpre[i] = pi_ld16(vr + (size_t)next * hd);
+                if (next < n_mine) vpre[i] = pi_ld16(vr + (size_t)next * hd);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], p, acc[k]);
             }
         }
-    if (owns_new && grp == n_old % ngrp) {                          // (the new cell is its group's last)
-        const float p = s[n_old];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc[k] = fmaf(vcur[sub * 8 + k], p, acc[k]);
-    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
     __syncthreads();
@@ -1635,14 +1766,12 @@ int pi_k_attn_fused(const float * qkv, const void * rope_table, void * k_cache, 
 }
 
 // ---- attention with the cells of a head split over n_parts workgroups --------------------------------------------
-static size_t attn_part_lds_bytes(int hd, int s_cap) {
-    return sizeof(float) * ((size_t)s_cap + (size_t)(kAttnPartBlock / (hd / 8)) * hd + 3 * (size_t)hd);
-}
 static bool attn_part_geometry_ok(int hd) {
     return hd > 0 && hd % 8 == 0 && kAttnPartBlock % (hd / 8) == 0 && PI_WAVE % (hd / 8) == 0 && hd / 2 + hd <= kAttnPartBlock && hd <= 1024;
 }
 int pi_k_attn_split_supported(int hd, int n_ctx, int n_parts) {
-    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && attn_part_lds_bytes(hd, (n_ctx + n_parts - 1) / n_parts + 1) <= kAttnLdsLimit;
+    // (what attn_part_rounded_kernel's scores leave room for; parts of as many cells, about 11 k, are too long for the other kernel's good too)
+    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && attn_rounded_lds(hd, (n_ctx + n_parts - 1) / n_parts + 1) <= kAttnLdsLimit;
 }
 size_t pi_k_attn_split_scratch_floats(int n_seq, int n_head, int hd, int n_parts) { return (size_t)n_seq * n_head * n_parts * ((size_t)hd + 2); }
 
@@ -1652,12 +1781,11 @@ int pi_k_attn_split(const float * qkv, int qkv_stride, const void * rope_table, 
     if (!qkv || !rope_table || !k_cache || !v_cache || !pos || !out || !scratch || n_seq <= 0) return pi::fail(PI_E_ARG, "pi_k_attn_split: bad arguments");
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (mode != 0 && mode != 2) || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_split: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
-    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)n_seq * n_head * n_parts * hd;
     hipStream_t st = (hipStream_t)stream;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<false, LPP>), dim3(n_head, n_parts, n_seq), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, qkv, (const float2 *)rope_table,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml, qkv_stride, cache_seq_stride));
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<false, LPP>), dim3(n_head, n_parts, n_seq), dim3(kAttnPartBlock), attn_part_lds(hd), st, qkv, (const float2 *)rope_table,
+                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, acc, ml, qkv_stride, cache_seq_stride));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_seq), dim3(hd), 0, st, acc, ml, n_parts, hd, out, out_stride, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_split");
 }
@@ -1667,12 +1795,11 @@ int pi_k_attn_split_cached(const float * q_rot, const void * k_cache, const void
     if (!q_rot || !k_cache || !v_cache || !pos || !out || !scratch || n_tok <= 0 || n_tok > 65535) return pi::fail(PI_E_ARG, "pi_k_attn_split_cached: bad arguments");
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_split_cached: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
-    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)n_tok * n_head * n_parts * hd;
     hipStream_t st = (hipStream_t)stream;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
-                       (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0));
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), attn_part_lds(hd), st, q_rot, (const float2 *)nullptr,
+                       (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_head, n_head_kv, hd, 0, n_ctx, pos, acc, ml, n_head * hd, (size_t)0));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_tok), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)nullptr);
     return pi::check_launch("pi_k_attn_split_cached");
 }
@@ -1815,11 +1942,11 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     hipStream_t st = (hipStream_t)stream;
     const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     if (rc != PI_OK) return rc;
-    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
     float * acc = scratch;
     float * ml = scratch + (size_t)T * n_head * n_parts * hd;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, T), dim3(kAttnPartBlock), attn_part_lds_bytes(hd, s_cap), st, q_rot, (const float2 *)nullptr,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, 0, n_ctx, s_cap, pos, acc, ml, n_head * hd, (size_t)0));
+    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_rounded_kernel<LPP>), dim3(n_head, n_parts, T), dim3(kAttnPartBlock), attn_rounded_lds(hd, s_cap), st, q_rot, (const __half *)k_cache,
+                       (const __half *)v_cache, n_head, n_head_kv, hd, n_ctx, s_cap, pos, acc, ml, n_head * hd));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, T), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_chunk_long");
 }
