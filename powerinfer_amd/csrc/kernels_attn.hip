@@ -387,29 +387,25 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
 // (18 us per 7B layer at 600 cells, growing by 2.4 us per 100 cells); with n_parts workgroups per head every unit takes a share and
 // the score buffer in LDS holds n_ctx / n_parts cells instead of all of them.
 // Part s owns cells [n_kv * s / n, n_kv * (s + 1) / n); the last part holds the new cell: it rotates and stores k, stores v, and
-// uses them from LDS.  Every part rotates q and goes through its cells once: a group of lanes holds a cell's K and V row, and keeps a maximum
-// m, l = sum of e^(s - m) and acc = sum of v e^(s - m) of the cells it has seen, so that nothing waits for another group before the
-// rows have been read; at the end the groups' three meet in LDS.  The part hands (m, l, acc) to attn_merge_kernel, which rescales by exp(m - M), adds
-// the parts in order and divides by the total.  Weights stay in fp32 (the single workgroup's are rounded to fp16: the two differ by
-// those roundings, 1e-4 of the output).
-// Bound by the trips to memory of a part's rows.  Eight cells of a group, K and V, are on their way at any time, requested without a guard (a guarded
-// load makes the compiler wait for all the others; rows past the last cell are the last one again), and what the rotation needs ahead of
-// them, because loads return in order.  Merge included, against scores, soft-max and values one after the other with guarded loads: 32 heads of 128 in
-// 8 parts, 1030 cells 12.4 -> 11.0 us, 3001 19.4 -> 16.1 (49 MB), 32000 in 16 parts 97 -> 93; 128 heads of 64 in 2 parts, 1030 cells 14.2 -> 11.7.
+// uses them from LDS.  Every part rotates q, computes its scores, e_i = fp16(exp(fp16(s_i - m))) with ITS maximum m (the rounding
+// points of the CPU path's table, ggml.c:10747-10759), l = sum e_i in double and acc = sum v_i * e_i, and hands (m, l, acc) to
+// attn_merge_kernel, which rescales by exp(m - M), adds the parts in order and divides by the total.  Against one workgroup per head,
+// which knows the global maximum before it rounds, results differ in the last places of the fp16 roundings (1e-4 of the output).
+// Bound by the trips to memory of a part's rows.  A group of lanes holds a cell's rows, the same cells of keys and values, so nothing but the maximum
+// passes between groups before their sums meet.  Eight cells of a group, K and V, are on their way at any time, requested without a guard (a
+// guarded load makes the compiler wait for all the others; past the last cell its rows are read again), and what the rotation
+// needs ahead of them, because loads return in order.  Merge included, against the same sums with guarded loads and the soft-max of the whole workgroup
+// between two barriers: 32 heads of 128 in 8 parts, 1030 cells 12.4 -> 11.0 us, 3001 19.4 -> 16.4 (49 MB), 32000 in 16 parts 97 -> 93.5; 128
+// heads of 64 in 2 parts, 1030 cells 14.2 -> 12.3.
 // ---------------------------------------------------------------------------------------------------
 // FROM_CACHE: the token's own K / V row is in the cache already and qkv holds its rotated q only ([n_head * hd] per token; a prompt chunk
 // behind rope_kv_store_kernel): nothing is rotated or stored, every cell is read from the cache.
 constexpr int kAttnPartBlock = 512;
-constexpr int kAttnPartCells = 4;        // cells of a group that are requested, scored and weighed together; two such batches are in flight
-constexpr int kAttnPartFloats = kAttnPartBlock * 8;      // [groups][hd]
-static size_t attn_part_lds(int hd) {    // the groups' sums, two words of each, what the parts of a head's values add up to, and q, k, v
-    return sizeof(float) * (kAttnPartFloats + 2 * (size_t)(kAttnPartFloats / hd) + kAttnPartBlock + 2 * (size_t)(kAttnPartBlock / hd) + 3 * (size_t)hd);
-}
-static size_t attn_rounded_lds(int hd, int s_cap) { return sizeof(float) * ((size_t)s_cap + kAttnPartFloats + 3 * (size_t)hd); }
+constexpr int kAttnPartCells = 4;        // cells of a group that are requested and used together; two such batches are in flight
 template <bool FROM_CACHE, int LPP>
 __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
                                                                    __half * __restrict__ k_cache, __half * __restrict__ v_cache,
-                                                                   int n_head, int n_head_kv, int hd, int mode, int n_ctx,
+                                                                   int n_head, int n_head_kv, int hd, int mode, int n_ctx, int s_cap,
                                                                    const int32_t * __restrict__ pos_p, float * __restrict__ part_acc, float * __restrict__ part_ml,
                                                                    int qkv_stride, size_t cache_seq_stride) {
     qkv += (size_t)blockIdx.z * qkv_stride;
@@ -417,20 +413,21 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     v_cache += (size_t)blockIdx.z * cache_seq_stride;
     pos_p += blockIdx.z;
     extern __shared__ __align__(16) unsigned char smem[];
-    const int lpp = LPP ? LPP : hd / 8, ngrp = kAttnPartBlock / lpp, n_sum = kAttnPartBlock / hd;      // (hd divides 512; eight groups to each of the n_sum sums)
-    float * part = reinterpret_cast<float *>(smem);               // [ngrp][hd]
-    float * gm = part + kAttnPartFloats, * gl = gm + ngrp;        // [ngrp] the groups' maxima and sums
-    float * half = gl + ngrp;                                     // [n_sum][hd]
-    float * hm = half + kAttnPartBlock, * hl = hm + n_sum;        // [n_sum]
-    float * qs = hl + n_sum;                                      // [hd] rotated q, rounded to fp16
+    const int lpp = LPP ? LPP : hd / 8, ngrp = kAttnPartBlock / lpp;
+    double * gl  = reinterpret_cast<double *>(smem);              // [ngrp] the groups' sums of e_i
+    float * part = reinterpret_cast<float *>(gl + ngrp);          // [ngrp][hd]
+    float * gm   = part + kAttnPartBlock * 8;                     // [ngrp] the groups' maxima
+    float * qs   = gm + ngrp;                                     // [hd] rotated q, rounded to fp16
     float * kcur = qs + hd;                                       // [hd] rotated k of this position, rounded to fp16
     float * vcur = kcur + hd;                                     // [hd]
+    float * s    = vcur + hd;                                     // [s_cap] scores of this part
     const int h = blockIdx.x, n_parts = gridDim.y, sp = blockIdx.y, grp_sz = n_head / n_head_kv, kvh = h / grp_sz;
     const int tid = threadIdx.x;
     const int pos = *pos_p, n_kv = pos + 1;
     const int lo = (int)((long long)n_kv * sp / n_parts), hi = (int)((long long)n_kv * (sp + 1) / n_parts);
     const bool owns_new = !FROM_CACHE && sp == n_parts - 1;        // hi == n_kv: the new cell is this part's last
     const size_t slot = ((size_t)blockIdx.z * n_head + h) * n_parts + sp;
+    if (hi - lo > s_cap) return;                                  // cannot happen for pos < n_ctx (the launcher sizes s_cap); never write past LDS
     const float * qsrc = qkv + (size_t)h * hd;
     const int sub = tid % lpp, grp = tid / lpp;
     const int n_old = (owns_new ? hi - 1 : hi) - lo;              // cells of this part that live in the cache
@@ -446,20 +443,14 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     }
     const __half * kr = k_cache + ((size_t)kvh * n_ctx + lo) * hd + sub * 8, * vr = v_cache + ((size_t)kvh * n_ctx + lo) * hd + sub * 8;
     pi_u32x4 kk[2][kAttnPartCells], vv[2][kAttnPartCells];
-    auto fetch = [&](auto slot, int c0) {
-        constexpr int S = decltype(slot)::value;
+    auto fetch = [&](pi_u32x4 * dst, const __half * rows, int c0) {
 #pragma unroll
-        for (int u = 0; u < kAttnPartCells; ++u) {
-            const size_t c = (size_t)max(min(c0 + u * ngrp + grp, n_old - 1), 0) * hd;
-            kk[S][u] = pi_ld16(kr + c); vv[S][u] = pi_ld16(vr + c);
-        }
+        for (int u = 0; u < kAttnPartCells; ++u) dst[u] = pi_ld16(rows + (size_t)max(min(c0 + u * ngrp + grp, n_old - 1), 0) * hd);
     };
-    using First = std::integral_constant<int, 0>;
-    using Second = std::integral_constant<int, 1>;
     const int step = kAttnPartCells * ngrp;
     __builtin_amdgcn_sched_barrier(0);
-    fetch(First{}, 0);
-    fetch(Second{}, step);
+    fetch(kk[0], kr, 0); fetch(kk[1], kr, step);
+    fetch(vv[0], vr, 0); fetch(vv[1], vr, step);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (FROM_CACHE) {
         if (tid < hd) qs[tid] = pi_round_f16(q0);
@@ -485,183 +476,90 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     __syncthreads();
 
     const float scale = pi_inv_sqrt((float)hd);
-    float qf[8], acc[8], m = -INFINITY, l = 0.0f;
+    float qf[8], top = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) { qf[i] = qs[sub * 8 + i]; acc[i] = 0.0f; }
-    // N cells' scores and values into m, l and acc; f(u, e, acc): the values of cell u under the weight e
-    auto add = [&](auto n, const float * s, auto && f) {
-        constexpr int N = decltype(n)::value;
-        float top = m;
-#pragma unroll
-        for (int u = 0; u < N; ++u) top = fmaxf(top, s[u]);
-        const float base = top == -INFINITY ? 0.0f : top, down = __expf(__fsub_rn(m, base));
-        m = top; l *= down;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc[k] *= down;
-#pragma unroll
-        for (int u = 0; u < N; ++u) {
-            const float e = __expf(__fsub_rn(s[u], base));
-            l += e;
-            f(u, e);
+    for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
+    // the two batches in turn; f(which, first cell) uses a batch, then its registers are requested again for the next cells but one
+    auto through = [&](pi_u32x4 (*regs)[kAttnPartCells], const __half * rows, auto && f) {
+        for (int c0 = 0; c0 < n_old; c0 += 2 * step) {
+            f(regs[0], c0);
+            if (c0 + step >= n_old) break;
+            fetch(regs[0], rows, c0 + 2 * step);
+            f(regs[1], c0 + step);
+            fetch(regs[1], rows, c0 + 3 * step);
         }
     };
-    auto batch = [&](auto slot, int c0) {
-        constexpr int S = decltype(slot)::value;
-        float s[kAttnPartCells];
+    through(kk, kr, [&](const pi_u32x4 * k, int c0) {
 #pragma unroll
-        for (int u = 0; u < kAttnPartCells; ++u) s[u] = pi_group_sum<LPP>(pi_dot8(kk[S][u], qf, 0.0f), lpp);
-#pragma unroll
-        for (int u = 0; u < kAttnPartCells; ++u) s[u] = c0 + u * ngrp + grp < n_old ? __fmul_rn(s[u], scale) : -INFINITY;
-        add(std::integral_constant<int, kAttnPartCells>{}, s, [&](int u, float e) {
-            float vf[8];
-            pi_unpack8(vv[S][u], vf);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], e, acc[k]);
-        });
-    };
-    for (int c0 = 0; c0 < n_old; c0 += 2 * step) {
-        batch(First{}, c0);
-        if (c0 + step >= n_old) break;
-        fetch(First{}, c0 + 2 * step);
-        batch(Second{}, c0 + step);
-        fetch(Second{}, c0 + 3 * step);
-    }
-    if (owns_new && grp == n_old % ngrp) {
+        for (int u = 0; u < kAttnPartCells; ++u) {
+            const int c = c0 + u * ngrp + grp;
+            const float d = __fmul_rn(pi_group_sum<LPP>(pi_dot8(k[u], qf, 0.0f), lpp), scale);
+            if (c < n_old) { top = fmaxf(top, d); if (sub == 0) s[c] = d; }
+        }
+    });
+    const bool mine = owns_new && grp == n_old % ngrp;              // the new cell is this group's last
+    if (mine) {
         float d = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) d = fmaf(kcur[sub * 8 + k], qf[k], d);
         d = __fmul_rn(pi_group_sum<LPP>(d, lpp), scale);
-        add(std::integral_constant<int, 1>{}, &d, [&](int, float e) {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) acc[k] = fmaf(vcur[sub * 8 + k], e, acc[k]);
-        });
+        top = fmaxf(top, d);
+        if (sub == 0) s[n_old] = d;
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
-    if (sub == 0) { gm[grp] = m; gl[grp] = l; }
+    if (sub == 0) gm[grp] = top;
     __syncthreads();
-    // value e of eight groups by every thread, then of the n_sum sums of eight by one
-    {
-        const int e = tid % hd, j = tid / hd;
-        float M = -INFINITY, L = 0.0f, v = 0.0f;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) M = fmaxf(M, gm[j * 8 + g]);
-        const float base = M == -INFINITY ? 0.0f : M;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const float w = __expf(__fsub_rn(gm[j * 8 + g], base));
-            L = fmaf(gl[j * 8 + g], w, L);
-            v = fmaf(part[(j * 8 + g) * hd + e], w, v);
-        }
-        half[j * hd + e] = v;
-        if (e == 0) { hm[j] = M; hl[j] = L; }
-    }
-    __syncthreads();
-    if (tid < hd) {
-        float M = -INFINITY, L = 0.0f, v = 0.0f;
-        for (int j = 0; j < n_sum; ++j) M = fmaxf(M, hm[j]);
-        const float base = M == -INFINITY ? 0.0f : M;
-        for (int j = 0; j < n_sum; ++j) {
-            const float w = __expf(__fsub_rn(hm[j], base));
-            L = fmaf(hl[j], w, L);
-            v = fmaf(half[j * hd + tid], w, v);
-        }
-        part_acc[slot * hd + tid] = v;
-        if (tid == 0) { part_ml[slot * 2] = M; part_ml[slot * 2 + 1] = L; }
-    }
-}
-
-// The same for the tokens of a prompt chunk (pi_k_attn_chunk_long; K / V rows and rotated queries are stored): scores first, then e_i = fp16(exp(fp16(s_i - m))) with the part's
-// maximum m, the rounding points of the CPU path's table (ggml.c:10747-10759), then the values.
-constexpr int kAttnPartPre = 8;          // passes whose K and V rows are in flight: one use of a row requests the row eight passes on
-template <int LPP>
-__global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_rounded_kernel(const float * __restrict__ q_rot, const __half * __restrict__ k_cache, const __half * __restrict__ v_cache, int n_head, int n_head_kv,
-                                                                             int hd, int n_ctx, int s_cap, const int32_t * __restrict__ pos_p, float * __restrict__ part_acc,
-                                                                             float * __restrict__ part_ml, int q_stride) {
-    q_rot += (size_t)blockIdx.z * q_stride;
-    pos_p += blockIdx.z;
-    extern __shared__ __align__(16) unsigned char smem[];
-    float * s    = reinterpret_cast<float *>(smem);               // [s_cap] scores of this part, then e_i
-    float * part = s + s_cap;                                     // [groups][hd]
-    float * qs   = part + kAttnPartFloats;                        // [hd] rotated q, rounded to fp16
-    __shared__ double red[16];
-    __shared__ float redf[16];
-    const int h = blockIdx.x, n_parts = gridDim.y, sp = blockIdx.y, grp_sz = n_head / n_head_kv, kvh = h / grp_sz;
-    const int tid = threadIdx.x;
-    const int n_kv = *pos_p + 1;
-    const int lo = (int)((long long)n_kv * sp / n_parts), hi = (int)((long long)n_kv * (sp + 1) / n_parts);
-    const size_t slot = ((size_t)blockIdx.z * n_head + h) * n_parts + sp;
-    if (hi - lo > s_cap) return;                                  // cannot happen for pos < n_ctx (the launcher sizes s_cap); never write past LDS
-    const int lpp = LPP ? LPP : hd / 8;
-    const int sub = tid % lpp, grp = tid / lpp, ngrp = kAttnPartBlock / lpp;
-    const __half * kb = k_cache + (size_t)kvh * n_ctx * hd;
-    const __half * vb = v_cache + (size_t)kvh * n_ctx * hd;
-    const int n_mine = hi - lo;
-    pi_u32x4 kpre[kAttnPartPre], vpre[kAttnPartPre];
-    const __half * kr = kb + (size_t)lo * hd + sub * 8, * vr = vb + (size_t)lo * hd + sub * 8;
-#pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_mine) kpre[i] = pi_ld16(kr + (size_t)c * hd); }
-#pragma unroll
-    for (int i = 0; i < kAttnPartPre; ++i) { const int c = i * ngrp + grp; if (c < n_mine) vpre[i] = pi_ld16(vr + (size_t)c * hd); }
-    if (tid < hd) qs[tid] = pi_round_f16(q_rot[(size_t)h * hd + tid]);
-    __syncthreads();
-
-    const float scale = pi_inv_sqrt((float)hd);
-    float qf[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) qf[i] = qs[sub * 8 + i];
-    for (int c0 = 0; c0 < n_mine; c0 += kAttnPartPre * ngrp)
-#pragma unroll
-        for (int i = 0; i < kAttnPartPre; ++i) {                    // (a row past the last is whatever the registers hold, and not used)
-            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
-            const float d = pi_group_sum<LPP>(pi_dot8(kpre[i], qf, 0.0f), lpp);
-            if (next < n_mine) kpre[i] = pi_ld16(kr + (size_t)next * hd);
-            if (c < n_mine && sub == 0) s[c] = __fmul_rn(d, scale);
-        }
-    __syncthreads();
-
     float mx = -INFINITY;
-    for (int c = tid; c < n_mine; c += kAttnPartBlock) mx = fmaxf(mx, s[c]);
-    mx = block_max_f32(mx, redf);
-    double sum = 0.0;
-    for (int c = tid; c < n_mine; c += kAttnPartBlock) {
-        const float e = pi_round_f16(expf(pi_round_f16(__fsub_rn(s[c], mx))));
-        s[c] = e;
-        sum += (double)e;
-    }
-    sum = block_sum_f64(sum, red);
+    for (int g = 0; g < ngrp; g += 8)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, gm[g + j]);
 
     float acc[8];
+    double sum = 0.0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.0f;
-    for (int c0 = 0; c0 < n_mine; c0 += kAttnPartPre * ngrp)
+    auto weight = [&](int c) { return pi_round_f16(expf(pi_round_f16(__fsub_rn(s[c], mx)))); };
+    through(vv, vr, [&](const pi_u32x4 * v, int c0) {
+        float e[kAttnPartCells];
 #pragma unroll
-        for (int i = 0; i < kAttnPartPre; ++i) {
-            const int c = c0 + i * ngrp + grp, next = c + kAttnPartPre * ngrp;
-            if (c < n_mine) {
-                const float p = s[c];
-                float vf[8];
-                pi_unpack8(vpre[i], vf);
-                if (next < n_mine) vpre[i] = pi_ld16(vr + (size_t)next * hd);
+        for (int u = 0; u < kAttnPartCells; ++u) e[u] = weight(min(c0 + u * ngrp + grp, n_old - 1));
 #pragma unroll
-                for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], p, acc[k]);
+        for (int u = 0; u < kAttnPartCells; ++u) {
+            float vf[8];
+            pi_unpack8(v[u], vf);
+            if (c0 + u * ngrp + grp < n_old) {
+                sum += (double)e[u];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) acc[k] = fmaf(vf[k], e[u], acc[k]);
             }
         }
+    });
+    if (mine) {
+        const float e = weight(n_old);
+        sum += (double)e;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] = fmaf(vcur[sub * 8 + k], e, acc[k]);
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
+    if (sub == 0) gl[grp] = sum;
     __syncthreads();
-    for (int e = tid; e < hd; e += kAttnPartBlock) {
-        float v = part[e];
+    if (tid < hd) {
+        float v = part[tid];
         for (int g0 = 0; g0 < ngrp; g0 += 8) {                     // (ngrp: a multiple of 8; eight reads in flight, added in order)
             float t[8];
 #pragma unroll
-            for (int g = 0; g < 8; ++g) t[g] = part[(g0 + g) * hd + e];
+            for (int g = 0; g < 8; ++g) t[g] = part[(g0 + g) * hd + tid];
 #pragma unroll
             for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
         }
-        part_acc[slot * hd + e] = v;
+        part_acc[slot * hd + tid] = v;
+    } else if (tid == hd) {                                         // (whole numbers of 2^-24: exact in any order)
+        double l = 0.0;
+        for (int g = 0; g < ngrp; g += 8)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) l += gl[g + j];
+        part_ml[slot * 2] = mx; part_ml[slot * 2 + 1] = (float)l;
     }
-    if (tid == 0) { part_ml[slot * 2] = n_mine > 0 ? mx : -INFINITY; part_ml[slot * 2 + 1] = (float)sum; }
 }
 
 // out[h][e] = sum_s acc_s[e] * exp(m_s - M) / sum_s l_s * exp(m_s - M), parts in ascending order; one workgroup of hd threads per head
@@ -1746,6 +1644,21 @@ int pi_k_attn_decode_supported(int hd, int n_ctx) {
 // the lanes of a cell are a constant for the two usual head sizes (their sums are then lane permutations)
 #define PI_ATTN_LPP(...) do { if (hd == 128) { constexpr int LPP = 16; __VA_ARGS__; } else if (hd == 64) { constexpr int LPP = 8; __VA_ARGS__; } \
                               else { constexpr int LPP = 0; __VA_ARGS__; } } while (0)
+// the parts and their merge; LDS: what pi_k_attn_split_supported counts and three words a group, 6 KB for heads of eight values
+template <bool FROM_CACHE>
+static int launch_attn_parts(const float * qkv, const float2 * rope_table, __half * k, __half * v, int n_tok, int n_head, int n_head_kv, int hd, int mode, int n_ctx, int n_parts, const int32_t * pos,
+                             float * scratch, int qkv_stride, size_t cache_seq_stride, float * out, int out_stride, __half * out_f16, hipStream_t st, const char * name) {
+    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
+    const size_t lds = sizeof(float) * ((size_t)s_cap + kAttnPartBlock * 8 + 3 * (size_t)hd + 3 * (size_t)(kAttnPartBlock * 8 / hd));
+    float * acc = scratch, * ml = scratch + (size_t)n_tok * n_head * n_parts * hd;
+    PI_ATTN_LPP(
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_part_kernel<FROM_CACHE, LPP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAttnLdsLimit + 8192);
+        if (raised != hipSuccess) return pi::hip_fail(raised, "attn_part: LDS size");
+        hipLaunchKernelGGL((attn_part_kernel<FROM_CACHE, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), lds, st, qkv, rope_table, k, v, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml,
+                           qkv_stride, cache_seq_stride));
+    hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_tok), dim3(hd), 0, st, acc, ml, n_parts, hd, out, out_stride, out_f16);
+    return pi::check_launch(name);
+}
 namespace pi {
 int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream) {
@@ -1770,8 +1683,7 @@ static bool attn_part_geometry_ok(int hd) {
     return hd > 0 && hd % 8 == 0 && kAttnPartBlock % (hd / 8) == 0 && PI_WAVE % (hd / 8) == 0 && hd / 2 + hd <= kAttnPartBlock && hd <= 1024;
 }
 int pi_k_attn_split_supported(int hd, int n_ctx, int n_parts) {
-    // (what attn_part_rounded_kernel's scores leave room for; parts of as many cells, about 11 k, are too long for the other kernel's good too)
-    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && attn_rounded_lds(hd, (n_ctx + n_parts - 1) / n_parts + 1) <= kAttnLdsLimit;
+    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && sizeof(float) * ((size_t)(n_ctx + n_parts - 1) / n_parts + 1 + kAttnPartBlock * 8 + 3 * (size_t)hd) <= kAttnLdsLimit;
 }
 size_t pi_k_attn_split_scratch_floats(int n_seq, int n_head, int hd, int n_parts) { return (size_t)n_seq * n_head * n_parts * ((size_t)hd + 2); }
 
@@ -1781,13 +1693,8 @@ int pi_k_attn_split(const float * qkv, int qkv_stride, const void * rope_table, 
     if (!qkv || !rope_table || !k_cache || !v_cache || !pos || !out || !scratch || n_seq <= 0) return pi::fail(PI_E_ARG, "pi_k_attn_split: bad arguments");
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || (mode != 0 && mode != 2) || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_split: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
-    float * acc = scratch;
-    float * ml = scratch + (size_t)n_seq * n_head * n_parts * hd;
-    hipStream_t st = (hipStream_t)stream;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<false, LPP>), dim3(n_head, n_parts, n_seq), dim3(kAttnPartBlock), attn_part_lds(hd), st, qkv, (const float2 *)rope_table,
-                       (__half *)k_cache, (__half *)v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos, acc, ml, qkv_stride, cache_seq_stride));
-    hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_seq), dim3(hd), 0, st, acc, ml, n_parts, hd, out, out_stride, (__half *)out_f16);
-    return pi::check_launch("pi_k_attn_split");
+    return launch_attn_parts<false>(qkv, (const float2 *)rope_table, (__half *)k_cache, (__half *)v_cache, n_seq, n_head, n_head_kv, hd, mode, n_ctx, n_parts, pos, scratch, qkv_stride,
+                                    cache_seq_stride, out, out_stride, (__half *)out_f16, (hipStream_t)stream, "pi_k_attn_split");
 }
 
 int pi_k_attn_split_cached(const float * q_rot, const void * k_cache, const void * v_cache, int n_tok, int n_head, int n_head_kv, int hd,
@@ -1795,13 +1702,8 @@ int pi_k_attn_split_cached(const float * q_rot, const void * k_cache, const void
     if (!q_rot || !k_cache || !v_cache || !pos || !out || !scratch || n_tok <= 0 || n_tok > 65535) return pi::fail(PI_E_ARG, "pi_k_attn_split_cached: bad arguments");
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || !pi_k_attn_split_supported(hd, n_ctx, n_parts))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_split_cached: head size, context per part or part count outside the kernel (pi_k_attn_split_supported)");
-    float * acc = scratch;
-    float * ml = scratch + (size_t)n_tok * n_head * n_parts * hd;
-    hipStream_t st = (hipStream_t)stream;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<true, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), attn_part_lds(hd), st, q_rot, (const float2 *)nullptr,
-                       (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_head, n_head_kv, hd, 0, n_ctx, pos, acc, ml, n_head * hd, (size_t)0));
-    hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_tok), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)nullptr);
-    return pi::check_launch("pi_k_attn_split_cached");
+    return launch_attn_parts<true>(q_rot, nullptr, (__half *)const_cast<void *>(k_cache), (__half *)const_cast<void *>(v_cache), n_tok, n_head, n_head_kv, hd, 0, n_ctx, n_parts, pos, scratch,
+                                   n_head * hd, 0, out, n_head * hd, nullptr, (hipStream_t)stream, "pi_k_attn_split_cached");
 }
 
 static int attn_fused_batch(const float * qkv, int qkv_stride, const void * rope_table, void * k_cache, void * v_cache, size_t cache_seq_stride,
@@ -1942,13 +1844,8 @@ int pi_k_attn_chunk_long(const float * qkv, int qkv_stride, int T, int n_head, i
     hipStream_t st = (hipStream_t)stream;
     const int rc = pi::rope_kv_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, k_cache, v_cache, st);
     if (rc != PI_OK) return rc;
-    float * acc = scratch;
-    float * ml = scratch + (size_t)T * n_head * n_parts * hd;
-    const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
-    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_rounded_kernel<LPP>), dim3(n_head, n_parts, T), dim3(kAttnPartBlock), attn_rounded_lds(hd, s_cap), st, q_rot, (const __half *)k_cache,
-                       (const __half *)v_cache, n_head, n_head_kv, hd, n_ctx, s_cap, pos, acc, ml, n_head * hd));
-    hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, T), dim3(hd), 0, st, acc, ml, n_parts, hd, out, n_head * hd, (__half *)out_f16);
-    return pi::check_launch("pi_k_attn_chunk_long");
+    return launch_attn_parts<true>(q_rot, nullptr, (__half *)k_cache, (__half *)v_cache, T, n_head, n_head_kv, hd, 0, n_ctx, n_parts, pos, scratch, n_head * hd, 0, out, n_head * hd,
+                                   (__half *)out_f16, st, "pi_k_attn_chunk_long");
 }
 
 static size_t attn_ggml_lds(int hd, int n_kv, int T) {
