@@ -645,6 +645,8 @@ typedef struct pi_group_gemm {
 PI_API int pi_k_group_gemm(int type, const pi_group_gemm * g, pi_stream_t stream);
 /* the same for many tokens, bf16, both operands tiled through LDS (cols % 64 == 0); tile_n 64 or 128 tokens per tile, as given to pi_k_moe_sort */
 PI_API int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream);
+/* the same in tiles of 256 tokens (tiles: pi_k_moe_sort's with tile_n 256): off != NULL, more than 64 rows, at least 256 columns */
+PI_API int pi_k_group_gemm_tall(const pi_group_gemm * g, pi_stream_t stream);
 /* (cos, sin)[t][i] of the angles pos[t] * base^(-2i / dims), i < dims / 2 */
 PI_API int pi_k_rope_angles(const int32_t * pos, int T, int dims, double base, void * cs_float2, pi_stream_t stream);
 /* the same with given frequencies (dims / 2 of them), cosine and sine times length */

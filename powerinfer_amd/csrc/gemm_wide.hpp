@@ -26,19 +26,19 @@ constexpr int kGwBand = 8;
 // than 128 rows first, then the shorter ones, which take half the time.  What does not fill the XCD's
 // workgroups once more at the end is cut into halves of 128 rows if that gives no workgroup two of them.
 struct WideDeal {
-    int rows, n_tiles, band, nl, xcd, slot, slots, per_long, per_short, n_long, rounds, rest_unit, rest_row, count;
+    int rows, n_tiles, band, tile, nl, xcd, slot, slots, per_long, per_short, n_long, rounds, rest_unit, rest_row, count;
     bool halves;
-    __device__ __forceinline__ WideDeal(int rows_, int n_tiles_, int band_) {
-        rows = rows_; n_tiles = n_tiles_; band = band_;
-        const int nx = (rows + kGwM - 1) / kGwM, last = rows - (nx - 1) * kGwM;
-        nl = last > kGwM / 2 ? nx : nx - 1;
+    __device__ __forceinline__ WideDeal(int rows_, int n_tiles_, int band_, int tile_ = kGwM) {
+        rows = rows_; n_tiles = n_tiles_; band = band_; tile = tile_;
+        const int nx = (rows + tile - 1) / tile, last = rows - (nx - 1) * tile;
+        nl = last > tile / 2 ? nx : nx - 1;
         xcd = (int)blockIdx.x % 8; slot = (int)blockIdx.x / 8; slots = (int)gridDim.x / 8;
         per_long = (n_tiles * nl + 7) / 8; per_short = nl < nx ? (n_tiles + 7) / 8 : 0;
         n_long = max(min(n_tiles * nl - xcd * per_long, per_long), 0);
         const int n = n_long + max(min(nl < nx ? n_tiles - xcd * per_short : 0, per_short), 0), rest = n % slots;
         rounds = n / slots;
         halves = rest > 0 && 2 * rest <= slots;
-        rest_unit = rounds * slots + (halves ? slot / 2 : slot); rest_row = halves ? slot % 2 * (kGwM / 2) : 0;
+        rest_unit = rounds * slots + (halves ? slot / 2 : slot); rest_row = halves ? slot % 2 * (tile / 2) : 0;
         count = rounds + (slot < (halves ? 2 * rest : rest) && !(rest_row && rest_unit >= n_long) ? 1 : 0);
     }
     // the c-th of them: its token tile, its first row and how many there are
@@ -46,12 +46,12 @@ struct WideDeal {
         const int u = c < rounds ? c * slots + slot : rest_unit;
         if (u < n_long) {
             const int at = xcd * per_long + u, b0 = at / (band * nl) * band, high = min(band, n_tiles - b0), in = at - b0 * nl;
-            ty = b0 + in % high; row0 = in / high * kGwM;
+            ty = b0 + in % high; row0 = in / high * tile;
         } else {
-            ty = xcd * per_short + u - n_long; row0 = (rows - 1) / kGwM * kGwM;
+            ty = xcd * per_short + u - n_long; row0 = (rows - 1) / tile * tile;
         }
         if (c >= rounds) row0 += rest_row;
-        n_rows = min(rows - row0, c < rounds || !halves ? kGwM : kGwM / 2);
+        n_rows = min(rows - row0, c < rounds || !halves ? tile : tile / 2);
     }
 };
 inline unsigned wide_blocks(long long units) { return (unsigned)(units < 128 ? (2 * units + 7) / 8 * 8 : 256); }
@@ -60,38 +60,47 @@ struct WidePlace { int grp, lo, n, row0, rows; };       // of a unit: group, fir
 
 // P (a product): nk stages of 64 columns; place(deal, c); base_a(p, w), base_b(p): where the rows of a tile's w-th 64 rows and its tokens start, and
 // off_a(p, r), off_b(p, r): the bytes from there to tile row and token r (in range: r is cut to the unit's); kPairs: a wave's rows
-// are two runs of MT / 2 tiles, `gap` rows apart beyond their own where MT is 4; store<MT>(p, rb, tb, acc, turn, lane): the
+// are two runs of MT / 2 tiles, `gap` rows apart beyond their own where MT is 4; read_once(p): no other unit reads these rows of W; first(p): the column stage a unit begins with; kM, kN: the tile; store<MT>(p, rb, tb, acc, turn, lane): the
 // outputs of rows rb .. and tokens tb .. of the tile.
 template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(const P & prod, const WideDeal & deal, unsigned char * smem) {
     if (deal.count == 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
+    constexpr int M = P::kM, N = P::kN, CA = M / 32, CB = N / 32;   // rows and tokens of a tile, copies of a wave a stage (twelve)
+    static_assert(CA + CB == 12, "the waits below count them");
     const int nk = prod.nk, count = deal.count;
     WidePlace * places = reinterpret_cast<WidePlace *>(smem + kGwStages * kGwStage);      // of this unit and those behind it, written by the first copying wave
     if (wave >= 4) {
         // A wave that copies.  Of each stage eight times eight rows of W and four times eight of x are its own, each 128 bytes; lane l brings
         // the piece that belongs at place l % 8 of row l / 8
         const int w = wave - 4, piece = ((lane & 7) ^ (lane >> 3)) * 16;
-        uint32_t va[8];
-        size_t vb[4];
+        uint32_t va[CA];
+        size_t vb[CB];
         const unsigned char * fa, * fb;
-        int k = 0, c = 0;
+        int k = 0, c = 0, first = 0;                                // a unit's stages are copied from column stage `first` on, around the end
+        bool once = false;
         auto aim = [&]() {
             const WidePlace p = prod.place(deal, c);
             if (w == 0 && lane == 0) places[c & 3] = p;
             ++c;
-            fa = prod.base_a(p, w); fb = prod.base_b(p);
+            fa = prod.base_a(p, w); fb = prod.base_b(p); once = prod.read_once(p); first = prod.first(p);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) va[j] = prod.off_a(p, min(64 * w + 8 * j + (lane >> 3), p.rows - 1)) + piece;
+            for (int j = 0; j < CA; ++j) va[j] = prod.off_a(p, min(8 * CA * w + 8 * j + (lane >> 3), p.rows - 1)) + piece;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) vb[j] = prod.off_b(p, min(32 * w + 8 * j + (lane >> 3), p.n - 1)) + piece;
+            for (int j = 0; j < CB; ++j) vb[j] = prod.off_b(p, min(8 * CB * w + 8 * j + (lane >> 3), p.n - 1)) + piece;
         };
         typedef const __attribute__((address_space(1))) void * gptr;
         typedef __attribute__((address_space(3))) void * lptr;
         auto copy_stage = [&](unsigned char * stage) {             // past the last unit the last stage is copied again, and not used
+            const size_t at = (size_t)(first + k < nk ? first + k : first + k - nk) * kGtRow;
+            if (once) {                                            // (the last operand of the builtin: 2 is the non-temporal hint)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + (size_t)k * kGtRow + va[j]), (lptr)(stage + (64 * w + 8 * j) * kGtRow), 16, 0, 0);
+                for (int j = 0; j < CA; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + at + va[j]), (lptr)(stage + 8 * (CA * w + j) * kGtRow), 16, 0, 2);
+            } else {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) __builtin_amdgcn_global_load_lds((gptr)(fb + (size_t)k * kGtRow + vb[j]), (lptr)(stage + (kGwM + 32 * w + 8 * j) * kGtRow), 16, 0, 0);
+                for (int j = 0; j < CA; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + at + va[j]), (lptr)(stage + 8 * (CA * w + j) * kGtRow), 16, 0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < CB; ++j) __builtin_amdgcn_global_load_lds((gptr)(fb + at + vb[j]), (lptr)(stage + (M + 8 * (CB * w + j)) * kGtRow), 16, 0, 0);
             if (++k < nk) return;
             if (c < count) { k = 0; aim(); } else k = nk - 1;
         };
@@ -124,7 +133,7 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
 #pragma unroll
             for (int n = 0; n < 4; ++n) acc[m][n] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
         pi_u32x4 f0a[MT], f0b[4], f1a[MT], f1b[4];
-        const int oa = (rb + i) * kGtRow, ob = (kGwM + tb + i) * kGtRow;
+        const int oa = (rb + i) * kGtRow, ob = (M + tb + i) * kGtRow;
         auto ld = [&](int off) { return *reinterpret_cast<const pi_u32x4 *>(smem + cb * kGwStage + off); };
         auto lda = [&](int m, int h) { return ld(oa + koff[h] + (m * 16 + (m >= MT / 2 ? kGap : 0)) * kGtRow); };
         auto ldb = [&](int n, int h) { return ld(ob + koff[h] + n * 16 * kGtRow); };
@@ -173,13 +182,27 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
         }
         prod.template store<MT>(p, rb, tb, acc, turn, lane);
     };
+    auto idle = [&]() {                                             // no tokens of this tile
+        for (int kt = 0; kt < nk; ++kt) {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            cb = cb == kGwStages - 1 ? 0 : cb + 1;
+        }
+        asm volatile("" ::: "memory");
+    };
     for (int c = 0; c < count; ++c) {
         const int * pl = reinterpret_cast<const int *>(places + (c & 3));
         WidePlace p;
         p.grp = __builtin_amdgcn_readfirstlane(pl[0]); p.lo = __builtin_amdgcn_readfirstlane(pl[1]); p.n = __builtin_amdgcn_readfirstlane(pl[2]); p.row0 = __builtin_amdgcn_readfirstlane(pl[3]);
         p.rows = __builtin_amdgcn_readfirstlane(pl[4]);
         constexpr int kStep = P::kPairs ? 32 : 64;
-        if (p.rows <= 128) run(std::integral_constant<int, 4>{}, p, kStep * (wave & 1), 64 * (wave >> 1));
+        if constexpr (M == 128) {
+            const bool half = p.rows <= 64, pairs = !half && p.n <= 128;
+            const int tb = pairs ? 64 * (wave >> 1) : 64 * wave;
+            if (tb >= p.n) idle();
+            else if (half || pairs) run(std::integral_constant<int, 4>{}, p, pairs ? 64 * (wave & 1) : 0, tb);
+            else run(std::integral_constant<int, 8>{}, p, 0, tb);
+        } else if (p.rows <= 128) run(std::integral_constant<int, 4>{}, p, kStep * (wave & 1), 64 * (wave >> 1));
         else if (p.n <= 64) run(std::integral_constant<int, 4>{}, p, 128 * (wave >> 1) + kStep * (wave & 1), 0);
         else run(std::integral_constant<int, 8>{}, p, 128 * (wave & 1), 64 * (wave >> 1));
     }

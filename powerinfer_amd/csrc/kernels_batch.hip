@@ -523,6 +523,11 @@ __global__ __launch_bounds__(256) void ffn_h_q8_ol_kernel(const float * __restri
 // accumulators lie.
 template <bool PAIRS, bool MASK> struct FfnProduct {
     static constexpr bool kPairs = PAIRS;
+    static constexpr int kM = kGwM, kN = kGwN;
+    __device__ __forceinline__ bool read_once(const WidePlace &) const { return false; }
+    // Rows a multiple of 4 KB apart lie in few of the memory's channels: an XCD's workgroups, which share what they read, begin at columns of their own (bits
+    // included, us: 32768 x 8192 alone, 129 tokens 160 -> 137, 200 173 -> 151, 2047 1009 -> 994; 11008 x 4096 twice, 2047 tokens 359 -> 354).
+    __device__ __forceinline__ int first(const WidePlace &) const { return cols % 2048 ? 0 : (int)(blockIdx.x % 8) * nk / 8; }
     const __half * up, * gate, * x; const float * logits; float thr; __half * h16;
     int ff, cols, T, nk;
     const unsigned long long * mask;
@@ -582,6 +587,9 @@ template <bool PAIRS, bool MASK> struct FfnProduct {
 // 1285; 13B 400 tokens 1408 -> 1378, 40B 700 tokens 1550 -> 1531.
 struct MaskProduct {
     static constexpr bool kPairs = false;
+    static constexpr int kM = kGwM, kN = kGwN;
+    __device__ __forceinline__ bool read_once(const WidePlace &) const { return false; }
+    __device__ __forceinline__ int first(const WidePlace &) const { return 0; }
     const __half * W, * x; float thr; unsigned long long * mask;
     int rows, cols, T, nk;
     __device__ __forceinline__ WidePlace place(const WideDeal & deal, int c) const {

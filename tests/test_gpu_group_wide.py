@@ -144,3 +144,65 @@ def test_what_products_under_bits_refuse():
     d = pl.DevBuf.zeros(1 << 20)
     call = lambda rank=256, ff=128, cols=256, fc2=d.ptr, mask=d.ptr, T=3: L.pi_k_ffn_wide_predicted_f16(fc2, rank, d.ptr, d.ptr, None, ff, cols, d.ptr, T, 0.0, mask, d.ptr, None)  # noqa: E731
     assert call(rank=128) != 0 and call(ff=64) != 0 and call(rank=300) != 0 and call(T=0) != 0 and call(fc2=d.ptr + 8) != 0 and call(mask=None) != 0 and call(mask=d.ptr + 8) != 0
+
+
+def listed(counts, rows, cols, kind, y_f32, tile, tall):
+    """One grouped product in tiles of `tile` tokens: what it wrote, as bits and as values, and float64 (None with a GLU)."""
+    rng = np.random.default_rng(rows + cols)
+    E, n, div = len(counts), sum(counts), 3
+    T = (n + div - 1) // div
+    W = rounded(rng.standard_normal((E, rows, cols), dtype=np.float32) / np.sqrt(cols))
+    x = rounded(rng.standard_normal((T, cols), dtype=np.float32))
+    perm = rng.permutation(T * div)[:n].astype(np.int32)
+    pw = rng.random(T * div).astype(np.float32)
+    off = np.concatenate([[0], np.cumsum(counts)])
+    glu = kind in ("glu", "pair")
+    ldy = ((rows // 2 if glu else rows) + 7) // 8 * 8
+    tl = np.array([(e, p) for e in range(E) for p in range(off[e], off[e + 1], tile)], np.int32)
+    bufs = [store(W.reshape(-1, cols), pl.BF16), store(x, pl.BF16), i32(off), i32(perm), dev(pw), i32(tl), i32([len(tl)]), pl.DevBuf.zeros(4 * n * ldy + 64)]
+    g = group_args(W=bufs[0].ptr, w_gs=rows * cols, rows=rows, cols=cols, ldw=cols, n_group=E, x=bufs[1].ptr, ldx=cols, T=T, ldy=ldy, y_f32=y_f32, relu2=int(kind == "relu2"),
+                   alpha=1.25, off=bufs[2].ptr, gather=bufs[3].ptr, gather_div=div, tiles=bufs[5].ptr, n_tiles=bufs[6].ptr, max_tiles=len(tl) + 3, glu=int(glu), glu_limit=5.0, glu_gain=1.5,
+                   pair_w=bufs[4].ptr if kind == "pair" else None, y=bufs[7].ptr)
+    print(rows, cols, kind, tile, tall, flush=True)
+    pl.check(pl.init().pi_k_group_gemm_tall(C.byref(g), None) if tall else pl.init().pi_k_group_gemm_tile(C.byref(g), tile, None))
+    pl.sync()
+    got = bufs[7].download(np.uint32 if y_f32 else np.uint16)
+    assert not got[n * ldy:].any()
+    want = None
+    if not glu:
+        want = np.concatenate([1.25 * (x[perm[off[e]:off[e + 1]] // div].astype(np.float64) @ W[e].T.astype(np.float64)) for e in range(E)])
+        want = np.maximum(want, 0) ** 2 if kind == "relu2" else want
+    return got[:n * ldy].reshape(n, ldy), fetch(bufs[7], pl.F32 if y_f32 else pl.BF16, (n, ldy))[:, :rows], want
+
+
+COUNTS = [0, 1, 16, 63, 64, 65, 128, 129, 192, 193, 0, 255, 256, 257, 300, 40]
+
+
+@pytest.mark.parametrize("rows,cols,kind,y_f32", [(72, 256, "plain", 0), (128, 320, "relu2", 0), (136, 256, "plain", 1), (192, 512, "glu", 0), (200, 256, "relu2", 0),
+                                                  (270, 256, "plain", 0), (528, 384, "glu", 0), (400, 256, "pair", 0), (300, 256, "glu", 0)])
+def test_tiles_of_256_tokens(rows, cols, kind, y_f32):
+    """128 rows x 256 tokens: the sums of the small tiles, in their order."""
+    small, _, _ = listed(COUNTS, rows, cols, kind, y_f32, 64, False)
+    tall, got, want = listed(COUNTS, rows, cols, kind, y_f32, 256, True)
+    same(small, tall, y_f32)
+    if want is not None:
+        assert np.abs(got - want).max() <= (1e-5 if y_f32 else 2.0 ** -7) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("rows,cols,tile", [(264, 2048, 128), (200, 4096, 256), (136, 2048, 256)])
+def test_units_that_begin_at_other_columns(rows, cols, tile):
+    """Rows a multiple of 4 KB apart: bf16 results of sums that begin at a column of the unit's own, within bf16's rounding of float64."""
+    counts = [5, 70, 0, 129, 260, 33, 1, 100, 64, 7]
+    _, got, want = listed(counts, rows, cols, "plain", 0, tile, tile == 256)
+    assert np.linalg.norm(got - want) <= 2.0 ** -8 * np.linalg.norm(want) and np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max()
+    if tile == 128:
+        _, got, want = listed(counts, rows, cols, "plain", 1, tile, False)
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
+def test_what_tiles_of_256_tokens_do_not_cover_is_refused():
+    L, b = pl.init(), pl.DevBuf(1 << 16)
+    p = lambda **kw: C.byref(group_args(**dict(dict(W=b.ptr, rows=128, cols=256, ldw=256, n_group=1, x=b.ptr, ldx=256, T=8, y=b.ptr, ldy=128, alpha=1.0, off=b.ptr, tiles=b.ptr, n_tiles=b.ptr, max_tiles=1), **kw)))  # noqa: E731
+    for bad in (dict(off=None), dict(rows=64), dict(cols=192), dict(cols=250), dict(max_tiles=0)):
+        assert L.pi_k_group_gemm_tall(p(**bad), None) != 0, bad
+    assert L.pi_k_group_gemm_tile(p(), 256, None) != 0
