@@ -491,7 +491,7 @@ __device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int 
 // the same product in the large tiles of gemm_wide.  256 rows by 128 tokens, or 128 by 256: an expert of more than 128 tokens then has its weights
 // read once, and by one workgroup.  64 experts, both products, us, tiles of 128 / 256 tokens: 192 tokens an expert on average 407 -> 390 (1408 x 4096), 624 -> 585
 // (with a gate); 8 experts of 140, 4096 x 4096 with a gate 245 -> 176; of 96 tokens 290 and 334.
-template <int M, int N> struct GroupProduct {
+template <int M, int N, bool LIST> struct GroupProduct {
     static constexpr bool kPairs = false;
     static constexpr int kM = M, kN = N;
     const pi_group_gemm & g;
@@ -501,7 +501,7 @@ template <int M, int N> struct GroupProduct {
         WidePlace p;
         int ty;
         deal.unit(c, ty, p.row0, p.rows);
-        if (g.off) {
+        if (LIST) {
             const int2 t = reinterpret_cast<const int2 *>(g.tiles)[ty];
             p.grp = t.x; p.lo = t.y; p.n = g.off[p.grp + 1] - p.lo;
         } else {
@@ -510,11 +510,15 @@ template <int M, int N> struct GroupProduct {
         p.n = min(p.n, N);
         return p;
     }
-    __device__ __forceinline__ bool read_once(const WidePlace & p) const { return g.off && g.off[p.grp + 1] - g.off[p.grp] <= N; }
-    // Rows a multiple of 4 KB apart lie in few of the memory's channels, and workgroups that began together would all read the same of them: they begin at
-    // different columns there (64 experts of 96 tokens, 1408 x 4096: 155 -> 138 us; 8 of 140, 8192 x 4096: 243 -> 190; 1408 or 5120 columns: no
-    // difference).  Results in fp32 keep the order of their sums.
-    __device__ __forceinline__ int first(const WidePlace & p) const { return g.y_f32 || g.ldw % 2048 ? 0 : (p.grp * 13 + p.row0 / M) % nk; }
+    __device__ __forceinline__ bool read_once(const WidePlace & p) const { return LIST && g.off[p.grp + 1] - g.off[p.grp] <= N; }
+    // Rows a multiple of 4 KB apart lie in few of the memory's channels, and workgroups that began together would all read the same of them: an expert's
+    // units begin at different columns there (64 experts of 96 tokens, 1408 x 4096: 155 -> 138 us; 8 of 140, 8192 x 4096: 243 -> 190; 1408 or 5120
+    // columns: no difference).  Without a list the workgroups of an XCD share what they read and begin together, those of another elsewhere (2043
+    // tokens, 22016 x 5120: 400 -> 380, x 4096 313 -> 311; every row tile at a column of its own: 325).  Results in fp32, and short rows, keep the order of their sums.
+    __device__ __forceinline__ int first(const WidePlace & p) const {
+        if (g.y_f32 || g.cols < 2048) return 0;
+        return !LIST ? (int)(blockIdx.x % 8) * nk / 8 : g.ldw % 2048 ? 0 : (p.grp * 13 + p.row0 / M) % nk;
+    }
     __device__ __forceinline__ const unsigned char * base_a(const WidePlace & p, int) const { return (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs); }
     __device__ __forceinline__ const unsigned char * base_b(const WidePlace & p) const { return (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs)); }
     __device__ __forceinline__ uint32_t off_a(const WidePlace & p, int r) const { return (uint32_t)(p.row0 + r) * (uint32_t)(g.ldw * 2); }
@@ -526,20 +530,21 @@ template <int M, int N> struct GroupProduct {
         else group_store(g, p.grp, p.lo, p.n, p.row0 + rb, tb, lane >> 4, lane & 15, acc);
     }
 };
-// n_tiles: token tiles of a product without a list
-template <int M, int N>
+// n_tiles: token tiles of a product without a list.  LIST: g.off; the two are kernels of their own because a choice of the hint at run time costs the copying
+// waves what matters to units that share their weights (22016 x 4096 by 400 tokens: 83 -> 88 us).
+template <int M, int N, bool LIST>
 __global__ __launch_bounds__(512, 1) void group_wide_kernel(pi_group_gemm g, int n_tiles) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const GroupProduct<M, N> prod{g, g.cols / kGtBK, (g.T + N - 1) / N, !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0};
-    gemm_wide<bf16>(prod, WideDeal(g.rows, g.off ? *g.n_tiles : n_tiles, g.n_group > 1 ? 1 : kGwBand, M), smem);       // (bands of experts' tiles measured no better)
+    const GroupProduct<M, N, LIST> prod{g, g.cols / kGtBK, (g.T + N - 1) / N, !g.y_f32 && g.rows % (g.glu ? 16 : 8) == 0 && g.ldy % 8 == 0 && g.y_gs % 8 == 0};
+    gemm_wide<bf16>(prod, WideDeal(g.rows, LIST ? *g.n_tiles : n_tiles, g.n_group > 1 ? 1 : kGwBand, M), smem);       // (bands of experts' tiles measured no better)
 }
 
-template <int M, int N> int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&group_wide_kernel<M, N>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
+template <int M, int N, bool LIST> int launch_group_wide(const pi_group_gemm & g, hipStream_t st) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&group_wide_kernel<M, N, LIST>), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
     if (raised != hipSuccess) return pi::hip_fail(raised, "group_wide: LDS size");
-    const long long tiles = g.off ? g.max_tiles : (long long)g.n_group * ((g.T + N - 1) / N), units = tiles * ((g.rows + M - 1) / M);
+    const long long tiles = LIST ? g.max_tiles : (long long)g.n_group * ((g.T + N - 1) / N), units = tiles * ((g.rows + M - 1) / M);
     if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: too many tiles");
-    hipLaunchKernelGGL((group_wide_kernel<M, N>), dim3(wide_blocks(units)), dim3(512), kGwLds, st, g, (int)tiles);
+    hipLaunchKernelGGL((group_wide_kernel<M, N, LIST>), dim3(wide_blocks(units)), dim3(512), kGwLds, st, g, (int)tiles);
     return pi::check_launch("pi_k_group_gemm_tile");
 }
 
@@ -745,7 +750,8 @@ int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream
     hipStream_t st = (hipStream_t)stream;
     // 256-row tiles from the second half on, and at least four stages for a unit's ends to hide behind: measured as fast or faster at every number of
     // tokens and groups from there on (32 heads' 256 x 512 products of 128 tokens: 11.4 us both; 4096 x 512 by 2048 tokens 20.6 -> 16.1)
-    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31)) return launch_group_wide<kGwM, kGwN>(*g, st);
+    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31)) 
+        return g->off ? launch_group_wide<kGwM, kGwN, true>(*g, st) : launch_group_wide<kGwM, kGwN, false>(*g, st);
     if (tile_n == 128) return launch_group_tile<128, 128, 2, 2>(*g, st);
     if (tile_n == 64) return g->rows <= 64 ? launch_group_tile<64, 64, 2, 2>(*g, st) : launch_group_tile<128, 64, 2, 2>(*g, st);
     return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: tile_n must be 64 or 128");
@@ -756,7 +762,7 @@ int pi_k_group_gemm_tall(const pi_group_gemm * g, pi_stream_t stream) {
     if (rc != PI_OK) return rc;
     if (!g->off || g->rows <= 64 || g->cols < 4 * kGtBK || (long long)g->rows * g->ldw >= (1LL << 31))
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_group_gemm_tall: lists of more than 64 rows, at least 256 columns and less than 2^31 values a group");
-    return launch_group_wide<128, 256>(*g, (hipStream_t)stream);
+    return launch_group_wide<128, 256, true>(*g, (hipStream_t)stream);
 }
 
 int pi_k_moe_combine(int type, const float * x, const float * mix, const void * y, const int32_t * inv, const float * weights, int n_top, int T, int cols,
