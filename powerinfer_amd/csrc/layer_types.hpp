@@ -10,6 +10,9 @@ __device__ __forceinline__ float bf16_to_f32(uint16_t b) { return __uint_as_floa
 template <typename ST> __device__ __forceinline__ ST to_st(float v) { return (ST)v; }           // bf16: round to nearest even
 template <typename ST> __device__ __forceinline__ float from_st(ST v) { return (float)v; }
 
+// e^x of a soft-max weight that is rounded to bf16: off by about |x| 2^-24 beside 2^-9
+__device__ __forceinline__ float exp_weight(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504f); }
+
 // eight consecutive columns of one row of a 16 x 32 operand tile (lane l: row l % 16, columns 8 * (l / 16) ..)
 template <typename ST> struct Frag;
 template <> struct Frag<bf16> { pi_u32x4 v; };

@@ -231,6 +231,15 @@ def test_scores_of_any_size(t):
         assert np.isfinite(got).all() and np.abs(got - want).max() <= tol(t, 3) * np.abs(want).max()
 
 
+@pytest.mark.parametrize("sink", [0.0, -np.inf])
+@pytest.mark.parametrize("scale", [30.0, -2.0, 0.0, 1e-38])
+def test_long_runs_with_scales_of_any_size(scale, sink):
+    """What weights are relative to is raised from tile to tile (scores in the hundreds), once (tiny scores), or stays where the first tile put it."""
+    for parts in (1, 3):
+        got, want = attend(pl.BF16, np.random.default_rng(4), [(140, 0), (20, 300)], 2, 1, 64, 64, parts, 1, scale, sink)
+        assert np.isfinite(got).all() and np.abs(got - want).max() <= tol(pl.BF16, 3) * np.abs(want).max()
+
+
 @pytest.mark.parametrize("t", TYPES)
 def test_shifted_keys(t):
     """Rotating a stored key by a distance gives the key of the other position (the division by its size commutes with it)."""

@@ -363,6 +363,23 @@ def test_expanded_attention_with_sinks_of_any_size(sink):
     assert np.abs(got - want).max() < 2e-2 * max(np.abs(want).max(), 1e-3)
 
 
+@pytest.mark.parametrize("scale", [20.0, -1.5, 0.0, 1e-38])
+def test_expanded_attention_with_scales_of_any_size(scale):
+    """What weights are relative to is raised from tile to tile (scores in the hundreds), once (tiny scores), or stays where the first tile put it.  Against
+    the expanded keys and values as they are stored, whose rounding such a scale would multiply."""
+    c = Case(pl.BF16, 3, 32, 16, 32, 64, [230], [list(range(60, 230))], 3)
+    c.scale = scale
+    got, cells = expanded(c, 170), c.cells[c.lists[0, :230]]
+    keys, vals = (as_stored(np.einsum("nr,hdr->nhd", cells[:, :64], w), pl.BF16).astype(np.float64) for w in (c.uk, c.uv))
+    want = np.empty(got.shape)
+    for i in range(170):
+        n = int(c.pos[i]) + 1
+        for h in range(3):
+            s = (keys[:n, h] @ c.q[i, h, :32].astype(np.float64) + cells[:n, c.rank_ld:c.rank_ld + 16].astype(np.float64) @ c.q[i, h, 32:]) * scale
+            want[i, h] = o.sink_softmax(s[None], c.sink[h:h + 1])[0] @ vals[:n, h]
+    assert np.isfinite(got).all() and np.abs(got - want).max() < 2e-2 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("own", [True, False])
 def test_latent_prep(t, own):
