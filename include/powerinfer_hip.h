@@ -233,6 +233,13 @@ PI_API int pi_k_sparse_ffn_partials(const void * fc2_f16, int ff, int r, const f
                                     pi_workspace * ws, pi_stream_t stream);
 PI_API int pi_k_sparse_ffn_reduce(int ff, int cols, int epilogue, const float * add1, const float * add2, float * out,
                                   int32_t * n_active, pi_workspace * ws, pi_stream_t stream);
+/* The whole block of one token in a small F16 layer, the predictor's first product included: x is the predictor's input as it is and, behind `norm`, the FFN's.
+ * A launch and the reduction above; out, epilogue and n_active as for pi_k_sparse_ffn.  Shapes: cols 512 or 1024, r 64, 128 or 256, r * cols <= 131072,
+ * ff % 32 == 0 up to 32768; matrices, x and the norm's weights 16-byte aligned. */
+PI_API int pi_k_sparse_ffn_small_supported(int ff, int r, int cols);
+PI_API int pi_k_sparse_ffn_small(const void * fc1_f16, const void * fc2_f16, int ff, int r, float threshold, const void * up_f16, const void * gate_f16,
+                                 const void * down_t_f16, int cols, const float * x, const pi_norm * norm, int epilogue, const float * add1,
+                                 const float * add2, float * out, int32_t * n_active, pi_workspace * ws, pi_stream_t stream);
 /* the same two launches for a hot/cold split layer (F16): only the GPU-resident neurons are computed, from the compact matrices of
  * the bucket (hot_words / hot_prefix as for pi_k_pred_upgate_q4); logits and xn_f16_out (the fp16-rounded normalised input, cols
  * values, optional) may be pinned host memory for the host share; _reduce_hot counts the resident active neurons, and its add1 /

@@ -212,6 +212,16 @@ int layer_forward(pi_model * m, int il, bool last_token) {
         fn = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
     }
 
+    // small layers: the launches are the time, not what they read (see ffn_small_f16_kernel; a caller's own device matrices may lie anywhere)
+    const bool f16 = up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && fc1.type == PI_TYPE_F16 && fc2.type == PI_TYPE_F16;
+    const bool aligned = (((uintptr_t)fc1.dev | (uintptr_t)fc2.dev | (uintptr_t)up.dev | (uintptr_t)gate.dev | (uintptr_t)down.dev | (uintptr_t)fn.w | (uintptr_t)fn.b) & 15) == 0;
+    if (f16 && aligned && !layer_hybrid && !m->capture && pi_k_sparse_ffn_small_supported(ff, r, d)) {
+        PI_TRY(pi_k_sparse_ffn_small(fc1.dev, fc2.dev, ff, r, hp.sparse_threshold, up.dev, falcon ? nullptr : gate.dev, down.dev, d, ffn_in, &fn,
+                                     falcon ? PI_EPI_ADD2 : PI_EPI_ADD, falcon ? m->attn_out : m->ffn_inp, falcon ? x : nullptr, m->x2, n_act, m->ws, st));
+        std::swap(m->x, m->x2);
+        return PI_OK;
+    }
+
     // predictor
     if (!branch) PI_TRY(pi_k_gemv(fc1.type, fc1.dev, r, d, pred_in, nullptr, PI_EPI_RELU, nullptr, nullptr, m->hidden, st));
     if (branch) {
