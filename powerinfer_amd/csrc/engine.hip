@@ -29,62 +29,80 @@ size_t row_bytes(int type, int64_t ne0) {
     }
 }
 
-// greedy choice of the finished step + bookkeeping for the next one: the chosen token becomes the next
-// input, the position advances, the token and the step's total active-row count are logged
-__global__ __launch_bounds__(1024) void argmax_advance_kernel(const float * __restrict__ logits, int n, int32_t * token, int32_t * pos,
-                                                              int32_t * step, int32_t * out_tokens, int32_t * out_active,
-                                                              const int32_t * __restrict__ n_active, int n_layer, int max_steps) {
-    __shared__ float bv[16];
-    __shared__ int   bi[16];
-    __shared__ int stot;
-    float best = -INFINITY; int idx = n;
-    // the bookkeeping operands are requested with the logits: one memory round trip for the whole kernel at vocabularies up to 32 K
-    int act = 0;
-    for (int l = threadIdx.x; l < n_layer; l += blockDim.x) act += n_active[l];
-    const int s_in = *step, p_in = *pos;
-    for (int base = 0; base < n; base += 8 * 4 * 1024) {
-        float4 v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = base + (u * 1024 + (int)threadIdx.x) * 4;
-            if (i + 3 < n) v[u] = *reinterpret_cast<const float4 *>(logits + i);
-            else v[u] = make_float4(i < n ? logits[i] : -INFINITY, i + 1 < n ? logits[i + 1] : -INFINITY, i + 2 < n ? logits[i + 2] : -INFINITY, -INFINITY);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = base + (u * 1024 + (int)threadIdx.x) * 4;
-            if (v[u].x > best) { best = v[u].x; idx = i; }
-            if (v[u].y > best) { best = v[u].y; idx = i + 1; }
-            if (v[u].z > best) { best = v[u].z; idx = i + 2; }
-            if (v[u].w > best) { best = v[u].w; idx = i + 3; }
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(idx, o, 64);
-        if (ov > best || (ov == best && oi < idx)) { best = ov; idx = oi; }
-    }
+// Greedy choice of the finished step, bookkeeping for the next one and the call's results: the chosen token becomes the next input, the position
+// advances, the token and the step's total active-row count are logged; where a call waits for them (pin), the token, the host threads' status and
+// (want_logits) the logits are stored in pinned memory: words 0 and 1, and from word kPickLogits on.  Bound by latency and by what one unit can
+// read: 32000 logits were 6.6 us for a single workgroup, and another 5.6 and a launch apart went to their copy; now 32 workgroups read them once for
+// both and the last one to arrive ends the step (6.9 us).  Ties go to the lowest index, as before.
+constexpr int kPickBlock = 256, kPickMost = 64, kPickLogits = 16;
+struct Pick {
+    const float * logits; int n; int32_t * token, * pos, * step, * out_tokens, * out_active; const int32_t * n_active; int n_layer, max_steps;
+    unsigned long long * best; unsigned int * arrived;              // [kPickMost] the workgroups' choices; 0 between two launches
+    uint32_t * pin; const uint32_t * status; int want_logits;
+};
+__global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
+    __shared__ float bv[kPickBlock / 64];
+    __shared__ int   bi[kPickBlock / 64];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (wave == 0) {                       // n_layer <= 1024 entries were spread over the threads; at most a few waves hold non-zeros
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) act += __shfl_xor(act, o, 64);
+    float best = -INFINITY; int idx = p.n;
+    // the bookkeeping operands are requested with the logits (by every workgroup: only the last one writes them)
+    int act = 0, s_in = 0, p_in = 0;
+    uint32_t status = 0;
+    if (wave == 0) {
+        for (int l = lane; l < p.n_layer; l += 64) act += p.n_active[l];
+        s_in = *p.step; p_in = *p.pos;
+        if (p.status) status = *p.status;
     }
-    if (threadIdx.x == 0) stot = 0;
+    float * out = p.pin && p.want_logits ? reinterpret_cast<float *>(p.pin + kPickLogits) : nullptr;
+    for (int i = ((int)blockIdx.x * kPickBlock + (int)threadIdx.x) * 4; i < p.n; i += (int)gridDim.x * kPickBlock * 4) {
+        if (i + 3 < p.n) {
+            const float4 v = *reinterpret_cast<const float4 *>(p.logits + i);
+            if (out) *reinterpret_cast<float4 *>(out + i) = v;
+            if (v.x > best) { best = v.x; idx = i; }
+            if (v.y > best) { best = v.y; idx = i + 1; }
+            if (v.z > best) { best = v.z; idx = i + 2; }
+            if (v.w > best) { best = v.w; idx = i + 3; }
+        } else {
+            for (int k = i; k < p.n; ++k) {
+                const float v = p.logits[k];
+                if (out) out[k] = v;
+                if (v > best) { best = v; idx = k; }
+            }
+        }
+    }
+    const auto merge = [&](float ov, int oi) { if (ov > best || (ov == best && oi < idx)) { best = ov; idx = oi; } };
+    const auto merge_wave = [&]() {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) { const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(idx, o, 64); merge(ov, oi); }
+    };
+    merge_wave();
     if (lane == 0) { bv[wave] = best; bi[wave] = idx; }
     __syncthreads();
-    if (wave != 0 && act != 0) atomicAdd(&stot, act);      // layers beyond the first 64 (LDS atomic, integer: order does not matter)
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < (int)(blockDim.x >> 6); ++w)
-            if (bv[w] > best || (bv[w] == best && bi[w] < idx)) { best = bv[w]; idx = bi[w]; }
-        if (idx >= n) idx = 0;
-        const int tot = act + stot;
-        const int s = s_in;
-        if (s < max_steps) { out_tokens[s] = idx; out_active[s] = tot; }
-        *token = idx;
-        *pos = p_in + 1;
-        *step = s + 1;
+    if (wave != 0) return;
+    for (int w = 1; w < kPickBlock / 64; ++w) merge(bv[w], bi[w]);
+    if (gridDim.x > 1) {
+        unsigned int before = 0;
+        if (lane == 0) {
+            __hip_atomic_store(p.best + blockIdx.x, (unsigned long long)__float_as_uint(best) << 32 | (unsigned int)idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            before = __hip_atomic_fetch_add(p.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (__builtin_amdgcn_readfirstlane(before) + 1 < gridDim.x) return;
+        if (lane < (int)gridDim.x) {                                // the last to arrive: every choice is there
+            const unsigned long long v = __hip_atomic_load(p.best + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            best = __uint_as_float((unsigned int)(v >> 32)); idx = (int)(unsigned int)v;
+        }
+        merge_wave();
+        if (lane == 0) __hip_atomic_store(p.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) act += __shfl_xor(act, o, 64);
+    if (lane != 0) return;
+    if (idx >= p.n) idx = 0;
+    if (s_in < p.max_steps) { p.out_tokens[s_in] = idx; p.out_active[s_in] = act; }
+    *p.token = idx;
+    *p.pos = p_in + 1;
+    *p.step = s_in + 1;
+    if (p.pin) { p.pin[0] = (uint32_t)idx; p.pin[1] = status; }
 }
 
 // dst row i = src row perm[i]; rows of row_bytes (a multiple of 16) bytes, one workgroup per row
@@ -356,10 +374,13 @@ int token_forward(pi_model * m, bool want_logits, bool last_token, int32_t token
     return PI_OK;
 }
 
-int launch_advance(pi_model * m) {
-    hipLaunchKernelGGL(argmax_advance_kernel, dim3(1), dim3(1024), 0, m->stream, m->logits, m->hp.n_vocab, m->d_token, m->d_pos, m->d_step,
-                       m->d_out_tokens, m->d_out_active, m->n_active, m->hp.n_layer, m->max_steps);
-    return pi::check_launch("argmax_advance");
+// pin (optional): pinned memory for the call's results
+int launch_pick(pi_model * m, uint32_t * pin, const uint32_t * status, bool want_logits) {
+    const int n = m->hp.n_vocab, blocks = std::min((n + kPickBlock * 4 - 1) / (kPickBlock * 4), kPickMost);
+    const Pick p{m->logits, n, m->d_token, m->d_pos, m->d_step, m->d_out_tokens, m->d_out_active, m->n_active, m->hp.n_layer, m->max_steps,
+                 m->pick_best, m->pick_arrived, pin, status, want_logits};
+    hipLaunchKernelGGL(pick_token_kernel, dim3(blocks), dim3(kPickBlock), 0, m->stream, p);
+    return pi::check_launch("pick_token");
 }
 
 }  // namespace
@@ -723,12 +744,13 @@ int pi_model_finalize(pi_model * m) {
     m->pred_logits = m->alloc<float>(ff); m->h_c = m->alloc<float>(ff); m->h_dense = m->alloc<float>(ff); m->logits = m->alloc<float>(hp.n_vocab);
     m->cold_out = m->alloc<float>(d);
     m->list = m->alloc<int32_t>(ff); m->n_active = m->alloc<int32_t>(hp.n_layer);
+    m->pick_best = m->alloc<unsigned long long>(kPickMost); m->pick_arrived = m->alloc<unsigned int>(1);
     m->d_token = m->alloc<int32_t>(1); m->d_pos = m->alloc<int32_t>(1); m->d_step = m->alloc<int32_t>(1);
     m->d_out_tokens = m->alloc<int32_t>(m->max_steps); m->d_out_active = m->alloc<int32_t>(m->max_steps);
     m->k_cache = m->alloc<__half>(kv); m->v_cache = m->alloc<__half>(kv);
     m->cap_ffn = m->alloc<float>((size_t)hp.n_layer * d); m->cap_logits = m->alloc<float>((size_t)hp.n_layer * ff); m->cap_src = m->alloc<float>((size_t)hp.n_layer * d);
     if (!m->x || !m->x2 || !m->qkv || !m->q_rot || !m->att || !m->attn_out || !m->ffn_inp || !m->hidden || !m->pred_logits || !m->h_c || !m->h_dense ||
-        !m->logits || !m->cold_out || !m->list || !m->n_active || !m->d_token || !m->d_pos || !m->d_step || !m->d_out_tokens || !m->d_out_active ||
+        !m->logits || !m->cold_out || !m->list || !m->n_active || !m->d_token || !m->d_pos || !m->d_step || !m->d_out_tokens || !m->d_out_active || !m->pick_best || !m->pick_arrived ||
         !m->k_cache || !m->v_cache || !m->cap_ffn || !m->cap_logits || !m->cap_src)
         return PI_E_HIP;
     PI_TRY(pi_memset(m->k_cache, 0, kv * 2));
@@ -762,6 +784,7 @@ int pi_model_finalize(pi_model * m) {
         return pi::fail(PI_E_UNSUPPORTED, "pi_model_finalize: head size or context outside every attention kernel (head size a multiple of 8 that divides 512, at most 64 parts of the context per head)");
     PI_TRY(pi_memset(m->n_active, 0, sizeof(int32_t) * hp.n_layer));
     PI_TRY(pi_memset(m->d_step, 0, 4));
+    PI_TRY(pi_memset(m->pick_arrived, 0, 4));
     PI_TRY(pi_memset(m->h_dense, 0, sizeof(float) * ff));
     if (m->hybrid && !m->rest_on_gpu) {
         m->cold = pi::cold_create(m);
@@ -831,12 +854,21 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
         PI_TRY(token_forward(m, last, last, tokens[i], n_past + i));
     }
     // greedy choice on the device; the state then points at the next position
-    PI_TRY(launch_advance(m));
     int32_t tok = -1;
     uint32_t status = 0;
     const uint32_t * d_status = m->cold ? pi::cold_status(m->cold) : nullptr;
-    const pi::HostCopy results[] = {{m->d_token, &tok, 4}, {d_status, d_status ? &status : nullptr, 4}, {m->logits, logits_out, sizeof(float) * m->hp.n_vocab}};
-    PI_TRY(m->stage.fetch(results, 3, m->stream));
+    const size_t logits = sizeof(float) * (size_t)m->hp.n_vocab, head = sizeof(uint32_t) * kPickLogits;
+    uint32_t * pin = (uint32_t *)m->stage.room(head + (logits_out ? logits : 0));
+    PI_TRY(launch_pick(m, pin, d_status, logits_out != nullptr));
+    if (pin) {
+        PI_TRY(m->stage.wait(m->stream));
+        tok = (int32_t)pin[0];
+        status = pin[1];
+        if (logits_out) memcpy(logits_out, pin + kPickLogits, logits);
+    } else {
+        const pi::HostCopy results[] = {{m->d_token, &tok, 4}, {d_status, d_status ? &status : nullptr, 4}, {m->logits, logits_out, logits}};
+        PI_TRY(m->stage.fetch(results, 3, m->stream));
+    }
     if (m->cold) PI_TRY(pi::cold_drain(m->cold, &status));
     return tok;
 }
@@ -865,7 +897,7 @@ int pi_model_generate(pi_model * m, int n_steps, int32_t * out_tokens, float * m
         m->building_graph = true;
         int rc = token_forward(m, true, false);
         m->building_graph = false;
-        if (rc == PI_OK) rc = launch_advance(m);
+        if (rc == PI_OK) rc = launch_pick(m, nullptr, nullptr, false);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(m->stream, &g);
         if (rc != PI_OK) { if (g) (void)hipGraphDestroy(g); return rc; }
@@ -880,7 +912,7 @@ int pi_model_generate(pi_model * m, int n_steps, int32_t * out_tokens, float * m
             PI_HIP_TRY(hipGraphLaunch(m->graph_exec, m->stream));
         } else {
             PI_TRY(token_forward(m, true, false));
-            PI_TRY(launch_advance(m));
+            PI_TRY(launch_pick(m, nullptr, nullptr, false));
         }
     }
     PI_HIP_TRY(hipEventRecord(m->ev1, m->stream));

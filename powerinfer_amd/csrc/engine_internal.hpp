@@ -59,6 +59,7 @@ struct pi_model {
     float *hidden = nullptr, *pred_logits = nullptr, *h_c = nullptr, *h_dense = nullptr, *logits = nullptr, *cold_out = nullptr;
     int32_t *list = nullptr, *n_active = nullptr, *d_token = nullptr, *d_pos = nullptr, *d_step = nullptr;
     int32_t *d_out_tokens = nullptr, *d_out_active = nullptr;
+    unsigned long long * pick_best = nullptr; unsigned int * pick_arrived = nullptr;      // of the greedy choice's workgroups
     __half *k_cache = nullptr, *v_cache = nullptr;
     float *rope_table = nullptr;          // float2 [n_ctx][hd/2] (cos, sin), when the fused or the split attention kernel is used
     int    attn_parts = 1;                // > 1: the cells of every head are split over this many workgroups (long contexts)

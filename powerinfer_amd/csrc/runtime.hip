@@ -96,6 +96,12 @@ void HostStage::release() {
     while (n) (void)hipHostFree(out[--n]);
 }
 
+int HostStage::wait(hipStream_t st) {
+    PI_HIP_TRY(hipStreamSynchronize(st));
+    busy = false;
+    return PI_OK;
+}
+
 int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
     HostCopy c[kMaxCopies];
     int m = 0;

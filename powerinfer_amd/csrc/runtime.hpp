@@ -39,6 +39,9 @@ struct HostStage {
     // queues the copies behind what the stream holds and returns when the stream is done and the results are in place; all but the
     // last copy together fit in 4 KB of the first piece (else ordinary copies)
     int fetch(const HostCopy * copies, int n, hipStream_t st);
+    // room for results that the call's own last launch stores (null: to be had with fetch only), and the wait for them
+    unsigned char * room(size_t bytes) { if (!pin || bytes > piece) return nullptr; busy = true; return pin; }
+    int wait(hipStream_t st);
 };
 
 // pi_k_attn_fused with such extra workgroups
