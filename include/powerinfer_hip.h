@@ -851,6 +851,11 @@ typedef struct pi_sum_norm {
     const float * w_next; const int32_t * rows; int32_t T, cols, groups; float eps; float * keep; void * h; int32_t ld, ol;
 } pi_sum_norm;
 PI_API int pi_k_sum_norm(int type, const pi_sum_norm * p, pi_stream_t stream);
+/* The same of up to 16 tokens (BF16, mix, h in the operand layout), and the choice that pi_k_route_scores makes of router [n_expert][ld_router] (BF16) times
+ * h.  sums: T * groups * n_expert floats of scratch; arrived: 16 counters, zero before the first call and left so. */
+PI_API int pi_k_sum_norm_route_supported(int T, int cols, int groups, int n_expert);
+PI_API int pi_k_sum_norm_route(const pi_sum_norm * p, const void * router, int ld_router, int n_expert, int n_top, int32_t * ids, float * weights, float * sums,
+                               uint32_t * arrived, pi_stream_t stream);
 /* A norm in groups and behind it a causal convolution over time on every channel: u = norm(x[t]) * w, h[t] = u_t + sum over j of taps_w[j][c] *
  * u_(t - taps + 1 + j) along the token's sequence, zeros ahead of it.  items [n_items] of eight integers: {first token, tokens, tokens of the run ahead of
  * them, tokens of the run, slot, 1 if nothing lies before the run, 0, 0}; a run's first item holds at least min(taps - 1, all) of its tokens, reads the last

@@ -158,6 +158,7 @@ struct LayerState {
     // step buffers for `cap` tokens (one allocation)
     int cap = 0;
     unsigned char * arena = nullptr;
+    float * route_sums = nullptr; uint32_t * route_arrived = nullptr;      // of norms and expert choices in one launch
     float *x = nullptr, *x2 = nullptr, *x0 = nullptr, *z = nullptr, *mix = nullptr, *rl = nullptr, *wts = nullptr, *lin_o = nullptr, *lin_den = nullptr, *lin_gates = nullptr;
     void *lin_q = nullptr, *lin_k = nullptr, *lin_v = nullptr, *lin_states = nullptr;
     void *h_a = nullptr, *h_b = nullptr, *q_un = nullptr, *q_lat = nullptr, *o_lat = nullptr, *att = nullptr, *act = nullptr, *y_exp = nullptr;
@@ -1112,7 +1113,7 @@ int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in
 }
 
 // A layer with norms before and after its sublayers.  Steps of up to 16 tokens (bf16) stream the weights past operands in the matrix cores' layout; the
-// sum that closes a sublayer and the norm ahead of the feed-forward are one launch, the norm ahead of the mixer and its convolution another.
+// sum that closes a sublayer, the norm ahead of the feed-forward and the expert choice behind it are one launch, the norm ahead of the mixer and its convolution another.
 int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in, float * keep) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
@@ -1168,10 +1169,14 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
     n.x = s->x; n.mix = s->mix; n.w = L.norm_a_after; n.mult = s->opts.residual_mult; n.T = T; n.cols = D; n.groups = s->opts.norm_groups; n.eps = m->hp.norm_eps;
     n.ld = s->d_ld; n.ol = step;
     if (moe) { n.h = s->h_b; n.w_next = L.norm_b; } else n.keep = keep;
-    PI_TRY(pi_k_sum_norm(type, &n, st));
-    if (!moe) return PI_OK;
-    PI_TRY(product(L.router, d.n_expert, s->h_b, s->rl));
-    PI_TRY(pi_k_route_scores(s->rl, T, d.n_expert, d.n_top, s->ids, s->wts, st));
+    if (moe && step && bf16_mode(s) && pi_k_sum_norm_route_supported(T, D, n.groups, d.n_expert)) {
+        PI_TRY(pi_k_sum_norm_route(&n, L.router, s->d_ld, d.n_expert, d.n_top, s->ids, s->wts, s->route_sums, s->route_arrived, st));
+    } else {
+        PI_TRY(pi_k_sum_norm(type, &n, st));
+        if (!moe) return PI_OK;
+        PI_TRY(product(L.router, d.n_expert, s->h_b, s->rl));
+        PI_TRY(pi_k_route_scores(s->rl, T, d.n_expert, d.n_top, s->ids, s->wts, st));
+    }
     n.w = L.norm_b_after; n.w_next = nullptr; n.h = nullptr; n.keep = keep;
     if (step) {
         PI_TRY(pi_k_expert_up_step(L.up, d.n_expert, d.expert_ff, s->d_ld, d.expert_limit, d.glu_gain, d.glu_plain_up, d.weigh_input, s->h_b, T, s->ids, s->wts, d.n_top, s->act, L.ff_ld, st));
@@ -1649,6 +1654,16 @@ int layers_finalize(pi_model * m) {
     s->g_work = m->alloc<int32_t>(4 * items);
     s->g_out = m->alloc<int32_t>((size_t)s->max_steps * kMaxLockstep);
     if (!s->g_work || !s->g_out) return PI_E_HIP;
+    if (s->family == kBothNorms) {
+        size_t n = 0;
+        for (const Layer & L : s->layers) if (L.moe() && bf16_mode(s) && pi_k_sum_norm_route_supported(1, m->hp.n_embd, s->opts.norm_groups, L.d.n_expert)) n = std::max(n, (size_t)L.d.n_expert);
+        if (n) {
+            s->route_sums = m->alloc<float>(16 * (size_t)s->opts.norm_groups * n);
+            s->route_arrived = m->alloc<uint32_t>(16);
+            if (!s->route_sums || !s->route_arrived) return PI_E_HIP;
+            PI_TRY(pi_memset(s->route_arrived, 0, 16 * 4));
+        }
+    }
     m->stage.init(sizeof(float) * 16 * (size_t)m->hp.n_vocab);
     PI_HIP_TRY(hipDeviceSynchronize());
     m->finalized = true;

@@ -2,6 +2,7 @@
 // one, and the norm with a causal convolution over time behind it.
 #include "layer_types.hpp"
 #include "mixers.hpp"
+#include "route.hpp"
 
 namespace {
 
@@ -180,6 +181,100 @@ template <typename ST> bool launch_sum_quads(const pi_sum_norm & p, hipStream_t 
     return true;
 }
 
+// The same for steps of up to 16 tokens, with the expert choice that reads the normed row: every group's workgroup multiplies its 512 M columns with the
+// router's, and the last of a token's to arrive adds the groups' sums in order and chooses.  Bound by latency: the router's rows (64 KB a
+// workgroup, 2 us for one unit) travel while the norms are formed, where a product of four workgroups with 128 KB each and the choice were
+// launches of their own.  4096 columns in 8 groups, 64 experts, one token: 4.0 + 5.6 + 3.9 -> 7.4 us.  Norms as above; the products in fp32 of the
+// row in bf16, as before.
+constexpr int kSrWaves = 8, kSrRows = 8, kSrExperts = 256, kSrGroups = 32;
+struct SumRoute { const bf16 * router; int ld, E, top; int32_t * ids; float * weights, * sums; unsigned int * arrived; };
+template <int M>
+__global__ __launch_bounds__(64 * kSrWaves) void sum_norm_route_kernel(pi_sum_norm p, SumRoute r) {
+    constexpr int SIZE = 512 * M, NW = SIZE / 256;                  // waves that form the norms
+    __shared__ float part[2][NW];
+    __shared__ __align__(16) bf16 hs[SIZE];
+    __shared__ __align__(16) float z[kSrExperts], sm[3 * kSrExperts];
+    __shared__ bool last;
+    const int t = blockIdx.x, g = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c0 = g * SIZE, col = c0 + wave * 256 + lane * 4;
+    const bool mine = wave < NW;
+    const size_t base = (size_t)t * p.cols;
+    float4 x{}, b{}, w{}, next{};
+    if (mine) {
+        b = *reinterpret_cast<const float4 *>(p.mix + base + col); x = *reinterpret_cast<const float4 *>(p.x + base + col);
+        w = *reinterpret_cast<const float4 *>(p.w + col); next = *reinterpret_cast<const float4 *>(p.w_next + col);
+    }
+    pi_u32x4 ld[kSrRows][M];
+    const auto rows = [&](int e0) {                                 // experts e0 + wave, e0 + wave + kSrWaves, ..
+#pragma unroll
+        for (int k = 0; k < kSrRows; ++k)
+#pragma unroll
+            for (int m = 0; m < M; ++m) ld[k][m] = pi_ld16(r.router + (size_t)min(e0 + wave + k * kSrWaves, r.E - 1) * r.ld + c0 + m * 512 + lane * 8);
+    };
+    rows(0);
+    const auto scaled = [&](const float4 & v, float * sums) -> float {
+        const float sum = pi_wave_sum(fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))));
+        if (mine && lane == 0) sums[wave] = sum;
+        __syncthreads();
+        float s = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) s += sums[k];
+        return pi_inv_sqrt(s / (float)SIZE + p.eps);
+    };
+    const float f = p.mult * scaled(b, part[0]);
+    x = make_float4(fmaf(f * b.x, w.x, x.x), fmaf(f * b.y, w.y, x.y), fmaf(f * b.z, w.z, x.z), fmaf(f * b.w, w.w, x.w));
+    const float f2 = scaled(x, part[1]);
+    if (mine) {
+        *reinterpret_cast<float4 *>(p.x + base + col) = x;
+        if (p.keep) *reinterpret_cast<float4 *>(p.keep + base + col) = x;
+        const float v[4] = {f2 * x.x * next.x, f2 * x.y * next.y, f2 * x.z * next.z, f2 * x.w * next.w};
+        store4((bf16 *)p.h + pi_ol_index(t, col), v, true, 4);
+        store4(hs + col - c0, v, true, 4);
+    }
+    __syncthreads();
+    float h[M][8];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const pi_u32x4 q = *reinterpret_cast<const pi_u32x4 *>(hs + m * 512 + lane * 8);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { h[m][2 * e] = __uint_as_float(q[e] << 16); h[m][2 * e + 1] = __uint_as_float(q[e] & 0xFFFF0000u); }
+    }
+    float * sums = r.sums + (size_t)t * p.groups * r.E;
+    for (int e0 = 0; e0 < r.E; e0 += kSrRows * kSrWaves) {
+        if (e0) rows(e0);
+        float s = 0.0f;                                             // lane k: the sum of row k
+#pragma unroll
+        for (int k = 0; k < kSrRows; ++k) {
+            float d = 0.0f;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    d = fmaf(__uint_as_float(ld[k][m][e] << 16), h[m][2 * e], d);
+                    d = fmaf(__uint_as_float(ld[k][m][e] & 0xFFFF0000u), h[m][2 * e + 1], d);
+                }
+            d = pi_wave_sum(d);
+            s = lane == k ? d : s;
+        }
+        const int e = e0 + wave + lane * kSrWaves;
+        if (lane < kSrRows && e < r.E) __hip_atomic_store(sums + g * r.E + e, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (tid == 0) last = __hip_atomic_fetch_add(r.arrived + t, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == (unsigned int)p.groups;
+    __syncthreads();
+    if (!last) return;
+    for (int e = tid; e < r.E; e += 64 * kSrWaves) {
+        float s = 0.0f;
+#pragma unroll 8
+        for (int k = 0; k < p.groups; ++k) s += __hip_atomic_load(sums + k * r.E + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        z[e] = s;
+    }
+    if (tid == 0) __hip_atomic_store(r.arrived + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    RouteArgs a{z, r.E, r.top, 1, 1, nullptr, r.ids + (size_t)t * r.top, r.weights + (size_t)t * r.top};
+    a.raw = true;
+    route_token(a, 0, sm);
+}
+
 // An item of consecutive tokens of one run a workgroup: first the groups' scales of every row the item touches, then column by column the normed
 // inputs of those rows and their convolution.
 __host__ __device__ inline int conv_rows(int tokens, int taps) { return tokens + 2 * taps; }
@@ -344,6 +439,21 @@ int pi_k_sum_norm(int type, const pi_sum_norm * p, pi_stream_t stream) {
     else if (type == PI_TYPE_F32) hipLaunchKernelGGL(sum_norm_kernel<float>, dim3(p->T), dim3(block), lds, (hipStream_t)stream, *p);
     else return pi::fail(PI_E_UNSUPPORTED, "pi_k_sum_norm: type");
     return pi::check_launch("pi_k_sum_norm");
+}
+
+int pi_k_sum_norm_route_supported(int T, int cols, int groups, int n_expert) {
+    return T > 0 && T <= kBtMaxT && groups > 0 && groups <= kSrGroups && n_expert > 0 && n_expert <= kSrExperts && (cols == 512 * groups || cols == 1024 * groups) && n_expert * (cols / groups) <= 65536;
+}
+
+int pi_k_sum_norm_route(const pi_sum_norm * p, const void * router, int ld_router, int n_expert, int n_top, int32_t * ids, float * weights, float * sums, uint32_t * arrived, pi_stream_t stream) {
+    if (!p || !p->x || !p->mix || !p->w || !p->w_next || !p->h || p->rows || p->y || !p->ol || p->ld < p->cols || p->ld % 8 || !router || ld_router < p->cols || ld_router % 8 || n_top <= 0 ||
+        n_top > n_expert || !ids || !weights || !sums || !arrived)
+        return pi::fail(PI_E_ARG, "pi_k_sum_norm_route: bad arguments");
+    if (!pi_k_sum_norm_route_supported(p->T, p->cols, p->groups, n_expert)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_sum_norm_route: groups of 512 or 1024 columns, up to 65536 values of the router a group");
+    const SumRoute r{(const bf16 *)router, ld_router, n_expert, n_top, ids, weights, sums, arrived};
+    if (p->cols == 512 * p->groups) hipLaunchKernelGGL(sum_norm_route_kernel<1>, dim3(p->T, p->groups), dim3(64 * kSrWaves), 0, (hipStream_t)stream, *p, r);
+    else hipLaunchKernelGGL(sum_norm_route_kernel<2>, dim3(p->T, p->groups), dim3(64 * kSrWaves), 0, (hipStream_t)stream, *p, r);
+    return pi::check_launch("pi_k_sum_norm_route");
 }
 
 int pi_k_conv_tokens(int T, int taps) { return T <= 16 ? (taps > 2 ? taps - 1 : 1) : taps > 5 ? taps - 1 : 4; }
