@@ -121,6 +121,7 @@ struct Step {
     std::vector<Work> apart;
     std::vector<const int32_t *> first;                // per kind: the first cell of each token's window (null: counted back from its last)
     int32_t * prev = nullptr; bool carry = false;
+    bool started = false;                              // the embeddings and angles are there
     const int32_t *lin = nullptr, *lin_long = nullptr, *lin_first = nullptr, *lin_chunks = nullptr;
     int n_lin = 0, n_lin_long = 0, n_lin_chunks = 0;
     const int32_t * conv = nullptr; int n_conv = 0;    // items of the convolutions
@@ -1221,15 +1222,16 @@ int pass_layers(pi_model * m, const Step & in) {
     LayerState * s = m->lay;
     const int type = s->opts.compute, T = in.T, D = m->hp.n_embd;
     hipStream_t st = m->stream;
-    if (s->family != kTwoNorms) PI_TRY(pi_k_embed_bigram(s->embed, D, in.tokens, in.prev, T, s->opts.embed_scale, s->bigram, s->opts.bigram_buckets, s->opts.bigram_mul_prev, s->opts.bigram_mul_cur,
-                                              in.carry, s->x, s->opts.loop_times > 0 ? s->x0 : nullptr, st));
+    if (in.started) {}
+    else if (s->family != kTwoNorms) PI_TRY(pi_k_embed_bigram(s->embed, D, in.tokens, in.prev, T, s->opts.embed_scale, s->bigram, s->opts.bigram_buckets, s->opts.bigram_mul_prev, s->opts.bigram_mul_cur,
+                                                   in.carry, s->x, s->opts.loop_times > 0 ? s->x0 : nullptr, st));
     else PI_TRY(pi_k_embed_norm(s->embed, D, in.tokens, T, s->embd_norm, m->hp.norm_eps, s->x, st));
     if (s->family == kPostNorm) {                      // the first product's operand
         pi_res_norm n{};
         n.x = n.out = s->x; n.T = T; n.cols = D; n.h = s->h_a; n.ld = s->d_ld; n.ol = bf16_mode(s) && pi_k_layer_step_supported(T, 0, 0);
         PI_TRY(pi_k_res_norm(type, &n, st));
     }
-    for (size_t k = 0; k < s->rots.size(); ++k) PI_TRY(rope_angles(m, (int)k, in.pos, T));
+    for (size_t k = in.started ? pi::PassStart::kRots : 0; k < s->rots.size(); ++k) PI_TRY(rope_angles(m, (int)k, in.pos, T));
     for (size_t k = 0; k < s->order.size(); ++k) {
         Layer & L = s->layers[s->order[k].layer];
         const bool moe = L.moe();
@@ -1492,6 +1494,32 @@ int copy_inputs(pi_model * m, size_t n) {
     return PI_OK;
 }
 
+// The pass's n integers and the new cells behind them (n_app triples) on their way, then its embeddings and angles.  kLinkTokens: most tokens whose ids and
+// positions are read across the link (a pass of four layers, us, across it and in two launches: 1 token 437 / 443, 64 1550 / 1553, 128 1596 / 1601, 256 1834 / 1829).
+constexpr int kLinkTokens = 128;
+int start_pass(pi_model * m, Step & in, size_t n, size_t at_app, int n_app) {
+    LayerState * s = m->lay;
+    const int T = in.T;
+    pi::PassStart p{};
+    p.src = s->h_in; p.dst = s->d_in; p.words = n; p.append = s->h_in + at_app; p.n_append = n_app; p.lists = s->lists; p.list_ld = (size_t)s->kv.n;
+    s->in_flight = true;
+    if (T > kLinkTokens) {
+        PI_TRY(pi::pass_start(p, m->stream));
+        p = pi::PassStart{};
+    }
+    const int32_t * from = T > kLinkTokens ? s->d_in : s->h_in;
+    const bool two = s->family == kTwoNorms;
+    p.table = s->embed; p.cols = m->hp.n_embd; p.T = T; p.tokens = from; p.pos = from + T; p.prev = from + 5 * (size_t)T; p.norm = two ? s->embd_norm : nullptr; p.eps = m->hp.norm_eps;
+    p.scale = s->opts.embed_scale; p.bigram = two ? nullptr : s->bigram; p.buckets = s->opts.bigram_buckets; p.mul_prev = s->opts.bigram_mul_prev; p.mul_cur = s->opts.bigram_mul_cur;
+    p.x = s->x; p.x0 = !two && s->opts.loop_times > 0 ? s->x0 : nullptr;
+    for (; p.n_rot < (int)std::min(s->rots.size(), (size_t)pi::PassStart::kRots); ++p.n_rot) {
+        const Rotation & r = s->rots[p.n_rot];
+        p.rot[p.n_rot] = {r.dims, r.base, r.length(), r.scaling ? r.freq : nullptr, s->cs[p.n_rot]};
+    }
+    in.started = true;
+    return pi::pass_start(p, m->stream);
+}
+
 int upload_appends(pi_model * m, const std::vector<int32_t> & app) {
     if (app.empty()) return PI_OK;
     LayerState * s = m->lay;
@@ -1715,7 +1743,7 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
     for (int t = 0; t < n_tokens; ++t) take_cell(s, cells[t], positions[t], seq_masks[t], tokens[t], app);
     s->kv.move_head(cells[n_tokens - 1] + 1);
     for (int t = 0; t < n_tokens; ++t) for (uint32_t b = seq_masks[t]; b; b &= b - 1) refresh_list(s, __builtin_ctz(b), app);
-    PI_TRY(upload_appends(m, app));
+    struct Pending { pi_model * m; std::vector<int32_t> & app; ~Pending() { if (!app.empty()) (void)upload_appends(m, app); } } pending{m, app};      // (a call that ends before its first pass)
     std::vector<int32_t> vis(n_tokens), seq(n_tokens), prev(n_tokens, -1);
     for (int t = 0; t < n_tokens; ++t) {
         seq[t] = __builtin_ctz(seq_masks[t]);                    // a token attends the cells of its first sequence
@@ -1724,6 +1752,7 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         if (vis[t] >= 2) prev[t] = s->cell_tok[s->list_cells[seq[t]][vis[t] - 2]];
     }
     std::vector<int32_t> rows, place, items, wide, lin;
+    bool waited = false;
     for (int t0 = 0; t0 < n_tokens; t0 += batch) {
         const int T = std::min(batch, n_tokens - t0);
         rows.clear(); place.clear(); items.clear();
@@ -1831,7 +1860,8 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             items.insert(items.end(), seq_r.begin(), seq_r.end());
         }
         const size_t n_in = (size_t)8 * T + items.size() + rows.size();
-        PI_TRY(ensure_inputs(m, n_in));
+        const int n_app = (int)(app.size() / 3);                   // (the first pass's)
+        PI_TRY(ensure_inputs(m, n_in + app.size()));
         PI_TRY(inputs_free(m));
         int32_t * h = s->h_in;
         memcpy(h, tokens + t0, 4 * (size_t)T); memcpy(h + T, positions + t0, 4 * (size_t)T); memcpy(h + 2 * T, cells.data() + t0, 4 * (size_t)T);
@@ -1839,7 +1869,7 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         memcpy(h + 5 * T, prev.data() + t0, 4 * (size_t)T);      // (the items behind start on a multiple of 16 bytes)
         if (!items.empty()) memcpy(h + 8 * T, items.data(), 4 * items.size());
         if (!rows.empty()) memcpy(h + 8 * T + items.size(), rows.data(), 4 * rows.size());
-        PI_TRY(copy_inputs(m, n_in));
+        if (n_app) memcpy(h + n_in, app.data(), 4 * app.size());
         in.tokens = s->d_in; in.pos = s->d_in + T; in.cell = s->d_in + 2 * T; in.n_vis = s->d_in + 3 * T; in.seq = s->d_in + 4 * T; in.prev = s->d_in + 5 * T;
         in.conv = s->d_in + 8 * T + at_conv;
         in.lin = s->d_in + 8 * T + at_lin; in.lin_long = in.lin + 4 * in.n_lin; in.lin_first = in.lin_long + 4 * in.n_lin_long; in.lin_chunks = in.lin_first + in.n_lin_long;
@@ -1884,6 +1914,8 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             in.last = &one;
         }
         struct Whole { LayerState * s; ~Whole() { if (s->tail) swap_tail(s); } } whole{s};      // however the pass ends, the buffers are in their own places behind it
+        app.clear();
+        PI_TRY(start_pass(m, in, n_in, n_in, n_app));
         PI_TRY(pass_layers(m, in));
         for (int r0 = 0; r0 < (int)rows.size(); r0 += kHeadRows) {
             const int n = std::min(kHeadRows, (int)rows.size() - r0);
@@ -1901,8 +1933,9 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
                 k = e;
             }
         }
+        waited = R > 0;                                            // (what was wanted has arrived)
     }
-    PI_HIP_TRY(hipStreamSynchronize(m->stream));
+    if (!waited) PI_HIP_TRY(hipStreamSynchronize(m->stream));
     s->in_flight = false;
     return PI_OK;
 }

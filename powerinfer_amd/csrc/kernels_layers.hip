@@ -19,11 +19,7 @@ template <typename LD> __device__ float row_rms_scale(int cols, float eps, doubl
     return pi_inv_sqrt((float)(s / cols) + eps);
 }
 
-__global__ __launch_bounds__(1024) void embed_norm_kernel(const uint16_t * __restrict__ table, int cols, const int32_t * __restrict__ tokens,
-                                                          const float * __restrict__ w, float eps, float * __restrict__ x) {
-    __shared__ double red[16];
-    const uint16_t * row = table + (size_t)tokens[blockIdx.x] * cols;
-    float * out = x + (size_t)blockIdx.x * cols;
+__device__ void embed_norm_row(const uint16_t * __restrict__ row, int cols, const float * __restrict__ w, float eps, float * __restrict__ out, double * red) {
     if (cols <= 8 * (int)blockDim.x) {              // row and weights requested together, kept in registers
         float v[8], wv[8];
         double s = 0.0;
@@ -42,6 +38,11 @@ __global__ __launch_bounds__(1024) void embed_norm_kernel(const uint16_t * __res
     }
     const float sc = row_rms_scale(cols, eps, red, [&](int i) { return bf16_to_f32(row[i]); });
     for (int i = threadIdx.x; i < cols; i += blockDim.x) out[i] = bf16_to_f32(row[i]) * sc * w[i];
+}
+__global__ __launch_bounds__(1024) void embed_norm_kernel(const uint16_t * __restrict__ table, int cols, const int32_t * __restrict__ tokens,
+                                                          const float * __restrict__ w, float eps, float * __restrict__ x) {
+    __shared__ double red[16];
+    embed_norm_row(table + (size_t)tokens[blockIdx.x] * cols, cols, w, eps, x + (size_t)blockIdx.x * cols, red);
 }
 
 template <typename ST>
@@ -82,21 +83,18 @@ __global__ __launch_bounds__(1024) void norm_pair_kernel(const float * __restric
     }
 }
 
-__global__ __launch_bounds__(256) void embed_bigram_kernel(const uint16_t * __restrict__ table, int cols, const int32_t * __restrict__ tokens, int32_t * prev, float scale,
-                                                           const uint16_t * __restrict__ bigram, int buckets, long long mul_prev, long long mul_cur, int carry,
-                                                           float * __restrict__ x, float * __restrict__ x0) {
-    const int t = blockIdx.x, tok = tokens[t], before = prev[t];
-    const uint16_t * a = table + (size_t)tok * cols, * b = nullptr;
-    if (bigram) b = bigram + (size_t)(before < 0 ? buckets : (int)(((long long)before * mul_prev + (long long)tok * mul_cur) % buckets)) * cols;
-    float * o = x + (size_t)t * cols, * o0 = x0 ? x0 + (size_t)t * cols : nullptr;
+struct Bigram { const uint16_t * table; float scale; const uint16_t * bigram; int buckets; long long mul_prev, mul_cur; };
+__device__ void embed_bigram_row(const Bigram & g, int cols, int tok, int before, float * __restrict__ o, float * __restrict__ o0) {
+    const uint16_t * a = g.table + (size_t)tok * cols, * b = nullptr;
+    if (g.bigram) b = g.bigram + (size_t)(before < 0 ? g.buckets : (int)(((long long)before * g.mul_prev + (long long)tok * g.mul_cur) % g.buckets)) * cols;
     if ((cols & 7) == 0) {
-        for (int i = threadIdx.x * 8; i < cols; i += 2048) {
+        for (int i = threadIdx.x * 8; i < cols; i += blockDim.x * 8) {
             const pi_u32x4 u = pi_ld16(a + i), w = b ? pi_ld16(b + i) : pi_u32x4{0, 0, 0, 0};
             float v[8];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                v[2 * j] = __uint_as_float(u[j] << 16) * scale + __uint_as_float(w[j] << 16);
-                v[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u) * scale + __uint_as_float(w[j] & 0xffff0000u);
+                v[2 * j] = __uint_as_float(u[j] << 16) * g.scale + __uint_as_float(w[j] << 16);
+                v[2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u) * g.scale + __uint_as_float(w[j] & 0xffff0000u);
             }
 #pragma unroll
             for (int j = 0; j < 8; j += 4) {
@@ -105,12 +103,16 @@ __global__ __launch_bounds__(256) void embed_bigram_kernel(const uint16_t * __re
             }
         }
     } else {
-        for (int i = threadIdx.x; i < cols; i += 256) {
-            const float v = bf16_to_f32(a[i]) * scale + (b ? bf16_to_f32(b[i]) : 0.0f);
+        for (int i = threadIdx.x; i < cols; i += blockDim.x) {
+            const float v = bf16_to_f32(a[i]) * g.scale + (b ? bf16_to_f32(b[i]) : 0.0f);
             o[i] = v;
             if (o0) o0[i] = v;
         }
     }
+}
+__global__ __launch_bounds__(256) void embed_bigram_kernel(Bigram g, int cols, const int32_t * __restrict__ tokens, int32_t * prev, int carry, float * __restrict__ x, float * __restrict__ x0) {
+    const int t = blockIdx.x, tok = tokens[t];
+    embed_bigram_row(g, cols, tok, prev[t], x + (size_t)t * cols, x0 ? x0 + (size_t)t * cols : nullptr);
     if (carry) {
         __syncthreads();                               // every thread has read prev[t]
         if (threadIdx.x == 0) prev[t] = tok;
@@ -306,21 +308,59 @@ __global__ __launch_bounds__(256) void group_gemm_kernel(pi_group_gemm g) {
 // ---------------------------------------------------------------------------------------------------------------------------------
 // rotation angles: formed and reduced in fp64, so that the fp32 cosine and sine are right at any position
 // ---------------------------------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ float2 rope_angle_at(int pos, int i, int dims, double base, const double * freq, double length) {
+    double s, c;
+    sincos((double)pos * (freq ? freq[i] : pow(base, -2.0 * (double)i / (double)dims)), &s, &c);
+    return freq ? make_float2((float)(length * c), (float)(length * s)) : make_float2((float)c, (float)s);
+}
 __global__ void rope_angles_kernel(const int32_t * __restrict__ pos, int T, int dims, double base, float2 * __restrict__ cs) {
     const int half = dims / 2, idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= T * half) return;
-    const int t = idx / half, i = idx % half;
-    double s, c;
-    sincos((double)pos[t] * pow(base, -2.0 * (double)i / (double)dims), &s, &c);
-    cs[idx] = make_float2((float)c, (float)s);
+    if (idx < T * half) cs[idx] = rope_angle_at(pos[idx / half], idx % half, dims, base, nullptr, 1.0);
 }
 
 __global__ void rope_table_kernel(const int32_t * __restrict__ pos, int T, int half, const double * __restrict__ freq, double length, float2 * __restrict__ cs) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= T * half) return;
-    double s, c;
-    sincos((double)pos[idx / half] * freq[idx % half], &s, &c);
-    cs[idx] = make_float2((float)(length * c), (float)(length * s));
+    if (idx < T * half) cs[idx] = rope_angle_at(pos[idx / half], idx % half, 2 * half, 0.0, freq, length);
+}
+
+// What a pass begins with, in one launch: its integers on their way from pinned memory to the device, the new cells into their sequences' lists, the
+// embeddings and the rotations' angles.  A copy and up to four launches were 11 us on the device and more for the host to issue, with nothing
+// to run beside them.  A short pass reads its tokens and positions in pinned memory as well; a long one is two launches, as each such read
+// crosses the link: the copy, then the rest from device memory.
+__global__ __launch_bounds__(1024) void pass_start_kernel(pi::PassStart p, Bigram g, int embeds, int copies, int appends) {
+    __shared__ double red[16];
+    const int tid = threadIdx.x, nt = blockDim.x;
+    int b = blockIdx.x;
+    if (b < embeds) {
+        const int tok = p.tokens[b];
+        float * x = p.x + (size_t)b * p.cols;
+        if (p.norm) embed_norm_row((const uint16_t *)p.table + (size_t)tok * p.cols, p.cols, p.norm, p.eps, x, red);
+        else embed_bigram_row(g, p.cols, tok, p.prev[b], x, p.x0 ? p.x0 + (size_t)b * p.cols : nullptr);
+        return;
+    }
+    b -= embeds;
+    if (b < copies) {                                  // (both sides start on 16 bytes)
+        const size_t i = ((size_t)b * nt + tid) * 4;
+        if (i + 4 <= p.words) *reinterpret_cast<int4 *>(p.dst + i) = *reinterpret_cast<const int4 *>(p.src + i);
+        else for (size_t k = i; k < p.words; ++k) p.dst[k] = p.src[k];
+        return;
+    }
+    b -= copies;
+    if (b < appends) {
+        const int i = b * nt + tid;
+        if (i < p.n_append) p.lists[(size_t)p.append[3 * i] * p.list_ld + p.append[3 * i + 1]] = p.append[3 * i + 2];
+        return;
+    }
+    b -= appends;
+    for (int k = 0; k < p.n_rot; ++k) {
+        const pi::PassStart::Rot & r = p.rot[k];
+        const int half = r.dims / 2, n = (p.T * half + nt - 1) / nt, idx = b * nt + tid;
+        if (b < n) {
+            if (idx < p.T * half) reinterpret_cast<float2 *>(r.cs)[idx] = rope_angle_at(p.pos[idx / half], idx % half, r.dims, r.base, r.freq, r.length);
+            return;
+        }
+        b -= n;
+    }
 }
 
 // expert choice, one workgroup per token
@@ -628,6 +668,20 @@ __global__ void cells_advance_kernel(int T, const int32_t * __restrict__ seq, co
 
 }  // namespace
 
+namespace pi {
+int pass_start(const PassStart & p, hipStream_t st) {
+    const int nt = p.norm && p.cols > 2048 ? 1024 : 256;
+    const auto blocks = [&](size_t n) { return (int)((n + nt - 1) / nt); };
+    const int embeds = p.table ? p.T : 0, copies = blocks((p.words + 3) / 4), appends = blocks((size_t)p.n_append);
+    int rots = 0;
+    for (int k = 0; k < p.n_rot; ++k) rots += blocks((size_t)p.T * (p.rot[k].dims / 2));
+    if (embeds + copies + appends + rots == 0) return PI_OK;
+    const Bigram g{(const uint16_t *)p.table, p.scale, (const uint16_t *)p.bigram, p.buckets, (long long)p.mul_prev, (long long)p.mul_cur};
+    hipLaunchKernelGGL(pass_start_kernel, dim3(embeds + copies + appends + rots), dim3(nt), 0, st, p, g, embeds, copies, appends);
+    return check_launch("pass_start");
+}
+}  // namespace pi
+
 extern "C" {
 
 int pi_k_embed_norm(const void * table, int cols, const int32_t * tokens, int T, const float * w, float eps, float * x, pi_stream_t stream) {
@@ -639,8 +693,8 @@ int pi_k_embed_norm(const void * table, int cols, const int32_t * tokens, int T,
 int pi_k_embed_bigram(const void * table, int cols, const int32_t * tokens, int32_t * prev, int T, float scale, const void * bigram, int32_t buckets, int64_t mul_prev,
                       int64_t mul_cur, int carry, float * x, float * x0, pi_stream_t stream) {
     if (!table || !tokens || !prev || !x || cols <= 0 || T <= 0 || (bigram && buckets <= 0)) return pi::fail(PI_E_ARG, "pi_k_embed_bigram: bad arguments");
-    hipLaunchKernelGGL(embed_bigram_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, (const uint16_t *)table, cols, tokens, prev, scale, (const uint16_t *)bigram, buckets,
-                       (long long)mul_prev, (long long)mul_cur, carry, x, x0);
+    hipLaunchKernelGGL(embed_bigram_kernel, dim3(T), dim3(256), 0, (hipStream_t)stream, Bigram{(const uint16_t *)table, scale, (const uint16_t *)bigram, buckets, (long long)mul_prev, (long long)mul_cur},
+                       cols, tokens, prev, carry, x, x0);
     return pi::check_launch("pi_k_embed_bigram");
 }
 

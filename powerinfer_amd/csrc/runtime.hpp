@@ -47,6 +47,18 @@ struct HostStage {
 // pi_k_attn_fused with such extra workgroups
 int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream);
+// What a pass of a model of layers begins with (pass_start_kernel): words from src to dst; triples (sequence, place, cell) into lists; T embeddings (table null:
+// none) with a norm or a scale and bigrams; angles of up to kRots rotations (freq null: from base).
+struct PassStart {
+    static constexpr int kRots = 8;
+    struct Rot { int dims; double base, length; const double * freq; void * cs; };
+    const int32_t * src; int32_t * dst; size_t words;
+    const int32_t * append; int n_append; int32_t * lists; size_t list_ld;
+    const void * table; int cols, T; const int32_t * tokens, * prev, * pos; const float * norm; float eps, scale;
+    const void * bigram; int buckets; int64_t mul_prev, mul_cur; float * x, * x0;
+    int n_rot; Rot rot[kRots];
+};
+int pass_start(const PassStart & p, hipStream_t st);
 // whether pi_k_attn_chunk takes the tokens of a chunk against n_kv_max cells 16 at a time on the matrix cores
 bool attn_chunk_by_16(int hd, int n_kv_max);
 int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
