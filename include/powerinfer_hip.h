@@ -405,6 +405,9 @@ PI_API int pi_k_dequant_q4_f16(const void * W_q4, const void * W_rest_q4, const 
 PI_API int pi_k_gemm_q4_chunk_supported(int rows, int cols);
 PI_API int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, const void * x_ol, int T, int epilogue, const float * add1, const float * add2,
                               float * y, int tile, pi_stream_t stream);
+/* The same with room for a transposed matrix's parts: bufs, six device buffers of T * rows floats (null: none).  Few tokens then have four workgroups a tile. */
+PI_API int pi_k_gemm_q4_chunk_parts(const void * W_q4, int rows, int cols, int transposed, const void * x_ol, int T, int epilogue, const float * add1, const float * add2,
+                                    float * y, int tile, float * const * bufs, pi_stream_t stream);
 /* the same transposed, out_f16[cols][rows]: rows % 8 == 0, cols % 256 == 0, operands 16-byte aligned (else PI_E_UNSUPPORTED) */
 PI_API int pi_k_dequant_q4_t_f16(const void * W_q4, const void * W_rest_q4, const uint32_t * hot_words, const int32_t * hot_prefix, int rows, int cols,
                                void * out_f16, pi_stream_t stream);

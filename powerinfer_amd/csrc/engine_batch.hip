@@ -565,7 +565,11 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     else PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     if (down_ol) {
         const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
-        PI_TRY(pi_k_gemm_q4_chunk(down.dev, d, ff, 1, b->h16, T, falcon ? PI_EPI_ADD2 : PI_EPI_ADD, a1, a2, b->x2, 0, st));
+        float * bufs[6] = {};                          // room in what the FFN is done with (T rows each where the products were apart)
+        int n = 0;
+        for (float * p : {b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits})
+            for (int k = 0; p && !one_kernel && k < ff / d && n < 6; ++k) bufs[n++] = p + (size_t)k * T * d;
+        PI_TRY(pi_k_gemm_q4_chunk_parts(down.dev, d, ff, 1, b->h16, T, falcon ? PI_EPI_ADD2 : PI_EPI_ADD, a1, a2, b->x2, 0, n == 6 ? bufs : nullptr, st));
         std::swap(b->x, b->x2);
         return PI_OK;
     }

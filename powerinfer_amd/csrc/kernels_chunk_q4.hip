@@ -24,6 +24,8 @@ namespace {
 // 5.1e-7 / 3.6e-7; expanded and multiplied by the library 4.1e-7, 5.7e-7, 5.9e-7 and 6.2e-7.  The longest sums, of the transposed
 // matrices, have the most; one part would be enough elsewhere, and two are kept where results have them: another order of sums rounds
 // activations to eight bits the other way here and there, which moves a model's logits by 1e-2.
+// Of few tokens of a transposed matrix, which has few row tiles, 32 rows a workgroup leave most of each line of 128 bytes to other workgroups and read the
+// tokens 128 times; four workgroups then share a tile of 64 rows, two parts of the sum each (kCqSlices).
 // What bounds it at 130 tokens of 12288 x 4096 (21 us; the blocks alone 5, the matrix instructions 6): about 12 us are launch, first
 // trip and last stores, which one workgroup a unit does not overlap with its products; the rest is shared about evenly between the
 // tokens' way from the L2 (270 MB), expanding and multiplying.
@@ -40,7 +42,10 @@ __device__ __forceinline__ uint32_t cq_high(uint32_t q, uint32_t d) { return cq_
 typedef uint32_t cq_words __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t cq_pair __attribute__((ext_vector_type(2), aligned(4)));
 
-struct ChunkQ4 { const unsigned char * W; const unsigned char * x; int T, rows, cols, nx, ny, parts, epi; const float * add1, * add2; float * y; };
+constexpr int kCqSlices = 4, kCqBufs = 2 * (kCqSlices - 1);
+// slices (transposed, eight parts): 1, or kCqSlices workgroups of a tile with two parts each: the first one leaves their sum in y, the others leave theirs
+// one by one in bufs, and chunk_parts_kernel adds them in the order of one workgroup
+struct ChunkQ4 { const unsigned char * W; const unsigned char * x; int T, rows, cols, nx, ny, parts, epi; const float * add1, * add2; float * y; int slices; float * bufs[kCqBufs]; };
 
 constexpr int cq_units(int MT, bool trans) { return !trans && MT > 4 ? 2 : 1; }          // pairs of blocks a lane expands of a stage
 constexpr int cq_expand(int MT, bool trans) { return MT / cq_units(MT, trans); }            // expanding waves (TRANS: of one of two sets)
@@ -54,7 +59,13 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
     // L2; with TRANS a line of W holds the blocks of seven 32-row tiles)
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8, per = (a.nx + 7) / 8, tx = xcd * per + slot / a.ny, ty = slot % a.ny;
     if (tx >= a.nx) return;                                         // (slot / ny < per: the grid is 8 per ny)
-    const int row0 = tx * 16 * MT, nk = a.cols / kCqBK;
+    const int row0 = tx * 16 * MT, slabs = a.cols / 128;
+    int nk = a.cols / kCqBK, k0 = 0, part = 0, until = a.parts;
+    const auto slabs_ahead = [&](int p) { return p * (slabs / a.parts) + std::min(p, slabs % a.parts); };      // of the parts ahead of p (the longer parts come first)
+    if (TRANS && a.slices > 1) {
+        part = 2 * (int)blockIdx.y; until = part + 2;
+        k0 = slabs_ahead(part) / 2; nk = slabs_ahead(until) / 2 - k0;   // (an even number of slabs)
+    }
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
     // where a fragment's piece of row i and columns 8 g .. lies: rows trade places so that an expanding wave's stores spread over the banks
     auto place = [](int s, int m, int gg, int ii) {
@@ -133,7 +144,7 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
             const uint32_t at = (uint32_t)(8 * ng * line) + block * 18, at_q = at + 4 * cw - (block & 1) * 2;
             const uint32_t mid = block & 1 ? 0x07060504u : 0x05040302u, scale = block & 1 ? 0x07060302u : 0x05040100u;
             auto fetch = [&](Raw & r, int k) {
-                const unsigned char * p = a.W + (size_t)k * kCqBK * line;
+                const unsigned char * p = a.W + (size_t)(k0 + k) * kCqBK * line;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) r.q[e] = *reinterpret_cast<const cq_pair *>(p + e * line + at_q);
             };
@@ -209,9 +220,9 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[m][n] = sum[m][n] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int slabs = a.cols / 128;
-    int part = 0, left = slabs / a.parts + (0 < slabs % a.parts ? 1 : 0);       // slabs of 128 columns left of it; the longer parts come first
+    int left = slabs / a.parts + (part < slabs % a.parts ? 1 : 0);  // slabs of 128 columns left of the present part
     auto fold = [&]() {
+        if (TRANS && blockIdx.y > 0 && part + 1 == until) return;      // (the second part of a slice behind the first stays by itself)
         left = slabs / a.parts + (++part < slabs % a.parts ? 1 : 0);
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -225,7 +236,7 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
     const int tile0 = (ty * WN + wave) * NT, tiles = (a.T + 15) / 16;
     const unsigned char * xt[NT];                                   // (tiles past the end read the last one and are not stored)
 #pragma unroll
-    for (int n = 0; n < NT; ++n) xt[n] = a.x + (size_t)std::min(tile0 + n, tiles - 1) * 32 * a.cols + lane * 16;
+    for (int n = 0; n < NT; ++n) xt[n] = a.x + (size_t)std::min(tile0 + n, tiles - 1) * 32 * a.cols + (size_t)k0 * (kCqSteps * kFrag) + lane * 16;
     // steps ahead a token's fragments are requested: a stage where the registers hold that many
     constexpr int kRegs = cq_threads(MT, WN, TRANS) > 512 ? 168 : 256, kHeld = MT * NT * 8 + MT * 8 + 44;
     constexpr int kRing = kHeld + NT * 32 <= kRegs ? kCqSteps : kHeld + NT * 16 <= kRegs ? kCqSteps / 2 : kCqSteps / 4;
@@ -269,6 +280,12 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
             if (tok >= a.T || row >= a.rows) continue;              // (rows % 4 == 0)
             const size_t o = (size_t)tok * a.rows + row;
             float v[4] = {acc[m][n][0], acc[m][n][1], acc[m][n][2], acc[m][n][3]};
+            if (TRANS && a.slices > 1) {
+                float * to = blockIdx.y ? a.bufs[2 * blockIdx.y - 2] : a.y;
+                *reinterpret_cast<float4 *>(to + o) = make_float4(v[0], v[1], v[2], v[3]);
+                if (blockIdx.y) *reinterpret_cast<float4 *>(a.bufs[2 * blockIdx.y - 1] + o) = make_float4(sum[m][n][0], sum[m][n][1], sum[m][n][2], sum[m][n][3]);
+                continue;
+            }
             if (a.epi == PI_EPI_RELU) { for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.0f); }
             else if (a.epi >= PI_EPI_ADD) {
                 const float4 a1 = *reinterpret_cast<const float4 *>(a.add1 + o);
@@ -282,6 +299,22 @@ __global__ __launch_bounds__(cq_threads(MT, WN, TRANS), 2) void gemm_q4_chunk_ke
         }
 }
 
+__global__ __launch_bounds__(256) void chunk_parts_kernel(ChunkQ4 a) {
+    const size_t o = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (o >= (size_t)a.T * a.rows) return;
+    float4 v = *reinterpret_cast<const float4 *>(a.y + o), b[kCqBufs], a1 = make_float4(0, 0, 0, 0), a2 = a1;
+#pragma unroll
+    for (int k = 0; k < kCqBufs; ++k) b[k] = *reinterpret_cast<const float4 *>(a.bufs[k] + o);
+    if (a.epi >= PI_EPI_ADD) a1 = *reinterpret_cast<const float4 *>(a.add1 + o);
+    if (a.epi == PI_EPI_ADD2) a2 = *reinterpret_cast<const float4 *>(a.add2 + o);
+#pragma unroll
+    for (int k = 0; k < kCqBufs; ++k) { v.x += b[k].x; v.y += b[k].y; v.z += b[k].z; v.w += b[k].w; }
+    if (a.epi == PI_EPI_RELU) v = make_float4(fmaxf(v.x, 0.0f), fmaxf(v.y, 0.0f), fmaxf(v.z, 0.0f), fmaxf(v.w, 0.0f));
+    if (a.epi >= PI_EPI_ADD) v = make_float4(__fadd_rn(v.x, a1.x), __fadd_rn(v.y, a1.y), __fadd_rn(v.z, a1.z), __fadd_rn(v.w, a1.w));
+    if (a.epi == PI_EPI_ADD2) v = make_float4(__fadd_rn(v.x, a2.x), __fadd_rn(v.y, a2.y), __fadd_rn(v.z, a2.z), __fadd_rn(v.w, a2.w));
+    *reinterpret_cast<float4 *>(a.y + o) = v;
+}
+
 template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hipStream_t st) {
     constexpr size_t lds = (size_t)2 * kCqSteps * MT * 1024;
     a.nx = (a.rows + 16 * MT - 1) / (16 * MT); a.ny = ((a.T + 15) / 16 + NT * WN - 1) / (NT * WN);
@@ -289,7 +322,7 @@ template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hip
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (raised != hipSuccess) return pi::hip_fail(raised, "pi_k_gemm_q4_chunk: LDS size");
     }
-    hipLaunchKernelGGL((gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), dim3((unsigned)(8 * ((a.nx + 7) / 8) * a.ny)), dim3(cq_threads(MT, WN, TRANS)), lds, st, a);
+    hipLaunchKernelGGL((gemm_q4_chunk_kernel<MT, NT, WN, TRANS>), dim3((unsigned)(8 * ((a.nx + 7) / 8) * a.ny), a.slices), dim3(cq_threads(MT, WN, TRANS)), lds, st, a);
     return pi::check_launch("pi_k_gemm_q4_chunk");
 }
 
@@ -297,7 +330,7 @@ template <int MT, int NT, int WN, bool TRANS> int launch_chunk_q4(ChunkQ4 a, hip
 // (no 96 rows with three token tiles for each of four waves: one round of that takes as long as two of 333 or 334, two workgroups of which share a
 // unit.  17 to 24 token tiles of 7B shapes: 11008 x 4096, us, 280 tokens 53.3 / 36.7, 360 tokens 55.0 / 42.2; 12288 x 4096 54.3 / 39.9)
 constexpr int kCqTiles[] = {112, 122, 123, 215, 232, 314, 323, 333, 334, 414, 423, 424, 434, 444, 624};
-constexpr int kCqTilesT[] = {212, 213, 215, 223, 422, 423, 424, 434};
+constexpr int kCqTilesT[] = {212, 213, 215, 223, 422, 423, 424, 433, 434};
 // What a launch takes goes with the rounds of workgroups over the compute units times what 32 columns of a tile take of a unit, in clocks: the
 // tokens' fragments at 64 bytes a clock, the matrix instructions of a SIMD, or the latency of a step where both are little; transposed, the
 // lines of 128 bytes that 18 or 36 are taken of, and the tokens.  Of 152 measured launches (19 lengths of 17 .. 512 tokens, the matrices of 7B
@@ -316,6 +349,28 @@ int cq_choose(int rows, int T, bool trans, int units) {
     return best;
 }
 
+// Whether the transposed product is done in slices, by what both ways take in clocks: rounds of workgroups over the units times the steps of one and what a
+// round takes by itself (with 32 rows also the lines of every row tile, which all token tiles share), and of slices a launch and 36 bytes a value more.
+// Over 80 launches (17 .. 512 tokens of 2048 x 5632, 4096 x 11008, 4096 x 16384, 5120 x 13824 and 8192 x 32768) slices take 0.84 of what one
+// workgroup a tile does on average and never more.  us, one and slices: 4096 x 11008, 17 tokens 25.6 / 19.5, 130 36.6 / 28.0, 192 40.9 / 33.2, 288 55.9 /
+// 50.5, 333 54.9 / 60.0 (not taken); 5120 x 13824, 130 tokens 55.0 / 47.8; 8192 x 32768, 64 tokens 113 / 73.
+double cq_clocks(int tile, int rows, int cols, int T, int slices, int units) {
+    const int m = tile / 100, t = tile / 10 % 10, w = tile % 10, nx = (rows + 16 * m - 1) / (16 * m);
+    const long long groups = (long long)nx * (((T + 15) / 16 + t * w - 1) / (t * w)) * slices;
+    const double step = m == 2 ? std::max(100.0 + 12.0 * t * w, 150.0 * std::min(1.0, (double)nx * slices / units)) : 180.0 + 13.0 * t * w;
+    return (double)((groups + units - 1) / units) * (step * cols / 32 / slices + (m == 2 ? 6000.0 : 4000.0)) + (slices > 1 ? 4600.0 + 0.018 * T * rows : 0.0);
+}
+int cq_slices(int & tile, int rows, int cols, int T, int units) {
+    int best = tile, slices = 1;
+    double least = cq_clocks(tile, rows, cols, T, 1, units);
+    for (int t : kCqTilesT) {
+        const double c = cq_clocks(t, rows, cols, T, kCqSlices, units);
+        if (c < least) { least = c; best = t; slices = kCqSlices; }
+    }
+    tile = best;
+    return slices;
+}
+
 }  // namespace
 
 extern "C" {
@@ -324,6 +379,11 @@ int pi_k_gemm_q4_chunk_supported(int rows, int cols) { return rows > 0 && cols >
 
 int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, const void * x_ol, int T, int epilogue, const float * add1, const float * add2,
                        float * y, int tile, pi_stream_t stream) {
+    return pi_k_gemm_q4_chunk_parts(W_q4, rows, cols, transposed, x_ol, T, epilogue, add1, add2, y, tile, nullptr, stream);
+}
+
+int pi_k_gemm_q4_chunk_parts(const void * W_q4, int rows, int cols, int transposed, const void * x_ol, int T, int epilogue, const float * add1, const float * add2,
+                             float * y, int tile, float * const * bufs, pi_stream_t stream) {
     if (!W_q4 || !x_ol || !y || T <= 0) return pi::fail(PI_E_ARG, "pi_k_gemm_q4_chunk: null pointer or empty shape");
     if (epilogue < 0 || epilogue > PI_EPI_ADD2 || (epilogue >= PI_EPI_ADD && !add1) || (epilogue == PI_EPI_ADD2 && !add2))
         return pi::fail(PI_E_ARG, "pi_k_gemm_q4_chunk: bad epilogue arguments");
@@ -331,9 +391,18 @@ int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, co
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_gemm_q4_chunk: cols % 256 == 0, rows % 64 == 0, W on 4 bytes and the other operands on 16");
     if (T > 65536) return pi::fail(PI_E_UNSUPPORTED, "pi_k_gemm_q4_chunk: at most 65536 tokens");
     const int parts = transposed ? 8 : rows > 2 * cols ? 2 : 1;
-    const ChunkQ4 a{(const unsigned char *)W_q4, (const unsigned char *)x_ol, T, rows, cols, 0, 0, std::min(parts, cols / 128), epilogue, add1, add2, y};
+    ChunkQ4 a{(const unsigned char *)W_q4, (const unsigned char *)x_ol, T, rows, cols, 0, 0, std::min(parts, cols / 128), epilogue, add1, add2, y, 1, {}};
     hipStream_t st = (hipStream_t)stream;
-    if (tile == 0) tile = cq_choose(rows, T, transposed != 0, pi::compute_units());
+    bool room = bufs && transposed && a.parts == 2 * kCqSlices;
+    for (int k = 0; room && k < kCqBufs; ++k) { a.bufs[k] = bufs[k]; room = bufs[k] && ((uintptr_t)bufs[k] & 15) == 0; }
+    if (tile >= 1000) { if (!room) return pi::fail(PI_E_ARG, "pi_k_gemm_q4_chunk_parts: no room for parts"); tile -= 1000; a.slices = kCqSlices; }
+    if (tile == 0) {
+        const int units = pi::compute_units();
+        if (units <= 0) return PI_E_HIP;
+        tile = cq_choose(rows, T, transposed != 0, units);
+        if (room) a.slices = cq_slices(tile, rows, cols, T, units);
+    }
+    const auto launch = [&]() -> int {
 #define PI_CQ1(M, N, W) case M * 100 + N * 10 + W: return launch_chunk_q4<M, N, W, false>(a, st)
 #define PI_CQ2(M, N, W) case M * 100 + N * 10 + W: return launch_chunk_q4<M, N, W, true>(a, st)
     if (!transposed) {
@@ -343,12 +412,17 @@ int pi_k_gemm_q4_chunk(const void * W_q4, int rows, int cols, int transposed, co
         }
     } else {
         switch (tile) {
-            PI_CQ2(2, 1, 2); PI_CQ2(2, 1, 3); PI_CQ2(2, 1, 5); PI_CQ2(2, 2, 3); PI_CQ2(4, 2, 2); PI_CQ2(4, 2, 3); PI_CQ2(4, 2, 4); PI_CQ2(4, 3, 4);
+            PI_CQ2(2, 1, 2); PI_CQ2(2, 1, 3); PI_CQ2(2, 1, 5); PI_CQ2(2, 2, 3); PI_CQ2(4, 2, 2); PI_CQ2(4, 2, 3); PI_CQ2(4, 2, 4); PI_CQ2(4, 3, 3); PI_CQ2(4, 3, 4);
         }
     }
 #undef PI_CQ1
 #undef PI_CQ2
     return pi::fail(PI_E_ARG, "pi_k_gemm_q4_chunk: no such tile");
+    };
+    const int rc = launch();
+    if (rc != PI_OK || a.slices == 1) return rc;
+    hipLaunchKernelGGL(chunk_parts_kernel, dim3((unsigned)(((size_t)T * rows / 4 + 255) / 256)), dim3(256), 0, st, a);
+    return pi::check_launch("pi_k_gemm_q4_chunk_parts");
 }
 
 }  // extern "C"

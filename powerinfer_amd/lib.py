@@ -197,6 +197,7 @@ _SIGS = {
     "pi_k_dequant_q4_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "pi_k_gemm_q4_chunk_supported": (_i, [_i, _i]),
     "pi_k_gemm_q4_chunk": (_i, [_vp, _i, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _vp]),
+    "pi_k_gemm_q4_chunk_parts": (_i, [_vp, _i, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _i, _vp, _vp]),
     "pi_k_dequant_q4_t_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "pi_k_assemble_rows_f16": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp]),
     "pi_k_embed_batch_q4": (_i, [_vp, _i, _vp, _i, _vp, _vp]),
