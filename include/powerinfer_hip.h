@@ -567,6 +567,11 @@ PI_API int pi_k_attn_chunk_once(const float * qkv, int qkv_stride, int T, int n_
 PI_API int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                            const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache,
                            float * out, int out_stride, void * out_f16, pi_stream_t stream);
+/* The same where the tokens are taken 16 at a time (head sizes 64 and 128, T > 1, cells whose scores fit): out_f16 receives the output rounded through Q8_0 blocks,
+ * in rows of `cols` values or (ol) in the operand layout. */
+PI_API int pi_k_attn_chunk_q8(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                              const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, int cols, void * out_f16, int ol,
+                              pi_stream_t stream);
 PI_API int pi_k_embed_batch(const void * table_f16, int cols, const int32_t * tokens, int T, float * x, pi_stream_t stream);
 PI_API int pi_k_argmax_batch(const float * logits, int n, int T, int32_t * tokens, int32_t * positions, int32_t * step,
                              int32_t * out_tokens, int max_steps, pi_stream_t stream);

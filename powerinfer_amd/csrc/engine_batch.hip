@@ -74,7 +74,8 @@ pi_norm mk_norm(int kind, float eps, const Tensor & w, const Tensor * b) {
 // the model is rounded to eight bits behind it and there are more than 16 tokens (against 16 tokens a workgroup, attn_chunk_mfma_kernel: 17
 // tokens 13.2 / 10.2 us, behind 1700 cells 48 / 37; 100 tokens 17.7 / 13.0), else the chunk kernels where the context fits them, the
 // split-over-cells path beyond
-int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size_t kv_off) {
+// q8: the output only as a Q4_0 matrix multiplies with it, by rows (1) or in the operand layout (2; t0 0), where the route has that (*q8 0 behind it)
+int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size_t kv_off, int * q8 = nullptr) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, hd = m->hd, gqa = m->gqa, mode = hp.arch == PI_ARCH_FALCON ? 2 : 0;
     const float * qkv = b->qkv + (size_t)t0 * (d + 2 * gqa);
@@ -85,6 +86,11 @@ int chunk_attention(pi_model * m, BatchState * b, int t0, int n, int kv_hi, size
         return pi_k_attn_chunk_once(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, nullptr, d, att16, m->stream);
     if (!b->route.scalar && pi_k_attn_chunk_rows_supported(hd, n, kv_hi) && !(b->route.pieces && pi::attn_chunk_by_16(hd, kv_hi)))
         return pi_k_attn_chunk_rows(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, att, d, att16, m->stream);
+    if (q8 && *q8 && n > 1 && !b->route.scalar && pi::attn_chunk_by_16(hd, kv_hi)) {
+        const int ol = *q8 == 2;
+        *q8 = 0;
+        return pi_k_attn_chunk_q8(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, d, att16, ol, m->stream);
+    }
     if (pi_k_attn_chunk_supported(hd, hp.n_ctx, kv_hi))
         return pi_k_attn_chunk(qkv, d + 2 * gqa, n, hp.n_head, hp.n_head_kv, hd, mode, m->theta_scale, m->freq_scale, pos, hp.n_ctx, kv_hi, q_rot, k, v, att, d, att16, m->stream);
     const int parts = m->attn_parts > 1 ? m->attn_parts : 2;
@@ -537,8 +543,11 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     }
     PI_TRY(chunk_product(m, b, il, PI_T_WQKV, qkv_ol, d + 2 * gqa, d, b->xa16, PI_EPI_NONE, nullptr, nullptr, b->qkv));
     if (cells_only(m, il)) return chunk_store(m, b, b->qkv + d, d + 2 * gqa, kv_off);
-    PI_TRY(in_pieces(b, [&](int t0, int n) { return chunk_attention(m, b, t0, n, b->kv_hi - (T - t0 - n), kv_off); }));
-    if (wo.type == PI_TYPE_Q4_0) PI_TRY(chunk_input(wo.type, wo_ol, b->att, T, d, &plain, b->att16, nullptr, st));
+    PI_TRY(in_pieces(b, [&](int t0, int n) -> int {                   // (the operand layout is of chunks in one piece)
+        int q8 = wo.type != PI_TYPE_Q4_0 ? 0 : wo_ol ? 2 : 1;
+        PI_TRY(chunk_attention(m, b, t0, n, b->kv_hi - (T - t0 - n), kv_off, &q8));
+        return q8 ? chunk_input(wo.type, wo_ol, b->att + (size_t)t0 * d, n, d, &plain, b->att16 + (size_t)t0 * d, nullptr, st) : PI_OK;
+    }));
     pi_norm fn;
     const __half * ffn_x = b->xf16;
     if (!falcon) {

@@ -614,6 +614,8 @@ __global__ void attn_merge_kernel(const float * __restrict__ part_acc, const flo
 //      them with two byte permutes per pair of cells and drops two 16-byte columns into its private LDS tile (32 cells a tile),
 //      from where the operand comes back with one 16-byte read.  No workgroup barrier inside the loops: the tile belongs to one
 //      wave and the LDS operations of a wave complete in order.  The waves' partial outputs meet in LDS in wave order.
+// q8: what the output matrix of a Q4_0 model multiplies with instead of the output, its values rounded through blocks of eight bits, by rows (1) or in
+// the operand layout (2); a launch of 5.2 us for 130 tokens of 4096 columns otherwise.
 // HD = 128 or 64.  LDS: 16 x (cells rounded up to 32, + 4) floats of scores + 4 x HD x 80 bytes of V tiles.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kAcVtStride = 40;                // halves per row of the transposed V tile: 32 cells + 8 of padding (conflict-free both ways)
@@ -621,7 +623,7 @@ template <int HD>
 __global__ __launch_bounds__(kBlock) void attn_chunk_mfma_kernel(const float * __restrict__ q_rot, const __half * __restrict__ k_cache,
                                                                  const __half * __restrict__ v_cache, int n_head, int n_head_kv, int n_ctx,
                                                                  const int32_t * __restrict__ pos_p, int T, float * __restrict__ out,
-                                                                 int q_stride, int out_stride, __half * __restrict__ out16, int s_stride) {
+                                                                 int q_stride, int out_stride, __half * __restrict__ out16, int s_stride, int q8) {
     static_assert(HD == 128 || HD == 64, "head size");
     extern __shared__ __align__(16) unsigned char smem[];
     float * s = reinterpret_cast<float *>(smem);                                       // [16][s_stride]
@@ -787,8 +789,13 @@ __global__ __launch_bounds__(kBlock) void attn_chunk_mfma_kernel(const float * _
             float v = 0.0f;
 #pragma unroll
             for (int w = 0; w < kWavesPerBlock; ++w) v += reinterpret_cast<const float *>(vt_all + (size_t)w * HD * kAcVtStride * 2)[q * PS + d];
-            out[(size_t)t * out_stride + (size_t)h * HD + d] = v;
-            if (out16) out16[(size_t)t * out_stride + (size_t)h * HD + d] = __float2half_rn(v);
+            const size_t o = (size_t)t * out_stride + (size_t)h * HD + d;
+            if (q8) {                                  // (a head is whole blocks of 32: half-waves go on together)
+                out16[q8 == 2 ? ol_index_of(t, h * HD + d, out_stride) : o] = __float2half_rn(q8_block_value(v));
+                continue;
+            }
+            out[o] = v;
+            if (out16) out16[o] = __float2half_rn(v);
         }
     }
 }
@@ -1745,10 +1752,10 @@ int pi_k_attn_fused_batch_ol(const float * qkv, int qkv_stride, const void * rop
     return attn_fused_batch(qkv, qkv_stride, rope_table, k_cache, v_cache, cache_seq_stride, n_seq, n_head, n_head_kv, hd, mode, n_ctx, pos, out, out_stride, out_ol, stream, 1);
 }
 
-int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+static int attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                     const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16,
-                    pi_stream_t stream) {
-    if (!qkv || !pos || !q_rot || !k_cache || !v_cache || !out || T <= 0 || T > kChunkMaxT) return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad arguments");
+                      int q8, pi_stream_t stream) {
+    if (!qkv || !pos || !q_rot || !k_cache || !v_cache || (q8 ? !out_f16 : !out) || T <= 0 || T > kChunkMaxT) return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad arguments");
     if (n_kv_max <= 0 || n_kv_max > n_ctx) n_kv_max = n_ctx;                  // cells the furthest token of the chunk attends: what the scores in LDS are sized for
     if (n_head <= 0 || n_head_kv <= 0 || n_head % n_head_kv || hd <= 0 || hd % 8 || hd / 2 > 1024 || kBlock % (hd / 8) || PI_WAVE % (hd / 8) || (mode != 0 && mode != 2))
         return pi::fail(PI_E_ARG, "pi_k_attn_chunk: bad head geometry or mode");
@@ -1770,16 +1777,29 @@ int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_
         }
         const dim3 grid(n_head, (T + 15) / 16);
         if (hd == 128) hipLaunchKernelGGL(attn_chunk_mfma_kernel<128>, grid, dim3(kBlock), sh_mfma, st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
-                                          n_head, n_head_kv, n_ctx, pos, T, out, n_head * hd, out_stride, (__half *)out_f16, s_stride);
+                                          n_head, n_head_kv, n_ctx, pos, T, out, n_head * hd, out_stride, (__half *)out_f16, s_stride, q8);
         else           hipLaunchKernelGGL(attn_chunk_mfma_kernel<64>, grid, dim3(kBlock), sh_mfma, st, q_rot, (const __half *)k_cache, (const __half *)v_cache,
-                                          n_head, n_head_kv, n_ctx, pos, T, out, n_head * hd, out_stride, (__half *)out_f16, s_stride);
+                                          n_head, n_head_kv, n_ctx, pos, T, out, n_head * hd, out_stride, (__half *)out_f16, s_stride, q8);
         return pi::check_launch("pi_k_attn_chunk");
     }
+    if (q8) return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_chunk_q8: head sizes 64 and 128, several tokens, cells whose scores fit");
     const size_t sh = sizeof(float) * ((size_t)n_ctx + (size_t)(kBlock / (hd / 8)) * hd);
     if (sh > 60 * 1024) return pi::fail(PI_E_UNSUPPORTED, "pi_k_attn_chunk: context too long for the single-pass kernel (pi_k_attn_chunk_supported)");
     hipLaunchKernelGGL(attn_decode_kernel, dim3(n_head, T), dim3(kBlock), sh, st,
                        q_rot, (const __half *)k_cache, (const __half *)v_cache, n_head, n_head_kv, hd, n_ctx, pos, out, n_head * hd, out_stride, (__half *)out_f16);
     return pi::check_launch("pi_k_attn_chunk");
+}
+
+int pi_k_attn_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                    const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, float * out, int out_stride, void * out_f16,
+                    pi_stream_t stream) {
+    return attn_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, n_kv_max, q_rot, k_cache, v_cache, out, out_stride, out_f16, 0, stream);
+}
+
+int pi_k_attn_chunk_q8(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
+                       const int32_t * pos, int n_ctx, int n_kv_max, float * q_rot, void * k_cache, void * v_cache, int cols, void * out_f16, int ol,
+                       pi_stream_t stream) {
+    return attn_chunk(qkv, qkv_stride, T, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, n_kv_max, q_rot, k_cache, v_cache, nullptr, cols, out_f16, ol ? 2 : 1, stream);
 }
 
 // where attn_chunk_rows_kernel is the faster one: fewer than 32 tokens against many cells are better off with attn_chunk_mfma_kernel, whose waves

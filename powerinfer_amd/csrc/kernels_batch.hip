@@ -16,25 +16,6 @@ namespace {
 // them to fp16 before every dot, ggml.c:9703-9716) and read by every tile from L2.
 // =====================================================================================================
 
-// the value a Q8_0 block keeps of v: q * fp16(amax / 127) with q = rint(v * 127 / amax) and amax over the 32 consecutive elements
-// the 32 lanes of a half-wave hold (quantize_row_q8_0, x86 path, ggml-quants.c:702-760), rounded to fp16 for a mat-mul input
-template <int N> __device__ __forceinline__ void q8_block_values(float (&v)[N], float amax) {       // values of a block whose largest magnitude is amax
-    const float d = pi_round_f16(pi_div(amax, 127.0f)), id = (amax != 0.0f) ? pi_div(127.0f, amax) : 0.0f;
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] = __fmul_rn((float)(int)rintf(__fmul_rn(v[q], id)), d);
-}
-__device__ __forceinline__ float q8_block_value(float v) {
-    float amax = fabsf(v);
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, PI_WAVE));
-    float one[1] = {v};
-    q8_block_values(one, amax);
-    return one[0];
-}
-
-// Token t, column i of tokens in the operand layout, 16 by 16
-__device__ __forceinline__ size_t ol_index_of(int t, int i, int cols) { return (size_t)(t >> 4) * 16 * cols + pi_ol_index(t & 15, i); }
-
 // q8 != 0 (cols % 32 == 0, cols <= 8192): the normalised row goes through Q8_0 blocks of 32 before the fp16 rounding, which is what
 // a Q4_0 mat-mul of the CPU path multiplies with (ggml_vec_dot_q4_0_q8_0, ggml-quants.c:2512-2650)
 // ol bit 0: out in the operand layout of the 16-token mat-muls, 16 tokens by 16 (pi_ol_index), instead of [token][cols]; bit 1: out_plain
