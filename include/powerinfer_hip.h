@@ -814,6 +814,11 @@ PI_API int pi_k_route(const float * z, int T, int n_expert, int n_top, int n_gro
                       pi_stream_t stream);
 /* the experts with the largest sigmoid scores, their weights the scores themselves */
 PI_API int pi_k_route_scores(const float * z, int T, int n_expert, int n_top, int32_t * ids, float * weights, pi_stream_t stream);
+/* The choice of pi_k_route (bias NULL: of pi_k_route_scores) with the router's product ahead of it (BF16, [n_expert][cols] and [T][cols]), for more than 16 tokens.  parts:
+ * scratch of pi_k_router_parts(T, n_expert, cols) * T * n_expert floats (0: sizes that are not supported). */
+PI_API int pi_k_router_parts(int T, int n_expert, int cols);
+PI_API int pi_k_route_long(const void * router, int n_expert, int cols, const void * x, int T, float * parts, int n_top, int n_group, int n_keep, const float * bias,
+                           int32_t * ids, float * weights, pi_stream_t stream);
 /* pairs (token, choice) in expert order: off [n_expert + 1], perm[place] = pair, inv[pair] = place.  tiles (optional): {expert, first
  * place} of every group of up to tile_n pairs of one expert; *n_tiles of them, at most n_pairs / tile_n + n_expert */
 PI_API int pi_k_moe_sort(const int32_t * ids, int n_pairs, int n_expert, int32_t * off, int32_t * perm, int32_t * inv, int tile_n, int32_t * tiles,

@@ -875,11 +875,25 @@ int experts(pi_model * m, Layer & L, const void * h, const Step & in) {
     return grouped(s, w, tile_n, st);
 }
 
+// a long pass's choice with its product, its parts where the mixer's joint projection was (1: done, 0: not of these sizes)
+int route_long(pi_model * m, Layer & L, int T, int n_group, int n_keep, const float * bias) {
+    LayerState * s = m->lay;
+    const pi_layer_desc & d = L.d;
+    const int parts = bf16_mode(s) ? pi_k_router_parts(T, d.n_expert, s->d_ld) : 0;
+    if (!parts || parts * d.n_expert > L.z_rows) return 0;
+    PI_TRY(pi_k_route_long(L.router, d.n_expert, s->d_ld, s->h_b, T, s->z, d.n_top, n_group, n_keep, bias, s->ids, s->wts, m->stream));
+    return 1;
+}
+
 int ffn_moe(pi_model * m, Layer & L, const Step & in) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
-    PI_TRY(dense(m, L.router, d.n_expert, s->d_ld, s->h_b, in.T, s->rl));
-    PI_TRY(pi_k_route(s->rl, in.T, d.n_expert, d.n_top, d.n_group, d.n_group_keep, L.bias, s->ids, s->wts, m->stream));
+    const int done = route_long(m, L, in.T, d.n_group, d.n_group_keep, L.bias);
+    if (done < 0) return done;
+    if (!done) {
+        PI_TRY(dense(m, L.router, d.n_expert, s->d_ld, s->h_b, in.T, s->rl));
+        PI_TRY(pi_k_route(s->rl, in.T, d.n_expert, d.n_top, d.n_group, d.n_group_keep, L.bias, s->ids, s->wts, m->stream));
+    }
     return experts(m, L, s->h_b, in);
 }
 
@@ -1175,8 +1189,12 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
     } else {
         PI_TRY(pi_k_sum_norm(type, &n, st));
         if (!moe) return PI_OK;
-        PI_TRY(product(L.router, d.n_expert, s->h_b, s->rl));
-        PI_TRY(pi_k_route_scores(s->rl, T, d.n_expert, d.n_top, s->ids, s->wts, st));
+        const int done = step ? 0 : route_long(m, L, T, 1, 1, nullptr);
+        if (done < 0) return done;
+        if (!done) {
+            PI_TRY(product(L.router, d.n_expert, s->h_b, s->rl));
+            PI_TRY(pi_k_route_scores(s->rl, T, d.n_expert, d.n_top, s->ids, s->wts, st));
+        }
     }
     n.w = L.norm_b_after; n.w_next = nullptr; n.h = nullptr; n.keep = keep;
     if (step) {

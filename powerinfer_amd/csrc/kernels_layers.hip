@@ -19,26 +19,46 @@ template <typename LD> __device__ float row_rms_scale(int cols, float eps, doubl
     return pi_inv_sqrt((float)(s / cols) + eps);
 }
 
+// eight columns a thread at a time, up to 8192 of them in the registers of 256 threads (rows on 16 bytes): a value a thread, 2 bytes of a row and 1024 threads took
+// 2048 tokens of 4096 columns 32 us, this 12
 __device__ void embed_norm_row(const uint16_t * __restrict__ row, int cols, const float * __restrict__ w, float eps, float * __restrict__ out, double * red) {
-    if (cols <= 8 * (int)blockDim.x) {              // row and weights requested together, kept in registers
-        float v[8], wv[8];
+    constexpr int N = 4;
+    if (cols % 8 == 0 && cols <= N * 8 * (int)blockDim.x && (((uintptr_t)row | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
+        pi_u32x4 r[N];
+        float4 wv[N][2];
         double s = 0.0;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int i = threadIdx.x + k * blockDim.x;
-            v[k] = i < cols ? bf16_to_f32(row[i]) : 0.0f;
-            wv[k] = i < cols ? w[i] : 0.0f;
-            s += (double)v[k] * (double)v[k];
+        for (int k = 0; k < N; ++k) {
+            const int i = ((int)threadIdx.x + k * (int)blockDim.x) * 8;
+            r[k] = pi_u32x4{0, 0, 0, 0};
+            if (i < cols) { r[k] = pi_ld16(row + i); wv[k][0] = *reinterpret_cast<const float4 *>(w + i); wv[k][1] = *reinterpret_cast<const float4 *>(w + i + 4); }
         }
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float lo = __uint_as_float(r[k][j] << 16), hi = __uint_as_float(r[k][j] & 0xffff0000u);
+                s += (double)lo * (double)lo + (double)hi * (double)hi;
+            }
         s = block_sum_f64(s, red);
         const float sc = pi_inv_sqrt((float)(s / cols) + eps);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) { const int i = threadIdx.x + k * blockDim.x; if (i < cols) out[i] = v[k] * sc * wv[k]; }
+        for (int k = 0; k < N; ++k) {
+            const int i = ((int)threadIdx.x + k * (int)blockDim.x) * 8;
+            if (i >= cols) break;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4 g = wv[k][h];
+                const float v[4] = {__uint_as_float(r[k][2 * h] << 16), __uint_as_float(r[k][2 * h] & 0xffff0000u), __uint_as_float(r[k][2 * h + 1] << 16), __uint_as_float(r[k][2 * h + 1] & 0xffff0000u)};
+                *reinterpret_cast<float4 *>(out + i + 4 * h) = make_float4(v[0] * sc * g.x, v[1] * sc * g.y, v[2] * sc * g.z, v[3] * sc * g.w);
+            }
+        }
         return;
     }
     const float sc = row_rms_scale(cols, eps, red, [&](int i) { return bf16_to_f32(row[i]); });
     for (int i = threadIdx.x; i < cols; i += blockDim.x) out[i] = bf16_to_f32(row[i]) * sc * w[i];
 }
+inline int embed_norm_block(int cols) { return cols % 8 == 0 && cols <= 8192 ? 256 : cols > 2048 ? 1024 : 256; }
 __global__ __launch_bounds__(1024) void embed_norm_kernel(const uint16_t * __restrict__ table, int cols, const int32_t * __restrict__ tokens,
                                                           const float * __restrict__ w, float eps, float * __restrict__ x) {
     __shared__ double red[16];
@@ -80,6 +100,43 @@ __global__ __launch_bounds__(1024) void norm_pair_kernel(const float * __restric
         const float v = xt[i] * sc;
         out_a[at(i)] = to_st<ST>(v * wa[i]);
         if (wb) out_b[at(i)] = to_st<ST>(v * wb[i]);
+    }
+}
+
+// the same with four columns a thread at a time, up to 4096 of them in the registers of 256 threads (rows, weights and outputs in whole quads): 2048 tokens of 4096
+// columns into two operands 22.8 -> 12.6 us.  For long passes: 16 waves a row are the better ones for a few (one token 4.8 us, this 5.1)
+template <typename ST>
+__global__ __launch_bounds__(256) void norm_pair_quads_kernel(const float * __restrict__ x, const int32_t * __restrict__ rows, int cols, float eps, const float * __restrict__ wa,
+                                                             ST * __restrict__ out_a, const float * __restrict__ wb, ST * __restrict__ out_b, int ld) {
+    constexpr int N = 4;
+    __shared__ double red[4];
+    const float * xt = x + (size_t)(rows ? rows[blockIdx.x] : blockIdx.x) * cols;
+    float4 xv[N], av[N], bv[N];
+    const int last = cols - 4;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int i = min(((int)threadIdx.x + k * 256) * 4, last);
+        xv[k] = *reinterpret_cast<const float4 *>(xt + i);
+        av[k] = *reinterpret_cast<const float4 *>(wa + i);
+        if (wb) bv[k] = *reinterpret_cast<const float4 *>(wb + i);
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        if (((int)threadIdx.x + k * 256) * 4 < cols) s += ((double)xv[k].x * (double)xv[k].x + (double)xv[k].y * (double)xv[k].y) + ((double)xv[k].z * (double)xv[k].z + (double)xv[k].w * (double)xv[k].w);
+    s = block_sum_f64(s, red);
+    const float sc = pi_inv_sqrt((float)(s / cols) + eps);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int i = ((int)threadIdx.x + k * 256) * 4;
+        if (i >= cols) break;
+        const size_t at = (size_t)blockIdx.x * ld + i;
+        const float a[4] = {xv[k].x * sc * av[k].x, xv[k].y * sc * av[k].y, xv[k].z * sc * av[k].z, xv[k].w * sc * av[k].w};
+        store4(out_a + at, a, true, 4);
+        if (wb) {
+            const float b[4] = {xv[k].x * sc * bv[k].x, xv[k].y * sc * bv[k].y, xv[k].z * sc * bv[k].z, xv[k].w * sc * bv[k].w};
+            store4(out_b + at, b, true, 4);
+        }
     }
 }
 
@@ -360,6 +417,43 @@ __global__ __launch_bounds__(1024) void pass_start_kernel(pi::PassStart p, Bigra
             return;
         }
         b -= n;
+    }
+}
+
+// The router's products of a long pass: 64 tokens and 512 columns a workgroup, whose sums go apart to the choice behind them, which adds them up.  As tiles of 64 rows
+// and 64 tokens over all columns they were one row of tiles, all on one of the eight XCDs, each reading 1 MB: 2048 tokens of 4096 columns, 64 experts
+// 25.3 -> 10.3 us (and 1.6 more for the choice).  Bound by the 128 KB that a unit reads: the experts' columns go through LDS (read by each wave for itself 15.4 us), a wave holds its 16
+// tokens' values.
+constexpr int kRouterCols = 512, kRouterExperts = 128, kRouterPitch = kRouterCols * 2 + 16;      // (16 bytes on: sixteen rows' pieces in different banks)
+__global__ __launch_bounds__(256) void router_parts_kernel(const bf16 * __restrict__ W, int E, int cols, const bf16 * __restrict__ x, int T, float * __restrict__ parts) {
+    extern __shared__ __align__(16) unsigned char smem[];           // [E rounded up to 16][kRouterPitch]
+    constexpr int N = kRouterCols / 32, ROWS = 16;                  // rows a wave requests together
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4, k0 = (int)blockIdx.y * kRouterCols, tok = (int)blockIdx.x * 64 + wave * 16 + i;
+    const int n_m = (E + 15) / 16;
+    pi_u32x4 b[N], w[ROWS];
+    const bf16 * xt = x + (size_t)min(tok, T - 1) * cols + k0 + g * 8;
+    for (int r0 = wave; r0 < n_m * 16; r0 += 4 * ROWS) {
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k) w[k] = pi_ld16(W + (size_t)min(r0 + 4 * k, E - 1) * cols + k0 + lane * 8);
+        if (r0 == wave) {
+#pragma unroll
+            for (int k = 0; k < N; ++k) b[k] = pi_ld16(xt + k * 32);
+        }
+#pragma unroll
+        for (int k = 0; k < ROWS; ++k)
+            if (r0 + 4 * k < n_m * 16) *reinterpret_cast<pi_u32x4 *>(smem + (size_t)(r0 + 4 * k) * kRouterPitch + lane * 16) = w[k];
+    }
+    __syncthreads();
+    float * out = parts + ((size_t)blockIdx.y * T + tok) * E;
+    for (int m = 0; m < n_m; ++m) {
+        pi_f4 acc[2] = {};
+        const unsigned char * p = smem + (size_t)(m * 16 + i) * kRouterPitch + g * 16;
+#pragma unroll
+        for (int k = 0; k < N; ++k) acc[k & 1] = mma16<__bf16>(*reinterpret_cast<const pi_u32x4 *>(p + k * 64), b[k], acc[k & 1]);
+        if (tok >= T) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (m * 16 + 4 * g + r < E) out[m * 16 + 4 * g + r] = acc[0][r] + acc[1][r];
     }
 }
 
@@ -670,7 +764,7 @@ __global__ void cells_advance_kernel(int T, const int32_t * __restrict__ seq, co
 
 namespace pi {
 int pass_start(const PassStart & p, hipStream_t st) {
-    const int nt = p.norm && p.cols > 2048 ? 1024 : 256;
+    const int nt = p.norm ? embed_norm_block(p.cols) : 256;
     const auto blocks = [&](size_t n) { return (int)((n + nt - 1) / nt); };
     const int embeds = p.table ? p.T : 0, copies = blocks((p.words + 3) / 4), appends = blocks((size_t)p.n_append);
     int rots = 0;
@@ -686,7 +780,7 @@ extern "C" {
 
 int pi_k_embed_norm(const void * table, int cols, const int32_t * tokens, int T, const float * w, float eps, float * x, pi_stream_t stream) {
     if (!table || !tokens || !w || !x || cols <= 0 || T <= 0) return pi::fail(PI_E_ARG, "pi_k_embed_norm: bad arguments");
-    hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(cols > 2048 ? 1024 : 256), 0, (hipStream_t)stream, (const uint16_t *)table, cols, tokens, w, eps, x);
+    hipLaunchKernelGGL(embed_norm_kernel, dim3(T), dim3(embed_norm_block(cols)), 0, (hipStream_t)stream, (const uint16_t *)table, cols, tokens, w, eps, x);
     return pi::check_launch("pi_k_embed_norm");
 }
 
@@ -733,6 +827,11 @@ int pi_k_norm_pair(int type, const float * x, const int32_t * rows, int T, int c
                    const float * wb, void * out_b, int ld, int ol, pi_stream_t stream) {
     if (!x || !wa || !out_a || (wb && !out_b) || T <= 0 || cols <= 0 || ld < cols) return pi::fail(PI_E_ARG, "pi_k_norm_pair: bad arguments");
     if (ol && (type != PI_TYPE_BF16 || T > kBtMaxT || ld % 8)) return pi::fail(PI_E_ARG, "pi_k_norm_pair: operand layout needs BF16, T <= 16, ld % 8 == 0");
+    if (T > kBtMaxT && cols % 4 == 0 && cols <= 4096 && ld % 4 == 0 && (((uintptr_t)x | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)out_a | (uintptr_t)out_b) & 15) == 0 && (type == PI_TYPE_BF16 || type == PI_TYPE_F32)) {
+        if (type == PI_TYPE_BF16) hipLaunchKernelGGL(norm_pair_quads_kernel<bf16>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, rows, cols, eps, wa, (bf16 *)out_a, wb, (bf16 *)out_b, ld);
+        else hipLaunchKernelGGL(norm_pair_quads_kernel<float>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, rows, cols, eps, wa, (float *)out_a, wb, (float *)out_b, ld);
+        return pi::check_launch("pi_k_norm_pair");
+    }
     const int block = cols > 2048 ? 1024 : cols > 512 ? 512 : 256;
     if (type == PI_TYPE_BF16)
         hipLaunchKernelGGL(norm_pair_kernel<bf16>, dim3(T), dim3(block), 0, (hipStream_t)stream, x, rows, cols, eps, wa, (bf16 *)out_a, wb, (bf16 *)out_b, ld, ol);
@@ -764,6 +863,27 @@ int pi_k_rope_angles_table(const int32_t * pos, int T, int dims, const double * 
     if (!pos || !cs || !freq || T <= 0 || dims <= 0 || dims % 2) return pi::fail(PI_E_ARG, "pi_k_rope_angles_table: bad arguments");
     hipLaunchKernelGGL(rope_table_kernel, dim3((T * (dims / 2) + 63) / 64), dim3(64), 0, (hipStream_t)stream, pos, T, dims / 2, freq, length, (float2 *)cs);
     return pi::check_launch("pi_k_rope_angles_table");
+}
+
+int pi_k_router_parts(int T, int n_expert, int cols) {
+    return T > kBtMaxT && n_expert > 0 && n_expert <= kRouterExperts && cols > 0 && cols % kRouterCols == 0 && cols / kRouterCols <= 65535 ? cols / kRouterCols : 0;
+}
+
+int pi_k_route_long(const void * router, int n_expert, int cols, const void * x, int T, float * parts, int n_top, int n_group, int n_keep, const float * bias, int32_t * ids, float * weights,
+                    pi_stream_t stream) {
+    const int n = pi_k_router_parts(T, n_expert, cols);
+    if (!n) return pi::fail(PI_E_UNSUPPORTED, "pi_k_route_long: more than 16 tokens, up to 128 experts, columns in 512s");
+    if (!router || !x || !parts || !ids || !weights || (((uintptr_t)router | (uintptr_t)x) & 15) || n_top <= 0 || n_group <= 0 || n_expert % n_group || n_keep <= 0 || n_keep > n_group ||
+        n_top > n_keep * (n_expert / n_group) || (!bias && n_group != 1))
+        return pi::fail(PI_E_ARG, "pi_k_route_long: bad arguments");
+    const size_t lds = (size_t)(n_expert + 15) / 16 * 16 * kRouterPitch;
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&router_parts_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kRouterExperts * kRouterPitch);
+    if (raised != hipSuccess) return pi::hip_fail(raised, "pi_k_route_long: LDS size");
+    hipLaunchKernelGGL(router_parts_kernel, dim3((T + 63) / 64, n), dim3(256), lds, (hipStream_t)stream, (const bf16 *)router, n_expert, cols, (const bf16 *)x, T, parts);
+    RouteArgs r{parts, n_expert, n_top, n_group, n_keep, bias, ids, weights};
+    r.raw = !bias; r.parts = n; r.part_ld = (size_t)T * n_expert;
+    hipLaunchKernelGGL(route_kernel, dim3(T), dim3(n_expert > 64 ? 128 : 64), route_lds_bytes(n_expert, n_group, n_top), (hipStream_t)stream, r);
+    return pi::check_launch("pi_k_route_long");
 }
 
 int pi_k_route_scores(const float * z, int T, int n_expert, int n_top, int32_t * ids, float * weights, pi_stream_t stream) {

@@ -6,8 +6,8 @@ namespace {
 
 // soft: the experts with the largest logits, their weights the soft-max over them; else sigmoid scores, a bias on the choice (optional) and groups,
 // weights over their sum or (raw) as they are.
-// ldz: values between the tokens' rows of z (0: E)
-struct RouteArgs { const float * z; int E, top, G, keep; const float * bias; int32_t * ids; float * weights; int ldz = 0; bool soft = false, raw = false; };
+// ldz: values between the tokens' rows of z (0: E); parts: z is the sum of so many arrays, part_ld values apart
+struct RouteArgs { const float * z; int E, top, G, keep; const float * bias; int32_t * ids; float * weights; int ldz = 0; bool soft = false, raw = false; int parts = 1; size_t part_ld = 0; };
 
 __host__ __device__ inline size_t route_lds_bytes(int E, int G, int top) { return sizeof(float) * (size_t)(2 * ((E + 3) / 4 * 4) + (G > top ? G : top)); }
 
@@ -20,7 +20,10 @@ __device__ void route_token(const RouteArgs & r, int t, float * sm) {
     for (int e = tid; e < E4; e += nt) {
         float s = 0.0f, c = -INFINITY;
         if (e < E) {
-            s = r.soft ? z[e] : 1.0f / (1.0f + expf(-z[e]));
+            float v = z[e];
+#pragma unroll 8
+            for (int k = 1; k < r.parts; ++k) v += z[k * r.part_ld + e];
+            s = r.soft ? v : 1.0f / (1.0f + expf(-v));
             c = r.soft || !r.bias ? s : s + r.bias[e];
             if (!(c == c)) c = -INFINITY;                      // not a number: never chosen over a number
         }

@@ -286,6 +286,8 @@ _SIGS = {
     "pi_k_gqa_talk": (_i, [C.POINTER(GqaAttn), C.POINTER(GqaMix), _vp, _vp, _i, _vp]),
     "pi_k_rope_angles_table": (_i, [_vp, _i, _i, _vp, C.c_double, _vp, _vp]),
     "pi_k_route_scores": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp]),
+    "pi_k_router_parts": (_i, [_i, _i, _i]),
+    "pi_k_route_long": (_i, [_vp, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "pi_k_expert_up_step": (_i, [_vp, _i, _i, _i, _f, _f, _i, _i, _vp, _i, _vp, _vp, _i, _vp, _i, _vp]),
     "pi_k_sum_norm": (_i, [_i, C.POINTER(SumNorm), _vp]),
     "pi_k_sum_norm_route_supported": (_i, [_i, _i, _i, _i]),
