@@ -879,6 +879,9 @@ typedef struct pi_conv_norm {
 } pi_conv_norm;
 PI_API int pi_k_conv_norm(int type, const pi_conv_norm * p, pi_stream_t stream);
 PI_API int pi_k_conv_tokens(int T, int taps);                                 /* tokens of an item of a step of T tokens */
+/* The sum of pi_k_sum_norm (mix, without h) and the norm and convolution of its result in one launch, for items that are whole runs. */
+PI_API int pi_k_sum_conv_supported(int cols, int groups, int taps, int ld, size_t slot_ld);
+PI_API int pi_k_sum_conv(int type, const pi_sum_norm * sum, const pi_conv_norm * conv, pi_stream_t stream);
 /* What closes a sublayer whose norm comes after the sum: s = alpha x[t] + g * mix[t] with g = sigmoid(gate_z[t][off_gate ..] + gate_b) (gate_z NULL: 1),
  * or s = x[t] (mix NULL); out[t] = rms_norm(s) * w (w NULL: s); h (optional): the same as the next product's operand, rows of ld values or
  * (ol, BF16, T <= 16) in the operand layout of pi_k_gemm_bf16_ol; keep (optional) receives a copy.  out may be x. */

@@ -125,6 +125,7 @@ struct Step {
     const int32_t *lin = nullptr, *lin_long = nullptr, *lin_first = nullptr, *lin_chunks = nullptr;
     int n_lin = 0, n_lin_long = 0, n_lin_chunks = 0;
     const int32_t * conv = nullptr; int n_conv = 0;    // items of the convolutions
+    bool conv_whole = false;                           // each of them is a whole run
     // the tokens whose logits are wanted, in this order (-1: not said, every token's stream is)
     const int32_t * rows = nullptr; int n_rows = -1;
     // (latent attention) the last layer has no cells of its own: these tokens as a step, which is then all that is run of it
@@ -159,6 +160,7 @@ struct LayerState {
     // step buffers for `cap` tokens (one allocation)
     int cap = 0;
     unsigned char * arena = nullptr;
+    pi_sum_norm last_sum{}; bool sum_left = false;     // the sum that closes a layer, left to the next one's first launch
     float * route_sums = nullptr; uint32_t * route_arrived = nullptr;      // of norms and expert choices in one launch
     float *x = nullptr, *x2 = nullptr, *x0 = nullptr, *z = nullptr, *mix = nullptr, *rl = nullptr, *wts = nullptr, *lin_o = nullptr, *lin_den = nullptr, *lin_gates = nullptr;
     void *lin_q = nullptr, *lin_k = nullptr, *lin_v = nullptr, *lin_states = nullptr;
@@ -1129,7 +1131,8 @@ int post_norm_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in
 
 // A layer with norms before and after its sublayers.  Steps of up to 16 tokens (bf16) stream the weights past operands in the matrix cores' layout; the
 // sum that closes a sublayer, the norm ahead of the feed-forward and the expert choice behind it are one launch, the norm ahead of the mixer and its convolution another.
-int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in, float * keep) {
+// next: the layer behind it, whose norm and convolution can take this one's last sum along (steps whose runs are single items)
+int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & in, float * keep, const Layer * next) {
     LayerState * s = m->lay;
     const pi_layer_desc & d = L.d;
     int T = in.T;
@@ -1141,7 +1144,9 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
         pi_conv_norm c{};
         c.x = s->x; c.w = L.norm_a; c.taps_w = L.conv; c.T = T; c.cols = D; c.groups = s->opts.norm_groups; c.taps = s->opts.conv_taps; c.eps = m->hp.norm_eps;
         c.state = L.conv_floats ? L.state[r.pass] + L.rec_floats() : nullptr; c.slot_ld = L.state_floats(); c.items = in.conv; c.n_items = in.n_conv; c.h = s->h_a; c.ld = s->d_ld; c.ol = step;
-        PI_TRY(pi_k_conv_norm(type, &c, st));
+        if (s->sum_left) PI_TRY(pi_k_sum_conv(type, &s->last_sum, &c, st));
+        else PI_TRY(pi_k_conv_norm(type, &c, st));
+        s->sum_left = false;
     } else {
         pi_sum_norm n{};
         n.x = s->x; n.w_next = L.norm_a; n.T = T; n.cols = D; n.groups = s->opts.norm_groups; n.eps = m->hp.norm_eps; n.h = s->h_a; n.ld = s->d_ld; n.ol = step;
@@ -1184,11 +1189,18 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
     n.x = s->x; n.mix = s->mix; n.w = L.norm_a_after; n.mult = s->opts.residual_mult; n.T = T; n.cols = D; n.groups = s->opts.norm_groups; n.eps = m->hp.norm_eps;
     n.ld = s->d_ld; n.ol = step;
     if (moe) { n.h = s->h_b; n.w_next = L.norm_b; } else n.keep = keep;
-    if (moe && step && bf16_mode(s) && pi_k_sum_norm_route_supported(T, D, n.groups, d.n_expert)) {
+    const bool leave = step && in.conv_whole && next && next->conv && pi_k_sum_conv_supported(D, n.groups, s->opts.conv_taps, s->d_ld, next->state_floats());
+    const auto last = [&]() -> int {
+        if (!leave || !n.mix) return pi_k_sum_norm(type, &n, st);
+        s->last_sum = n;
+        s->sum_left = true;
+        return PI_OK;
+    };
+    if (!moe) return last();
+    if (step && bf16_mode(s) && pi_k_sum_norm_route_supported(T, D, n.groups, d.n_expert)) {
         PI_TRY(pi_k_sum_norm_route(&n, L.router, s->d_ld, d.n_expert, d.n_top, s->ids, s->wts, s->route_sums, s->route_arrived, st));
     } else {
         PI_TRY(pi_k_sum_norm(type, &n, st));
-        if (!moe) return PI_OK;
         const int done = step ? 0 : route_long(m, L, T, 1, 1, nullptr);
         if (done < 0) return done;
         if (!done) {
@@ -1205,7 +1217,7 @@ int both_norms_layer(pi_model * m, Layer & L, const LayerRun & r, const Step & i
         PI_TRY(experts(m, L, s->h_b, in));
         n.mix = nullptr; n.y = s->y_exp; n.inv = s->inv; n.top = d.n_top; n.y_w = d.weigh_input ? nullptr : s->wts;
     }
-    return pi_k_sum_norm(type, &n, st);
+    return last();
 }
 
 // a layer of a step of up to 16 tokens (bf16): six launches
@@ -1250,12 +1262,13 @@ int pass_layers(pi_model * m, const Step & in) {
         PI_TRY(pi_k_res_norm(type, &n, st));
     }
     for (size_t k = in.started ? pi::PassStart::kRots : 0; k < s->rots.size(); ++k) PI_TRY(rope_angles(m, (int)k, in.pos, T));
+    s->sum_left = false;
     for (size_t k = 0; k < s->order.size(); ++k) {
         Layer & L = s->layers[s->order[k].layer];
         const bool moe = L.moe();
         float * keep = s->streams_T ? s->streams + k * (size_t)s->streams_T * D : nullptr;
         if (s->family == kBothNorms) {
-            PI_TRY(both_norms_layer(m, L, s->order[k], in, keep));
+            PI_TRY(both_norms_layer(m, L, s->order[k], in, keep, k + 1 < s->order.size() ? &s->layers[s->order[k + 1].layer] : nullptr));
             continue;
         }
         if (s->family == kPostNorm) {
@@ -1818,6 +1831,8 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
                 a = b;
             }
             in.n_conv = (int)(items.size() - at_conv) / 8;
+            in.conv_whole = true;
+            for (size_t k = at_conv; k < items.size(); k += 8) in.conv_whole = in.conv_whole && items[k + 1] == items[k + 3];
         }
         const size_t at_lin = items.size();
         if (s->recurrent) {                                       // runs walked token by token, long runs, their first chunks, the chunks
@@ -2079,7 +2094,7 @@ int layers_generate(pi_model * m, int own, int n_steps, int32_t * out_tokens, fl
     if (s->opts.conv_taps > 0) {
         std::vector<int32_t> conv;
         for (int t = 0; t < T; ++t) { const int32_t item[8] = {t, 1, 0, 1, std::max(s->slot_of[q0 + t], 0), 0, 0, 0}; conv.insert(conv.end(), item, item + 8); }
-        in.conv = s->g_conv; in.n_conv = T;
+        in.conv = s->g_conv; in.n_conv = T; in.conv_whole = true;
         PI_TRY(pi_memcpy_h2d(s->g_conv, conv.data(), 4 * conv.size()));
     }
     in.prev = s->g_prev; in.carry = true;

@@ -293,6 +293,8 @@ _SIGS = {
     "pi_k_sum_norm_route_supported": (_i, [_i, _i, _i, _i]),
     "pi_k_sum_norm_route": (_i, [C.POINTER(SumNorm), _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),
     "pi_k_conv_norm": (_i, [_i, C.POINTER(ConvNorm), _vp]),
+    "pi_k_sum_conv_supported": (_i, [_i, _i, _i, _i, _sz]),
+    "pi_k_sum_conv": (_i, [_i, C.POINTER(SumNorm), C.POINTER(ConvNorm), _vp]),
     "pi_k_conv_tokens": (_i, [_i, _i]),
     "pi_k_linear_chunk": (_i, []),
     "pi_k_linear_supported": (_i, [_i, _i]),
