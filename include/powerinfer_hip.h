@@ -618,6 +618,11 @@ PI_API int pi_k_attn_decode_supported(int hd, int n_ctx);
 
 /* x[cols] = row *token of the embedding table (k_get_rows, ggml-cuda.cu:1664) */
 PI_API int pi_k_embed(int wtype, const void * table, int cols, const int32_t * token, float * x, pi_stream_t stream);
+/* y = W . norm(row of the embedding) in one launch, which also leaves the row in x [cols]; table and W: wtype.  The token lies in device memory, or is `id` at
+ * position pos with token null: the launch then writes d_token, d_pos and 0 to d_step.  _supported: 1 or 0 */
+PI_API int    pi_k_first_gemv_supported(int wtype, const void * table, const void * W, int rows, int cols, const pi_norm * norm, const float * x);
+PI_API int    pi_k_first_gemv(int wtype, const void * table, const int32_t * token, int32_t id, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, const void * W,
+                              int rows, int cols, const pi_norm * norm, float * x, float * y, pi_stream_t stream);
 
 /* greedy sampling: *token_out = index of the first maximum (llama_sample_token_greedy, llama.cpp:8617-8631) */
 PI_API int pi_k_argmax(const float * logits, int n, int32_t * token_out, pi_stream_t stream);

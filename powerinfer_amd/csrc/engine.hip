@@ -157,7 +157,25 @@ size_t ahead_rows(pi::Ahead & a, const Tensor & t, int rows_per_unit, int slot, 
     return bytes - n * unit;
 }
 
-int layer_forward(pi_model * m, int il, bool last_token) {
+// Falcon's FFN beside its attention, on a stream of its own
+bool ffn_beside(pi_model * m, int il) {
+    const pi_hparams & hp = m->hp;
+    const Tensor & up = m->L(il, PI_T_FFN_UP);
+    return hp.arch == PI_ARCH_FALCON && m->stream2 && !m->L(il, PI_T_GPU_BUCKET).dev && up.type != PI_TYPE_Q4_0 && !m->capture &&
+           pi_k_sparse_ffn_supported(hp.n_ff, (int)m->L(il, PI_T_FC1).ne1, hp.n_embd);
+}
+// norm in front of a layer's q|k|v
+pi_norm attn_norm(pi_model * m, int il) {
+    const float eps = m->hp.norm_eps;
+    if (m->hp.arch != PI_ARCH_FALCON) return make_norm(1, eps, m->L(il, PI_T_ATTN_NORM), nullptr);
+    if (m->L(il, PI_T_ATTN_NORM_2).dev) return make_norm(2, eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
+    return make_norm(2, eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
+}
+// the token that a pass starts with (id < 0: the one the device's state names)
+struct StartToken { int32_t id, pos; };
+
+// start: the layer forms its input itself, the embedding of this token (whole_start)
+int layer_forward(pi_model * m, int il, bool last_token, const StartToken * start) {
     const pi_hparams & hp = m->hp;
     const int d = hp.n_embd, ff = hp.n_ff, hd = m->hd, gqa = m->gqa;
     hipStream_t st = m->stream;
@@ -179,7 +197,7 @@ int layer_forward(pi_model * m, int il, bool last_token) {
     const bool layer_hybrid = bk != nullptr;
     float * x = m->x;
 
-    const bool branch = falcon && m->stream2 && !layer_hybrid && !q4 && !m->capture && pi_k_sparse_ffn_supported(ff, r, d);
+    const bool branch = ffn_beside(m, il);
     if (branch) {
         pi_norm fnb = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         PI_HIP_TRY(hipEventRecord(m->ev_fork[il], st));
@@ -201,11 +219,14 @@ int layer_forward(pi_model * m, int il, bool last_token) {
     }
 
     // attention
-    pi_norm an;
-    if (!falcon) an = make_norm(1, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), nullptr);
-    else if (m->L(il, PI_T_ATTN_NORM_2).dev) an = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
-    else an = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
-    PI_TRY(pi_k_gemv(wqkv.type, wqkv.dev, d + 2 * gqa, d, x, &an, PI_EPI_NONE, nullptr, nullptr, m->qkv, st));
+    const pi_norm an = attn_norm(m, il);
+    if (start) {
+        const Tensor & table = m->glob[PI_T_TOK_EMBD];
+        PI_TRY(pi_k_first_gemv(table.type, table.dev, start->id < 0 ? m->d_token : nullptr, start->id, start->pos, m->d_token, m->d_pos, m->d_step, wqkv.dev, d + 2 * gqa, d, &an, x,
+                              m->qkv, st));
+    } else {
+        PI_TRY(pi_k_gemv(wqkv.type, wqkv.dev, d + 2 * gqa, d, x, &an, PI_EPI_NONE, nullptr, nullptr, m->qkv, st));
+    }
     if (m->attn_parts > 1) {
         PI_TRY(pi_k_attn_split(m->qkv, 0, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, 0, 1, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0,
                                hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, 0, nullptr, st));
@@ -363,9 +384,14 @@ int token_forward(pi_model * m, bool want_logits, bool last_token, int32_t token
     // the host threads expect this token's hybrid layers (a graph under construction runs nothing: its replays are announced one by one)
     if (pi::cold_async(m->cold) && !m->capture && !m->building_graph) PI_TRY(pi::cold_post_token(m->cold));
     const Tensor & table = m->glob[PI_T_TOK_EMBD];
-    if (token < 0) PI_TRY(pi_k_embed(table.type, table.dev, hp.n_embd, m->d_token, m->x, st));
+    const Tensor & wqkv = m->L(0, PI_T_WQKV);
+    const pi_norm an = attn_norm(m, 0);
+    const StartToken start{token, pos};
+    const bool whole_start = table.type == wqkv.type && !ffn_beside(m, 0) && pi_k_first_gemv_supported(table.type, table.dev, wqkv.dev, hp.n_embd + 2 * m->gqa, hp.n_embd, &an, m->x);
+    if (whole_start) {}
+    else if (token < 0) PI_TRY(pi_k_embed(table.type, table.dev, hp.n_embd, m->d_token, m->x, st));
     else PI_TRY(pi::embed_start(table.type, table.dev, hp.n_embd, token, pos, m->d_token, m->d_pos, m->d_step, m->x, st));
-    for (int il = 0; il < hp.n_layer; ++il) PI_TRY(layer_forward(m, il, last_token));
+    for (int il = 0; il < hp.n_layer; ++il) PI_TRY(layer_forward(m, il, last_token, il == 0 && whole_start ? &start : nullptr));
     if (want_logits) {
         const bool falcon = hp.arch == PI_ARCH_FALCON;
         pi_norm on = make_norm(falcon ? 2 : 1, hp.norm_eps, m->glob[PI_T_OUTPUT_NORM], falcon ? &m->glob[PI_T_OUTPUT_NORM_B] : nullptr);

@@ -56,7 +56,8 @@ __device__ float block_max_f32(float v, float * red) {
 // RMSNorm as ggml.c:9238-9284 (double sum of fp32 squares, scale = 1/sqrtf(mean+eps), then * w as a
 // second fp32 multiply: llm_build_norm, llama.cpp:4420-4450); LayerNorm as ggml.c:9169-9236.
 // ---------------------------------------------------------------------------------------------------
-__device__ void stage_x_f16(__half * xs, const float * __restrict__ x, int cols, NormArgs na, double * red) {
+template <typename X>                                  // a pointer to floats, or what else yields x[i]
+__device__ void stage_x_f16(__half * xs, X x, int cols, NormArgs na, double * red) {
     float mean = 0.0f, scale = 1.0f;
     constexpr int kHeld = 4;
     if (cols <= kHeld * (int)blockDim.x) {

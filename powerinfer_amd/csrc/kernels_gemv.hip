@@ -15,6 +15,7 @@ namespace {
 // TAG only separates instantiations by role so that kernel traces can tell them apart.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kGemvBlocks = 512;
+constexpr int kFirstMostCols = 1024;   // widest vectors that stage_x_f16 holds in registers
 
 template <int RPW, int U, int TAG>
 __global__ __launch_bounds__(kBlock) void gemv_f16_kernel(const __half * __restrict__ W, const float * __restrict__ x, NormArgs na,
@@ -81,6 +82,37 @@ __global__ __launch_bounds__(kBlock) void gemv_f16_kernel(const __half * __restr
     }
 }
 
+// state: the token loop's state, written where the host names the token (embed_start); token is then null
+struct TokenStart { int32_t token, pos; int32_t * d_token, * d_pos, * d_step; };
+__device__ __forceinline__ int32_t start_token(const int32_t * token, const TokenStart & s) {
+    if (token) return __builtin_amdgcn_readfirstlane(*token);      // (in scalar registers, and no merge of the two reads through an address on the stack)
+    if (blockIdx.x == 0 && threadIdx.x == 0) { *s.d_token = s.token; *s.d_pos = s.pos; *s.d_step = 0; }
+    return s.token;
+}
+// The embedding row a mat-vec takes as its input: what a token begins with is no launch of its own where the first layer's q|k|v reads the row itself
+// and its first workgroup leaves it in fp32 for the residual (and the state, see TokenStart).
+struct EmbedRow { const void * table; const int32_t * token; TokenStart start; float * x; };
+__device__ __forceinline__ float q4_value(const pi_block_q4_0 * b, int j) {
+    uint16_t dbits; __builtin_memcpy(&dbits, &b->d, 2);
+    const int q = (j < 16) ? (b->qs[j] & 0x0F) : (b->qs[j - 16] >> 4);
+    return __fmul_rn((float)(q - 8), pi_f16_from_bits(dbits));
+}
+// eight columns from o on (a multiple of 8), stored by the first workgroup
+template <bool Q4>
+__device__ __forceinline__ void embed_eight(const EmbedRow & e, int32_t token, int cols, int o, float * v) {
+    if (Q4) {
+        const pi_block_q4_0 * b = (const pi_block_q4_0 *)e.table + (size_t)token * (cols / 32) + (o >> 5);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = q4_value(b, (o & 31) + k);
+    } else {
+        pi_unpack8(pi_ld16((const __half *)e.table + (size_t)token * cols + o), v);
+    }
+    if (blockIdx.x == 0) {
+        *reinterpret_cast<float4 *>(e.x + o) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4 *>(e.x + o + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    }
+}
+
 // Register-resident variant for cols == 512 * NCH (4096, 5120, 8192): a wave owns whole rows
 // (row = wave_id, wave_id + n_waves, ...), lane l holds the activations of columns 8*l + 512*j as packed fp16 in
 // registers, so the row loop touches neither LDS nor a workgroup barrier.  The prologue is shared by the four
@@ -92,11 +124,11 @@ __global__ __launch_bounds__(kBlock) void gemv_f16_kernel(const __half * __restr
 // MULTI: up to three matrices of the same width against the one vector in a single launch (the q, k and v projections of a host
 // that keeps them as separate tensors): row r of the launch is row r of the first matrix, or row r - rows[0] of the second, ...
 struct GemvMulti { const __half * W[3]; float * y[3]; int rows[3]; };
-template <int NCH, int KIND, bool MULTI>
+template <int NCH, int KIND, bool MULTI, bool FIRST = false>
 __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W, const float * __restrict__ x,
                                                   const float * __restrict__ nw, const float * __restrict__ nb, float eps,
                                                   int epi, const float * __restrict__ add1, const float * __restrict__ add2,
-                                                  float * __restrict__ y, int rows, const GemvMulti & mm) {
+                                                  float * __restrict__ y, int rows, const GemvMulti & mm, const EmbedRow & first = {}) {
     constexpr int cols = NCH * 512;
     auto row_base = [&](int r) -> const __half * {
         if (!MULTI) return W + (size_t)r * cols;
@@ -139,13 +171,17 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
     // ---- shared prologue ---------------------------------------------------------------------------------
     {
         float xv[MYCH][8], wv[MYCH][8], bv[MYCH][8];
+        const int32_t token = FIRST ? start_token(first.token, first.start) : 0;
 #pragma unroll
         for (int i = 0; i < MYCH; ++i) {
             const int j = wave + i * kWavesPerBlock;
             if (j < NCH) {
                 const int o = j * 512 + lane * 8;
-                const float4 a = *reinterpret_cast<const float4 *>(x + o), b = *reinterpret_cast<const float4 *>(x + o + 4);
-                xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w; xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+                if (FIRST) embed_eight<false>(first, token, cols, o, xv[i]);
+                else {
+                    const float4 a = *reinterpret_cast<const float4 *>(x + o), b = *reinterpret_cast<const float4 *>(x + o + 4);
+                    xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w; xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+                }
                 if (KIND >= 1) {
                     const float4 c = *reinterpret_cast<const float4 *>(nw + o), e = *reinterpret_cast<const float4 *>(nw + o + 4);
                     wv[i][0] = c.x; wv[i][1] = c.y; wv[i][2] = c.z; wv[i][3] = c.w; wv[i][4] = e.x; wv[i][5] = e.y; wv[i][6] = e.z; wv[i][7] = e.w;
@@ -259,6 +295,11 @@ __global__ __launch_bounds__(kBlock, 2) void gemv_f16_reg_kernel(const __half * 
     gemv_f16_reg_body<NCH, KIND, false>(W, x, nw, nb, eps, epi, add1, add2, y, rows, GemvMulti{});
 }
 template <int NCH, int KIND>
+__global__ __launch_bounds__(kBlock, 2) void gemv_f16_first_kernel(const __half * __restrict__ W, EmbedRow first, const float * __restrict__ nw, const float * __restrict__ nb, float eps,
+                                                                  float * __restrict__ y, int rows) {
+    gemv_f16_reg_body<NCH, KIND, false, true>(W, nullptr, nw, nb, eps, PI_EPI_NONE, nullptr, nullptr, y, rows, GemvMulti{}, first);
+}
+template <int NCH, int KIND>
 __global__ __launch_bounds__(kBlock, 2) void gemv_multi_f16_reg_kernel(GemvMulti mm, const float * __restrict__ x,
                                                                     const float * __restrict__ nw, const float * __restrict__ nb, float eps, int rows) {
     gemv_f16_reg_body<NCH, KIND, true>(nullptr, x, nw, nb, eps, PI_EPI_NONE, nullptr, nullptr, nullptr, rows, mm);
@@ -281,11 +322,11 @@ __global__ __launch_bounds__(kBlock, 2) void gemv_multi_f16_reg_kernel(GemvMulti
 // (copied by single words: 32000 x 4096 21.6).
 // ---------------------------------------------------------------------------------------------------
 constexpr int kQ4Threads = kBlock + PI_WAVE;
-template <int CB, int KIND, int TAG, bool OFF>
-__global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsigned char * __restrict__ W, const float * __restrict__ x,
-                                                             const float * __restrict__ nw, const float * __restrict__ nb, float eps,
-                                                             int epi, const float * __restrict__ add1, const float * __restrict__ add2,
-                                                             float * __restrict__ y, int rows) {
+template <int CB, int KIND, bool OFF, bool FIRST>
+__device__ __forceinline__ void gemv_q4_reg_body(const unsigned char * __restrict__ W, const float * __restrict__ x,
+                                                 const float * __restrict__ nw, const float * __restrict__ nb, float eps,
+                                                 int epi, const float * __restrict__ add1, const float * __restrict__ add2,
+                                                 float * __restrict__ y, int rows, const EmbedRow & first) {
     constexpr int cols = CB * 4096, NCH = cols / 512, nblk = cols / 32;
     constexpr int NBUF = CB == 1 ? 5 : 2;                          // steps in LDS
     constexpr int MYCH = NCH / kWavesPerBlock;
@@ -335,11 +376,15 @@ __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsign
     // ---- shared prologue: norm, Q8_0 quantisation -------------------------------------------------------------
     {
         float xv[MYCH][8], wv[MYCH][8], bv[MYCH][8];
+        const int32_t token = FIRST ? start_token(first.token, first.start) : 0;
 #pragma unroll
         for (int i = 0; i < MYCH; ++i) {
             const int o = (wave + i * kWavesPerBlock) * 512 + lane * 8;
-            const float4 a = *reinterpret_cast<const float4 *>(x + o), b = *reinterpret_cast<const float4 *>(x + o + 4);
-            xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w; xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+            if (FIRST) embed_eight<true>(first, token, cols, o, xv[i]);
+            else {
+                const float4 a = *reinterpret_cast<const float4 *>(x + o), b = *reinterpret_cast<const float4 *>(x + o + 4);
+                xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w; xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
+            }
             if (KIND >= 1) {
                 const float4 c = *reinterpret_cast<const float4 *>(nw + o), e = *reinterpret_cast<const float4 *>(nw + o + 4);
                 wv[i][0] = c.x; wv[i][1] = c.y; wv[i][2] = c.z; wv[i][3] = c.w; wv[i][4] = e.x; wv[i][5] = e.y; wv[i][6] = e.z; wv[i][7] = e.w;
@@ -463,12 +508,27 @@ __global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsign
     }
 }
 
+template <int CB, int KIND, int TAG, bool OFF>
+__global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_reg_kernel(const unsigned char * __restrict__ W, const float * __restrict__ x,
+                                                             const float * __restrict__ nw, const float * __restrict__ nb, float eps,
+                                                             int epi, const float * __restrict__ add1, const float * __restrict__ add2,
+                                                             float * __restrict__ y, int rows) {
+    gemv_q4_reg_body<CB, KIND, OFF, false>(W, x, nw, nb, eps, epi, add1, add2, y, rows, EmbedRow{});
+}
+template <int CB, int KIND, bool OFF>
+__global__ __launch_bounds__(kQ4Threads, 2) void gemv_q4_first_kernel(const unsigned char * __restrict__ W, EmbedRow first, const float * __restrict__ nw, const float * __restrict__ nb,
+                                                                     float eps, float * __restrict__ y, int rows) {
+    gemv_q4_reg_body<CB, KIND, OFF, true>(W, nullptr, nw, nb, eps, PI_EPI_NONE, nullptr, nullptr, y, rows, first);
+}
+
 // Any shape with cols % 8 == 0: one wave per row, grid-stride.  Short rows are bound by latency: the input's round trip and its norm, then
 // the row's.  The first row's first 2048 columns are therefore requested before the input is staged (clamped addresses: a load under a branch
 // of its own would be waited for before the next): with the input held in registers, 3.75 -> 3.35 us at 512 columns and 512..1536 rows.
-__global__ __launch_bounds__(kBlock) void gemv_f16_generic_kernel(const __half * __restrict__ W, const float * __restrict__ x, NormArgs na,
-                                                                  int epi, const float * add1, const float * add2,
-                                                                  float * __restrict__ y, int rows, int cols) {
+struct HalfRow { const __half * p; __device__ __forceinline__ float operator[](int i) const { return __half2float(p[i]); } };
+template <bool FIRST>
+__device__ __forceinline__ void gemv_f16_generic_body(const __half * __restrict__ W, const float * __restrict__ x, NormArgs na,
+                                                      int epi, const float * add1, const float * add2,
+                                                      float * __restrict__ y, int rows, int cols, const EmbedRow & embed) {
     extern __shared__ __align__(16) unsigned char smem[];
     __half * xs = reinterpret_cast<__half *>(smem);
     __shared__ double red[16];
@@ -479,7 +539,13 @@ __global__ __launch_bounds__(kBlock) void gemv_f16_generic_kernel(const __half *
     const __half * w0 = W + (size_t)min(r, rows - 1) * cols;
 #pragma unroll
     for (int u = 0; u < kFirst; ++u) first[u] = pi_ld_stream(w0 + min((u * PI_WAVE + lane) * 8, cols - 8));
-    stage_x_f16(xs, x, cols, na, red);
+    if (FIRST) {
+        const HalfRow row{(const __half *)embed.table + (size_t)start_token(embed.token, embed.start) * cols};
+        if (blockIdx.x == 0) for (int i = threadIdx.x; i < cols; i += kBlock) embed.x[i] = row[i];
+        stage_x_f16(xs, row, cols, na, red);
+    } else {
+        stage_x_f16(xs, x, cols, na, red);
+    }
     bool held = true;
     for (; r < rows; r += gridDim.x * kWavesPerBlock) {
         float acc = 0.0f;
@@ -503,6 +569,14 @@ __global__ __launch_bounds__(kBlock) void gemv_f16_generic_kernel(const __half *
         acc = pi_wave_sum(acc);
         if (lane == 0) y[r] = apply_epilogue(acc, epi, add1, add2, r);
     }
+}
+__global__ __launch_bounds__(kBlock) void gemv_f16_generic_kernel(const __half * __restrict__ W, const float * __restrict__ x, NormArgs na,
+                                                                  int epi, const float * add1, const float * add2,
+                                                                  float * __restrict__ y, int rows, int cols) {
+    gemv_f16_generic_body<false>(W, x, na, epi, add1, add2, y, rows, cols, EmbedRow{});
+}
+__global__ __launch_bounds__(kBlock) void gemv_f16_generic_first_kernel(const __half * __restrict__ W, EmbedRow first, NormArgs na, float * __restrict__ y, int rows, int cols) {
+    gemv_f16_generic_body<true>(W, nullptr, na, PI_EPI_NONE, nullptr, nullptr, y, rows, cols, first);
 }
 
 
@@ -540,13 +614,6 @@ __global__ __launch_bounds__(kBlock) void gemv_q4_kernel(const pi_block_q4_0 * _
     }
 }
 
-// state: the token loop's state, written where the host names the token (embed_start); token is then null
-struct TokenStart { int32_t token, pos; int32_t * d_token, * d_pos, * d_step; };
-__device__ __forceinline__ int32_t start_token(const int32_t * token, const TokenStart & s) {
-    if (token) return *token;
-    if (blockIdx.x == 0 && threadIdx.x == 0) { *s.d_token = s.token; *s.d_pos = s.pos; *s.d_step = 0; }
-    return s.token;
-}
 __global__ void embed_f16_kernel(const __half * __restrict__ table, int cols, const int32_t * __restrict__ token, float * __restrict__ x, TokenStart start) {
     const __half * row = table + (size_t)start_token(token, start) * cols;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cols; i += gridDim.x * blockDim.x) x[i] = __half2float(row[i]);
@@ -556,11 +623,7 @@ __global__ void embed_q4_kernel(const pi_block_q4_0 * __restrict__ table, int co
     const pi_block_q4_0 * row = table + (size_t)start_token(token ? token + blockIdx.y : nullptr, start) * (cols / 32);
     x += (size_t)blockIdx.y * cols;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < cols; i += gridDim.x * blockDim.x) {
-        const pi_block_q4_0 * b = row + (i >> 5);
-        uint16_t dbits; __builtin_memcpy(&dbits, &b->d, 2);
-        const int j = i & 31;
-        const int q = (j < 16) ? (b->qs[j] & 0x0F) : (b->qs[j - 16] >> 4);
-        x[i] = __fmul_rn((float)(q - 8), pi_f16_from_bits(dbits));
+        x[i] = q4_value(row + (i >> 5), i & 31);
     }
 }
 // Rows of a chunk's tokens, which travel as the kernel's arguments: copying 130 of them and their positions to the device and waiting for the copies took
@@ -834,6 +897,41 @@ static int embed_one(int wtype, const void * table, int cols, const int32_t * to
 int pi_k_embed(int wtype, const void * table, int cols, const int32_t * token, float * x, pi_stream_t stream) {
     if (!table || !token || !x || cols <= 0) return pi::fail(PI_E_ARG, "pi_k_embed: bad arguments");
     return embed_one(wtype, table, cols, token, TokenStart{}, x, (hipStream_t)stream);
+}
+
+// W . norm(row of the embedding), for the widths of the mat-vecs that hold their input in registers and for what the kernel for any F16 shape takes.  Not for
+// the others, whose input travels to LDS as it lies in memory.  A token's embedding launch was 2.1 to 2.9 us, and a gap, for a row that every
+// workgroup of the next launch could read as well.  Eight tokens of a call each, us: 7B F16 3995 -> 3961, 7B Q4_0
+// behind 2.8 k cells 3890 -> 3845; sixteen of three layers of 512 columns 1660 -> 1645.
+int pi_k_first_gemv_supported(int wtype, const void * table, const void * W, int rows, int cols, const pi_norm * norm, const float * x) {
+    const NormArgs na = to_norm(norm);
+    if (!table || !W || !x || rows <= 0 || cols <= 0 || (((uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b) & 15) || na.kind < 1 || na.kind > 2 || !na.w || (na.kind == 2) != (na.b != nullptr)) return 0;
+    if (wtype == PI_TYPE_Q4_0) return (cols == 4096 || cols == 8192) && !((uintptr_t)W & 3);
+    if (wtype != PI_TYPE_F16 || ((uintptr_t)table & 15) || cols % 8) return 0;
+    return cols == 4096 || cols == 5120 || cols == 8192 || cols <= kFirstMostCols;
+}
+int pi_k_first_gemv(int wtype, const void * table, const int32_t * token, int32_t id, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, const void * W, int rows, int cols,
+               const pi_norm * norm, float * x, float * y, pi_stream_t stream) {
+    if (!pi_k_first_gemv_supported(wtype, table, W, rows, cols, norm, x) || !y || (!token && (!d_token || !d_pos || !d_step))) return pi::fail(PI_E_ARG, "pi_k_first_gemv: bad arguments");
+    hipStream_t st = (hipStream_t)stream;
+    const NormArgs na = to_norm(norm);
+    const EmbedRow first{table, token, {id, pos, d_token, d_pos, d_step}, x};
+    const int full = (rows + kWavesPerBlock - 1) / kWavesPerBlock, blocks = std::min(full, kGemvBlocks);
+    const bool layer = na.kind == 2, off = ((uintptr_t)W & 15) != 0;
+#define PI_FIRST_F16(NCH, KIND) hipLaunchKernelGGL((gemv_f16_first_kernel<NCH, KIND>), dim3(blocks), dim3(kBlock), 0, st, (const __half *)W, first, na.w, na.b, na.eps, y, rows)
+#define PI_FIRST_Q4(CB, KIND, OFF) hipLaunchKernelGGL((gemv_q4_first_kernel<CB, KIND, OFF>), dim3(blocks), dim3(kQ4Threads), 0, st, (const unsigned char *)W, first, na.w, na.b, na.eps, y, rows)
+#define PI_FIRST_Q4_K(CB, KIND) do { if (off) PI_FIRST_Q4(CB, KIND, true); else PI_FIRST_Q4(CB, KIND, false); } while (0)
+    if (wtype == PI_TYPE_Q4_0) {
+        if (cols == 4096) { if (layer) PI_FIRST_Q4_K(1, 2); else PI_FIRST_Q4_K(1, 1); }
+        else { if (layer) PI_FIRST_Q4_K(2, 2); else PI_FIRST_Q4_K(2, 1); }
+    } else if (cols == 4096) { if (layer) PI_FIRST_F16(8, 2); else PI_FIRST_F16(8, 1); }
+    else if (cols == 5120) { if (layer) PI_FIRST_F16(10, 2); else PI_FIRST_F16(10, 1); }
+    else if (cols == 8192) { if (layer) PI_FIRST_F16(16, 2); else PI_FIRST_F16(16, 1); }
+    else hipLaunchKernelGGL(gemv_f16_generic_first_kernel, dim3(std::min(full, 2048)), dim3(kBlock), (size_t)cols * 2, st, (const __half *)W, first, na, y, rows, cols);
+#undef PI_FIRST_Q4_K
+#undef PI_FIRST_Q4
+#undef PI_FIRST_F16
+    return pi::check_launch("pi_k_first_gemv");
 }
 
 }  // extern "C"

@@ -246,6 +246,8 @@ _SIGS = {
     "pi_k_attn_decode_supported": (_i, [_i, _i]),
     "pi_k_attn_fused": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "pi_k_embed": (_i, [_i, _vp, _i, _vp, _vp, _vp]),
+    "pi_k_first_gemv_supported": (_i, [_i, _vp, _vp, _i, _i, C.POINTER(Norm), _vp]),
+    "pi_k_first_gemv": (_i, [_i, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _i, _i, C.POINTER(Norm), _vp, _vp, _vp]),
     "pi_k_argmax": (_i, [_vp, _i, _vp, _vp]),
     "pi_k_embed_norm": (_i, [_vp, _i, _vp, _i, _vp, _f, _vp, _vp]),
     "pi_k_norm_pair": (_i, [_i, _vp, _vp, _i, _i, _f, _vp, _vp, _vp, _vp, _i, _i, _vp]),
