@@ -1312,12 +1312,12 @@ __global__ __launch_bounds__(kBlock) void rope_kv_chunk_kernel(const float * __r
     }
 }
 
-// The same where rows and heads allow 16-byte accesses: eight values of a head at a time (neighbours, or four and the four they rotate with), six
-// such pieces of a thread requested before the angles are formed.  The loop above made a memory trip an iteration, two values in it: 2046 tokens,
-// 32 heads of 128 (167 MB in and out): 48 us, here 33 (what
-// a copy of as much takes).
+// The same where rows and heads allow 16-byte accesses: a thread has eight values of a head (neighbours, or four and the four they rotate with), requested
+// before the angles are formed, and a workgroup 256 such pieces of a token.  Bound by the trip there and back in short chunks, by the copy in long
+// ones (167 MB in and out of 2046 tokens).  The angles of a token are formed once a workgroup, which costs less than more pieces of a thread one after the other do: 32
+// heads of 128, a workgroup of a token (four up to 511 tokens, sixteen up to 127) with up to six pieces a thread in flight / this, us: 21 tokens 5.0 / 4.2, 130 6.6 / 5.7,
+// 300 8.3 / 7.0, 508 12.3 / 10.0; queries in fp16, 508 12.9 / 10.2, 999 15.6 / 15.9, 2046 29.4 / 28.4.
 // Q16: the rotated queries leave rounded to fp16, rows of n_head * hd of them (what attn_chunk_rows_once_kernel reads: half the bytes of both launches).
-constexpr int kRopeUn = 6;
 template <bool Q16>
 __global__ __launch_bounds__(kBlock) void rope_kv_chunk_wide_kernel(const float * __restrict__ qkv, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale,
                                                                      const int32_t * __restrict__ pos_p, int n_ctx, float * __restrict__ q_rot,
@@ -1329,51 +1329,35 @@ __global__ __launch_bounds__(kBlock) void rope_kv_chunk_wide_kernel(const float 
     float * qd = q_rot + (size_t)t * q_stride;
     const bool neox = (mode & 2) != 0;
     const int step = neox ? 4 : 8, second = neox ? half : 4;             // of a piece: where it starts in the head (times its number), where its second four are
-    bool have = false;
-    for (int e0 = blockIdx.y * kBlock + tid; e0 - tid < n; e0 += kRopeUn * gridDim.y * kBlock) {
-        float4 a[kRopeUn], b[kRopeUn];
+    const int e = min((int)blockIdx.y * kBlock + tid, n - 1), h = e / per, j = e % per;     // (past the end the last piece again, not stored)
+    const float4 a = *reinterpret_cast<const float4 *>(src + (size_t)h * hd + j * step), b = *reinterpret_cast<const float4 *>(src + (size_t)h * hd + j * step + second);
+    for (int k = tid; k < half; k += kBlock) {
+        const float theta = rope_angle((float)pos, k, mode, theta_scale, freq_scale);
+        cs[k] = make_float2(cosf(theta), sinf(theta));
+    }
+    __syncthreads();
+    if ((int)blockIdx.y * kBlock + tid >= n) return;
+    float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    if (h < n_head + n_head_kv) {
 #pragma unroll
-        for (int u = 0; u < kRopeUn; ++u) {
-            const int e = min(e0 + u * (int)gridDim.y * kBlock, n - 1);  // (past the end the last piece again, not stored)
-            const float * at = src + (size_t)(e / per) * hd + (e % per) * step;
-            a[u] = *reinterpret_cast<const float4 *>(at);
-            b[u] = *reinterpret_cast<const float4 *>(at + second);
+        for (int q = 0; q < 4; ++q) {
+            float & x0 = neox ? x[q] : x[2 * q], & x1 = neox ? x[q + 4] : x[2 * q + 1];
+            const float2 w = cs[4 * j + q];
+            const float y0 = __fsub_rn(__fmul_rn(x0, w.x), __fmul_rn(x1, w.y)), y1 = __fadd_rn(__fmul_rn(x0, w.y), __fmul_rn(x1, w.x));
+            x0 = y0; x1 = y1;
         }
-        if (!have) {
-            have = true;
-            for (int j = tid; j < half; j += kBlock) {
-                const float theta = rope_angle((float)pos, j, mode, theta_scale, freq_scale);
-                cs[j] = make_float2(cosf(theta), sinf(theta));
-            }
-            __syncthreads();
-        }
-#pragma unroll
-        for (int u = 0; u < kRopeUn; ++u) {
-            const int e = e0 + u * (int)gridDim.y * kBlock, h = e / per, j = e % per;
-            if (e >= n) break;
-            float x[8] = {a[u].x, a[u].y, a[u].z, a[u].w, b[u].x, b[u].y, b[u].z, b[u].w};
-            if (h < n_head + n_head_kv) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float & x0 = neox ? x[q] : x[2 * q], & x1 = neox ? x[q + 4] : x[2 * q + 1];
-                    const float2 w = cs[4 * j + q];
-                    const float y0 = __fsub_rn(__fmul_rn(x0, w.x), __fmul_rn(x1, w.y)), y1 = __fadd_rn(__fmul_rn(x0, w.y), __fmul_rn(x1, w.x));
-                    x0 = y0; x1 = y1;
-                }
-            }
-            if (!Q16 && h < n_head) {
-                float * dst = qd + (size_t)h * hd + j * step;
-                *reinterpret_cast<float4 *>(dst) = make_float4(x[0], x[1], x[2], x[3]);
-                *reinterpret_cast<float4 *>(dst + second) = make_float4(x[4], x[5], x[6], x[7]);
-            } else {
-                const int hk = h - n_head;
-                __half * dst = (h < n_head ? reinterpret_cast<__half *>(q_rot) + (size_t)t * q_stride + (size_t)h * hd
-                                : hk < n_head_kv ? k_cache + ((size_t)hk * n_ctx + pos) * hd : v_cache + ((size_t)(hk - n_head_kv) * n_ctx + pos) * hd) + j * step;
-                typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-                *reinterpret_cast<h4 *>(dst) = h4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
-                *reinterpret_cast<h4 *>(dst + second) = h4{(_Float16)x[4], (_Float16)x[5], (_Float16)x[6], (_Float16)x[7]};
-            }
-        }
+    }
+    if (!Q16 && h < n_head) {
+        float * dst = qd + (size_t)h * hd + j * step;
+        *reinterpret_cast<float4 *>(dst) = make_float4(x[0], x[1], x[2], x[3]);
+        *reinterpret_cast<float4 *>(dst + second) = make_float4(x[4], x[5], x[6], x[7]);
+    } else {
+        const int hk = h - n_head;
+        __half * dst = (h < n_head ? reinterpret_cast<__half *>(q_rot) + (size_t)t * q_stride + (size_t)h * hd
+                        : hk < n_head_kv ? k_cache + ((size_t)hk * n_ctx + pos) * hd : v_cache + ((size_t)(hk - n_head_kv) * n_ctx + pos) * hd) + j * step;
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<h4 *>(dst) = h4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+        *reinterpret_cast<h4 *>(dst + second) = h4{(_Float16)x[4], (_Float16)x[5], (_Float16)x[6], (_Float16)x[7]};
     }
 }
 
@@ -1566,16 +1550,16 @@ namespace pi {
 int rope_kv_chunk(const float * qkv, int qkv_stride, int T, int n_head, int n_head_kv, int hd, int mode, float theta_scale, float freq_scale, const int32_t * pos, int n_ctx,
                   float * q_rot, void * k_cache, void * v_cache, hipStream_t st, bool q16) {
     // 16 tokens and fewer: a workgroup per head and token (16 tokens, 32 heads of 128, attention included: 11.8 against 12.3 us); a chunk's angles
-    // are worth forming once a token from there on.  A workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
+    // are worth forming less often from there on.  Other rows: a workgroup per token fills the chip from 512 tokens; shorter chunks split its heads
     if (T <= kBtMaxT) {
         hipLaunchKernelGGL(rope_kv_store_kernel, dim3(n_head + 2 * n_head_kv, T), dim3(hd / 2), 0, st,
                            qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot, (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
         return pi::check_launch("rope_kv_store");
     }
-    const int split = T >= 512 ? 1 : T >= 128 ? 4 : 16;
     // 16-byte rows: heads of a multiple of eight values, and everything that starts on one
     const bool wide = hd % 8 == 0 && qkv_stride % 4 == 0 && (((uintptr_t)qkv | (uintptr_t)q_rot | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
     if (q16 && (!wide || T <= kBtMaxT)) return pi::fail(PI_E_ARG, "rope_kv_chunk: fp16 queries need rows of 16 bytes and more than 16 tokens");
+    const int split = wide ? ((n_head + 2 * n_head_kv) * (hd / 8) + kBlock - 1) / kBlock : T >= 512 ? 1 : T >= 128 ? 4 : 16;
     const auto kernel = q16 ? rope_kv_chunk_wide_kernel<true> : wide ? rope_kv_chunk_wide_kernel<false> : rope_kv_chunk_kernel;
     hipLaunchKernelGGL(kernel, dim3(T, split), dim3(kBlock), sizeof(float2) * (hd / 2), st, qkv, n_head, n_head_kv, hd, mode, theta_scale, freq_scale, pos, n_ctx, q_rot,
                        (__half *)k_cache, (__half *)v_cache, qkv_stride, n_head * hd);
