@@ -1413,10 +1413,15 @@ int choose_parts(LayerState * s, int n_work, int n_vis_max) {
 }
 
 // ---- cells -----------------------------------------------------------------------------------------------------------------------
-// the host's list of a sequence's cells, rebuilt after an edit; `app` receives what the device has to learn
+// the host's list of a sequence's cells, rebuilt after an edit; `app` receives what the device has to learn, (sequence, place, cell) with every place of a
+// sequence once: the kernels that store them do so in no order
 void refresh_list(LayerState * s, int q, std::vector<int32_t> & app) {
     if (!(s->kv.edited >> q & 1u)) return;
     s->kv.edited &= ~(1u << q);
+    size_t kept = 0;                                               // what app says of the sequence so far is its list before the edit
+    for (size_t k = 0; k < app.size(); k += 3)
+        if (app[k] != q) { std::copy_n(app.begin() + k, 3, app.begin() + kept); kept += 3; }
+    app.resize(kept);
     std::vector<std::pair<int32_t, int32_t>> v;
     for (int i = 0; i < s->kv.n; ++i) if (s->kv.pos[i] >= 0 && (s->kv.seq[i] >> q & 1u)) v.push_back({s->kv.pos[i], i});
     std::sort(v.begin(), v.end());

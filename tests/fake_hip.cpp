@@ -17,6 +17,7 @@ std::map<void *, size_t> live;
 size_t live_bytes = 0, peak_bytes = 0, limit_bytes = ~(size_t)0;
 int n_launch = 0, fail_at = -1, grid_x = 0;
 hipError_t last = hipSuccess;
+void (*watcher)(const char *, void **) = nullptr;
 char some[64];
 template <typename T> hipError_t give(T * p) { *p = (T)some; return hipSuccess; }
 }  // namespace
@@ -24,6 +25,7 @@ template <typename T> hipError_t give(T * p) { *p = (T)some; return hipSuccess; 
 extern "C" {
 void fake_fail_launch(int k) { n_launch = 0; fail_at = k; last = hipSuccess; }
 int fake_launches() { return n_launch; }
+void fake_watch(void (*f)(const char *, void **)) { watcher = f; }      // called with the name and the arguments of every launch that does not fail
 int fake_grid() { return grid_x; }                     // workgroups of the last launch
 void fake_limit(size_t free_bytes) { limit_bytes = free_bytes == ~(size_t)0 ? free_bytes : live_bytes + free_bytes; }
 size_t fake_live() { return live_bytes; }
@@ -41,9 +43,11 @@ void __hipRegisterFunction(void **, const void * f, char *, const char * name, u
 void __hipRegisterVar(void **, void *, char *, char *, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3, size_t, hipStream_t) { grid_x = g.x; return hipSuccess; }
 hipError_t __hipPopCallConfiguration(dim3 * g, dim3 * b, size_t * sh, hipStream_t * st) { *g = dim3(1); *b = dim3(1); *sh = 0; *st = nullptr; return hipSuccess; }
-hipError_t hipLaunchKernel(const void * f, dim3, dim3, void **, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void * f, dim3, dim3, void ** args, size_t, hipStream_t) {
     ++counts[names()[f]];
-    return n_launch++ == fail_at ? (last = hipErrorInvalidValue) : hipSuccess;
+    if (n_launch++ == fail_at) return last = hipErrorInvalidValue;
+    if (watcher) watcher(names()[f].c_str(), args);
+    return hipSuccess;
 }
 hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }
 const char * hipGetErrorString(hipError_t) { return "fake"; }
