@@ -156,6 +156,7 @@ struct LayerState {
     bool auto_pool = false;                            // sized by the engine (decode, batch_init), not by the caller
     int32_t * lists = nullptr;                         // device [32][kv.n]: a sequence's cells in position order
     std::vector<int32_t> list_cells[32], list_pos[32]; // the same on the host
+    std::vector<int32_t> news;                         // what the device has not learned yet: (sequence, place, cell), each place of a sequence once
     int32_t * d_delta = nullptr;
     // step buffers for `cap` tokens (one allocation)
     int cap = 0;
@@ -1413,12 +1414,13 @@ int choose_parts(LayerState * s, int n_work, int n_vis_max) {
 }
 
 // ---- cells -----------------------------------------------------------------------------------------------------------------------
-// the host's list of a sequence's cells, rebuilt after an edit; `app` receives what the device has to learn, (sequence, place, cell) with every place of a
-// sequence once: the kernels that store them do so in no order
-void refresh_list(LayerState * s, int q, std::vector<int32_t> & app) {
+// the host's list of a sequence's cells, rebuilt after an edit.  s->news receives what the device has to learn, every place of a sequence once (the kernels
+// that store it do so in no order), and holds it until a launch that carries it has been queued, whatever becomes of the call
+void refresh_list(LayerState * s, int q) {
     if (!(s->kv.edited >> q & 1u)) return;
     s->kv.edited &= ~(1u << q);
-    size_t kept = 0;                                               // what app says of the sequence so far is its list before the edit
+    std::vector<int32_t> & app = s->news;
+    size_t kept = 0;                                               // what it says of the sequence so far is its list before the edit
     for (size_t k = 0; k < app.size(); k += 3)
         if (app[k] != q) { std::copy_n(app.begin() + k, 3, app.begin() + kept); kept += 3; }
     app.resize(kept);
@@ -1439,14 +1441,14 @@ int live_cells(LayerState * s, int q) {
 }
 
 // takes the cell for sequences `mask` at position p; false: some sequence's list has to be rebuilt (the position is not behind its last)
-void take_cell(LayerState * s, int cell, int32_t p, uint32_t mask, int32_t tok, std::vector<int32_t> & app) {
+void take_cell(LayerState * s, int cell, int32_t p, uint32_t mask, int32_t tok) {
     s->kv.take(cell, p, mask);
     s->cell_tok[cell] = tok;
     for (uint32_t b = mask; b; b &= b - 1) {
         const int q = __builtin_ctz(b);
         if (s->kv.edited >> q & 1u) continue;                      // rebuilt as a whole later
         if (!s->list_pos[q].empty() && s->list_pos[q].back() >= p) { s->kv.edited |= 1u << q; continue; }
-        app.push_back(q); app.push_back((int32_t)s->list_pos[q].size()); app.push_back(cell);
+        s->news.insert(s->news.end(), {q, (int32_t)s->list_pos[q].size(), cell});
         s->list_pos[q].push_back(p); s->list_cells[q].push_back(cell);
     }
 }
@@ -1530,7 +1532,7 @@ int copy_inputs(pi_model * m, size_t n) {
     return PI_OK;
 }
 
-// The pass's n integers and the new cells behind them (n_app triples) on their way, then its embeddings and angles.  kLinkTokens: most tokens whose ids and
+// The pass's n integers and the news behind them (n_app triples) on their way, then its embeddings and angles.  kLinkTokens: most tokens whose ids and
 // positions are read across the link (a pass of four layers, us, across it and in two launches: 1 token 437 / 443, 64 1550 / 1553, 128 1596 / 1601, 256 1834 / 1829).
 constexpr int kLinkTokens = 128;
 int start_pass(pi_model * m, Step & in, size_t n, size_t at_app, int n_app) {
@@ -1541,6 +1543,7 @@ int start_pass(pi_model * m, Step & in, size_t n, size_t at_app, int n_app) {
     s->in_flight = true;
     if (T > kLinkTokens) {
         PI_TRY(pi::pass_start(p, m->stream));
+        s->news.clear();
         p = pi::PassStart{};
     }
     const int32_t * from = T > kLinkTokens ? s->d_in : s->h_in;
@@ -1553,17 +1556,23 @@ int start_pass(pi_model * m, Step & in, size_t n, size_t at_app, int n_app) {
         p.rot[p.n_rot] = {r.dims, r.base, r.length(), r.scaling ? r.freq : nullptr, s->cs[p.n_rot]};
     }
     in.started = true;
-    return pi::pass_start(p, m->stream);
+    PI_TRY(pi::pass_start(p, m->stream));
+    s->news.clear();
+    return PI_OK;
 }
 
-int upload_appends(pi_model * m, const std::vector<int32_t> & app) {
-    if (app.empty()) return PI_OK;
+// the news in a launch of its own
+int send_news(pi_model * m) {
     LayerState * s = m->lay;
+    const std::vector<int32_t> & app = s->news;
+    if (app.empty()) return PI_OK;
     if (app.size() <= AppendArgs::kMost) {                         // a step's cells travel as arguments: no copy, and nothing to wait for
         AppendArgs args;
         memcpy(args.v, app.data(), app.size() * 4);
         hipLaunchKernelGGL(cells_append_args_kernel, dim3(1), dim3(64), 0, m->stream, args, (int)(app.size() / 3), s->lists, (size_t)s->kv.n);
-        return pi::check_launch("cells_append");
+        PI_TRY(pi::check_launch("cells_append"));
+        s->news.clear();
+        return PI_OK;
     }
     PI_TRY(ensure_inputs(m, app.size()));
     PI_TRY(inputs_free(m));
@@ -1571,7 +1580,9 @@ int upload_appends(pi_model * m, const std::vector<int32_t> & app) {
     PI_TRY(copy_inputs(m, app.size()));
     const int n = (int)(app.size() / 3);
     hipLaunchKernelGGL(cells_append_kernel, dim3((n + 255) / 256), dim3(256), 0, m->stream, s->d_in, n, s->lists, (size_t)s->kv.n);
-    return pi::check_launch("cells_append");
+    PI_TRY(pi::check_launch("cells_append"));
+    s->news.clear();
+    return PI_OK;
 }
 
 }  // namespace
@@ -1606,6 +1617,7 @@ static int resize_pool(pi_model * m, int n_cells) {
     if (!s->lists || !s->d_delta) return PI_E_HIP;
     PI_TRY(pi_memset(s->lists, 0, sizeof(int32_t) * 32 * (size_t)n_cells));
     PI_TRY(pi_sync());
+    s->news.clear();                                               // (every list is rebuilt)
     if (s->kv.n) s->kv.grow(n_cells); else s->kv.init(n_cells);
     return PI_OK;
 }
@@ -1755,12 +1767,12 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
     for (int w = 0; w < n_want; ++w) if (want[w] < 0 || want[w] >= n_tokens) return fail(PI_E_ARG, "pi_model_kv_cells_step: a wanted place is outside the step");
     for (int t = 0; t < n_tokens; ++t)
         if (tokens[t] < 0 || tokens[t] >= m->hp.n_vocab || positions[t] < 0 || seq_masks[t] == 0) return fail(PI_E_ARG, "pi_model_kv_cells_step: a token needs an id, a position and a sequence");
-    std::vector<int32_t> cells(n_tokens), app;
+    std::vector<int32_t> cells(n_tokens);
     if (!s->kv.find_free(n_tokens, cells.data())) return fail(PI_E_STATE, "pi_model_kv_cells_step: not enough free cells");
     const int batch = s->opts.max_batch > 0 ? s->opts.max_batch : 2048;
     PI_TRY(ensure_capacity(m, std::min(n_tokens, batch)));
     PI_TRY(apply_shift(m));
-    for (int t = 0; t < n_tokens; ++t) for (uint32_t b = seq_masks[t]; b; b &= b - 1) refresh_list(s, __builtin_ctz(b), app);
+    for (int t = 0; t < n_tokens; ++t) for (uint32_t b = seq_masks[t]; b; b &= b - 1) refresh_list(s, __builtin_ctz(b));
     uint32_t fresh = 0;                                          // recurrent models: sequences whose state starts at zero
     if (s->recurrent) {
         uint32_t met = 0;
@@ -1773,13 +1785,12 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             else if (!s->list_pos[q].empty() && s->list_pos[q].back() >= positions[t]) why = "pi_model_kv_cells_step: a recurrent state takes its tokens in order";
             else { met |= 1u << q; if (s->list_pos[q].empty()) fresh |= 1u << q; }
         }
-        if (why) { PI_TRY(upload_appends(m, app)); return fail(PI_E_UNSUPPORTED, why); }
+        if (why) return fail(PI_E_UNSUPPORTED, why);
         for (uint32_t b = met; b; b &= b - 1) PI_TRY(take_slot(m, __builtin_ctz(b), met));
     }
-    for (int t = 0; t < n_tokens; ++t) take_cell(s, cells[t], positions[t], seq_masks[t], tokens[t], app);
+    for (int t = 0; t < n_tokens; ++t) take_cell(s, cells[t], positions[t], seq_masks[t], tokens[t]);
     s->kv.move_head(cells[n_tokens - 1] + 1);
-    for (int t = 0; t < n_tokens; ++t) for (uint32_t b = seq_masks[t]; b; b &= b - 1) refresh_list(s, __builtin_ctz(b), app);
-    struct Pending { pi_model * m; std::vector<int32_t> & app; ~Pending() { if (!app.empty()) (void)upload_appends(m, app); } } pending{m, app};      // (a call that ends before its first pass)
+    for (int t = 0; t < n_tokens; ++t) for (uint32_t b = seq_masks[t]; b; b &= b - 1) refresh_list(s, __builtin_ctz(b));
     std::vector<int32_t> vis(n_tokens), seq(n_tokens), prev(n_tokens, -1);
     for (int t = 0; t < n_tokens; ++t) {
         seq[t] = __builtin_ctz(seq_masks[t]);                    // a token attends the cells of its first sequence
@@ -1898,8 +1909,8 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             items.insert(items.end(), seq_r.begin(), seq_r.end());
         }
         const size_t n_in = (size_t)8 * T + items.size() + rows.size();
-        const int n_app = (int)(app.size() / 3);                   // (the first pass's)
-        PI_TRY(ensure_inputs(m, n_in + app.size()));
+        const int n_app = (int)(s->news.size() / 3);               // (the first pass's)
+        PI_TRY(ensure_inputs(m, n_in + s->news.size()));
         PI_TRY(inputs_free(m));
         int32_t * h = s->h_in;
         memcpy(h, tokens + t0, 4 * (size_t)T); memcpy(h + T, positions + t0, 4 * (size_t)T); memcpy(h + 2 * T, cells.data() + t0, 4 * (size_t)T);
@@ -1907,7 +1918,7 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
         memcpy(h + 5 * T, prev.data() + t0, 4 * (size_t)T);      // (the items behind start on a multiple of 16 bytes)
         if (!items.empty()) memcpy(h + 8 * T, items.data(), 4 * items.size());
         if (!rows.empty()) memcpy(h + 8 * T + items.size(), rows.data(), 4 * rows.size());
-        if (n_app) memcpy(h + n_in, app.data(), 4 * app.size());
+        if (n_app) memcpy(h + n_in, s->news.data(), 4 * s->news.size());
         in.tokens = s->d_in; in.pos = s->d_in + T; in.cell = s->d_in + 2 * T; in.n_vis = s->d_in + 3 * T; in.seq = s->d_in + 4 * T; in.prev = s->d_in + 5 * T;
         in.conv = s->d_in + 8 * T + at_conv;
         in.lin = s->d_in + 8 * T + at_lin; in.lin_long = in.lin + 4 * in.n_lin; in.lin_first = in.lin_long + 4 * in.n_lin_long; in.lin_chunks = in.lin_first + in.n_lin_long;
@@ -1952,7 +1963,6 @@ int layers_step(pi_model * m, const int32_t * tokens, const int32_t * positions,
             in.last = &one;
         }
         struct Whole { LayerState * s; ~Whole() { if (s->tail) swap_tail(s); } } whole{s};      // however the pass ends, the buffers are in their own places behind it
-        app.clear();
         PI_TRY(start_pass(m, in, n_in, n_in, n_app));
         PI_TRY(pass_layers(m, in));
         for (int r0 = 0; r0 < (int)rows.size(); r0 += kHeadRows) {
@@ -1989,18 +1999,16 @@ static int ensure_pool(pi_model * m, int64_t n) {
 // tokens at n_past .. of sequence q, behind exactly n_past cells (what lies at n_past and beyond is dropped first)
 static int continue_at(pi_model * m, int q, int n_past) {
     LayerState * s = m->lay;
-    std::vector<int32_t> app;
-    refresh_list(s, q, app);
-    PI_TRY(upload_appends(m, app));
+    refresh_list(s, q);
+    PI_TRY(send_news(m));
     const auto & lp = s->list_pos[q];
     const int before = (int)(std::lower_bound(lp.begin(), lp.end(), n_past) - lp.begin());
     if (before != n_past || (n_past && (lp[0] != 0 || lp[n_past - 1] != n_past - 1))) return fail(PI_E_STATE, "the sequence's cells do not hold the positions 0 .. n_past - 1");
     if ((int)lp.size() == before) return PI_OK;
     if (s->recurrent && before > 0) return fail(PI_E_UNSUPPORTED, "a model with recurrent states cannot go back to an earlier position");
     s->kv.seq_rm(q, n_past, -1);
-    app.clear();
-    refresh_list(s, q, app);
-    return upload_appends(m, app);
+    refresh_list(s, q);
+    return send_news(m);
 }
 
 int layers_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_past, float * logits_out) {
@@ -2052,11 +2060,11 @@ int layers_generate(pi_model * m, int own, int n_steps, int32_t * out_tokens, fl
     const int T = own ? 1 : s->n_seq, q0 = own ? kOwnSeq : 0;
     if (!T || !s->kv.n) return fail(PI_E_STATE, "pi_model_generate: decode a prompt first");
     if (n_steps <= 0 || n_steps > s->max_steps || !out_tokens) return fail(PI_E_ARG, "pi_model_generate: bad step count");
-    std::vector<int32_t> tok(T), pos(T), vis(T), seq(T), cell(T), prev(T), lin(4 * T), cells((size_t)n_steps * T), app;
+    std::vector<int32_t> tok(T), pos(T), vis(T), seq(T), cell(T), prev(T), lin(4 * T), cells((size_t)n_steps * T);
     PI_TRY(apply_shift(m));
     for (int t = 0; t < T; ++t) {
         seq[t] = q0 + t; tok[t] = s->last_tok[q0 + t]; pos[t] = s->last_pos[q0 + t];
-        refresh_list(s, q0 + t, app);
+        refresh_list(s, q0 + t);
         if (pos[t] + n_steps > m->hp.n_ctx) return fail(PI_E_ARG, "pi_model_generate: would run past the context");
         if ((int)s->list_pos[q0 + t].size() != pos[t]) return fail(PI_E_STATE, "pi_model_generate: a sequence's cells do not end at its next position");
         prev[t] = pos[t] ? s->cell_tok[s->list_cells[q0 + t].back()] : -1;
@@ -2068,9 +2076,9 @@ int layers_generate(pi_model * m, int own, int n_steps, int32_t * out_tokens, fl
     }
     if (!s->kv.find_free(n_steps * T, cells.data())) return fail(PI_E_STATE, "pi_model_generate: not enough free cells");
     for (int k = 0; k < n_steps; ++k)
-        for (int t = 0; t < T; ++t) take_cell(s, cells[(size_t)k * T + t], pos[t] + k, 1u << (q0 + t), k ? -1 : tok[t], app);
+        for (int t = 0; t < T; ++t) take_cell(s, cells[(size_t)k * T + t], pos[t] + k, 1u << (q0 + t), k ? -1 : tok[t]);
     s->kv.move_head(cells.back() + 1);
-    PI_TRY(upload_appends(m, app));
+    PI_TRY(send_news(m));
     PI_TRY(ensure_capacity(m, T));
     for (int t = 0; t < T; ++t) { vis[t] = pos[t] + 1; cell[t] = cells[t]; }
     std::vector<int32_t> items;

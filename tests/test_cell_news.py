@@ -59,3 +59,43 @@ shared = list(125 + np.argsort(both))
 holds(0, list(np.argsort(pos)) + [121, 122, 120] + shared)
 holds(1, [124, 123] + shared)
 """)
+
+
+def test_a_call_that_fails_loses_nothing():
+    """Whichever launch of a step fails, one pass or several, and whatever refuses a call behind an edit of the cells: the next call's launches say what is missing."""
+    fake_hip.run(DEVICE + """
+L = pl.load()
+def refused(f):
+    try:
+        f()
+    except pl.PiError:
+        return
+    raise AssertionError("not refused")
+for n in (40, 200):                                     # one launch that a pass begins with, two
+    m.kv_cells_clear()
+    lists.clear()
+    F.fake_fail_launch(-1)
+    step(range(n), [1] * n)
+    launches = F.fake_launches()
+    for k in range(launches):
+        m.kv_cells_clear()
+        lists.clear()
+        F.fake_fail_launch(k)
+        refused(lambda: step(range(n), [1] * n))
+        F.fake_fail_launch(-1)
+        step([n], [1])
+        cells = [c for _, c in sorted((place, c) for (q, place), c in lists.items() if q == 0)]
+        assert len(cells) == n + 1 and len(set(cells)) == n + 1, (n, k, len(cells))
+m.close()
+
+m = lerasun.build(cfg, weights(cfg, 17), compute=pl.F32, n_ctx=64)
+lists.clear()
+m.decode(list(range(1, 31)), 0)
+kept = next(iter(lists))[0]                             # the model's own sequence
+m.kv_seq_rm(10, 20)
+m.kv_seq_shift(20, 30, -10)                             # the device's list still names the first thirty cells
+refused(lambda: m.generate(60))                         # past the context, which is seen behind the rebuild of the list
+m.decode([5], 20)
+holds(kept, [*range(10), *range(20, 30), lists[kept, 20]])
+m.close()
+""")
