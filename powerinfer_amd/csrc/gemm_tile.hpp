@@ -32,9 +32,9 @@ struct GemmTile {
     static __device__ __forceinline__ int chunk_row(int j) { return j * (kThreads / 8) + (int)threadIdx.x / 8; }
     static __device__ __forceinline__ int chunk_col() { return ((int)threadIdx.x % 8) * 8; }
 
-    // ga, gb: where this thread's chunks of the first stage lie; nk stages of kGtBK columns.  acc[m][n][r] belongs to the tile's row
+    // ga, gb: where this thread's chunks of column 0 lie; nk stages of kGtBK columns, taken from stage `first` on around the end.  acc[m][n][r] belongs to the tile's row
     // wm * WM + m * 16 + 4 g + r and token wn * WN + n * 16 + i (lane = 16 g + i, wave = wn * WGM + wm)
-    static __device__ __forceinline__ void run(unsigned char * smem, const EL * const (&ga)[ACH], const EL * const (&gb)[BCH], int nk, pi_f4 (&acc)[MT][NT]) {
+    static __device__ __forceinline__ void run(unsigned char * smem, const EL * const (&ga)[ACH], const EL * const (&gb)[BCH], int nk, pi_f4 (&acc)[MT][NT], int first = 0) {
         unsigned char * sa = smem;                                     // [2][BM][kGtRow]
         unsigned char * sb = smem + 2 * BM * kGtRow;                   // [2][BN][kGtRow]
         const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
@@ -54,10 +54,11 @@ struct GemmTile {
         pi_u32x4 ra[2][ACH], rb[2][BCH];
         auto fetch = [&](auto slot, int kt) {
             constexpr int S = decltype(slot)::value;
+            const size_t at = (size_t)(first + kt < nk ? first + kt : first + kt - nk) * kGtBK;
 #pragma unroll
-            for (int j = 0; j < ACH; ++j) ra[S][j] = pi_ld16(ga[j] + (size_t)kt * kGtBK);
+            for (int j = 0; j < ACH; ++j) ra[S][j] = pi_ld16(ga[j] + at);
 #pragma unroll
-            for (int j = 0; j < BCH; ++j) rb[S][j] = pi_ld16(gb[j] + (size_t)kt * kGtBK);
+            for (int j = 0; j < BCH; ++j) rb[S][j] = pi_ld16(gb[j] + at);
         };
         auto stash = [&](auto slot) {              // registers of slot S -> LDS half S
             constexpr int S = decltype(slot)::value;

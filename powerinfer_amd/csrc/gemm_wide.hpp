@@ -1,4 +1,4 @@
-// The matrix-core product of long prompts in tiles of 256 rows x 128 tokens, shared by the experts' products and the sparse FFN's.
+// The matrix-core product of long prompts in tiles of 256 rows x 128 tokens or 128 x 256, shared by the experts' products and the sparse FFN's.
 #pragma once
 #include "gemm_tile.hpp"
 
@@ -11,8 +11,9 @@ namespace {
 // below).  A multiplying wave reads the fragments of a stage's second 32 columns under the products of the first and those of the
 // next stage's first 32 under the products of the second, with the one barrier of a stage in between: behind it the next stage is
 // whole and the present one is free to be copied over.  LDS rows and swizzle are GemmTile's; a copy's 64 lanes bring eight rows of
-// 128 bytes and take the swizzle on the side they read from.  Where half a tile or less is wanted (128 rows, 64 tokens) the four
-// waves share that half, 64 x 64 outputs each.  The sums are formed in GemmTile's order.
+// 128 bytes and take the swizzle on the side they read from.  Where half a tile or less is wanted (half its rows, or so few tokens that a wave would
+// have none) the four waves share that half, 64 x 64 outputs each.  The sums are formed in GemmTile's order: 32 columns a step, beginning at a stage that
+// depends on the product and the row alone (first), so that a token's outputs are the same bits whichever tiles it falls into.
 // Measured (us; 128 x 128 tiles of GemmTile before): 64 experts of 192 tokens on average, 1408 x 4096: 301 -> 215, 4096 x 1408:
 // 307 -> 226 (weights alone: 123 at 6 TB/s); one group of 12288: 199 -> 133, 1.07 PFLOP/s; 16 experts of 128: 51 -> 45 and 38 -> 34.
 // ---------------------------------------------------------------------------------------------------------------------------------
@@ -24,7 +25,7 @@ constexpr int kGwBand = 8;
 // The units of this workgroup: the products (token tile, 256 rows) are dealt out so that an XCD works through a contiguous range of them,
 // band token tiles by row tiles (its L2 then serves a band's tokens and a few row tiles to all of its workgroups), the row tiles of more
 // than 128 rows first, then the shorter ones, which take half the time.  What does not fill the XCD's
-// workgroups once more at the end is cut into halves of 128 rows if that gives no workgroup two of them.
+// workgroups once more at the end is cut into halves of a tile's rows if that gives no workgroup two of them.  (256 rows: `tile` of them.)
 struct WideDeal {
     int rows, n_tiles, band, tile, nl, xcd, slot, slots, per_long, per_short, n_long, rounds, rest_unit, rest_row, count;
     bool halves;
@@ -60,7 +61,8 @@ struct WidePlace { int grp, lo, n, row0, rows; };       // of a unit: group, fir
 
 // P (a product): nk stages of 64 columns; place(deal, c); base_a(p, w), base_b(p): where the rows of a tile's w-th 64 rows and its tokens start, and
 // off_a(p, r), off_b(p, r): the bytes from there to tile row and token r (in range: r is cut to the unit's); kPairs: a wave's rows
-// are two runs of MT / 2 tiles, `gap` rows apart beyond their own where MT is 4; read_once(p): no other unit reads these rows of W; first(p): the column stage a unit begins with; kM, kN: the tile; store<MT>(p, rb, tb, acc, turn, lane): the
+// are two runs of MT / 2 tiles, `gap` rows apart beyond their own where MT is 4; read_once(p): no other unit reads these rows of W; first(p): the column stage a unit begins with, which may depend on nothing
+// but its group and rows; kM, kN: the tile; store<MT>(p, rb, tb, acc, turn, lane): the
 // outputs of rows rb .. and tokens tb .. of the tile.
 template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(const P & prod, const WideDeal & deal, unsigned char * smem) {
     if (deal.count == 0) return;
@@ -70,7 +72,7 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
     const int nk = prod.nk, count = deal.count;
     WidePlace * places = reinterpret_cast<WidePlace *>(smem + kGwStages * kGwStage);      // of this unit and those behind it, written by the first copying wave
     if (wave >= 4) {
-        // A wave that copies.  Of each stage eight times eight rows of W and four times eight of x are its own, each 128 bytes; lane l brings
+        // A wave that copies.  Of each stage CA times eight rows of W and CB times eight of x are its own, each 128 bytes; lane l brings
         // the piece that belongs at place l % 8 of row l / 8
         const int w = wave - 4, piece = ((lane & 7) ^ (lane >> 3)) * 16;
         uint32_t va[CA];

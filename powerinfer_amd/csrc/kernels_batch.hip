@@ -509,9 +509,10 @@ template <bool PAIRS, bool MASK> struct FfnProduct {
     static constexpr bool kPairs = PAIRS;
     static constexpr int kM = kGwM, kN = kGwN;
     __device__ __forceinline__ bool read_once(const WidePlace &) const { return false; }
-    // Rows a multiple of 4 KB apart lie in few of the memory's channels: an XCD's workgroups, which share what they read, begin at columns of their own (bits
-    // included, us: 32768 x 8192 alone, 129 tokens 160 -> 137, 200 173 -> 151, 2047 1009 -> 994; 11008 x 4096 twice, 2047 tokens 359 -> 354).
-    __device__ __forceinline__ int first(const WidePlace &) const { return cols % 2048 ? 0 : (int)(blockIdx.x % 8) * nk / 8; }
+    // Rows a multiple of 16 KB apart lie in few of the memory's channels: every 2048 of them begin at columns of their own (bits included, us, one place for all /
+    // this: 32768 x 8192 alone, 129 tokens 161 / 142, 200 175 / 155, 400 247 / 252, 700 381 / 390, 2047 1027 / 1029; 4096 columns, twice 11008 rows: 129 tokens 63.2 /
+    // 64.5, 2047 372 / 370, so not there).  The place goes by the row alone: a token's sums have one order however many come along.
+    __device__ __forceinline__ int first(const WidePlace & p) const { return cols % 8192 ? 0 : p.row0 / 2048 % 8 * nk / 8; }
     const __half * up, * gate, * x; const float * logits; float thr; __half * h16;
     int ff, cols, T, nk;
     const unsigned long long * mask;

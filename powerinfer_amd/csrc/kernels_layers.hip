@@ -550,6 +550,17 @@ __device__ __forceinline__ void group_store(const pi_group_gemm & g, int grp, in
         }
 }
 
+// The column stage that the sums of these rows of a listed group begin with, in tiles of any size.  Rows a multiple of 4 KB apart lie in few of the memory's
+// channels, and workgroups that began together would all read the same of them: 256 rows of a group have a place of their own there.  Tiles of 128
+// and 256 tokens, us, one place for all / this: 64 experts of 96 tokens, 1408 x 4096 162 / 140, of 192 190 / 184; 8 experts of 64, 8192 x 4096 123 / 88, of
+// 140 136 / 123; 1408 columns: no difference.  Tiles of 64 tokens gain nothing from it (16 experts of 33, 2816 x 2048: 36.1 / 36.5), but they keep the
+// order of the larger ones.  The place goes by group and row alone, so that a token's outputs do not depend on how many come along.  Products without a list share
+// their rows between many workgroups and begin at column 0 (every 2048 rows of 22016 x 5120 at another one: 400 tokens 1.5 % slower, 2043 tokens 3 % faster), as results in
+// fp32 and short rows do.
+__device__ __forceinline__ int group_first(const pi_group_gemm & g, int grp, int row0) {
+    return !g.off || g.y_f32 || g.cols < 2048 || g.ldw % 2048 ? 0 : (grp * 13 + row0 / kGwM) % (g.cols / kGtBK);
+}
+
 template <int BM, int BN, int WGM, int WGN>
 __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192 ? 3 : 2)) void group_tile_kernel(pi_group_gemm g, int nx, int max_units) {
     using Tile = GemmTile<bf16, BM, BN, WGM, WGN>;
@@ -582,7 +593,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, (WGM * WGN > 4 ? 1 : BM + BN <= 192
         gb[j] = x + (size_t)(g.gather ? g.gather[s] / g.gather_div : s) * g.ldx + Tile::chunk_col();
     }
     pi_f4 acc[MT][NT];
-    Tile::run(smem, ga, gb, g.cols / kGtBK, acc);
+    Tile::run(smem, ga, gb, g.cols / kGtBK, acc, group_first(g, grp, row0));
     group_store(g, grp, lo, n, row0 + wm * WM, wn * WN, q, i, acc);
 }
 
@@ -645,14 +656,7 @@ template <int M, int N, bool LIST> struct GroupProduct {
         return p;
     }
     __device__ __forceinline__ bool read_once(const WidePlace & p) const { return LIST && g.off[p.grp + 1] - g.off[p.grp] <= N; }
-    // Rows a multiple of 4 KB apart lie in few of the memory's channels, and workgroups that began together would all read the same of them: an expert's
-    // units begin at different columns there (64 experts of 96 tokens, 1408 x 4096: 155 -> 138 us; 8 of 140, 8192 x 4096: 243 -> 190; 1408 or 5120
-    // columns: no difference).  Without a list the workgroups of an XCD share what they read and begin together, those of another elsewhere (2043
-    // tokens, 22016 x 5120: 400 -> 380, x 4096 313 -> 311; every row tile at a column of its own: 325).  Results in fp32, and short rows, keep the order of their sums.
-    __device__ __forceinline__ int first(const WidePlace & p) const {
-        if (g.y_f32 || g.cols < 2048) return 0;
-        return !LIST ? (int)(blockIdx.x % 8) * nk / 8 : g.ldw % 2048 ? 0 : (p.grp * 13 + p.row0 / M) % nk;
-    }
+    __device__ __forceinline__ int first(const WidePlace & p) const { return LIST ? group_first(g, p.grp, p.row0) : 0; }
     __device__ __forceinline__ const unsigned char * base_a(const WidePlace & p, int) const { return (const unsigned char *)((const bf16 *)g.W + (size_t)p.grp * g.w_gs); }
     __device__ __forceinline__ const unsigned char * base_b(const WidePlace & p) const { return (const unsigned char *)((const bf16 *)g.x + (g.off ? 0 : (size_t)p.grp * g.x_gs)); }
     __device__ __forceinline__ uint32_t off_a(const WidePlace & p, int r) const { return (uint32_t)(p.row0 + r) * (uint32_t)(g.ldw * 2); }
@@ -924,7 +928,7 @@ int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream
     hipStream_t st = (hipStream_t)stream;
     // 256-row tiles from the second half on, and at least four stages for a unit's ends to hide behind: measured as fast or faster at every number of
     // tokens and groups from there on (32 heads' 256 x 512 products of 128 tokens: 11.4 us both; 4096 x 512 by 2048 tokens 20.6 -> 16.1)
-    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31)) 
+    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31))
         return g->off ? launch_group_wide<kGwM, kGwN, true>(*g, st) : launch_group_wide<kGwM, kGwN, false>(*g, st);
     if (tile_n == 128) return launch_group_tile<128, 128, 2, 2>(*g, st);
     if (tile_n == 64) return g->rows <= 64 ? launch_group_tile<64, 64, 2, 2>(*g, st) : launch_group_tile<128, 64, 2, 2>(*g, st);

@@ -200,6 +200,50 @@ def test_units_that_begin_at_other_columns(rows, cols, tile):
         assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("rows,cols,kind", [(264, 2048, "plain"), (520, 4096, "relu2"), (300, 4096, "plain"), (528, 2048, "glu"), (392, 4096, "pair"), (72, 4096, "plain")])
+def test_one_order_of_sums_in_tiles_of_every_size(rows, cols, kind):
+    """Rows a multiple of 4 KB apart, whose sums begin at columns of the group's and the row's own: the same in tiles of 64, 128 and 256 tokens, so that a token's outputs
+    do not depend on the tile it falls into."""
+    small, _, _ = listed(COUNTS, rows, cols, kind, 0, 64, False)
+    for tile in (128, 256):
+        other, _, _ = listed(COUNTS, rows, cols, kind, 0, tile, tile == 256)
+        if kind in ("glu", "pair"):
+            same(small, other, 0)
+        else:
+            assert np.array_equal(small, other), tile
+
+
+@pytest.mark.parametrize("rows,cols,T", [(2304, 2048, 400), (1280, 5120, 300)])
+def test_one_order_of_sums_without_a_list(rows, cols, T):
+    """Small tiles, large ones, and large ones of other tokens beside these: the same bits."""
+    rng = np.random.default_rng(T)
+    wb, xb = store(rounded(rng.standard_normal((rows, cols)) / np.sqrt(cols)), pl.BF16), store(rounded(rng.standard_normal((T, cols))), pl.BF16)
+    got = []
+    for tile, n in ((64, T), (128, T), (128, T // 2)):
+        g = group_args(W=wb.ptr, rows=rows, cols=cols, ldw=cols, n_group=1, x=xb.ptr, ldx=cols, T=n, ldy=rows, alpha=1.0)
+        got.append(run(g, tile, n, rows, 0)[0])
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0][:T // 2], got[2])
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("ff,cols", [(2304, 4096), (4352, 8192)])
+def test_a_chunks_neurons_do_not_depend_on_its_length(ff, cols, gated):
+    """The sparse FFN's large tiles: the first tokens of a chunk have the same bits whatever follows them."""
+    L, rng = pl.init(), np.random.default_rng(ff)
+    T = 300
+    up, gate, x = (dev((rng.standard_normal(s, dtype=np.float32) / np.sqrt(s[1]) ** (s[0] != T)).astype(np.float16)) for s in ((ff, cols), (ff, cols), (T, cols)))
+    lg = dev(rng.standard_normal((T, ff)).astype(np.float32))
+    got = []
+    for n in (T, 129, 70):
+        h = pl.DevBuf.zeros(2 * T * ff)
+        print(ff, cols, n, gated, flush=True)
+        pl.check(L.pi_k_ffn_wide_f16(up.ptr, gate.ptr if gated else None, ff, cols, x.ptr, n, lg.ptr, 0.25, h.ptr, None))
+        pl.sync()
+        got.append(h.download(np.uint16)[:n * ff].reshape(n, ff))
+    for g in got[1:]:
+        assert np.array_equal(got[0][:len(g)], g)
+
+
 def test_what_tiles_of_256_tokens_do_not_cover_is_refused():
     L, b = pl.init(), pl.DevBuf(1 << 16)
     p = lambda **kw: C.byref(group_args(**dict(dict(W=b.ptr, rows=128, cols=256, ldw=256, n_group=1, x=b.ptr, ldx=256, T=8, y=b.ptr, ldy=128, alpha=1.0, off=b.ptr, tiles=b.ptr, n_tiles=b.ptr, max_tiles=1), **kw)))  # noqa: E731
