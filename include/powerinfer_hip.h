@@ -665,8 +665,10 @@ typedef struct pi_group_gemm {
 PI_API int pi_k_group_gemm(int type, const pi_group_gemm * g, pi_stream_t stream);
 /* the same for many tokens, bf16, both operands tiled through LDS (cols % 64 == 0); tile_n 64 or 128 tokens per tile, as given to pi_k_moe_sort */
 PI_API int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream);
-/* the same in tiles of 256 tokens (tiles: pi_k_moe_sort's with tile_n 256): off != NULL, more than 64 rows, at least 256 columns */
+/* the same in tiles of 256 tokens (tiles: pi_k_moe_sort's with tile_n 256): off != NULL, more than 64 rows, at least 256 columns, less than 2^31 values a group */
 PI_API int pi_k_group_gemm_tall(const pi_group_gemm * g, pi_stream_t stream);
+/* tokens a tile (64, 128 or 256) of both products of n_expert experts, [up_rows][up_ld] and [down_rows][down_ld] each, for n_pairs rows of theirs together */
+PI_API int pi_k_expert_tile(int64_t n_pairs, int n_expert, int up_rows, int up_ld, int down_rows, int down_ld);
 /* (cos, sin)[t][i] of the angles pos[t] * base^(-2i / dims), i < dims / 2 */
 PI_API int pi_k_rope_angles(const int32_t * pos, int T, int dims, double base, void * cs_float2, pi_stream_t stream);
 /* the same with given frequencies (dims / 2 of them), cosine and sine times length */

@@ -853,16 +853,7 @@ int experts(pi_model * m, Layer & L, const void * h, const Step & in) {
     const pi_layer_desc & d = L.d;
     const int T = in.T, D = m->hp.n_embd, per = d.ffn == PI_FFN_GLU_MOE ? 2 : 1;
     hipStream_t st = m->stream;
-    // Tokens per tile, by the tokens an expert has on average (multinomial counts).  Experts' matrices of 512 MB and more (2 MB a compute unit) go through
-    // the large tiles whatever the number: a workgroup streams them at the memory's rate, and 64 and 128 x 128 tiles do not.  Both products of five shapes
-    // (experts x ff x width, * with a gate; us in tiles of 64, 128 and 256 tokens at 16 / 64 / 160 tokens): 64 x 1408 x 4096 272, 249, 283 / 359, 279,
-    // 324 / 573, 404, 378; the same * 390, 342, 420 / 517, 393, 473 / 879, 607, 560; 64 x 1408 x 2048 * 205, 179, 229 / 264, 211, 257 / 419, 319, 306;
-    // 8 x 4096 x 4096 * 151, 134, 147 / 211, 138, 152 / 433, 248, 180; 160 x 1536 x 5120 900, 817, 983 at 16.  Less than that, 16 x 1408 x 2048 *, 32 x 1024 x 1024
-    // and 64 x 256 x 1024 *: at 16 tokens 55, 57, 31, 35 and 27, 29 in tiles of 64 and 128, so 64 until they start to need two an expert, which is at
-    // 52 tokens; in tiles of 128 and 256 at 150 tokens 94, 87, 43, 45 and 48, 47, at 192 82, 93, 45, 49 and 46, 50.
-    const long long pairs = (long long)T * d.n_top, E = d.n_expert, bytes = 2 * E * ((long long)per * d.expert_ff * s->d_ld + (long long)D * L.ff_ld);
-    const bool large = bytes >= 512LL << 20 && per * d.expert_ff > 128 && D > 128 && s->d_ld >= 256 && L.ff_ld >= 256;
-    const int tile_n = large && pairs > 132 * E ? 256 : large || pairs > 52 * E ? 128 : 64;
+    const int tile_n = pi_k_expert_tile((int64_t)T * d.n_top, d.n_expert, per * d.expert_ff, s->d_ld, D, L.ff_ld);
     PI_TRY(pi_k_moe_sort(s->ids, T * d.n_top, d.n_expert, s->off, s->perm, s->inv, tile_n, s->tiles, s->n_tiles, st));
     pi_group_gemm g{};
     g.W = L.up; g.w_gs = (size_t)per * d.expert_ff * s->d_ld; g.rows = per * d.expert_ff; g.cols = s->d_ld; g.ldw = s->d_ld; g.n_group = d.n_expert; g.alpha = 1.0f;

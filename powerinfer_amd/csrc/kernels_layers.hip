@@ -633,6 +633,7 @@ __device__ __forceinline__ void group_store_turned(const pi_group_gemm & g, int 
     }
 }
 
+constexpr long long kGwValues = 1LL << 31;                          // of a group's matrix: off_a counts its bytes in 32 bits
 // the same product in the large tiles of gemm_wide.  256 rows by 128 tokens, or 128 by 256: an expert of more than 128 tokens then has its weights
 // read once, and by one workgroup.  64 experts, both products, us, tiles of 128 / 256 tokens: 192 tokens an expert on average 407 -> 390 (1408 x 4096), 624 -> 585
 // (with a gate); 8 experts of 140, 4096 x 4096 with a gate 245 -> 176; of 96 tokens 290 and 334.
@@ -928,17 +929,31 @@ int pi_k_group_gemm_tile(const pi_group_gemm * g, int tile_n, pi_stream_t stream
     hipStream_t st = (hipStream_t)stream;
     // 256-row tiles from the second half on, and at least four stages for a unit's ends to hide behind: measured as fast or faster at every number of
     // tokens and groups from there on (32 heads' 256 x 512 products of 128 tokens: 11.4 us both; 4096 x 512 by 2048 tokens 20.6 -> 16.1)
-    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < (1LL << 31))
+    if (tile_n == 128 && g->rows > 128 && g->cols >= 4 * kGtBK && (long long)g->rows * g->ldw < kGwValues)
         return g->off ? launch_group_wide<kGwM, kGwN, true>(*g, st) : launch_group_wide<kGwM, kGwN, false>(*g, st);
     if (tile_n == 128) return launch_group_tile<128, 128, 2, 2>(*g, st);
     if (tile_n == 64) return g->rows <= 64 ? launch_group_tile<64, 64, 2, 2>(*g, st) : launch_group_tile<128, 64, 2, 2>(*g, st);
     return pi::fail(PI_E_ARG, "pi_k_group_gemm_tile: tile_n must be 64 or 128");
 }
 
+// Tokens per tile, by the tokens an expert has on average (multinomial counts).  Experts' matrices of 512 MB and more (2 MB a compute unit) go through
+// the large tiles whatever the number: a workgroup streams them at the memory's rate, and 64 and 128 x 128 tiles do not.  Both products of five shapes
+// (experts x ff x width, * with a gate; us in tiles of 64, 128 and 256 tokens at 16 / 64 / 160 tokens): 64 x 1408 x 4096 272, 249, 283 / 359, 279,
+// 324 / 573, 404, 378; the same * 390, 342, 420 / 517, 393, 473 / 879, 607, 560; 64 x 1408 x 2048 * 205, 179, 229 / 264, 211, 257 / 419, 319, 306;
+// 8 x 4096 x 4096 * 151, 134, 147 / 211, 138, 152 / 433, 248, 180; 160 x 1536 x 5120 900, 817, 983 at 16.  Less than that, 16 x 1408 x 2048 *, 32 x 1024 x 1024
+// and 64 x 256 x 1024 *: at 16 tokens 55, 57, 31, 35 and 27, 29 in tiles of 64 and 128, so 64 until they start to need two an expert, which is at
+// 52 tokens; in tiles of 128 and 256 at 150 tokens 94, 87, 43, 45 and 48, 47, at 192 82, 93, 45, 49 and 46, 50.
+int pi_k_expert_tile(int64_t n_pairs, int n_expert, int up_rows, int up_ld, int down_rows, int down_ld) {
+    const int64_t up = (int64_t)up_rows * up_ld, down = (int64_t)down_rows * down_ld;
+    const bool large = 2 * n_expert * (up + down) >= 512LL << 20 && up_rows > 128 && down_rows > 128 && up_ld >= 4 * kGtBK && down_ld >= 4 * kGtBK;
+    // (beyond kGwValues an expert's matrix has no tiles of 256 tokens, and those of 128 go another way)
+    return large && n_pairs > 132LL * n_expert && up < kGwValues && down < kGwValues ? 256 : large || n_pairs > 52LL * n_expert ? 128 : 64;
+}
+
 int pi_k_group_gemm_tall(const pi_group_gemm * g, pi_stream_t stream) {
     const int rc = group_tile_args(g);
     if (rc != PI_OK) return rc;
-    if (!g->off || g->rows <= 64 || g->cols < 4 * kGtBK || (long long)g->rows * g->ldw >= (1LL << 31))
+    if (!g->off || g->rows <= 64 || g->cols < 4 * kGtBK || (long long)g->rows * g->ldw >= kGwValues)
         return pi::fail(PI_E_UNSUPPORTED, "pi_k_group_gemm_tall: lists of more than 64 rows, at least 256 columns and less than 2^31 values a group");
     return launch_group_wide<128, 256, true>(*g, (hipStream_t)stream);
 }

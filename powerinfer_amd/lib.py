@@ -254,6 +254,7 @@ _SIGS = {
     "pi_k_group_gemm": (_i, [_i, C.POINTER(GroupGemm), _vp]),
     "pi_k_group_gemm_tile": (_i, [C.POINTER(GroupGemm), _i, _vp]),
     "pi_k_group_gemm_tall": (_i, [C.POINTER(GroupGemm), _vp]),
+    "pi_k_expert_tile": (_i, [C.c_int64, _i, _i, _i, _i, _i]),
     "pi_k_rope_angles": (_i, [_vp, _i, _i, C.c_double, _vp, _vp]),
     "pi_k_latent_prep": (_i, [_i, C.POINTER(LatentPrep), _vp]),
     "pi_k_latent_attn_rows": (_i, [_i]),
