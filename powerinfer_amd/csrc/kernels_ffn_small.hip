@@ -152,6 +152,7 @@ __global__ __launch_bounds__(kSmBlock) void ffn_small_f16_kernel(const __half * 
             a = pi_wave_sum(a);
             if (GATE) b = pi_wave_sum(b);
             const float h = pi_round_f16(GATE ? __fmul_rn(fmaxf(b, 0.0f), a) : fmaxf(a, 0.0f));
+            if (h == 0.0f) continue;                                // (no term, as on the CPU path: a zero times an infinite weight would be one)
 #pragma unroll
             for (int j = 0; j < CH; ++j) {
                 float f[8];

@@ -60,6 +60,39 @@ def test_small_ffn_in_one_launch(ff, r, cols, kind, gate, active):
     assert (np.abs(got - want) <= bound).all()
 
 
+@pytest.mark.parametrize("cols,gate", [(512, True), (1024, False)])
+def test_active_neurons_of_value_zero(cols, gate):
+    """Neurons that the predictor calls active and whose value is zero, or rounds to zero in fp16, add nothing, whatever their rows of the down projection hold."""
+    L, rng = pl.init(), np.random.default_rng(cols)
+    ff, r = 256, 64
+    half = lambda *s: (rng.standard_normal(s) * s[-1] ** -0.5).astype(np.float16)
+    fc1, fc2, up, gt, down = half(r, cols), half(ff, r), half(ff, cols), half(ff, cols), half(ff, cols)
+    x = np.abs(rng.standard_normal(cols)).astype(np.float32)
+    zero, tiny, bad = np.arange(0, ff, 3), np.arange(1, ff, 9), np.float16(np.inf)
+    (gt if gate else up)[zero] = -np.abs((gt if gate else up)[zero])          # negative products of positive inputs
+    up[tiny] = 0
+    if gate:
+        gt[tiny] = np.abs(gt[tiny])
+        up[tiny, 0], x[0] = np.float16(6e-8), np.float32(2.0 ** -14)          # a product far below fp16's smallest value
+    down[zero], down[tiny, ::2], down[tiny, 1::2] = bad, -bad, np.nan
+    bufs = [pl.DevBuf(host=v) for v in (fc1, fc2, up, gt, down, x)]
+    d1, d2, du, dg, dd, dx = (v.ptr for v in bufs)
+    out, n = pl.DevBuf(host=np.full(cols, np.nan, np.float32)), pl.DevBuf(host=np.full(1, -1, np.int32))
+    ws, nrm = L.pi_workspace_create(ff, cols), pl.Norm(0, 1e-5, None, None)
+    pl.check(L.pi_k_sparse_ffn_small(d1, d2, ff, r, float("-inf"), du, dg if gate else None, dd, cols, dx, C.byref(nrm), 0, None, None, out.ptr, n.ptr, ws, None), "small")
+    got = out.download(np.float32)
+    L.pi_workspace_destroy(ws)
+    assert n.download(np.int32)[0] == ff
+    keep = np.ones(ff, bool)
+    keep[zero] = keep[tiny] = False
+    x64 = x.astype(np.float16).astype(np.float64)
+    U, G, D = (m[keep].astype(np.float64) for m in (up, gt, down))
+    h = np.maximum(G @ x64, 0) * (U @ x64) if gate else np.maximum(U @ x64, 0)
+    eh = (np.abs(G) @ x64) * (np.abs(U) @ x64) * cols * 2.0 ** -22 if gate else (np.abs(U) @ x64) * cols * 2.0 ** -24
+    bound = (eh + np.abs(h) * 2.0 ** -11 + 2.0 ** -25) @ np.abs(D) + (np.abs(h) @ np.abs(D)) * (ff + 8) * 2.0 ** -24
+    assert (np.abs(got - h @ D) <= bound).all()
+
+
 def test_refusals():
     L = pl.init()
     for ff, r, cols in ((48, 128, 512), (0, 128, 512), (4096, 512, 512), (4096, 256, 1024), (4096, 128, 768), (4096, 96, 512)):
