@@ -258,6 +258,9 @@ __global__ __launch_bounds__(64 * kSrWaves) void sum_norm_route_kernel(pi_sum_no
         const int e = e0 + wave + lane * kSrWaves;
         if (lane < kSrRows && e < r.E) __hip_atomic_store(sums + g * r.E + e, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    // every wave waits for its own sums to have arrived before the workgroup says so: a barrier waits for LDS alone, and the release ahead of the count for the
+    // stores of the wave that counts
+    __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0)
     __syncthreads();
     if (tid == 0) last = __hip_atomic_fetch_add(r.arrived + t, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1 == (unsigned int)p.groups;
     __syncthreads();
