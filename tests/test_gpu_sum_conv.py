@@ -45,12 +45,24 @@ def test_as_in_two_launches(t, cols, groups, taps, ol):
         got.append([xb.download(np.float32), keep.download(np.float32), sb.download(np.float32), fetch(h, t, (ld // 8, 16, 8)) if ol else fetch(h, t, (T, ld))[:, :cols]])
     (x1, k1, s1, h1), (x2, k2, s2, h2) = got
     assert np.array_equal(x1, x2) and np.array_equal(k1, k2)
-    # the groups' sums of squares run in another order: n squares' sums differ by n * 2^-24 of themselves at most, their roots by half of that; behind them sums of taps + 1
-    # products of such inputs, and one rounding of the result
-    off = cols // groups * 2.0 ** -24
+    # The groups' sums of squares run in another order: a chain of at most size / 64 additions of a lane (four squares of every 256 columns), 6 of a wave and 16 of the waves, so that two of
+    # them are within that many 2^-24 of the squares' sum on either side, and their roots within half of both together.  Two roundings behind it for an input; an output is
+    # taps + 1 products of inputs (the last one's tap and itself), a rounding each, and one of the result in bf16 that may fall the other way.
+    size = cols // groups
+    off = (size / 64 + 22 + 4) * 2.0 ** -24
     assert (np.abs(s1 - s2) <= off * np.abs(s1)).all()
-    top = np.abs(x1).max() * 40                                       # (of a normed input times a weight)
-    assert np.abs(h1 - h2).max() <= off * top * (taps + 1) + (2.0 ** -8 if t == pl.BF16 else 2.0 ** -22) * np.abs(h1).max()
+    rows = lambda h: h.transpose(1, 0, 2).reshape(16, ld)[:T, :cols] if ol else h      # noqa: E731
+    u = x1.reshape(T, groups, size).astype(np.float64)
+    u = (u / np.sqrt((u ** 2).mean(-1, keepdims=True) + 1e-5)).reshape(T, cols) * w2
+    for (first, n, _, _, slot, fresh, _, _) in items:
+        past = np.zeros((taps - 1, cols)) if fresh else state[slot, :(taps - 1) * cols].reshape(taps - 1, cols)
+        run = np.abs(np.concatenate([past, u[first:first + n]]))
+        for k in range(n):
+            terms = run[taps - 1 + k] + (np.abs(taps_w) * run[k:k + taps]).sum(0)
+            a, b = rows(h1)[first + k], rows(h2)[first + k]
+            assert (np.abs(a - b) <= (off + (taps + 1) * 2.0 ** -24) * terms + (2.0 ** -7 * np.abs(a) if t == pl.BF16 else 0)).all()
+            want = u[first + k] + (taps_w * np.concatenate([past, u[first:first + n]])[k:k + taps]).sum(0)
+            assert (np.abs(b - want) <= (off + (taps + 1) * 2.0 ** -24) * terms + (2.0 ** -8 * np.abs(want) if t == pl.BF16 else 0)).all()
 
 
 def test_sizes_that_are_not_supported():
