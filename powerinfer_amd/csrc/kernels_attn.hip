@@ -396,7 +396,7 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
 // guarded load makes the compiler wait for all the others; past the last cell its rows are read again), and what the rotation
 // needs ahead of them, because loads return in order.  Merge included, against the same sums with guarded loads and the soft-max of the whole workgroup
 // between two barriers: 32 heads of 128 in 8 parts, 1030 cells 12.4 -> 11.0 us, 3001 19.4 -> 16.4 (49 MB), 32000 in 16 parts 97 -> 93.5; 128
-// heads of 64 in 2 parts, 1030 cells 14.2 -> 12.3.
+// heads of 64 in 2 parts, 1030 cells 14.2 -> 12.3; 64 heads of 8 in 8 parts 17.5 -> 17.1, of 16 14.7 -> 14.2 (25.6 and 18.0 with what their 512 or 256 groups leave read one by one).
 // ---------------------------------------------------------------------------------------------------
 // FROM_CACHE: the token's own K / V row is in the cache already and qkv holds its rotated q only ([n_head * hd] per token; a prompt chunk
 // behind rope_kv_store_kernel): nothing is rotated or stored, every cell is read from the cache.
@@ -414,10 +414,12 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     pos_p += blockIdx.z;
     extern __shared__ __align__(16) unsigned char smem[];
     const int lpp = LPP ? LPP : hd / 8, ngrp = kAttnPartBlock / lpp;
-    double * gl  = reinterpret_cast<double *>(smem);              // [ngrp] the groups' sums of e_i
-    float * part = reinterpret_cast<float *>(gl + ngrp);          // [ngrp][hd]
-    float * gm   = part + kAttnPartBlock * 8;                     // [ngrp] the groups' maxima
-    float * qs   = gm + ngrp;                                     // [hd] rotated q, rounded to fp16
+    // sums of e_i and maxima, of the groups (32 or 64 of them: read at once) or, of the many groups of small heads and where their number is not a constant, of the waves
+    constexpr int N = LPP ? kAttnPartBlock / LPP : kAttnPartBlock / PI_WAVE;
+    __shared__ double sums[N];
+    __shared__ float  tops[N];
+    float * part = reinterpret_cast<float *>(smem);               // [ngrp][hd]
+    float * qs   = part + kAttnPartBlock * 8;                     // [hd] rotated q, rounded to fp16
     float * kcur = qs + hd;                                       // [hd] rotated k of this position, rounded to fp16
     float * vcur = kcur + hd;                                     // [hd]
     float * s    = vcur + hd;                                     // [s_cap] scores of this part
@@ -506,12 +508,14 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
         top = fmaxf(top, d);
         if (sub == 0) s[n_old] = d;
     }
-    if (sub == 0) gm[grp] = top;
+    const int slot_of = LPP ? grp : tid / PI_WAVE, lane_of = LPP ? sub : tid & (PI_WAVE - 1);
+    if (!LPP) for (int o = lpp; o < PI_WAVE; o <<= 1) top = fmaxf(top, __shfl_xor(top, o, PI_WAVE));
+    if (lane_of == 0) tops[slot_of] = top;
     __syncthreads();
     float mx = -INFINITY;
-    for (int g = 0; g < ngrp; g += 8)
+    for (int g = 0; g < N; g += 8)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, gm[g + j]);
+        for (int j = 0; j < 8; ++j) mx = fmaxf(mx, tops[g + j]);
 
     float acc[8];
     double sum = 0.0;
@@ -541,7 +545,8 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) part[grp * hd + sub * 8 + i] = acc[i];
-    if (sub == 0) gl[grp] = sum;
+    if (!LPP) for (int o = lpp; o < PI_WAVE; o <<= 1) sum += __shfl_xor(sum, o, PI_WAVE);       // (whole numbers of 2^-24: exact in any order)
+    if (lane_of == 0) sums[slot_of] = sum;
     __syncthreads();
     if (tid < hd) {
         float v = part[tid];
@@ -553,11 +558,11 @@ __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const floa
             for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
         }
         part_acc[slot * hd + tid] = v;
-    } else if (tid == hd) {                                         // (whole numbers of 2^-24: exact in any order)
+    } else if (tid == hd) {
         double l = 0.0;
-        for (int g = 0; g < ngrp; g += 8)
+        for (int g = 0; g < N; g += 8)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) l += gl[g + j];
+            for (int j = 0; j < 8; ++j) l += sums[g + j];
         part_ml[slot * 2] = mx; part_ml[slot * 2 + 1] = (float)l;
     }
 }
@@ -1635,17 +1640,15 @@ int pi_k_attn_decode_supported(int hd, int n_ctx) {
 // the lanes of a cell are a constant for the two usual head sizes (their sums are then lane permutations)
 #define PI_ATTN_LPP(...) do { if (hd == 128) { constexpr int LPP = 16; __VA_ARGS__; } else if (hd == 64) { constexpr int LPP = 8; __VA_ARGS__; } \
                               else { constexpr int LPP = 0; __VA_ARGS__; } } while (0)
-// the parts and their merge; LDS: what pi_k_attn_split_supported counts and three words a group, 6 KB for heads of eight values
+// the parts and their merge
+static size_t attn_part_lds(int hd, int s_cap) { return sizeof(float) * ((size_t)s_cap + kAttnPartBlock * 8 + 3 * (size_t)hd); }
 template <bool FROM_CACHE>
 static int launch_attn_parts(const float * qkv, const float2 * rope_table, __half * k, __half * v, int n_tok, int n_head, int n_head_kv, int hd, int mode, int n_ctx, int n_parts, const int32_t * pos,
                              float * scratch, int qkv_stride, size_t cache_seq_stride, float * out, int out_stride, __half * out_f16, hipStream_t st, const char * name) {
     const int s_cap = (n_ctx + n_parts - 1) / n_parts + 1;
-    const size_t lds = sizeof(float) * ((size_t)s_cap + kAttnPartBlock * 8 + 3 * (size_t)hd + 3 * (size_t)(kAttnPartBlock * 8 / hd));
+    const size_t lds = attn_part_lds(hd, s_cap);
     float * acc = scratch, * ml = scratch + (size_t)n_tok * n_head * n_parts * hd;
-    PI_ATTN_LPP(
-        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_part_kernel<FROM_CACHE, LPP>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAttnLdsLimit + 8192);
-        if (raised != hipSuccess) return pi::hip_fail(raised, "attn_part: LDS size");
-        hipLaunchKernelGGL((attn_part_kernel<FROM_CACHE, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), lds, st, qkv, rope_table, k, v, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml,
+    PI_ATTN_LPP(hipLaunchKernelGGL((attn_part_kernel<FROM_CACHE, LPP>), dim3(n_head, n_parts, n_tok), dim3(kAttnPartBlock), lds, st, qkv, rope_table, k, v, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos, acc, ml,
                            qkv_stride, cache_seq_stride));
     hipLaunchKernelGGL(attn_merge_kernel, dim3(n_head, n_tok), dim3(hd), 0, st, acc, ml, n_parts, hd, out, out_stride, out_f16);
     return pi::check_launch(name);
@@ -1674,7 +1677,7 @@ static bool attn_part_geometry_ok(int hd) {
     return hd > 0 && hd % 8 == 0 && kAttnPartBlock % (hd / 8) == 0 && PI_WAVE % (hd / 8) == 0 && hd / 2 + hd <= kAttnPartBlock && hd <= 1024;
 }
 int pi_k_attn_split_supported(int hd, int n_ctx, int n_parts) {
-    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && sizeof(float) * ((size_t)(n_ctx + n_parts - 1) / n_parts + 1 + kAttnPartBlock * 8 + 3 * (size_t)hd) <= kAttnLdsLimit;
+    return attn_part_geometry_ok(hd) && n_ctx > 0 && n_parts >= 1 && n_parts <= 64 && attn_part_lds(hd, (n_ctx + n_parts - 1) / n_parts + 1) <= kAttnLdsLimit;
 }
 size_t pi_k_attn_split_scratch_floats(int n_seq, int n_head, int hd, int n_parts) { return (size_t)n_seq * n_head * n_parts * ((size_t)hd + 2); }
 
