@@ -325,31 +325,26 @@ __global__ __launch_bounds__(256) void conv_norm_kernel(pi_conv_norm p, int max_
 }
 
 // The same, four columns a thread, for up to BACK inputs ahead of a token and N >= BACK tokens of an item: a thread's inputs lie in registers, all requested together.
+// groups: those of a workgroup, `size` columns each
 template <typename ST, int BACK, int N>
-__global__ __launch_bounds__(1024) void conv_norm_quads_kernel(pi_conv_norm p, int max_rows, int groups) {
+__global__ __launch_bounds__(1024) void conv_norm_quads_kernel(pi_conv_norm p, int max_rows, int groups, int size) {
     extern __shared__ __align__(16) float sm[];
-    const int size = p.cols / p.groups, lo = (int)blockIdx.y * groups * size, hi = lo + groups * size;
-    const int c0 = min(lo + (int)threadIdx.x * 4, hi - 4);           // (threads without columns request the last ones and do no more)
-    float4 w, tw[BACK + 1];
-    const auto weights = [&](int c) {
-        w = *reinterpret_cast<const float4 *>(p.w + c);
-#pragma unroll
-        for (int j = 0; j <= BACK; ++j) tw[j] = *reinterpret_cast<const float4 *>(p.taps_w + (size_t)j * p.cols + c);
-    };
-    weights(c0);
     const int4 a = reinterpret_cast<const int4 *>(p.items)[2 * blockIdx.x], b = reinterpret_cast<const int4 *>(p.items)[2 * blockIdx.x + 1];
-    const int t0 = a.x, n = min(a.y, N), off = a.z, len = a.w, slot = b.x;
+    const int t0 = a.x, n = min(a.y, N), off = a.z, len = a.w, slot = b.x, lo = (int)blockIdx.y * groups * size, hi = lo + groups * size;
     const bool head = off == 0, fresh = b.y != 0;
     const int before = min(off, BACK), run0 = t0 - off, n_a = n + before, tail = head ? max(n, len - BACK) : len, rows = n_a + (head ? len - tail : 0);
     if (rows > max_rows) return;                       // (the launcher's bound)
     float * scale = sm, * part = sm + max_rows * groups;
+    group_scales(part, scale, rows, groups, groups * size, p.eps, [&](int r) { return p.x + (size_t)(r < n_a ? t0 - before + r : run0 + tail + (r - n_a)) * p.cols + lo; });
     float * state = p.state ? p.state + slot * p.slot_ld : nullptr;
     ST * h = (ST *)p.h;
-    const int step = blockDim.x * 4;
-    float4 u[BACK + N];                                // inputs: place k - BACK of the item
-    // (the first columns' inputs and weights are on their way while the groups' scales are formed)
-    const auto fetch = [&](int c) {
+    for (int c = lo + threadIdx.x * 4; c < hi; c += blockDim.x * 4) {
+        const int g = (c - lo) / size;
         const auto quad = [&](const float * q) { return *reinterpret_cast<const float4 *>(q + c); };
+        float4 u[BACK + N], tw[BACK + 1];              // inputs: place k - BACK of the item
+        const float4 w = quad(p.w);
+#pragma unroll
+        for (int j = 0; j <= BACK; ++j) tw[j] = quad(p.taps_w + (size_t)j * p.cols);
 #pragma unroll
         for (int k = 0; k < BACK + N; ++k) {
             const int i = k - BACK;
@@ -358,13 +353,6 @@ __global__ __launch_bounds__(1024) void conv_norm_quads_kernel(pi_conv_norm p, i
             if (i + before >= 0) u[k] = quad(p.x + (size_t)(t0 + i) * p.cols);
             else if (head && !fresh) u[k] = quad(state + (size_t)k * p.cols);
         }
-    };
-    fetch(c0);
-    group_scales(part, scale, rows, groups, groups * size, p.eps, [&](int r) { return p.x + (size_t)(r < n_a ? t0 - before + r : run0 + tail + (r - n_a)) * p.cols + lo; });
-    for (int c = lo + threadIdx.x * 4; c < hi; c += step) {
-        const int g = (c - lo) / size;
-        const auto quad = [&](const float * q) { return *reinterpret_cast<const float4 *>(q + c); };
-        if (c != c0) { weights(c); fetch(c); }
 #pragma unroll
         for (int k = 0; k < BACK + N; ++k) {
             const int r = k - BACK + before;
@@ -458,18 +446,20 @@ template <typename ST> void launch_sum_conv(const pi_sum_norm & p, const pi_conv
 }
 template <typename ST> bool launch_conv_quads(const pi_conv_norm & p, int rows, size_t lds, hipStream_t st) {
     if ((p.cols / p.groups) % 4 || p.ld % 4 || p.slot_ld % 4 || p.taps > 5) return false;
-    // workgroups of as many whole groups as leave the chip two a unit (one token's 160 KB are 6.6 us for one unit, 4.7 for eight)
+    // As many workgroups of whole groups as run at once: two a unit, one of 1024 threads (whose registers leave no room for another: 700 tokens of 6144 columns in 4 groups, 350
+    // workgroups of two groups 14.5 us, 175 of all 11.8).  One token's 160 KB are 6.6 us for one unit, 4.7 for eight.
+    const int size = p.cols / p.groups;
+    const auto threads = [&](int groups) { return groups * size > 2048 ? 1024 : groups * size > 1024 ? 512 : 256; };
     int groups = p.groups;
     for (int d = 2; d <= p.groups && p.n_items * d <= 2 * pi::compute_units(); ++d)
-        if (p.groups % d == 0) groups = p.groups / d;
-    const int cols = p.cols / p.groups * groups;
-    const dim3 grid(p.n_items, p.groups / groups), block(cols > 2048 ? 1024 : cols > 1024 ? 512 : 256);
+        if (p.groups % d == 0 && p.n_items * d <= pi::compute_units() * (threads(p.groups / d) > 512 ? 1 : 2)) groups = p.groups / d;
+    const dim3 grid(p.n_items, p.groups / groups), block(threads(groups));
     switch (p.taps) {
-        case 1: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 0, 4>), grid, block, lds, st, p, rows, groups); break;
-        case 2: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 1, 4>), grid, block, lds, st, p, rows, groups); break;
-        case 3: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 2, 4>), grid, block, lds, st, p, rows, groups); break;
-        case 4: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 3, 4>), grid, block, lds, st, p, rows, groups); break;
-        default: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 4, 4>), grid, block, lds, st, p, rows, groups);
+        case 1: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 0, 4>), grid, block, lds, st, p, rows, groups, size); break;
+        case 2: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 1, 4>), grid, block, lds, st, p, rows, groups, size); break;
+        case 3: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 2, 4>), grid, block, lds, st, p, rows, groups, size); break;
+        case 4: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 3, 4>), grid, block, lds, st, p, rows, groups, size); break;
+        default: hipLaunchKernelGGL((conv_norm_quads_kernel<ST, 4, 4>), grid, block, lds, st, p, rows, groups, size);
     }
     return true;
 }
