@@ -104,7 +104,8 @@ __global__ __launch_bounds__(1024) void norm_pair_kernel(const float * __restric
 }
 
 // the same with four columns a thread at a time, up to 4096 of them in the registers of 256 threads (rows, weights and outputs in whole quads): 2048 tokens of 4096
-// columns into two operands 22.8 -> 12.6 us.  For long passes: 16 waves a row are the better ones for a few (one token 4.8 us, this 5.1)
+// columns into two operands 22.8 -> 12.6 us.  For long passes: 16 waves a row are the better ones for a few (one token 4.8 us, this 5.1); and beyond 512 columns,
+// below which most threads have none (2048 tokens of 512 columns 4.5 us, this 5.4; of 768 7.4 and 5.8)
 template <typename ST>
 __global__ __launch_bounds__(256) void norm_pair_quads_kernel(const float * __restrict__ x, const int32_t * __restrict__ rows, int cols, float eps, const float * __restrict__ wa,
                                                              ST * __restrict__ out_a, const float * __restrict__ wb, ST * __restrict__ out_b, int ld) {
@@ -832,7 +833,7 @@ int pi_k_norm_pair(int type, const float * x, const int32_t * rows, int T, int c
                    const float * wb, void * out_b, int ld, int ol, pi_stream_t stream) {
     if (!x || !wa || !out_a || (wb && !out_b) || T <= 0 || cols <= 0 || ld < cols) return pi::fail(PI_E_ARG, "pi_k_norm_pair: bad arguments");
     if (ol && (type != PI_TYPE_BF16 || T > kBtMaxT || ld % 8)) return pi::fail(PI_E_ARG, "pi_k_norm_pair: operand layout needs BF16, T <= 16, ld % 8 == 0");
-    if (T > kBtMaxT && cols % 4 == 0 && cols <= 4096 && ld % 4 == 0 && (((uintptr_t)x | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)out_a | (uintptr_t)out_b) & 15) == 0 && (type == PI_TYPE_BF16 || type == PI_TYPE_F32)) {
+    if (T > kBtMaxT && cols % 4 == 0 && cols > 512 && cols <= 4096 && ld % 4 == 0 && (((uintptr_t)x | (uintptr_t)wa | (uintptr_t)wb | (uintptr_t)out_a | (uintptr_t)out_b) & 15) == 0 && (type == PI_TYPE_BF16 || type == PI_TYPE_F32)) {
         if (type == PI_TYPE_BF16) hipLaunchKernelGGL(norm_pair_quads_kernel<bf16>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, rows, cols, eps, wa, (bf16 *)out_a, wb, (bf16 *)out_b, ld);
         else hipLaunchKernelGGL(norm_pair_quads_kernel<float>, dim3(T), dim3(256), 0, (hipStream_t)stream, x, rows, cols, eps, wa, (float *)out_a, wb, (float *)out_b, ld);
         return pi::check_launch("pi_k_norm_pair");
