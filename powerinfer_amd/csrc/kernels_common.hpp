@@ -56,17 +56,28 @@ __device__ float block_max_f32(float v, float * red) {
 // RMSNorm as ggml.c:9238-9284 (double sum of fp32 squares, scale = 1/sqrtf(mean+eps), then * w as a
 // second fp32 multiply: llm_build_norm, llama.cpp:4420-4450); LayerNorm as ggml.c:9169-9236.
 // ---------------------------------------------------------------------------------------------------
+// (Of workgroups of kBlock threads, which is a constant here: read from the launch it was a load from memory that waited for the weights requested ahead of it.)
 template <typename X>                                  // a pointer to floats, or what else yields x[i]
 __device__ void stage_x_f16(__half * xs, X x, int cols, NormArgs na, double * red) {
+    const auto own_sum = [&](double v) -> double {
+        v = pi_wave_sum_f64(v);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < kWavesPerBlock; ++i) s += red[i];
+        return s;
+    };
     float mean = 0.0f, scale = 1.0f;
     constexpr int kHeld = 4;
-    if (cols <= kHeld * (int)blockDim.x) {
+    if (cols <= kHeld * kBlock) {
         // short vectors: the values and the norm's weights are requested together and stay in registers (the same operations in the same order)
         float xv[kHeld], wv[kHeld], bv[kHeld];
         const bool has_w = na.kind != 0 && na.w, has_b = na.kind != 0 && na.b;
 #pragma unroll
         for (int k = 0; k < kHeld; ++k) {
-            const int i = threadIdx.x + k * blockDim.x;
+            const int i = threadIdx.x + k * kBlock;
             xv[k] = i < cols ? x[i] : 0.0f;
             wv[k] = has_w && i < cols ? na.w[i] : 1.0f;
             bv[k] = has_b && i < cols ? na.b[i] : 0.0f;
@@ -75,19 +86,19 @@ __device__ void stage_x_f16(__half * xs, X x, int cols, NormArgs na, double * re
             double s = 0.0;
 #pragma unroll
             for (int k = 0; k < kHeld; ++k) s += (double)__fmul_rn(xv[k], xv[k]);
-            scale = pi_inv_sqrt((float)(block_sum_f64(s, red) / cols) + na.eps);
+            scale = pi_inv_sqrt((float)(own_sum(s) / cols) + na.eps);
         } else if (na.kind == 2) {
             double s = 0.0, s2 = 0.0;
 #pragma unroll
             for (int k = 0; k < kHeld; ++k) s += (double)xv[k];
-            mean = (float)(block_sum_f64(s, red) / cols);
+            mean = (float)(own_sum(s) / cols);
 #pragma unroll
-            for (int k = 0; k < kHeld; ++k) { const float v = __fsub_rn(xv[k], mean); if (threadIdx.x + k * blockDim.x < (unsigned)cols) s2 += (double)__fmul_rn(v, v); }
-            scale = pi_inv_sqrt((float)(block_sum_f64(s2, red) / cols) + na.eps);
+            for (int k = 0; k < kHeld; ++k) { const float v = __fsub_rn(xv[k], mean); if (threadIdx.x + k * kBlock < (unsigned)cols) s2 += (double)__fmul_rn(v, v); }
+            scale = pi_inv_sqrt((float)(own_sum(s2) / cols) + na.eps);
         }
 #pragma unroll
         for (int k = 0; k < kHeld; ++k) {
-            const int i = threadIdx.x + k * blockDim.x;
+            const int i = threadIdx.x + k * kBlock;
             float v = xv[k];
             if (na.kind != 0) {
                 v = __fmul_rn(na.kind == 2 ? __fsub_rn(v, mean) : v, scale);
@@ -101,20 +112,20 @@ __device__ void stage_x_f16(__half * xs, X x, int cols, NormArgs na, double * re
     }
     if (na.kind == 1) {
         double s = 0.0;
-        for (int i = threadIdx.x; i < cols; i += blockDim.x) { const float v = x[i]; s += (double)__fmul_rn(v, v); }
-        s = block_sum_f64(s, red);
+        for (int i = threadIdx.x; i < cols; i += kBlock) { const float v = x[i]; s += (double)__fmul_rn(v, v); }
+        s = own_sum(s);
         scale = pi_inv_sqrt((float)(s / cols) + na.eps);
     } else if (na.kind == 2) {
         double s = 0.0;
-        for (int i = threadIdx.x; i < cols; i += blockDim.x) s += (double)x[i];
-        s = block_sum_f64(s, red);
+        for (int i = threadIdx.x; i < cols; i += kBlock) s += (double)x[i];
+        s = own_sum(s);
         mean = (float)(s / cols);
         double s2 = 0.0;
-        for (int i = threadIdx.x; i < cols; i += blockDim.x) { const float v = __fsub_rn(x[i], mean); s2 += (double)__fmul_rn(v, v); }
-        s2 = block_sum_f64(s2, red);
+        for (int i = threadIdx.x; i < cols; i += kBlock) { const float v = __fsub_rn(x[i], mean); s2 += (double)__fmul_rn(v, v); }
+        s2 = own_sum(s2);
         scale = pi_inv_sqrt((float)(s2 / cols) + na.eps);
     }
-    for (int i = threadIdx.x; i < cols; i += blockDim.x) {
+    for (int i = threadIdx.x; i < cols; i += kBlock) {
         float v = x[i];
         if (na.kind != 0) {
             v = __fmul_rn(na.kind == 2 ? __fsub_rn(v, mean) : v, scale);
