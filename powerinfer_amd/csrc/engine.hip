@@ -376,6 +376,13 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
     return PI_OK;
 }
 
+int head_forward(pi_model * m) {
+    const pi_hparams & hp = m->hp;
+    const bool falcon = hp.arch == PI_ARCH_FALCON;
+    const pi_norm on = make_norm(falcon ? 2 : 1, hp.norm_eps, m->glob[PI_T_OUTPUT_NORM], falcon ? &m->glob[PI_T_OUTPUT_NORM_B] : nullptr);
+    return pi_k_gemv(m->glob[PI_T_OUTPUT].type, m->glob[PI_T_OUTPUT].dev, hp.n_vocab, hp.n_embd, m->x, &on, PI_EPI_NONE, nullptr, nullptr, m->logits, m->stream);
+}
+
 // one token: embedding -> layers -> (final norm + lm-head + greedy)
 // (token < 0: the one the device's state names; otherwise this one, at position pos)
 int token_forward(pi_model * m, bool want_logits, bool last_token, int32_t token = -1, int32_t pos = 0) {
@@ -392,12 +399,13 @@ int token_forward(pi_model * m, bool want_logits, bool last_token, int32_t token
     else if (token < 0) PI_TRY(pi_k_embed(table.type, table.dev, hp.n_embd, m->d_token, m->x, st));
     else PI_TRY(pi::embed_start(table.type, table.dev, hp.n_embd, token, pos, m->d_token, m->d_pos, m->d_step, m->x, st));
     for (int il = 0; il < hp.n_layer; ++il) PI_TRY(layer_forward(m, il, last_token, il == 0 && whole_start ? &start : nullptr));
-    if (want_logits) {
-        const bool falcon = hp.arch == PI_ARCH_FALCON;
-        pi_norm on = make_norm(falcon ? 2 : 1, hp.norm_eps, m->glob[PI_T_OUTPUT_NORM], falcon ? &m->glob[PI_T_OUTPUT_NORM_B] : nullptr);
-        PI_TRY(pi_k_gemv(m->glob[PI_T_OUTPUT].type, m->glob[PI_T_OUTPUT].dev, hp.n_vocab, hp.n_embd, m->x, &on, PI_EPI_NONE, nullptr, nullptr, m->logits, st));
-    }
-    return PI_OK;
+    return want_logits ? head_forward(m) : PI_OK;
+}
+// a prompt's last token behind the chunk that it came along in: the last layer and the head
+int last_row_forward(pi_model * m, const float * row, int32_t token, int32_t pos) {
+    PI_TRY(pi::resume_token(row, m->hp.n_embd, token, pos, m->d_token, m->d_pos, m->d_step, m->x, m->stream));
+    PI_TRY(layer_forward(m, m->hp.n_layer - 1, true, nullptr));
+    return head_forward(m);
 }
 
 // pin (optional): pinned memory for the call's results
@@ -854,21 +862,25 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
     for (int i = 0; i < n_tokens; ++i)
         if (tokens[i] < 0 || tokens[i] >= m->hp.n_vocab) return pi::fail(PI_E_ARG, "pi_model_decode: token id out of range");
     int first = 0;
+    const float * last_row = nullptr;      // of a prompt whose last token has come along in a chunk: its input of the last layer
     if (n_tokens > 2) {
         // the prompt goes through in chunks (weights read once per chunk): up to 2048 tokens where the dense chunk path covers the
         // model (F16 or Q4_0 matrices, hybrid layers included), up to 16 for the remainder of an F16 model that is whole on the
-        // device; what is left, and at least the last token, takes the single-token path below, which produces the logits
-        const bool wide = pi::prefill_wide_supported(m), small = pi::prefill_supported(m);
+        // device; what is left takes the single-token path below, which produces the logits: the last token from the start, or (prefill_ends) its
+        // last layer alone
+        const bool wide = pi::prefill_wide_supported(m), small = pi::prefill_supported(m), ends = pi::prefill_ends(m);
         pi::WideRoute route = wide ? pi::prefill_wide_route(m) : pi::WideRoute{};
-        while (n_tokens - 1 - first >= 2) {
-            const int left = n_tokens - 1 - first;
-            if (wide && left > 16) {
-                const int T = pi::prefill_wide_chunk(m, tokens + first, left, n_past + first, route);
+        // (16 tokens and one alone, 1281 us of eight 7B-shaped layers, are faster than a wide chunk of 17, 1356)
+        const int most = ends ? n_tokens : n_tokens - 1, few = ends && small ? 17 : 16;
+        while (most - first >= 2) {
+            const int left = most - first;
+            if (wide && left > few) {
+                const int T = pi::prefill_wide_chunk(m, tokens + first, left, n_past + first, route, ends ? &last_row : nullptr);
                 if (T < 0) return T;
                 first += T;
             } else if (small) {
                 const int T = left < 16 ? left : 16;
-                PI_TRY(pi::prefill_chunk(m, tokens + first, T, n_past + first));
+                PI_TRY(pi::prefill_chunk(m, tokens + first, T, n_past + first, ends && T == left ? &last_row : nullptr));
                 first += T;
             } else {
                 break;
@@ -879,6 +891,7 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
         const bool last = i == n_tokens - 1;
         PI_TRY(token_forward(m, last, last, tokens[i], n_past + i));
     }
+    if (last_row) PI_TRY(last_row_forward(m, last_row, tokens[n_tokens - 1], n_past + n_tokens - 1));
     // greedy choice on the device; the state then points at the next position
     int32_t tok = -1;
     uint32_t status = 0;

@@ -23,6 +23,7 @@ struct BatchState {
     std::vector<char> dense_ffn, graph_dense;
     float dense_above = 1.0f;
     bool prefill = false;                 // prompt chunks of the model's own sequence: tokens share the model's KV cache
+    bool ends = false;                    // the chunk's last token is the prompt's: what it fires in a layer counts
     float * q_rot = nullptr;
     size_t cache_seq_stride = 0;          // elements per sequence: n_layer * n_head_kv * n_ctx * hd
     __half *k_cache = nullptr, *v_cache = nullptr;
@@ -296,6 +297,7 @@ int batch_layer(pi_model * m, BatchState * b, int il) {
     // predictor
     PI_TRY(pi_k_gemm_f16_ol(fc1.dev, r, d, b->xp16, T, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16, st));
     PI_TRY(pi_k_batch_predictor_fc2_ol(fc2.dev, ff, r, b->hid16, T, hp.sparse_threshold, b->pred_logits, m->ws, st));
+    if (b->prefill && b->ends) PI_TRY(pi::count_active(b->pred_logits, nullptr, T, ff, hp.sparse_threshold, m->n_active + il, st));
     // Dense cross-over (the reference's switch from its batch-sparse kernels to a plain mat-mul, ggml-cuda.cu:8787-8814, 7717-7756):
     // when the sequences' active sets together cover nearly all of the layer, gathering rows costs more than streaming all of them.
     // Measured on the 13B shape, 40 layers, 16 sequences, 128-token prompts (ms per step, union kernels / dense): union 0.41 of n_ff
@@ -563,7 +565,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
         else ffn_x = b->xa16;
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
-    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, T);
+    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, b->ends ? T - 1 : T);      // (the token that comes along does not change how the others go)
     if (!bits) PI_TRY(chunk_gemm(m, b, fc2.dev, ff, r, b->hid16, PI_EPI_NONE, nullptr, nullptr, b->pred_logits, nullptr));
     if (!one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_UP, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->up_out));
     if (!falcon && !one_kernel) PI_TRY(chunk_product(m, b, il, PI_T_FFN_GATE, up_ol, ff, d, ffn_x, PI_EPI_NONE, nullptr, nullptr, b->gate_out));
@@ -572,6 +574,7 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     else if (down_ol) PI_TRY(pi_k_ffn_h_q8_f16_ol(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else if (down.type == PI_TYPE_Q4_0) PI_TRY(pi_k_ffn_h_q8_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
     else PI_TRY(pi_k_ffn_h_f16(b->up_out, falcon ? nullptr : b->gate_out, b->pred_logits, hp.sparse_threshold, T, ff, b->h16, st));
+    if (b->ends) PI_TRY(pi::count_active(b->pred_logits, bits ? b->pred_logits : nullptr, T, ff, hp.sparse_threshold, m->n_active + il, st));
     if (down_ol) {
         const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
         float * bufs[6] = {};                          // room in what the FFN is done with (T rows each where the products were apart)
@@ -699,7 +702,20 @@ static int wide_buffers(pi_model * m, BatchState * b, int rows) {
     return PI_E_HIP;
 }
 
-int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route) {
+// A prompt's last token goes through all layers but the last as one more row of its last chunk, which costs the chunk next to nothing, and only through the
+// last one by itself.  Alone it reads every weight again.  Prompts of eight 7B-shaped layers, us, alone / along: 3 tokens 1119 / 828, 64 1836 / 1496, 400
+// 3020 / 2603, 2047 7564 / 7105; four 13B-shaped ones, 700 tokens 2500 / 2255; four 40B-shaped ones, 300 tokens 3062 / 2742.  For F16 matrices that are whole
+// on the device, whose products round at the same places for one token and for many; Q4_0 ones of chunks round their values to fp16 besides, and
+// a layer that is split has the host's share of a lone token.  (The route without the library is there to be compared with, and stays as it is.)
+bool prefill_ends(pi_model * m) {
+    if (m->hybrid || m->capture || m->hp.n_layer < 2 || (!m->gemm_lib && prefill_own_gemm())) return false;
+    for (int il = 0; il < m->hp.n_layer; ++il)
+        for (int k : {PI_T_WQKV, PI_T_WO, PI_T_FFN_UP, PI_T_FFN_GATE, PI_T_FFN_DOWN_T, PI_T_FC1, PI_T_FC2})
+            if (!(k == PI_T_FFN_GATE && m->hp.arch == PI_ARCH_FALCON) && m->L(il, k).type != PI_TYPE_F16) return false;
+    return true;
+}
+
+int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route, const float ** last_row) {
     const pi_hparams & hp = m->hp;
     if (!m->prefill_wide) {
         if (!prefill_own_gemm() && !m->gemm_lib) {
@@ -771,6 +787,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_pas
     }
     b->n_seq = T;
     b->kv_hi = n_past + T;
+    b->ends = last_row && T == left;
     b->route = route;
     PI_TRY(pi::embed_chunk(m->glob[PI_T_TOK_EMBD].type, m->glob[PI_T_TOK_EMBD].dev, hp.n_embd, tokens, T, n_past, b->x, b->d_pos, m->stream));
     b->staged_layer[0] = b->staged_layer[1] = -1;
@@ -782,6 +799,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_pas
         PI_TRY(wide_layer(m, b, il));
         if (staged) { PI_HIP_TRY(hipEventRecord(b->ev_free[il & 1], m->stream)); b->free_recorded[il & 1] = true; }
     }
+    if (b->ends) *last_row = b->x + (size_t)(T - 1) * hp.n_embd;      // (the last layer stores cells and leaves x as it is)
     return T;
 }
 
@@ -791,7 +809,7 @@ bool prefill_supported(pi_model * m) {
 
 // T <= 16 consecutive prompt tokens of the model's own sequence in one step: the weights are read once for the chunk
 // (the prompt-phase counterpart of llama_decode with n_tokens > 1; the reference's batch kernels, ggml-cuda.cu:6994-7034)
-int prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
+int prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const float ** last_row) {
     if (T < 1 || T > 16) return pi::fail(PI_E_ARG, "prefill_chunk: 1 <= T <= 16");
     if (batch_unsupported(m) != nullptr) PI_TRY(ensure_q4_split(m));          // a Q4_0 model: the integer matrix-core route
     if (!m->prefill) {
@@ -801,8 +819,10 @@ int prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past) {
     BatchState * b = m->prefill;
     b->n_seq = T;
     b->kv_hi = n_past + T;
+    b->ends = last_row != nullptr;
     PI_TRY(pi::embed_chunk(m->glob[PI_T_TOK_EMBD].type, m->glob[PI_T_TOK_EMBD].dev, m->hp.n_embd, tokens, T, n_past, b->x, b->d_pos, m->stream));
     for (int il = 0; il < m->hp.n_layer; ++il) PI_TRY(batch_layer(m, b, il));
+    if (b->ends) *last_row = b->x + (size_t)(T - 1) * m->hp.n_embd;
     return PI_OK;
 }
 

@@ -134,9 +134,12 @@ int  layers_seq_cp(pi_model * m, int src, int dst, int p0, int p1);
 int  kv_edit(pi_model * m, __half * k_cache, __half * v_cache, int32_t * d_pos, std::vector<int32_t> & kv_pos, int p0, int p1, int delta, bool shift);
 void batch_destroy(pi_model * m);       // frees the batched-decoding state (graphs; device buffers belong to the model)
 bool prefill_supported(pi_model * m);   // F16 weights, every neuron on the GPU, shapes the multi-token kernels cover
-int  prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past);
+bool prefill_ends(pi_model * m);        // the token that ends a prompt goes along in its last chunk
+// n_past: of the chunk's first token; last_row: null, or (prefill_ends) the chunk ends the prompt, and where its last token's input of the last layer lies is left there
+int  prefill_chunk(pi_model * m, const int32_t * tokens, int T, int n_past, const float ** last_row);
 bool prefill_wide_supported(pi_model * m);   // F16 or Q4_0 matrices (fp16 predictor), hybrid layers included; n_embd, n_ff and the predictor rank multiples of 256
 int  gather_rest_rows(pi_model * m, int il);  // hybrid layer: rows of the non-resident neurons into pinned host memory (rest_up / rest_gate / rest_down)
 WideRoute prefill_wide_route(pi_model * m);
-int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route);     // left > 16; the tokens taken, or an error (< 0)
+// left > 16; the tokens taken, or an error (< 0).  last_row (as above): set if they are all that is left
+int  prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_past, WideRoute & route, const float ** last_row);
 }

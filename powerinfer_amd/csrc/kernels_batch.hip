@@ -614,6 +614,25 @@ template <bool PAIRS, bool MASK> __global__ __launch_bounds__(512, 1) void ffn_w
     gemm_wide<__half>(prod, WideDeal(PAIRS ? 2 * prod.ff : prod.ff, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
 }
 
+// The neurons that fire for the last of T tokens, by logits or by bits (MaskProduct); bound by one trip to memory and the launch
+__global__ __launch_bounds__(1024) void count_active_kernel(const float * __restrict__ logits, const unsigned long long * __restrict__ mask, int T, int ff, float thr, int32_t * __restrict__ n_active) {
+    __shared__ int part[16];
+    int n = 0;
+    if (mask) {
+        const unsigned long long * tile = mask + (size_t)((T - 1) / 16) * (ff / 4), mine = 0x0001000100010001ull << ((T - 1) & 15);
+        for (int w = threadIdx.x; w < ff / 4; w += 1024) n += __popcll(tile[w] & mine);
+    } else {
+        const float * row = logits + (size_t)(T - 1) * ff;
+        for (int c = threadIdx.x; c < ff; c += 1024) n += !(row[c] < thr);
+    }
+    n = (int)pi_wave_sum((float)n);                                      // (whole numbers below 2^24)
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x) return;
+    for (int w = 1; w < 16; ++w) n += part[w];
+    *n_active = n;
+}
+
 // out[c][r] = in[r][c] for an fp16 matrix [rows][cols] (32 x 32 tiles through LDS)
 __global__ void transpose_f16_kernel(const __half * __restrict__ in, int rows, int cols, __half * __restrict__ out) {
     __shared__ __half t[32][33];
@@ -1423,6 +1442,14 @@ static int gemm_tile_launch(const void * W, int rows, int cols, const void * xn_
 #undef PI_GEMM_TILE
     return pi::check_launch("pi_k_gemm_tile");
 }
+
+namespace pi {
+int count_active(const float * logits, const void * mask, int T, int ff, float thr, int32_t * n_active, pi_stream_t stream) {
+    if ((!logits && !mask) || !n_active || T <= 0 || ff <= 0 || (mask && ff % 16)) return fail(PI_E_ARG, "count_active: bad arguments");
+    hipLaunchKernelGGL(count_active_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, logits, (const unsigned long long *)mask, T, ff, thr, n_active);
+    return check_launch("count_active");
+}
+}  // namespace pi
 
 // logits or mask, not both
 static int ffn_wide(const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, const float * logits, const unsigned long long * mask, float threshold, void * h_f16,

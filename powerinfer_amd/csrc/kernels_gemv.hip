@@ -89,6 +89,11 @@ __device__ __forceinline__ int32_t start_token(const int32_t * token, const Toke
     if (blockIdx.x == 0 && threadIdx.x == 0) { *s.d_token = s.token; *s.d_pos = s.pos; *s.d_step = 0; }
     return s.token;
 }
+__global__ void resume_token_kernel(const float * __restrict__ row, int cols, TokenStart start, float * __restrict__ x) {
+    start_token(nullptr, start);
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < cols) x[c] = row[c];
+}
 // The embedding row a mat-vec takes as its input: what a token begins with is no launch of its own where the first layer's q|k|v reads the row itself
 // and its first workgroup leaves it in fp32 for the residual (and the state, see TokenStart).
 struct EmbedRow { const void * table; const int32_t * token; TokenStart start; float * x; };
@@ -939,6 +944,11 @@ namespace pi {
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream) {
     if (!table || !d_token || !d_pos || !d_step || !x || cols <= 0) return fail(PI_E_ARG, "embed_start: bad arguments");
     return embed_one(wtype, table, cols, nullptr, TokenStart{token, pos, d_token, d_pos, d_step}, x, (hipStream_t)stream);
+}
+int resume_token(const float * row, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream) {
+    if (!row || !d_token || !d_pos || !d_step || !x || cols <= 0) return fail(PI_E_ARG, "resume_token: bad arguments");
+    hipLaunchKernelGGL(resume_token_kernel, dim3((cols + 255) / 256), dim3(256), 0, (hipStream_t)stream, row, cols, TokenStart{token, pos, d_token, d_pos, d_step}, x);
+    return check_launch("resume_token");
 }
 int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream) {
     const bool q4 = wtype == PI_TYPE_Q4_0;

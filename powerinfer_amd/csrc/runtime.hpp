@@ -68,6 +68,10 @@ int expert_relu2_step(const void * up, int n_expert, int ff, int cols, const voi
                       pi_stream_t stream);
 // the embedding row of a token that the host names; also writes the token loop's state (token, position, step counter 0)
 int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
+// where a prompt's last token goes on alone behind a chunk that it came along in: its input of the next layer, and the loop's state as embed_start leaves it
+int resume_token(const float * row, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
+// how many neurons of a chunk's last token (T of them) fire, by the predictor's logits [T][ff] or its bits (pi_k_ffn_wide_predicted_f16)
+int count_active(const float * logits, const void * mask, int T, int ff, float thr, int32_t * n_active, pi_stream_t stream);
 // the embedding rows of tokens that the host names, at positions from `pos` on, and these positions
 int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream);
 
