@@ -4,6 +4,19 @@
 
 namespace {
 
+// Sixteen rows by 32 columns of an operand that lies column by column in LDS, 512 bytes (256 rows) each: the matrix cores want eight consecutive columns of
+// one row in a lane, which ds_read_b64_tr_b16 turns out of four columns of sixteen rows at a time.  A column's 32-byte pieces are stored at
+// piece ^ turned_key(column): the eight columns that half a wave reads the same piece of fall on different banks.
+__device__ __forceinline__ int turned_key(int column) { return (column & 3) | (column >> 3 & 1) << 2; }
+__device__ __forceinline__ pi_u32x4 turned_fragment(const unsigned char * p) {
+    typedef short s4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s4 * ptr;
+    union { s4 half[2]; pi_u32x4 whole; } f;
+    f.half[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)p);
+    f.half[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ptr)(p + 4 * 512));
+    return f.whole;
+}
+
 // ---------------------------------------------------------------------------------------------------------------------------------
 // One workgroup per compute unit that stays for all of its units.  Four waves multiply (128 x 64 outputs each), four copy: a stage of 64
 // columns goes from memory straight to LDS, three stages deep and on into the next unit, and a copy that has to wait for the
@@ -62,39 +75,63 @@ struct WidePlace { int grp, lo, n, row0, rows; };       // of a unit: group, fir
 // P (a product): nk stages of 64 columns; place(deal, c); base_a(p, w), base_b(p): where the rows of a tile's w-th 64 rows and its tokens start, and
 // off_a(p, r), off_b(p, r): the bytes from there to tile row and token r (in range: r is cut to the unit's); kPairs: a wave's rows
 // are two runs of MT / 2 tiles, `gap` rows apart beyond their own where MT is 4; read_once(p): no other unit reads these rows of W; first(p): the column stage a unit begins with, which may depend on nothing
-// but its group and rows; kM, kN: the tile; store<MT>(p, rb, tb, acc, turn, lane): the
+// but its group and rows; kM, kN: the tile; kList: a tile's rows are not consecutive: entry(p, w, lane) says which the w-th 64 are and off_entry where
+// one starts; kTurned: W lies with its rows along the contiguous dimension, and the column of it that a product's column c is stands in turned[c]
+// (col_bytes from one to the next, base_a(p, w) is the tile's place in column 0; M 256, columns multiples of 64), and a unit may have a part of the stages: stages(p)
+// of them from first(p) on; store<MT>(p, rb, tb, acc, turn, lane): the
 // outputs of rows rb .. and tokens tb .. of the tile.
-template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(const P & prod, const WideDeal & deal, unsigned char * smem) {
+template <typename EL, typename P, typename D> __device__ __forceinline__ void gemm_wide(const P & prod, const D & deal, unsigned char * smem) {
     if (deal.count == 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, i = lane & 15, q = lane >> 4;
     constexpr int M = P::kM, N = P::kN, CA = M / 32, CB = N / 32;   // rows and tokens of a tile, copies of a wave a stage (twelve)
     static_assert(CA + CB == 12, "the waits below count them");
-    const int nk = prod.nk, count = deal.count;
+    const int count = deal.count;
+    const auto stages = [&](const WidePlace & p) { if constexpr (P::kTurned) return prod.stages(p); else return prod.nk; };
     WidePlace * places = reinterpret_cast<WidePlace *>(smem + kGwStages * kGwStage);      // of this unit and those behind it, written by the first copying wave
     if (wave >= 4) {
         // A wave that copies.  Of each stage CA times eight rows of W and CB times eight of x are its own, each 128 bytes; lane l brings
         // the piece that belongs at place l % 8 of row l / 8
         const int w = wave - 4, piece = ((lane & 7) ^ (lane >> 3)) * 16;
-        uint32_t va[CA];
+        uint32_t va[CA];                                            // (kTurned: the pieces of a column, by two bits of its number)
         size_t vb[CB];
         const unsigned char * fa, * fb;
-        int k = 0, c = 0, first = 0;                                // a unit's stages are copied from column stage `first` on, around the end
+        int k = 0, c = 0, first = 0, nk = prod.nk;                                // a unit's stages are copied from column stage `first` on, around the end
         bool once = false;
+        int entry = 0;
+        if constexpr (P::kList) { static_assert(M == 256, "a wave's entries are 64"); entry = prod.entry(prod.place(deal, 0), w, lane); }
         auto aim = [&]() {
             const WidePlace p = prod.place(deal, c);
             if (w == 0 && lane == 0) places[c & 3] = p;
             ++c;
-            fa = prod.base_a(p, w); fb = prod.base_b(p); once = prod.read_once(p); first = prod.first(p);
+            fa = prod.base_a(p, w); fb = prod.base_b(p); once = prod.read_once(p); first = prod.first(p); nk = stages(p);
+            if constexpr (P::kList) {
 #pragma unroll
-            for (int j = 0; j < CA; ++j) va[j] = prod.off_a(p, min(8 * CA * w + 8 * j + (lane >> 3), p.rows - 1)) + piece;
+                for (int j = 0; j < CA; ++j) va[j] = prod.off_entry(__shfl(entry, 8 * j + (lane >> 3))) + piece;
+                entry = prod.entry(prod.place(deal, min(c, count - 1)), w, lane);      // a unit ahead: nothing waits for them but what is older anyway
+            } else if constexpr (P::kTurned) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) va[j] = min(((lane >> 1 & 15) ^ turned_key(2 * (j & 1) + 8 * (j >> 1) + (lane >> 5))) * 32 + (lane & 1) * 16, p.rows * 2 - 16);
+            } else {
+#pragma unroll
+                for (int j = 0; j < CA; ++j) va[j] = prod.off_a(p, min(8 * CA * w + 8 * j + (lane >> 3), p.rows - 1)) + piece;
+            }
 #pragma unroll
             for (int j = 0; j < CB; ++j) vb[j] = prod.off_b(p, min(8 * CB * w + 8 * j + (lane >> 3), p.n - 1)) + piece;
         };
         typedef const __attribute__((address_space(1))) void * gptr;
         typedef __attribute__((address_space(3))) void * lptr;
         auto copy_stage = [&](unsigned char * stage) {             // past the last unit the last stage is copied again, and not used
-            const size_t at = (size_t)(first + k < nk ? first + k : first + k - nk) * kGtRow;
-            if (once) {                                            // (the last operand of the builtin: 2 is the non-temporal hint)
+            const int ks = P::kTurned || first + k < nk ? first + k : first + k - nk;
+            const size_t at = (size_t)ks * kGtRow;
+            if constexpr (P::kTurned) {                            // columns 16 w .. of the stage, two a copy
+                typedef const __attribute__((address_space(4))) int32_t * sptr;
+                const sptr list = (sptr)(prod.turned + ks * kGtBK + 16 * w);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t o0 = (uint32_t)list[2 * j] * prod.col_bytes, o1 = (uint32_t)list[2 * j + 1] * prod.col_bytes;
+                    __builtin_amdgcn_global_load_lds((gptr)(fa + ((lane & 32 ? o1 : o0) + va[(j & 1) | (j >> 2) << 1])), (lptr)(stage + (16 * w + 2 * j) * 512), 16, 0, 0);
+                }
+            } else if (once) {                                            // (the last operand of the builtin: 2 is the non-temporal hint)
 #pragma unroll
                 for (int j = 0; j < CA; ++j) __builtin_amdgcn_global_load_lds((gptr)(fa + at + va[j]), (lptr)(stage + 8 * (CA * w + j) * kGtRow), 16, 0, 2);
             } else {
@@ -106,7 +143,8 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
             if (++k < nk) return;
             if (c < count) { k = 0; aim(); } else k = nk - 1;
         };
-        const int total = count * nk;
+        int total = count * nk;
+        if constexpr (P::kTurned) { total = 0; for (int u = 0; u < count; ++u) total += stages(prod.place(deal, u)); }
         aim();
         for (int st = 0; st < kGwStages; ++st) copy_stage(smem + st * kGwStage);
         __builtin_amdgcn_s_waitcnt(0x4078);                         // vmcnt(24): the first stage; lgkmcnt(0): its place
@@ -128,6 +166,7 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
     asm volatile("" ::: "memory");
     const int koff[2] = {(q ^ (i & 7)) * 16, ((4 + q) ^ (i & 7)) * 16};
     auto run = [&](auto mt, const WidePlace & p, int rb, int tb) {  // rows rb .. and tokens tb .. of the tile are this wave's
+        const int nk = stages(p);
         constexpr int MT = decltype(mt)::value, kGap = P::kPairs && MT == 4 ? 32 : 0;
         pi_f4 acc[MT][4];
 #pragma unroll
@@ -136,8 +175,12 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
             for (int n = 0; n < 4; ++n) acc[m][n] = pi_f4{0.0f, 0.0f, 0.0f, 0.0f};
         pi_u32x4 f0a[MT], f0b[4], f1a[MT], f1b[4];
         const int oa = (rb + i) * kGtRow, ob = (M + tb + i) * kGtRow;
+        const int ot = (8 * q + (i >> 2)) * 512 + (i & 3) * 8, key = turned_key(8 * q + (i >> 2));
         auto ld = [&](int off) { return *reinterpret_cast<const pi_u32x4 *>(smem + cb * kGwStage + off); };
-        auto lda = [&](int m, int h) { return ld(oa + koff[h] + (m * 16 + (m >= MT / 2 ? kGap : 0)) * kGtRow); };
+        auto lda = [&](int m, int h) {
+            if constexpr (P::kTurned) return turned_fragment(smem + cb * kGwStage + ot + h * 32 * 512 + ((rb / 16 + m) ^ key) * 32);
+            else return ld(oa + koff[h] + (m * 16 + (m >= MT / 2 ? kGap : 0)) * kGtRow);
+        };
         auto ldb = [&](int n, int h) { return ld(ob + koff[h] + n * 16 * kGtRow); };
 #pragma unroll
         for (int m = 0; m < MT; ++m) f0a[m] = lda(m, 0);
@@ -184,8 +227,8 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
         }
         prod.template store<MT>(p, rb, tb, acc, turn, lane);
     };
-    auto idle = [&]() {                                             // no tokens of this tile
-        for (int kt = 0; kt < nk; ++kt) {
+    auto idle = [&](const WidePlace & p) {                          // no tokens of this tile
+        for (int kt = 0, nk = stages(p); kt < nk; ++kt) {
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             cb = cb == kGwStages - 1 ? 0 : cb + 1;
@@ -201,7 +244,7 @@ template <typename EL, typename P> __device__ __forceinline__ void gemm_wide(con
         if constexpr (M == 128) {
             const bool half = p.rows <= 64, pairs = !half && p.n <= 128;
             const int tb = pairs ? 64 * (wave >> 1) : 64 * wave;
-            if (tb >= p.n) idle();
+            if (tb >= p.n) idle(p);
             else if (half || pairs) run(std::integral_constant<int, 4>{}, p, pairs ? 64 * (wave & 1) : 0, tb);
             else run(std::integral_constant<int, 8>{}, p, 0, tb);
         } else if (p.rows <= 128) run(std::integral_constant<int, 4>{}, p, kStep * (wave & 1), 64 * (wave >> 1));

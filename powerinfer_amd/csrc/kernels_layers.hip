@@ -639,7 +639,7 @@ constexpr long long kGwValues = 1LL << 31;                          // of a grou
 // read once, and by one workgroup.  64 experts, both products, us, tiles of 128 / 256 tokens: 192 tokens an expert on average 407 -> 390 (1408 x 4096), 624 -> 585
 // (with a gate); 8 experts of 140, 4096 x 4096 with a gate 245 -> 176; of 96 tokens 290 and 334.
 template <int M, int N, bool LIST> struct GroupProduct {
-    static constexpr bool kPairs = false;
+    static constexpr bool kPairs = false, kList = false, kTurned = false;
     static constexpr int kM = M, kN = N;
     const pi_group_gemm & g;
     int nk, tt;                                                     // tt: token tiles of a group without a list

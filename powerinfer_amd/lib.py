@@ -187,6 +187,9 @@ _SIGS = {
     "pi_k_gemm_tile_bf16": (_i, [_vp, _i, _i, _vp, _i, _i, _vp, _vp, _vp, _vp, _i, _vp]),
     "pi_k_ffn_wide_supported": (_i, [_i, _i]),
     "pi_k_ffn_wide_f16": (_i, [_vp, _vp, _i, _i, _vp, _i, _vp, _f, _vp, _vp]),
+    "pi_k_ffn_union_supported": (_i, [_i, _i, _i]),
+    "pi_k_ffn_union_scratch": (C.c_size_t, [_i, _i]),
+    "pi_k_ffn_union_f16": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, _i, _f, _vp, _vp, C.POINTER(_vp), _vp, _vp, _vp, _vp, _vp]),
     "pi_k_ffn_wide_predicted_f16": (_i, [_vp, _i, _vp, _vp, _vp, _i, _i, _vp, _i, _f, _vp, _vp, _vp]),
     "pi_k_ffn_h_f16": (_i, [_vp, _vp, _vp, _f, _i, _i, _vp, _vp]),
     "pi_k_transpose_f16": (_i, [_vp, _i, _i, _vp, _vp]),
