@@ -198,6 +198,17 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
     float * x = m->x;
 
     const bool branch = ffn_beside(m, il);
+    const pi_norm an = attn_norm(m, il);
+    if (branch && m->rope_table && pi::attn_ffn_supported(ff, r, d, hd, hp.n_ctx, m->attn_parts) && pi::gemv_pair_supported(wqkv.type, fc1.type, d, &an, x)) {
+        const pi_norm fnb = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
+        PI_TRY(pi::gemv_pair(wqkv.dev, d + 2 * gqa, &an, m->qkv, fc1.dev, r, m->hidden, d, x, st));
+        const pi::DecodeAttn a{m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, 2, hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, m->attn_arrived};
+        PI_TRY(pi::attn_ffn(a, fc2.dev, ff, r, m->hidden, hp.sparse_threshold, up.dev, down.dev, d, x, &fnb, m->ws, st));
+        PI_TRY(pi_k_gemv(wo.type, wo.dev, d, d, m->att, nullptr, PI_EPI_NONE, nullptr, nullptr, m->attn_out, st));
+        PI_TRY(pi_k_sparse_ffn_reduce(ff, d, PI_EPI_ADD2, m->attn_out, x, m->x2, n_act, m->ws, st));
+        std::swap(m->x, m->x2);
+        return PI_OK;
+    }
     if (branch) {
         pi_norm fnb = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         PI_HIP_TRY(hipEventRecord(m->ev_fork[il], st));
@@ -219,7 +230,6 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
     }
 
     // attention
-    const pi_norm an = attn_norm(m, il);
     if (start) {
         const Tensor & table = m->glob[PI_T_TOK_EMBD];
         PI_TRY(pi_k_first_gemv(table.type, table.dev, start->id < 0 ? m->d_token : nullptr, start->id, start->pos, m->d_token, m->d_pos, m->d_step, wqkv.dev, d + 2 * gqa, d, &an, x,
@@ -806,7 +816,9 @@ int pi_model_finalize(pi_model * m) {
         if (pi_k_attn_split_supported(m->hd, hp.n_ctx, parts)) {
             m->attn_parts = parts;
             m->attn_scratch = m->alloc<float>(pi_k_attn_split_scratch_floats(1, hp.n_head, m->hd, parts));
-            if (!m->attn_scratch) return PI_E_HIP;
+            m->attn_arrived = m->alloc<uint32_t>(hp.n_head);
+            if (!m->attn_scratch || !m->attn_arrived) return PI_E_HIP;
+            PI_TRY(pi_memset(m->attn_arrived, 0, 4 * (size_t)hp.n_head));
         }
     }
     if (fused_ok || m->attn_parts > 1) {

@@ -1,7 +1,7 @@
 // The sparse FFN of one token as one launch plus a reduction (F16: one workgroup per compute unit or per 32 neurons; Q4_0: per 32
 // neurons, one Q8_0 block of h), the two-phase forms of hybrid layers with their hand-over kernels, and the entry point that allocates
 // nothing.
-#include "kernels_common.hpp"
+#include "attn_decode.hpp"
 
 namespace {
 
@@ -34,8 +34,9 @@ constexpr int kPfChunk = 8;                       // active neurons per round tr
 // a hand-over to the host announced by the first lane of a launch (see host_signal_kernel): device counter and word 0 of the pinned flags
 struct HostAnnounce { uint32_t * seq; uint32_t * flags; uint32_t * words_out = nullptr; };    // words_out: a second copy of the activity words (pinned memory) for the logits-only launch
 
+template <int RCH> constexpr int kPfRowsLds = kPfWaves * 4 * RCH * 1024;
 template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
-__global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half * __restrict__ W2, const float * __restrict__ hidden,
+__device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, const float * __restrict__ hidden,
                                                                    const __half * __restrict__ Wup, const __half * __restrict__ Wgate,
                                                                    const __half * __restrict__ Wdown,
                                                                    const float * __restrict__ x, NormArgs na, float thr,
@@ -43,9 +44,9 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
                                                                    float * __restrict__ partial,
                                                                    const uint32_t * __restrict__ hot_words, const int32_t * __restrict__ hot_prefix,
                                                                    uint32_t * __restrict__ words_hot, __half * __restrict__ xn_out,
-                                                                   float * __restrict__ logits2, HostAnnounce ann) {
+                                                                   float * __restrict__ logits2, HostAnnounce ann, const int blk, unsigned char * rows_lds) {
     static_assert(PHASE == 0 || G == 1, "the two-phase form takes one group per workgroup");
-    if (PHASE == 2 && ann.flags && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (PHASE == 2 && ann.flags && blk == 0 && threadIdx.x == 0) {
         // what was queued before this launch is complete and visible to the host: a new hand-over starts here, without a launch of its own
         const uint32_t sq = *ann.seq + 1u;
         *ann.seq = sq;
@@ -57,18 +58,32 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
     __shared__ double red[2][kPfWaves];
     __shared__ float  part[kPfWaves][CH][2];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int n0 = blockIdx.x * 32 * G;
+    int n0 = blk * 32 * G;
     const int cbase = wave * CPW * 512 + lane * 8;     // chunk c of this lane starts at column cbase + 512*c
 
     // ---- A: loads ------------------------------------------------------------------------------------------
+    // Several groups: a group's predictor rows go to LDS (rows_lds, kPfRowsLds<RCH> bytes; a wave reads only what it requested), and the next group's travel while this group's
+    // FFN rows are fetched and used.  In registers they would leave a unit no room for other workgroups beside this one.
+    const auto request = [&](int first) {
+        typedef const __attribute__((address_space(1))) void * gptr;
+        typedef __attribute__((address_space(3))) void * lptr;
+        const int w = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < RCH; ++j)
+                __builtin_amdgcn_global_load_lds((gptr)(W2 + (size_t)(first + w * 4 + i) * r + (j * PI_WAVE + lane) * 8), (lptr)(rows_lds + ((w * 4 + i) * RCH + j) * 1024), 16, 0, 2);
+    };
     pi_u32x4 a[4][RCH];
     float4 hv[RCH][2];
     float logit_in = 0.0f;
     if (PHASE != 2) {
+        if constexpr (G > 1) request(n0);
+        else
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(n0 + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
+                for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(n0 + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
 #pragma unroll
         for (int j = 0; j < RCH; ++j) {
             hv[j][0] = *reinterpret_cast<const float4 *>(hidden + j * 512 + lane * 8);
@@ -101,20 +116,16 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
                              __floats2half2_rn(hv[j][1].x, hv[j][1].y), __floats2half2_rn(hv[j][1].z, hv[j][1].w)};
             hr[j] = *reinterpret_cast<const pi_u32x4 *>(hh);
         }
+        if constexpr (G == 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float acc = 0.0f;
+            for (int i = 0; i < 4; ++i) {
+                float acc = 0.0f;
 #pragma unroll
-            for (int j = 0; j < RCH; ++j) acc = pi_dot8h(a[i][j], hr[j], acc);
-            acc = pi_wave_sum(acc);
-            if (lane == 0) lg[0][wave * 4 + i] = acc;
+                for (int j = 0; j < RCH; ++j) acc = pi_dot8h(a[i][j], hr[j], acc);
+                acc = pi_wave_sum(acc);
+                if (lane == 0) lg[0][wave * 4 + i] = acc;
+            }
         }
-    }
-    if (G > 1) {       // the next group's predictor rows travel while this group's FFN rows are fetched and used
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(n0 + 32 + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
     }
     // ---- A: norm statistics across the 8 slices ---------------------------------------------------------------
     float mean = 0.0f, scale = 1.0f;
@@ -175,7 +186,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
         __half2 hh[4] = {__floats2half2_rn(xs[c][0], xs[c][1]), __floats2half2_rn(xs[c][2], xs[c][3]),
                          __floats2half2_rn(xs[c][4], xs[c][5]), __floats2half2_rn(xs[c][6], xs[c][7])};
         xr[c] = *reinterpret_cast<const pi_u32x4 *>(hh);
-        if (HYB && blockIdx.x == 0 && xn_out) *reinterpret_cast<pi_u32x4 *>(xn_out + cbase + c * 512) = xr[c];
+        if (HYB && blk == 0 && xn_out) *reinterpret_cast<pi_u32x4 *>(xn_out + cbase + c * 512) = xr[c];
     }
     float acc[CPW][8];
 #pragma unroll
@@ -184,29 +195,29 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
         for (int k = 0; k < 8; ++k) acc[c][k] = 0.0f;
 #pragma unroll 1
     for (int g = 0; g < G; ++g, n0 += 32) {
-    if (g > 0) {
+    if constexpr (G > 1) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0): the rows have arrived (what was requested behind them has been used)
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float lacc = 0.0f;
 #pragma unroll
-            for (int j = 0; j < RCH; ++j) lacc = pi_dot8h(a[i][j], hr[j], lacc);
+            for (int j = 0; j < RCH; ++j) lacc = pi_dot8h(*reinterpret_cast<const pi_u32x4 *>(rows_lds + ((wave * 4 + i) * RCH + j) * 1024 + lane * 16), hr[j], lacc);
             lacc = pi_wave_sum(lacc);
             if (lane == 0) lg[g & 1][wave * 4 + i] = lacc;
         }
-        if (g + 1 < G) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(n0 + 32 + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
-        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);                             // lgkmcnt(0): read, before the next ones come
+        asm volatile("" ::: "memory");
+        if (g + 1 < G) request(n0 + 32);
         __syncthreads();
     }
     // ---- activity word (identical in every wave; lg[g & 1] is complete after the barrier above) ----------------
     const float my_logit = PHASE == 2 ? logit_in : lg[g & 1][lane & 31];
     const bool my_act = !(my_logit < thr);
     const uint32_t all = (uint32_t)__ballot(my_act);
-    const uint32_t hot = HYB ? hot_words[blockIdx.x * G + g] : 0xFFFFFFFFu;
-    const int base_row = HYB ? hot_prefix[blockIdx.x * G + g] : n0;
+    const uint32_t hot = HYB ? hot_words[blk * G + g] : 0xFFFFFFFFu;
+    const int base_row = HYB ? hot_prefix[blk * G + g] : n0;
     const uint32_t mask = all & hot;
     if (wave == 0) {
         if (lane < 32) {
@@ -214,7 +225,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
             if (PHASE == 1) logits2[n0 + lane] = my_logit;
             if (PHASE != 1 && h_dense && !((mask >> lane) & 1u)) h_dense[n0 + lane] = 0.0f;
         }
-        if (lane == 0) { words[blockIdx.x * G + g] = all; if (HYB) words_hot[blockIdx.x * G + g] = mask; if (PHASE == 1 && ann.words_out) ann.words_out[blockIdx.x * G + g] = all; }
+        if (lane == 0) { words[blk * G + g] = all; if (HYB) words_hot[blk * G + g] = mask; if (PHASE == 1 && ann.words_out) ann.words_out[blk * G + g] = all; }
     }
     if (PHASE == 1) return;
     // ---- B + C ---------------------------------------------------------------------------------------------
@@ -272,10 +283,62 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
     }   // groups: the barrier behind the next group's logits also orders this group's last reads of part[] and lg[]
 #pragma unroll
     for (int c = 0; c < CPW; ++c) {
-        float4 * po = reinterpret_cast<float4 *>(partial + (size_t)blockIdx.x * cols + cbase + c * 512);
+        float4 * po = reinterpret_cast<float4 *>(partial + (size_t)blk * cols + cbase + c * 512);
         po[0] = make_float4(acc[c][0], acc[c][1], acc[c][2], acc[c][3]);
         po[1] = make_float4(acc[c][4], acc[c][5], acc[c][6], acc[c][7]);
     }
+}
+
+template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
+__global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half * __restrict__ W2, const float * __restrict__ hidden,
+                                                                   const __half * __restrict__ Wup, const __half * __restrict__ Wgate,
+                                                                   const __half * __restrict__ Wdown,
+                                                                   const float * __restrict__ x, NormArgs na, float thr,
+                                                                   float * __restrict__ logits, uint32_t * __restrict__ words, float * __restrict__ h_dense,
+                                                                   float * __restrict__ partial,
+                                                                   const uint32_t * __restrict__ hot_words, const int32_t * __restrict__ hot_prefix,
+                                                                   uint32_t * __restrict__ words_hot, __half * __restrict__ xn_out,
+                                                                   float * __restrict__ logits2, HostAnnounce ann) {
+    __shared__ __align__(16) unsigned char rows[G > 1 ? kPfRowsLds<RCH> : 16];
+    pred_ffn_groups<CPW, RCH, GATE, G, HYB, PHASE>(W2, hidden, Wup, Wgate, Wdown, x, na, thr, logits, words, h_dense, partial, hot_words, hot_prefix, words_hot, xn_out, logits2, ann, blockIdx.x, rows);
+}
+
+// Falcon's attention and FFN both read the layer's input: the attention's workgroups and the FFN's in one launch (F16, 8192 columns, four groups of 32 neurons a workgroup),
+// behind one that has q|k|v and the predictor's hidden units (gemv_pair_f16_reg_kernel).  The FFN is bound by what a unit pulls (174 MB of predictor and active rows in 35 us),
+// the attention by its chain of round trips: two workgroups fit a unit (128 registers, the predictor's rows in LDS), so that the one runs beside the other.
+// On two streams, the events of a fork and a join kept ~8 us each on the path.  Falcon-40B (128 heads of 64), 40 us a layer at 100 cells as at 1024 and 3000; a run of 8 tokens
+// 4 layers deep 5000 -> 4780 us at 100 cells and 5000 -> 4690 at 1024, 3 layers deep 4230 -> 4015 at 900, 4360 -> 4055 at 3000, 4860 -> 4700 at 12000.
+// PARTS: cells split (attn_part_kernel's workgroups), and the last one of a head merges, beside the FFN (a launch of its own: 4780 us at 1024 cells, 4140 at 3000).  They are hundreds,
+// which ahead of the FFN's would take both places of a unit (4905 -> 4820 us behind them, with the merge apart); a workgroup a head comes first (behind: 4800 -> 4855 at 100 cells).
+template <int RCH, int LPP, bool PARTS>
+__global__ __launch_bounds__(kPfBlock, 4) void attn_ffn_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table, __half * __restrict__ k_cache, __half * __restrict__ v_cache,
+                                                               int n_head, int n_head_kv, int hd, int mode, int n_ctx, int s_cap, int n_parts, const int32_t * __restrict__ pos_p,
+                                                               float * __restrict__ out, float * __restrict__ part_acc, float * __restrict__ part_ml, uint32_t * __restrict__ arrived,
+                                                               const __half * __restrict__ W2, const float * __restrict__ hidden, const __half * __restrict__ Wup, const __half * __restrict__ Wdown,
+                                                               const float * __restrict__ x, NormArgs na, float thr, uint32_t * __restrict__ words, float * __restrict__ partial) {
+    static_assert(kPfBlock == kAttnPartBlock, "one size of workgroup");
+    extern __shared__ __align__(16) unsigned char smem[];              // the attention's, or the FFN's predictor rows: two workgroups a unit
+    const int n_attn = n_head * (PARTS ? n_parts : 1), n_ffn = (int)gridDim.x - n_attn;
+    const int b = !PARTS ? (int)blockIdx.x : (int)blockIdx.x < n_ffn ? n_attn + (int)blockIdx.x : (int)blockIdx.x - n_ffn;
+    if (b < n_attn) {
+        if constexpr (PARTS) {
+            __shared__ int last;
+            const int h = b % n_head;
+            attn_part_head<false, LPP, true>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, s_cap, pos_p, part_acc, part_ml, 0, 0, h, b / n_head, n_parts, 0);
+            // Every wave waits for its own stores (past the caches of its die) to have arrived before the workgroup counts itself; the head's last workgroup merges.  The count
+            // is relaxed: release and acquire would write back and drop the die's L2 under the FFN's rows (40.5 -> 51.7 us a launch).
+            __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0)
+            __syncthreads();
+            if (threadIdx.x == 0) last = __hip_atomic_fetch_add(arrived + h, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (unsigned)n_parts;
+            __syncthreads();
+            if (!last) return;
+            if ((int)threadIdx.x < hd) out[(size_t)h * hd + threadIdx.x] = attn_merge_value<true>(part_acc, part_ml, n_parts, hd, (size_t)h * n_parts, threadIdx.x);
+            if (threadIdx.x == 0) __hip_atomic_store(arrived + h, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else
+            attn_fused_head<kPfBlock, LPP>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos_p, out, 0, 0, 0, nullptr, 0, nullptr, nullptr, nullptr, b, 0);
+        return;
+    }
+    pred_ffn_groups<2, RCH, false, 4, false>(W2, hidden, Wup, nullptr, Wdown, x, na, thr, nullptr, words, nullptr, partial, nullptr, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, b - n_attn, smem);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1272,6 +1335,42 @@ static int sparse_ffn_partials_impl(const char * who, const void * fc2_f16, int 
 #undef PI_PF_LAUNCH2
     return pi::check_launch(who);
 }
+
+}  // extern "C"
+namespace pi {
+bool attn_ffn_supported(int ff, int r, int cols, int hd, int n_ctx, int n_parts) {
+    return cols == 8192 && (r == 512 || r == 1024) && pf_grouped_shape(ff, r, cols) && pf_groups(ff, cols) == 4 && (hd == 64 || hd == 128) &&
+           (n_parts > 1 ? pi_k_attn_split_supported(hd, n_ctx, n_parts) : pi_k_attn_fused_supported(hd, n_ctx) != 0);
+}
+int attn_ffn(const DecodeAttn & a, const void * fc2_f16, int ff, int r, const float * hidden, float threshold, const void * up_f16, const void * down_t_f16, int cols, const float * x, const pi_norm * norm,
+             pi_workspace * ws, pi_stream_t stream) {
+    if (!a.qkv || !a.rope_table || !a.k_cache || !a.v_cache || !a.pos || !a.out || (a.n_parts > 1 && (!a.scratch || !a.arrived)) || !fc2_f16 || !hidden || !up_f16 || !down_t_f16 || !x || !ws)
+        return fail(PI_E_ARG, "attn_ffn: null pointer");
+    if (a.n_head <= 0 || a.n_head_kv <= 0 || a.n_head % a.n_head_kv || (a.mode != 0 && a.mode != 2) || !attn_ffn_supported(ff, r, cols, a.hd, a.n_ctx, a.n_parts) || ff > ws->max_ff || cols > ws->max_d)
+        return fail(PI_E_UNSUPPORTED, "attn_ffn: shape outside the kernel");
+    const NormArgs na = to_norm(norm);
+    if ((((uintptr_t)hidden | (uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b) & 15) != 0) return fail(PI_E_ARG, "attn_ffn: vectors must be 16-byte aligned");
+    ws->pf_parts = ff / 128; ws->pf_words = ff / 32;
+    const bool parts = a.n_parts > 1;
+    const int s_cap = (a.n_ctx + a.n_parts - 1) / a.n_parts + 1;
+    float * ml = parts ? a.scratch + (size_t)a.n_head * a.n_parts * a.hd : nullptr;
+    const size_t lds = std::max(parts ? attn_part_lds(a.hd, s_cap) : attn_fused_lds_bytes(a.hd, a.n_ctx, kPfBlock), (size_t)kPfRowsLds<1> * (r / 512));
+    const dim3 grid(a.n_head * (parts ? a.n_parts : 1) + ws->pf_parts);
+#define PI_AF(RCH, LPP, PARTS) do { \
+        static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_ffn_kernel<RCH, LPP, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024); \
+        if (raised != hipSuccess) return hip_fail(raised, "attn_ffn: LDS size"); \
+        hipLaunchKernelGGL((attn_ffn_kernel<RCH, LPP, PARTS>), grid, dim3(kPfBlock), lds, (hipStream_t)stream, a.qkv, (const float2 *)a.rope_table, (__half *)a.k_cache, (__half *)a.v_cache, \
+            a.n_head, a.n_head_kv, a.hd, a.mode, a.n_ctx, s_cap, a.n_parts, a.pos, a.out, a.scratch, ml, a.arrived, (const __half *)fc2_f16, hidden, (const __half *)up_f16, (const __half *)down_t_f16, x, na, threshold, ws->words, ws->ffn_partial); \
+    } while (0)
+#define PI_AF_P(RCH, LPP) do { if (parts) PI_AF(RCH, LPP, true); else PI_AF(RCH, LPP, false); } while (0)
+    if (r == 1024) { if (a.hd == 64) PI_AF_P(2, 8); else PI_AF_P(2, 16); }
+    else           { if (a.hd == 64) PI_AF_P(1, 8); else PI_AF_P(1, 16); }
+#undef PI_AF_P
+#undef PI_AF
+    return check_launch("attn_ffn");
+}
+}  // namespace pi
+extern "C" {
 
 int pi_k_sparse_ffn_partials(const void * fc2_f16, int ff, int r, const float * hidden, float threshold,
                              const void * up_f16, const void * gate_f16, const void * down_t_f16, int cols, const float * x, const pi_norm * norm,
