@@ -199,13 +199,12 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
 
     const bool branch = ffn_beside(m, il);
     const pi_norm an = attn_norm(m, il);
-    if (branch && m->rope_table && pi::attn_ffn_supported(ff, r, d, hd, hp.n_ctx, m->attn_parts) && pi::gemv_pair_supported(wqkv.type, fc1.type, d, &an, x)) {
+    if (branch && m->rope_table && pi::attn_ffn_supported(fc2.dev, ff, r, d, hd, hp.n_ctx, m->attn_parts) && wo.type == PI_TYPE_F16 && pi::gemv_pair_supported(wqkv.type, fc1.type, d, &an, x)) {
         const pi_norm fnb = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         PI_TRY(pi::gemv_pair(wqkv.dev, d + 2 * gqa, &an, m->qkv, fc1.dev, r, m->hidden, d, x, st));
         const pi::DecodeAttn a{m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, 2, hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, m->attn_arrived};
         PI_TRY(pi::attn_ffn(a, fc2.dev, ff, r, m->hidden, hp.sparse_threshold, up.dev, down.dev, d, x, &fnb, m->ws, st));
-        PI_TRY(pi_k_gemv(wo.type, wo.dev, d, d, m->att, nullptr, PI_EPI_NONE, nullptr, nullptr, m->attn_out, st));
-        PI_TRY(pi_k_sparse_ffn_reduce(ff, d, PI_EPI_ADD2, m->attn_out, x, m->x2, n_act, m->ws, st));
+        PI_TRY(pi::gemv_ffn_out(wo.dev, d, m->att, x, m->x2, n_act, m->ws, st));
         std::swap(m->x, m->x2);
         return PI_OK;
     }

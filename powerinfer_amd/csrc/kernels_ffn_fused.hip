@@ -1319,8 +1319,8 @@ static int sparse_ffn_partials_impl(const char * who, const void * fc2_f16, int 
         return pi::check_launch(who);
     }
     if (!pf_grouped_shape(ff, r, cols)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_sparse_ffn: this shape runs only with every neuron resident and a norm the kernel carries (5120 columns, rank 1280)");
-    ws->pf_parts = ff / (32 * pf_groups(ff, cols)); ws->pf_words = ff / 32;
-    const int G = pf_groups(ff, cols);
+    const int G = ((uintptr_t)fc2_f16 & 15) == 0 ? pf_groups(ff, cols) : 1;      // the copies to LDS of several groups' predictor rows want whole pieces
+    ws->pf_parts = ff / (32 * G); ws->pf_words = ff / 32;
     const dim3 grid(ff / (32 * G)), block(kPfBlock);
 #define PI_PF_LAUNCH2(CPW, RCH, GATE, GG, HYB) hipLaunchKernelGGL((pred_ffn_f16_kernel<CPW, RCH, GATE, GG, HYB>), grid, block, 0, st, w2, hidden, u, g, dn, x, na, threshold, logits, ws->words, h_dense, ws->ffn_partial, hot_words, hot_prefix, ws->words_hot, (__half *)xn_f16_out, nullptr, HostAnnounce{nullptr, nullptr})
 #define PI_PF_LAUNCH(CPW, RCH, GATE, GG) do { if (hyb) PI_PF_LAUNCH2(CPW, RCH, GATE, GG, true); else PI_PF_LAUNCH2(CPW, RCH, GATE, GG, false); } while (0)
@@ -1338,15 +1338,15 @@ static int sparse_ffn_partials_impl(const char * who, const void * fc2_f16, int 
 
 }  // extern "C"
 namespace pi {
-bool attn_ffn_supported(int ff, int r, int cols, int hd, int n_ctx, int n_parts) {
-    return cols == 8192 && (r == 512 || r == 1024) && pf_grouped_shape(ff, r, cols) && pf_groups(ff, cols) == 4 && (hd == 64 || hd == 128) &&
+bool attn_ffn_supported(const void * fc2_f16, int ff, int r, int cols, int hd, int n_ctx, int n_parts) {
+    return cols == 8192 && (r == 512 || r == 1024) && ((uintptr_t)fc2_f16 & 15) == 0 && pf_grouped_shape(ff, r, cols) && pf_groups(ff, cols) == 4 && (hd == 64 || hd == 128) &&
            (n_parts > 1 ? pi_k_attn_split_supported(hd, n_ctx, n_parts) : pi_k_attn_fused_supported(hd, n_ctx) != 0);
 }
 int attn_ffn(const DecodeAttn & a, const void * fc2_f16, int ff, int r, const float * hidden, float threshold, const void * up_f16, const void * down_t_f16, int cols, const float * x, const pi_norm * norm,
              pi_workspace * ws, pi_stream_t stream) {
     if (!a.qkv || !a.rope_table || !a.k_cache || !a.v_cache || !a.pos || !a.out || (a.n_parts > 1 && (!a.scratch || !a.arrived)) || !fc2_f16 || !hidden || !up_f16 || !down_t_f16 || !x || !ws)
         return fail(PI_E_ARG, "attn_ffn: null pointer");
-    if (a.n_head <= 0 || a.n_head_kv <= 0 || a.n_head % a.n_head_kv || (a.mode != 0 && a.mode != 2) || !attn_ffn_supported(ff, r, cols, a.hd, a.n_ctx, a.n_parts) || ff > ws->max_ff || cols > ws->max_d)
+    if (a.n_head <= 0 || a.n_head_kv <= 0 || a.n_head % a.n_head_kv || (a.mode != 0 && a.mode != 2) || !attn_ffn_supported(fc2_f16, ff, r, cols, a.hd, a.n_ctx, a.n_parts) || ff > ws->max_ff || cols > ws->max_d)
         return fail(PI_E_UNSUPPORTED, "attn_ffn: shape outside the kernel");
     const NormArgs na = to_norm(norm);
     if ((((uintptr_t)hidden | (uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b) & 15) != 0) return fail(PI_E_ARG, "attn_ffn: vectors must be 16-byte aligned");

@@ -129,11 +129,15 @@ __device__ __forceinline__ void embed_eight(const EmbedRow & e, int32_t token, i
 // MULTI: up to three matrices of the same width against the one vector in a single launch (the q, k and v projections of a host
 // that keeps them as separate tensors): row r of the launch is row r of the first matrix, or row r - rows[0] of the second, ...
 struct GemvMulti { const __half * W[3]; float * y[3]; int rows[3]; };
-template <int NCH, int KIND, bool MULTI, bool FIRST = false>
+// STRIP: a workgroup owns kStripRows neighbouring rows and adds what a sparse FFN's workgroups left for them (out = FFN + W x + residual, the sums of ffn_reduce_kernel in its
+// order).  Those vectors travel under the weights, and a launch behind this one is saved.  Workgroups with halves of a 128-byte line share a die.
+constexpr int kStripRows = 16;
+struct StripSum { const float * partial; int n_part; const uint32_t * words; int n_words; int32_t * n_active; const float * resid; };
+template <int NCH, int KIND, bool MULTI, bool FIRST = false, bool STRIP = false>
 __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W, const float * __restrict__ x,
                                                   const float * __restrict__ nw, const float * __restrict__ nb, float eps,
                                                   int epi, const float * __restrict__ add1, const float * __restrict__ add2,
-                                                  float * __restrict__ y, int rows, const GemvMulti & mm, const EmbedRow & first = {}, const int blk = blockIdx.x, const int n_blk = gridDim.x) {
+                                                  float * __restrict__ y, int rows, const GemvMulti & mm, const EmbedRow & first = {}, const int blk = blockIdx.x, const int n_blk = gridDim.x, const StripSum & strip = {}) {
     constexpr int cols = NCH * 512;
     auto row_base = [&](int r) -> const __half * {
         if (!MULTI) return W + (size_t)r * cols;
@@ -156,11 +160,13 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
     __shared__ __align__(16) __half xs[cols];
     __shared__ double red[2][kWavesPerBlock];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int n_waves = n_blk * kWavesPerBlock, wid = blk * kWavesPerBlock + wave;
+    const int first_row = STRIP ? ((blk & 7) * (n_blk >> 3) + (blk >> 3)) * kStripRows : 0;
+    const int n_waves = STRIP ? kWavesPerBlock : n_blk * kWavesPerBlock, wid = STRIP ? first_row + wave : blk * kWavesPerBlock + wave;
+    const int end = STRIP ? first_row + kStripRows : rows;
     pi_u32x4 buf[2][CPB];
     float r1[2] = {0.0f, 0.0f}, r2[2] = {0.0f, 0.0f};
     auto issue = [&](int b, int r) {
-        if (r < rows) {
+        if (r < end) {
             const __half * wp = row_base(r) + lane * 8 + (kWide ? b * CPB * 512 : 0);
 #pragma unroll
             for (int j = 0; j < CPB; ++j) buf[b][j] = pi_ld_stream(wp + j * 512);
@@ -170,6 +176,13 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
             }
         }
     };
+    constexpr int kStripSlots = 64, kStripAhead = 4;              // vectors of workgroups slot, slot + 64, ...: four lanes have a strip's columns
+    static_assert(!STRIP || kBlock == 4 * kStripSlots, "a slot is four lanes");
+    const int slot = threadIdx.x >> 2;
+    float4 ffn[STRIP ? kStripAhead : 1];
+    float resid = 0.0f;
+    int count = 0;
+    __shared__ float dots[STRIP ? kStripRows : 1], tops[STRIP ? 8 : 1][kStripRows];
     issue(0, wid);
     issue(1, kWide ? wid : wid + n_waves);
 
@@ -196,6 +209,15 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
                     bv[i][0] = c.x; bv[i][1] = c.y; bv[i][2] = c.z; bv[i][3] = c.w; bv[i][4] = e.x; bv[i][5] = e.y; bv[i][6] = e.z; bv[i][7] = e.w;
                 }
             }
+        }
+        if constexpr (STRIP) {
+#pragma unroll
+            for (int u = 0; u < kStripAhead; ++u) {
+                const int p = slot + u * kStripSlots;
+                ffn[u] = *reinterpret_cast<const float4 *>(strip.partial + (size_t)(p < strip.n_part ? p : slot) * cols + first_row + (threadIdx.x & 3) * 4);
+            }
+            if (threadIdx.x < kStripRows) resid = strip.resid[first_row + threadIdx.x];
+            if (blk == 0) for (int w = threadIdx.x; w < strip.n_words; w += kBlock) count += __popc(strip.words[w]);
         }
         float mean = 0.0f, scale = 1.0f;
         if (KIND >= 1) {
@@ -258,10 +280,11 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
         if (epi == PI_EPI_RELU) acc = fmaxf(acc, 0.0f);
         else if (epi == PI_EPI_ADD) acc = __fadd_rn(acc, a1);
         else if (epi == PI_EPI_ADD2) acc = __fadd_rn(__fadd_rn(acc, a1), a2);
-        if (lane == 0) *out_ptr(r) = acc;
+        if constexpr (STRIP) { if (lane == 0) dots[r - first_row] = acc; }
+        else if (lane == 0) *out_ptr(r) = acc;
     };
     if constexpr (kWide) {
-        for (int r = wid; r < rows; r += n_waves) {
+        for (int r = wid; r < end; r += n_waves) {
             // keep the activations packed: widening them once outside the loop would double their register footprint
 #pragma unroll
             for (int j = 0; j < NCH; ++j) asm volatile("" : "+v"(xr[j].x), "+v"(xr[j].y), "+v"(xr[j].z), "+v"(xr[j].w));
@@ -276,11 +299,11 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
             finish(acc, a1, a2, r);
         }
     } else {
-        for (int r = wid; r < rows; r += 2 * n_waves) {
+        for (int r = wid; r < end; r += 2 * n_waves) {
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const int rr = r + b * n_waves;
-                if (rr < rows) {
+                if (rr < end) {
                     float acc = 0.0f;
 #pragma unroll
                     for (int j = 0; j < NCH; ++j) acc = pi_dot8h(buf[b][j], xr[j], acc);
@@ -289,6 +312,27 @@ __device__ __forceinline__ void gemv_f16_reg_body(const __half * __restrict__ W,
                 issue(b, rr + 2 * n_waves);
             }
         }
+    }
+    if constexpr (STRIP) {
+        float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const auto add = [&](const float4 & v) { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; };
+#pragma unroll
+        for (int u = 0; u < kStripAhead; ++u) if (slot + u * kStripSlots < strip.n_part) add(ffn[u]);
+        for (int p = slot + kStripAhead * kStripSlots; p < strip.n_part; p += kStripSlots) add(*reinterpret_cast<const float4 *>(strip.partial + (size_t)p * cols + first_row + (threadIdx.x & 3) * 4));
+#pragma unroll
+        for (int o = 4; o < 32; o <<= 1) {                          // eight slots
+            sum.x += __shfl_xor(sum.x, o, PI_WAVE); sum.y += __shfl_xor(sum.y, o, PI_WAVE); sum.z += __shfl_xor(sum.z, o, PI_WAVE); sum.w += __shfl_xor(sum.w, o, PI_WAVE);
+        }
+        if ((lane & 31) < 4) *reinterpret_cast<float4 *>(&tops[wave * 2 + (lane >> 5)][(lane & 3) * 4]) = sum;
+        if (blk == 0) { count = pi_wave_sum_i32(count); if (lane == 0) red[0][wave] = count; }
+        __syncthreads();
+        if (threadIdx.x < kStripRows) {
+            float f = tops[0][threadIdx.x];
+#pragma unroll
+            for (int g = 1; g < 8; ++g) f += tops[g][threadIdx.x];
+            y[first_row + threadIdx.x] = __fadd_rn(__fadd_rn(f, dots[threadIdx.x]), resid);
+        }
+        if (blk == 0 && threadIdx.x == 0 && strip.n_active) *strip.n_active = (int)(red[0][0] + red[0][1] + red[0][2] + red[0][3]);
     }
 }
 
@@ -303,6 +347,12 @@ template <int NCH, int KIND>
 __global__ __launch_bounds__(kBlock, 2) void gemv_f16_first_kernel(const __half * __restrict__ W, EmbedRow first, const float * __restrict__ nw, const float * __restrict__ nb, float eps,
                                                                   float * __restrict__ y, int rows) {
     gemv_f16_reg_body<NCH, KIND, false, true>(W, nullptr, nw, nb, eps, PI_EPI_NONE, nullptr, nullptr, y, rows, GemvMulti{}, first);
+}
+// A mat-vec and the sums of a sparse FFN's vectors.  Bound by HBM: 134 MB of weights and 8 MB of vectors in 25.0 us (5.7 TB/s); as two launches 22.9 + 4.8 and the gap between
+// them.  Falcon-40B shapes, 8 tokens of 4 layers: 4680 -> 4620 us at 1024 cells, 4780 -> 4690 at 100.
+template <int NCH>
+__global__ __launch_bounds__(kBlock, 2) void gemv_strip_f16_kernel(const __half * __restrict__ W, const float * __restrict__ x, float * __restrict__ y, StripSum strip) {
+    gemv_f16_reg_body<NCH, 0, false, false, true>(W, x, nullptr, nullptr, 0.0f, PI_EPI_NONE, nullptr, nullptr, y, NCH * 512, GemvMulti{}, EmbedRow{}, blockIdx.x, gridDim.x, strip);
 }
 // Two matrices of one vector, the second one without a norm and with a ReLU: workgroups in proportion to their rows.  Bound by HBM: 9216 + 1024 rows of 8192 columns, 168 MB
 // in 28.5 us (5.9 TB/s).
@@ -965,6 +1015,13 @@ int gemv_pair(const void * W, int rows, const pi_norm * norm, float * y, const v
     hipLaunchKernelGGL((gemv_pair_f16_reg_kernel<16, 2>), dim3(kGemvBlocks), dim3(kBlock), 0, (hipStream_t)stream, (const __half *)W, x, na.w, na.b, na.eps, y, rows, kGemvBlocks - second,
                        (const __half *)W2, y2, rows2);
     return check_launch("gemv_pair");
+}
+int gemv_ffn_out(const void * W, int cols, const float * x, const float * resid, float * y, int32_t * n_active, pi_workspace * ws, pi_stream_t stream) {
+    if (!W || !x || !resid || !y || !ws || cols != 8192 || cols > ws->max_d || ((uintptr_t)x & 15)) return fail(PI_E_ARG, "gemv_ffn_out: bad arguments");
+    if (ws->pf_parts < 64 || ws->pf_words <= 0 || ws->pf_words > ws->max_ff / 32 + 2048) return fail(PI_E_STATE, "gemv_ffn_out: no fused launch has filled this workspace");
+    hipLaunchKernelGGL((gemv_strip_f16_kernel<16>), dim3(cols / kStripRows), dim3(kBlock), 0, (hipStream_t)stream, (const __half *)W, x, y,
+                       StripSum{ws->ffn_partial, ws->pf_parts, ws->words, ws->pf_words, n_active, resid});
+    return check_launch("gemv_ffn_out");
 }
 int resume_token(const float * row, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream) {
     if (!row || !d_token || !d_pos || !d_step || !x || cols <= 0) return fail(PI_E_ARG, "resume_token: bad arguments");

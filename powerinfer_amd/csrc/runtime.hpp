@@ -50,11 +50,13 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
 // Attention of one decoded token and its sparse FFN's partial vectors in one launch (attn_ffn_kernel): what pi_k_attn_split (n_parts > 1: scratch) or pi_k_attn_fused and
 // pi_k_sparse_ffn_partials leave
 struct DecodeAttn { const float * qkv; const void * rope_table; void * k_cache, * v_cache; int n_head, n_head_kv, hd, mode, n_ctx, n_parts; const int32_t * pos; float * scratch, * out; uint32_t * arrived; };   // arrived: [n_head], 0 between two launches
-bool attn_ffn_supported(int ff, int r, int cols, int hd, int n_ctx, int n_parts);
+bool attn_ffn_supported(const void * fc2_f16, int ff, int r, int cols, int hd, int n_ctx, int n_parts);
 int attn_ffn(const DecodeAttn & a, const void * fc2_f16, int ff, int r, const float * hidden, float threshold, const void * up_f16, const void * down_t_f16, int cols, const float * x, const pi_norm * norm,
              pi_workspace * ws, pi_stream_t stream);
 // two mat-vecs of one vector in one launch (F16, 8192 columns): y = W norm(x), LayerNorm with its bias, and y2 = relu(W2 x)
 bool gemv_pair_supported(int type, int type2, int cols, const pi_norm * norm, const float * x);
+// y = W x + resid + the vectors of the workspace's sparse FFN (F16, 8192 columns and rows), and its active neurons
+int gemv_ffn_out(const void * W, int cols, const float * x, const float * resid, float * y, int32_t * n_active, pi_workspace * ws, pi_stream_t stream);
 int gemv_pair(const void * W, int rows, const pi_norm * norm, float * y, const void * W2, int rows2, float * y2, int cols, const float * x, pi_stream_t stream);
 // What a pass of a model of layers begins with (pass_start_kernel): words from src to dst; triples (sequence, place, cell) into lists; T embeddings (table null:
 // none) with a norm or a scale and bigrams; angles of up to kRots rotations (freq null: from base).

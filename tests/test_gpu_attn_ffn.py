@@ -8,13 +8,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.timeout(300)
-@pytest.mark.parametrize("heads,kv_heads,rank", [(128, 8, 1024), (128, 16, 512), (64, 64, 512), (64, 8, 1024)])
-def test_decode_beside_the_ffn(heads, kv_heads, rank):
-    """Contexts whose cells a head takes whole and split, few and many cells.  Both sides round q, k, v, the probabilities and h to fp16 at the same places and sum in fp32
+@pytest.mark.parametrize("heads,kv_heads,rank,ff", [(128, 8, 1024, 32768), (128, 16, 512, 36992), (64, 64, 512, 32896), (64, 8, 1024, 32768)])
+def test_decode_beside_the_ffn(heads, kv_heads, rank, ff):
+    """Contexts whose cells a head takes whole and split, few and many cells; as many of the FFN's partial vectors as its sums request ahead, and more.  Both sides round q, k, v, the probabilities and h to fp16 at the same places and sum in fp32
     in another order, so that a value may round to the neighbouring fp16 number: up to 2^-11 of it, over two layers 2e-3 of the largest of 2048 logits.  Every decision of
     the predictor has a margin.  The loop that decodes by itself gives the tokens of its steps one by one, bit for bit."""
     from powerinfer_amd.model import Model
-    hp = synth.hparams("falcon-40b", n_layer=2, n_head=heads, n_head_kv=kv_heads, n_rank=rank, n_vocab=2048, seed=5, pred_margin=True)
+    hp = synth.hparams("falcon-40b", n_layer=2, n_head=heads, n_head_kv=kv_heads, n_rank=rank, n_ff=ff, n_vocab=2048, seed=5, pred_margin=True)
     model = synth.make_model(hp)
     rng = np.random.default_rng(heads + rank)
     for n_ctx, prompts in ((96, (0, 1, 90)), (1200, (0, 9, 1190))):
