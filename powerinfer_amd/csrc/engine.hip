@@ -33,12 +33,13 @@ size_t row_bytes(int type, int64_t ne0) {
 // advances, the token and the step's total active-row count are logged; where a call waits for them (pin), the token, the host threads' status and
 // (want_logits) the logits are stored in pinned memory: words 0 and 1, and from word kPickLogits on.  Bound by latency and by what one unit can
 // read: 32000 logits were 6.6 us for a single workgroup, and another 5.6 and a launch apart went to their copy; now 32 workgroups read them once for
-// both and the last one to arrive ends the step (6.9 us).  Ties go to the lowest index, as before.
+// both and the last one to arrive ends the step (6.9 us).  The host waits for its word (HostDone).  Ties go to the lowest index, as before.
 constexpr int kPickBlock = 256, kPickMost = 64, kPickLogits = 16;
 struct Pick {
     const float * logits; int n; int32_t * token, * pos, * step, * out_tokens, * out_active; const int32_t * n_active; int n_layer, max_steps;
     unsigned long long * best; unsigned int * arrived;              // [kPickMost] the workgroups' choices; 0 between two launches
     uint32_t * pin; const uint32_t * status; int want_logits;
+    pi::HostDone done;                                              // (pin) said when all of it is in place
 };
 __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
     __shared__ float bv[kPickBlock / 64];
@@ -76,6 +77,7 @@ __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
         for (int o = 32; o > 0; o >>= 1) { const float ov = __shfl_xor(best, o, 64); const int oi = __shfl_xor(idx, o, 64); merge(ov, oi); }
     };
     merge_wave();
+    if (p.pin) __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0): this wave's part of the results is under way before the workgroup counts itself
     if (lane == 0) { bv[wave] = best; bi[wave] = idx; }
     __syncthreads();
     if (wave != 0) return;
@@ -84,6 +86,7 @@ __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
         unsigned int before = 0;
         if (lane == 0) {
             __hip_atomic_store(p.best + blockIdx.x, (unsigned long long)__float_as_uint(best) << 32 | (unsigned int)idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (p.pin) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");   // and in the host's memory (stores past the caches, eight bytes each, took a millisecond)
             before = __hip_atomic_fetch_add(p.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (__builtin_amdgcn_readfirstlane(before) + 1 < gridDim.x) return;
@@ -102,7 +105,10 @@ __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
     *p.token = idx;
     *p.pos = p_in + 1;
     *p.step = s_in + 1;
-    if (p.pin) { p.pin[0] = (uint32_t)idx; p.pin[1] = status; }
+    if (p.pin) {
+        p.pin[0] = (uint32_t)idx; p.pin[1] = status;
+        __hip_atomic_store(p.done.word, p.done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // dst row i = src row perm[i]; rows of row_bytes (a multiple of 16) bytes, one workgroup per row
@@ -421,7 +427,7 @@ int last_row_forward(pi_model * m, const float * row, int32_t token, int32_t pos
 int launch_pick(pi_model * m, uint32_t * pin, const uint32_t * status, bool want_logits) {
     const int n = m->hp.n_vocab, blocks = std::min((n + kPickBlock * 4 - 1) / (kPickBlock * 4), kPickMost);
     const Pick p{m->logits, n, m->d_token, m->d_pos, m->d_step, m->d_out_tokens, m->d_out_active, m->n_active, m->hp.n_layer, m->max_steps,
-                 m->pick_best, m->pick_arrived, pin, status, want_logits};
+                 m->pick_best, m->pick_arrived, pin, status, want_logits, pin ? m->stage.next() : pi::HostDone{}};
     hipLaunchKernelGGL(pick_token_kernel, dim3(blocks), dim3(kPickBlock), 0, m->stream, p);
     return pi::check_launch("pick_token");
 }

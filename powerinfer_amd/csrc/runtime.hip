@@ -1,4 +1,5 @@
 // Device/runtime plumbing of the C ABI: init, memory, copies, events, error string.
+#include <chrono>
 #include <mutex>
 #include "runtime.hpp"
 #include "../../include/powerinfer_hip.h"
@@ -39,20 +40,23 @@ int compute_units() {
 
 namespace {
 struct CopyOut { const uint32_t * src[pi::HostStage::kMaxCopies]; uint32_t words[pi::HostStage::kMaxCopies], at[pi::HostStage::kMaxCopies]; };
-__global__ __launch_bounds__(256) void copy_out_kernel(CopyOut c, uint32_t * __restrict__ dst) {
+__global__ __launch_bounds__(256) void copy_out_kernel(CopyOut c, uint32_t * __restrict__ dst, pi::HostDone done) {
     const uint32_t i0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
 #pragma unroll
     for (int r = 0; r < pi::HostStage::kMaxCopies; ++r) {
         const uint32_t * s = c.src[r];
         uint32_t * d = dst + c.at[r];
-        uint32_t done = 0;
+        uint32_t done4 = 0;
         if (((uintptr_t)s & 15) == 0) {                             // (places in the buffer are multiples of 64 bytes)
             const uint32_t n4 = c.words[r] / 4;
             for (uint32_t i = i0; i < n4; i += step) reinterpret_cast<uint4 *>(d)[i] = reinterpret_cast<const uint4 *>(s)[i];
-            done = n4 * 4;
+            done4 = n4 * 4;
         }
-        for (uint32_t i = done + i0; i < c.words[r]; i += step) d[i] = s[i];
+        for (uint32_t i = done4 + i0; i < c.words[r]; i += step) d[i] = s[i];
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0): this wave's stores are under way
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(done.word + blockIdx.x, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 }  // namespace
 
@@ -75,13 +79,13 @@ void HostStage::init(size_t usual_bytes) {
         for (int i = 0; i < pinned_n && !pin; ++i)
             if (pinned_kept[i].bytes == piece * n_pieces) { pin = pinned_kept[i].p; pinned_kept[i] = pinned_kept[--pinned_n]; }
     }
-    if (!pin && hipHostMalloc((void **)&pin, piece * n_pieces, hipHostMallocPortable) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
-    for (int i = 0; i < n_pieces && pin; ++i)
-        if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) { ev[i] = nullptr; (void)hipGetLastError(); release(); }
+    if (!pin && hipHostMalloc((void **)&pin, piece * n_pieces + 4 * kPieces * kBlocks, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
+    done = reinterpret_cast<uint32_t *>(pin + piece * n_pieces);
+    memset(done, 0, 4 * kPieces * kBlocks);
+    seq = 0;
 }
 
 void HostStage::release() {
-    for (hipEvent_t & e : ev) if (e) { (void)hipEventDestroy(e); e = nullptr; }
     if (!counted) return;
     counted = false;
     unsigned char * out[kKept + 1];
@@ -96,8 +100,18 @@ void HostStage::release() {
     while (n) (void)hipHostFree(out[--n]);
 }
 
+int HostStage::until(const HostDone & d, int words, hipStream_t st) {
+    const auto end = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+    for (int w = 0, k = 1; w < words; ++k) {
+        if (__atomic_load_n(d.word + w, __ATOMIC_ACQUIRE) == d.value) { ++w; continue; }
+        // what does not get through, or takes longer than a token, is the runtime's to wait for
+        if (k % 64 == 0 && std::chrono::steady_clock::now() > end) { PI_HIP_TRY(hipStreamSynchronize(st)); return PI_OK; }
+        __builtin_ia32_pause();
+    }
+    return PI_OK;
+}
 int HostStage::wait(hipStream_t st) {
-    PI_HIP_TRY(hipStreamSynchronize(st));
+    if (const int rc = until({done, seq}, 1, st)) return rc;
     busy = false;
     return PI_OK;
 }
@@ -120,6 +134,8 @@ int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
     const HostCopy & big = c[m - 1];
     size_t sent = 0, taken = 0;                                     // bytes of it
     size_t from[kPieces] = {}, len[kPieces] = {};
+    HostDone through[kPieces] = {};
+    int blocks[kPieces] = {};
     int queued = 0, fetched = 0;
     while (taken < big.bytes) {
         while (sent < big.bytes && queued - fetched < n_pieces) {
@@ -129,16 +145,14 @@ int HostStage::fetch(const HostCopy * copies, int n, hipStream_t st) {
             CopyOut o{};
             for (int i = 0; i + 1 < m && !queued; ++i) { o.src[i] = (const uint32_t *)c[i].dev; o.words[i] = (uint32_t)(c[i].bytes / 4); o.at[i] = (uint32_t)(at[i] / 4); }
             o.src[kMaxCopies - 1] = (const uint32_t *)((const unsigned char *)big.dev + sent); o.words[kMaxCopies - 1] = (uint32_t)(b / 4); o.at[kMaxCopies - 1] = (uint32_t)(head / 4);
-            const unsigned blocks = (unsigned)((b / 16 + 255) / 256);
-            hipLaunchKernelGGL(copy_out_kernel, dim3(blocks ? blocks : 1), dim3(256), 0, st, o, reinterpret_cast<uint32_t *>(pin + (size_t)slot * piece));
+            blocks[slot] = std::min(std::max((int)((b / 16 + 255) / 256), 1), kBlocks);
+            through[slot] = next(slot);
+            hipLaunchKernelGGL(copy_out_kernel, dim3(blocks[slot]), dim3(256), 0, st, o, reinterpret_cast<uint32_t *>(pin + (size_t)slot * piece), through[slot]);
             if (const int rc = check_launch("copy_out")) return rc;
             from[slot] = sent; len[slot] = b; sent += b; ++queued;
-            if (sent < big.bytes) PI_HIP_TRY(hipEventRecord(ev[slot], st));
         }
         const int slot = fetched % n_pieces;
-        const bool last = sent == big.bytes && fetched + 1 == queued;
-        if (last) PI_HIP_TRY(hipStreamSynchronize(st));
-        else PI_HIP_TRY(hipEventSynchronize(ev[slot]));
+        if (const int rc = until(through[slot], blocks[slot], st)) return rc;      // (the last one: everything the stream held)
         const unsigned char * s = pin + (size_t)slot * piece;
         if (!fetched) for (int i = 0; i + 1 < m; ++i) memcpy(c[i].host, s + at[i], c[i].bytes);
         memcpy((unsigned char *)big.host + from[slot], s + (fetched ? 0 : small), len[slot]);
