@@ -24,7 +24,8 @@ __device__ __forceinline__ void attn_fused_head(const float * __restrict__ qkv, 
                                                             const int32_t * __restrict__ pos_p, float * __restrict__ out,
                                                             int qkv_stride, size_t cache_seq_stride, int out_stride, __half * __restrict__ out16, int out16_ol,
                                                             int8_t * __restrict__ q8_q, float * __restrict__ q8_d, int * __restrict__ q8_s,
-                                                const int h, const int y) {
+                                                const int h, const int y, __half * out_lds = nullptr) {
+    // out_lds: instead of out, this head's values in fp16
     // q8_q != nullptr: the output also as the Q8_0 blocks an integer mat-mul of a Q4_0 matrix multiplies with (the blocks, scales and
     // -8 * sums pi_k_norm_q8_blocks makes of the same values: a head's hd outputs are whole blocks of 32, one per half-wave)
     // y: sequence of a batched step (its own token, position and cache); 0 for single-sequence decoding
@@ -32,7 +33,7 @@ __device__ __forceinline__ void attn_fused_head(const float * __restrict__ qkv, 
     qkv += (size_t)y * qkv_stride;
     k_cache += (size_t)y * cache_seq_stride;
     v_cache += (size_t)y * cache_seq_stride;
-    out += (size_t)y * out_stride;
+    if (!out_lds) out += (size_t)y * out_stride;
     if (out16 && !out16_ol) out16 += (size_t)y * out_stride;      // optional fp16 copy: the input of the next mat-mul of a batched step
     pos_p += y;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -192,6 +193,7 @@ __device__ __forceinline__ void attn_fused_head(const float * __restrict__ qkv, 
             for (int g = 0; g < 8; ++g) if (g0 + g) v += t[g];
         }
         if (n_grp < ngrp) v += 0.0f;
+        if (out_lds) { out_lds[e] = __float2half_rn(v); continue; }
         out[(size_t)h * hd + e] = v;
         if (out16) out16[out16_ol ? pi_ol_index(y, h * hd + e) : (size_t)h * hd + e] = __float2half_rn(v);
         if (q8_q) {                                               // (hd % 32 == 0: the lanes of a block run this together)

@@ -177,6 +177,12 @@ pi_norm attn_norm(pi_model * m, int il) {
     if (m->L(il, PI_T_ATTN_NORM_2).dev) return make_norm(2, eps, m->L(il, PI_T_ATTN_NORM_2), &m->L(il, PI_T_ATTN_NORM_2_B));
     return make_norm(2, eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
 }
+pi::DecodeAttn decode_attn(pi_model * m, int il) {
+    const pi_hparams & hp = m->hp;
+    const size_t kv_off = (size_t)il * hp.n_head_kv * hp.n_ctx * m->hd;
+    return {m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, m->hd, hp.arch == PI_ARCH_FALCON ? 2 : 0, hp.n_ctx, m->attn_parts, m->d_pos,
+            m->attn_scratch, m->att, m->attn_arrived};
+}
 // the token that a pass starts with (id < 0: the one the device's state names)
 struct StartToken { int32_t id, pos; };
 
@@ -208,8 +214,7 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
     if (branch && m->rope_table && pi::attn_ffn_supported(fc2.dev, ff, r, d, hd, hp.n_ctx, m->attn_parts) && wo.type == PI_TYPE_F16 && pi::gemv_pair_supported(wqkv.type, fc1.type, d, &an, x)) {
         const pi_norm fnb = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
         PI_TRY(pi::gemv_pair(wqkv.dev, d + 2 * gqa, &an, m->qkv, fc1.dev, r, m->hidden, d, x, st));
-        const pi::DecodeAttn a{m->qkv, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, 2, hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, m->attn_arrived};
-        PI_TRY(pi::attn_ffn(a, fc2.dev, ff, r, m->hidden, hp.sparse_threshold, up.dev, down.dev, d, x, &fnb, m->ws, st));
+        PI_TRY(pi::attn_ffn(decode_attn(m, il), fc2.dev, ff, r, m->hidden, hp.sparse_threshold, up.dev, down.dev, d, x, &fnb, m->ws, st));
         PI_TRY(pi::gemv_ffn_out(wo.dev, d, m->att, x, m->x2, n_act, m->ws, st));
         std::swap(m->x, m->x2);
         return PI_OK;
@@ -242,6 +247,17 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
     } else {
         PI_TRY(pi_k_gemv(wqkv.type, wqkv.dev, d + 2 * gqa, d, x, &an, PI_EPI_NONE, nullptr, nullptr, m->qkv, st));
     }
+    // small layers: the launches are the time, not what they read (see ffn_small_f16_kernel; a caller's own device matrices may lie anywhere)
+    const pi_norm fn = falcon ? make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B)) : make_norm(1, hp.norm_eps, m->L(il, PI_T_FFN_NORM), nullptr);
+    const bool f16 = up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && fc1.type == PI_TYPE_F16 && fc2.type == PI_TYPE_F16;
+    const bool aligned = (((uintptr_t)fc1.dev | (uintptr_t)fc2.dev | (uintptr_t)up.dev | (uintptr_t)gate.dev | (uintptr_t)down.dev | (uintptr_t)fn.w | (uintptr_t)fn.b) & 15) == 0;
+    const bool small = f16 && aligned && !layer_hybrid && !m->capture && pi_k_sparse_ffn_small_supported(ff, r, d);
+    if (small && m->out_parts && m->attn_parts <= 1 && wo.type == PI_TYPE_F16 && ((uintptr_t)wo.dev & 15) == 0) {
+        PI_TRY(pi::attn_out_small(decode_attn(m, il), wo.dev, d, m->out_parts, st));
+        PI_TRY(pi::sparse_ffn_small_of(m->out_parts, hp.n_head, m->ffn_inp, fc1.dev, fc2.dev, ff, r, hp.sparse_threshold, up.dev, gate.dev, down.dev, d, x, &fn, m->x2, n_act, m->ws, st));
+        std::swap(m->x, m->x2);
+        return PI_OK;
+    }
     if (m->attn_parts > 1) {
         PI_TRY(pi_k_attn_split(m->qkv, 0, m->rope_table, m->k_cache + kv_off, m->v_cache + kv_off, 0, 1, hp.n_head, hp.n_head_kv, hd, falcon ? 2 : 0,
                                hp.n_ctx, m->attn_parts, m->d_pos, m->attn_scratch, m->att, 0, nullptr, st));
@@ -254,22 +270,17 @@ int layer_forward(pi_model * m, int il, bool last_token, const StartToken * star
         PI_TRY(pi_k_attn_decode(m->q_rot, m->k_cache + kv_off, m->v_cache + kv_off, hp.n_head, hp.n_head_kv, hd, hp.n_ctx, m->d_pos, m->att, st));
     }
 
-    const float * pred_in; const float * ffn_in; pi_norm fn;
+    const float * pred_in; const float * ffn_in;
     if (!falcon) {
         // ffn_inp = wo.att + x   (ggml_add(cur, inpSA), llama.cpp:5022)
         PI_TRY(pi_k_gemv(wo.type, wo.dev, d, d, m->att, nullptr, PI_EPI_ADD, x, nullptr, m->ffn_inp, st));
         pred_in = m->ffn_inp; ffn_in = m->ffn_inp;
-        fn = make_norm(1, hp.norm_eps, m->L(il, PI_T_FFN_NORM), nullptr);
     } else {
         PI_TRY(pi_k_gemv(wo.type, wo.dev, d, d, m->att, nullptr, PI_EPI_NONE, nullptr, nullptr, m->attn_out, st));
         pred_in = x; ffn_in = x;                       // Falcon: predictor sees the layer input, FFN sees attn_norm(layer input)
-        fn = make_norm(2, hp.norm_eps, m->L(il, PI_T_ATTN_NORM), &m->L(il, PI_T_ATTN_NORM_B));
     }
 
-    // small layers: the launches are the time, not what they read (see ffn_small_f16_kernel; a caller's own device matrices may lie anywhere)
-    const bool f16 = up.type == PI_TYPE_F16 && down.type == PI_TYPE_F16 && fc1.type == PI_TYPE_F16 && fc2.type == PI_TYPE_F16;
-    const bool aligned = (((uintptr_t)fc1.dev | (uintptr_t)fc2.dev | (uintptr_t)up.dev | (uintptr_t)gate.dev | (uintptr_t)down.dev | (uintptr_t)fn.w | (uintptr_t)fn.b) & 15) == 0;
-    if (f16 && aligned && !layer_hybrid && !m->capture && pi_k_sparse_ffn_small_supported(ff, r, d)) {
+    if (small) {
         PI_TRY(pi_k_sparse_ffn_small(fc1.dev, fc2.dev, ff, r, hp.sparse_threshold, up.dev, falcon ? nullptr : gate.dev, down.dev, d, ffn_in, &fn,
                                      falcon ? PI_EPI_ADD2 : PI_EPI_ADD, falcon ? m->attn_out : m->ffn_inp, falcon ? x : nullptr, m->x2, n_act, m->ws, st));
         std::swap(m->x, m->x2);
@@ -825,6 +836,10 @@ int pi_model_finalize(pi_model * m) {
             if (!m->attn_scratch || !m->attn_arrived) return PI_E_HIP;
             PI_TRY(pi_memset(m->attn_arrived, 0, 4 * (size_t)hp.n_head));
         }
+    }
+    if (hp.arch != PI_ARCH_FALCON && m->attn_parts <= 1 && (d == 512 || d == 1024) && pi::attn_out_small_supported(hp.n_head, m->hd, hp.n_ctx)) {
+        m->out_parts = m->alloc<float>((size_t)hp.n_head * d);
+        if (!m->out_parts) return PI_E_HIP;
     }
     if (fused_ok || m->attn_parts > 1) {
         m->rope_table = m->alloc<float>((size_t)hp.n_ctx * m->hd);

@@ -64,6 +64,7 @@ struct pi_model {
     float *rope_table = nullptr;          // float2 [n_ctx][hd/2] (cos, sin), when the fused or the split attention kernel is used
     int    attn_parts = 1;                // > 1: the cells of every head are split over this many workgroups (long contexts)
     float *attn_scratch = nullptr;        // partial results of those workgroups for one token
+    float *out_parts = nullptr;           // small models: the heads' shares of the output projection [n_head][n_embd]
     uint32_t *attn_arrived = nullptr;     // and how many of a head's have theirs, where the last one merges (0 between two launches)
     float *attn_scratch_chunk = nullptr;  // and for a prompt chunk (allocated at the first chunk that needs it)
 

@@ -186,6 +186,38 @@ __global__ __launch_bounds__(BLOCK, 8) void attn_fused_kernel(const float * __re
     attn_fused_head<BLOCK, LPP>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos_p, out, qkv_stride, cache_seq_stride, out_stride, out16, out16_ol, q8_q, q8_d, q8_s,
                                 blockIdx.x, blockIdx.y);
 }
+// Attention and output projection of a small model's token: a head's workgroup multiplies what it attended with its columns of wo, whose rows travel under the attention, and leaves
+// a vector of the model's width; ffn_small_f16_kernel adds the heads'.  Bound by latency like the attention alone: 7.3 us at 20
+// cells where that takes 7.0 and the projection 3.4 behind it (the FFN then takes 9.1 instead of 8.2).  8 tokens of three layers of 512 x 4096, 8 heads: 790 -> 705 us at 20 cells, 830 -> 750
+// at 300.
+constexpr int kOutPre = 4;              // rows of wo a group of lanes requests ahead
+template <int LPP>
+__global__ __launch_bounds__(kAttnBlock, 4) void attn_out_small_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table, __half * __restrict__ k_cache, __half * __restrict__ v_cache,
+                                                                       int n_head, int n_head_kv, int hd, int mode, int n_ctx, const int32_t * __restrict__ pos_p, const __half * __restrict__ wo, int d,
+                                                                       float * __restrict__ parts) {
+    __shared__ __align__(16) __half att[LPP * 8];
+    const int h = blockIdx.x, sub = threadIdx.x % LPP, grp = threadIdx.x / LPP;
+    constexpr int kGroups = kAttnBlock / LPP;
+    const __half * w = wo + (size_t)h * hd + sub * 8;
+    auto row = [&](int r) { return pi_ld16(w + (size_t)min(r, d - 1) * ((size_t)n_head * hd)); };
+    pi_u32x4 ahead[kOutPre];
+#pragma unroll
+    for (int k = 0; k < kOutPre; ++k) ahead[k] = row(grp + k * kGroups);
+    attn_fused_head<kAttnBlock, LPP>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos_p, nullptr, 0, 0, 0, nullptr, 0, nullptr, nullptr, nullptr, h, 0, att);
+    __syncthreads();
+    const pi_u32x4 a = *reinterpret_cast<const pi_u32x4 *>(att + sub * 8);
+    float * out = parts + (size_t)h * d;
+    for (int r0 = grp; r0 < d; r0 += kOutPre * kGroups) {
+        if (r0 != grp)
+#pragma unroll
+            for (int k = 0; k < kOutPre; ++k) ahead[k] = row(r0 + k * kGroups);
+#pragma unroll
+        for (int k = 0; k < kOutPre; ++k) {
+            const float v = pi_group_sum<LPP>(pi_dot8h(ahead[k], a, 0.0f), LPP);
+            if (sub == 0 && r0 + k * kGroups < d) out[r0 + k * kGroups] = v;
+        }
+    }
+}
 template <bool FROM_CACHE, int LPP>
 __global__ __launch_bounds__(kAttnPartBlock, 4) void attn_part_kernel(const float * __restrict__ qkv, const float2 * __restrict__ rope_table,
                                                                    __half * __restrict__ k_cache, __half * __restrict__ v_cache,
@@ -1244,6 +1276,17 @@ static int launch_attn_parts(const float * qkv, const float2 * rope_table, __hal
     return pi::check_launch(name);
 }
 namespace pi {
+bool attn_out_small_supported(int n_head, int hd, int n_ctx) { return n_head <= kOutHeads && (hd == 64 || hd == 128) && pi_k_attn_fused_supported(hd, n_ctx); }
+int attn_out_small(const DecodeAttn & a, const void * wo_f16, int d, float * parts, pi_stream_t stream) {
+    if (!a.qkv || !a.rope_table || !a.k_cache || !a.v_cache || !a.pos || !wo_f16 || !parts || d <= 0 || ((uintptr_t)wo_f16 & 15)) return fail(PI_E_ARG, "attn_out_small: bad arguments");
+    if (a.n_head <= 0 || a.n_head_kv <= 0 || a.n_head % a.n_head_kv || (a.mode != 0 && a.mode != 2) || !attn_out_small_supported(a.n_head, a.hd, a.n_ctx))
+        return fail(PI_E_UNSUPPORTED, "attn_out_small: shape outside the kernel");
+    const size_t sh = attn_fused_lds_bytes(a.hd, a.n_ctx);
+    const auto kernel = a.hd == 128 ? attn_out_small_kernel<16> : attn_out_small_kernel<8>;
+    hipLaunchKernelGGL(kernel, dim3(a.n_head), dim3(kAttnBlock), sh, (hipStream_t)stream, a.qkv, (const float2 *)a.rope_table, (__half *)a.k_cache, (__half *)a.v_cache, a.n_head, a.n_head_kv, a.hd, a.mode,
+                       a.n_ctx, a.pos, (const __half *)wo_f16, d, parts);
+    return check_launch("attn_out_small");
+}
 int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void * v_cache, int n_head, int n_head_kv, int hd, int mode,
                int n_ctx, const int32_t * pos, float * out, const Ahead & ahead, pi_stream_t stream) {
     if (!qkv || !rope_table || !k_cache || !v_cache || !pos || !out) return pi::fail(PI_E_ARG, "pi_k_attn_fused: null pointer");

@@ -1,6 +1,8 @@
 // The sparse FFN of one token in a small F16 model, predictor included: both of its products, the active rows and the down projection in one launch
 // and a reduction, where wider models need the predictor's hidden units and the rows of one launch spread over the chip.
 #include "kernels_common.hpp"
+#include "runtime.hpp"
+#include "../../include/powerinfer_hip.h"
 
 namespace {
 
@@ -13,10 +15,12 @@ namespace {
 // Rounding as in those: hidden units, normed input and h to fp16, everything else fp32; logits have the same order of sums.
 // KIND: norm of the FFN's input (0 none, 1 RMS, 2 LayerNorm); the predictor reads x as it is.
 constexpr int kSmBlock = 256, kSmNeurons = 32, kSmFc1 = 16, kSmAtOnce = 4;      // rows of fc1 in flight a wave; neurons whose rows a wave requests together
-template <int CH, int R, bool GATE, int KIND>      // columns: 512 CH
+// SUM: x is what the heads' shares of the output projection make of it (attn_out_small_kernel), and the first workgroup leaves it for the residual.
+template <int CH, int R, bool GATE, int KIND, bool SUM = false>      // columns: 512 CH
 __global__ __launch_bounds__(kSmBlock) void ffn_small_f16_kernel(const __half * __restrict__ fc1, const __half * __restrict__ fc2, const __half * __restrict__ up, const __half * __restrict__ gate,
                                                                  const __half * __restrict__ down, const float * __restrict__ x, const float * __restrict__ nw, const float * __restrict__ nb,
-                                                                 float eps, float thr, uint32_t * __restrict__ words, float * __restrict__ partial) {
+                                                                 float eps, float thr, uint32_t * __restrict__ words, float * __restrict__ partial,
+                                                                 const float * __restrict__ shares, int n_shares, float * __restrict__ xsum) {
     constexpr int COLS = 512 * CH, LPN = R / 8, NPL = 64 / LPN, NL = 8 / NPL, OWN = R / 4, HELD = kSmFc1 / CH, NB = OWN / HELD;
     static_assert(LPN == 8 || LPN == 16 || LPN == 32, "rank");
     __shared__ __align__(16) __half hid[R];
@@ -30,6 +34,15 @@ __global__ __launch_bounds__(kSmBlock) void ffn_small_f16_kernel(const __half * 
     };
 #pragma unroll
     for (int j = 0; j < CH; ++j) fetch8(xv[j], x + j * 512 + lane * 8);
+    constexpr int kSmShares = 8;                                    // vectors a wave requests together
+    float sv[SUM ? kSmShares : 1][CH][8];
+    auto fetch_shares = [&](int s0) {                               // (past the last one its values again, not added)
+#pragma unroll
+        for (int s = 0; s < kSmShares; ++s)
+#pragma unroll
+            for (int j = 0; j < CH; ++j) fetch8(sv[s][j], shares + (size_t)min(s0 + s, n_shares - 1) * COLS + j * 512 + lane * 8);
+    };
+    if constexpr (SUM) fetch_shares(0);
     pi_u32x4 f1[2][HELD][CH], f2[NL];
     auto fetch1 = [&](pi_u32x4 (&f)[HELD][CH], int b) {
 #pragma unroll
@@ -49,6 +62,25 @@ __global__ __launch_bounds__(kSmBlock) void ffn_small_f16_kernel(const __half * 
         const __half2 h[4] = {__floats2half2_rn(v[0], v[1]), __floats2half2_rn(v[2], v[3]), __floats2half2_rn(v[4], v[5]), __floats2half2_rn(v[6], v[7])};
         return *reinterpret_cast<const pi_u32x4 *>(h);
     };
+    if constexpr (SUM) {
+        for (int s0 = 0; s0 < n_shares; s0 += kSmShares) {
+            if (s0) fetch_shares(s0);
+#pragma unroll
+            for (int s = 0; s < kSmShares; ++s)
+                if (s0 + s < n_shares)
+#pragma unroll
+                    for (int j = 0; j < CH; ++j)
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) xv[j][k] += sv[s][j][k];
+        }
+        if (blockIdx.x == 0 && wave == 0)
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                float * p = xsum + j * 512 + lane * 8;
+                *reinterpret_cast<float4 *>(p) = make_float4(xv[j][0], xv[j][1], xv[j][2], xv[j][3]);
+                *reinterpret_cast<float4 *>(p + 4) = make_float4(xv[j][4], xv[j][5], xv[j][6], xv[j][7]);
+            }
+    }
     pi_u32x4 xr[CH];
 #pragma unroll
     for (int j = 0; j < CH; ++j) xr[j] = packed(xv[j]);
@@ -174,6 +206,37 @@ __global__ __launch_bounds__(kSmBlock) void ffn_small_f16_kernel(const __half * 
 
 }  // namespace
 
+static int ffn_small(const float * shares, int n_shares, float * xsum, const void * fc1_f16, const void * fc2_f16, int ff, int r, float threshold, const void * up_f16, const void * gate_f16, const void * down_t_f16, int cols, const float * x,
+                          const pi_norm * norm, int epilogue, const float * add1, const float * add2, float * out, int32_t * n_active, pi_workspace * ws, pi_stream_t stream) {
+    if (!fc1_f16 || !fc2_f16 || !up_f16 || !down_t_f16 || !x || !out || !ws) return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: null pointer");
+    const NormArgs na{norm ? norm->kind : 0, norm ? norm->eps : 0.0f, norm ? norm->w : nullptr, norm ? norm->b : nullptr};
+    if (!pi_k_sparse_ffn_small_supported(ff, r, cols) || !(na.kind == 0 || (na.kind == 1 && na.w && !na.b) || (na.kind == 2 && na.w && na.b)))
+        return pi::fail(PI_E_UNSUPPORTED, "pi_k_sparse_ffn_small: 512 or 1024 columns, rank 64, 128 or 256, predictor of at most 131072 values, ff % 32 == 0, a norm with its weights");
+    if (ff > ws->max_ff || cols > ws->max_d) return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: shape exceeds the workspace");
+    if ((((uintptr_t)fc1_f16 | (uintptr_t)fc2_f16 | (uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)down_t_f16 | (uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b) & 15) != 0)
+        return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: operands must be 16-byte aligned");
+    const __half * a = (const __half *)fc1_f16, * b = (const __half *)fc2_f16, * u = (const __half *)up_f16, * g = (const __half *)gate_f16, * d = (const __half *)down_t_f16;
+#define PI_SM(CH, R, GATE, KIND, SUM) hipLaunchKernelGGL((ffn_small_f16_kernel<CH, R, GATE, KIND, SUM>), dim3(ff / kSmNeurons), dim3(kSmBlock), 0, (hipStream_t)stream, a, b, u, g, d, x, na.w, na.b, na.eps, threshold, ws->words, ws->ffn_partial, shares, n_shares, xsum)
+#define PI_SM_K(CH, R, GATE) do { if (na.kind == 0) PI_SM(CH, R, GATE, 0, false); else if (na.kind == 1) PI_SM(CH, R, GATE, 1, false); else PI_SM(CH, R, GATE, 2, false); } while (0)
+#define PI_SM_G(CH, R) do { if (shares) PI_SM(CH, R, true, 1, true); else if (g) PI_SM_K(CH, R, true); else PI_SM_K(CH, R, false); } while (0)
+    if (cols == 512) { if (r == 64) PI_SM_G(1, 64); else if (r == 128) PI_SM_G(1, 128); else PI_SM_G(1, 256); }
+    else             { if (r == 64) PI_SM_G(2, 64); else PI_SM_G(2, 128); }
+#undef PI_SM_G
+#undef PI_SM_K
+#undef PI_SM
+    ws->pf_parts = ws->pf_words = ff / kSmNeurons;
+    const int rc = pi::check_launch("pi_k_sparse_ffn_small");
+    return rc != PI_OK ? rc : pi_k_sparse_ffn_reduce(ff, cols, epilogue, add1, add2, out, n_active, ws, stream);
+}
+
+namespace pi {
+int sparse_ffn_small_of(const float * parts, int n_parts, float * xsum, const void * fc1_f16, const void * fc2_f16, int ff, int r, float threshold, const void * up_f16, const void * gate_f16,
+                        const void * down_t_f16, int cols, const float * x, const pi_norm * norm, float * out, int32_t * n_active, pi_workspace * ws, pi_stream_t stream) {
+    if (!parts || n_parts <= 0 || n_parts > kOutHeads || !xsum || !gate_f16 || !norm || norm->kind != 1 || (((uintptr_t)parts | (uintptr_t)xsum) & 15)) return fail(PI_E_ARG, "sparse_ffn_small_of: bad arguments");
+    return ffn_small(parts, n_parts, xsum, fc1_f16, fc2_f16, ff, r, threshold, up_f16, gate_f16, down_t_f16, cols, x, norm, PI_EPI_ADD, xsum, nullptr, out, n_active, ws, stream);
+}
+}  // namespace pi
+
 extern "C" {
 
 // A first predictor matrix of 256 KB at most.  Against the four launches, with a tenth (half) of the neurons active, us: 512 columns, rank 64, 1024 neurons
@@ -185,25 +248,7 @@ int pi_k_sparse_ffn_small_supported(int ff, int r, int cols) {
 
 int pi_k_sparse_ffn_small(const void * fc1_f16, const void * fc2_f16, int ff, int r, float threshold, const void * up_f16, const void * gate_f16, const void * down_t_f16, int cols, const float * x,
                           const pi_norm * norm, int epilogue, const float * add1, const float * add2, float * out, int32_t * n_active, pi_workspace * ws, pi_stream_t stream) {
-    if (!fc1_f16 || !fc2_f16 || !up_f16 || !down_t_f16 || !x || !out || !ws) return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: null pointer");
-    const NormArgs na{norm ? norm->kind : 0, norm ? norm->eps : 0.0f, norm ? norm->w : nullptr, norm ? norm->b : nullptr};
-    if (!pi_k_sparse_ffn_small_supported(ff, r, cols) || !(na.kind == 0 || (na.kind == 1 && na.w && !na.b) || (na.kind == 2 && na.w && na.b)))
-        return pi::fail(PI_E_UNSUPPORTED, "pi_k_sparse_ffn_small: 512 or 1024 columns, rank 64, 128 or 256, predictor of at most 131072 values, ff % 32 == 0, a norm with its weights");
-    if (ff > ws->max_ff || cols > ws->max_d) return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: shape exceeds the workspace");
-    if ((((uintptr_t)fc1_f16 | (uintptr_t)fc2_f16 | (uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)down_t_f16 | (uintptr_t)x | (uintptr_t)na.w | (uintptr_t)na.b) & 15) != 0)
-        return pi::fail(PI_E_ARG, "pi_k_sparse_ffn_small: operands must be 16-byte aligned");
-    const __half * a = (const __half *)fc1_f16, * b = (const __half *)fc2_f16, * u = (const __half *)up_f16, * g = (const __half *)gate_f16, * d = (const __half *)down_t_f16;
-#define PI_SM(CH, R, GATE, KIND) hipLaunchKernelGGL((ffn_small_f16_kernel<CH, R, GATE, KIND>), dim3(ff / kSmNeurons), dim3(kSmBlock), 0, (hipStream_t)stream, a, b, u, g, d, x, na.w, na.b, na.eps, threshold, ws->words, ws->ffn_partial)
-#define PI_SM_K(CH, R, GATE) do { if (na.kind == 0) PI_SM(CH, R, GATE, 0); else if (na.kind == 1) PI_SM(CH, R, GATE, 1); else PI_SM(CH, R, GATE, 2); } while (0)
-#define PI_SM_G(CH, R) do { if (g) PI_SM_K(CH, R, true); else PI_SM_K(CH, R, false); } while (0)
-    if (cols == 512) { if (r == 64) PI_SM_G(1, 64); else if (r == 128) PI_SM_G(1, 128); else PI_SM_G(1, 256); }
-    else             { if (r == 64) PI_SM_G(2, 64); else PI_SM_G(2, 128); }
-#undef PI_SM_G
-#undef PI_SM_K
-#undef PI_SM
-    ws->pf_parts = ws->pf_words = ff / kSmNeurons;
-    const int rc = pi::check_launch("pi_k_sparse_ffn_small");
-    return rc != PI_OK ? rc : pi_k_sparse_ffn_reduce(ff, cols, epilogue, add1, add2, out, n_active, ws, stream);
+    return ffn_small(nullptr, 0, nullptr, fc1_f16, fc2_f16, ff, r, threshold, up_f16, gate_f16, down_t_f16, cols, x, norm, epilogue, add1, add2, out, n_active, ws, stream);
 }
 
 }  // extern "C"

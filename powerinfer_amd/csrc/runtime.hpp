@@ -57,6 +57,13 @@ int attn_fused(const float * qkv, const void * rope_table, void * k_cache, void 
 // Attention of one decoded token and its sparse FFN's partial vectors in one launch (attn_ffn_kernel): what pi_k_attn_split (n_parts > 1: scratch) or pi_k_attn_fused and
 // pi_k_sparse_ffn_partials leave
 struct DecodeAttn { const float * qkv; const void * rope_table; void * k_cache, * v_cache; int n_head, n_head_kv, hd, mode, n_ctx, n_parts; const int32_t * pos; float * scratch, * out; uint32_t * arrived; };   // arrived: [n_head], 0 between two launches
+// Attention and output projection of one decoded token of a small model in one launch: parts[h] [d], a head's share of wo att (attn_out_small_kernel)
+constexpr int kOutHeads = 16;
+bool attn_out_small_supported(int n_head, int hd, int n_ctx);
+int attn_out_small(const DecodeAttn & a, const void * wo_f16, int d, float * parts, pi_stream_t stream);
+// pi_k_sparse_ffn_small of x + the n_parts vectors of `parts`, which go to xsum as well and are its residual
+int sparse_ffn_small_of(const float * parts, int n_parts, float * xsum, const void * fc1_f16, const void * fc2_f16, int ff, int r, float threshold, const void * up_f16, const void * gate_f16,
+                        const void * down_t_f16, int cols, const float * x, const pi_norm * norm, float * out, int32_t * n_active, pi_workspace * ws, pi_stream_t stream);
 bool attn_ffn_supported(const void * fc2_f16, int ff, int r, int cols, int hd, int n_ctx, int n_parts);
 int attn_ffn(const DecodeAttn & a, const void * fc2_f16, int ff, int r, const float * hidden, float threshold, const void * up_f16, const void * down_t_f16, int cols, const float * x, const pi_norm * norm,
              pi_workspace * ws, pi_stream_t stream);
