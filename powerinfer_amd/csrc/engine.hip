@@ -932,7 +932,7 @@ int pi_model_decode(pi_model * m, const int32_t * tokens, int n_tokens, int n_pa
     uint32_t * pin = (uint32_t *)m->stage.room(head + (logits_out ? logits : 0));
     PI_TRY(launch_pick(m, pin, d_status, logits_out != nullptr));
     if (pin) {
-        PI_TRY(m->stage.wait(m->stream));
+        PI_TRY(m->stage.wait(m->stream, m->cold != nullptr));      // (a split model's host threads keep the cores: 2.8 to 3.0 ms a run of 8 tokens either way)
         tok = (int32_t)pin[0];
         status = pin[1];
         if (logits_out) memcpy(logits_out, pin + kPickLogits, logits);

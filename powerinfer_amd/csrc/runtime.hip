@@ -110,8 +110,9 @@ int HostStage::until(const HostDone & d, int words, hipStream_t st) {
     }
     return PI_OK;
 }
-int HostStage::wait(hipStream_t st) {
-    if (const int rc = until({done, seq}, 1, st)) return rc;
+int HostStage::wait(hipStream_t st, bool apart) {
+    if (apart) PI_HIP_TRY(hipStreamSynchronize(st));
+    else if (const int rc = until({done, seq}, 1, st)) return rc;
     busy = false;
     return PI_OK;
 }

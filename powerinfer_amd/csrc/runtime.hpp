@@ -47,7 +47,8 @@ struct HostStage {
     // room for results that the call's own last launch stores (null: to be had with fetch only), and the wait for them
     unsigned char * room(size_t bytes) { if (!pin || bytes > piece) return nullptr; busy = true; return pin; }
     HostDone next(int slot = 0) { return {done + slot * kBlocks, ++seq}; }
-    int wait(hipStream_t st);              // for the launch that the last `next()` went to, the last of the stream, one of whose workgroups speaks for all
+    // for the launch that the last `next()` went to, the last of the stream, one of whose workgroups speaks for all; apart: the runtime's wait, which leaves the core to others
+    int wait(hipStream_t st, bool apart = false);
     int until(const HostDone & d, int words, hipStream_t st);
 };
 
