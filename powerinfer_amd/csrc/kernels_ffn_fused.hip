@@ -35,7 +35,8 @@ constexpr int kPfChunk = 8;                       // active neurons per round tr
 struct HostAnnounce { uint32_t * seq; uint32_t * flags; uint32_t * words_out = nullptr; };    // words_out: a second copy of the activity words (pinned memory) for the logits-only launch
 
 template <int RCH> constexpr int kPfRowsLds = kPfWaves * 4 * RCH * 1024;
-template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
+// ANYWHERE: W2 may start off a multiple of 16 bytes
+template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0, bool ANYWHERE = true>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
 __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, const float * __restrict__ hidden,
                                                                    const __half * __restrict__ Wup, const __half * __restrict__ Wgate,
                                                                    const __half * __restrict__ Wdown,
@@ -68,6 +69,18 @@ __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, 
         typedef const __attribute__((address_space(1))) void * gptr;
         typedef __attribute__((address_space(3))) void * lptr;
         const int w = __builtin_amdgcn_readfirstlane(wave);
+        if (ANYWHERE && ((uintptr_t)W2 & 15) != 0) {                    // (copies to LDS want whole pieces)
+            pi_u32x4 v[4][RCH];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < RCH; ++j) v[i][j] = pi_ld_stream(W2 + (size_t)(first + w * 4 + i) * r + (j * PI_WAVE + lane) * 8);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < RCH; ++j) *reinterpret_cast<pi_u32x4 *>(rows_lds + ((w * 4 + i) * RCH + j) * 1024 + lane * 16) = v[i][j];
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -338,7 +351,7 @@ __global__ __launch_bounds__(kPfBlock, 4) void attn_ffn_kernel(const float * __r
             attn_fused_head<kPfBlock, LPP>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos_p, out, 0, 0, 0, nullptr, 0, nullptr, nullptr, nullptr, b, 0);
         return;
     }
-    pred_ffn_groups<2, RCH, false, 4, false>(W2, hidden, Wup, nullptr, Wdown, x, na, thr, nullptr, words, nullptr, partial, nullptr, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, b - n_attn, smem);
+    pred_ffn_groups<2, RCH, false, 4, false, 0, false>(W2, hidden, Wup, nullptr, Wdown, x, na, thr, nullptr, words, nullptr, partial, nullptr, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, b - n_attn, smem);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1319,8 +1332,8 @@ static int sparse_ffn_partials_impl(const char * who, const void * fc2_f16, int 
         return pi::check_launch(who);
     }
     if (!pf_grouped_shape(ff, r, cols)) return pi::fail(PI_E_UNSUPPORTED, "pi_k_sparse_ffn: this shape runs only with every neuron resident and a norm the kernel carries (5120 columns, rank 1280)");
-    const int G = ((uintptr_t)fc2_f16 & 15) == 0 ? pf_groups(ff, cols) : 1;      // the copies to LDS of several groups' predictor rows want whole pieces
-    ws->pf_parts = ff / (32 * G); ws->pf_words = ff / 32;
+    ws->pf_parts = ff / (32 * pf_groups(ff, cols)); ws->pf_words = ff / 32;
+    const int G = pf_groups(ff, cols);
     const dim3 grid(ff / (32 * G)), block(kPfBlock);
 #define PI_PF_LAUNCH2(CPW, RCH, GATE, GG, HYB) hipLaunchKernelGGL((pred_ffn_f16_kernel<CPW, RCH, GATE, GG, HYB>), grid, block, 0, st, w2, hidden, u, g, dn, x, na, threshold, logits, ws->words, h_dense, ws->ffn_partial, hot_words, hot_prefix, ws->words_hot, (__half *)xn_f16_out, nullptr, HostAnnounce{nullptr, nullptr})
 #define PI_PF_LAUNCH(CPW, RCH, GATE, GG) do { if (hyb) PI_PF_LAUNCH2(CPW, RCH, GATE, GG, true); else PI_PF_LAUNCH2(CPW, RCH, GATE, GG, false); } while (0)
