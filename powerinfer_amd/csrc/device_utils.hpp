@@ -24,6 +24,15 @@ __host__ __device__ __forceinline__ float pi_inv_sqrt(float v) {
 // a / b rounded once to fp32, as IEEE division on the CPU is (the quotient is formed in fp64 and rounded: innocuous for fp32 operands)
 __host__ __device__ __forceinline__ float pi_div(float a, float b) { return (float)((double)a / (double)b); }
 
+// What this wave's workgroup has stored (every wave waits for its own stores ahead of a barrier) is in memory, or (SYSTEM) where the host finds it, before what follows.
+// The release's write-back of the L2 is itself something to wait for, and the compiler counts stores only: where an explicit wait has left none on their way it drops
+// the wait behind the write-back, and a count or a flag gets ahead of the values (a step's logits of which whole rows or single lines were the last step's).
+template <bool SYSTEM> __device__ __forceinline__ void pi_release() {
+    if (SYSTEM) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    else __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0)
+}
+
 // Wave-wide reductions through DPP (data-parallel primitives: lane permutations inside the VALU, no LDS
 // crossbar round trip): pairs, quads, half rows and rows by quad_perm / row_half_mirror / row_mirror, then the
 // last lane of row 0 (2) is added into row 1 (3) and lane 31 into rows 2-3, so lane 63 holds the total, which

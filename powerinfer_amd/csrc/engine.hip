@@ -3,6 +3,7 @@
 // llama.cpp:4652-4757) issued as a fixed chain of fused HIP kernels on one stream and, for the greedy
 // token loop, captured once into a HIP graph and replayed per token (the reference rebuilds and walks a
 // ~40-node-per-layer graph every token, llama.cpp:6408, 6922).
+#include "device_utils.hpp"
 #include "runtime.hpp"
 #include "cold_path.hpp"
 #include <limits.h>
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
         unsigned int before = 0;
         if (lane == 0) {
             __hip_atomic_store(p.best + blockIdx.x, (unsigned long long)__float_as_uint(best) << 32 | (unsigned int)idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (p.pin) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");   // and in the host's memory (stores past the caches, eight bytes each, took a millisecond)
+            if (p.pin) pi_release<true>();                             // and in the host's memory (stores past the caches, eight bytes each, took a millisecond)
             before = __hip_atomic_fetch_add(p.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (__builtin_amdgcn_readfirstlane(before) + 1 < gridDim.x) return;
@@ -107,7 +108,8 @@ __global__ __launch_bounds__(kPickBlock) void pick_token_kernel(Pick p) {
     *p.step = s_in + 1;
     if (p.pin) {
         p.pin[0] = (uint32_t)idx; p.pin[1] = status;
-        __hip_atomic_store(p.done.word, p.done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        pi_release<true>();
+        __hip_atomic_store(p.done.word, p.done.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 

@@ -1102,7 +1102,10 @@ __global__ void host_wait_kernel(const uint32_t * __restrict__ seq, uint32_t * _
                                  unsigned long long limit, int signal_word) {
     if (threadIdx.x != 0) return;
     const uint32_t want = *seq;
-    if (signal_word >= 0) __hip_atomic_store(flags + signal_word, want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);     // host_signal_kernel without advance
+    if (signal_word >= 0) {                                             // host_signal_kernel without advance
+        pi_release<true>();
+        __hip_atomic_store(flags + signal_word, want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     if (__hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u) return;
     const unsigned long long t0 = wall_clock64();
     for (;;) {

@@ -16,7 +16,7 @@ __device__ bool last_block_done(unsigned int * counter, unsigned int n_blocks, i
     __builtin_amdgcn_s_waitcnt(0x0F70);      // vmcnt(0): every wave's stores have arrived (the barrier waits for LDS alone, the fence below for its own wave's)
     __syncthreads();
     if (threadIdx.x == 0) {
-        __threadfence();          // publishes the whole block's stores, ordered before the ticket
+        pi_release<false>();      // publishes the whole block's stores, ordered before the ticket
         const unsigned int t = atomicAdd(counter, 1u);
         *sflag = (t == n_blocks - 1);
         if (t == n_blocks - 1) { *counter = 0; __threadfence(); }

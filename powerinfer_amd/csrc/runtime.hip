@@ -1,6 +1,7 @@
 // Device/runtime plumbing of the C ABI: init, memory, copies, events, error string.
 #include <chrono>
 #include <mutex>
+#include "device_utils.hpp"
 #include "runtime.hpp"
 #include "../../include/powerinfer_hip.h"
 
@@ -56,7 +57,10 @@ __global__ __launch_bounds__(256) void copy_out_kernel(CopyOut c, uint32_t * __r
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0): this wave's stores are under way
     __syncthreads();
-    if (threadIdx.x == 0) __hip_atomic_store(done.word + blockIdx.x, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (threadIdx.x == 0) {
+        pi_release<true>();
+        __hip_atomic_store(done.word + blockIdx.x, done.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 }  // namespace
 
