@@ -29,7 +29,8 @@ int  noalloc_setup();                                  // resolves the static sc
 // A launch that stores results says so in words of the pinned memory, behind its stores, and the host looks there: the runtime's own wait puts a packet behind
 // the launch, 5 us a token, and takes 30 us where the work has ended before it is called (the last piece of several).  Us, stream wait and events / this: 8 tokens of a 7B shape of 4
 // layers 2254 -> 2201, of three layers of 512 x 4096 830 -> 780, of Falcon-40B's of 4 4641 -> 4582; 4 steps of 16 sequences (13B, 4 layers) 3252 -> 3200; a prompt pass and 12
-// steps of 16 requests 17180 -> 16790; a prompt of 333 and 16 tokens 9220 -> 8950.
+// steps of 16 requests 17180 -> 16790; a prompt of 333 and 16 tokens 9220 -> 8950.  (Before the wait behind the write-back, pi_release, without which a word may get ahead of its
+// values; with it these are as fast within the spread.)
 struct HostDone { uint32_t * word; uint32_t value; };
 struct HostCopy { const void * dev; void * host; size_t bytes; };        // multiples of 4 bytes, dev 4-byte aligned; host null: not wanted
 struct HostStage {
