@@ -231,6 +231,8 @@ int pi_k_ffn_union_f16(const void * fc2_f16, int rank, const void * hid_f16, con
     if ((((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)down_t_f16 | (uintptr_t)xn_f16 | (uintptr_t)scratch | (uintptr_t)h_f16 | (uintptr_t)add1 |
           (uintptr_t)add2 | (uintptr_t)out) & 15) != 0)
         return pi::fail(PI_E_ARG, "pi_k_ffn_union_f16: operands must be 16-byte aligned");
+    for (int k = 0; parts && k < kUnionParts - 1; ++k)                  // (stored to and read in pieces of 16 bytes)
+        if (!parts[k] || ((uintptr_t)parts[k] & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_ffn_union_f16: parts must be three buffers on 16 bytes");
     const long long units = (long long)((2 * (long long)ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
     if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_union_f16: too many tiles");
     static const int raised = [] {

@@ -74,3 +74,17 @@ def test_what_it_refuses():
     d = pl.DevBuf.zeros(1 << 20)
     go = lambda rank=256, ff=256, cols=256, T=3, at=d.ptr: L.pi_k_ffn_union_f16(at, rank, d.ptr, d.ptr, None, d.ptr, ff, cols, d.ptr, T, 0.0, d.ptr, d.ptr, None, d.ptr, None, d.ptr, None, None)  # noqa: E731
     assert go(rank=128) != 0 and go(ff=128) != 0 and go(ff=300) != 0 and go(ff=32768 + 128) != 0 and go(cols=384) != 0 and go(T=0) != 0 and go(at=None) != 0 and go(at=d.ptr + 8) != 0
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("off", [None, 4, 8])
+def test_parts_that_it_refuses(which, off):
+    """A null among the three buffers, or one off 16 bytes: refused ahead of every launch, so that nothing is written."""
+    L = pl.init()
+    d, out = pl.DevBuf.zeros(1 << 20), pl.DevBuf.zeros(1 << 12)
+    pl.check(L.pi_memset(out.ptr, 0xAB, out.nbytes))
+    at = [d.ptr + (1 << 18) * (k + 1) for k in range(3)]
+    at[which] = None if off is None else at[which] + off
+    assert L.pi_k_ffn_union_f16(d.ptr, 256, d.ptr, d.ptr, None, d.ptr, 256, 256, d.ptr, 3, 0.0, d.ptr, d.ptr, (C.c_void_p * 3)(*at), d.ptr, None, out.ptr, None, None) != 0
+    pl.sync()
+    assert (out.download(np.uint8) == 0xAB).all()
