@@ -16,7 +16,8 @@ constexpr int kUnionLeast = 256;             // listed ones at least (four stage
 // The neurons that fire for a token of the chunk in ascending order, filled up to a multiple of 128 with one of them (h is 0 there), and the predictor's bits in that
 // order.  A workgroup for 16 tokens' bits, one for the list; each finds the neurons' places by itself.  n_active: of the last token.
 // Bound by latency (a few KB a workgroup): 4 us, 10 for 2047 tokens of 11008 neurons in one that went through a tile's words bit by bit.
-__global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * __restrict__ any, int any_rows, const unsigned long long * __restrict__ mask, int T, int ff, int32_t * __restrict__ list,
+// From `all_from` neurons on the list is all of them, and nobody packs anything (bits one by one for every neuron: 26 us for 32768 of them).
+__global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * __restrict__ any, int any_rows, const unsigned long long * __restrict__ mask, int T, int ff, int all_from, int32_t * __restrict__ list,
                                                               int32_t * __restrict__ count, unsigned long long * __restrict__ packed, int32_t * __restrict__ n_active) {
     extern __shared__ __align__(16) uint16_t bits[];                    // of the listed neurons, as a tile's words hold them
     __shared__ int sums[16], last;
@@ -40,21 +41,27 @@ __global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * _
     int n = 0;
     for (int k = 0; k < 16; ++k) { if (k == wave) at += n; n += sums[k]; }
     at -= own;
-    const int padded = max(kUnionLeast, (n + 127) / 128 * 128);
+    const int padded = n >= all_from ? ff : max(kUnionLeast, (n + 127) / 128 * 128);
     const auto place = [](int p) { return ((p >> 4) * 4 + (p & 3)) * 4 + (p >> 2 & 3); };
-    if (n + t < padded) bits[place(n + t)] = 0;
+    if (padded < ff && n + t < padded) bits[place(n + t)] = 0;
     if (own && at + own == n) last = 32 * t + 31 - __clz(fires);
     const unsigned long long word[8] = {w[0].x, w[0].y, w[1].x, w[1].y, w[2].x, w[2].y, w[3].x, w[3].y};
     if (tile == (int)gridDim.x - 1) {                                   // the list
+        if (padded == ff) {
+            for (int p = t; p < ff; p += 1024) list[p] = p;
+            if (t == 0) *count = ff;
+            return;
+        }
         for (int p = at; fires; fires &= fires - 1) list[p++] = 32 * t + __builtin_ctz(fires);
         __syncthreads();
         if (n + t < padded) list[n + t] = last;
         if (t == 0) *count = padded;
         return;
     }
+    if (padded < ff)
 #pragma unroll
-    for (int b = 0, p = at; b < 32; ++b)
-        if (fires >> b & 1) bits[place(p++)] = (uint16_t)(word[(b >> 4) * 4 + (b & 3)] >> 16 * (b >> 2 & 3));
+        for (int b = 0, p = at; b < 32; ++b)
+            if (fires >> b & 1) bits[place(p++)] = (uint16_t)(word[(b >> 4) * 4 + (b & 3)] >> 16 * (b >> 2 & 3));
     if (n_active && tile == (T - 1) / 16) {                             // (count_active_kernel has the same word)
         int mine = 0;
 #pragma unroll
@@ -65,15 +72,27 @@ __global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * _
         __syncthreads();
         if (t == 0) { int all = 0; for (int k = 0; k < 16; ++k) all += sums[k]; *n_active = all; }
     }
+    if (padded == ff) return;
     __syncthreads();
     for (int k = t; k < padded / 8; k += 1024) reinterpret_cast<uint4 *>(packed + (size_t)tile * (padded / 4))[k] = reinterpret_cast<const uint4 *>(bits)[k];
 }
 
+// How many may stay silent for all of them to be gone through as they lie, as ffn_wide_kernel does: what the list costs (its packing, and rows looked up one by one) is 15 to 50 us, what it
+// saves goes with the tokens.  Four layers, us, list / all.  All neurons fire: 7B 400 tokens 1194 / 1172, 13B 140 1200 / 1185, 300 1531 / 1463, 1800 4623 / 4574, 40B 57 1628 / 1520, 600 3705 /
+// 3617, 1900 8491 / 8367.  0.95 of them: 13B 90 tokens 1088 / 1101, 300 1508 / 1466, 40B 18 1547 / 1483, 320 2567 / 2479; but 13B 1800 4476 / 4537, 40B 1900 8294 / 8427.
+inline int union_silent(int ff, int T) { return ff / (T > 512 ? 32 : 16); }
+
 // gate, up and h of the listed neurons: h [T][count]
-template <bool PAIRS> __global__ __launch_bounds__(512, 1) void ffn_wide_union_kernel(FfnProduct<PAIRS, true, true> prod, const int32_t * __restrict__ count) {
+template <bool PAIRS> __global__ __launch_bounds__(512, 1) void ffn_wide_union_kernel(FfnProduct<PAIRS, true, true> prod, const unsigned long long * __restrict__ mask, const int32_t * __restrict__ count) {
     extern __shared__ __align__(16) unsigned char smem[];
-    prod.ff = *count;
-    gemm_wide<__half>(prod, WideDeal(PAIRS ? 2 * prod.ff : prod.ff, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
+    const int n = *count;
+    const WideDeal deal(PAIRS ? 2 * n : n, (prod.T + kGwN - 1) / kGwN, kGwBand);
+    if (n == prod.ff) {
+        gemm_wide<__half>(FfnProduct<PAIRS, true, false>{prod.up, prod.gate, prod.x, nullptr, prod.thr, prod.h16, n, prod.cols, prod.T, prod.nk, mask, nullptr}, deal, smem);
+        return;
+    }
+    prod.ff = n;
+    gemm_wide<__half>(prod, deal, smem);
 }
 
 // How the down projection's workgroups share its units (256 rows of a token tile): each XCD a contiguous range, band by band, as WideDeal has it.  What does not fill
@@ -250,11 +269,11 @@ int pi_k_ffn_union_f16(const void * fc2_f16, int rank, const void * hid_f16, con
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(mask_wide_any_kernel, dim3(wide_blocks(wide_tiles(ff, T))), dim3(512), kGwLds, st,
                        MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, mask, ff, rank, T, rank / kGtBK, (uint16_t *)(s + at.any)});
-    hipLaunchKernelGGL(ffn_union_list_kernel, dim3((T + 15) / 16 + 1), dim3(1024), (size_t)ff * 2, st, (const uint32_t *)(s + at.any), (T + 63) / 64, mask, T, ff, list, count, packed, n_active);
+    hipLaunchKernelGGL(ffn_union_list_kernel, dim3((T + 15) / 16 + 1), dim3(1024), (size_t)ff * 2, st, (const uint32_t *)(s + at.any), (T + 63) / 64, mask, T, ff, ff - union_silent(ff, T), list, count, packed, n_active);
     const auto wide = [&](auto pairs) {
         constexpr bool P = decltype(pairs)::value;
         hipLaunchKernelGGL(ffn_wide_union_kernel<P>, dim3(wide_blocks(wide_tiles(P ? 2 * ff : ff, T))), dim3(512), kGwLds, st,
-                           FfnProduct<P, true, true>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, nullptr, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK, packed, list}, count);
+                           FfnProduct<P, true, true>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, nullptr, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK, packed, list}, mask, count);
     };
     if (gate_f16) wide(std::true_type{}); else wide(std::false_type{});
     DownProduct d{(const __half *)down_t_f16, (const __half *)h_f16, list, add1, add2, out, cols, T, (uint32_t)(cols * 2), parts != nullptr, {}, 0, 0};

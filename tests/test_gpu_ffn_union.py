@@ -9,13 +9,16 @@ from powerinfer_amd import lib as pl
 pytestmark = pytest.mark.gpu
 
 
-def call(ff, rank, cols, T, gated, two, share, fill=None, split=True):
+def call(ff, rank, cols, T, gated, two, share, fill=None, split=True, silent=None):
     """share: of the neurons, how many may fire at all.  Factors of the predictor are small whole numbers, so that thresholds are met exactly."""
     L, rng = pl.init(), np.random.default_rng(ff + T + rank)
     up, gate, x, down = ((rng.standard_normal(s) / np.sqrt(s[1]) ** (s[0] != T)).astype(np.float16) for s in ((ff, cols), (ff, cols), (T, cols), (ff, cols)))
     fc2, hid = rng.integers(-3, 4, (ff, rank)).astype(np.float16), rng.integers(0, 3, (T, rank)).astype(np.float16)
     hid[:, 0] = 1
     fc2[rng.random(ff) >= share, 0] = -30000                              # never fires
+    if silent is not None:                                                # exactly as many never fire, the others for some token or all of them
+        fc2[:, 0] = 400
+        fc2[rng.choice(ff, silent, replace=False), 0] = -30000
     a1, a2 = rng.standard_normal((2, T, cols)).astype(np.float32)
     lg = (hid.astype(np.float64) @ fc2.astype(np.float64).T).astype(np.float32)
     thr = 20.0
@@ -45,6 +48,7 @@ def call(ff, rank, cols, T, gated, two, share, fill=None, split=True):
     got = out.download(np.float32)[:T * cols].reshape(T, cols)
     assert n.download(np.int32)[0] == active[-1].sum()
     assert (np.abs(got - want) <= bound + 1e-6 * np.abs(want)).all(), float((np.abs(got - want) / (bound + 1e-6 * np.abs(want))).max())
+    call.listed = scratch.download(np.int32)[-20]                         # (the last word but three ahead of the guard)
     return active.any(0).sum()
 
 
@@ -53,6 +57,15 @@ def call(ff, rank, cols, T, gated, two, share, fill=None, split=True):
                                                   (1024, 256, 1280, 257, 0.9), (11008, 1024, 4096, 140, 0.4), (32768, 256, 256, 130, 0.6), (512, 256, 4096, 2100, 0.7)])
 def test_matches_float64(ff, rank, cols, T, share, gated, two):
     call(ff, rank, cols, T, gated, two, share)
+
+
+@pytest.mark.parametrize("gated,two", [(True, False), (False, True)])
+@pytest.mark.parametrize("T,silent", [(300, 513), (300, 512), (300, 0), (530, 257), (530, 256)])
+def test_around_the_share_from_which_all_neurons_are_gone_through(T, silent, gated, two):
+    """8192 neurons: where no more than 512 stay silent (256 from 513 tokens on) bits and rows are gone through as they lie; beyond that the rows of silent ones are not read (NaN)."""
+    listed = silent > (256 if T > 512 else 512)
+    assert call(8192, 256, 256, T, gated, two, 1.0, silent=silent, fill=np.nan if listed else None) == 8192 - silent
+    assert call.listed == ((8192 - silent + 127) // 128 * 128 if listed else 8192)
 
 
 @pytest.mark.parametrize("ff,rank,cols,T", [(640, 256, 256, 64), (1024, 256, 4096, 600), (11008, 1024, 4096, 140)])
