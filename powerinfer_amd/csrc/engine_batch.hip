@@ -524,9 +524,16 @@ bool ffn_bits(pi_model * m, int il, int T) {
 // half of the 7B's fire: 130 tokens 1738 / 1562, 400 2487 / 1992, 2047 6746 / 5255; 0.43 of the 40B's: 18 tokens 1401 / 1149, 300 2692 / 1775, 1900 7730 / 5379;
 // 0.53 of the 13B's: 50 tokens 940 / 902, 700 2160 / 1810, 1800 4329 / 3513.  All of them (tokens with nothing in common): 7B 130 tokens 1784 / 1729,
 // 2047 6719 / 6707, 13B 140 1145 / 1165, 700 2181 / 2189, 1800 4357 / 4520, 40B 300 2692 / 2420, 900 4130 / 4174, 1900 7705 / 8284.
-bool ffn_union(pi_model * m, int il) {
+bool ffn_union_shape(pi_model * m, int il) {
     const int r = (int)m->L(il, PI_T_FC1).ne1;
     return ffn_in_one(m, il) && pi_k_ffn_union_supported(m->hp.n_ff, r, m->hp.n_embd) && (((uintptr_t)m->L(il, PI_T_FC2).dev | (uintptr_t)m->L(il, PI_T_FFN_DOWN_T).dev) & 15) == 0;
+}
+// Smaller matrices are the launches' time in shorter chunks, of which the list has more.  The FFN alone, us, all neurons / listed, where all, three quarters and half of them fire: 5632 x 2048,
+// 200 tokens 43 / 55, 56 and 52, 400 56 / 63, 60 and 54, 700 82 / 90, 72 and 64; 8192 x 3072, 130 74 / 84, 85 and 74, 200 83 / 84, 89 and 78, 400 102 / 105, 99 and 86; 11008 x 4096, 130
+// 123 / 120, 111 and 99.
+constexpr int kUnionSmallRows = 256;
+bool ffn_union(pi_model * m, int il, int T) {
+    return ffn_union_shape(m, il) && ffn_bits(m, il, T) && ((long long)m->hp.n_ff * m->hp.n_embd >= 32LL << 20 || T > kUnionSmallRows);
 }
 
 int wide_layer(pi_model * m, BatchState * b, int il) {
@@ -575,9 +582,8 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
         else ffn_x = b->xa16;
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
-    // (the token that comes along does not change how the others go)
-    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, b->ends ? T - 1 : T);
-    if (ffn_union(m, il) && ffn_bits(m, il, b->ends ? T - 1 : T)) {
+    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, T);
+    if (ffn_union(m, il, T)) {
         float * const parts[3] = {b->qkv, b->att, falcon ? b->ffn_inp : b->attn_out};      // (of no use any more, T * d values and more)
         PI_TRY(pi_k_ffn_union_f16(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, down.dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, parts,
                                   falcon ? b->attn_out : b->ffn_inp, falcon ? x : nullptr, b->x2, b->ends ? m->n_active + il : nullptr, st));
@@ -701,7 +707,7 @@ static int wide_buffers(pi_model * m, BatchState * b, int rows) {
     m->give_back(b->sized);
     b->rows = 0;
     int apart = 0;
-    for (int il = 0; il < m->hp.n_layer; ++il) apart = std::max(apart, !ffn_in_one(m, il) ? rows : ffn_large(m) && !ffn_union(m, il) ? kFfnOneRows : 0);
+    for (int il = 0; il < m->hp.n_layer; ++il) apart = std::max(apart, !ffn_in_one(m, il) ? rows : ffn_large(m) && !ffn_union_shape(m, il) ? kFfnOneRows : 0);
     const bool falcon = m->hp.arch == PI_ARCH_FALCON;
     const size_t mark = m->owned.size(), ff = m->hp.n_ff;
     bool ok = step_buffers(m, b, rows, false);
@@ -768,7 +774,7 @@ int prefill_wide_chunk(pi_model * m, const int32_t * tokens, int left, int n_pas
             if (m->L(il, PI_T_WO).type == PI_TYPE_Q4_0) w16 = std::max(w16, (size_t)hp.n_embd * hp.n_embd);
             if (split || m->L(il, PI_T_FFN_UP).type == PI_TYPE_Q4_0 || m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_Q4_0) w16 = std::max(w16, (size_t)hp.n_ff * hp.n_embd);
             if (split || m->L(il, PI_T_FFN_DOWN_T).type == PI_TYPE_Q4_0) { scratch = true; continue; }
-            if (!cells_only(m, il) && !(ffn_large(m) && ffn_union(m, il))) PI_TRY(ensure_down_rows(m, il));      // (read row by row there)
+            if (!cells_only(m, il) && !(ffn_large(m) && ffn_union_shape(m, il))) PI_TRY(ensure_down_rows(m, il));      // (read row by row there)
         }
         if (w16) b->w16 = m->alloc<__half>(w16);
         if (scratch) b->w16t = m->alloc<__half>((size_t)hp.n_embd * hp.n_ff);
