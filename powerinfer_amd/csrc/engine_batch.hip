@@ -520,10 +520,11 @@ bool ffn_bits(pi_model * m, int il, int T) {
 }
 
 // Only the neurons that fire for one of the chunk's tokens (pi_k_ffn_union_f16), where the predictor leaves bits: what no token fires is neither read nor multiplied.
-// How many that are is the text's: words that come again fire what fired before.  Eight 7B-shaped layers, four of the others, us, all neurons / listed.  Where
-// half of the 7B's fire: 130 tokens 1738 / 1562, 400 2487 / 1992, 2047 6746 / 5255; 0.43 of the 40B's: 18 tokens 1401 / 1149, 300 2692 / 1775, 1900 7730 / 5379;
-// 0.53 of the 13B's: 50 tokens 940 / 902, 700 2160 / 1810, 1800 4329 / 3513.  All of them (tokens with nothing in common): 7B 130 tokens 1784 / 1729,
-// 2047 6719 / 6707, 13B 140 1145 / 1165, 700 2181 / 2189, 1800 4357 / 4520, 40B 300 2692 / 2420, 900 4130 / 4174, 1900 7705 / 8284.
+// How many that are is the text's: words that come again fire what fired before, and where nearly all do its launches leave the list alone.  Prompts of four layers, us, all neurons by the
+// library's down projection / listed.  Half of them fire: 7B 130 tokens 873 / 789, 400 1228 / 974, 2047 3136 / 2485; 13B 50 967 / 918, 700 2176 / 1793, 1800 4419 / 3461; 40B 18 1439 / 1275, 300
+// 2779 / 1887, 1900 8072 / 5936.  All of them do (tokens with nothing in common): 7B 130 890 / 874, 1200 2181 / 2226, 2047 3185 / 3157; 13B 50 1009 / 1049, 300 1482 / 1468, 900 2592 / 2634, 1800
+// 4483 / 4611; 40B 18 1500 / 1477, 57 1739 / 1503, 300 2862 / 2431, 600 3384 / 3476, 1400 6356 / 6623, 1600 8414 / 7532, 1900 8251 / 8658: the library's product over so many rows is up to a
+// sixth faster than this one's tiles at some lengths and a quarter slower at others, and would have to be asked for before anybody knows the count.
 bool ffn_union_shape(pi_model * m, int il) {
     const int r = (int)m->L(il, PI_T_FC1).ne1;
     return ffn_in_one(m, il) && pi_k_ffn_union_supported(m->hp.n_ff, r, m->hp.n_embd) && (((uintptr_t)m->L(il, PI_T_FC2).dev | (uintptr_t)m->L(il, PI_T_FFN_DOWN_T).dev) & 15) == 0;

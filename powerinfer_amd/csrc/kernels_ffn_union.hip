@@ -117,7 +117,7 @@ struct DownDeal {
         ty = b0 + in % high; row0 = in / high * kGwM;
     }
     // the workgroup's c-th: and which part of its neurons (of `parts`, 1: all)
-    __device__ __forceinline__ void unit(int c, int & ty, int & row0, int & rows, int & part, int & of) const {
+    __host__ __device__ __forceinline__ void unit(int c, int & ty, int & row0, int & rows, int & part, int & of) const {
         const bool last = c >= rounds;
         const int sub = slot % (parts * halves);
         tile(last ? rounds * slots + slot / (parts * halves) : c * slots + slot, ty, row0);
@@ -127,17 +127,41 @@ struct DownDeal {
     }
 };
 
+// DownDeal, and where what does not fill the XCD's workgroups once more is from a half to three quarters of them: its units in three or four parts, which the workgroups take in two
+// or three turns, all units' first parts first (workgroups side by side go through the same rows; an equal range of stages for each, wherever it begins, is slower than leaving the
+// others idle: 40B, 600 tokens, four layers 3600 -> 4000 us).  Prompts of four layers, us, whole / in turns, all neurons firing: 13B 800 tokens 2597 / 2469, 1000 2948 / 2780, 40B 520 3521 / 3312, 600
+// 3710 / 3455, 1600 7813 / 7534; half of them: 13B 800 2028 / 2002, 40B 600 2765 / 2639.  Shorter lists gain less than the sums take (7B, 86 stages of 172, 1200 tokens: 1749 / 1760).  The launch that adds the parts comes whether this list is long enough or not, so it is asked for by the longest one.
+constexpr int kUnionMostStages = 64, kUnionStages = 24;               // of a part: of the longest list, and of this one
+struct DownSplit {
+    DownDeal deal;
+    int parts, count;
+    bool turns;
+    // most: stages of all neurons (no room for parts: 0), nk: of the listed ones
+    __host__ __device__ __forceinline__ DownSplit(const DownDeal & d, int most, int nk) : deal(d) {
+        parts = d.rest * 3 <= d.slots * 2 ? 3 : 4;
+        turns = d.rest * 2 > d.slots && d.rest * 4 <= d.slots * 3 && most >= kUnionMostStages * parts && nk >= kUnionStages * parts;
+        if (!turns) parts = d.parts;
+        count = turns ? d.rounds + (d.rest * parts - d.slot + d.slots - 1) / d.slots : d.count;
+    }
+    __host__ __device__ __forceinline__ void unit(int c, int & ty, int & row0, int & rows, int & part, int & of) const {
+        if (!turns || c < deal.rounds) return deal.unit(c, ty, row0, rows, part, of);
+        const int at = deal.slot + (c - deal.rounds) * deal.slots;
+        deal.tile(deal.rounds * deal.slots + at % deal.rest, ty, row0);
+        rows = kGwM; part = at / deal.rest; of = parts;
+    }
+};
+
 // out[t][c] = sum over the listed neurons of h[t][k] down_t[list[k]][c], and what is added to it
 struct DownProduct {
     static constexpr bool kPairs = false, kList = false, kTurned = true;
     static constexpr int kM = kGwM, kN = kGwN;
     const __half * down, * h; const int32_t * turned; const float * add1, * add2; float * out;
-    int rows, T; uint32_t col_bytes; bool room; float * parts[kUnionParts - 1];
+    int rows, T; uint32_t col_bytes; int most; float * parts[kUnionParts - 1];
     int n, nk;                                                          // listed neurons, stages of them
     __device__ __forceinline__ bool read_once(const WidePlace &) const { return false; }
     __device__ __forceinline__ int first(const WidePlace & p) const { return nk * (p.grp & 7) / (p.grp >> 3); }
     __device__ __forceinline__ int stages(const WidePlace & p) const { return nk * ((p.grp & 7) + 1) / (p.grp >> 3) - first(p); }
-    __device__ __forceinline__ WidePlace place(const DownDeal & deal, int c) const {       // (grp: which part, and of how many)
+    __device__ __forceinline__ WidePlace place(const DownSplit & deal, int c) const {      // (grp: which part, and of how many)
         WidePlace p;
         int ty, part, of;
         deal.unit(c, ty, p.row0, p.rows, part, of);
@@ -188,15 +212,16 @@ struct DownProduct {
 __global__ __launch_bounds__(512, 1) void ffn_union_down_kernel(DownProduct a, const int32_t * __restrict__ count) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int n = *count;
-    const DownDeal deal(a.rows, (a.T + kGwN - 1) / kGwN, a.room, (int)blockIdx.x % 8, (int)blockIdx.x / 8, (int)gridDim.x / 8);
-    const DownProduct prod{a.down, a.h, a.turned, a.add1, a.add2, a.out, a.rows, a.T, a.col_bytes, a.room, {a.parts[0], a.parts[1], a.parts[2]}, n, n / kGtBK};
-    gemm_wide<__half>(prod, deal, smem);
+    const DownDeal deal(a.rows, (a.T + kGwN - 1) / kGwN, a.most > 0, (int)blockIdx.x % 8, (int)blockIdx.x / 8, (int)gridDim.x / 8);
+    const DownProduct prod{a.down, a.h, a.turned, a.add1, a.add2, a.out, a.rows, a.T, a.col_bytes, a.most, {a.parts[0], a.parts[1], a.parts[2]}, n, n / kGtBK};
+    gemm_wide<__half>(prod, DownSplit(deal, a.most, prod.nk), smem);
 }
-// Units that were shared: out += the other parts in their order, and what is added to them; 1024 values of a unit a workgroup, four a thread
+// (count: null where no list has turns)  Units that were shared: out += the other parts in their order, and what is added to them; 1024 values of a unit a workgroup, four a thread
 constexpr int kUnionGrid = 256;              // workgroups of the down projection
-__global__ __launch_bounds__(256) void ffn_union_sum_kernel(DownProduct a) {
-    const DownDeal deal(a.rows, (a.T + kGwN - 1) / kGwN, a.room, (int)blockIdx.z, 0, kUnionGrid / 8);
-    if (deal.parts == 1 || (int)blockIdx.y >= deal.rest) return;
+__global__ __launch_bounds__(256) void ffn_union_sum_kernel(DownProduct a, const int32_t * __restrict__ count) {
+    const DownDeal deal(a.rows, (a.T + kGwN - 1) / kGwN, a.most > 0, (int)blockIdx.z, 0, kUnionGrid / 8);
+    const int parts = count ? DownSplit(deal, a.most, *count / kGtBK).parts : deal.parts;
+    if (parts == 1 || (int)blockIdx.y >= deal.rest) return;
     int ty, row0;
     deal.tile(deal.rounds * deal.slots + (int)blockIdx.y, ty, row0);
     const int t = ty * kGwN + (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6);
@@ -205,11 +230,11 @@ __global__ __launch_bounds__(256) void ffn_union_sum_kernel(DownProduct a) {
     float4 v = *reinterpret_cast<const float4 *>(a.out + o), b[kUnionParts - 1] = {}, a1 = *reinterpret_cast<const float4 *>(a.add1 + o), a2{};
 #pragma unroll
     for (int k = 0; k < kUnionParts - 1; ++k)
-        if (k + 1 < deal.parts) b[k] = *reinterpret_cast<const float4 *>(a.parts[k] + o);
+        if (k + 1 < parts) b[k] = *reinterpret_cast<const float4 *>(a.parts[k] + o);
     if (a.add2) a2 = *reinterpret_cast<const float4 *>(a.add2 + o);
 #pragma unroll
     for (int k = 0; k < kUnionParts - 1; ++k)
-        if (k + 1 < deal.parts) { v.x += b[k].x; v.y += b[k].y; v.z += b[k].z; v.w += b[k].w; }
+        if (k + 1 < parts) { v.x += b[k].x; v.y += b[k].y; v.z += b[k].z; v.w += b[k].w; }
     v = make_float4(__fadd_rn(v.x, a1.x), __fadd_rn(v.y, a1.y), __fadd_rn(v.z, a1.z), __fadd_rn(v.w, a1.w));
     if (a.add2) v = make_float4(__fadd_rn(v.x, a2.x), __fadd_rn(v.y, a2.y), __fadd_rn(v.z, a2.z), __fadd_rn(v.w, a2.w));
     *reinterpret_cast<float4 *>(a.out + o) = v;
@@ -276,15 +301,17 @@ int pi_k_ffn_union_f16(const void * fc2_f16, int rank, const void * hid_f16, con
                            FfnProduct<P, true, true>{(const __half *)up_f16, (const __half *)gate_f16, (const __half *)xn_f16, nullptr, threshold, (__half *)h_f16, ff, cols, T, cols / kGtBK, packed, list}, mask, count);
     };
     if (gate_f16) wide(std::true_type{}); else wide(std::false_type{});
-    DownProduct d{(const __half *)down_t_f16, (const __half *)h_f16, list, add1, add2, out, cols, T, (uint32_t)(cols * 2), parts != nullptr, {}, 0, 0};
+    DownProduct d{(const __half *)down_t_f16, (const __half *)h_f16, list, add1, add2, out, cols, T, (uint32_t)(cols * 2), parts ? ff / kGtBK : 0, {}, 0, 0};
     for (int k = 0; parts && k < kUnionParts - 1; ++k) d.parts[k] = parts[k];
     hipLaunchKernelGGL(ffn_union_down_kernel, dim3(kUnionGrid), dim3(512), kGwLds, st, d, count);
     int shared = 0;                                                      // units of an XCD that were
+    bool turns = false;                                                  // (or may be, by how many are listed)
     for (int x = 0; x < 8; ++x) {
-        const DownDeal deal(cols, (T + kGwN - 1) / kGwN, d.room, x, 0, kUnionGrid / 8);
-        if (deal.parts > 1) shared = std::max(shared, deal.rest);
+        const DownSplit deal(DownDeal(cols, (T + kGwN - 1) / kGwN, parts != nullptr, x, 0, kUnionGrid / 8), d.most, d.most);
+        turns = turns || deal.turns;
+        if (deal.parts > 1) shared = std::max(shared, deal.deal.rest);
     }
-    if (shared) hipLaunchKernelGGL(ffn_union_sum_kernel, dim3(kGwN / 4, shared, 8), dim3(256), 0, st, d);
+    if (shared) hipLaunchKernelGGL(ffn_union_sum_kernel, dim3(kGwN / 4, shared, 8), dim3(256), 0, st, d, turns ? count : nullptr);
     return pi::check_launch("pi_k_ffn_union_f16");
 }
 

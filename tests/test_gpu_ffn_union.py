@@ -59,6 +59,13 @@ def test_matches_float64(ff, rank, cols, T, share, gated, two):
     call(ff, rank, cols, T, gated, two, share)
 
 
+# 160 and 192 units of the down projection for 256 workgroups: in three parts from 72 stages on (4608 listed neurons) where all are 192 and more, in four from 96 (6144) of 256, whole otherwise
+@pytest.mark.parametrize("ff,cols,T,silent", [(12288, 4096, 1200, 0), (12288, 4096, 1200, 12288 - 4608), (12288, 4096, 1200, 12288 - 4480), (12160, 4096, 1200, 0), (16384, 4096, 1500, 512),
+                                              (16384, 4096, 1500, 16384 - 6144), (16384, 4096, 1500, 16384 - 6016), (16256, 4096, 1500, 0), (12288, 8192, 520, 1000)])
+def test_units_that_do_not_fill_the_chip(ff, cols, T, silent):
+    call(ff, 256, cols, T, False, True, 1.0, silent=silent)
+
+
 @pytest.mark.parametrize("gated,two", [(True, False), (False, True)])
 @pytest.mark.parametrize("T,silent", [(300, 513), (300, 512), (300, 0), (530, 257), (530, 256)])
 def test_around_the_share_from_which_all_neurons_are_gone_through(T, silent, gated, two):
