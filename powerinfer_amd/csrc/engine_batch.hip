@@ -523,8 +523,7 @@ bool ffn_bits(pi_model * m, int il, int T) {
 // How many that are is the text's: words that come again fire what fired before, and where nearly all do its launches leave the list alone.  Prompts of four layers, us, all neurons by the
 // library's down projection / listed.  Half of them fire: 7B 130 tokens 873 / 789, 400 1228 / 974, 2047 3136 / 2485; 13B 50 967 / 918, 700 2176 / 1793, 1800 4419 / 3461; 40B 18 1439 / 1275, 300
 // 2779 / 1887, 1900 8072 / 5936.  All of them do (tokens with nothing in common): 7B 130 890 / 874, 1200 2181 / 2226, 2047 3185 / 3157; 13B 50 1009 / 1049, 300 1482 / 1468, 900 2592 / 2634, 1800
-// 4483 / 4611; 40B 18 1500 / 1477, 57 1739 / 1503, 300 2862 / 2431, 600 3384 / 3476, 1400 6356 / 6623, 1600 8414 / 7532, 1900 8251 / 8658: the library's product over so many rows is up to a
-// sixth faster than this one's tiles at some lengths and a quarter slower at others, and would have to be asked for before anybody knows the count.
+// 4483 / 4611; 40B 18 1500 / 1477, 57 1739 / 1503, 300 2862 / 2431, 600 3384 / 3476, 1400 6356 / 6623, 1600 8414 / 7532, 1900 8251 / 8658.
 bool ffn_union_shape(pi_model * m, int il) {
     const int r = (int)m->L(il, PI_T_FC1).ne1;
     return ffn_in_one(m, il) && pi_k_ffn_union_supported(m->hp.n_ff, r, m->hp.n_embd) && (((uintptr_t)m->L(il, PI_T_FC2).dev | (uintptr_t)m->L(il, PI_T_FFN_DOWN_T).dev) & 15) == 0;
@@ -536,6 +535,12 @@ constexpr int kUnionSmallRows = 256;
 bool ffn_union(pi_model * m, int il, int T) {
     return ffn_union_shape(m, il) && ffn_bits(m, il, T) && ((long long)m->hp.n_ff * m->hp.n_embd >= 32LL << 20 || T > kUnionSmallRows);
 }
+
+// With all neurons the library's product is faster than these tiles at some lengths and slower at others, which no rule tells apart, but for the longest chunks, of which long prompts
+// consist: bits, FFN and sums, us, own / library: 32768 x 8192 (no gate) 1600 tokens 1727 / 1962, 1792 1772 / 2024, 1900 1910 / 1770, 2047 1917 / 1784; 28672 x 8192 1792 2248 / 2422, 1900 2378 /
+// 2248, 2047 2357 / 2223; 13824 x 5120 1700 750 / 729, 1900 834 / 792, 2047 836 / 803; 11008 x 4096 2047 518 / 529.  The host has to know for it: it hears of the list's length while gate and
+// up, half a millisecond and more, are on their way.  The copy that it reads is made when a layer first comes to it; where there is no memory for that the layer stays with the stored rows.
+constexpr int kUnionAskRows = 1792;
 
 int wide_layer(pi_model * m, BatchState * b, int il) {
     const pi_hparams & hp = m->hp;
@@ -586,8 +591,15 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, T);
     if (ffn_union(m, il, T)) {
         float * const parts[3] = {b->qkv, b->att, falcon ? b->ffn_inp : b->attn_out};      // (of no use any more, T * d values and more)
-        PI_TRY(pi_k_ffn_union_f16(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, down.dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, parts,
-                                  falcon ? b->attn_out : b->ffn_inp, falcon ? x : nullptr, b->x2, b->ends ? m->n_active + il : nullptr, st));
+        const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
+        uint32_t * told = ffn_large(m) && T > kUnionAskRows && !b->route.pieces ? m->stage.ask() : nullptr, listed = 0;
+        PI_TRY(pi::ffn_union_hidden(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, b->ends ? m->n_active + il : nullptr,
+                                    told, st));
+        if (told) PI_TRY(m->stage.answer(st, &listed));
+        const bool lib = told && (int)listed == ff && ensure_down_rows(m, il) == PI_OK;
+        (void)hipGetLastError();                                    // (no memory for the copy: the next launch's check is not to find this)
+        if (lib) PI_TRY(chunk_gemm(m, b, m->down_rows[il], d, ff, b->h16, falcon ? PI_EPI_ADD2 : PI_EPI_ADD, a1, a2, b->x2, nullptr));
+        else PI_TRY(pi::ffn_union_down(down.dev, ff, d, T, b->pred_logits, b->h16, parts, a1, a2, b->x2, st));
         std::swap(b->x, b->x2);
         return PI_OK;
     }

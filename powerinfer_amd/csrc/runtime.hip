@@ -1,6 +1,7 @@
 // Device/runtime plumbing of the C ABI: init, memory, copies, events, error string.
 #include <chrono>
 #include <mutex>
+#include <thread>
 #include "device_utils.hpp"
 #include "runtime.hpp"
 #include "../../include/powerinfer_hip.h"
@@ -83,9 +84,10 @@ void HostStage::init(size_t usual_bytes) {
         for (int i = 0; i < pinned_n && !pin; ++i)
             if (pinned_kept[i].bytes == piece * n_pieces) { pin = pinned_kept[i].p; pinned_kept[i] = pinned_kept[--pinned_n]; }
     }
-    if (!pin && hipHostMalloc((void **)&pin, piece * n_pieces + 4 * kPieces * kBlocks, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
+    if (!pin && hipHostMalloc((void **)&pin, piece * n_pieces + 4 * kPieces * kBlocks + 64, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) { pin = nullptr; (void)hipGetLastError(); return; }
     done = reinterpret_cast<uint32_t *>(pin + piece * n_pieces);
-    memset(done, 0, 4 * kPieces * kBlocks);
+    told = done + kPieces * kBlocks;
+    memset(done, 0, 4 * kPieces * kBlocks + 64);
     seq = 0;
 }
 
@@ -101,6 +103,7 @@ void HostStage::release() {
         if (--pinned_users == 0) while (pinned_n) out[n++] = pinned_kept[--pinned_n].p;
     }
     pin = nullptr;
+    told = nullptr;
     while (n) (void)hipHostFree(out[--n]);
 }
 
@@ -111,6 +114,19 @@ int HostStage::until(const HostDone & d, int words, hipStream_t st) {
         // what does not get through, or takes longer than a token, is the runtime's to wait for
         if (k % 64 == 0 && std::chrono::steady_clock::now() > end) { PI_HIP_TRY(hipStreamSynchronize(st)); return PI_OK; }
         __builtin_ia32_pause();
+    }
+    return PI_OK;
+}
+int HostStage::answer(hipStream_t st, uint32_t * value) {
+    const auto soon = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+    for (int k = 1; !(*value = __atomic_load_n(told, __ATOMIC_ACQUIRE)); ++k) {
+        if (k % 64 || std::chrono::steady_clock::now() < soon) { __builtin_ia32_pause(); continue; }
+        std::this_thread::sleep_for(std::chrono::microseconds(50));
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+        if (e != hipSuccess) return hip_fail(e, "HostStage::answer");
+        if (!(*value = __atomic_load_n(told, __ATOMIC_ACQUIRE))) return fail(PI_E_STATE, "HostStage::answer: no launch has answered");
+        break;
     }
     return PI_OK;
 }

@@ -39,6 +39,7 @@ struct HostStage {
     unsigned char * pin = nullptr;         // null (no pinned memory to be had): ordinary copies
     size_t piece = 0; int n_pieces = 0;
     bool counted = false, busy = false;    // one of the pool's users; a call ended early, work on the memory may be left
+    uint32_t * told = nullptr;             // a word behind those: what a launch in the middle of a call says, for what the host queues next
     uint32_t * done = nullptr, seq = 0;    // [kPieces][kBlocks] behind the pieces: where the workgroups that store results say that they are through, and what the last launch's say
     void init(size_t usual_bytes);
     void release();
@@ -51,6 +52,9 @@ struct HostStage {
     // for the launch that the last `next()` went to, the last of the stream, one of whose workgroups speaks for all; apart: the runtime's wait, which leaves the core to others
     int wait(hipStream_t st, bool apart = false);
     int until(const HostDone & d, int words, hipStream_t st);
+    // room for a number above 0 (null: none) that a launch to come stores, and the wait for it: it may have much ahead of it, so the host looks rarely before long
+    uint32_t * ask() { if (told) __atomic_store_n(told, 0u, __ATOMIC_RELEASE); return told; }
+    int answer(hipStream_t st, uint32_t * value);
 };
 
 // pi_k_attn_fused with such extra workgroups
@@ -99,6 +103,10 @@ int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t 
 int resume_token(const float * row, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
 // how many neurons of a chunk's last token (T of them) fire, by the predictor's logits [T][ff] or its bits (pi_k_ffn_wide_predicted_f16)
 int count_active(const float * logits, const void * mask, int T, int ff, float thr, int32_t * n_active, pi_stream_t stream);
+// The two halves of pi_k_ffn_union_f16, checked as there: predictor bits, list and h [T][number of listed ones], which `told` gets too (ff: all of them, and in their order), and the down projection
+int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold, void * scratch,
+                     void * h_f16, int32_t * n_active, uint32_t * told, pi_stream_t stream);
+int ffn_union_down(const void * down_t_f16, int ff, int cols, int T, const void * scratch, const void * h_f16, float * const * parts, const float * add1, const float * add2, float * out, pi_stream_t stream);
 // the embedding rows of tokens that the host names, at positions from `pos` on, and these positions
 int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream);
 
