@@ -34,9 +34,11 @@ constexpr int kPfChunk = 8;                       // active neurons per round tr
 // a hand-over to the host announced by the first lane of a launch (see host_signal_kernel): device counter and word 0 of the pinned flags
 struct HostAnnounce { uint32_t * seq; uint32_t * flags; uint32_t * words_out = nullptr; };    // words_out: a second copy of the activity words (pinned memory) for the logits-only launch
 
+// LDS: a group's predictor rows go there (rows_lds, kPfRowsLds<RCH> bytes, W2 on 16; a wave reads only what it requested): in registers they would leave a unit no room for other workgroups
+// beside this one.  Where nothing else is to run there registers are faster (32768 neurons of 8192 columns, rank 1024, us, registers / LDS: 36.0 / 38.8, with a gate 44.9 / 47.7, 0.6 of the
+// neurons on the device 28.6 / 31.5; rank 512 31.6 / 34.4).
 template <int RCH> constexpr int kPfRowsLds = kPfWaves * 4 * RCH * 1024;
-// ANYWHERE: W2 may start off a multiple of 16 bytes
-template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0, bool ANYWHERE = true>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
+template <int CPW, int RCH, bool GATE, int G, bool HYB, int PHASE = 0, bool LDS = false>      // cols == 8 waves * CPW chunks * 512; r == RCH * 512; G groups of 32 neurons
 __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, const float * __restrict__ hidden,
                                                                    const __half * __restrict__ Wup, const __half * __restrict__ Wgate,
                                                                    const __half * __restrict__ Wdown,
@@ -63,40 +65,29 @@ __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, 
     const int cbase = wave * CPW * 512 + lane * 8;     // chunk c of this lane starts at column cbase + 512*c
 
     // ---- A: loads ------------------------------------------------------------------------------------------
-    // Several groups: a group's predictor rows go to LDS (rows_lds, kPfRowsLds<RCH> bytes; a wave reads only what it requested), and the next group's travel while this group's
-    // FFN rows are fetched and used.  In registers they would leave a unit no room for other workgroups beside this one.
-    const auto request = [&](int first) {
-        typedef const __attribute__((address_space(1))) void * gptr;
-        typedef __attribute__((address_space(3))) void * lptr;
-        const int w = __builtin_amdgcn_readfirstlane(wave);
-        if (ANYWHERE && ((uintptr_t)W2 & 15) != 0) {                    // (copies to LDS want whole pieces)
-            pi_u32x4 v[4][RCH];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < RCH; ++j) v[i][j] = pi_ld_stream(W2 + (size_t)(first + w * 4 + i) * r + (j * PI_WAVE + lane) * 8);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < RCH; ++j) *reinterpret_cast<pi_u32x4 *>(rows_lds + ((w * 4 + i) * RCH + j) * 1024 + lane * 16) = v[i][j];
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < RCH; ++j)
-                __builtin_amdgcn_global_load_lds((gptr)(W2 + (size_t)(first + w * 4 + i) * r + (j * PI_WAVE + lane) * 8), (lptr)(rows_lds + ((w * 4 + i) * RCH + j) * 1024), 16, 0, 2);
-    };
+    // (several groups: the next group's predictor rows travel while this group's FFN rows are fetched and used)
     pi_u32x4 a[4][RCH];
+    const auto request = [&](int first) {
+        if constexpr (LDS) {
+            typedef const __attribute__((address_space(1))) void * gptr;
+            typedef __attribute__((address_space(3))) void * lptr;
+            const int w = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < RCH; ++j)
+                    __builtin_amdgcn_global_load_lds((gptr)(W2 + (size_t)(first + w * 4 + i) * r + (j * PI_WAVE + lane) * 8), (lptr)(rows_lds + ((w * 4 + i) * RCH + j) * 1024), 16, 0, 2);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(first + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
+        }
+    };
     float4 hv[RCH][2];
     float logit_in = 0.0f;
     if (PHASE != 2) {
-        if constexpr (G > 1) request(n0);
-        else
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < RCH; ++j) a[i][j] = pi_ld_stream(W2 + (size_t)(n0 + wave * 4 + i) * r + (j * PI_WAVE + lane) * 8);
+        request(n0);
 #pragma unroll
         for (int j = 0; j < RCH; ++j) {
             hv[j][0] = *reinterpret_cast<const float4 *>(hidden + j * 512 + lane * 8);
@@ -122,6 +113,16 @@ __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, 
     }
     // ---- A: logits (the CPU path rounds the hidden vector to fp16 before the dot, ggml.c:9703-9716) ------------
     pi_u32x4 hr[RCH];
+    const auto logits_of = [&](int g) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float lacc = 0.0f;
+#pragma unroll
+            for (int j = 0; j < RCH; ++j) lacc = pi_dot8h(LDS ? *reinterpret_cast<const pi_u32x4 *>(rows_lds + ((wave * 4 + i) * RCH + j) * 1024 + lane * 16) : a[i][j], hr[j], lacc);
+            lacc = pi_wave_sum(lacc);
+            if (lane == 0) lg[g & 1][wave * 4 + i] = lacc;
+        }
+    };
     if (PHASE != 2) {
 #pragma unroll
         for (int j = 0; j < RCH; ++j) {
@@ -129,15 +130,9 @@ __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, 
                              __floats2half2_rn(hv[j][1].x, hv[j][1].y), __floats2half2_rn(hv[j][1].z, hv[j][1].w)};
             hr[j] = *reinterpret_cast<const pi_u32x4 *>(hh);
         }
-        if constexpr (G == 1) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float acc = 0.0f;
-#pragma unroll
-                for (int j = 0; j < RCH; ++j) acc = pi_dot8h(a[i][j], hr[j], acc);
-                acc = pi_wave_sum(acc);
-                if (lane == 0) lg[0][wave * 4 + i] = acc;
-            }
+        if constexpr (!LDS) {
+            logits_of(0);
+            if (G > 1) request(n0 + 32);
         }
     }
     // ---- A: norm statistics across the 8 slices ---------------------------------------------------------------
@@ -208,20 +203,17 @@ __device__ __forceinline__ void pred_ffn_groups(const __half * __restrict__ W2, 
         for (int k = 0; k < 8; ++k) acc[c][k] = 0.0f;
 #pragma unroll 1
     for (int g = 0; g < G; ++g, n0 += 32) {
-    if constexpr (G > 1) {
+    if constexpr (LDS) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0x0F70);                             // vmcnt(0): the rows have arrived (what was requested behind them has been used)
         asm volatile("" ::: "memory");
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float lacc = 0.0f;
-#pragma unroll
-            for (int j = 0; j < RCH; ++j) lacc = pi_dot8h(*reinterpret_cast<const pi_u32x4 *>(rows_lds + ((wave * 4 + i) * RCH + j) * 1024 + lane * 16), hr[j], lacc);
-            lacc = pi_wave_sum(lacc);
-            if (lane == 0) lg[g & 1][wave * 4 + i] = lacc;
-        }
+        logits_of(g);
         __builtin_amdgcn_s_waitcnt(0xC07F);                             // lgkmcnt(0): read, before the next ones come
         asm volatile("" ::: "memory");
+        if (g + 1 < G) request(n0 + 32);
+        __syncthreads();
+    } else if (g > 0) {
+        logits_of(g);
         if (g + 1 < G) request(n0 + 32);
         __syncthreads();
     }
@@ -312,8 +304,7 @@ __global__ __launch_bounds__(kPfBlock, 2) void pred_ffn_f16_kernel(const __half 
                                                                    const uint32_t * __restrict__ hot_words, const int32_t * __restrict__ hot_prefix,
                                                                    uint32_t * __restrict__ words_hot, __half * __restrict__ xn_out,
                                                                    float * __restrict__ logits2, HostAnnounce ann) {
-    __shared__ __align__(16) unsigned char rows[G > 1 ? kPfRowsLds<RCH> : 16];
-    pred_ffn_groups<CPW, RCH, GATE, G, HYB, PHASE>(W2, hidden, Wup, Wgate, Wdown, x, na, thr, logits, words, h_dense, partial, hot_words, hot_prefix, words_hot, xn_out, logits2, ann, blockIdx.x, rows);
+    pred_ffn_groups<CPW, RCH, GATE, G, HYB, PHASE>(W2, hidden, Wup, Wgate, Wdown, x, na, thr, logits, words, h_dense, partial, hot_words, hot_prefix, words_hot, xn_out, logits2, ann, blockIdx.x, nullptr);
 }
 
 // Falcon's attention and FFN both read the layer's input: the attention's workgroups and the FFN's in one launch (F16, 8192 columns, four groups of 32 neurons a workgroup),
@@ -351,7 +342,7 @@ __global__ __launch_bounds__(kPfBlock, 4) void attn_ffn_kernel(const float * __r
             attn_fused_head<kPfBlock, LPP>(qkv, rope_table, k_cache, v_cache, n_head, n_head_kv, hd, mode, n_ctx, pos_p, out, 0, 0, 0, nullptr, 0, nullptr, nullptr, nullptr, b, 0);
         return;
     }
-    pred_ffn_groups<2, RCH, false, 4, false, 0, false>(W2, hidden, Wup, nullptr, Wdown, x, na, thr, nullptr, words, nullptr, partial, nullptr, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, b - n_attn, smem);
+    pred_ffn_groups<2, RCH, false, 4, false, 0, true>(W2, hidden, Wup, nullptr, Wdown, x, na, thr, nullptr, words, nullptr, partial, nullptr, nullptr, nullptr, nullptr, nullptr, HostAnnounce{nullptr, nullptr}, b - n_attn, smem);
 }
 
 // ---------------------------------------------------------------------------------------------------
