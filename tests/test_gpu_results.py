@@ -56,3 +56,28 @@ def test_models_that_come_and_go():
         t.join()
     print(len(got), flush=True)
     assert len(got) == 12 and all(np.array_equal(g, want) for g in got)
+
+
+@pytest.mark.parametrize("n_vocab", [1000, 9001, 40003])
+def test_no_step_gets_results_of_the_one_before(n_vocab):
+    """Steps of two sets of tokens in turn, whose logits differ everywhere: every row is bit for bit what the same step gave when it was repeated, where results that are late are the same ones.
+    16 rows are one piece of pinned memory, two, and five, which is more than the ring has; a single token's are stored by the launch that chooses the next one."""
+    from powerinfer_amd.model import Model
+    hp = synth.hparams("llama-tiny", n_vocab=n_vocab, n_ctx=64, seed=11, sparse_threshold=-1e30)
+    gm = Model(hp).load(synth.make_model(hp))
+    gm.batch_init(16)
+    rng = np.random.default_rng(n_vocab)
+    sets = rng.permutation(n_vocab)[:32].astype(np.int32).reshape(2, 16)
+    where = np.zeros(16, np.int32)
+    rows = [[(n.copy(), lg.copy()) for n, lg in (gm.batch_decode(s, where) for _ in range(3))][-1] for s in sets]
+    ones = [[(n, lg.copy()) for n, lg in (gm.decode([s[0]], 0) for _ in range(3))][-1] for s in sets]
+    assert (rows[0][1] != rows[1][1]).mean() > 0.99 and (ones[0][1] != ones[1][1]).mean() > 0.99
+    for k in range(400):
+        if k % 100 == 0:
+            print(n_vocab, k, flush=True)
+        i = k & 1
+        nxt, lg = gm.batch_decode(sets[i], where)
+        assert np.array_equal(lg, rows[i][1]) and np.array_equal(nxt, rows[i][0]), k
+        one, lg = gm.decode([sets[i][0]], 0)
+        assert one == ones[i][0] and np.array_equal(lg, ones[i][1]), k
+    gm.close()
