@@ -59,6 +59,13 @@ def test_matches_float64(ff, rank, cols, T, share, gated, two):
     call(ff, rank, cols, T, gated, two, share)
 
 
+@pytest.mark.parametrize("gated,two", [(True, False), (False, True)])
+@pytest.mark.parametrize("ff,T,share", [(4224, 20, 0.5), (5120, 70, 0.5), (4352, 150, 0.9), (2304, 257, 1.0)])
+def test_matches_float64_of_8192_columns(ff, T, share, gated, two):
+    """A row's sum begins at a column stage that goes with its place, in the list or (the last) among all neurons: places from 2048 on begin elsewhere."""
+    call(ff, 256, 8192, T, gated, two, share)
+
+
 # 160 and 192 units of the down projection for 256 workgroups: in three parts from 72 stages on (4608 listed neurons) where all are 192 and more, in four from 96 (6144) of 256, whole otherwise
 @pytest.mark.parametrize("ff,cols,T,silent", [(12288, 4096, 1200, 0), (12288, 4096, 1200, 12288 - 4608), (12288, 4096, 1200, 12288 - 4480), (12160, 4096, 1200, 0), (16384, 4096, 1500, 512),
                                               (16384, 4096, 1500, 16384 - 6144), (16384, 4096, 1500, 16384 - 6016), (16256, 4096, 1500, 0), (12288, 8192, 520, 1000)])
