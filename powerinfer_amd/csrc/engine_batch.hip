@@ -520,7 +520,8 @@ bool ffn_bits(pi_model * m, int il, int T) {
 }
 
 // Only the neurons that fire for one of the chunk's tokens (pi_k_ffn_union_f16), where the predictor leaves bits: what no token fires is neither read nor multiplied.
-// How many that are is the text's: words that come again fire what fired before, and where nearly all do its launches leave the list alone.  Prompts of four layers, us, all neurons by the
+// How many that are is the text's: words that come again fire what fired before, and where nearly all do its launches leave the list alone.
+// Results are repeatable, but the last bits of a token's FFN depend on its company: on the chunk's length, as the library's plans do, and on what the other tokens fire.  Prompts of four layers, us, all neurons by the
 // library's down projection / listed.  Half of them fire: 7B 130 tokens 873 / 789, 400 1228 / 974, 2047 3136 / 2485; 13B 50 967 / 918, 700 2176 / 1793, 1800 4419 / 3461; 40B 18 1439 / 1275, 300
 // 2779 / 1887, 1900 8072 / 5936.  All of them do (tokens with nothing in common): 7B 130 890 / 874, 1200 2181 / 2226, 2047 3185 / 3157; 13B 50 1009 / 1049, 300 1482 / 1468, 900 2592 / 2634, 1800
 // 4483 / 4611; 40B 18 1500 / 1477, 57 1739 / 1503, 300 2862 / 2431, 600 3384 / 3476, 1400 6356 / 6623, 1600 8414 / 7532, 1900 8251 / 8658.
@@ -744,6 +745,8 @@ static int wide_buffers(pi_model * m, BatchState * b, int rows) {
 // 3020 / 2603, 2047 7564 / 7105; four 13B-shaped ones, 700 tokens 2500 / 2255; four 40B-shaped ones, 300 tokens 3062 / 2742.  For F16 matrices that are whole
 // on the device, whose products round at the same places for one token and for many; Q4_0 ones of chunks round their values to fp16 besides, and
 // a layer that is split has the host's share of a lone token.  (The route without the library is there to be compared with, and stays as it is.)
+// A neuron that does not fire is no term for a token alone and a product with 0 in a chunk: an infinite weight in a row that another token fires makes the last token's cells NaN,
+// which its logits were anyway, through that token's cells.
 bool prefill_ends(pi_model * m) {
     if (m->hybrid || m->capture || m->hp.n_layer < 2 || (!m->gemm_lib && prefill_own_gemm())) return false;
     for (int il = 0; il < m->hp.n_layer; ++il)

@@ -18,7 +18,8 @@ template <bool PAIRS, bool MASK, bool LIST = false> struct FfnProduct {
     __device__ __forceinline__ bool read_once(const WidePlace &) const { return false; }
     // Rows a multiple of 16 KB apart lie in few of the memory's channels: every 2048 of them begin at columns of their own (bits included, us, one place for all /
     // this: 32768 x 8192 alone, 17 tokens 124 / 94 and 128 135 / 104 (no bits), 129 tokens 161 / 142, 200 175 / 155, 400 247 / 252, 700 381 / 390, 2047 1027 / 1029; 4096 columns, twice 11008 rows: 129 tokens 63.2 /
-    // 64.5, 2047 372 / 370, so not there).  The place goes by the row alone: a token's sums have one order however many come along.
+    // 64.5, 2047 372 / 370, so not there).  The place goes by the row alone: a token's sums have one order
+    // however many come along.  With LIST it is a row's place in the list, which the other tokens of the chunk decide.
     __device__ __forceinline__ int first(const WidePlace & p) const { return cols % 8192 ? 0 : p.row0 / 2048 % 8 * nk / 8; }
     const __half * up, * gate, * x; const float * logits; float thr; __half * h16;
     int ff, cols, T, nk;

@@ -26,7 +26,8 @@ __device__ __forceinline__ pi_u32x4 turned_fragment(const unsigned char * p) {
 // whole and the present one is free to be copied over.  LDS rows and swizzle are GemmTile's; a copy's 64 lanes bring eight rows of
 // 128 bytes and take the swizzle on the side they read from.  Where half a tile or less is wanted (half its rows, or so few tokens that a wave would
 // have none) the four waves share that half, 64 x 64 outputs each.  The sums are formed in GemmTile's order: 32 columns a step, beginning at a stage that
-// depends on the product and the row alone (first), so that a token's outputs are the same bits whichever tiles it falls into.
+// depends on the product and the row alone (first), so that a token's outputs are the same bits whichever tiles it falls into.  Not so over
+// listed neurons: the list, where a row's sum begins and (kTurned) into which parts it is cut are the chunk's, by its length and by what all of its tokens fire.
 // Measured (us; 128 x 128 tiles of GemmTile before): 64 experts of 192 tokens on average, 1408 x 4096: 301 -> 215, 4096 x 1408:
 // 307 -> 226 (weights alone: 123 at 6 TB/s); one group of 12288: 199 -> 133, 1.07 PFLOP/s; 16 experts of 128: 51 -> 45 and 38 -> 34.
 // ---------------------------------------------------------------------------------------------------------------------------------

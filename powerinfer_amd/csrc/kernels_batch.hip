@@ -1342,6 +1342,13 @@ int count_active(const float * logits, const void * mask, int T, int ff, float t
     hipLaunchKernelGGL(count_active_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, logits, (const unsigned long long *)mask, T, ff, thr, n_active);
     return check_launch("count_active");
 }
+int predictor_bits(const void * fc2_f16, int ff, int rank, const void * hid_f16, int T, float threshold, void * mask, void * any, pi_stream_t stream) {
+    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&mask_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
+    if (raised != hipSuccess) return hip_fail(raised, "mask_wide: LDS size");
+    hipLaunchKernelGGL(mask_wide_kernel, dim3(wide_blocks((long long)((ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN))), dim3(512), kGwLds, (hipStream_t)stream,
+                       MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, (unsigned long long *)mask, ff, rank, T, rank / kGtBK, (uint16_t *)any});
+    return check_launch("mask_wide");
+}
 }  // namespace pi
 
 // logits or mask, not both
@@ -1397,11 +1404,7 @@ int pi_k_ffn_wide_predicted_f16(const void * fc2_f16, int rank, const void * hid
     if ((((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)mask) & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_predicted_f16: operands must be 16-byte aligned");
     const long long units = (long long)((ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
     if (units > (1 << 30)) return pi::fail(PI_E_ARG, "pi_k_ffn_wide_predicted_f16: too many tiles");
-    static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(&mask_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kGwLds);
-    if (raised != hipSuccess) return pi::hip_fail(raised, "mask_wide: LDS size");
-    hipLaunchKernelGGL(mask_wide_kernel, dim3(wide_blocks(units)), dim3(512), kGwLds, (hipStream_t)stream,
-                       MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, (unsigned long long *)mask, ff, rank, T, rank / kGtBK, nullptr});
-    if (const int rc = pi::check_launch("mask_wide")) return rc;
+    if (const int rc = pi::predictor_bits(fc2_f16, ff, rank, hid_f16, T, threshold, mask, nullptr, stream)) return rc;
     return ffn_wide(up_f16, gate_f16, ff, cols, xn_f16, T, nullptr, (const unsigned long long *)mask, threshold, h_f16, stream);
 }
 

@@ -239,10 +239,6 @@ __global__ __launch_bounds__(256) void ffn_union_sum_kernel(DownProduct a, const
     if (a.add2) v = make_float4(__fadd_rn(v.x, a2.x), __fadd_rn(v.y, a2.y), __fadd_rn(v.z, a2.z), __fadd_rn(v.w, a2.w));
     *reinterpret_cast<float4 *>(a.out + o) = v;
 }
-__global__ __launch_bounds__(512, 1) void mask_wide_any_kernel(MaskProduct prod) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    gemm_wide<__half>(prod, WideDeal(prod.rows, (prod.T + kGwN - 1) / kGwN, kGwBand), smem);
-}
 
 template <typename K> int raise_lds(K kernel, int bytes) {
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -279,8 +275,7 @@ int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const
     const long long units = (long long)((2 * (long long)ff + kGwM - 1) / kGwM) * ((T + kGwN - 1) / kGwN);
     if (units > (1 << 30)) return fail(PI_E_ARG, "pi_k_ffn_union_f16: too many tiles");
     static const int raised = [] {
-        int rc = raise_lds(mask_wide_any_kernel, kGwLds);
-        if (rc == PI_OK) rc = raise_lds(ffn_union_list_kernel, 2 * kUnionMost);
+        int rc = raise_lds(ffn_union_list_kernel, 2 * kUnionMost);
         if (rc == PI_OK) rc = raise_lds(ffn_wide_union_kernel<true>, kGwLds);
         return rc == PI_OK ? raise_lds(ffn_wide_union_kernel<false>, kGwLds) : rc;
     }();
@@ -290,8 +285,7 @@ int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const
     unsigned long long * mask = (unsigned long long *)s, * packed = (unsigned long long *)(s + at.packed);
     int32_t * list = (int32_t *)(s + at.list), * count = (int32_t *)(s + at.count);
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(mask_wide_any_kernel, dim3(wide_blocks(wide_tiles(ff, T))), dim3(512), kGwLds, st,
-                       MaskProduct{(const __half *)fc2_f16, (const __half *)hid_f16, threshold, mask, ff, rank, T, rank / kGtBK, (uint16_t *)(s + at.any)});
+    if (const int rc = predictor_bits(fc2_f16, ff, rank, hid_f16, T, threshold, mask, s + at.any, stream)) return rc;
     hipLaunchKernelGGL(ffn_union_list_kernel, dim3((T + 15) / 16 + 1), dim3(1024), (size_t)ff * 2, st, (const uint32_t *)(s + at.any), (T + 63) / 64, mask, T, ff, ff - union_silent(ff, T), told, list, count, packed,
                        n_active);
     const auto wide = [&](auto pairs) {

@@ -103,6 +103,8 @@ int embed_start(int wtype, const void * table, int cols, int32_t token, int32_t 
 int resume_token(const float * row, int cols, int32_t token, int32_t pos, int32_t * d_token, int32_t * d_pos, int32_t * d_step, float * x, pi_stream_t stream);
 // how many neurons of a chunk's last token (T of them) fire, by the predictor's logits [T][ff] or its bits (pi_k_ffn_wide_predicted_f16)
 int count_active(const float * logits, const void * mask, int T, int ff, float thr, int32_t * n_active, pi_stream_t stream);
+// the predictor's bits of a chunk (pi_k_ffn_wide_predicted_f16, which checks the operands) and, where `any` is not null, 64 tokens at a time, which neurons fire for one of them, a bit a neuron
+int predictor_bits(const void * fc2_f16, int ff, int rank, const void * hid_f16, int T, float threshold, void * mask, void * any, pi_stream_t stream);
 // The two halves of pi_k_ffn_union_f16, checked as there: predictor bits, list and h [T][number of listed ones], which `told` gets too (ff: all of them, and in their order), and the down projection
 int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold, void * scratch,
                      void * h_f16, int32_t * n_active, uint32_t * told, pi_stream_t stream);
