@@ -589,8 +589,9 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
         else ffn_x = b->xa16;
     }
     PI_TRY(chunk_gemm(m, b, fc1.dev, r, d, b->xp16, PI_EPI_RELU, nullptr, nullptr, b->hidden, b->hid16));
-    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, T);
-    if (ffn_union(m, il, T)) {
+    const int others = b->ends ? T - 1 : T;                         // (bits or logits, listed or not: as for the same tokens of a prompt that goes on)
+    const bool one_kernel = ffn_in_one(m, il) && (T > kFfnOneRows || !ffn_large(m)), bits = one_kernel && ffn_bits(m, il, others);
+    if (ffn_union(m, il, others)) {
         float * const parts[3] = {b->qkv, b->att, falcon ? b->ffn_inp : b->attn_out};      // (of no use any more, T * d values and more)
         const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
         uint32_t * told = ffn_large(m) && T > kUnionAskRows && !b->route.pieces ? m->stage.ask() : nullptr, listed = 0;
