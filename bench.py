@@ -900,7 +900,7 @@ def main():
             out["prompt_phase"] = {"tokens": args.prompt_bench, "ms": round(dt * 1e3, 2), "tok_per_s": round(args.prompt_bench / dt, 1),
                                    "gemm": "own LDS-tiled MFMA kernel" if os.environ.get("PI_PREFILL_GEMM") == "own" else "hipBLASLt plans",
                                    "what": "pi_model_decode of the whole prompt: chunks of up to 2048 tokens (dense mat-muls through hipBLASLt plans, or on this library's own kernel with PI_PREFILL_GEMM=own; each weight "
-                                           "row read once per chunk, predictor mask applied to h), last token through the single-token path"
+                                           "row read once per chunk, predictor mask applied to h), last token alone through the last layer (F16) or through all of them"
                                            + ("; Q4_0 matrices expanded to fp16 per chunk, activations through Q8_0 blocks" if hp.wtype != pl.F16 else "")
                                            + ("; non-resident FFN rows read from pinned host memory once per chunk" if hybrid else "")}
             m2.close()

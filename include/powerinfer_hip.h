@@ -383,7 +383,8 @@ PI_API int pi_k_ffn_wide_predicted_f16(const void * fc2_f16, int rank, const voi
                                        const void * xn_f16, int T, float threshold, void * mask, void * h_f16, pi_stream_t stream);
 /* The whole sparse FFN over the neurons that fire for a token of the chunk: out[t][c] = add1[t][c] (+ add2[t][c]) + sum of h[t][n] down_t[n][c], down_t [ff][cols].  scratch:
  * pi_k_ffn_union_scratch(ff, T) bytes; h_f16: T * ff values of room; parts: null or room for three times T * cols values, with which a short chunk's down projection
- * is shared by more workgroups; n_active (may be null): how many fire for the last token.  All operands 16-byte aligned. */
+ * is shared by more workgroups; n_active (may be null): how many fire for the last token.  All operands 16-byte aligned.  Where nearly all neurons fire, all of them are gone through.
+ * A token's sums have the order that T and what its company fires give them. */
 PI_API int pi_k_ffn_union_supported(int ff, int rank, int cols);
 PI_API size_t pi_k_ffn_union_scratch(int ff, int T);
 PI_API int pi_k_ffn_union_f16(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, const void * down_t_f16, int ff, int cols,
