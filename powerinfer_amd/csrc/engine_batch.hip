@@ -594,11 +594,12 @@ int wide_layer(pi_model * m, BatchState * b, int il) {
     if (ffn_union(m, il, others)) {
         float * const parts[3] = {b->qkv, b->att, falcon ? b->ffn_inp : b->attn_out};      // (of no use any more, T * d values and more)
         const float * a1 = falcon ? b->attn_out : b->ffn_inp, * a2 = falcon ? x : nullptr;
-        uint32_t * told = ffn_large(m) && T > kUnionAskRows && !b->route.pieces ? m->stage.ask() : nullptr, listed = 0;
+        const pi::HostAsk told = ffn_large(m) && T > kUnionAskRows && !b->route.pieces ? m->stage.ask() : pi::HostAsk{};
+        uint32_t listed = 0;
         PI_TRY(pi::ffn_union_hidden(fc2.dev, r, b->hid16, up.dev, falcon ? nullptr : m->L(il, PI_T_FFN_GATE).dev, ff, d, ffn_x, T, hp.sparse_threshold, b->pred_logits, b->h16, b->ends ? m->n_active + il : nullptr,
                                     told, st));
-        if (told) PI_TRY(m->stage.answer(st, &listed));
-        const bool lib = told && (int)listed == ff && ensure_down_rows(m, il) == PI_OK;
+        if (told.word) PI_TRY(m->stage.answer(st, &listed));
+        const bool lib = told.word && (int)listed == ff && ensure_down_rows(m, il) == PI_OK;
         (void)hipGetLastError();                                    // (no memory for the copy: the next launch's check is not to find this)
         if (lib) PI_TRY(chunk_gemm(m, b, m->down_rows[il], d, ff, b->h16, falcon ? PI_EPI_ADD2 : PI_EPI_ADD, a1, a2, b->x2, nullptr));
         else PI_TRY(pi::ffn_union_down(down.dev, ff, d, T, b->pred_logits, b->h16, parts, a1, a2, b->x2, st));

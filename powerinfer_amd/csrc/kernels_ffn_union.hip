@@ -16,8 +16,8 @@ constexpr int kUnionLeast = 256;             // listed ones at least (four stage
 // The neurons that fire for a token of the chunk in ascending order, filled up to a multiple of 128 with one of them (h is 0 there), and the predictor's bits in that
 // order.  A workgroup for 16 tokens' bits, one for the list; each finds the neurons' places by itself.  n_active: of the last token.
 // Bound by latency (a few KB a workgroup): 4 us, 10 for 2047 tokens of 11008 neurons in one that went through a tile's words bit by bit.
-// told (or null): a word of the host's that gets their number.  From `all_from` neurons on the list is all of them, and nobody packs anything (bits one by one for every neuron: 26 us for 32768 of them).
-__global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * __restrict__ any, int any_rows, const unsigned long long * __restrict__ mask, int T, int ff, int all_from, uint32_t * __restrict__ told, int32_t * __restrict__ list,
+// told (its word may be null): gets their number, 16 bits.  From `all_from` neurons on the list is all of them, and nobody packs anything (bits one by one for every neuron: 26 us for 32768 of them).
+__global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * __restrict__ any, int any_rows, const unsigned long long * __restrict__ mask, int T, int ff, int all_from, pi::HostAsk told, int32_t * __restrict__ list,
                                                               int32_t * __restrict__ count, unsigned long long * __restrict__ packed, int32_t * __restrict__ n_active) {
     extern __shared__ __align__(16) uint16_t bits[];                    // of the listed neurons, as a tile's words hold them
     __shared__ int sums[16], last;
@@ -49,13 +49,13 @@ __global__ __launch_bounds__(1024) void ffn_union_list_kernel(const uint32_t * _
     if (tile == (int)gridDim.x - 1) {                                   // the list
         if (padded == ff) {
             for (int p = t; p < ff; p += 1024) list[p] = p;
-            if (t == 0) { *count = ff; if (told) __hip_atomic_store(told, (uint32_t)ff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+            if (t == 0) { *count = ff; if (told.word) __hip_atomic_store(told.word, told.tag | (uint32_t)ff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
             return;
         }
         for (int p = at; fires; fires &= fires - 1) list[p++] = 32 * t + __builtin_ctz(fires);
         __syncthreads();
         if (n + t < padded) list[n + t] = last;
-        if (t == 0) { *count = padded; if (told) __hip_atomic_store(told, (uint32_t)padded, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+        if (t == 0) { *count = padded; if (told.word) __hip_atomic_store(told.word, told.tag | (uint32_t)padded, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
         return;
     }
     if (padded < ff)
@@ -267,7 +267,7 @@ size_t pi_k_ffn_union_scratch(int ff, int T) { return UnionScratch(ff, T).bytes;
 }  // extern "C"
 namespace pi {
 int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold, void * scratch,
-                     void * h_f16, int32_t * n_active, uint32_t * told, pi_stream_t stream) {
+                     void * h_f16, int32_t * n_active, const HostAsk & told, pi_stream_t stream) {
     if (!fc2_f16 || !hid_f16 || !up_f16 || !xn_f16 || !scratch || !h_f16 || T <= 0) return fail(PI_E_ARG, "pi_k_ffn_union_f16: bad arguments");
     if (!pi_k_ffn_union_supported(ff, rank, cols)) return fail(PI_E_UNSUPPORTED, "pi_k_ffn_union_f16: ff a multiple of 128 from 256 to 32768, cols one of 256, rank one of 64 from 256 on");
     if ((((uintptr_t)fc2_f16 | (uintptr_t)hid_f16 | (uintptr_t)up_f16 | (uintptr_t)gate_f16 | (uintptr_t)xn_f16 | (uintptr_t)scratch | (uintptr_t)h_f16) & 15) != 0)
@@ -324,7 +324,7 @@ int pi_k_ffn_union_f16(const void * fc2_f16, int rank, const void * hid_f16, con
     if ((((uintptr_t)down_t_f16 | (uintptr_t)add1 | (uintptr_t)add2 | (uintptr_t)out) & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_ffn_union_f16: operands must be 16-byte aligned");
     for (int k = 0; parts && k < kUnionParts - 1; ++k)                  // (stored to and read in pieces of 16 bytes)
         if (!parts[k] || ((uintptr_t)parts[k] & 15) != 0) return pi::fail(PI_E_ARG, "pi_k_ffn_union_f16: parts must be three buffers on 16 bytes");
-    const int rc = pi::ffn_union_hidden(fc2_f16, rank, hid_f16, up_f16, gate_f16, ff, cols, xn_f16, T, threshold, scratch, h_f16, n_active, nullptr, stream);
+    const int rc = pi::ffn_union_hidden(fc2_f16, rank, hid_f16, up_f16, gate_f16, ff, cols, xn_f16, T, threshold, scratch, h_f16, n_active, pi::HostAsk{}, stream);
     return rc != PI_OK ? rc : pi::ffn_union_down(down_t_f16, ff, cols, T, scratch, h_f16, parts, add1, add2, out, stream);
 }
 

@@ -88,7 +88,7 @@ void HostStage::init(size_t usual_bytes) {
     done = reinterpret_cast<uint32_t *>(pin + piece * n_pieces);
     told = done + kPieces * kBlocks;
     memset(done, 0, 4 * kPieces * kBlocks + 64);
-    seq = 0;
+    seq = asked = 0;
 }
 
 void HostStage::release() {
@@ -119,13 +119,18 @@ int HostStage::until(const HostDone & d, int words, hipStream_t st) {
 }
 int HostStage::answer(hipStream_t st, uint32_t * value) {
     const auto soon = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
-    for (int k = 1; !(*value = __atomic_load_n(told, __ATOMIC_ACQUIRE)); ++k) {
+    const auto here = [&] {
+        const uint32_t v = __atomic_load_n(told, __ATOMIC_ACQUIRE);
+        *value = v & 0xFFFF;
+        return (v & ~0xFFFFu) == asked;
+    };
+    for (int k = 1; !here(); ++k) {
         if (k % 64 || std::chrono::steady_clock::now() < soon) { __builtin_ia32_pause(); continue; }
         std::this_thread::sleep_for(std::chrono::microseconds(50));
         const hipError_t e = hipStreamQuery(st);
         if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
         if (e != hipSuccess) return hip_fail(e, "HostStage::answer");
-        if (!(*value = __atomic_load_n(told, __ATOMIC_ACQUIRE))) return fail(PI_E_STATE, "HostStage::answer: no launch has answered");
+        if (!here()) return fail(PI_E_STATE, "HostStage::answer: no launch has answered");
         break;
     }
     return PI_OK;

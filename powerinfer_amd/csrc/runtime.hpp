@@ -32,6 +32,7 @@ int  noalloc_setup();                                  // resolves the static sc
 // steps of 16 requests 17180 -> 16790; a prompt of 333 and 16 tokens 9220 -> 8950.  (Before the wait behind the write-back, pi_release, without which a word may get ahead of its
 // values; with it these are as fast within the spread.)
 struct HostDone { uint32_t * word; uint32_t value; };
+struct HostAsk { uint32_t * word = nullptr; uint32_t tag = 0; };
 struct HostCopy { const void * dev; void * host; size_t bytes; };        // multiples of 4 bytes, dev 4-byte aligned; host null: not wanted
 struct HostStage {
     static constexpr int kPieces = 4, kMaxCopies = 4, kKept = 4, kBlocks = 64;      // (kBlocks: workgroups of a copy)
@@ -39,7 +40,7 @@ struct HostStage {
     unsigned char * pin = nullptr;         // null (no pinned memory to be had): ordinary copies
     size_t piece = 0; int n_pieces = 0;
     bool counted = false, busy = false;    // one of the pool's users; a call ended early, work on the memory may be left
-    uint32_t * told = nullptr;             // a word behind those: what a launch in the middle of a call says, for what the host queues next
+    uint32_t * told = nullptr, asked = 0;  // a word behind those: what a launch in the middle of a call says, for what the host queues next, and the tag of the last question
     uint32_t * done = nullptr, seq = 0;    // [kPieces][kBlocks] behind the pieces: where the workgroups that store results say that they are through, and what the last launch's say
     void init(size_t usual_bytes);
     void release();
@@ -52,8 +53,9 @@ struct HostStage {
     // for the launch that the last `next()` went to, the last of the stream, one of whose workgroups speaks for all; apart: the runtime's wait, which leaves the core to others
     int wait(hipStream_t st, bool apart = false);
     int until(const HostDone & d, int words, hipStream_t st);
-    // room for a number above 0 (null: none) that a launch to come stores, and the wait for it: it may have much ahead of it, so the host looks rarely before long
-    uint32_t * ask() { if (told) __atomic_store_n(told, 0u, __ATOMIC_RELEASE); return told; }
+    // a question that a launch to come answers with tag | a number of 16 bits (word null: nowhere to), and the wait for the answer, which may have much ahead of it: the host looks rarely
+    // before long.  The tags differ, so that an answer left by a call that failed is nobody's.
+    HostAsk ask() { asked += 1u << 16; if (!asked) asked = 1u << 16; return {told, asked}; }
     int answer(hipStream_t st, uint32_t * value);
 };
 
@@ -107,7 +109,7 @@ int count_active(const float * logits, const void * mask, int T, int ff, float t
 int predictor_bits(const void * fc2_f16, int ff, int rank, const void * hid_f16, int T, float threshold, void * mask, void * any, pi_stream_t stream);
 // The two halves of pi_k_ffn_union_f16, checked as there: predictor bits, list and h [T][number of listed ones], which `told` gets too (ff: all of them, and in their order), and the down projection
 int ffn_union_hidden(const void * fc2_f16, int rank, const void * hid_f16, const void * up_f16, const void * gate_f16, int ff, int cols, const void * xn_f16, int T, float threshold, void * scratch,
-                     void * h_f16, int32_t * n_active, uint32_t * told, pi_stream_t stream);
+                     void * h_f16, int32_t * n_active, const HostAsk & told, pi_stream_t stream);
 int ffn_union_down(const void * down_t_f16, int ff, int cols, int T, const void * scratch, const void * h_f16, float * const * parts, const float * add1, const float * add2, float * out, pi_stream_t stream);
 // the embedding rows of tokens that the host names, at positions from `pos` on, and these positions
 int embed_chunk(int wtype, const void * table, int cols, const int32_t * tokens, int T, int pos, float * x, int32_t * d_pos, pi_stream_t stream);

@@ -18,14 +18,17 @@ for il in range(hp.n_layer):
         m.set_tensor(il, k, a)
 m.finalize()
 
+class Ask(C.Structure):                          # HostAsk of runtime.hpp
+    _fields_ = [("word", C.c_void_p), ("tag", C.c_uint32)]
+
 say, asked = None, []
 @C.CFUNCTYPE(None, C.c_char_p, C.POINTER(C.c_void_p))
 def watch(name, args):
     if b"ffn_union_list_kernel" in name:
-        told = C.cast(args[6], C.POINTER(C.c_void_p))[0]
-        asked.append(bool(told))
-        if told and say:
-            C.cast(told, C.POINTER(C.c_uint32))[0] = say
+        told = C.cast(args[6], C.POINTER(Ask))[0]
+        asked.append(bool(told.word))
+        if told.word and say:
+            C.cast(told.word, C.POINTER(C.c_uint32))[0] = told.tag | say
 F.fake_watch(watch)
 
 def go(n, number):
@@ -61,9 +64,9 @@ m.close()
 
 
 def test_a_launch_that_does_not_answer():
-    """An error and not a wait for ever."""
+    """An error and not a wait for ever, nor the number of the call before."""
     fake_hip.run(CODE + """
-go(1792, ff)
+assert go(2000, ff)[1] == 0
 try:
     go(2000, 0)
     raise SystemExit("no error")
